@@ -214,7 +214,7 @@ int smx_reduce_forces_device(smx_model* m, int num_atoms, const int* d_sender_at
  * inputs (the forces of the model's last evaluation, d_sender_atom[num_edges] on the device, receiver i = atom i),
  * outputs in device memory (d_atom_forces[3*num_atoms], d_virial[6]; either may be NULL), work enqueued on `stream`
  * without synchronising.  The per-atom sender lists and the partial virial sums live in a fixed array of about
- * 20 MiB that every GPU holds from the first model load to the end of the process, so sizes beyond
+ * 35 MiB that every GPU holds from the first model load to the end of the process, so sizes beyond
  * SMX_NOALLOC_MAX_ATOMS atoms or SMX_NOALLOC_MAX_EDGES edges are refused with SMX_EINVAL, and calls that overlap on
  * one GPU race (all of them share that GPU's array).  `stream` must be the stream of the evaluation whose forces
  * are reduced, or be ordered after it by the caller (an event wait): the call reads the model's node_forces and
@@ -245,6 +245,11 @@ void smx_nlist_free(smx_nlist* nl);
 int smx_nlist_build(smx_nlist* nl, int num_atoms, const double* d_positions, const int* d_types, int num_shifts,
                     const int* shift_int, const double* shift_vec, double r_list, double r_cut, void* stream,
                     long* num_edges);
+/* smx_compute_device followed by smx_reduce_forces_device on the arrays of a list built from host positions, with the
+ * results in host memory: energies[num_atoms], atom_forces[num_atoms][3], virial[6].  One call for callers that hand
+ * over positions and want atoms' forces back (the calculator): the evaluation's sender lists serve the reduction and
+ * everything returns in one copy. */
+int smx_evaluate_list(smx_model* m, smx_nlist* nl, double* energies, double* atom_forces, double* virial);
 /* Same list from new positions without a new search: the pairs found within r_list by the last build are
  * re-measured and those inside r_cut kept, in the same canonical order (the cutoff filter that the LAMMPS caller
  * applies to its skin list every step, pair_symmetrix_mace.cpp:287-315).  Equal to a fresh build at r_cut as long
@@ -257,6 +262,11 @@ int smx_nlist_update(smx_nlist* nl, const double* d_positions, const int* d_type
  * last build. */
 int smx_nlist_build_host(smx_nlist* nl, int num_atoms, const double* positions, const int* types, int num_shifts,
                          const int* shift_int, const double* shift_vec, double r_list, double r_cut, long* num_edges);
+/* smx_nlist_build_host for an orthorhombic cell of the given edge lengths: folds the positions into the cell along the
+ * axes with pbc[k] != 0, considers every image shift that covers r_list, and reports the lattice offsets taken off
+ * (offsets[num_atoms][3], positions = folded + offsets * cell; *folded tells whether one of them is not zero). */
+int smx_nlist_build_box(smx_nlist* nl, int num_atoms, const double* positions, const int* types, const double* cell,
+                        const int* pbc, double r_list, double r_cut, long long* offsets, int* folded, long* num_edges);
 int smx_nlist_update_host(smx_nlist* nl, const double* positions, double r_cut, long* num_edges);
 int smx_nlist_inputs(smx_nlist* nl, const double** d_positions, const int** d_types);
 int smx_nlist_arrays(smx_nlist* nl, const int** num_neigh, const int** first_neigh, const int** neigh_indices,

@@ -48,28 +48,21 @@ class SymmetrixCalculator:
                 f"and pass the JSON file it writes.") from exc
         self.cutoff = self.evaluator.r_cut
         self.results = {}
+        # species index of every atomic number, -1 where the model does not have the element
+        self._species = np.full(max(self.evaluator.atomic_numbers) + 1, -1, dtype=np.int32)
+        self._species[self.evaluator.atomic_numbers] = np.arange(len(self.evaluator.atomic_numbers))
         self._nlist = neighbors.DeviceNeighborList() if neighbor_list == "device" else None
 
     def compute(self, positions, cell, atomic_numbers, pbc=(True, True, True)):
-        Z = [int(z) for z in atomic_numbers]
-        table = self.evaluator.atomic_numbers
-        try:
-            species = np.array([table.index(z) for z in Z], dtype=np.int32)
-        except ValueError as exc:
-            raise ValueError("an atom's element is not in the model") from exc
+        Z = np.asarray(atomic_numbers).astype(np.int64).reshape(-1)
+        species = self._species[Z] if len(Z) == 0 or (Z.min() >= 0 and Z.max() < len(self._species)) else np.array([-1])
+        if len(species) and species.min() < 0:
+            raise ValueError("an atom's element is not in the model")
         ev = self.evaluator
         n_atoms = len(Z)
         if self._nlist is not None:
-            E = self._nlist.build_host(positions, species, cell, self.cutoff, pbc)
-            p = self._nlist.ptr
-            ev.compute_device(n_atoms, p["node_types"], p["num_neigh"], p["neigh_indices"], p["neigh_types"], p["xyz"],
-                              p["r"], E)
-            ev.synchronize()
-            energies = ev.node_energies
-            if E:
-                forces, virial = ev.reduce_forces_device(n_atoms, p["neigh_indices"], virial=True)
-            else:
-                forces, virial = np.zeros((n_atoms, 3)), np.zeros(6)
+            self._nlist.build_host(positions, species, cell, self.cutoff, pbc)
+            energies, forces, virial = ev.evaluate_list(self._nlist)
         else:
             nl = neighbors.neighbor_list(positions, cell, self.cutoff, pbc)
             ea = neighbors.edge_arrays(nl, species)
@@ -78,10 +71,16 @@ class SymmetrixCalculator:
             energies = ev.node_energies
             forces, virial = ev.reduce_forces(n_atoms, nl["j"], virial=True)
         cell = np.asarray(cell, dtype=np.float64)
-        volume = abs(np.linalg.det(np.diag(cell) if cell.shape == (3,) else cell))
+        if cell.shape == (3,):
+            volume = abs(cell[0] * cell[1] * cell[2])
+        else:
+            volume = abs(cell[0, 0] * (cell[1, 1] * cell[2, 2] - cell[1, 2] * cell[2, 1])
+                         - cell[0, 1] * (cell[1, 0] * cell[2, 2] - cell[1, 2] * cell[2, 0])
+                         + cell[0, 2] * (cell[1, 0] * cell[2, 1] - cell[1, 1] * cell[2, 0]))
         # symmetrix_calc.py:102: stress = -(pair_forces^T xyz)/V in Voigt order xx,yy,zz,yz,xz,xy
         stress = -np.array([virial[0], virial[1], virial[2], virial[5], virial[4], virial[3]]) / volume
-        self.results = {"energy": float(energies.sum()), "free_energy": float(energies.sum()),
+        total = float(energies.sum())
+        self.results = {"energy": total, "free_energy": total,
                         "energies": energies, "forces": forces, "stress": stress}
         return self.results
 

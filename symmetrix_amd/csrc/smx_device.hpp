@@ -206,6 +206,57 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// very long buckets only: in place, by one lane
+__device__ inline void insertion_sort(int* v, int n)
+{
+    for (int a = 1; a < n; ++a) {
+        const int x = v[a];
+        int b = a - 1;
+        while (b >= 0 && v[b] > x) { v[b + 1] = v[b]; --b; }
+        v[b + 1] = x;
+    }
+}
+// how many of buf[0 .. n), padded with larger values to a multiple of four, are below v (four to a 16-byte LDS read)
+__device__ __forceinline__ int count_below(const int* buf, int n, int v)
+{
+    int rank = 0;
+    for (int b = 0; b < n; b += 4) {
+        const int4 w = *reinterpret_cast<const int4*>(buf + b);
+        rank += (w.x < v) + (w.y < v) + (w.z < v) + (w.w < v);
+    }
+    return rank;
+}
+// The n distinct entries list[s0 ..] in ascending order, for the wavefront that calls: in `buf` (LDS, CAP entries of this
+// wavefront, 16-byte aligned; the rank of an entry is the number of smaller ones), or, for a longer bucket, in place.
+template <int CAP>
+__device__ __forceinline__ const int* wave_sorted_bucket(int* list, int s0, int n, int* buf, int lane)
+{
+    static_assert(CAP % 64 == 0, "whole rounds of a wavefront");
+    if (n > CAP) {
+        if (lane == 0) insertion_sort(list + s0, n);
+        __threadfence();
+        return list + s0;
+    }
+    int v[CAP / 64];
+#pragma unroll
+    for (int q = 0; q < CAP / 64; ++q)
+        if (64 * q < n) {   // (whole rounds: the padding counts as larger than everything)
+            v[q] = 64 * q + lane < n ? list[s0 + 64 * q + lane] : 0x7fffffff;
+            buf[64 * q + lane] = v[q];
+        }
+    wave_lds_sync();
+    int rank[CAP / 64];
+#pragma unroll
+    for (int q = 0; q < CAP / 64; ++q)
+        if (64 * q < n) rank[q] = count_below(buf, n, v[q]);
+    wave_lds_sync();
+#pragma unroll
+    for (int q = 0; q < CAP / 64; ++q)
+        if (64 * q + lane < n) buf[rank[q]] = v[q];
+    wave_lds_sync();
+    return buf;
+}
+
 // CPL consecutive elements moved with one load or store
 template <typename F, int N>
 struct alignas(sizeof(F) * N) Vec {

@@ -97,6 +97,71 @@ struct DVec {
     }
 };
 
+// Growable pinned host array: copies between it and the device are asynchronous and go through no staging of the runtime's.
+// Whoever fills it again has waited for the last copy from or to it.
+template <typename T>
+struct HostBuf {
+    T* p = nullptr;
+    size_t cap = 0;
+    ~HostBuf() { if (p) (void)hipHostFree(p); }
+    HostBuf() = default;
+    HostBuf(const HostBuf&) = delete;
+    HostBuf& operator=(const HostBuf&) = delete;
+    T* room(size_t m)
+    {
+        if (m > cap) {
+            const size_t newcap = m + m / 8 + 64;
+            if (p) { HIPCHK(hipHostFree(p)); p = nullptr; cap = 0; }
+            HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&p), newcap * sizeof(T)));
+            cap = newcap;
+        }
+        return p;
+    }
+};
+// Host to device in pieces through a ring of pinned slots: the copy of one piece runs while the next is being filled.
+struct Uploader {
+    static constexpr size_t SLOT = (size_t)2 << 20;
+    static constexpr int SLOTS = 4;
+    HostBuf<char> ring;
+    hipEvent_t done[SLOTS] = {};
+    bool busy[SLOTS] = {};
+    int slot = 0;
+    size_t fill = 0;          // bytes of the current slot taken
+    ~Uploader() { for (auto& e : done) if (e) (void)hipEventDestroy(e); }
+    void put(char* dst, const void* src_, size_t n, hipStream_t s)
+    {
+        const char* src = static_cast<const char*>(src_);
+        ring.room(SLOT * SLOTS);
+        while (n > 0) {
+            if (fill == 0 && busy[slot]) { HIPCHK(hipEventSynchronize(done[slot])); busy[slot] = false; }
+            const size_t m = std::min(n, SLOT - fill);
+            char* at = ring.p + (size_t)slot * SLOT + fill;
+            std::memcpy(at, src, m);
+            HIPCHK(hipMemcpyAsync(dst, at, m, hipMemcpyHostToDevice, s));
+            dst += m; src += m; n -= m; fill += (m + 255) / 256 * 256;
+            if (fill >= SLOT) next(s);
+        }
+    }
+    // n bytes of an empty slot, to be filled and copied by the caller
+    char* take(size_t n)
+    {
+        ring.room(SLOT * SLOTS);
+        if (busy[slot]) { HIPCHK(hipEventSynchronize(done[slot])); busy[slot] = false; }
+        fill = n;
+        return ring.p + (size_t)slot * SLOT;
+    }
+    // the current slot is not written again before its copies are done
+    void next(hipStream_t s)
+    {
+        if (fill == 0) return;
+        if (!done[slot]) HIPCHK(hipEventCreateWithFlags(&done[slot], hipEventDisableTiming));
+        HIPCHK(hipEventRecord(done[slot], s));
+        busy[slot] = true;
+        slot = (slot + 1) % SLOTS;
+        fill = 0;
+    }
+};
+
 template <typename T, typename S>
 static void upload_as(DVec<T>& d, const std::vector<S>& h, hipStream_t s)
 {
@@ -141,7 +206,10 @@ struct EngineBase {
     virtual void set_array(const char* name, const double* in, long n) = 0;
     virtual void fill_array(const char* name, long n, double value) = 0;
     virtual void forces_view(ForcesView* v) = 0;
-    virtual void check_device_status() = 0;
+    virtual void check_device_status(bool on_device) = 0;   // the stream has been waited for
+    virtual void evaluate_list(int N, const int* node_types, const int* num_neigh, const int* neigh_indices,
+                               const int* neigh_types, const double* xyz, const double* r, long E, double* energies,
+                               double* forces, double* virial) = 0;
     virtual void reduce_forces(int num_atoms, const int* sender_atom, const int* receiver_atom,
                                double* atom_forces, double* virial, bool sender_on_device) = 0;
 
@@ -195,12 +263,17 @@ struct Engine : EngineBase {
 
     // ---- geometry of the current edge list (device)
     DVec<int> g_node_types, g_num_neigh, g_neigh_indices, g_neigh_types;
+    DVec<char> g_in;               // host arrays of a whole-pipeline call, one behind the other
+    Uploader uploader;
+    HostBuf<char> host_out;        // results on their way to the caller
+    HostBuf<int> sticky;           // failed input checks not yet reported: [0] device-resident calls, [1] host-array calls
     DVec<double> g_xyz, g_r;
     const int *node_types = nullptr, *num_neigh = nullptr, *neigh_indices = nullptr, *neigh_types = nullptr;
     const double *xyz = nullptr, *r = nullptr;
     long E = 0;
     long E1 = 0;   // leading edges whose receivers take part in layer 1 (all of them unless ghost nodes follow)
     int N_geo = 0;
+    long geo_edges = 0;   // edges of the N_geo receivers
     DVec<int> first_neigh, recv_order, scan_tmp, s_count, s_start, s_list, t_count, t_start, t_cursor, t_perm, flags;
     int sender_rows = 0;
     // pair terms: ZBL constants per species pair, density-normalisation splines, divisors of the last forward pass
@@ -227,7 +300,8 @@ struct Engine : EngineBase {
     double* forces_copy = nullptr;
     bool senders_counted = false;   // the sender histogram (and s_rank) was formed by the fused node-list launch
     DVec<int> s_rank;               // place of every edge inside its sender's bucket
-    long counters_clean = 0;        // leading entries of s_count known to be zero
+    long counters_clean = 0;        // leading entries of s_count known to be zero (every sender-list build leaves them so)
+    long rf_clean = 0;              // the same for rf_count
 
     // ---- state (mace.hpp members)
     DVec<F> Phi0, A0, A0_adj, M0, M0_grad, M0_adj, H1, H1_adj, Phi1, dPhi1, A1, A1_adj, M1, M1_grad, M1_adj, msg;
@@ -367,17 +441,19 @@ struct Engine : EngineBase {
         if (M1_tables) slabs(M1_slabs, &hm.P1, 1);
         poly_tables = (M0_tables ? 1 : 0) | (M1_tables ? 2 : 0);
         flags.resize(8, s);
+        sticky.room(2); sticky.p[0] = sticky.p[1] = 0;
         HIPCHK(hipStreamSynchronize(s));
     }
 
-    // ---- input checks of device-resident evaluations.  flags[0]: host-array calls (read back at once);
-    // flags[1]: sticky status of device-resident calls, read by the next synchronising call; flags[2]: the word the
-    // checks of the running device-resident evaluation raise; flags[3]: its copy for the kernels after the list
-    // preparation ("live": raised -> energies and forces are NaN).  The evaluation clears flags[2] again in its
+    // ---- input checks of an evaluation.  flags[0]: stage-level calls (read back at once); flags[2]: the word the checks
+    // of the running evaluation raise; flags[3]: its copy for the kernels after the list preparation ("live": raised ->
+    // energies and forces are NaN); flags[4]: ticket of the list preparation.  The evaluation clears flags[2] again in its
     // readout launch, after the last reader, so every evaluation, eager or a replayed graph, starts from a clean word.
-    long device_calls = 0;
-    int* guard_status = nullptr;   // check word of the running evaluation (nullptr: host-array call, checked already)
+    // sticky: what failed and has not been reported, in host memory, written by the list preparation and read by the next
+    // call that waits for the stream (a host-array call reports at its own end).
+    int* guard_status = nullptr;   // check word of the running evaluation
     bool guard_clear_enqueued = false;   // ... and a launch that clears it again is in the stream
+    bool guard_on_device = false;
     const int* guard_live() const { return guard_status ? flags.p + 3 : nullptr; }
     InputGuard input_guard(int N)
     {
@@ -385,25 +461,23 @@ struct Engine : EngineBase {
         if (!guard_status) return g;
         g.status = guard_status;
         g.live = flags.p + 3;
-        g.sticky = flags.p + 1;
+        g.sticky = sticky.p + (guard_on_device ? 0 : 1);
         g.first_neigh = first_neigh.p; g.n_first = N + 1;
         g.tstart = t_start.p; g.n_tstart = hm.T + 1;
         return g;
     }
-    void check_device_status() override
+    void check_device_status(bool on_device) override
     {
-        if (!device_calls) return;
-        int f = 0;
-        HIPCHK(hipMemcpyAsync(&f, flags.p + 1, sizeof(int), hipMemcpyDeviceToHost, stream));
-        HIPCHK(hipStreamSynchronize(stream));
+        volatile int* w = sticky.p + (on_device ? 0 : 1);
+        const int f = *w;
         if (!f) return;
-        HIPCHK(launch_fill<int>(flags.p + 1, 1, 0, stream));
+        *w = 0;
+        const std::string what = on_device ? "a device-resident evaluation was skipped: " : "";
+        const std::string then = on_device ? " (its node energies and forces are NaN)" : "";
         if (f & 1)
-            throw Error(SMX_EINVAL, "a device-resident evaluation was skipped: node_types / neigh_types / neigh_indices hold an "
-                                    "index outside the model or the node range, or num_neigh does not add up to the number "
-                                    "of edges (its node energies and forces are NaN)");
-        throw Error(SMX_ERANGE, "a device-resident evaluation was skipped: an edge length lies outside (0, r_cut) "
-                                "(its node energies and forces are NaN)");
+            throw Error(SMX_EINVAL, what + "node_types / neigh_types / neigh_indices hold an index outside the model or the node range" +
+                                    (on_device ? ", or num_neigh does not add up to the number of edges" : "") + then);
+        throw Error(SMX_ERANGE, what + "an edge length lies outside (0, r_cut): the radial spline tables do not cover it" + then);
     }
 
     // Regroup a radial table per channel slice, or return 0 when the slice path does not apply.
@@ -539,6 +613,32 @@ struct Engine : EngineBase {
         }
         if (E_ >= 0) { E = E_; E1 = E_; }
     }
+    // the host arrays of a whole-pipeline call
+    void upload_inputs(int N, const int* nt, const int* nn, const int* ni, const int* nty, const double* x, const double* rr, long E_)
+    {
+        auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+        const size_t n4 = up((size_t)N * 4), e4 = up((size_t)E_ * 4), e8 = up((size_t)E_ * 8), e24 = up((size_t)E_ * 24);
+        g_in.size_to(2 * n4 + 2 * e4 + e8 + e24, stream);
+        char* d = g_in.p;
+        const bool one = g_in.n <= Uploader::SLOT;   // small: the arrays laid out in one slot, one copy
+        char* h = one ? uploader.take(g_in.n) : nullptr;
+        auto put = [&](const void* src, size_t bytes, size_t room) {
+            char* at = d;
+            if (bytes && one) std::memcpy(h + (at - g_in.p), src, bytes);
+            else if (bytes) uploader.put(at, src, bytes, stream);
+            d += room;
+            return at;
+        };
+        node_types = reinterpret_cast<int*>(put(nt, (size_t)N * 4, n4));
+        num_neigh = reinterpret_cast<int*>(put(nn, (size_t)N * 4, n4));
+        neigh_indices = reinterpret_cast<int*>(put(ni, (size_t)E_ * 4, e4));
+        neigh_types = reinterpret_cast<int*>(put(nty, (size_t)E_ * 4, e4));
+        r = reinterpret_cast<double*>(put(rr, (size_t)E_ * 8, e8));
+        xyz = reinterpret_cast<double*>(put(x, (size_t)E_ * 24, e24));
+        if (one && g_in.n) HIPCHK(hipMemcpyAsync(g_in.p, h, g_in.n, hipMemcpyHostToDevice, stream));
+        uploader.next(stream);
+        E = E_; E1 = E_;
+    }
     void build_first_neigh(int N)
     {
         hipStream_t s = stream;
@@ -557,33 +657,25 @@ struct Engine : EngineBase {
         scan_tmp.size_to((size_t)std::max(N, T) / 1024 + 2, s);
         HIPCHK(launch_type_groups(node_types, N, T, t_count.p, t_start.p, t_cursor.p, t_perm.p, scan_tmp.p, s));
     }
+    // counters that a list build finds at zero
+    void clean_counters(DVec<int>& c, long rows, long& clean)
+    {
+        const int* before = c.p;
+        c.size_to((size_t)rows, stream);
+        if (c.p != before) clean = 0;
+        if (clean < rows) { HIPCHK(launch_fill<int>(c.p, rows, 0, stream)); clean = rows; }
+    }
     void build_sender_lists(int rows)
     {
         hipStream_t s = stream;
-        s_count.size_to((size_t)2 * rows, s); s_start.size_to((size_t)rows + 1, s);
-        s_list.size_to((size_t)E1, s);
+        if (!senders_counted) clean_counters(s_count, rows, counters_clean);
+        s_start.size_to((size_t)rows + 1, s);
+        s_list.size_to((size_t)E1, s); s_rank.size_to((size_t)E1, s);
         scan_tmp.size_to((size_t)rows / 1024 + 2, s);
-        HIPCHK(launch_sender_lists(neigh_indices, (int)E1, rows, s_count.p, s_start.p, s_count.p + rows, s_list.p, scan_tmp.p,
-                                   senders_counted ? 2 : 0, senders_counted ? s_rank.p : nullptr, s, input_guard(N_geo)));
+        HIPCHK(launch_sender_lists(neigh_indices, E1, rows, s_count.p, s_rank.p, s_start.p, s_list.p, scan_tmp.p,
+                                   senders_counted, nullptr, s, input_guard(N_geo)));
         senders_counted = false;
-        counters_clean = 2L * rows;   // every build leaves its counters and cursors at zero
         sender_rows = rows;
-    }
-    // Host-path validation of what the reference leaves unchecked (mace.cpp:17-64 trusts
-    // its caller; cubic_spline_set.cpp:54 reads past the table for r >= r_cut).
-    void validate(int N, int rows)
-    {
-        hipStream_t s = stream;
-        HIPCHK(hipMemsetAsync(flags.p, 0, sizeof(int), s));
-        HIPCHK(launch_check_range(node_types, N, hm.T, flags.p, s));
-        HIPCHK(launch_check_range(neigh_types, E, hm.T, flags.p, s));
-        HIPCHK(launch_check_range(neigh_indices, E1, rows, flags.p, s));
-        HIPCHK(launch_check_r(r, E, hm.r_cut, flags.p, s));
-        int f = 0;
-        HIPCHK(hipMemcpyAsync(&f, flags.p, sizeof(int), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        if (f & 1) throw Error(SMX_EINVAL, "node_types / neigh_types / neigh_indices hold an index outside the model or the node range");
-        if (f & 2) throw Error(SMX_ERANGE, "an edge length lies outside (0, r_cut): the radial spline tables do not cover it");
     }
     // stage-level calls: check whichever integer arrays this call brought
     void validate_stage_inputs(int N, bool have_nt, bool have_ni, bool have_nty, bool have_r)
@@ -947,7 +1039,7 @@ struct Engine : EngineBase {
                                                   M0_adj.p, stream));
             reverse_H1_done = true;
         } else {
-            HIPCHK(launch_sender_reduce<F>(rows, nlm * k, s_start.p, s_list.p, msg.p, H1_adj.p, zero_H1_adj ? 1 : 0, 0, E1, stream));
+            HIPCHK(launch_sender_reduce<F>(rows, nlm * k, s_start.p, s_list.p, msg.p, H1_adj.p, zero_H1_adj ? 1 : 0, false, 0, E1, stream));
         }
         stage_end(ST_SRED);
     }
@@ -987,6 +1079,7 @@ struct Engine : EngineBase {
         const int groups = agg_bwd_groups<F>(hm.L_max, k);
         if (groups > 1) fpart.size_to((size_t)groups * 3 * E, stream);
         if (sender_rows != rows) build_sender_lists(rows);
+        HIPCHK(launch_sort_buckets(s_start.p, rows, s_list.p, stream));   // the windows below need the order in memory
         stage_begin(ST_AGG1B);
         for (int c = 0; c < nchunks; ++c) {
             auto p = agg_params(1, bnd[c + 1]);
@@ -995,7 +1088,7 @@ struct Engine : EngineBase {
             p.fpart = groups > 1 ? fpart.p : nullptr;
             HIPCHK(launch_agg_bwd<F>(hm.L_max, p, stream));
             HIPCHK(launch_sender_reduce<F>(rows, nlm * k, s_start.p, s_list.p, msg.p, H1_adj.p,
-                                           (c == 0 && zero_H1_adj) ? 1 : 0, fe[c], fe[c + 1], stream));
+                                           (c == 0 && zero_H1_adj) ? 1 : 0, true, fe[c], fe[c + 1], stream));
         }
         stage_end(ST_AGG1B);
         stage_begin(ST_FSUM1);
@@ -1067,6 +1160,7 @@ struct Engine : EngineBase {
             carried_edges = 0; carry_forces = false; fuse_reverse_H1 = false;
             // checks of the failed call may have raised the word that only its readout launch would have cleared
             if (guard_status && !guard_clear_enqueued) (void)launch_fill<int>(guard_status, 1, 0, stream);
+            (void)launch_fill<int>(flags.p + 4, 1, 0, stream);
             guard_status = nullptr;
             throw;
         }
@@ -1095,43 +1189,37 @@ struct Engine : EngineBase {
             return;
         }
         stage_begin(ST_PREP);
-        set_geometry_ptrs(N, nt, nn, ni, nty, x, rr, E_, on_device);
+        if (on_device) set_geometry_ptrs(N, nt, nn, ni, nty, x, rr, E_, true);
+        else upload_inputs(N, nt, nn, ni, nty, x, rr, E_);
         if (N1 < N) E1 = E_local;
-        // range checks come before any kernel that uses these integers as indices: host arrays are checked with a
-        // read-back below; device arrays inside the list preparation, whose last launch empties the lists when a
-        // check failed (input_guard)
-        guard_status = nullptr; guard_clear_enqueued = false;
-        if (on_device) {
-            guard_status = flags.p + 2;
-            ++device_calls;
-        }
-        if (on_device && N <= 65536) {
-            // one launch for first_neigh, degree order, species groups and the sender histogram
+        geo_edges = E_;
+        // Range checks come before any kernel that uses these integers as indices: inside the list preparation, whose last
+        // launch empties the lists when a check failed (input_guard).  Host arrays are checked the same way and the result
+        // is looked at when the call waits for the stream anyway.
+        guard_status = flags.p + 2; guard_clear_enqueued = false; guard_on_device = on_device;
+        if (!on_device && (hm.A0_scaled || hm.A1_scaled)) HIPCHK(launch_fill<int>(flags.p, 1, 0, stream));
+        if (N <= 65536) {
+            // one launch for first_neigh, degree order, species groups, the sender histogram and the sender offsets
             hipStream_t s = stream;
             first_neigh.size_to((size_t)N + 1, s); recv_order.size_to((size_t)N, s);
             t_start.size_to((size_t)hm.T + 1, s); t_perm.size_to((size_t)N, s);
-            const int* before = s_count.p;
-            s_count.size_to((size_t)2 * N, s); s_start.size_to((size_t)N + 1, s);
-            scan_tmp.size_to((size_t)N / 1024 + 2, s);
-            if (s_count.p != before || counters_clean < 2L * N) HIPCHK(launch_fill<int>(s_count.p, 2L * N, 0, s));
+            clean_counters(s_count, N, counters_clean);
+            s_start.size_to((size_t)N + 1, s);
             s_rank.size_to((size_t)E1, s);
             InputChecks chk;
             chk.status = guard_status; chk.neigh_types = neigh_types; chk.r = r; chk.r_cut = hm.r_cut; chk.num_edges = E;
             chk.num_local_nodes = N1;
             HIPCHK(launch_node_lists_count(num_neigh, N, first_neigh.p, recv_order.p, node_types, hm.T, t_start.p, t_perm.p,
-                                           neigh_indices, E1, N, s_count.p, s_rank.p, chk, s));
+                                           neigh_indices, E1, N, s_count.p, s_rank.p, s_start.p, flags.p + 4, chk, s));
             N_geo = N;
             senders_counted = true;
         } else {
             build_first_neigh(N);
-            if (!on_device) validate(N, N);
-            else {
-                HIPCHK(launch_check_counts(num_neigh, N, first_neigh.p, N1, E, E1, guard_status, stream));
-                HIPCHK(launch_check_range(node_types, N, hm.T, guard_status, stream));
-                HIPCHK(launch_check_range(neigh_types, E, hm.T, guard_status, stream));
-                HIPCHK(launch_check_range(neigh_indices, E1, N, guard_status, stream));
-                HIPCHK(launch_check_r(r, E, hm.r_cut, guard_status, stream));
-            }
+            HIPCHK(launch_check_counts(num_neigh, N, first_neigh.p, N1, E, E1, guard_status, stream));
+            HIPCHK(launch_check_range(node_types, N, hm.T, guard_status, stream));
+            HIPCHK(launch_check_range(neigh_types, E, hm.T, guard_status, stream));
+            HIPCHK(launch_check_range(neigh_indices, E1, N, guard_status, stream));
+            HIPCHK(launch_check_r(r, E, hm.r_cut, guard_status, stream));
             build_type_groups(N);
         }
         sender_rows = -1;
@@ -1232,7 +1320,7 @@ struct Engine : EngineBase {
             if (own_edges > have) throw Error(SMX_EINVAL, "sum(num_neigh) exceeds the number of edges");
         }
         set_geometry_ptrs(N, nt, nn, ni, nty, x, rr, E_, false);
-        if (nn) { build_first_neigh(N); E1 = own_edges; }
+        if (nn) { build_first_neigh(N); E1 = own_edges; geo_edges = own_edges; }
         validate_stage_inputs(N, nt != nullptr, ni != nullptr, nty != nullptr, rr != nullptr);
         if (s == "Y" || s == "R0" || s == "R1") return;  // geometry remembered; evaluated inside the fused kernels
         if (s == "A0") { build_type_groups(N); st_agg0_fwd(N); st_A0_lin(N, false); }
@@ -1301,47 +1389,69 @@ struct Engine : EngineBase {
         if (n == "node_forces") return {nullptr, &node_forces};
         return {nullptr, nullptr};
     }
+    // entries of a named array as get_array would copy them
+    size_t array_length(const std::string& s)
+    {
+        if (s == "Y") return (size_t)E * 16;
+        if (s == "Y_grad") return (size_t)E * 48;
+        if (s == "R0") return (size_t)E * hm.nspl0;
+        if (s == "R1") return (size_t)E * hm.nspl1;
+        if (s == "M0_grad" && pending_M0_grad >= 0) return (size_t)pending_M0_grad * NLM() * 16 * K();
+        if (s == "A1_adj" && pending_A1_adj >= 0) return A1.n;
+        if (s == "A0_adj" && pending_A0_adj >= 0) return A0.n;
+        Named v = find(s);
+        if (!v.f && !v.d) throw Error(SMX_EINVAL, "unknown array '" + s + "'");
+        return v.d ? v.d->n : v.f->n;
+    }
     void get_array(const char* name, double* out, long cap, long* n) override
     {
         const std::string s(name);
         hipStream_t st = stream;
-        materialise_adjoints(s == "M0_grad");
+        const size_t len = array_length(s);
+        if (n) *n = (long)len;
+        if (s == "Y" || s == "Y_grad") need(xyz, "xyz (compute_Y)");
+        if (s == "R0" || s == "R1") { need(r, "r (compute_R0/R1)"); need(first_neigh.p, "num_neigh"); need(node_types, "node_types"); }
+        if (!out) return;
+        // (arrays the evaluation left unwritten are formed when they are asked for; the others do not wait for that)
+        if (s == "A1_adj" || s == "A0_adj" || s == "M0_grad") materialise_adjoints(s == "M0_grad");
         const double* src = nullptr;
-        size_t len = 0;
         if (s == "Y" || s == "Y_grad") {
-            need(xyz, "xyz (compute_Y)");
             scratch_d.size_to((size_t)E * 64, st);
             HIPCHK(launch_sph_harm(xyz, E, scratch_d.p, scratch_d.p + (size_t)E * 16, st));
             src = s == "Y" ? scratch_d.p : scratch_d.p + (size_t)E * 16;
-            len = s == "Y" ? (size_t)E * 16 : (size_t)E * 48;
         } else if (s == "R0" || s == "R1") {
-            need(r, "r (compute_R0/R1)"); need(first_neigh.p, "num_neigh"); need(node_types, "node_types");
             const bool l1 = s == "R1";
-            const int nspl = l1 ? hm.nspl1 : hm.nspl0;
-            scratch_d.size_to((size_t)E * nspl, st);
+            scratch_d.size_to(len, st);
             HIPCHK(launch_radial<F>(N_geo, first_neigh.p, node_types, neigh_types, r, l1 ? tab1.p : tab0.p,
-                                    l1 ? pair_table1.p : pair_table0.p, hm.T, hm.spl_nodes, hm.spl_h, nspl, scratch_d.p, st));
-            src = scratch_d.p; len = (size_t)E * nspl;
+                                    l1 ? pair_table1.p : pair_table0.p, hm.T, hm.spl_nodes, hm.spl_h, l1 ? hm.nspl1 : hm.nspl0,
+                                    scratch_d.p, st));
+            src = scratch_d.p;
         } else {
             Named v = find(s);
-            if (!v.f && !v.d) throw Error(SMX_EINVAL, "unknown array '" + s + "'");
-            if (v.d) { src = v.d->p; len = v.d->n; }
+            if (v.d) src = v.d->p;
+            else if (std::is_same<F, double>::value) src = reinterpret_cast<const double*>(v.f->p);
             else {
-                len = v.f->n;
-                if (std::is_same<F, double>::value) src = reinterpret_cast<const double*>(v.f->p);
-                else {
-                    scratch_d.size_to(len, st);
-                    HIPCHK((launch_convert<F, double>(v.f->p, scratch_d.p, (long)len, st)));
-                    src = scratch_d.p;
-                }
+                scratch_d.size_to(len, st);
+                HIPCHK((launch_convert<F, double>(v.f->p, scratch_d.p, (long)len, st)));
+                src = scratch_d.p;
             }
         }
-        if (n) *n = (long)len;
-        if (out && cap > 0 && len > 0) {
-            const size_t m = std::min((size_t)cap, len);
-            HIPCHK(hipMemcpyAsync(out, src, m * sizeof(double), hipMemcpyDeviceToHost, st));
+        if (cap > 0 && len > 0) download(out, src, std::min((size_t)cap, len) * sizeof(double));
+        else HIPCHK(hipStreamSynchronize(st));
+    }
+    // device to caller's memory, and the stream waited for: through pinned memory while that is small (the runtime's own
+    // staging of pageable memory costs 30 us a copy)
+    void download(void* out, const void* src, size_t bytes)
+    {
+        if (bytes > ((size_t)32 << 20)) {
+            HIPCHK(hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, stream));
+            HIPCHK(hipStreamSynchronize(stream));
+            return;
         }
-        HIPCHK(hipStreamSynchronize(st));
+        char* h = host_out.room(bytes);
+        HIPCHK(hipMemcpyAsync(h, src, bytes, hipMemcpyDeviceToHost, stream));
+        HIPCHK(hipStreamSynchronize(stream));
+        std::memcpy(out, h, bytes);
     }
     void set_array(const char* name, const double* in, long n) override
     {
@@ -1386,79 +1496,120 @@ struct Engine : EngineBase {
     }
 
     // ------------------------------------------------------------------
-    DVec<int> rf_send, rf_recv, rf_count, rf_sstart, rf_cursor, rf_slist, rf_rstart, rf_rlist;
-    DVec<double> rf_out;
+    DVec<int> rf_send, rf_nodes, rf_count, rf_rank, rf_sstart, rf_slist;
+    HostBuf<int> rf_nodes_host;
+    DVec<double> rf_out, rf_part;   // rf_out: [RF_HEAD: range flag, -, virial[6]][num_atoms][3]
+    static constexpr size_t RF_HEAD = 8;
+    double* reduction_room(int num_atoms)
+    {
+        const double* before = rf_out.p;
+        rf_out.size_to(RF_HEAD + (size_t)3 * num_atoms, stream);
+        if (rf_out.p != before) HIPCHK(launch_fill<double>(rf_out.p, RF_HEAD, 0.0, stream));
+        return rf_out.p;
+    }
     void reduce_forces(int num_atoms, const int* sender_atom, const int* receiver_atom, double* atom_forces,
                        double* virial, bool sender_on_device) override
     {
         hipStream_t s = stream;
         need(node_forces.p, "node_forces");
         if (node_forces.n != (size_t)3 * E) throw Error(SMX_EINVAL, "node_forces does not match the current edge list");
+        if (!atom_forces && !virial) return;
+        ForceGather g{};
+        g.num_nodes = N_geo; g.first_neigh = first_neigh.p; g.forces = node_forces.p; g.xyz = xyz;
+        int atoms = N_geo;
         if (atom_forces) {
+            atoms = num_atoms;
             if (num_atoms <= 0) throw Error(SMX_EINVAL, "num_atoms must be positive");
             if (!sender_atom) throw Error(SMX_EINVAL, "sender_atom is required");
-            const int* send = sender_atom;
-            if (!sender_on_device) { rf_send.upload(sender_atom, (size_t)E, s); send = rf_send.p; }
-            rf_count.size_to(num_atoms, s); rf_cursor.size_to(num_atoms, s);
-            rf_sstart.size_to((size_t)num_atoms + 1, s); rf_slist.size_to((size_t)E, s);
-            scan_tmp.size_to((size_t)num_atoms / 1024 + 2, s);
-            HIPCHK(hipMemsetAsync(flags.p, 0, sizeof(int), s));
-            HIPCHK(launch_check_range(send, E, num_atoms, flags.p, s));
-            {
-                int f = 0;
-                HIPCHK(hipMemcpyAsync(&f, flags.p, sizeof(int), hipMemcpyDeviceToHost, s));
-                HIPCHK(hipStreamSynchronize(s));
-                if (f) throw Error(SMX_EINVAL, "sender_atom out of range");
-            }
-            const int* rstart = nullptr;
-            const int* rlist = nullptr;
             if (receiver_atom) {
-                // receiver_atom[i] = atom row of receiver block i -> expand to edges
-                std::vector<int> hn(N_geo), hr((size_t)E);
-                HIPCHK(hipMemcpyAsync(hn.data(), num_neigh, (size_t)N_geo * sizeof(int), hipMemcpyDeviceToHost, s));
-                HIPCHK(hipStreamSynchronize(s));
-                size_t e = 0;
+                // receiver_atom[i] = atom row of receiver block i: the blocks of every atom, in ascending order
+                if (geo_edges != E) throw Error(SMX_EINVAL, "num_neigh of the last call does not cover every edge");
+                int* start = rf_nodes_host.room((size_t)num_atoms + 1 + N_geo);
+                int* list = start + num_atoms + 1;
+                std::fill(start, start + num_atoms + 1, 0);
                 for (int i = 0; i < N_geo; ++i) {
                     if (receiver_atom[i] < 0 || receiver_atom[i] >= num_atoms) throw Error(SMX_EINVAL, "receiver_atom out of range");
-                    if (hn[i] < 0 || e + (size_t)hn[i] > (size_t)E) throw Error(SMX_EINVAL, "num_neigh does not match the number of edges");
-                    for (int j = 0; j < hn[i]; ++j) hr[e++] = receiver_atom[i];
+                    ++start[receiver_atom[i]];
                 }
-                if (e != (size_t)E) throw Error(SMX_EINVAL, "num_neigh of the last call does not cover every edge");
-                rf_recv.upload(hr.data(), hr.size(), s);
-                HIPCHK(hipStreamSynchronize(s));
-                rf_rstart.size_to((size_t)num_atoms + 1, s); rf_rlist.size_to((size_t)E, s);
-                HIPCHK(launch_sender_lists(rf_recv.p, (int)E, num_atoms, rf_count.p, rf_rstart.p, rf_cursor.p, rf_rlist.p, scan_tmp.p, 0, nullptr, s));
-                rstart = rf_rstart.p; rlist = rf_rlist.p;
-            } else {
-                if (num_atoms < N_geo) throw Error(SMX_EINVAL, "num_atoms is smaller than the number of receivers");
-                // receiver block i is atom i: CSR offsets padded with E for atoms beyond the receivers
-                std::vector<int> h((size_t)num_atoms + 1);
-                HIPCHK(hipMemcpyAsync(h.data(), first_neigh.p, ((size_t)N_geo + 1) * sizeof(int), hipMemcpyDeviceToHost, s));
-                HIPCHK(hipStreamSynchronize(s));
-                for (int i = N_geo + 1; i <= num_atoms; ++i) h[i] = h[N_geo];
-                rf_rstart.upload(h.data(), h.size(), s);
-                HIPCHK(hipStreamSynchronize(s));
-                rstart = rf_rstart.p;
+                int acc = 0;
+                for (int a = 0; a <= num_atoms; ++a) { const int c = start[a]; start[a] = acc; acc += c; }
+                for (int i = 0; i < N_geo; ++i) list[start[receiver_atom[i]]++] = i;
+                for (int a = num_atoms; a > 0; --a) start[a] = start[a - 1];
+                start[0] = 0;
+                rf_nodes.upload(start, (size_t)num_atoms + 1 + N_geo, s);
+                g.node_start = rf_nodes.p; g.node_list = rf_nodes.p + num_atoms + 1;
+            } else if (num_atoms < N_geo) {
+                throw Error(SMX_EINVAL, "num_atoms is smaller than the number of receivers");
             }
-            HIPCHK(launch_sender_lists(send, (int)E, num_atoms, rf_count.p, rf_sstart.p, rf_cursor.p, rf_slist.p, scan_tmp.p, 0, nullptr, s));
-            rf_out.size_to((size_t)3 * num_atoms, s);
-            HIPCHK(launch_force_scatter(num_atoms, rstart, rlist, rf_sstart.p, rf_slist.p, node_forces.p, rf_out.p, s));
-            HIPCHK(hipMemcpyAsync(atom_forces, rf_out.p, (size_t)3 * num_atoms * sizeof(double), hipMemcpyDeviceToHost, s));
-            HIPCHK(hipStreamSynchronize(s));
+        } else if (receiver_atom && geo_edges != E) {
+            throw Error(SMX_EINVAL, "num_neigh of the last call does not cover every edge");
         }
-        if (virial) {
-            const int nb = 64;
-            scratch_d.size_to((size_t)nb * 6, s);
-            HIPCHK(launch_virial(E, xyz, node_forces.p, scratch_d.p, nb, s));
-            std::vector<double> part((size_t)nb * 6);
-            HIPCHK(hipMemcpyAsync(part.data(), scratch_d.p, part.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-            HIPCHK(hipStreamSynchronize(s));
-            for (int q = 0; q < 6; ++q) {
-                double v = 0;
-                for (int b = 0; b < nb; ++b) v += part[(size_t)b * 6 + q];
-                virial[q] = v;
+        double* out = reduction_room(atom_forces ? num_atoms : 0);
+        int* flag = reinterpret_cast<int*>(out);
+        if (atom_forces) {
+            const int* send = sender_atom;
+            if (!sender_on_device) {
+                rf_send.size_to((size_t)E, s);
+                uploader.put(reinterpret_cast<char*>(rf_send.p), sender_atom, (size_t)E * sizeof(int), s);
+                uploader.next(s);
+                send = rf_send.p;
             }
+            clean_counters(rf_count, num_atoms, rf_clean);
+            rf_rank.size_to((size_t)E, s);
+            rf_sstart.size_to((size_t)num_atoms + 1, s); rf_slist.size_to((size_t)E, s);
+            scan_tmp.size_to((size_t)num_atoms / 1024 + 2, s);
+            HIPCHK(launch_sender_lists(send, E, num_atoms, rf_count.p, rf_rank.p, rf_sstart.p, rf_slist.p, scan_tmp.p, false,
+                                       flag, s));
+            g.send_start = rf_sstart.p; g.send_list = rf_slist.p;
+            g.atom_forces = out + RF_HEAD;
         }
+        gather_forces(g, atoms, virial ? out + 2 : nullptr);
+        fetch_reduction(atom_forces, virial, num_atoms, 0, nullptr);
+    }
+    void gather_forces(ForceGather& g, int atoms, double* d_virial)
+    {
+        g.num_atoms = atoms;
+        if (d_virial) {
+            rf_part.size_to((size_t)6 * std::max(1, force_gather_blocks(atoms)), stream);
+            g.partial = rf_part.p;
+            if (atoms == 0) HIPCHK(launch_fill<double>(d_virial, 6, 0.0, stream));
+        }
+        HIPCHK(launch_force_gather(g, d_virial, stream));
+    }
+    // the sums in one copy, and whatever `more` doubles follow them
+    void fetch_reduction(double* atom_forces, double* virial, int num_atoms, size_t more, double* more_out)
+    {
+        const size_t nf = atom_forces ? (size_t)3 * num_atoms : 0, total = RF_HEAD + nf + more;
+        double* h = reinterpret_cast<double*>(host_out.room(total * sizeof(double)));
+        HIPCHK(hipMemcpyAsync(h, rf_out.p, total * sizeof(double), hipMemcpyDeviceToHost, stream));
+        HIPCHK(hipStreamSynchronize(stream));
+        if (*reinterpret_cast<const int*>(h)) {
+            HIPCHK(launch_fill<double>(rf_out.p, 1, 0.0, stream));
+            throw Error(SMX_EINVAL, "sender_atom out of range");
+        }
+        if (atom_forces) std::memcpy(atom_forces, h + RF_HEAD, nf * sizeof(double));
+        if (virial) std::memcpy(virial, h + 2, 6 * sizeof(double));
+        if (more) std::memcpy(more_out, h + RF_HEAD + nf, more * sizeof(double));
+    }
+    // Evaluation and reduction of one list on the device (receiver i and sender index are atoms) with the results in the
+    // caller's memory: the sender lists of the evaluation serve the reduction too, and everything comes back in one copy.
+    void evaluate_list(int N, const int* nt, const int* nn, const int* ni, const int* nty, const double* x, const double* rr,
+                       long E_, double* energies, double* forces, double* virial) override
+    {
+        double* out = nullptr;
+        {
+            const double* before = rf_out.p;
+            rf_out.size_to(RF_HEAD + (size_t)4 * N, stream);
+            out = rf_out.p;
+            if (out != before) HIPCHK(launch_fill<double>(out, RF_HEAD, 0.0, stream));
+        }
+        compute(N, nt, nn, ni, nty, x, rr, E_, true, out + RF_HEAD + (size_t)3 * N, nullptr, -1, -1);
+        ForceGather g{};
+        g.num_nodes = N; g.first_neigh = first_neigh.p; g.forces = node_forces.p; g.xyz = xyz;
+        g.send_start = s_start.p; g.send_list = s_list.p;
+        g.atom_forces = out + RF_HEAD;
+        gather_forces(g, N, out + 2);
+        fetch_reduction(forces, virial, N, (size_t)N, energies);
     }
 };
 
@@ -1506,6 +1657,9 @@ int guarded(Fn&& fn)
 
 void require_device()
 {
+    static thread_local int checked = -1;   // ordinal this thread has looked at already
+    int cur = -1;
+    if (checked >= 0 && hipGetDevice(&cur) == hipSuccess && cur == checked) return;
     int n = 0;
     hipError_t e = hipGetDeviceCount(&n);
     if (e != hipSuccess || n <= 0)
@@ -1516,6 +1670,7 @@ void require_device()
     if (hipGetDeviceProperties(&prop, dev) != hipSuccess) throw smx::Error(SMX_ENODEVICE, "hipGetDeviceProperties failed");
     if (std::string(prop.gcnArchName).rfind("gfx950", 0) != 0)
         throw smx::Error(SMX_ENODEVICE, std::string("kernels are built for gfx950 only; found ") + prop.gcnArchName);
+    checked = dev;
 }
 
 smx::EngineBase& E(smx_model* m)
@@ -1530,73 +1685,178 @@ smx::EngineBase& E(smx_model* m)
 // Device neighbour list (canonical order; see smx_kernels_nlist.hip)
 namespace smx {
 struct NeighborList {
-    DVec<double> part, shift_vec, xyz, r;
-    DVec<int> shift_int, atom_bin, bin_count, bin_start, bin_atoms, count, cfirst, first, num_neigh, neigh_indices,
+    DVec<double> part, xyz, r;
+    DVec<char> in_dev;        // [shift vectors][shift integers] and, for host inputs, [positions][species]
+    DVec<int> atom_bin, bin_count, bin_start, bin_atoms, count, cfirst, first, num_neigh, neigh_indices,
         neigh_types, neigh_shift, scan_tmp;
     DVec<long long> keys, sorted;
-    DVec<double> pos_dev;     // copies of host inputs (smx_nlist_build_host / smx_nlist_update_host)
-    DVec<int> types_dev;
+    HostBuf<char> in_host;    // the same on its way there; every call waits for the stream before it returns
+    HostBuf<int> totals;
+    const double* shift_vec = nullptr;
+    const int* shift_int = nullptr;
+    double* pos_dev = nullptr;     // copies of host inputs (smx_nlist_build_host / smx_nlist_update_host)
+    int* types_dev = nullptr;
+    int host_atoms = -1;           // number of them, -1: none
     int N = 0, num_shifts = 0;
     long E = 0, num_candidates = 0;
     double r_list = 0.0;
 
-    // candidates: every (receiver, sender, image) closer than r_list, sorted per receiver
-    void build(int N_, const double* d_pos, int num_shifts_, const int* h_shift_int, const double* h_shift_vec,
-               double r_list_, hipStream_t s)
+    // Lists of up to this many atoms try every atom as a sender: the three launches that bin the atoms take longer.
+    static constexpr int ALL_ATOMS = 512;
+
+    NlEdgeArrays edge_arrays(const int* d_types)
     {
-        if (N_ < 0 || num_shifts_ <= 0 || !(r_list_ > 0.0) || !h_shift_int || !h_shift_vec || (N_ > 0 && !d_pos))
+        NlEdgeArrays a;
+        a.types = d_types; a.shift_int = shift_int; a.first = first.p; a.num_neigh = num_neigh.p;
+        a.neigh_indices = neigh_indices.p; a.neigh_types = neigh_types.p; a.neigh_shift = neigh_shift.p; a.xyz = xyz.p; a.r = r.p;
+        return a;
+    }
+    void edge_room(size_t n, hipStream_t s)
+    {
+        neigh_indices.size_to(n, s); neigh_types.size_to(n, s); neigh_shift.size_to(3 * n, s);
+        xyz.size_to(3 * n, s); r.size_to(n, s);
+    }
+    long edge_capacity() const
+    {
+        return (long)std::min({neigh_indices.cap, neigh_types.cap, neigh_shift.cap / 3, xyz.cap / 3, r.cap});
+    }
+    static size_t up(size_t n) { return (n + 255) / 256 * 256; }
+    // shifts (and host inputs) to the device in one copy
+    void send_inputs(const double* h_pos, const int* h_types, const int* h_shift_int, const double* h_shift_vec, hipStream_t s)
+    {
+        const size_t bv = up((size_t)24 * num_shifts), bi = up((size_t)12 * num_shifts), bp = h_pos ? up((size_t)24 * N) : 0;
+        const size_t total = bv + bi + bp + (h_pos ? up((size_t)4 * N) : 0);
+        in_dev.size_to(total, s);
+        char* h = in_host.room(total);
+        std::memcpy(h, h_shift_vec, (size_t)24 * num_shifts);
+        std::memcpy(h + bv, h_shift_int, (size_t)12 * num_shifts);
+        if (h_pos && N > 0) {
+            std::memcpy(h + bv + bi, h_pos, (size_t)24 * N);
+            std::memcpy(h + bv + bi + bp, h_types, (size_t)4 * N);
+        }
+        HIPCHK(hipMemcpyAsync(in_dev.p, h, total, hipMemcpyHostToDevice, s));
+        shift_vec = reinterpret_cast<const double*>(in_dev.p);
+        shift_int = reinterpret_cast<const int*>(in_dev.p + bv);
+        pos_dev = h_pos ? reinterpret_cast<double*>(in_dev.p + bv + bi) : nullptr;
+        types_dev = h_pos ? reinterpret_cast<int*>(in_dev.p + bv + bi + bp) : nullptr;
+        host_atoms = h_pos ? N : -1;
+    }
+    void bounding_box(const double* d_pos, const double* h_pos, double* lo, double* hi, hipStream_t s)
+    {
+        for (int k = 0; k < 3; ++k) { lo[k] = 1e300; hi[k] = -1e300; }
+        if (h_pos) {
+            for (int i = 0; i < N; ++i)
+                for (int k = 0; k < 3; ++k) {
+                    const double v = h_pos[3 * (size_t)i + k];
+                    if (!(std::fabs(v) < 1e300)) throw Error(SMX_EINVAL, "neighbour list: positions are not finite");
+                    lo[k] = std::min(lo[k], v); hi[k] = std::max(hi[k], v);
+                }
+        } else {
+            // per-block partials, finished on the host
+            const int nblk = std::min(256, (N + 255) / 256);
+            part.size_to((size_t)nblk * 6, s);
+            HIPCHK(launch_nl_bbox(d_pos, N, part.p, nblk, s));
+            std::vector<double> hp((size_t)nblk * 6);
+            HIPCHK(hipMemcpyAsync(hp.data(), part.p, hp.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+            HIPCHK(hipStreamSynchronize(s));
+            for (int k = 0; k < 3; ++k)
+                for (int b = 0; b < nblk; ++b) { lo[k] = std::min(lo[k], hp[(size_t)b * 6 + k]); hi[k] = std::max(hi[k], hp[(size_t)b * 6 + 3 + k]); }
+        }
+        for (int k = 0; k < 3; ++k)
+            if (!(lo[k] <= hi[k]) || !(hi[k] - lo[k] < 1e300)) throw Error(SMX_EINVAL, "neighbour list: positions are not finite");
+    }
+
+    // Candidates: every (receiver, sender, image) closer than r_list, ordered per receiver.  Edges: those closer than r_cut.
+    // Everything is enqueued with the room that is there; the host waits once, for the totals, and where the room did not
+    // suffice it makes more and repeats the part that did not fit (kernels that lack room write nothing).
+    long build(int N_, const double* d_pos, const double* h_pos, const int* d_types, const int* h_types, int num_shifts_,
+               const int* h_shift_int, const double* h_shift_vec, double r_list_, double r_cut, hipStream_t s)
+    {
+        if (N_ < 0 || num_shifts_ <= 0 || !(r_list_ > 0.0) || !h_shift_int || !h_shift_vec || (N_ > 0 && !d_pos && !h_pos))
             throw Error(SMX_EINVAL, "neighbour list: bad arguments");
         int zero_shift = -1;
         for (int q = 0; q < num_shifts_; ++q)
             if (h_shift_int[3 * q] == 0 && h_shift_int[3 * q + 1] == 0 && h_shift_int[3 * q + 2] == 0) zero_shift = q;
         N = N_; num_shifts = num_shifts_; r_list = r_list_; E = 0; num_candidates = 0;
-        cfirst.size_to((size_t)N + 1, s);
-        if (N == 0) return;
-        shift_int.upload(h_shift_int, (size_t)3 * num_shifts, s);
-        shift_vec.upload(h_shift_vec, (size_t)3 * num_shifts, s);
-        // bounding box (per-block partials, finished on the host)
-        const int nblk = std::min(256, (N + 255) / 256);
-        part.size_to((size_t)nblk * 6, s);
-        HIPCHK(launch_nl_bbox(d_pos, N, part.p, nblk, s));
-        std::vector<double> hp((size_t)nblk * 6);
-        HIPCHK(hipMemcpyAsync(hp.data(), part.p, hp.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        NlGrid g{};
-        long nbins = 1;
-        for (int k = 0; k < 3; ++k) {
-            double lo = 1e300, hi = -1e300;
-            for (int b = 0; b < nblk; ++b) { lo = std::min(lo, hp[(size_t)b * 6 + k]); hi = std::max(hi, hp[(size_t)b * 6 + 3 + k]); }
-            if (!(lo <= hi) || !(hi - lo < 1e300)) throw Error(SMX_EINVAL, "neighbour list: positions are not finite");
-            g.lo[k] = lo; g.hi[k] = hi;
-            const double ext = hi - lo;
-            int nb = (int)std::floor(std::min(ext / r_list, 1e6));
-            nb = std::max(1, std::min(nb, 128));
-            g.nb[k] = nb;
-            g.inv_bs[k] = ext > 0.0 ? nb / ext : 0.0;
-            nbins *= nb;
+        cfirst.size_to((size_t)N + 1, s); first.size_to((size_t)N + 1, s); num_neigh.size_to((size_t)N, s);
+        totals.room(2);
+        send_inputs(h_pos, h_types, h_shift_int, h_shift_vec, s);
+        if (h_pos) { d_pos = pos_dev; d_types = types_dev; }
+        if (N == 0) {
+            edge_room(0, s);
+            HIPCHK(hipMemsetAsync(first.p, 0, sizeof(int), s));
+            HIPCHK(hipStreamSynchronize(s));
+            return 0;
         }
-        atom_bin.size_to((size_t)N, s); bin_count.size_to((size_t)2 * nbins, s); bin_start.size_to((size_t)nbins + 1, s);
-        bin_atoms.size_to((size_t)N, s); scan_tmp.size_to((size_t)std::max<long>(nbins, N) / 1024 + 2, s);
-        HIPCHK(hipMemsetAsync(bin_count.p, 0, (size_t)2 * nbins * sizeof(int), s));
-        HIPCHK(launch_nl_bins(d_pos, N, g, atom_bin.p, bin_count.p, s));
-        HIPCHK(launch_scan_exclusive(bin_count.p, bin_start.p, (int)nbins, scan_tmp.p, s));
-        HIPCHK(launch_nl_bin_fill(N, atom_bin.p, bin_start.p, bin_count.p + nbins, bin_atoms.p, s));
+        NlGrid g{};
+        bounding_box(d_pos, h_pos, g.lo, g.hi, s);
+        const bool all = N <= ALL_ATOMS;
+        scan_tmp.size_to((size_t)N / 1024 + 2, s);
+        if (!all) {
+            long nbins = 1;
+            for (int k = 0; k < 3; ++k) {
+                const double ext = g.hi[k] - g.lo[k];
+                int nb = (int)std::floor(std::min(ext / r_list, 1e6));
+                nb = std::max(1, std::min(nb, 128));
+                g.nb[k] = nb;
+                g.inv_bs[k] = ext > 0.0 ? nb / ext : 0.0;
+                nbins *= nb;
+            }
+            atom_bin.size_to((size_t)N, s); bin_count.size_to((size_t)2 * nbins, s); bin_start.size_to((size_t)nbins + 1, s);
+            bin_atoms.size_to((size_t)N, s); scan_tmp.size_to((size_t)std::max<long>(nbins, N) / 1024 + 2, s);
+            HIPCHK(launch_fill<int>(bin_count.p, 2 * nbins, 0, s));
+            HIPCHK(launch_nl_bins(d_pos, N, g, atom_bin.p, bin_count.p, s));
+            HIPCHK(launch_scan_exclusive(bin_count.p, bin_start.p, (int)nbins, scan_tmp.p, s));
+            HIPCHK(launch_nl_bin_fill(N, atom_bin.p, bin_start.p, bin_count.p + nbins, bin_atoms.p, s));
+        }
+        const int* bs = all ? nullptr : bin_start.p;
+        const int* ba = all ? nullptr : bin_atoms.p;
         count.size_to((size_t)N, s);
-        HIPCHK(launch_nl_search(false, d_pos, N, g, bin_start.p, bin_atoms.p, num_shifts, shift_vec.p, zero_shift, r_list,
-                                count.p, nullptr, nullptr, s));
+        HIPCHK(launch_nl_search(false, d_pos, N, g, bs, ba, num_shifts, shift_vec, zero_shift, r_list, count.p, nullptr, 0,
+                                nullptr, nullptr, nullptr, s));
         HIPCHK(launch_scan_exclusive(count.p, cfirst.p, N, scan_tmp.p, s));
-        int total = 0;
-        HIPCHK(hipMemcpyAsync(&total, cfirst.p + N, sizeof(int), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        if (total < 0) throw Error(SMX_EINVAL, "neighbour list: more than 2^31 candidate pairs");
-        num_candidates = total;
-        keys.size_to((size_t)num_candidates, s); sorted.size_to((size_t)num_candidates, s);
-        HIPCHK(launch_nl_search(true, d_pos, N, g, bin_start.p, bin_atoms.p, num_shifts, shift_vec.p, zero_shift, r_list,
-                                nullptr, cfirst.p, keys.p, s));
-        HIPCHK(launch_nl_sort(N, cfirst.p, keys.p, sorted.p, s));
+        const bool direct = r_list == r_cut;   // no skin: the candidates are the edges
+        if (sorted.cap == 0) { keys.size_to((size_t)64 * N, s); sorted.size_to((size_t)64 * N, s); }
+        if (edge_capacity() == 0) edge_room((size_t)64 * N, s);
+        for (;;) {
+            const long room = (long)std::min(keys.cap, sorted.cap);
+            const NlEdgeArrays edges = edge_arrays(d_types);
+            HIPCHK(launch_nl_search(true, d_pos, N, g, bs, ba, num_shifts, shift_vec, zero_shift, r_list, nullptr, cfirst.p,
+                                    direct ? std::min(room, edge_capacity()) : room, keys.p, sorted.p, direct ? &edges : nullptr, s));
+            HIPCHK(hipMemcpyAsync(totals.p, cfirst.p + N, sizeof(int), hipMemcpyDeviceToHost, s));
+            if (!direct) E = filter(d_pos, d_types, r_cut, room, s);   // waits for the stream
+            else HIPCHK(hipStreamSynchronize(s));
+            const long total = totals.p[0];
+            if (total < 0) throw Error(SMX_EINVAL, "neighbour list: more than 2^31 candidate pairs");
+            num_candidates = total;
+            if (direct) E = total;
+            if (total <= room && (!direct || total <= edge_capacity())) break;
+            keys.size_to((size_t)total, s); sorted.size_to((size_t)total, s);
+            if (direct) edge_room((size_t)total, s);
+        }
+        edge_room((size_t)E, s);
+        return E;
     }
 
-    // edges: the candidates closer than r_cut at the given positions, in candidate order
+    // edges: the candidates closer than r_cut at the given positions, in candidate order (`room`: what the candidate arrays
+    // hold; a list that does not fit has not been written and is not read)
+    long filter(const double* d_pos, const int* d_types, double r_cut, long room, hipStream_t s)
+    {
+        totals.room(2);
+        if (edge_capacity() == 0) edge_room((size_t)64 * N, s);
+        HIPCHK(launch_nl_filter(false, d_pos, N, cfirst.p, sorted.p, room, num_shifts, shift_vec, r_cut, num_neigh.p, nullptr, 0, nullptr, s));
+        HIPCHK(launch_scan_exclusive(num_neigh.p, first.p, N, scan_tmp.p, s));
+        for (;;) {
+            const long cap = edge_capacity();
+            const NlEdgeArrays edges = edge_arrays(d_types);
+            HIPCHK(launch_nl_filter(true, d_pos, N, cfirst.p, sorted.p, room, num_shifts, shift_vec, r_cut, nullptr, first.p, cap, &edges, s));
+            HIPCHK(hipMemcpyAsync(totals.p + 1, first.p + N, sizeof(int), hipMemcpyDeviceToHost, s));
+            HIPCHK(hipStreamSynchronize(s));
+            const long total = totals.p[1];
+            if (total <= cap) return total;
+            edge_room((size_t)total, s);
+        }
+    }
     long update(const double* d_pos, const int* d_types, double r_cut, hipStream_t s)
     {
         if (!(r_cut > 0.0) || r_cut > r_list || (N > 0 && !d_pos))
@@ -1607,18 +1867,38 @@ struct NeighborList {
             HIPCHK(hipMemsetAsync(first.p, 0, sizeof(int), s));
             return 0;
         }
-        HIPCHK(launch_nl_filter(false, d_pos, d_types, N, cfirst.p, sorted.p, num_shifts, shift_vec.p, shift_int.p, r_cut,
-                                num_neigh.p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, s));
-        HIPCHK(launch_scan_exclusive(num_neigh.p, first.p, N, scan_tmp.p, s));
-        int total = 0;
-        HIPCHK(hipMemcpyAsync(&total, first.p + N, sizeof(int), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        E = total;
-        neigh_indices.size_to((size_t)E, s); neigh_types.size_to((size_t)E, s); neigh_shift.size_to((size_t)3 * E, s);
-        xyz.size_to((size_t)3 * E, s); r.size_to((size_t)E, s);
-        HIPCHK(launch_nl_filter(true, d_pos, d_types, N, cfirst.p, sorted.p, num_shifts, shift_vec.p, shift_int.p, r_cut,
-                                nullptr, first.p, neigh_indices.p, neigh_types.p, neigh_shift.p, xyz.p, r.p, s));
+        E = filter(d_pos, d_types, r_cut, num_candidates, s);
+        edge_room((size_t)E, s);
         return E;
+    }
+    // positions of an orthorhombic cell folded into it along the periodic axes (in place) with the lattice offsets taken
+    // off, and the image shifts that cover r_list: the arithmetic of wrap_positions / image_shifts of
+    // symmetrix_amd/neighbors.py for such cells, operation by operation.  Returns whether an offset is not zero.
+    static bool fold_box(int N, const double* pos, const double* cell, const int* pbc, double* folded, long long* off)
+    {
+        bool any = false;
+        const double inv[3] = {1.0 / cell[0], 1.0 / cell[1], 1.0 / cell[2]};
+        for (long i = 0; i < 3L * N; ++i) {
+            const int k = (int)(i % 3);
+            const double f = pos[i] * inv[k];
+            if (!std::isfinite(f)) throw Error(SMX_EINVAL, "positions are not finite");
+            const double o = pbc[k] ? std::floor(f) : 0.0;
+            off[i] = (long long)o;
+            any = any || o != 0.0;
+            folded[i] = pos[i] - o * cell[k];
+        }
+        return any;
+    }
+    static void box_shifts(const double* cell, const int* pbc, double r_list, std::vector<int>& si, std::vector<double>& sv)
+    {
+        int n[3];
+        for (int k = 0; k < 3; ++k) n[k] = pbc[k] ? (int)std::ceil(r_list / cell[k]) : 0;
+        for (int a = -n[0]; a <= n[0]; ++a)
+            for (int b = -n[1]; b <= n[1]; ++b)
+                for (int c = -n[2]; c <= n[2]; ++c) {
+                    si.insert(si.end(), {a, b, c});
+                    sv.insert(sv.end(), {a * cell[0], b * cell[1], c * cell[2]});
+                }
     }
 };
 }  // namespace smx
@@ -1718,6 +1998,7 @@ int smx_compute_node_energies_forces(smx_model* m, int num_nodes, const int* nod
         e.stream = nullptr;
         e.compute(num_nodes, node_types, num_neigh, neigh_indices, neigh_types, xyz, r, num_edges, false, nullptr, nullptr, -1, -1);
         HIPCHK(hipStreamSynchronize(e.stream));
+        e.check_device_status(false);
     });
 }
 
@@ -1749,6 +2030,7 @@ int smx_compute_ghosted(smx_model* m, int num_local_nodes, int num_ghost_nodes, 
         e.compute(n, node_types, num_neigh, neigh_indices, neigh_types, xyz, r, num_edges, false, nullptr, nullptr,
                   num_local_nodes, -1);
         HIPCHK(hipStreamSynchronize(e.stream));
+        e.check_device_status(false);
     });
 }
 
@@ -1888,8 +2170,8 @@ int smx_get_array(smx_model* m, const char* name, double* out, long cap, long* n
 {
     return guarded([&] {
         if (!name) throw smx::Error(SMX_EINVAL, "null name");
-        E(m).check_device_status();
         E(m).get_array(name, out, cap, n);
+        if (out) E(m).check_device_status(true);
     });
 }
 int smx_set_array(smx_model* m, const char* name, const double* in, long n)
@@ -1943,7 +2225,7 @@ int smx_synchronize(smx_model* m)
     return guarded([&] {
         auto& e = E(m);
         HIPCHK(hipStreamSynchronize(e.stream));
-        e.check_device_status();
+        e.check_device_status(true);
     });
 }
 int smx_reduce_forces(smx_model* m, int num_atoms, const int* sender_atom, const int* receiver_atom,
@@ -1951,14 +2233,29 @@ int smx_reduce_forces(smx_model* m, int num_atoms, const int* sender_atom, const
 {
     return guarded([&] {
         E(m).reduce_forces(num_atoms, sender_atom, receiver_atom, atom_forces, virial, false);
-        E(m).check_device_status();   // forces of a skipped device-resident evaluation are NaN: say why
+        E(m).check_device_status(true);   // forces of a skipped device-resident evaluation are NaN: say why
     });
 }
 int smx_reduce_forces_device(smx_model* m, int num_atoms, const int* d_sender_atom, double* atom_forces, double* virial)
 {
     return guarded([&] {
         E(m).reduce_forces(num_atoms, d_sender_atom, nullptr, atom_forces, virial, true);
-        E(m).check_device_status();
+        E(m).check_device_status(true);
+    });
+}
+
+int smx_evaluate_list(smx_model* m, smx_nlist* nl, double* energies, double* atom_forces, double* virial)
+{
+    return guarded([&] {
+        auto& e = E(m);
+        if (!nl || !energies || !atom_forces || !virial) throw smx::Error(SMX_EINVAL, "null argument");
+        auto& n = *reinterpret_cast<smx::NeighborList*>(nl);
+        if (n.host_atoms != n.N) throw smx::Error(SMX_EINVAL, "smx_evaluate_list needs a list built from host positions");
+        e.stream = nullptr;
+        if (n.N == 0) { for (int q = 0; q < 6; ++q) virial[q] = 0.0; return; }
+        e.evaluate_list(n.N, n.types_dev, n.num_neigh.p, n.neigh_indices.p, n.neigh_types.p, n.xyz.p, n.r.p, n.E, energies,
+                        atom_forces, virial);
+        e.check_device_status(true);
     });
 }
 
@@ -1976,9 +2273,8 @@ int smx_nlist_build(smx_nlist* nl, int num_atoms, const double* d_positions, con
     return guarded([&] {
         if (!nl || !shift_int || !shift_vec || (num_atoms > 0 && !d_positions)) throw smx::Error(SMX_EINVAL, "null argument");
         if (!(r_cut > 0.0) || r_cut > r_list) throw smx::Error(SMX_EINVAL, "neighbour list: need 0 < r_cut <= r_list");
-        auto& n = *reinterpret_cast<smx::NeighborList*>(nl);
-        n.build(num_atoms, d_positions, num_shifts, shift_int, shift_vec, r_list, (hipStream_t)stream);
-        const long e = n.update(d_positions, d_types, r_cut, (hipStream_t)stream);
+        const long e = reinterpret_cast<smx::NeighborList*>(nl)->build(num_atoms, d_positions, nullptr, d_types, nullptr,
+            num_shifts, shift_int, shift_vec, r_list, r_cut, (hipStream_t)stream);
         if (num_edges) *num_edges = e;
     });
 }
@@ -1999,12 +2295,28 @@ int smx_nlist_build_host(smx_nlist* nl, int num_atoms, const double* positions, 
             throw smx::Error(SMX_EINVAL, "null argument");
         if (!(r_cut > 0.0) || r_cut > r_list) throw smx::Error(SMX_EINVAL, "neighbour list: need 0 < r_cut <= r_list");
         require_device();
-        auto& n = *reinterpret_cast<smx::NeighborList*>(nl);
-        n.pos_dev.upload(positions, (size_t)3 * num_atoms, nullptr);
-        n.types_dev.upload(types, (size_t)num_atoms, nullptr);
-        n.build(num_atoms, n.pos_dev.p, num_shifts, shift_int, shift_vec, r_list, nullptr);
-        const long e = n.update(n.pos_dev.p, n.types_dev.p, r_cut, nullptr);
-        HIPCHK(hipStreamSynchronize(nullptr));
+        const long e = reinterpret_cast<smx::NeighborList*>(nl)->build(num_atoms, nullptr, positions ? positions : shift_vec,
+            nullptr, types, num_shifts, shift_int, shift_vec, r_list, r_cut, nullptr);
+        if (num_edges) *num_edges = e;
+    });
+}
+int smx_nlist_build_box(smx_nlist* nl, int num_atoms, const double* positions, const int* types, const double* cell,
+                        const int* pbc, double r_list, double r_cut, long long* offsets, int* folded, long* num_edges)
+{
+    return guarded([&] {
+        if (!nl || !cell || !pbc || !offsets || num_atoms < 0 || (num_atoms > 0 && (!positions || !types)))
+            throw smx::Error(SMX_EINVAL, "null argument");
+        if (!(r_cut > 0.0) || r_cut > r_list) throw smx::Error(SMX_EINVAL, "neighbour list: need 0 < r_cut <= r_list");
+        for (int k = 0; k < 3; ++k)
+            if (!(cell[k] > 0.0) || !std::isfinite(cell[k])) throw smx::Error(SMX_EINVAL, "neighbour list: cell lengths must be positive");
+        require_device();
+        std::vector<double> pos((size_t)3 * num_atoms + 3), sv;
+        std::vector<int> si;
+        const bool any = smx::NeighborList::fold_box(num_atoms, positions, cell, pbc, pos.data(), offsets);
+        smx::NeighborList::box_shifts(cell, pbc, r_list, si, sv);
+        const long e = reinterpret_cast<smx::NeighborList*>(nl)->build(num_atoms, nullptr, pos.data(), nullptr, types,
+            (int)(si.size() / 3), si.data(), sv.data(), r_list, r_cut, nullptr);
+        if (folded) *folded = any ? 1 : 0;
         if (num_edges) *num_edges = e;
     });
 }
@@ -2013,10 +2325,14 @@ int smx_nlist_update_host(smx_nlist* nl, const double* positions, double r_cut, 
     return guarded([&] {
         if (!nl) throw smx::Error(SMX_EINVAL, "null argument");
         auto& n = *reinterpret_cast<smx::NeighborList*>(nl);
-        if (n.types_dev.n != (size_t)n.N || (n.N > 0 && !positions))
+        if (n.host_atoms != n.N || (n.N > 0 && !positions))
             throw smx::Error(SMX_EINVAL, "neighbour list: update from host positions needs a build from host positions first");
-        n.pos_dev.upload(positions, (size_t)3 * n.N, nullptr);
-        const long e = n.update(n.pos_dev.p, n.types_dev.p, r_cut, nullptr);
+        if (n.N > 0) {
+            char* h = n.in_host.room((size_t)24 * n.N);
+            std::memcpy(h, positions, (size_t)24 * n.N);
+            HIPCHK(hipMemcpyAsync(n.pos_dev, h, (size_t)24 * n.N, hipMemcpyHostToDevice, nullptr));
+        }
+        const long e = n.update(n.pos_dev, n.types_dev, r_cut, nullptr);
         HIPCHK(hipStreamSynchronize(nullptr));
         if (num_edges) *num_edges = e;
     });
@@ -2026,8 +2342,8 @@ int smx_nlist_inputs(smx_nlist* nl, const double** d_positions, const int** d_ty
     return guarded([&] {
         if (!nl) throw smx::Error(SMX_EINVAL, "null argument");
         auto& n = *reinterpret_cast<smx::NeighborList*>(nl);
-        if (d_positions) *d_positions = n.pos_dev.p;
-        if (d_types) *d_types = n.types_dev.p;
+        if (d_positions) *d_positions = n.pos_dev;
+        if (d_types) *d_types = n.types_dev;
     });
 }
 int smx_nlist_arrays(smx_nlist* nl, const int** num_neigh, const int** first_neigh, const int** neigh_indices,

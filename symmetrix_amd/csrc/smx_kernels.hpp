@@ -93,16 +93,16 @@ template <typename F> hipError_t launch_slice_bwd(const SliceParams<F>& p, hipSt
 hipError_t launch_fpart_reduce(long edges, long E, int nslices, const double* fpart, double* forces, int accumulate,
                                double* copy, hipStream_t s, const int* guard = nullptr);
 
-// H1_adj[j] (+)= sum over edges with sender j of msg[e], in ascending edge order.
-// H_adj[j] (+)= sum of msg[e - e_lo] over the edges e of sender j with e_lo <= e < e_hi, in ascending edge order
+// H_adj[j] (+)= sum of msg[e - e_lo] over the edges e of sender j, in ascending edge order; window: over those with
+// e_lo <= e < e_hi, and slist is in ascending order already (launch_sort_buckets)
 template <typename F>
-hipError_t launch_sender_reduce(int rows, int width, const int* sstart, const int* slist, const F* msg, F* H_adj,
-                                int zero_first, long e_lo, long e_hi, hipStream_t s);
+hipError_t launch_sender_reduce(int rows, int width, const int* sstart, int* slist, const F* msg, F* H_adj,
+                                int zero_first, bool window, long e_lo, long e_hi, hipStream_t s);
 // The same sum for rows of K scalar features, followed by M_adj[rows][K] = H_adj . W^T (W [K][K], row n holding
 // the weights of input channel n: reverse_H1 of an L_max = 0 model) in the same launch; K as sender_reduce_linear_ok
 bool sender_reduce_linear_ok(int K);
 template <typename F>
-hipError_t launch_sender_reduce_linear(int rows, int K, const int* sstart, const int* slist, const F* msg, F* H_adj,
+hipError_t launch_sender_reduce_linear(int rows, int K, const int* sstart, int* slist, const F* msg, F* H_adj,
                                        int zero_first, const F* W, F* M_adj, hipStream_t s);
 
 // ---------------------------------------------------------------------------
@@ -116,14 +116,28 @@ hipError_t launch_nl_bbox(const double* pos, int N, double* part, int nblocks, h
 hipError_t launch_nl_bins(const double* pos, int N, const NlGrid& g, int* atom_bin, int* bin_count, hipStream_t s);
 hipError_t launch_nl_bin_fill(int N, const int* atom_bin, const int* bin_start, int* bin_cursor, int* bin_atoms,
                               hipStream_t s);
+// edge arrays that the list kernels fill; first and num_neigh are written by a search that emits edges
+struct NlEdgeArrays {
+    const int* types;          // species of the atoms, or null
+    const int* shift_int;      // [num_shifts][3]
+    int* first;
+    int* num_neigh;
+    int* neigh_indices;
+    int* neigh_types;
+    int* neigh_shift;
+    double* xyz;
+    double* r;
+};
+// bin_start == nullptr: every atom is tried, no bins.  fill: the ordered keys go to `sorted` (keys: scratch of the same
+// size), and with `edges` every candidate is written as an edge.  Nothing is written where first[N] > capacity.
 hipError_t launch_nl_search(bool fill, const double* pos, int N, const NlGrid& g, const int* bin_start,
                             const int* bin_atoms, int num_shifts, const double* shift_vec, int zero_shift,
-                            double r_cut, int* count, const int* first, long long* keys, hipStream_t s);
-hipError_t launch_nl_sort(int N, const int* cfirst, const long long* keys, long long* sorted, hipStream_t s);
-hipError_t launch_nl_filter(bool emit, const double* pos, const int* types, int N, const int* cfirst,
-                            const long long* sorted, int num_shifts, const double* shift_vec, const int* shift_int,
-                            double r_cut, int* count, const int* first, int* neigh_indices, int* neigh_types,
-                            int* neigh_shift, double* xyz, double* r, hipStream_t s);
+                            double r_cut, int* count, const int* first, long capacity, long long* keys, long long* sorted,
+                            const NlEdgeArrays* edges, hipStream_t s);
+// `room`: keys that `sorted` holds; with more candidates than that there are none in it, and no edges
+hipError_t launch_nl_filter(bool emit, const double* pos, int N, const int* cfirst, const long long* sorted, long room, int num_shifts,
+                            const double* shift_vec, double r_cut, int* count, const int* first, long capacity,
+                            const NlEdgeArrays* edges, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Pair terms of the edge length alone (smx_kernels_pair.hip)
@@ -158,11 +172,8 @@ hipError_t launch_scale_bwd(int N, const int* first_neigh, const int* node_types
 hipError_t launch_scan_exclusive(const int* in, int* out, int n, int* block_sums, hipStream_t s);  // out[n] = total
 // order[N]: receivers by decreasing degree
 hipError_t launch_degree_order(int N, const int* first_neigh, int* order, hipStream_t s);
-// counters_are_zero: 0 = clear count and cursor first, 1 = they are zero, 2 = the histogram is already in count and
-// rank[E] holds every entry's place inside its bucket (launch_node_lists_count);
-// count and cursor are zero again when the launches have run
-// Guard of a device-resident evaluation, carried by the last launch of the sender-list build: when the checks of
-// this evaluation raised the status word, first_neigh[n_first] and tstart[n_tstart] are zeroed (no edges, no species
+// Guard of an evaluation, carried by the last launch of the sender-list build: when the checks of this evaluation
+// raised the status word, first_neigh[n_first], tstart[n_tstart] and the sender offsets are zeroed (no edges, no species
 // groups: the kernels that follow then touch no unchecked index) and the status is ORed into the sticky word the
 // host reads later.  Raised or not, the status is copied into the `live` word, which the kernels after this launch
 // read (energies and forces become NaN); the status word itself is cleared again by the readout kernel of the same
@@ -185,20 +196,22 @@ struct InputChecks {
     long num_edges = 0;
     int num_local_nodes = 0;
 };
-hipError_t launch_sender_lists(const int* gather, int E, int rows, int* count, int* sstart, int* cursor,
-                               int* slist, int* block_sums, int counters_are_zero, const int* rank, hipStream_t s,
+// Edges by sender: sstart[rows + 1] offsets, slist[E] the edges of every row in no particular order (readers order a
+// bucket as they read it; launch_sort_buckets does it in memory).  count[rows] must be zero on entry and is zero again
+// when the launches have run; rank[E] is scratch.  counted: histogram, ranks and offsets came with
+// launch_node_lists_count.  range_flag (or null): bit 1 raised where a key is outside [0, rows).
+hipError_t launch_sender_lists(const int* gather, long E, int rows, int* count, int* rank, int* sstart, int* slist,
+                               int* block_sums, bool counted, int* range_flag, hipStream_t s,
                                const InputGuard& guard = InputGuard());
+hipError_t launch_sort_buckets(const int* start, int rows, int* list, hipStream_t s);
 hipError_t launch_check_counts(const int* num_neigh, int N, const int* first_neigh, int num_local_nodes, long num_edges,
                                long num_local_edges, int* status, hipStream_t s);
-// first_neigh, degree order, species groups and `zero_n` cleared counters in one single-block launch
-// (N <= 65536; larger systems use the separate launches, where the extra launches do not matter)
-hipError_t launch_node_lists(const int* num_neigh, int N, int* first_neigh, int* order, const int* node_types, int T,
-                             int* tstart, int* perm, int* zero_p, long zero_n, hipStream_t s);
-// launch_node_lists plus the sender histogram count[rows] of `key[n]` in the same launch, with rank[n] = the place
-// each entry took in its bucket; the counters must be zero on entry (every sender-list build leaves them so)
+// first_neigh, degree order, species groups, the sender histogram count[rows] of `key[n]` with rank[n] = the place each
+// entry took in its bucket, and the sender offsets sstart[rows + 1], in one launch (N, rows <= 65536).  The counters and
+// *ticket must be zero on entry (every sender-list build leaves them so).
 hipError_t launch_node_lists_count(const int* num_neigh, int N, int* first_neigh, int* order, const int* node_types, int T,
                                    int* tstart, int* perm, const int* key, long n, int rows, int* count, int* rank,
-                                   const InputChecks& chk, hipStream_t s);
+                                   int* sstart, int* ticket, const InputChecks& chk, hipStream_t s);
 hipError_t launch_type_groups(const int* node_types, int N, int T, int* tcount, int* tstart, int* cursor,
                               int* perm, int* block_sums, hipStream_t s);
 // flags[0] |= 1 if any index is outside [0, limit)
@@ -322,11 +335,19 @@ hipError_t launch_radial(int N, const int* first_neigh, const int* node_types, c
                          const double* r, const F* tab, const int* pair_table, int T, int nodes, double h,
                          int nspl, double* R, hipStream_t s);
 
-// atom_forces[j] += f_e, atom_forces[i] -= f_e in a fixed order per atom, virial sums
-hipError_t launch_force_scatter(int num_atoms, const int* recv_start, const int* recv_list,
-                                const int* send_start, const int* send_list, const double* forces,
-                                double* atom_forces, hipStream_t s);
-hipError_t launch_virial(long E, const double* xyz, const double* forces, double* partial, int nblocks,
-                         hipStream_t s);
+// atom_forces[j] += f_e, atom_forces[i] -= f_e in a fixed order per atom; virial[6] = sum xyz (x) f, in LAMMPS order
+struct ForceGather {
+    int num_atoms;
+    const int* send_start; int* send_list;           // edges by sender atom (null: no sender side)
+    const int* node_start; const int* node_list;     // nodes whose edges count as received by the atom; null: node i is atom i
+    int num_nodes;
+    const int* first_neigh;                          // [num_nodes + 1]
+    const double* forces; const double* xyz;         // [E][3]
+    double* atom_forces;                             // [num_atoms][3] or null
+    double* partial;                                 // [force_gather_blocks][6], needed for the virial, else null
+    const int* flag;                                 // raised: the outputs are NaN (or null)
+};
+int force_gather_blocks(int num_atoms);
+hipError_t launch_force_gather(const ForceGather& g, double* virial, hipStream_t s);
 
 }  // namespace smx

@@ -754,15 +754,37 @@ template int agg_bwd_groups<float>(int, int);
 namespace {
 // V consecutive elements per thread (16-byte accesses when the row width allows); four messages are requested
 // before the first is added, the additions keep the ascending edge order
-template <typename F, int V>
-__global__ void k_sender_reduce(int rows, int width, const int* sstart, const int* slist, const F* msg,
+// WINDOW: slist is in ascending order in memory and the messages of the edges [e_lo, e_hi) are taken; otherwise all
+// messages of the row are, and the block orders the row's edges in LDS first.
+constexpr int SENDER_CAP = 1024;
+template <typename F, int V, bool WINDOW>
+__global__ void k_sender_reduce(int rows, int width, const int* sstart, int* slist_, const F* msg,
                                 F* H_adj, int zero_first, long e_lo, long e_hi)
 {
+    __shared__ __align__(16) int bucket[WINDOW ? 1 : 2 * SENDER_CAP];
     const int j = blockIdx.x;
     int s0 = sstart[j], s1 = sstart[j + 1];
-    // the sender's edges are listed in ascending order: narrow to those inside [e_lo, e_hi)
-    while (s0 < s1 && slist[s0] < e_lo) ++s0;
-    while (s1 > s0 && slist[s1 - 1] >= e_hi) --s1;
+    const int* slist = slist_;
+    if constexpr (WINDOW) {
+        // narrow to the edges inside [e_lo, e_hi)
+        while (s0 < s1 && slist[s0] < e_lo) ++s0;
+        while (s1 > s0 && slist[s1 - 1] >= e_hi) --s1;
+    } else if (s1 - s0 <= SENDER_CAP) {
+        const int n = s1 - s0;
+        for (int t = threadIdx.x; t < (n + 3) / 4 * 4; t += blockDim.x) bucket[t] = t < n ? slist[s0 + t] : 0x7fffffff;
+        __syncthreads();
+        for (int t = threadIdx.x; t < n; t += blockDim.x) {
+            const int v = bucket[t];
+            bucket[SENDER_CAP + count_below(bucket, n, v)] = v;
+        }
+        __syncthreads();
+        slist = bucket + SENDER_CAP;
+        s0 = 0; s1 = n;
+    } else {
+        if (threadIdx.x == 0) insertion_sort(slist_ + s0, s1 - s0);
+        __threadfence();
+        __syncthreads();
+    }
     if (s0 == s1 && !zero_first) return;
     for (int q = threadIdx.x * V; q < width; q += blockDim.x * V) {
         Vec<F, V> acc;
@@ -793,20 +815,21 @@ __global__ void k_sender_reduce(int rows, int width, const int* sstart, const in
 }  // namespace
 
 template <typename F>
-hipError_t launch_sender_reduce(int rows, int width, const int* sstart, const int* slist, const F* msg,
-                                F* H_adj, int zero_first, long e_lo, long e_hi, hipStream_t s)
+hipError_t launch_sender_reduce(int rows, int width, const int* sstart, int* slist, const F* msg,
+                                F* H_adj, int zero_first, bool window, long e_lo, long e_hi, hipStream_t s)
 {
     if (rows <= 0) return hipSuccess;
     constexpr int V = 16 / (int)sizeof(F);
+    auto go = [&](auto kern, int bs) {
+        hipLaunchKernelGGL(kern, dim3(rows), dim3(bs), 0, s, rows, width, sstart, slist, msg, H_adj, zero_first, e_lo, e_hi);
+    };
     if (width % V == 0) {
         const int lanes = width / V;
         const int bs = lanes <= 64 ? 64 : (lanes <= 128 ? 128 : 256);
-        hipLaunchKernelGGL((k_sender_reduce<F, V>), dim3(rows), dim3(bs), 0, s, rows, width, sstart, slist, msg, H_adj,
-                           zero_first, e_lo, e_hi);
+        if (window) go(k_sender_reduce<F, V, true>, bs); else go(k_sender_reduce<F, V, false>, bs);
     } else {
         const int bs = width <= 64 ? 64 : (width <= 128 ? 128 : 256);
-        hipLaunchKernelGGL((k_sender_reduce<F, 1>), dim3(rows), dim3(bs), 0, s, rows, width, sstart, slist, msg, H_adj,
-                           zero_first, e_lo, e_hi);
+        if (window) go(k_sender_reduce<F, 1, true>, bs); else go(k_sender_reduce<F, 1, false>, bs);
     }
     return hipGetLastError();
 }
@@ -820,11 +843,13 @@ hipError_t launch_sender_reduce(int rows, int width, const int* sstart, const in
 namespace {
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 template <typename F, int KT>
-__global__ __launch_bounds__(1024) void k_sender_reduce_linear(int rows, const int* sstart, const int* slist, const F* msg,
+__global__ __launch_bounds__(1024) void k_sender_reduce_linear(int rows, const int* sstart, int* slist_, const F* msg,
                                                               F* H_adj, int zero_first, const F* W, F* M_adj)
 {
     constexpr int K = 16 * KT, ld = K + 1, V = 16 / (int)sizeof(F);
+    constexpr int ROW_CAP = 256;
     __shared__ double X[16 * ld];
+    __shared__ __align__(16) int bucket[16][ROW_CAP];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
     const int row0 = blockIdx.x * 16;
@@ -841,12 +866,14 @@ __global__ __launch_bounds__(1024) void k_sender_reduce_linear(int rows, const i
     {
         const int rr = wave, j = row0 + rr;
         const int q = lane * V;
+        const int first = j < rows ? sstart[j] : 0, n = j < rows ? sstart[j + 1] - first : 0;
+        const int* slist = wave_sorted_bucket<ROW_CAP>(slist_, first, n, bucket[wave], lane);
         if (q < K) {
             Vec<F, V> acc;
 #pragma unroll
             for (int c = 0; c < V; ++c) acc.v[c] = F(0);
             if (j < rows) {
-                const int s0 = sstart[j], s1 = sstart[j + 1];
+                const int s0 = 0, s1 = n;
                 if (!zero_first) acc = ldv<F, V>(H_adj + (size_t)j * K + q);
                 int t = s0;
                 for (; t + 4 <= s1; t += 4) {
@@ -889,7 +916,7 @@ __global__ __launch_bounds__(1024) void k_sender_reduce_linear(int rows, const i
 bool sender_reduce_linear_ok(int K) { return K == 32 || K == 48 || K == 64 || K == 96 || K == 128; }
 
 template <typename F>
-hipError_t launch_sender_reduce_linear(int rows, int K, const int* sstart, const int* slist, const F* msg, F* H_adj,
+hipError_t launch_sender_reduce_linear(int rows, int K, const int* sstart, int* slist, const F* msg, F* H_adj,
                                        int zero_first, const F* W, F* M_adj, hipStream_t s)
 {
     if (!sender_reduce_linear_ok(K)) return hipErrorInvalidValue;
@@ -904,11 +931,11 @@ hipError_t launch_sender_reduce_linear(int rows, int K, const int* sstart, const
     }
     return hipGetLastError();
 }
-template hipError_t launch_sender_reduce_linear<double>(int, int, const int*, const int*, const double*, double*, int, const double*, double*, hipStream_t);
-template hipError_t launch_sender_reduce_linear<float>(int, int, const int*, const int*, const float*, float*, int, const float*, float*, hipStream_t);
+template hipError_t launch_sender_reduce_linear<double>(int, int, const int*, int*, const double*, double*, int, const double*, double*, hipStream_t);
+template hipError_t launch_sender_reduce_linear<float>(int, int, const int*, int*, const float*, float*, int, const float*, float*, hipStream_t);
 
-template hipError_t launch_sender_reduce<double>(int, int, const int*, const int*, const double*, double*, int, long, long, hipStream_t);
-template hipError_t launch_sender_reduce<float>(int, int, const int*, const int*, const float*, float*, int, long, long, hipStream_t);
+template hipError_t launch_sender_reduce<double>(int, int, const int*, int*, const double*, double*, int, bool, long, long, hipStream_t);
+template hipError_t launch_sender_reduce<float>(int, int, const int*, int*, const float*, float*, int, bool, long, long, hipStream_t);
 
 // ---------------------------------------------------------------------------
 namespace {

@@ -8,6 +8,7 @@
 //     image = x_j + shift;  d = image - x_i;  r2 = (d0*d0 + d1*d1) + d2*d2
 // so that the list is bit-identical to the host builder
 // (symmetrix_amd/neighbors.py), whatever the compiler would contract.
+#include "smx_device.hpp"
 #include "smx_kernels.hpp"
 
 namespace smx {
@@ -74,75 +75,135 @@ __global__ void k_nl_bin_fill(int N, const int* atom_bin, const int* bin_start, 
     bin_atoms[bin_start[b] + atomicAdd(&bin_cursor[b], 1)] = i;
 }
 
-// One thread per receiver walks every image shift and the bins that the cutoff sphere of the shifted
-// receiver can touch.  FILL = false counts, FILL = true writes the keys sender * num_shifts + shift index
-// (in whatever order the bins deliver them: k_nl_sort orders them).
-template <bool FILL>
-__global__ void k_nl_search(const double* pos, int N, NlGrid g, const int* bin_start, const int* bin_atoms,
-                            int num_shifts, const double* shift_vec, int zero_shift, double r_cut, double r2cut,
-                            int* count, const int* first, long long* keys)
+// One wavefront per receiver.  Its lanes first test 64 image shifts at a time against the bounding box of the atoms; for
+// every shift that can hold neighbours the senders are walked 64 at a time: ALL false, the runs of atoms in the bins that
+// the cutoff sphere of the shifted receiver touches (bins along the last axis are adjacent in memory, so a run is a row of
+// bins); ALL true, every atom, without bins (short lists: binning is three launches, and a small cell is one bin anyway).
+// FILL false counts.  FILL true collects the keys sender * num_shifts + shift index in LDS and writes them in ascending
+// order, which is the canonical edge order; EMIT writes the edge arrays as well (a list without a skin: every candidate is
+// an edge, at the positions of the search).
+// Bound by latency: a receiver takes about nine dependent steps (one thread per receiver, as this was before, took as many
+// as there are candidate pairs: 570 us against 8 us at 107 atoms in a cell smaller than twice the cutoff).
+constexpr int SORT_KEYS = 256;   // keys per wavefront that are ordered in LDS (2 KB each, four wavefronts per block)
+using NlEdges = NlEdgeArrays;
+__device__ __forceinline__ void emit_edge(const NlEdges& o, size_t e, int j, int s, const Cand& cd)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    o.neigh_indices[e] = j;
+    o.neigh_types[e] = o.types ? o.types[j] : 0;
+    o.neigh_shift[3 * e] = o.shift_int[3 * s]; o.neigh_shift[3 * e + 1] = o.shift_int[3 * s + 1];
+    o.neigh_shift[3 * e + 2] = o.shift_int[3 * s + 2];
+    o.xyz[3 * e] = cd.d0; o.xyz[3 * e + 1] = cd.d1; o.xyz[3 * e + 2] = cd.d2;
+    o.r[e] = __dsqrt_rn(cd.r2);
+}
+template <bool FILL, bool ALL, bool EMIT>
+__global__ __launch_bounds__(256) void k_nl_search(const double* pos, int N, NlGrid g, const int* bin_start,
+                                                   const int* bin_atoms, int num_shifts, const double* shift_vec,
+                                                   int zero_shift, double r_cut, double r2cut, int* count,
+                                                   const int* first, long capacity, long long* keys, long long* sorted,
+                                                   NlEdges out)
+{
+    __shared__ long long buf[FILL ? 4 : 1][FILL ? SORT_KEYS : 1];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int i = blockIdx.x * 4 + wave;
     if (i >= N) return;
+    const int e0 = FILL ? first[i] : 0, n = FILL ? first[i + 1] - e0 : 0;
+    if (FILL && EMIT && lane == 0) {
+        out.first[i] = e0; out.num_neigh[i] = n;
+        if (i == N - 1) out.first[N] = first[N];
+    }
+    // room for the whole list was taken before its length was known: nothing is written when it does not fit (the host
+    // looks at the total and takes more room)
+    if (FILL && first[N] > capacity) return;
+    const bool in_lds = n <= SORT_KEYS;
     const double xi[3] = {pos[3 * (size_t)i], pos[3 * (size_t)i + 1], pos[3 * (size_t)i + 2]};
     const double reach = r_cut * (1.0 + 1e-9) + 1e-12;
     int c = 0;
-    long long* out = FILL ? keys + first[i] : nullptr;
-    for (int s = 0; s < num_shifts; ++s) {
-        const double* sv = shift_vec + 3 * s;
-        int blo[3], bhi[3];
-        bool empty = false;
-        for (int k = 0; k < 3; ++k) {
-            const double q = xi[k] - sv[k];   // senders within reach of q see the receiver through shift s
-            if (q + reach < g.lo[k] || q - reach > g.hi[k]) { empty = true; break; }
-            blo[k] = bin_of(q - reach, g.lo[k], g.inv_bs[k], g.nb[k]);
-            bhi[k] = bin_of(q + reach, g.lo[k], g.inv_bs[k], g.nb[k]);
+    for (int s0 = 0; s0 < num_shifts; s0 += 64) {
+        bool here = s0 + lane < num_shifts;
+        if (here) {
+            const double* sv = shift_vec + 3 * (s0 + lane);
+            for (int k = 0; k < 3; ++k) {
+                const double q = xi[k] - sv[k];   // senders within reach of q see the receiver through shift s
+                here = here && !(q + reach < g.lo[k] || q - reach > g.hi[k]);
+            }
         }
-        if (empty) continue;
-        for (int b0 = blo[0]; b0 <= bhi[0]; ++b0)
-            for (int b1 = blo[1]; b1 <= bhi[1]; ++b1)
-                for (int b2 = blo[2]; b2 <= bhi[2]; ++b2) {
-                    const int b = (b0 * g.nb[1] + b1) * g.nb[2] + b2;
-                    for (int t = bin_start[b]; t < bin_start[b + 1]; ++t) {
-                        const int j = bin_atoms[t];
-                        if (j == i && s == zero_shift) continue;
-                        const Cand cd = displacement(pos, i, j, sv);
-                        if (cd.r2 < r2cut) {
-                            if (FILL) out[c] = (long long)j * num_shifts + s;
-                            ++c;
-                        }
+        for (unsigned long long todo = __ballot(here); todo; todo &= todo - 1) {
+            const int s = s0 + __ffsll((long long)todo) - 1;
+            const double sv[3] = {shift_vec[3 * s], shift_vec[3 * s + 1], shift_vec[3 * s + 2]};
+            auto walk = [&](int t0, int t1) {
+                for (int tb = t0; tb < t1; tb += 64) {
+                    const int t = tb + lane;
+                    bool hit = false;
+                    int j = 0;
+                    if (t < t1) {
+                        j = ALL ? t : bin_atoms[t];
+                        hit = !(j == i && s == zero_shift) && displacement(pos, i, j, sv).r2 < r2cut;
                     }
+                    const unsigned long long mask = __ballot(hit);
+                    if (FILL && hit) {
+                        const int at = c + __popcll(mask & ((1ull << lane) - 1ull));
+                        const long long key = (long long)j * num_shifts + s;
+                        if (in_lds) buf[wave][at] = key;
+                        else keys[(size_t)e0 + at] = key;
+                    }
+                    c += __popcll(mask);
                 }
+            };
+            if constexpr (ALL) {
+                walk(0, N);
+            } else {
+                int blo[3], bhi[3];
+                for (int k = 0; k < 3; ++k) {
+                    const double q = xi[k] - sv[k];
+                    blo[k] = bin_of(q - reach, g.lo[k], g.inv_bs[k], g.nb[k]);
+                    bhi[k] = bin_of(q + reach, g.lo[k], g.inv_bs[k], g.nb[k]);
+                }
+                for (int b0 = blo[0]; b0 <= bhi[0]; ++b0)
+                    for (int b1 = blo[1]; b1 <= bhi[1]; ++b1) {
+                        const int row = (b0 * g.nb[1] + b1) * g.nb[2];
+                        walk(bin_start[row + blo[2]], bin_start[row + bhi[2] + 1]);
+                    }
+            }
+        }
     }
-    if (!FILL) count[i] = c;
-}
-
-// One wavefront per receiver: rank of every key among the receiver's keys (they are distinct); the keys are
-// rewritten in ascending order, which is the canonical edge order of the receiver.
-__global__ __launch_bounds__(256) void k_nl_sort(int N, const int* cfirst, const long long* keys, long long* sorted)
-{
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (i >= N) return;
-    const int e0 = cfirst[i], n = cfirst[i + 1] - e0;
-    for (int a = lane; a < n; a += 64) {
-        const long long key = keys[e0 + a];
-        int rank = 0;
-        for (int b = 0; b < n; ++b) rank += keys[e0 + b] < key ? 1 : 0;
-        sorted[(size_t)e0 + rank] = key;
+    if constexpr (!FILL) {
+        if (lane == 0) count[i] = c;
+    } else {
+        // rank of every key among the receiver's keys (they are distinct)
+        if (in_lds) wave_lds_sync();
+        else __threadfence();
+        for (int a = lane; a < n; a += 64) {
+            const long long key = in_lds ? buf[wave][a] : keys[(size_t)e0 + a];
+            int rank = 0;
+            if (in_lds) {
+                for (int b = 0; b < n; ++b) rank += buf[wave][b] < key ? 1 : 0;
+            } else {
+                for (int b = 0; b < n; ++b) rank += keys[(size_t)e0 + b] < key ? 1 : 0;
+            }
+            sorted[(size_t)e0 + rank] = key;
+            if constexpr (EMIT) {
+                const int j = (int)(key / num_shifts), s = (int)(key % num_shifts);
+                emit_edge(out, (size_t)e0 + rank, j, s, displacement(pos, i, j, shift_vec + 3 * s));
+            }
+        }
     }
 }
 
 // One wavefront per receiver walks its sorted candidates with the current positions and keeps those inside
 // the cutoff, in order.  EMIT = false counts; EMIT = true writes the edge arrays at first[i] + (number kept before).
+// (room for `capacity` edges was taken before their number was known: none is written when they do not fit)
 template <bool EMIT>
-__global__ __launch_bounds__(256) void k_nl_filter(const double* pos, const int* types, int N, const int* cfirst,
-                                                   const long long* sorted, int num_shifts, const double* shift_vec,
-                                                   const int* shift_int, double r2cut, int* count, const int* first,
-                                                   int* neigh_indices, int* neigh_types, int* neigh_shift, double* xyz,
-                                                   double* r)
+__global__ __launch_bounds__(256) void k_nl_filter(const double* pos, int N, const int* cfirst, const long long* sorted,
+                                                   long room, int num_shifts, const double* shift_vec, double r2cut,
+                                                   int* count, const int* first, long capacity, NlEdges out)
 {
     const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (i >= N) return;
+    if (cfirst[N] > room) {          // the candidates themselves did not fit: nothing was written to `sorted`
+        if (!EMIT && lane == 0) count[i] = 0;
+        return;
+    }
+    if (EMIT && first[N] > capacity) return;
     const int c0 = cfirst[i], n = cfirst[i + 1] - c0;
     int kept = 0;
     const size_t e0 = EMIT ? (size_t)first[i] : 0;
@@ -158,15 +219,7 @@ __global__ __launch_bounds__(256) void k_nl_filter(const double* pos, const int*
             pass = cd.r2 < r2cut;
         }
         const unsigned long long mask = __ballot(pass);
-        if (EMIT && pass) {
-            const size_t e = e0 + kept + __popcll(mask & ((1ull << lane) - 1ull));
-            neigh_indices[e] = j;
-            neigh_types[e] = types ? types[j] : 0;
-            neigh_shift[3 * e] = shift_int[3 * s]; neigh_shift[3 * e + 1] = shift_int[3 * s + 1];
-            neigh_shift[3 * e + 2] = shift_int[3 * s + 2];
-            xyz[3 * e] = cd.d0; xyz[3 * e + 1] = cd.d1; xyz[3 * e + 2] = cd.d2;
-            r[e] = __dsqrt_rn(cd.r2);
-        }
+        if (EMIT && pass) emit_edge(out, e0 + kept + __popcll(mask & ((1ull << lane) - 1ull)), j, s, cd);
         kept += __popcll(mask);
     }
     if (!EMIT && lane == 0) count[i] = kept;
@@ -192,36 +245,34 @@ hipError_t launch_nl_bin_fill(int N, const int* atom_bin, const int* bin_start, 
 }
 hipError_t launch_nl_search(bool fill, const double* pos, int N, const NlGrid& g, const int* bin_start,
                             const int* bin_atoms, int num_shifts, const double* shift_vec, int zero_shift,
-                            double r_cut, int* count, const int* first, long long* keys, hipStream_t s)
+                            double r_cut, int* count, const int* first, long capacity, long long* keys, long long* sorted,
+                            const NlEdgeArrays* edges, hipStream_t s)
 {
     if (N <= 0) return hipSuccess;
-    const double r2cut = r_cut * r_cut;
-    if (fill)
-        hipLaunchKernelGGL(k_nl_search<true>, dim3((N + 63) / 64), dim3(64), 0, s, pos, N, g, bin_start, bin_atoms,
-                           num_shifts, shift_vec, zero_shift, r_cut, r2cut, count, first, keys);
-    else
-        hipLaunchKernelGGL(k_nl_search<false>, dim3((N + 63) / 64), dim3(64), 0, s, pos, N, g, bin_start, bin_atoms,
-                           num_shifts, shift_vec, zero_shift, r_cut, r2cut, count, first, keys);
+    const NlEdges o = edges ? *edges : NlEdges{};
+    const bool all = bin_start == nullptr;
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((N + 3) / 4), dim3(256), 0, s, pos, N, g, bin_start, bin_atoms, num_shifts, shift_vec,
+                           zero_shift, r_cut, r_cut * r_cut, count, first, capacity, keys, sorted, o);
+    };
+    if (!fill) { if (all) go(k_nl_search<false, true, false>); else go(k_nl_search<false, false, false>); }
+    else if (!edges) { if (all) go(k_nl_search<true, true, false>); else go(k_nl_search<true, false, false>); }
+    else { if (all) go(k_nl_search<true, true, true>); else go(k_nl_search<true, false, true>); }
     return hipGetLastError();
 }
-hipError_t launch_nl_sort(int N, const int* cfirst, const long long* keys, long long* sorted, hipStream_t s)
-{
-    if (N > 0) hipLaunchKernelGGL(k_nl_sort, dim3((N + 3) / 4), dim3(256), 0, s, N, cfirst, keys, sorted);
-    return hipGetLastError();
-}
-hipError_t launch_nl_filter(bool emit, const double* pos, const int* types, int N, const int* cfirst,
-                            const long long* sorted, int num_shifts, const double* shift_vec, const int* shift_int,
-                            double r_cut, int* count, const int* first, int* neigh_indices, int* neigh_types,
-                            int* neigh_shift, double* xyz, double* r, hipStream_t s)
+hipError_t launch_nl_filter(bool emit, const double* pos, int N, const int* cfirst, const long long* sorted, long room, int num_shifts,
+                            const double* shift_vec, double r_cut, int* count, const int* first, long capacity,
+                            const NlEdgeArrays* edges, hipStream_t s)
 {
     if (N <= 0) return hipSuccess;
+    const NlEdges o = edges ? *edges : NlEdges{};
     const double r2cut = r_cut * r_cut;
     if (emit)
-        hipLaunchKernelGGL(k_nl_filter<true>, dim3((N + 3) / 4), dim3(256), 0, s, pos, types, N, cfirst, sorted, num_shifts,
-                           shift_vec, shift_int, r2cut, count, first, neigh_indices, neigh_types, neigh_shift, xyz, r);
+        hipLaunchKernelGGL(k_nl_filter<true>, dim3((N + 3) / 4), dim3(256), 0, s, pos, N, cfirst, sorted, room, num_shifts, shift_vec,
+                           r2cut, count, first, capacity, o);
     else
-        hipLaunchKernelGGL(k_nl_filter<false>, dim3((N + 3) / 4), dim3(256), 0, s, pos, types, N, cfirst, sorted, num_shifts,
-                           shift_vec, shift_int, r2cut, count, first, neigh_indices, neigh_types, neigh_shift, xyz, r);
+        hipLaunchKernelGGL(k_nl_filter<false>, dim3((N + 3) / 4), dim3(256), 0, s, pos, N, cfirst, sorted, room, num_shifts, shift_vec,
+                           r2cut, count, first, capacity, o);
     return hipGetLastError();
 }
 

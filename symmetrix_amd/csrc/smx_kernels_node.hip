@@ -72,48 +72,53 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_add(int* out, int n, const 
     if (i < n) out[i] += block_sums[blockIdx.x];
 }
 
-// keys outside [0, rows) are ignored (callers that hand over device arrays are not range-checked)
-__global__ void k_count(const int* key, long n, int rows, int* count)
+// Histogram of the keys, and the place that every entry took inside its bucket (whatever order the atomics leave: readers
+// order the bucket by entry).  Keys outside [0, rows) are left out and raise bit 1 of *flag (if not null).
+__global__ void k_count_ranked(const int* key, long n, int rows, int* count, int* rank, int* flag)
 {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
         const int j = key[i];
-        if (j >= 0 && j < rows) atomicAdd(&count[j], 1);
+        if (j >= 0 && j < rows) rank[i] = atomicAdd(&count[j], 1);
+        else if (flag) atomicOr(flag, 1);
     }
 }
-__global__ void k_place(const int* key, long n, int rows, const int* start, int* cursor, int* list)
+// Placement of entries that know their place inside the bucket: no atomics.  The counters are dead by now: they are cleared
+// here, so that the next list build finds them at zero without a launch of its own.
+// With a guard (arrays that no host code has looked at): when the checks of this evaluation raised its status word, the CSR
+// offsets, the sender lists and the species groups are set to "no edges, no nodes", so that no later kernel of the
+// evaluation uses an unchecked integer as an address; the status goes into the sticky word the host reads at its next
+// synchronising call and, raised or not, into the word the later kernels read.
+__global__ void k_place_ranked(const int* key, const int* rank, long n, int rows, int* start, int* list, int* count,
+                               InputGuard g)
 {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < rows) count[i] = 0;
+    if (g.status) {
+        const int st = *g.status;
+        if (i == 0) {
+            *g.live = st;
+            if (st) *g.sticky |= st;   // one thread of one launch on the stream: no other writer
+        }
+        if (st) {
+            if (i < g.n_first) g.first_neigh[i] = 0;
+            if (i < g.n_tstart) g.tstart[i] = 0;
+            if (i <= rows) start[i] = 0;
+            return;
+        }
+    }
     if (i < n) {
         const int j = key[i];
-        if (j >= 0 && j < rows) list[start[j] + atomicAdd(&cursor[j], 1)] = (int)i;
+        if (j >= 0 && j < rows) list[start[j] + rank[i]] = (int)i;
     }
 }
-// Ascending order inside every bucket (the atomic placement above is unordered).
-// One wavefront per bucket; entries are distinct, so the rank of an entry is the
-// number of smaller ones: bucket staged in LDS, every lane counts for its entries.
+// Ascending order inside every bucket, in memory: for readers that take a window of the edges (the others order a bucket in
+// LDS as they read it).  One wavefront per bucket.
 constexpr int SORT_LDS = 1024;
-// The bucket's counter and cursor are dead by now: they are cleared here, so that the next list build
-// finds them at zero without a launch of its own.
-// With a guard (device-resident callers, whose arrays no host code has looked at): when the checks of this
-// evaluation raised its status word, the CSR offsets and the species groups are set to "no edges, no nodes", so
-// that no later kernel of the evaluation uses an unchecked integer as an address; the status goes into the sticky
-// word the host reads at its next synchronising call and, raised or not, into the word the later kernels read.
-__global__ __launch_bounds__(64) void k_sort_buckets(const int* start, int rows, int* list, int* count, int* cursor,
-                                                     InputGuard g)
+__global__ __launch_bounds__(64) void k_sort_buckets(const int* start, int rows, int* list)
 {
     __shared__ int buf[SORT_LDS];
     const int j = blockIdx.x;
-    if (g.status) {
-        const int st = *g.status;
-        if (st) {
-            for (int i = j * 64 + threadIdx.x; i < g.n_first; i += gridDim.x * 64) g.first_neigh[i] = 0;
-            for (int i = j * 64 + threadIdx.x; i < g.n_tstart; i += gridDim.x * 64) g.tstart[i] = 0;
-            if (j == 0 && threadIdx.x == 0) atomicOr(g.sticky, st);
-        }
-        if (j == 0 && threadIdx.x == 0) *g.live = st;
-    }
-    if (threadIdx.x == 0) { count[j] = 0; cursor[j] = 0; }
     const int s0 = start[j], n = start[j + 1] - s0;
     if (n <= 1) return;
     if (n <= SORT_LDS) {
@@ -126,13 +131,7 @@ __global__ __launch_bounds__(64) void k_sort_buckets(const int* start, int rows,
             list[s0 + rank] = v;
         }
     } else if (threadIdx.x == 0) {
-        // very long bucket: in-place insertion sort by one lane (correct, slow, not expected in practice)
-        for (int a = s0 + 1; a < s0 + n; ++a) {
-            const int v = list[a];
-            int b = a - 1;
-            while (b >= s0 && list[b] > v) { list[b + 1] = list[b]; --b; }
-            list[b + 1] = v;
-        }
+        insertion_sort(list + s0, n);
     }
 }
 // species groups in one block: LDS histogram, scan over the (few) species, placement
@@ -248,31 +247,10 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_single(const int* in, int* 
 {
     scan_single_body(in, out, n);
 }
-// The node-level lists of one evaluation in one launch (one block): first_neigh = exclusive scan of
-// num_neigh, receivers by decreasing degree, species groups, and the zeroing of `zero_n` counters that the
-// sender-list kernels count into.  Each part is the body of the stand-alone kernel of the same name.
-__global__ __launch_bounds__(SCAN_BLOCK) void k_node_lists(const int* num_neigh, int N, int* first_neigh, int* order,
-                                                          const int* node_types, int T, int* tstart, int* perm,
-                                                          int* zero_p, long zero_n)
+__device__ void node_lists_part(const int* num_neigh, int N, int* first_neigh, int* order, const int* node_types, int T,
+                                int* tstart, int* perm, const int* key, long n, int rows, int* count, int* rank,
+                                const InputChecks& chk, int* sh)
 {
-    extern __shared__ int sh[];
-    for (long i = threadIdx.x; i < zero_n; i += SCAN_BLOCK) zero_p[i] = 0;
-    scan_single_body(num_neigh, first_neigh, N);
-    __syncthreads();   // first_neigh, written by this block, is read back below
-    degree_order_body(N, first_neigh, order);
-    __syncthreads();
-    type_groups_body(node_types, N, T, tstart, perm, sh);
-}
-// The same with the sender histogram in the same launch: blocks 0, 1, 2 form one node list each, the other blocks
-// count the senders (counters at zero on entry), which does not depend on the node lists.
-// With `chk.status` set the launch also checks everything the later kernels use as an address or a table argument
-// (species, sender rows, edge lengths, counts that add up to the edge totals) and raises bits in the status word.
-__global__ __launch_bounds__(SCAN_BLOCK) void k_node_lists_count(const int* num_neigh, int N, int* first_neigh, int* order,
-                                                                const int* node_types, int T, int* tstart, int* perm,
-                                                                const int* key, long n, int rows, int* count, int* rank,
-                                                                InputChecks chk)
-{
-    extern __shared__ int sh[];
     // the three node lists are independent of each other: a block each
     if (blockIdx.x == 0) {
         scan_single_body(num_neigh, first_neigh, N);
@@ -305,6 +283,34 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_node_lists_count(const int* num_
         if (bad) atomicOr(chk.status, bad);
     }
 }
+// The node-level lists of one evaluation and its sender histogram in one launch: blocks 0, 1, 2 form one node list each
+// (first_neigh = exclusive scan of num_neigh, receivers by decreasing degree, species groups), the other blocks count the
+// senders (counters at zero on entry), which does not depend on the node lists.  With a ticket, the block that finishes last
+// turns the histogram into the sender offsets: a launch of its own costs 6 to 8 us of a small evaluation, but the fences of
+// the ticket cost more than that over many blocks (80 us over 2 048), so the launcher hands out tickets to small grids only.
+// With `chk.status` set the launch also checks everything the later kernels use as an address or a table argument
+// (species, sender rows, edge lengths, counts that add up to the edge totals) and raises bits in the status word.
+__global__ __launch_bounds__(SCAN_BLOCK) void k_node_lists_count(const int* num_neigh, int N, int* first_neigh, int* order,
+                                                                const int* node_types, int T, int* tstart, int* perm,
+                                                                const int* key, long n, int rows, int* count, int* rank,
+                                                                int* sstart, int* ticket, InputChecks chk)
+{
+    extern __shared__ int sh[];
+    node_lists_part(num_neigh, N, first_neigh, order, node_types, T, tstart, perm, key, n, rows, count, rank, chk, sh);
+    if (!ticket) return;
+    // every block's counts are out before it takes its ticket
+    __shared__ int last;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence();
+        last = atomicAdd(ticket, 1) == (int)gridDim.x - 1;
+        __threadfence();
+    }
+    __syncthreads();
+    if (!last) return;
+    scan_single_body(count, sstart, rows);
+    if (threadIdx.x == 0) *ticket = 0;
+}
 // the same checks as separate work for lists too long for the single-block scan
 __global__ void k_check_counts(const int* num_neigh, int N, const int* first_neigh, int num_local_nodes, long num_edges,
                                long num_local_edges, int* status)
@@ -315,26 +321,19 @@ __global__ void k_check_counts(const int* num_neigh, int N, const int* first_nei
         bad |= (first_neigh[N] != (int)num_edges) | (first_neigh[num_local_nodes] != (int)num_local_edges);
     if (bad) atomicOr(status, 1);
 }
-// placement of entries that know their place inside the bucket: no atomics
-__global__ void k_place_ranked(const int* key, const int* rank, long n, int rows, const int* start, int* list)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        const int j = key[i];
-        if (j >= 0 && j < rows) list[start[j] + rank[i]] = (int)i;
-    }
-}
 }  // namespace
 
 hipError_t launch_node_lists_count(const int* num_neigh, int N, int* first_neigh, int* order, const int* node_types, int T,
                                    int* tstart, int* perm, const int* key, long n, int rows, int* count, int* rank,
-                                   const InputChecks& chk, hipStream_t s)
+                                   int* sstart, int* ticket, const InputChecks& chk, hipStream_t s)
 {
     if (N <= 0 || N > 64 * SCAN_BLOCK || T <= 0) return hipErrorInvalidValue;
     const long work = chk.status ? std::max(n, chk.num_edges) : n;
     const unsigned nb = 3 + (unsigned)std::max<long>(1, std::min<long>((work + SCAN_BLOCK - 1) / SCAN_BLOCK, 2048));
+    const bool with_scan = nb <= 160;
     hipLaunchKernelGGL(k_node_lists_count, dim3(nb), dim3(SCAN_BLOCK), 2 * T * sizeof(int), s, num_neigh, N, first_neigh,
-                       order, node_types, T, tstart, perm, key, n, rows, count, rank, chk);
+                       order, node_types, T, tstart, perm, key, n, rows, count, rank, sstart, with_scan ? ticket : nullptr, chk);
+    if (!with_scan) hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(SCAN_BLOCK), 0, s, count, sstart, rows);
     return hipGetLastError();
 }
 hipError_t launch_check_counts(const int* num_neigh, int N, const int* first_neigh, int num_local_nodes, long num_edges,
@@ -343,15 +342,6 @@ hipError_t launch_check_counts(const int* num_neigh, int N, const int* first_nei
     if (N > 0)
         hipLaunchKernelGGL(k_check_counts, dim3(std::min<unsigned>(nblk(N, 256), 1024u)), dim3(256), 0, s, num_neigh, N,
                            first_neigh, num_local_nodes, num_edges, num_local_edges, status);
-    return hipGetLastError();
-}
-
-hipError_t launch_node_lists(const int* num_neigh, int N, int* first_neigh, int* order, const int* node_types, int T,
-                             int* tstart, int* perm, int* zero_p, long zero_n, hipStream_t s)
-{
-    if (N <= 0 || N > 64 * SCAN_BLOCK || T <= 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_node_lists, dim3(1), dim3(SCAN_BLOCK), 2 * T * sizeof(int), s, num_neigh, N, first_neigh, order,
-                       node_types, T, tstart, perm, zero_p, zero_n);
     return hipGetLastError();
 }
 
@@ -368,32 +358,23 @@ hipError_t launch_scan_exclusive(const int* in, int* out, int n, int* block_sums
     return hipGetLastError();
 }
 
-hipError_t launch_sender_lists(const int* gather, int E, int rows, int* count, int* sstart, int* cursor,
-                               int* slist, int* block_sums, int counters_are_zero, const int* rank, hipStream_t s,
-                               const InputGuard& guard)
+hipError_t launch_sender_lists(const int* gather, long E, int rows, int* count, int* rank, int* sstart, int* slist,
+                               int* block_sums, bool counted, int* range_flag, hipStream_t s, const InputGuard& guard)
 {
     if (rows <= 0) return hipSuccess;
-    const bool counted = counters_are_zero == 2;   // the histogram came with the node lists
-    if (counters_are_zero) {
-        // cleared by the previous build (or by k_node_lists)
-    } else if (cursor == count + rows) {
-        hipLaunchKernelGGL(k_fill<int>, dim3(nblk(2L * rows, 256)), dim3(256), 0, s, count, 2L * rows, 0);
-    } else {
-        hipLaunchKernelGGL(k_fill<int>, dim3(nblk(rows, 256)), dim3(256), 0, s, count, (long)rows, 0);
-        hipLaunchKernelGGL(k_fill<int>, dim3(nblk(rows, 256)), dim3(256), 0, s, cursor, (long)rows, 0);
+    if (!counted) {
+        if (E > 0) hipLaunchKernelGGL(k_count_ranked, dim3(nblk(E, 256)), dim3(256), 0, s, gather, E, rows, count, rank, range_flag);
+        hipError_t err = launch_scan_exclusive(count, sstart, rows, block_sums, s);
+        if (err != hipSuccess) return err;
     }
-    if (E > 0 && !counted) hipLaunchKernelGGL(k_count, dim3(nblk(E, 256)), dim3(256), 0, s, gather, (long)E, rows, count);
-    hipError_t err = launch_scan_exclusive(count, sstart, rows, block_sums, s);
-    if (err != hipSuccess) return err;
-    if (E > 0) {
-        if (counted && rank)
-            hipLaunchKernelGGL(k_place_ranked, dim3(nblk(E, 256)), dim3(256), 0, s, gather, rank, (long)E, rows, sstart, slist);
-        else
-            hipLaunchKernelGGL(k_place, dim3(nblk(E, 256)), dim3(256), 0, s, gather, (long)E, rows, sstart, cursor, slist);
-    }
-    // the guard's bookkeeping rides on this launch, so it also runs for an edge list that claims to be empty
-    if (E > 0 || guard.status)
-        hipLaunchKernelGGL(k_sort_buckets, dim3(rows), dim3(64), 0, s, sstart, rows, slist, count, cursor, guard);
+    // (the counters and the guard's bookkeeping ride on this launch, so it also runs for an empty edge list)
+    const long threads = std::max<long>({E, (long)rows + 1, (long)guard.n_first, (long)guard.n_tstart});
+    hipLaunchKernelGGL(k_place_ranked, dim3(nblk(threads, 256)), dim3(256), 0, s, gather, rank, E, rows, sstart, slist, count, guard);
+    return hipGetLastError();
+}
+hipError_t launch_sort_buckets(const int* start, int rows, int* list, hipStream_t s)
+{
+    if (rows > 0) hipLaunchKernelGGL(k_sort_buckets, dim3(rows), dim3(64), 0, s, start, rows, list);
     return hipGetLastError();
 }
 
@@ -1015,58 +996,80 @@ template hipError_t launch_readout_fused<float>(int, int, int, int, const int*, 
 
 
 // ===========================================================================
-// Caller-side reductions: per-edge forces -> per-atom forces (each atom sums its
-// own incoming and outgoing edges in ascending edge order: no atomics), virial.
+// Caller-side reductions: per-edge forces -> per-atom forces, virial.
+// One wavefront per atom and step: the edges on which the atom is the sender are ordered in LDS, its lanes add them up (and
+// the edges of its receivers, which are contiguous) in a fixed assignment and a fixed tree, so the sums are
+// bit-reproducible.  A wavefront's share of the virial stays in its registers; every block leaves one partial sum.
+// Bound by latency at small sizes (one thread per atom, as this was before: 52 us at 107 atoms, 31 us at 501), by the
+// gather of 24-byte forces at large ones.
 namespace {
-__global__ void k_force_scatter(int num_atoms, const int* recv_start, const int* recv_list, const int* send_start,
-                                const int* send_list, const double* forces, double* atom_forces)
+constexpr int GATHER_CAP = 512;
+__global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
 {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= num_atoms) return;
-    double fx = 0, fy = 0, fz = 0;
-    for (int t = send_start[a]; t < send_start[a + 1]; ++t) {
-        const size_t e = send_list[t];
-        fx += forces[3 * e]; fy += forces[3 * e + 1]; fz += forces[3 * e + 2];
-    }
-    for (int t = recv_start[a]; t < recv_start[a + 1]; ++t) {
-        const size_t e = recv_list ? recv_list[t] : t;
-        fx -= forces[3 * e]; fy -= forces[3 * e + 1]; fz -= forces[3 * e + 2];
-    }
-    atom_forces[3 * (size_t)a] = fx; atom_forces[3 * (size_t)a + 1] = fy; atom_forces[3 * (size_t)a + 2] = fz;
-}
-__global__ __launch_bounds__(256) void k_virial(long E, const double* xyz, const double* f, double* partial)
-{
-    __shared__ double red[6][256];
+    __shared__ __align__(16) int bucket[4][GATHER_CAP];
+    __shared__ double red[4][6];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     double v[6] = {0, 0, 0, 0, 0, 0};
-    // fixed assignment of edges to threads, fixed tree: deterministic
-    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < E; e += (long)gridDim.x * blockDim.x) {
-        const double x = xyz[3 * e], y = xyz[3 * e + 1], z = xyz[3 * e + 2];
-        const double fx = f[3 * e], fy = f[3 * e + 1], fz = f[3 * e + 2];
-        v[0] += x * fx; v[1] += y * fy; v[2] += z * fz;
-        v[3] += 0.5 * (x * fy + y * fx); v[4] += 0.5 * (x * fz + z * fx); v[5] += 0.5 * (y * fz + z * fy);
+    for (int at = blockIdx.x * 4 + wave; at < a.num_atoms; at += gridDim.x * 4) {
+        double fx = 0, fy = 0, fz = 0;
+        if (a.send_start) {
+            const int s0 = a.send_start[at], n = a.send_start[at + 1] - s0;
+            const int* sorted = wave_sorted_bucket<GATHER_CAP>(a.send_list, s0, n, bucket[wave], lane);
+            for (int t = lane; t < n; t += 64) {
+                const double* f = a.forces + 3 * (size_t)sorted[t];
+                fx += f[0]; fy += f[1]; fz += f[2];
+            }
+        }
+        // nodes whose receivers belong to this atom: a list of them, or node at itself
+        const int n0 = a.node_start ? a.node_start[at] : at;
+        const int n1 = a.node_start ? a.node_start[at + 1] : (at < a.num_nodes ? at + 1 : at);
+        for (int q = n0; q < n1; ++q) {
+            const int node = a.node_list ? a.node_list[q] : q;
+            for (int e = a.first_neigh[node] + lane; e < a.first_neigh[node + 1]; e += 64) {
+                const double* f = a.forces + 3 * (size_t)e;
+                const double* d = a.xyz + 3 * (size_t)e;
+                const double x = d[0], y = d[1], z = d[2];
+                fx -= f[0]; fy -= f[1]; fz -= f[2];
+                v[0] += x * f[0]; v[1] += y * f[1]; v[2] += z * f[2];
+                v[3] += 0.5 * (x * f[1] + y * f[0]); v[4] += 0.5 * (x * f[2] + z * f[0]); v[5] += 0.5 * (y * f[2] + z * f[1]);
+            }
+        }
+        if (a.atom_forces) {
+            fx = wave_sum(fx); fy = wave_sum(fy); fz = wave_sum(fz);
+            if (a.flag && *a.flag) fx = fy = fz = __builtin_nan("");
+            if (lane < 3) a.atom_forces[3 * (size_t)at + lane] = lane == 0 ? fx : (lane == 1 ? fy : fz);
+        }
+        wave_lds_sync();   // the next atom's bucket overwrites this one's
     }
-    for (int q = 0; q < 6; ++q) red[q][threadIdx.x] = v[q];
+    if (!a.partial) return;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+        const double t = wave_sum(v[q]);
+        if (lane == 0) red[wave][q] = t;
+    }
     __syncthreads();
-    for (int off = 128; off >= 1; off >>= 1) {
-        if ((int)threadIdx.x < off)
-            for (int q = 0; q < 6; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x < 6) partial[blockIdx.x * 6 + threadIdx.x] = red[threadIdx.x][0];
+    if (threadIdx.x < 6)
+        a.partial[(size_t)blockIdx.x * 6 + threadIdx.x] =
+            (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
+}
+// the blocks' partial sums in a fixed order
+__global__ __launch_bounds__(384) void k_virial_finish(const double* partial, int nblocks, const int* flag, double* virial)
+{
+    const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    double v = 0.0;
+    for (int b = lane; b < nblocks; b += 64) v += partial[(size_t)b * 6 + q];
+    v = wave_sum(v);
+    if (lane == 0) virial[q] = flag && *flag ? __builtin_nan("") : v;
 }
 }  // namespace
 
-hipError_t launch_force_scatter(int num_atoms, const int* recv_start, const int* recv_list, const int* send_start,
-                                const int* send_list, const double* forces, double* atom_forces, hipStream_t s)
+int force_gather_blocks(int num_atoms) { return std::min((num_atoms + 3) / 4, 2048); }
+hipError_t launch_force_gather(const ForceGather& g, double* virial, hipStream_t s)
 {
-    if (num_atoms > 0)
-        hipLaunchKernelGGL(k_force_scatter, dim3(nblk(num_atoms, 128)), dim3(128), 0, s, num_atoms, recv_start,
-                           recv_list, send_start, send_list, forces, atom_forces);
-    return hipGetLastError();
-}
-hipError_t launch_virial(long E, const double* xyz, const double* forces, double* partial, int nblocks, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_virial, dim3(nblocks), dim3(256), 0, s, E, xyz, forces, partial);
+    const int nb = force_gather_blocks(g.num_atoms);
+    if (nb <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_force_gather, dim3(nb), dim3(256), 0, s, g);
+    if (virial) hipLaunchKernelGGL(k_virial_finish, dim3(1), dim3(384), 0, s, g.partial, nb, g.flag, virial);
     return hipGetLastError();
 }
 

@@ -15,17 +15,17 @@ namespace {
 
 constexpr int kMaxAtoms = SMX_NOALLOC_MAX_ATOMS;
 constexpr long kMaxEdges = SMX_NOALLOC_MAX_EDGES;
-constexpr int kVirialBlocks = 64;
+constexpr int kVirialBlocks = 2048;   // most that launch_force_gather leaves partial sums for
 
 constexpr size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 // layout of the scratch array (byte offsets, every part 256-byte aligned)
 constexpr size_t kOffFlag = 0;                                                          // int[64]
-constexpr size_t kOffCount = kOffFlag + 256;                                            // int[2 * atoms]: counters, cursors
-constexpr size_t kOffSendStart = kOffCount + align256(2 * (size_t)kMaxAtoms * sizeof(int));     // int[atoms + 1]
-constexpr size_t kOffRecvStart = kOffSendStart + align256(((size_t)kMaxAtoms + 1) * sizeof(int)); // int[atoms + 1]
-constexpr size_t kOffBlockSums = kOffRecvStart + align256(((size_t)kMaxAtoms + 1) * sizeof(int)); // int[atoms / 1024 + 2]
+constexpr size_t kOffCount = kOffFlag + 256;                                            // int[atoms]: counters
+constexpr size_t kOffSendStart = kOffCount + align256((size_t)kMaxAtoms * sizeof(int));     // int[atoms + 1]
+constexpr size_t kOffBlockSums = kOffSendStart + align256(((size_t)kMaxAtoms + 1) * sizeof(int)); // int[atoms / 1024 + 2]
 constexpr size_t kOffSendList = kOffBlockSums + align256(((size_t)kMaxAtoms / 1024 + 2) * sizeof(int)); // int[edges]
-constexpr size_t kOffVirial = kOffSendList + align256((size_t)kMaxEdges * sizeof(int));  // double[64 * 6]
+constexpr size_t kOffRank = kOffSendList + align256((size_t)kMaxEdges * sizeof(int));    // int[edges]
+constexpr size_t kOffVirial = kOffRank + align256((size_t)kMaxEdges * sizeof(int));      // double[2048 * 6]
 constexpr size_t kScratchBytes = kOffVirial + align256((size_t)kVirialBlocks * 6 * sizeof(double));
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -34,29 +34,6 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 // in host code)
 constexpr int kMaxDevices = 64;
 unsigned char* g_scratch_ptr[kMaxDevices] = {};
-
-// receiver block i is atom i: CSR offsets of the receivers, padded with the edge count for atoms beyond them
-__global__ void k_pad_starts(const int* first_neigh, int num_receivers, int num_atoms, int* out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i <= num_atoms) out[i] = first_neigh[i < num_receivers ? i : num_receivers];
-}
-// the partial sums in ascending block order, as the allocating entry point adds them on the host
-__global__ void k_virial_finish(const double* partial, int nblocks, const int* flag, double* virial)
-{
-    const int q = threadIdx.x;
-    if (q >= 6) return;
-    double v = 0.0;
-    for (int b = 0; b < nblocks; ++b) v += partial[(size_t)b * 6 + q];
-    virial[q] = *flag ? __builtin_nan("") : v;
-}
-// an out-of-range sender index cannot be reported through a return code without a host synchronisation:
-// the outputs are NaN instead
-__global__ void k_poison_if_flag(const int* flag, double* out, long n)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && *flag) out[i] = __builtin_nan("");
-}
 
 }  // namespace
 
@@ -121,36 +98,27 @@ extern "C" int smx_reduce_forces_device_noalloc(smx_model* m, int num_atoms, con
     int* flag = reinterpret_cast<int*>(base + kOffFlag);
     int* count = reinterpret_cast<int*>(base + kOffCount);
     int* send_start = reinterpret_cast<int*>(base + kOffSendStart);
-    int* recv_start = reinterpret_cast<int*>(base + kOffRecvStart);
     int* block_sums = reinterpret_cast<int*>(base + kOffBlockSums);
     int* send_list = reinterpret_cast<int*>(base + kOffSendList);
+    int* rank = reinterpret_cast<int*>(base + kOffRank);
     double* partial = reinterpret_cast<double*>(base + kOffVirial);
     const long E = v.num_edges;
+    // an out-of-range sender index cannot be reported through a return code without a host synchronisation: the outputs
+    // are NaN instead
     hipError_t e = smx::launch_fill<int>(flag, 1, 0, s);
-    if (e == hipSuccess) e = smx::launch_check_range(d_sender_atom, E, num_atoms, flag, s);
-    if (e == hipSuccess && d_atom_forces) {
-        // counters and cursors of the last call are cleared inside (a fill kernel, no memset node)
-        e = smx::launch_sender_lists(d_sender_atom, (int)E, num_atoms, count, send_start, count + num_atoms, send_list,
-                                     block_sums, 0, nullptr, s);
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_pad_starts, dim3((num_atoms + 256) / 256), dim3(256), 0, s, v.first_neigh, v.num_receivers,
-                               num_atoms, recv_start);
-            e = hipGetLastError();
-        }
-        if (e == hipSuccess) e = smx::launch_force_scatter(num_atoms, recv_start, nullptr, send_start, send_list, v.node_forces, d_atom_forces, s);
-        if (e == hipSuccess) {
-            const long n = 3L * num_atoms;
-            hipLaunchKernelGGL(k_poison_if_flag, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, flag, d_atom_forces, n);
-            e = hipGetLastError();
-        }
+    smx::ForceGather g{};
+    g.num_atoms = num_atoms; g.num_nodes = v.num_receivers; g.first_neigh = v.first_neigh;
+    g.forces = v.node_forces; g.xyz = v.xyz; g.atom_forces = d_atom_forces; g.flag = flag;
+    if (d_virial) g.partial = partial;
+    if (d_atom_forces) {
+        if (e == hipSuccess) e = smx::launch_fill<int>(count, num_atoms, 0, s);
+        if (e == hipSuccess)
+            e = smx::launch_sender_lists(d_sender_atom, E, num_atoms, count, rank, send_start, send_list, block_sums, false, flag, s);
+        g.send_start = send_start; g.send_list = send_list;
+    } else if (e == hipSuccess) {
+        e = smx::launch_check_range(d_sender_atom, E, num_atoms, flag, s);
     }
-    if (e == hipSuccess && d_virial) {
-        e = smx::launch_virial(E, v.xyz, v.node_forces, partial, kVirialBlocks, s);
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(k_virial_finish, dim3(1), dim3(64), 0, s, partial, kVirialBlocks, flag, d_virial);
-            e = hipGetLastError();
-        }
-    }
+    if (e == hipSuccess) e = smx::launch_force_gather(g, d_virial, s);
     if (e != hipSuccess) {
         smx::set_last_error(std::string("smx_reduce_forces_device_noalloc: ") + hipGetErrorString(e));
         return SMX_EHIP;

@@ -164,6 +164,15 @@ class MACE:
                                                     _pd(V) if virial else None))
         return (F, V) if virial else F
 
+    def evaluate_list(self, nlist):
+        """Energies [N], forces [N,3] and virial [6] of the atoms of a DeviceNeighborList built from host positions."""
+        n = nlist.num_atoms
+        out = np.empty(4 * n + 6)
+        base = out.ctypes.data
+        _lib.check(self._L.smx_evaluate_list(self._h, C.c_void_p(nlist._h), C.c_void_p(base), C.c_void_p(base + 8 * n),
+                                             C.c_void_p(base + 32 * n)))
+        return out[:n], out[n:4 * n].reshape(n, 3), out[4 * n:]
+
     # --- stages --------------------------------------------------------------
     @property
     def zbl(self):

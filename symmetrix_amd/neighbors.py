@@ -263,6 +263,17 @@ def image_shifts(cell, r_cut, pbc=(True, True, True)):
     return np.ascontiguousarray(ints, dtype=np.int32), np.ascontiguousarray(vecs, dtype=np.float64)
 
 
+def _box_lengths(cell):
+    """Edge lengths of an orthorhombic cell given as three lengths or as a diagonal matrix, else None."""
+    cell = np.asarray(cell, dtype=np.float64)
+    if cell.shape != (3,):
+        if cell.shape != (3, 3) or np.count_nonzero(cell) != np.count_nonzero(cell.diagonal()):
+            return None
+        cell = cell.diagonal()
+    lengths = np.ascontiguousarray(cell)
+    return lengths if np.all(lengths > 0.0) and np.all(np.isfinite(lengths)) else None
+
+
 class DeviceNeighborList:
     """The same list built on the GPU from device-resident positions (smx_nlist_* of the C ABI).
 
@@ -277,6 +288,8 @@ class DeviceNeighborList:
         self._C, self._lib = C, _lib
         self._L = _lib.lib()
         self._h = self._L.smx_nlist_create()
+        self._out = (C.c_void_p * 9)()          # addresses of the edge arrays and of the device copies of host inputs
+        self._out_refs = [C.c_void_p(C.addressof(self._out) + q * C.sizeof(C.c_void_p)) for q in range(9)]
         if not self._h:
             raise RuntimeError("smx_nlist_create failed: " + self._L.smx_last_error().decode())
         self.num_atoms = 0
@@ -297,17 +310,14 @@ class DeviceNeighborList:
         except Exception:
             pass
 
-    _names = ("num_neigh", "first_neigh", "neigh_indices", "neigh_types", "neigh_shift", "xyz", "r")
+    _names = ("num_neigh", "first_neigh", "neigh_indices", "neigh_types", "neigh_shift", "xyz", "r", "positions", "node_types")
 
     def _refresh(self, E):
-        C = self._C
+        h, refs = self._C.c_void_p(self._h), self._out_refs
         self.num_edges = int(E)
-        out = [C.c_void_p(0) for _ in self._names]
-        self._lib.check(self._L.smx_nlist_arrays(C.c_void_p(self._h), *[C.byref(o) for o in out]))
-        self.ptr = {n: (o.value or 0) for n, o in zip(self._names, out)}
-        dp, dt = C.c_void_p(0), C.c_void_p(0)
-        self._lib.check(self._L.smx_nlist_inputs(C.c_void_p(self._h), C.byref(dp), C.byref(dt)))
-        self.ptr["positions"], self.ptr["node_types"] = dp.value or 0, dt.value or 0
+        self._lib.check(self._L.smx_nlist_arrays(h, *refs[:7]))
+        self._lib.check(self._L.smx_nlist_inputs(h, *refs[7:]))
+        self.ptr = {n: (p or 0) for n, p in zip(self._names, self._out)}
         return self.num_edges
 
     def build(self, num_atoms, positions_ptr, types_ptr, cell, r_cut, pbc=(True, True, True), skin=0.0, stream=0):
@@ -331,6 +341,9 @@ class DeviceNeighborList:
         """build() from numpy positions [N][3] and species indices [N]; device copies are kept in the list object
         (addresses in .ptr["positions"], .ptr["node_types"])."""
         C = self._C
+        lengths = _box_lengths(cell)
+        if lengths is not None:
+            return self._build_box(positions, types, lengths, r_cut, pbc, skin)
         # folded into the cell: the image shifts below cover one cell span (an update keeps these offsets, so
         # that the remembered pairs stay the same pairs)
         pos, self._wrap = wrap_positions(positions, cell, pbc)
@@ -346,6 +359,24 @@ class DeviceNeighborList:
             C.c_void_p(self._h), len(pos), pos.ctypes.data_as(C.POINTER(C.c_double)), ty.ctypes.data_as(C.POINTER(C.c_int)),
             len(ints), ints.ctypes.data_as(C.POINTER(C.c_int)), vecs.ctypes.data_as(C.POINTER(C.c_double)),
             C.c_double(r_list), C.c_double(r_cut), C.byref(E)))
+        self.num_atoms = len(pos)
+        return self._refresh(E.value)
+
+    def _build_box(self, positions, types, lengths, r_cut, pbc, skin):
+        """build_host for an orthorhombic cell: folding and image shifts on the library's side."""
+        C = self._C
+        pos = np.ascontiguousarray(positions, dtype=np.float64).reshape(-1, 3)
+        ty = np.ascontiguousarray(types, dtype=np.int32)
+        if len(ty) != len(pos):
+            raise ValueError("positions and types differ in length")
+        per = (C.c_int * 3)(*[int(bool(p)) for p in pbc])
+        offsets = np.empty((len(pos), 3), dtype=np.int64)
+        folded, E = C.c_int(0), C.c_long(0)
+        self._lib.check(self._L.smx_nlist_build_box(
+            C.c_void_p(self._h), len(pos), C.c_void_p(pos.ctypes.data), C.c_void_p(ty.ctypes.data),
+            C.c_void_p(lengths.ctypes.data), per, C.c_double(float(r_cut) + float(skin)), C.c_double(r_cut),
+            C.c_void_p(offsets.ctypes.data), C.byref(folded), C.byref(E)))
+        self._wrap, self._cell = offsets, np.diag(lengths)
         self.num_atoms = len(pos)
         return self._refresh(E.value)
 

@@ -832,3 +832,48 @@ def test_layer0_gradients_on_request_follow_the_calls(gpu, tmp_models, dtype):
     eng.compute_node_energies_forces(*H.call_args(ea))
     assert np.array_equal(eng.node_forces, fA) and np.array_equal(eng.node_energies, eA)
     assert np.abs(eng.M0_grad - orc.M0_grad).max() <= tol * max(1.0, np.abs(orc.M0_grad).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("natoms,density,rc,skin", [(1, 0.2, 6.0, 0.0), (512, 0.1, 4.5, 0.0), (513, 0.1, 4.5, 0.0), (700, 0.9, 4.5, 0.0),
+                                                    (200, 0.9, 4.5, 0.3), (600, 0.1, 3.0, 1.5)])
+def test_list_search_at_the_edges_of_its_ways(natoms, density, rc, skin):
+    """All atoms tried (up to 512) or bins, candidates of a receiver ordered in LDS (up to 256) or in memory, lists that
+    outgrow the room first taken, with and without a skin: bit for bit the host builder's, twice on the same object."""
+    from symmetrix_amd import neighbors
+    rng = np.random.default_rng(natoms)
+    cell = np.full(3, (natoms / density) ** (1 / 3)) * np.array([1.0, 1.1, 1 / 1.1])
+    types = rng.integers(0, 3, size=natoms).astype(np.int32)
+    dnl = neighbors.DeviceNeighborList()
+    for rep in range(2):
+        pos = rng.uniform(-0.2, 1.2, size=(natoms, 3)) * cell
+        ref = neighbors.neighbor_list(pos, cell, rc)
+        print(f"{natoms} atoms, {len(ref['r'])} edges", flush=True)
+        E = dnl.build_host(pos, types, cell, rc, skin=skin)
+        got = dnl.to_host()
+        assert E == len(ref["r"])
+        for k in ("i", "j", "S", "xyz", "r", "first_neigh"):
+            assert np.array_equal(got[k], ref[k].reshape(got[k].shape)), k
+        assert np.array_equal(got["neigh_types"], types[ref["j"]])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L_max,K,edge", [(0, 32, 2.6), (0, 32, 1.9), (0, 32, 1.35), (1, 8, 1.9), (1, 8, 1.35)])
+def test_senders_with_many_edges(gpu, tmp_models, L_max, K, edge):
+    """One atom in a small cell is the sender of all edges: buckets that are ordered in LDS, and longer ones."""
+    model = H.tiny_model(K=K, L_max=L_max, n_pts=64, seed=50, r_cut=9.0, pair=False)
+    path = H.write_model(model, tmp_models / f"many{L_max}{K}.json")
+    nl, ea = H.edges_of(np.array([[0.1, 0.2, 0.3]]), np.full(3, edge), np.array([1], dtype=np.int32), 9.0)
+    print(f"{len(ea['r'])} edges", flush=True)
+    orc = _oracle()(model)
+    orc.compute_node_energies_forces(*H.call_args(ea))
+    eng = gpu(path, "float64")
+    eng.compute_node_energies_forces(*H.call_args(ea))
+    assert np.abs(eng.node_energies - orc.node_energies).max() <= 1e-10 * np.abs(orc.node_energies).max()
+    scale = max(1.0, np.abs(orc.node_forces).max())
+    assert np.abs(eng.node_forces - orc.node_forces).max() <= 1e-9 * scale
+    F, V = eng.reduce_forces(1, nl["j"], receiver_atom=np.zeros(1, dtype=np.int32), virial=True)
+    assert np.abs(F).max() <= 1e-9 * scale * len(ea["r"])
+    f, d = orc.node_forces.reshape(-1, 3), ea["xyz"].reshape(-1, 3)
+    W = 0.5 * (d.T @ f + f.T @ d)
+    assert np.abs(V - W[[0, 1, 2, 0, 0, 1], [0, 1, 2, 1, 2, 2]]).max() <= 1e-9 * max(1.0, np.abs(W).max())
