@@ -242,6 +242,8 @@ struct Engine : EngineBase {
     // (empty when the forward table already has that row length, or when the kernel does not apply)
     DVec<F> tabE0, tabE1;
     DVec<F> tabF0, tabF1;   // forward-kernel layout of the same slices (when a slice is 32 bytes of channels)
+    int more_terms1 = 0;       // an entry of layer 1's coupling list has more than two terms
+    int split_nodes = 0;       // receivers that are not ghosts, of the evaluation under way
     bool edge_lanes = false;
     double cdiag1[16] = {};
     DVec<double> fpart;
@@ -341,12 +343,14 @@ struct Engine : EngineBase {
         auto regroup = [&](const std::vector<std::vector<double>>& tables, int nspl, DVec<F>& dst) {
             const int R = hm.spl_nodes - 1, Kc = hm.K, Pn = nspl / Kc;
             std::vector<double> out((size_t)tables.size() * R * nspl * 4);
+            constexpr int V = 16 / sizeof(F);      // coefficients of 16 bytes stay together
             size_t o = 0;
             for (auto& t : tables)
                 for (int n = 0; n < R; ++n)
                     for (int pth = 0; pth < Pn; ++pth)
-                        for (int k = 0; k < Kc; ++k)
-                            for (int q = 0; q < 4; ++q) out[o++] = t[((size_t)n * 4 + q) * nspl + pth * Kc + k];
+                        for (int h = 0; h < 4; h += V)
+                            for (int k = 0; k < Kc; ++k)
+                                for (int q = h; q < h + V; ++q) out[o++] = t[((size_t)n * 4 + q) * nspl + pth * Kc + k];
             upload_as(dst, out, s);
         };
         if (!slice_CH0) regroup(hm.tables0, hm.nspl0, tabK0);
@@ -362,6 +366,7 @@ struct Engine : EngineBase {
         upload_as(B1_start, hm.B_start, s);
         upload_as(B1_lm1, hm.B_lm1, s);
         upload_as(B1_c, hm.B_c, s);
+        for (int b = 0; b < hm.num_B; ++b) more_terms1 |= hm.B_start[b + 1] - hm.B_start[b] > 2;
         upload_as(H2w_H1, hm.H2_weights_for_H1, s);
         upload_as(H2w_M1, hm.H2_weights_for_M1, s);
         upload_as(ro1, hm.readout_1_weights, s);
@@ -713,13 +718,13 @@ struct Engine : EngineBase {
         p.num_nodes = N; p.K = hm.K;
         p.first_neigh = first_neigh.p; p.node_types = node_types; p.neigh_types = neigh_types;
         p.xyz = xyz; p.r = r; p.T = hm.T; p.spl_nodes = hm.spl_nodes; p.spl_h = hm.spl_h; p.spl_inv_h = 1.0 / hm.spl_h;
-        p.num_edges = E;
+        p.num_edges = E; p.split_nodes = split_nodes > 0 ? split_nodes : N;
         if (layer == 0) {
             p.gather = neigh_types; p.Hsrc = H0.p; p.tab = tab0.p; p.tabK = tabK0.p; p.pair_table = pair_table0.p;
-            p.B_start = B0_start.p; p.B_lm1 = B0_lm1.p; p.B_c = B0_c.p; p.num_terms = (int)B0_c.n;
+            p.B_start = B0_start.p; p.B_lm1 = B0_lm1.p; p.B_c = B0_c.p;
         } else {
             p.gather = neigh_indices; p.Hsrc = H1.p; p.tab = tab1.p; p.tabK = tabK1.p; p.pair_table = pair_table1.p;
-            p.B_start = B1_start.p; p.B_lm1 = B1_lm1.p; p.B_c = B1_c.p; p.num_terms = (int)B1_c.n;
+            p.B_start = B1_start.p; p.B_lm1 = B1_lm1.p; p.B_c = B1_c.p; p.more_terms = more_terms1;
         }
         return p;
     }
@@ -1192,7 +1197,7 @@ struct Engine : EngineBase {
         if (on_device) set_geometry_ptrs(N, nt, nn, ni, nty, x, rr, E_, true);
         else upload_inputs(N, nt, nn, ni, nty, x, rr, E_);
         if (N1 < N) E1 = E_local;
-        geo_edges = E_;
+        geo_edges = E_; split_nodes = N1;
         // Range checks come before any kernel that uses these integers as indices: inside the list preparation, whose last
         // launch empties the lists when a check failed (input_guard).  Host arrays are checked the same way and the result
         // is looked at when the call waits for the stream anyway.
@@ -1303,7 +1308,7 @@ struct Engine : EngineBase {
     {
         const std::string s(name);
         energies_copy = nullptr; forces_copy = nullptr;
-        carried_edges = 0; carry_forces = false; fuse_reverse_H1 = false; guard_status = nullptr;
+        carried_edges = 0; carry_forces = false; fuse_reverse_H1 = false; guard_status = nullptr; split_nodes = 0;
         materialise_adjoints(true);
         if (N < 0) throw Error(SMX_EINVAL, "negative num_nodes");
         // A stage may cover the leading nodes of a longer edge list (the pair style runs layer 1 on its local

@@ -30,7 +30,7 @@ struct AggParams {
     const double* r;          // [E]
     const F* Hsrc;            // [rows][NLM][K]
     const F* tab;             // [table][nodes-1][4][P*K]
-    const F* tabK;            // the same numbers with the coefficients of a spline adjacent, [table][nodes-1][P][K][4] (general edge kernels)
+    const F* tabK;            // the same numbers for the general edge kernels: [table][nodes-1][P][K][4], in double [table][nodes-1][P][2][K][2]
     const int* pair_table;    // [T(T+1)/2] -> table
     int T;
     int spl_nodes;
@@ -46,7 +46,8 @@ struct AggParams {
     F* msg;                   // bwd: [E][NLM][K] adjoint message to the sender row, or null
     double* fpart;            // bwd: [channel groups][E][3] partial forces, needed when agg_bwd_groups() > 1
     long num_edges;
-    int num_terms;            // entries of B_lm1 / B_c
+    int more_terms;           // some entry of the coupling list has more than two terms
+    int split_nodes;          // fwd, general kernel: receivers that decide how many wavefronts share one (the local nodes of a call with ghosts)
     // bwd, general kernel only: receivers [node_begin, num_nodes) are processed and the message of edge e goes to
     // row e - msg_edge_begin of msg (edge lists too long for one staging buffer are taken in receiver chunks)
     int node_begin;

@@ -1,18 +1,33 @@
 // Edge kernels for gfx950, general form: fused harmonics + radial splines +
 // receiver-segmented aggregation, and the analytic edge-force adjoint, for any
-// path list (scalar or l <= 1 hidden features) and any number of radial tables.
+// path list (hidden features up to l = 2) and any number of radial tables.
 //
-// Work decomposition.  The edge list is receiver-sorted (CSR).  One wavefront
-// owns one receiver; lane j owns CPL consecutive channels, so every table or
-// feature load of the wavefront is one contiguous run.  Accumulators (NE per
-// channel) live in registers for the whole neighbour loop, so sums run in edge
-// order with no atomics and are bit-reproducible.  Edges are taken in chunks of
-// EC.  Per chunk, the first EC lanes evaluate direction, harmonics and spline
-// interval of one edge each; then all 64 lanes share the EC x NB entries of the
-// Clebsch-Gordan-contracted harmonics B (and their gradients in the adjoint);
-// both go through LDS, from where the channel loop reads them as broadcasts.
-// The four wavefronts of a block share nothing but the coupling list, so the
-// only block-wide barrier is the one after that list is copied to LDS.
+// Work decomposition.  The edge list is receiver-sorted (CSR).  A wavefront owns a
+// receiver, or one of two or four parts of a receiver's edges where there are few
+// receivers; lane j owns channels j, j + 64, ..., so every table or feature load of
+// the wavefront is one contiguous run.  Accumulators (NE per channel) live in
+// registers for the whole neighbour loop and parts are added in a fixed order: no
+// atomics, bit-reproducible.  Edges are taken in chunks of 16: one lane per edge
+// forms direction, harmonics and spline interval; then all 64 lanes share the
+// entries of the Clebsch-Gordan-contracted harmonics B (and their gradients in the
+// adjoint) of a few edges at a time.
+//
+// How B meets the channels.  An entry of B multiplies the value of every channel, so
+// it has to reach all lanes.  Read from LDS as a broadcast it costs 16 to 64 bytes
+// of the LDS pipe's 128 bytes per cycle and lane group, 88 entries of three numbers
+// per edge for l <= 1: with that the LDS bounded the adjoint (3 300 cycles per edge and
+// wavefront in single precision, 5 400 in double).  Now the wavefront holds the block
+// of an edge in a few registers, every lane some of its entries, and the instructions
+// that use them do the broadcast:
+//   single precision  v_mfma_f32_4x4x1_16b: four rows of B times one value per lane in
+//                     8 cycles; the block-broadcast field of the instruction (cbsz = 4,
+//                     abid = n) takes the four rows from lanes 4n .. 4n+3, and result row
+//                     i of channel j lands in register i of lane j, where the vector code
+//                     wants it.  (The matrix pipe does not run beside the vector pipe
+//                     here; per multiply-add it costs the same as a vector instruction.)
+//   double precision  v_fmac_f64 with the row broadcast of its DPP operand (row_newbcast:n),
+//                     at the rate of the plain instruction; every 16-lane row holds the
+//                     block.
 #include "smx_device.hpp"
 #include "smx_kernels.hpp"
 #include "smx_paths.hpp"
@@ -21,99 +36,100 @@ namespace smx {
 
 namespace {
 
+constexpr int kChunk = 16;   // edges whose geometry is formed together
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <typename F>
+constexpr bool kMatrix = sizeof(F) == 4;
+
+// Which entry of B[path][m][m2] (and of its two tangential derivatives) every lane and register holds.
+//   matrix form:  register g / 16, lanes 4 (g % 16) + i hold row 4 tile + i of group g; a group is one matrix
+//                 instruction: (path, row tile, inner index).  Forward: rows m, inner m2; adjoint: rows 3 m2 + t, inner m.
+//   DPP form:     register v / 16, lane v % 16 of every row: v = 3 (boff + m n2 + m2) + t, forward v = boff + m n2 + m2
+template <int LMAXH, bool BWD, bool MATRIX>
+struct BlockLayout {
+    using PT = Paths<LMAXH>;
+    static constexpr int n2(int p) { return 2 * PT::l2(p) + 1; }
+    static constexpr int nm(int p) { return 2 * PT::l(p) + 1; }
+    static constexpr int rows(int p) { return BWD ? 3 * n2(p) : nm(p); }
+    static constexpr int inner(int p) { return BWD ? nm(p) : n2(p); }
+    static constexpr int tiles(int p) { return (rows(p) + 3) / 4; }
+    static constexpr int tile_off(int p)
+    {
+        int n = 0;
+        for (int q = 0; q < p; ++q) n += tiles(q);
+        return n;
+    }
+    static constexpr int group_off(int p)
+    {
+        int n = 0;
+        for (int q = 0; q < p; ++q) n += tiles(q) * inner(q);
+        return n;
+    }
+    static constexpr int group(int p, int tile, int in) { return group_off(p) + tile * inner(p) + in; }
+    static constexpr int TILES = tile_off(PT::P);
+    static constexpr int REGS = MATRIX ? (group_off(PT::P) + 15) / 16 : (PT::NB * (BWD ? 3 : 1) + 15) / 16;
+    static constexpr int LANES = MATRIX ? 64 : 16;      // lanes that hold different entries
+    static constexpr int NV = REGS * LANES;
+    struct Table {
+        short entry[NV];           // index into B, or -1: zero
+        unsigned char comp[NV];    // 0: B, 1, 2: derivative along the first, second tangent
+    };
+    static constexpr Table make()
+    {
+        Table t{};
+        for (int v = 0; v < NV; ++v) { t.entry[v] = -1; t.comp[v] = 0; }
+        for (int p = 0; p < PT::P; ++p) {
+            const int N2 = n2(p), NM = nm(p), bo = PT::boff(p), go = group_off(p), R = rows(p), IN = inner(p);
+            if (MATRIX) {
+                for (int tl = 0; tl < tiles(p); ++tl)
+                    for (int in = 0; in < IN; ++in)
+                        for (int i = 0; i < 4; ++i) {
+                            const int row = 4 * tl + i;
+                            if (row >= R) continue;
+                            const int v = (go + tl * IN + in) * 4 + i;
+                            t.entry[v] = (short)(BWD ? bo + in * N2 + row / 3 : bo + row * N2 + in);
+                            t.comp[v] = (unsigned char)(BWD ? row % 3 : 0);
+                        }
+            } else {
+                for (int b = 0; b < NM * N2; ++b)
+                    for (int c = 0; c < (BWD ? 3 : 1); ++c) {
+                        const int v = BWD ? 3 * (bo + b) + c : bo + b;
+                        t.entry[v] = (short)(bo + b);
+                        t.comp[v] = (unsigned char)c;
+                    }
+            }
+        }
+        return t;
+    }
+};
+template <int LMAXH, bool BWD, bool MATRIX>
+__device__ const typename BlockLayout<LMAXH, BWD, MATRIX>::Table block_table = BlockLayout<LMAXH, BWD, MATRIX>::make();
+
+// LDS of a block: the coefficients of the block entries, then a part for each of its four wavefronts
 template <typename F, int LMAXH, bool BWD>
-struct WaveLds {
-    using PT = Paths<LMAXH>;
-    static constexpr int NBP = (PT::NB + 3) / 4 * 4;          // B row padded for 16-byte reads
-    static constexpr int NY = BWD ? 64 : 16;                  // Y (and dY/dx, dY/dy, dY/dz)
-    static constexpr int NBT = BWD ? 4 * NBP : NBP;
-    __host__ __device__ static constexpr size_t per_wave(int EC)
-    {
-        size_t b = (size_t)EC * (NY * sizeof(double) + (BWD ? 12 * sizeof(double) : 0) + NBT * sizeof(F));
-        b += (size_t)EC * (sizeof(double) + 2 * sizeof(int));   // x (held as double-sized slot), rows, gather rows
-        return (b + 15) / 16 * 16;
-    }
-    // Double-precision forward kernel with vector sender features: the coefficients of the first PRE paths of the
-    // next edge wait in LDS, brought there by loads that bypass the registers (32 bytes per lane and path).
-    static constexpr bool PREFETCH = !BWD && sizeof(F) == 8 && LMAXH == 1;
-    static constexpr int PRE = PREFETCH ? PT::P / 2 : 0;
-    __host__ __device__ static constexpr size_t prefetch_per_wave() { return (size_t)PRE * 64 * 32; }
-    __host__ __device__ static constexpr size_t lists(int num_terms)
-    {
-        return ((size_t)num_terms * (sizeof(double) + sizeof(int)) + (PT::NB + 1) * sizeof(int) + 15) / 16 * 16;
-    }
+struct EdgeLds {
+    using BL = BlockLayout<LMAXH, BWD, kMatrix<F>>;
+    static constexpr int NY = BWD ? 48 : 16;     // harmonics (and their two tangential derivatives) of an edge
+    // edges whose blocks are in LDS at a time: as many as leave room for two thread blocks on a CU
+    static constexpr int SUB = BL::NV * (int)sizeof(F) > 3000 ? 2 : (BL::NV * (int)sizeof(F) > 1000 ? 4 : 8);
+    static constexpr size_t lists = ((size_t)BL::NV * (2 * sizeof(double) + sizeof(int)) + 15) / 16 * 16;
+    static constexpr size_t y_bytes = (size_t)kChunk * NY * sizeof(double);
+    static constexpr size_t frame_bytes = BWD ? (size_t)kChunk * 10 * sizeof(double) : 0;    // direction over r, tangents
+    static constexpr size_t head_bytes = (size_t)(kChunk + 1) * (sizeof(double) + 2 * sizeof(int)) + 8;  // x, table row, sender row
+    static constexpr size_t sum_bytes = BWD ? (size_t)kChunk * 4 * sizeof(F) : 0;
+    static constexpr size_t block_bytes = (size_t)SUB * BL::NV * sizeof(F);
+    static constexpr size_t per_wave = (y_bytes + frame_bytes + head_bytes + sum_bytes + block_bytes + 15) / 16 * 16;
+    static constexpr size_t total = lists + 4 * per_wave;
 };
 
-// The steps in which the adjoint kernel walks the coupling block B[path][m][m2] of an edge.  Wide steps (single
-// precision): all rows m of a path with a scalar sender feature, three rows at a time of a path with a vector one
-// (at most nine entries).  Narrow steps (double precision, where an entry takes eight registers): at most three
-// entries, i.e. three rows of a scalar path or one row of a vector path.
-template <int LMAXH, bool NARROW>
-struct BwdSteps {
-    using PT = Paths<LMAXH>;
-    static constexpr int rows(int p) { return 2 * PT::l(p) + 1; }
-    static constexpr int group(int p)
-    {
-        if (NARROW) return PT::l2(p) == 0 ? (rows(p) < 3 ? rows(p) : 3) : 1;
-        return PT::l2(p) == 0 ? rows(p) : (PT::l2(p) == 1 ? 3 : 1);
-    }
-    static constexpr int groups(int p) { return (rows(p) + group(p) - 1) / group(p); }
-    static constexpr int count()
-    {
-        int n = 0;
-        for (int p = 0; p < PT::P; ++p) n += groups(p);
-        return n;
-    }
-    static constexpr int path(int s)
-    {
-        for (int p = 0; p < PT::P; ++p) {
-            if (s < groups(p)) return p;
-            s -= groups(p);
-        }
-        return -1;
-    }
-    static constexpr int m0(int s)
-    {
-        for (int p = 0; p < PT::P; ++p) {
-            if (s < groups(p)) return s * group(p);
-            s -= groups(p);
-        }
-        return -1;
-    }
-    static constexpr int m1(int s)
-    {
-        const int p = path(s), e = m0(s) + group(p);
-        return e < rows(p) ? e : rows(p);
-    }
-    static constexpr int len(int s) { return (m1(s) - m0(s)) * (2 * PT::l2(path(s)) + 1); }
-    static constexpr int max_len()
-    {
-        int n = 0;
-        for (int s = 0; s < count(); ++s) n = len(s) > n ? len(s) : n;
-        return n;
-    }
-    static constexpr int MAXLEN = max_len();
-};
-
-// Everything addressed through boffs after this point is scheduled after the three sums are final.
-template <typename F>
-__device__ __forceinline__ void order_after(F& g1, F& g2, F& srad, int& boffs)
+// Lane-broadcast multiply-add of the double-precision kernels: acc += (b of lane N of the lane's 16-lane row) * v.  The
+// instruction reads b through DPP: b must not come from the vector instruction right before (here it comes from LDS).
+template <int N>
+__device__ __forceinline__ void fmac_lane(double& acc, double b, double v)
 {
-    asm volatile("" : "+v"(g1), "+v"(g2), "+v"(srad), "+v"(boffs));
-}
-
-// The value is final here: keeps an accumulation from drifting past the fences (its operands would stay live).
-template <typename F>
-__device__ __forceinline__ void pin(F& v)
-{
-    asm volatile("" : "+v"(v));
-}
-
-// v is final here, and what is addressed through off afterwards is not loaded before
-template <typename F>
-__device__ __forceinline__ void tie(F& v, int& off)
-{
-    asm volatile("" : "+v"(v), "+v"(off));
+    asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(b), "v"(v), "n"(N));
 }
 
 template <typename F, int CPL>
@@ -122,253 +138,355 @@ __device__ __forceinline__ Vec<F, CPL> ldv(const F* p)
     return *reinterpret_cast<const Vec<F, CPL>*>(p);
 }
 
-// Entry b of the coupling block, B[b] = sum_t c_t Y[lm1_t], as one lane holds it for the whole kernel: lane L owns the
-// entries L and L + 64.  The first two terms sit in registers (most entries have one or two); further terms, if a
-// model file has them, are read from the lists in LDS.
-struct BlockEntry {
-    double c0, c1;
-    int l0, l1, t2, t_end;
-};
-__device__ __forceinline__ BlockEntry block_entry(int b, int NB, const int* cg_start, const double* cg_c, const int* cg_lm1)
+// Loads and stores of a wavefront's rows: an address that is the same for all lanes, held in scalar registers, plus a 32-bit
+// offset per lane.
+template <typename T>
+__device__ __forceinline__ T load_at(const char* row, unsigned lane_bytes)
 {
-    BlockEntry e{0.0, 0.0, 0, 0, 0, 0};
-    if (b < NB) {
-        const int s0 = cg_start[b], s1 = cg_start[b + 1];
-        if (s1 > s0) { e.c0 = cg_c[s0]; e.l0 = cg_lm1[s0]; e.l1 = e.l0; }
-        if (s1 > s0 + 1) { e.c1 = cg_c[s0 + 1]; e.l1 = cg_lm1[s0 + 1]; }
-        e.t2 = s0 + 2 < s1 ? s0 + 2 : s1;
-        e.t_end = s1;
+    return *reinterpret_cast<const T*>(row + lane_bytes);
+}
+// The four coefficients of one spline: 16 bytes in single precision, two halves of 16 bytes in double (a table row is
+// [path][half][K][16 bytes], so that every load instruction of a wavefront covers 1 KB without gaps).
+template <typename F>
+__device__ __forceinline__ Vec<F, 4> load_spline(const char* row, int path, unsigned K, unsigned k)
+{
+    if constexpr (sizeof(F) == 4) return load_at<Vec<F, 4>>(row + path * (K * 16), k * 16);
+    else {
+        Vec<F, 4> c;
+        const Vec<F, 2> lo = load_at<Vec<F, 2>>(row + 2 * path * (K * 16), k * 16);
+        const Vec<F, 2> hi = load_at<Vec<F, 2>>(row + (2 * path + 1) * (K * 16), k * 16);
+        c.v[0] = lo.v[0]; c.v[1] = lo.v[1]; c.v[2] = hi.v[0]; c.v[3] = hi.v[1];
+        return c;
     }
-    return e;
+}
+// row n of an array of rows of that many bytes, n the same in all lanes
+__device__ __forceinline__ const char* uniform_row(const void* base, int n, unsigned row_bytes)
+{
+    return reinterpret_cast<const char*>(base) + (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(n) * row_bytes;
+}
+// The value is final here: keeps the compiler from collecting the arithmetic of several paths, whose operands would all stay
+// live (it moves plain arithmetic across scheduling fences).
+template <typename F>
+__device__ __forceinline__ void pin(F& v)
+{
+    asm volatile("" : "+v"(v));
+}
+
+// Three sums over the 64 lanes at once: on return the lanes of row 0 hold the first, of row 2 the second, of rows 1 and 3
+// the third (a fixed tree).  Two values swap halves of the wavefront and are added, which sums both over the halves.
+template <typename F>
+__device__ __forceinline__ void swap_halves(F& a, F& b)
+{
+    if constexpr (sizeof(F) == 4) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+    } else {
+        const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+        const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+        a = __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]);
+        b = __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
+    }
+}
+template <typename F>
+__device__ __forceinline__ void swap_rows(F& a, F& b)
+{
+    if constexpr (sizeof(F) == 4) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+    } else {
+        const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+        const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+        a = __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]);
+        b = __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
+    }
+}
+template <typename F>
+__device__ __forceinline__ F wave_sum3(F s, F g1, F g2)
+{
+    F zero = g2;
+    swap_halves(s, g1);
+    const F a = s + g1;              // rows 0, 1: s; rows 2, 3: g1
+    swap_halves(g2, zero);
+    F x = a, y = g2 + zero;          // every row: g2
+    swap_rows(x, y);
+    return row_sum_strided<1>(x + y);
+}
+
+// What the lanes need of an edge before its features: spline interval and argument, table row, sender row.
+template <typename F>
+__device__ __forceinline__ void edge_head(const AggParams<F>& a, int e, int ti, double& r, double& x, int& row, int& grow)
+{
+    r = a.r[e];
+    const int n = spline_interval(r, a.spl_inv_h, a.spl_nodes - 2);
+    x = r - a.spl_h * n;
+    row = a.pair_table[pair_index(a.T, ti, a.neigh_types[e])] * (a.spl_nodes - 1) + n;
+    grow = a.gather[e];
+}
+
+// The coefficients of the block entries: value v = c0 Y[o0] + c1 Y[o1] (an entry of a real coupling has at most two terms;
+// a file with longer ones sets more_terms and pays for a loop), copied to LDS once per thread block.
+template <int LMAXH, bool BWD, bool MATRIX, typename F>
+__device__ __forceinline__ void block_lists(const AggParams<F>& a, double* coef, int* offs)
+{
+    using BL = BlockLayout<LMAXH, BWD, MATRIX>;
+    for (int v = threadIdx.x; v < BL::NV; v += 256) {
+        const int b = block_table<LMAXH, BWD, MATRIX>.entry[v], comp = block_table<LMAXH, BWD, MATRIX>.comp[v];
+        double c0 = 0.0, c1 = 0.0;
+        int o0 = 0, o1 = 0;
+        if (b >= 0) {
+            const int s0 = a.B_start[b], s1 = a.B_start[b + 1];
+            if (s1 > s0) { c0 = a.B_c[s0]; o0 = a.B_lm1[s0]; }
+            if (s1 > s0 + 1) { c1 = a.B_c[s0 + 1]; o1 = a.B_lm1[s0 + 1]; }
+        }
+        coef[2 * v] = c0; coef[2 * v + 1] = c1;
+        offs[v] = (comp * 16 + o0) | ((comp * 16 + o1) << 16);
+    }
+}
+template <int LMAXH, bool BWD, bool MATRIX, typename F, int NY, int SUB>
+__device__ __forceinline__ void block_values(const AggParams<F>& a, const double* coef, const int* offs, const double* Yt, int ns,
+                                             F* vals, int lane)
+{
+    using BL = BlockLayout<LMAXH, BWD, MATRIX>;
+#pragma unroll
+    for (int j = 0; j < (BL::NV + 63) / 64; ++j) {
+        const int v = lane + 64 * j;
+        if (BL::NV % 64 == 0 || v < BL::NV) {
+            const double c0 = coef[2 * v], c1 = coef[2 * v + 1];
+            const int o = offs[v], o0 = o & 0xffff, o1 = o >> 16;
+#pragma unroll
+            for (int le = 0; le < SUB; ++le)      // (past the chunk's last edge: numbers nobody reads)
+                vals[le * BL::NV + v] = (F)(c0 * Yt[le * NY + o0] + c1 * Yt[le * NY + o1]);
+        }
+    }
+    if (a.more_terms) {
+        for (int v = lane; v < BL::NV; v += 64) {
+            const int b = block_table<LMAXH, BWD, MATRIX>.entry[v];
+            if (b < 0) continue;
+            for (int le = 0; le < ns; ++le) {
+                const double* y = Yt + le * NY + (offs[v] & 0xfff0);
+                double s = 0.0;
+                for (int t = a.B_start[b]; t < a.B_start[b + 1]; ++t) s += a.B_c[t] * y[a.B_lm1[t]];
+                vals[le * BL::NV + v] = (F)s;
+            }
+        }
+    }
+}
+
+// Thread blocks per CU (wavefronts per SIMD) the kernels are compiled for: 128 to 512 registers a lane.  In double precision
+// an l = 2 edge holds 71 sums and 46 block registers, twice as wide, and has the SIMD for itself.
+template <typename F, int LMAXH, int CPL, bool BWD>
+constexpr int agg_blocks()
+{
+    if (LMAXH >= 2) return sizeof(F) == 8 ? 1 : 2;
+    if (LMAXH == 1 && sizeof(F) == 4 && CPL == 1) return 3;
+    return 2;
 }
 
 // ---------------------------------------------------------------------------
-// (Hidden features up to l = 2: 17 paths and 71 sums per channel.  Those instantiations take one block per CU, so
-// that a wavefront has the whole register file of its SIMD.)
-template <typename F, int LMAXH, int CPL, int EC>
-__global__ __launch_bounds__(256, LMAXH >= 2 ? 1 : 2) void k_agg_fwd(const AggParams<F> a, const int num_terms)
+// Forward: out[i, lme, k] = sum over the edges of R_path(r)[k] sum_m2 B[lme, m2] H[sender, m2, k].
+// Bound by the coefficient rows: P splines of 16 (32) bytes per channel and edge, 10 KB (20 KB) per edge and wavefront at
+// l <= 1, of the 64 bytes per cycle that a CU's vector cache hands out.
+template <typename F, int LMAXH, int CPL>
+__global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_agg_fwd(const AggParams<F> a, const int parts)
 {
+    constexpr bool MX = kMatrix<F>;
     using PT = Paths<LMAXH>;
-    using WL = WaveLds<F, LMAXH, false>;
-    constexpr int NB = PT::NB, NBP = WL::NBP, NE = PT::NE, P = PT::P, NLM = PT::NLM;
+    using BL = BlockLayout<LMAXH, false, MX>;
+    using EL = EdgeLds<F, LMAXH, false>;
+    constexpr int NE = PT::NE, P = PT::P, NLM = PT::NLM, SUB = EL::SUB;
+    constexpr int W = P <= 5 ? P : 5;     // splines of the ring: requested W paths ahead
     extern __shared__ __align__(16) unsigned char smem[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    double* cg_c = reinterpret_cast<double*>(smem);                               // [num_terms]
-    int* cg_lm1 = reinterpret_cast<int*>(cg_c + num_terms);                       // [num_terms]
-    int* cg_start = cg_lm1 + num_terms;                                           // [NB+1]
-    unsigned char* base = smem + WL::lists(num_terms) + (size_t)wave * WL::per_wave(EC);
-    double* Yt = reinterpret_cast<double*>(base);                                 // [EC][16]
-    double* xs = Yt + EC * 16;                                                    // [EC]
-    F* Bs = reinterpret_cast<F*>(xs + EC);                                        // [EC][NBP]
-    int* rows = reinterpret_cast<int*>(Bs + EC * NBP);                            // [EC]
-    int* grows = rows + EC;                                                       // [EC]
+    double* coef = reinterpret_cast<double*>(smem);
+    int* offs = reinterpret_cast<int*>(coef + 2 * BL::NV);
+    unsigned char* base = smem + EL::lists + (size_t)wave * EL::per_wave;
+    double* Yt = reinterpret_cast<double*>(base);                                 // [kChunk][16]
+    F* vals = reinterpret_cast<F*>(base + EL::y_bytes);                           // [SUB][NV]
+    double* xs = reinterpret_cast<double*>(base + EL::y_bytes + EL::block_bytes); // [kChunk + 1]
+    int* rows = reinterpret_cast<int*>(xs + kChunk + 1);                          // [kChunk + 1]
+    int* grows = rows + kChunk + 1;                                               // [kChunk + 1]
 
-    for (int t = threadIdx.x; t < num_terms; t += 256) { cg_c[t] = a.B_c[t]; cg_lm1[t] = a.B_lm1[t]; }
-    for (int t = threadIdx.x; t <= NB; t += 256) cg_start[t] = a.B_start[t];
+    block_lists<LMAXH, false, MX>(a, coef, offs);
     __syncthreads();
-    // lane-owned entries of the coupling block: measured faster in double precision; in single precision their
-    // registers cost a wavefront per SIMD and the kernel runs 15 % slower
-    constexpr bool OWNED = sizeof(F) == 8;
-    constexpr int NSLOT = OWNED ? (NB + 63) / 64 : 1;
-    BlockEntry ent[NSLOT];
-    if constexpr (OWNED) {
-#pragma unroll
-        for (int j = 0; j < NSLOT; ++j) ent[j] = block_entry(lane + 64 * j, NB, cg_start, cg_c, cg_lm1);
-    }
 
-    const int K = a.K;
+    const unsigned K = (unsigned)a.K;
     // One-dimensional grid, channel group fastest: consecutive blocks go to the dies in turn, so a die only ever
     // works on the channel groups congruent to its number and its L2 holds that share of the spline table alone
     // (half of it at two groups of 64 channels).
-    const int groups = (K + 64 * CPL - 1) / (64 * CPL);
+    const int groups = (a.K + 64 * CPL - 1) / (64 * CPL);
     const int cgroup = blockIdx.x % groups;
-    const int i = (blockIdx.x / groups) * 4 + wave;
-    if (i >= a.num_nodes) return;
-    const int k0 = (cgroup * 64 + lane) * CPL;
-    const bool active = k0 < K;
-    const int e0 = a.first_neigh[i], e1 = a.first_neigh[i + 1], ti = a.node_types[i];
+    const int unit = (blockIdx.x / groups) * 4 + wave;
+    const int i = __builtin_amdgcn_readfirstlane(unit / parts), part = unit - i * parts;
+    const bool real = i < a.num_nodes;
+    unsigned k[CPL];
+    bool active[CPL];
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+        const int ch = (cgroup * CPL + c) * 64 + lane;
+        active[c] = ch < a.K;
+        k[c] = active[c] ? (unsigned)ch : 0u;      // lanes beyond the last channel repeat channel 0 and store nothing
+    }
+    int e0 = 0, e1 = 0, ti = 0;
+    if (real) {
+        const int b = a.first_neigh[i], n = a.first_neigh[i + 1] - b;
+        e0 = b + (int)((long)n * part / parts); e1 = b + (int)((long)n * (part + 1) / parts);
+        ti = a.node_types[i];
+    }
+    e0 = __builtin_amdgcn_readfirstlane(e0); e1 = __builtin_amdgcn_readfirstlane(e1);
 
-    F acc[CPL][NE];
+    f32x4 tile[MX ? CPL : 1][MX ? BL::TILES : 1];
+    F acc[MX ? 1 : CPL][MX ? 1 : NE];
 #pragma unroll
-    for (int c = 0; c < CPL; ++c)
+    for (int c = 0; c < CPL; ++c) {
+        if constexpr (MX) {
 #pragma unroll
-        for (int q = 0; q < NE; ++q) acc[c][q] = F(0);
-
-    for (int eb = e0; eb < e1; eb += EC) {
-        const int nE = min(EC, e1 - eb);
-        wave_lds_sync();
-        if (lane < nE) {
-            const int e = eb + lane;
-            const double dx = a.xyz[3 * (size_t)e], dy = a.xyz[3 * (size_t)e + 1], dz = a.xyz[3 * (size_t)e + 2];
-            const double inv = rsqrt_pos(dx * dx + dy * dy + dz * dz);
-            double Y[16];
-            sph_l3(dz * inv, dx * inv, dy * inv, Y);
-#pragma unroll
-            for (int q = 0; q < 16; ++q) Yt[lane * 16 + q] = Y[q];
-            const double r = a.r[e];
-            const int n = spline_interval(r, a.spl_inv_h, a.spl_nodes - 2);
-            xs[lane] = r - a.spl_h * n;
-            const int tbl = a.pair_table[pair_index(a.T, ti, a.neigh_types[e])];
-            rows[lane] = tbl * (a.spl_nodes - 1) + n;
-            grows[lane] = a.gather[e];
-        }
-        wave_lds_sync();
-        if constexpr (OWNED) {
-#pragma unroll
-            for (int j = 0; j < NSLOT; ++j) {
-                const int b = lane + 64 * j;
-                if (b < NB) {
-                    const BlockEntry& en = ent[j];
-                    for (int le = 0; le < nE; ++le) {
-                        const double* y = Yt + le * 16;
-                        double s = en.c0 * y[en.l0] + en.c1 * y[en.l1];
-                        for (int t = en.t2; t < en.t_end; ++t) s += cg_c[t] * y[cg_lm1[t]];
-                        Bs[le * NBP + b] = (F)s;
-                    }
-                }
-            }
+            for (int q = 0; q < BL::TILES; ++q) tile[c][q] = f32x4{0, 0, 0, 0};
         } else {
-            for (int it = lane; it < nE * NB; it += 64) {
-                const int le = it / NB, b = it - le * NB;
-                double s = 0.0;
-                for (int t = cg_start[b]; t < cg_start[b + 1]; ++t) s += cg_c[t] * Yt[le * 16 + cg_lm1[t]];
-                Bs[le * NBP + b] = (F)s;
+#pragma unroll
+            for (int q = 0; q < NE; ++q) acc[c][q] = F(0);
+        }
+    }
+
+    Vec<F, 4> cf[CPL][W];
+    F H[CPL][NLM], Hn[CPL][NLM];
+    const unsigned row_bytes = P * K * 4 * sizeof(F), sender_bytes = NLM * K * sizeof(F);
+    auto request_spline = [&](const char* row, int path) {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) cf[c][path % W] = load_spline<F>(row, path, K, k[c]);
+    };
+    auto request_sender = [&](int le) {
+        const char* row = uniform_row(a.Hsrc, grows[le], sender_bytes);
+#pragma unroll
+        for (int c = 0; c < CPL; ++c)
+#pragma unroll
+            for (int q = 0; q < NLM; ++q) Hn[c][q] = load_at<F>(row + q * (K * sizeof(F)), k[c] * sizeof(F));
+    };
+    const char* cur = nullptr;      // table row of the edge under way
+    for (int eb = e0; eb < e1; eb += kChunk) {
+        const int nE = min(kChunk, e1 - eb);
+        wave_lds_sync();
+        if (lane <= nE) {
+            // lane nE: the first edge of the next chunk, whose features are requested at the end of this one
+            // (past the last edge of the part: the last one again)
+            const int e = min(eb + lane, e1 - 1);
+            double r, x;
+            int row, grow;
+            edge_head(a, e, ti, r, x, row, grow);
+            xs[lane] = x; rows[lane] = row; grows[lane] = grow;
+            if (lane < nE) {
+                const double dx = a.xyz[3 * (size_t)e], dy = a.xyz[3 * (size_t)e + 1], dz = a.xyz[3 * (size_t)e + 2];
+                const double inv = rsqrt_pos(dx * dx + dy * dy + dz * dz);
+                double Y[16];
+                sph_l3(dz * inv, dx * inv, dy * inv, Y);
+#pragma unroll
+                for (int q = 0; q < 16; ++q) Yt[lane * 16 + q] = Y[q];
             }
         }
         wave_lds_sync();
-        if (!active) continue;
-        // Spline coefficients (P x CPL 16-byte loads, contiguous across the lanes for one path) and the sender
-        // row of an edge.  In single precision those of the next edge are requested while the current edge is
-        // worked on (AHEAD).  In double precision there are registers for half of that at most (HALF: the first
-        // five paths and the sender row requested an edge ahead, the other five at the start of the edge).
-        constexpr bool AHEAD = sizeof(F) == 4 && (CPL == 1 || LMAXH == 0) && LMAXH <= 1;
-        constexpr bool HALF = false;   // measured slower than requesting all ten at the start of the edge (10.4 against 9.1 ms)
-        constexpr int PA = HALF ? P / 2 : P;     // paths of the first part
-        Vec<F, 4> cf[P][CPL];
-        Vec<F, CPL> H[NLM];
-        auto request = [&](int le_, auto first, auto last, bool sender) {
-            constexpr int p0 = decltype(first)::value, p1 = decltype(last)::value;
-            const int row = __builtin_amdgcn_readfirstlane(rows[le_]);
-            const F* rowp = a.tabK + ((size_t)row * P * K + k0) * 4;
-            if (sender) {
-                const int grow = __builtin_amdgcn_readfirstlane(grows[le_]);
-                const F* Hp = a.Hsrc + (size_t)grow * NLM * K + k0;
-#pragma unroll
-                for (int q = 0; q < NLM; ++q) H[q] = ldv<F, CPL>(Hp + q * K);
-            }
-#pragma unroll
-            for (int q = p0; q < p1; ++q)
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) cf[q][c] = ldv<F, 4>(rowp + ((size_t)q * K + c) * 4);
-        };
-        constexpr std::integral_constant<int, 0> c0{};
-        constexpr std::integral_constant<int, PA> cA{};
-        constexpr std::integral_constant<int, P> cP{};
-        if ((AHEAD || HALF) && nE > 0) request(0, c0, cA, true);
-        F w[P][CPL][2 * LMAXH + 1];   // radial value times sender feature per path and sender component
-        auto products = [&](F x, auto first, auto last) {
-            static_for<decltype(first)::value, decltype(last)::value>([&](auto qc) {
-                constexpr int q = decltype(qc)::value, l2 = PT::l2(q);
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) {
-                    const Vec<F, 4> k4 = cf[q][c];
-                    const F R = k4.v[0] + x * (k4.v[1] + x * (k4.v[2] + x * k4.v[3]));
-#pragma unroll
-                    for (int m2 = 0; m2 < 2 * l2 + 1; ++m2) w[q][c][m2] = R * H[l2 * l2 + m2].v[c];
-                }
-            });
-        };
-        // coefficient buffer of this wavefront: [PRE paths][2 halves][64 lanes] 16-byte words
-        unsigned char* pre = smem + WL::lists(num_terms) + 4 * WL::per_wave(EC) + (size_t)wave * WL::prefetch_per_wave();
-        constexpr int PRE = WL::PRE;
-        Vec<F, CPL> Hn[NLM];
-        auto request_lds = [&](int le_) {
-            typedef const __attribute__((address_space(1))) void* GlobalPtr;
-            typedef __attribute__((address_space(3))) void* LdsPtr;
-            const int row = __builtin_amdgcn_readfirstlane(rows[le_]);
-            const char* rowp = reinterpret_cast<const char*>(a.tabK + ((size_t)row * P * K + k0) * 4);
-#pragma unroll
-            for (int q = 0; q < PRE; ++q) {
-                const char* src = rowp + (size_t)q * K * 4 * sizeof(F);
-                __builtin_amdgcn_global_load_lds((GlobalPtr)src, (LdsPtr)(pre + (q * 2) * 1024), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds((GlobalPtr)(src + 16), (LdsPtr)(pre + (q * 2 + 1) * 1024), 16, 0, 0);
-            }
-            const int grow = __builtin_amdgcn_readfirstlane(grows[le_]);
-            const F* Hp = a.Hsrc + (size_t)grow * NLM * K + k0;
-#pragma unroll
-            for (int q = 0; q < NLM; ++q) Hn[q] = ldv<F, CPL>(Hp + q * K);
-        };
-        if constexpr (WL::PREFETCH) {
-            if (nE > 0) { request_lds(0); request(0, std::integral_constant<int, PRE>{}, std::integral_constant<int, P>{}, false); }
+        if (eb == e0) {
+            cur = uniform_row(a.tabK, rows[0], row_bytes);
+            static_for<0, W>([&](auto qc) { request_spline(cur, decltype(qc)::value); });
+            request_sender(0);
         }
-        for (int le = 0; le < nE; ++le) {
-            const F x = (F)xs[le];
-            const F* B = Bs + le * NBP;
-            auto accumulate = [&](auto pc) {
-                constexpr int p = decltype(pc)::value;
-                constexpr int l = PT::l(p), l2 = PT::l2(p), bo = PT::boff(p);
-                constexpr int lme0 = PT::lme(p, 0), es = PT::num_e(l), n2 = 2 * l2 + 1;
-                F Bv[(2 * l + 1) * n2];
+        for (int sb = 0; sb < nE; sb += SUB) {
+            const int ns = min(SUB, nE - sb);
+            if (sb) wave_lds_sync();
+            block_values<LMAXH, false, MX, F, 16, SUB>(a, coef, offs, Yt + sb * 16, ns, vals, lane);
+            wave_lds_sync();
+            for (int le = sb; le < sb + ns; ++le) {
+                const F x = (F)xs[le];
+                F B[BL::REGS];
 #pragma unroll
-                for (int q = 0; q < (2 * l + 1) * n2; ++q) Bv[q] = B[bo + q];
+                for (int j = 0; j < BL::REGS; ++j) B[j] = vals[(le - sb) * BL::NV + j * BL::LANES + (lane & (BL::LANES - 1))];
 #pragma unroll
-                for (int c = 0; c < CPL; ++c) {
+                for (int c = 0; c < CPL; ++c)
 #pragma unroll
-                    for (int m = 0; m < 2 * l + 1; ++m) {
-                        F z = acc[c][lme0 + m * es];
+                    for (int q = 0; q < NLM; ++q) H[c][q] = Hn[c][q];
+                request_sender(le + 1);
+                const char* next = uniform_row(a.tabK, rows[le + 1], row_bytes);
+                static_for<0, P>([&](auto pc) {
+                    constexpr int p = decltype(pc)::value, l = PT::l(p), l2 = PT::l2(p), n2 = 2 * l2 + 1;
+                    F w[CPL][n2];
 #pragma unroll
-                        for (int m2 = 0; m2 < n2; ++m2) z += Bv[m * n2 + m2] * w[p][c][m2];
-                        acc[c][lme0 + m * es] = z;
+                    for (int c = 0; c < CPL; ++c) {
+                        const Vec<F, 4> k4 = cf[c][p % W];
+                        const F R = k4.v[0] + x * (k4.v[1] + x * (k4.v[2] + x * k4.v[3]));
+#pragma unroll
+                        for (int m2 = 0; m2 < n2; ++m2) w[c][m2] = R * H[c][l2 * l2 + m2];
                     }
-                }
-            };
-            // requests for a following edge are unconditional (the last edge of a chunk asks for its own operands
-            // again): a conditional request makes the values carried round the loop a merge of old and new registers,
-            // which costs a register copy per value
-            const int le_next = le + 1 < nE ? le + 1 : le;
-            if constexpr (WL::PREFETCH) {
-                constexpr std::integral_constant<int, PRE> cPre{};
-                // first paths from the buffer (filled while the previous edge was worked on), sender row likewise
+                    if constexpr (p + W < P) request_spline(cur, p + W); else request_spline(next, p % W);
+                    if constexpr (MX) {
+                        static_for<0, n2>([&](auto mc) {
+                            static_for<0, BL::tiles(p)>([&](auto tc) {
+                                constexpr int g = BL::group(p, decltype(tc)::value, decltype(mc)::value), t = BL::tile_off(p) + decltype(tc)::value;
 #pragma unroll
-                for (int q = 0; q < NLM; ++q) H[q] = Hn[q];
+                                for (int c = 0; c < CPL; ++c)
+                                    tile[c][t] = __builtin_amdgcn_mfma_f32_4x4x1f32(B[g / 16], w[c][decltype(mc)::value], tile[c][t], 4, g % 16, 0);
+                            });
+                        });
+                    } else {
+                        constexpr int bo = PT::boff(p), lme0 = PT::lme(p, 0), es = PT::num_e(l);
+                        static_for<0, n2>([&](auto mc) {
+                            static_for<0, 2 * l + 1>([&](auto rc) {
+                                constexpr int v = bo + decltype(rc)::value * n2 + decltype(mc)::value;
 #pragma unroll
-                for (int q = 0; q < PRE; ++q) {
-                    const Vec<F, 2> lo = *reinterpret_cast<const Vec<F, 2>*>(pre + (q * 2) * 1024 + lane * 16);
-                    const Vec<F, 2> hi = *reinterpret_cast<const Vec<F, 2>*>(pre + (q * 2 + 1) * 1024 + lane * 16);
-                    cf[q][0].v[0] = lo.v[0]; cf[q][0].v[1] = lo.v[1]; cf[q][0].v[2] = hi.v[0]; cf[q][0].v[3] = hi.v[1];
-                }
-                products(x, c0, cPre);
-                static_for<0, PRE>(accumulate);
-                products(x, cPre, cP);                    // the other paths came through registers, requested an edge ago
-                // the next edge's operands: first paths into the buffer (these requests are the older ones, so the
-                // wait for them at the top of the next edge leaves the register loads in flight), the rest into the
-                // registers the products above have just freed
-                request_lds(le_next);
-                request(le_next, cPre, cP, false);
-                static_for<PRE, P>(accumulate);
-                continue;
-            }
-            if (!AHEAD && !HALF) request(le, c0, cP, true);
-            if (HALF) request(le, cA, cP, false);
-            products(x, c0, cA);
-            if (AHEAD) request(le_next, c0, cP, true);
-            static_for<0, PA>(accumulate);
-            if constexpr (HALF) {
-                products(x, cA, cP);
-                request(le_next, c0, cA, true);
-                static_for<PA, P>(accumulate);
+                                for (int c = 0; c < CPL; ++c)
+                                    fmac_lane<v % 16>(acc[c][lme0 + decltype(rc)::value * es], B[v / 16], w[c][decltype(mc)::value]);
+                            });
+                        });
+                    }
+                    // path by path
+                    if constexpr (MX) {
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                            for (int t = BL::tile_off(p); t < BL::tile_off(p) + BL::tiles(p); ++t) pin(tile[c][t]);
+                        __builtin_amdgcn_sched_group_barrier(0x002, (3 + n2) * CPL, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x008, BL::tiles(p) * n2 * CPL, 0);
+                    } else {
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                            for (int m = 0; m < 2 * l + 1; ++m) pin(acc[c][PT::lme(p, 0) + m * PT::num_e(l)]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                cur = next;
             }
         }
     }
-    if (active) {
+    // sum lme of channel c of this lane
+    auto value = [&](auto pc, auto mc, int c) -> F& {
+        constexpr int p = decltype(pc)::value, m = decltype(mc)::value;
+        if constexpr (MX) return reinterpret_cast<F*>(&tile[c][BL::tile_off(p) + m / 4])[m % 4];
+        else return acc[c][PT::lme(p, 0) + m * PT::num_e(PT::l(p))];
+    };
+    auto every = [&](auto&& f) {      // f(lme, channel slot, sum)
+        static_for<0, P>([&](auto pc) {
+            static_for<0, 2 * PT::l(decltype(pc)::value) + 1>([&](auto mc) {
+                constexpr int q = PT::lme(decltype(pc)::value, decltype(mc)::value);
 #pragma unroll
-        for (int q = 0; q < NE; ++q) {
-            Vec<F, CPL> o;
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) o.v[c] = acc[c][q];
-            *reinterpret_cast<Vec<F, CPL>*>(a.out + ((size_t)i * NE + q) * K + k0) = o;
-        }
+                for (int c = 0; c < CPL; ++c) f(q, c, value(pc, mc, c));
+            });
+        });
+    };
+    // the parts of a receiver lie in one thread block: the upper half of them hands its sums to the lower half, in LDS
+    F* half = reinterpret_cast<F*>(smem);
+    for (int h = parts >> 1; h >= 1; h >>= 1) {
+        __syncthreads();
+        // slot of a receiver's part pair: the sums of the units of a block that give, in order
+        const int slot = (wave / parts) * h + part % h;
+        F* at = half + (size_t)slot * NE * CPL * 64 + lane;
+        if (part >= h && part < 2 * h) every([&](int q, int c, F& v) { at[(size_t)(q * CPL + c) * 64] = v; });
+        __syncthreads();
+        if (part < h) every([&](int q, int c, F& v) { v += at[(size_t)(q * CPL + c) * 64]; });
     }
+    if (!real || part != 0) return;
+    every([&](int q, int c, F& v) {
+        if (active[c]) a.out[((size_t)i * NE + q) * K + k[c]] = v;
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -377,79 +495,95 @@ __global__ __launch_bounds__(256, LMAXH >= 2 ? 1 : 2) void k_agg_fwd(const AggPa
 // row (mace.cpp:579-604), staged per edge for the deterministic sender-side sum.
 // With more than one channel group each group writes its share
 // of the force to fpart[group][edge][3]; the caller adds the groups up.
-template <typename F, int LMAXH, int CPL, int EC>
-__global__ __launch_bounds__(256, LMAXH >= 2 ? 1 : 2) void k_agg_bwd(const AggParams<F> a, const int num_terms)
+//
+// The harmonics depend on the direction only, so their gradient is tangential: two components in a frame (t1, t2)
+// orthogonal to the direction carry it.  Per path the rows of B, dB.t1, dB.t2 meet the receiver's adjoint first,
+// u[m2][t] = sum_m d[m] (B, dB.t1, dB.t2)[m][m2]; with R and R' of the path they add to four sums per m2,
+//   message R u[.][0],  R u[.][1],  R u[.][2],  R' u[.][0],
+// and only at the end of the edge these meet the sender feature (radial and two tangential forces).
+template <typename F, int LMAXH, int CPL>
+__global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_agg_bwd(const AggParams<F> a, const int parts)
 {
+    constexpr bool MX = kMatrix<F>;
     using PT = Paths<LMAXH>;
-    using WL = WaveLds<F, LMAXH, true>;
-    constexpr int NB = PT::NB, NBP = WL::NBP, NE = PT::NE, P = PT::P, NLM = PT::NLM;
+    using BL = BlockLayout<LMAXH, true, MX>;
+    using EL = EdgeLds<F, LMAXH, true>;
+    constexpr int NE = PT::NE, P = PT::P, NLM = PT::NLM, SUB = EL::SUB;
+    constexpr int W = P <= 5 ? P : 5;     // splines of the ring: requested W paths ahead
     extern __shared__ __align__(16) unsigned char smem[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    double* cg_c = reinterpret_cast<double*>(smem);
-    int* cg_lm1 = reinterpret_cast<int*>(cg_c + num_terms);
-    int* cg_start = cg_lm1 + num_terms;
-    unsigned char* base = smem + WL::lists(num_terms) + (size_t)wave * WL::per_wave(EC);
-    // the B block below is read with 4 * sizeof(F)-byte accesses: the doubles in front of it must keep that alignment
-    static_assert((EC * (64 + 12 + 1) * sizeof(double)) % (4 * sizeof(F)) == 0, "chunk size breaks the alignment of the B block");
-    double* Yt = reinterpret_cast<double*>(base);                                 // [EC][4][16]: Y, dY/dx, dY/dy, dY/dz
-    double* us = Yt + EC * 64;                                                    // [EC][12]: xyz/r, -, tangent t1, tangent t2, -, -
-    double* xs = us + EC * 12;                                                    // [EC]
-    // The harmonics depend on the direction only, so their gradient is tangential: two components in a frame
-    // (t1, t2) orthogonal to the direction carry it, and the contraction below costs three multiply-adds per
-    // entry instead of four.
-    F* Bs = reinterpret_cast<F*>(xs + EC);                                        // [EC][NBP][4]: B, dB.t1, dB.t2, -
-    int* rows = reinterpret_cast<int*>(Bs + EC * 4 * NBP);
-    int* grows = rows + EC;
+    double* coef = reinterpret_cast<double*>(smem);
+    int* offs = reinterpret_cast<int*>(coef + 2 * BL::NV);
+    unsigned char* base = smem + EL::lists + (size_t)wave * EL::per_wave;
+    double* Yt = reinterpret_cast<double*>(base);                                 // [kChunk][3][16]: Y, dY.t1, dY.t2
+    double* us = reinterpret_cast<double*>(base + EL::y_bytes);                   // [kChunk][10]: xyz / r, t1, t2, -
+    F* vals = reinterpret_cast<F*>(base + EL::y_bytes + EL::frame_bytes);         // [SUB][NV]
+    F* sums = vals + (size_t)SUB * BL::NV;                                        // [kChunk][4]: radial, t2, t1, (t2)
+    double* xs = reinterpret_cast<double*>(base + EL::y_bytes + EL::frame_bytes + EL::block_bytes + EL::sum_bytes);
+    int* rows = reinterpret_cast<int*>(xs + kChunk + 1);
+    int* grows = rows + kChunk + 1;
 
-    for (int t = threadIdx.x; t < num_terms; t += 256) { cg_c[t] = a.B_c[t]; cg_lm1[t] = a.B_lm1[t]; }
-    for (int t = threadIdx.x; t <= NB; t += 256) cg_start[t] = a.B_start[t];
+    block_lists<LMAXH, true, MX>(a, coef, offs);
     __syncthreads();
-    // lane-owned entries of the coupling block (registers for them exist in single precision only)
-    constexpr bool OWNED = sizeof(F) == 4;
-    constexpr int NSLOT = OWNED ? (NB + 63) / 64 : 1;
-    BlockEntry ent[NSLOT];
-    if constexpr (OWNED) {
-#pragma unroll
-        for (int j = 0; j < NSLOT; ++j) ent[j] = block_entry(lane + 64 * j, NB, cg_start, cg_c, cg_lm1);
-    }
 
-    const int K = a.K;
+    const unsigned K = (unsigned)a.K;
     // one-dimensional grid, channel group fastest (see k_agg_fwd)
-    const int groups = (K + 64 * CPL - 1) / (64 * CPL);
+    const int groups = (a.K + 64 * CPL - 1) / (64 * CPL);
     const int cgroup = blockIdx.x % groups;
-    const int i = a.node_begin + (blockIdx.x / groups) * 4 + wave;
+    const int unit = (blockIdx.x / groups) * 4 + wave;
+    const int rel = __builtin_amdgcn_readfirstlane(unit / parts), part = unit - rel * parts, i = a.node_begin + rel;
     if (i >= a.num_nodes) return;
     // Lanes beyond the last channel work on channel 0 with a zero adjoint (all their sums are zero) and skip the
-    // message store: no branch on the lane's channel inside the edge loop, hence no merges of old and new registers.
-    const bool active = (cgroup * 64 + lane) * CPL < K;
-    const int k0 = active ? (cgroup * 64 + lane) * CPL : 0;
-    const int e0 = a.first_neigh[i], e1 = a.first_neigh[i + 1], ti = a.node_types[i];
+    // message store: no branch on the lane's channel inside the edge loop.
+    unsigned k[CPL];
+    bool active[CPL];
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+        const int ch = (cgroup * CPL + c) * 64 + lane;
+        active[c] = ch < a.K;
+        k[c] = active[c] ? (unsigned)ch : 0u;
+    }
+    const int first = a.first_neigh[i], deg = a.first_neigh[i + 1] - first, ti = a.node_types[i];
+    const int e0 = __builtin_amdgcn_readfirstlane(first + (int)((long)deg * part / parts));
+    const int e1 = __builtin_amdgcn_readfirstlane(first + (int)((long)deg * (part + 1) / parts));
     double* fout = groups > 1 ? a.fpart + (size_t)cgroup * 3 * a.num_edges : a.forces;
     const bool add_forces = groups == 1 && a.accumulate_forces;
+    if (e0 >= e1) return;
 
     F d[CPL][NE];
 #pragma unroll
-    for (int q = 0; q < NE; ++q) {
-        const Vec<F, CPL> v = ldv<F, CPL>(a.d_out + ((size_t)i * NE + q) * K + k0);
+    for (int c = 0; c < CPL; ++c)
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) d[c][q] = active ? v.v[c] : F(0);
-    }
+        for (int q = 0; q < NE; ++q) {
+            const F v = a.d_out[((size_t)i * NE + q) * K + k[c]];
+            d[c][q] = active[c] ? v : F(0);
+        }
 
-    for (int eb = e0; eb < e1; eb += EC) {
-        const int nE = min(EC, e1 - eb);
+    Vec<F, 4> cf[CPL][W];
+    const unsigned row_bytes = P * K * 4 * sizeof(F), sender_bytes = NLM * K * sizeof(F);
+    auto request_spline = [&](const char* row, int path) {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) cf[c][path % W] = load_spline<F>(row, path, K, k[c]);
+    };
+    const char* cur = nullptr;      // table row of the edge under way
+    for (int eb = e0; eb < e1; eb += kChunk) {
+        const int nE = min(kChunk, e1 - eb);
         wave_lds_sync();
-        if (lane < nE) {
-            const int e = eb + lane;
-            const double dx = a.xyz[3 * (size_t)e], dy = a.xyz[3 * (size_t)e + 1], dz = a.xyz[3 * (size_t)e + 2];
-            const double inv = rsqrt_pos(dx * dx + dy * dy + dz * dz);
-            sph_l3_grad_store<16>(dz * inv, dx * inv, dy * inv, inv, Yt + lane * 64);
-            const double r = a.r[e];
-            // radial direction as the reference forms it: xyz / r with the caller's r
-            const double ir = rcp_pos(r);
-            us[lane * 12] = dx * ir; us[lane * 12 + 1] = dy * ir; us[lane * 12 + 2] = dz * ir;
-            {
-                // t1 = n x a / |n x a| with a the axis the direction n is least aligned with (|n x a|^2 >= 2/3), t2 = n x t1
+        if (lane <= nE) {
+            // lane nE: the first edge of the next chunk, whose splines are requested at the end of this one
+            // (past the last edge of the part: the last one again)
+            const int e = min(eb + lane, e1 - 1);
+            double r, x;
+            int row, grow;
+            edge_head(a, e, ti, r, x, row, grow);
+            xs[lane] = x; rows[lane] = row; grows[lane] = grow;
+            if (lane < nE) {
+                const double dx = a.xyz[3 * (size_t)e], dy = a.xyz[3 * (size_t)e + 1], dz = a.xyz[3 * (size_t)e + 2];
+                const double inv = rsqrt_pos(dx * dx + dy * dy + dz * dz);
+                // radial direction as the reference forms it: xyz / r with the caller's r
+                const double ir = rcp_pos(r);
                 const double nx = dx * inv, ny = dy * inv, nz = dz * inv;
+                // t1 = n x a / |n x a| with a the axis the direction n is least aligned with (|n x a|^2 >= 2/3), t2 = n x t1
                 const double ax = fabs(nx), ay = fabs(ny), az = fabs(nz);
                 double t1x, t1y, t1z;
                 if (ax <= ay && ax <= az) { t1x = 0.0; t1y = nz; t1z = -ny; }
@@ -457,254 +591,227 @@ __global__ __launch_bounds__(256, LMAXH >= 2 ? 1 : 2) void k_agg_bwd(const AggPa
                 else { t1x = ny; t1y = -nx; t1z = 0.0; }
                 const double tn = rsqrt_pos(t1x * t1x + t1y * t1y + t1z * t1z);
                 t1x *= tn; t1y *= tn; t1z *= tn;
-                double* fr = us + lane * 12 + 4;
-                fr[0] = t1x; fr[1] = t1y; fr[2] = t1z;
-                fr[3] = ny * t1z - nz * t1y; fr[4] = nz * t1x - nx * t1z; fr[5] = nx * t1y - ny * t1x;
+                const double t2x = ny * t1z - nz * t1y, t2y = nz * t1x - nx * t1z, t2z = nx * t1y - ny * t1x;
+                double* fr = us + lane * 10;
+                fr[0] = dx * ir; fr[1] = dy * ir; fr[2] = dz * ir;
+                fr[3] = t1x; fr[4] = t1y; fr[5] = t1z; fr[6] = t2x; fr[7] = t2y; fr[8] = t2z;
+                // The derivative of a harmonic of the direction along a tangent is that of its homogeneous form over the
+                // length.  The harmonics' axes are the permuted ones (z, x, y).
+                double* y = Yt + lane * 48;
+                static_for<0, 16>([&](auto lc) {
+                    constexpr int lm = decltype(lc)::value;
+                    double Y, g0, g1, g2;
+                    ylm_g<lm>(nz, nx, ny, Y, g0, g1, g2);
+                    y[lm] = Y;
+                    y[16 + lm] = (g0 * t1z + g1 * t1x + g2 * t1y) * inv;
+                    y[32 + lm] = (g0 * t2z + g1 * t2x + g2 * t2y) * inv;
+                    if constexpr (lm % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // short live ranges
+                });
             }
-            const int n = spline_interval(r, a.spl_inv_h, a.spl_nodes - 2);
-            xs[lane] = r - a.spl_h * n;
-            const int tbl = a.pair_table[pair_index(a.T, ti, a.neigh_types[e])];
-            rows[lane] = tbl * (a.spl_nodes - 1) + n;
-            grows[lane] = a.gather[e];
         }
         wave_lds_sync();
-        if constexpr (OWNED) {
-#pragma unroll
-            for (int j = 0; j < NSLOT; ++j) {
-                const int b = lane + 64 * j;
-                if (b < NB) {
-                    const BlockEntry& en = ent[j];
-                    for (int le = 0; le < nE; ++le) {
-                        const double* y0 = Yt + le * 64 + en.l0;
-                        const double* y1 = Yt + le * 64 + en.l1;
-                        double s = en.c0 * y0[0] + en.c1 * y1[0], sx = en.c0 * y0[16] + en.c1 * y1[16];
-                        double sy = en.c0 * y0[32] + en.c1 * y1[32], sz = en.c0 * y0[48] + en.c1 * y1[48];
-                        for (int t = en.t2; t < en.t_end; ++t) {
-                            const double cc = cg_c[t];
-                            const double* y = Yt + le * 64 + cg_lm1[t];
-                            s += cc * y[0]; sx += cc * y[16]; sy += cc * y[32]; sz += cc * y[48];
-                        }
-                        const double* fr = us + le * 12 + 4;
-                        Vec<F, 4> o;
-                        o.v[0] = (F)s;
-                        o.v[1] = (F)(sx * fr[0] + sy * fr[1] + sz * fr[2]);
-                        o.v[2] = (F)(sx * fr[3] + sy * fr[4] + sz * fr[5]);
-                        o.v[3] = F(0);
-                        *reinterpret_cast<Vec<F, 4>*>(Bs + ((size_t)le * NBP + b) * 4) = o;
-                    }
-                }
-            }
-        } else {
-        for (int it = lane; it < nE * NB; it += 64) {
-            const int le = it / NB, b = it - le * NB;
-            double s = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
-            for (int t = cg_start[b]; t < cg_start[b + 1]; ++t) {
-                const double cc = cg_c[t];
-                const double* y = Yt + le * 64 + cg_lm1[t];
-                s += cc * y[0]; sx += cc * y[16]; sy += cc * y[32]; sz += cc * y[48];
-            }
-            const double* fr = us + le * 12 + 4;
-            Vec<F, 4> o;
-            o.v[0] = (F)s;
-            o.v[1] = (F)(sx * fr[0] + sy * fr[1] + sz * fr[2]);
-            o.v[2] = (F)(sx * fr[3] + sy * fr[4] + sz * fr[5]);
-            o.v[3] = F(0);
-            *reinterpret_cast<Vec<F, 4>*>(Bs + ((size_t)le * NBP + b) * 4) = o;
+        if (eb == e0) {
+            cur = uniform_row(a.tabK, rows[0], row_bytes);
+            static_for<0, W>([&](auto qc) { request_spline(cur, decltype(qc)::value); });
         }
-        }
-        wave_lds_sync();
-        // Spline coefficients of one edge: P x CPL 16-byte loads, contiguous across the lanes for one path.  In single
-        // precision the next edge's coefficients are requested while the current edge is worked on (40
-        // registers in flight); in double precision they are requested together at the start of the edge.
-        constexpr bool AHEAD = sizeof(F) == 4 && LMAXH <= 1;
-        Vec<F, 4> cf[P][CPL];
-        auto load_cf = [&](int le_) {
-            const int row = __builtin_amdgcn_readfirstlane(rows[le_]);
-            const F* rowp = a.tabK + ((size_t)row * P * K + k0) * 4;
-#pragma unroll
-            for (int q = 0; q < P; ++q)
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) cf[q][c] = ldv<F, 4>(rowp + ((size_t)q * K + c) * 4);
-        };
-        if (AHEAD && nE > 0) load_cf(0);
-        // One edge.  The loop below runs it with the request for the next edge's coefficients for all edges but the
-        // last of the chunk, which runs without: a request under a condition inside one loop body would make the
-        // coefficients carried round the loop a merge of old and new registers (a register copy per value and edge).
-        auto edge = [&](const int le, auto ahead) {
-            F srad = F(0), g1 = F(0), g2 = F(0);
-            {
+        for (int sb = 0; sb < nE; sb += SUB) {
+            const int ns = min(SUB, nE - sb);
+            if (sb) wave_lds_sync();
+            block_values<LMAXH, true, MX, F, 48, SUB>(a, coef, offs, Yt + sb * 48, ns, vals, lane);
+            wave_lds_sync();
+            for (int le = sb; le < sb + ns; ++le) {
                 const F x = (F)xs[le];
-                const int grow = __builtin_amdgcn_readfirstlane(grows[le]);
-                // element offset of this edge's B block; it passes through the fences below, which keep the
-                // LDS reads of a group behind the arithmetic of the group before it (all reads at once would
-                // need several hundred registers)
-                int boffs = le * 4 * NBP;
-                const F* Hp = a.Hsrc + (size_t)grow * NLM * K + k0;
-                Vec<F, CPL> H[NLM], mg[NLM];
+                // the sender row is met at the end of the edge only: requested here, it has the whole edge to arrive
+                F H[CPL][NLM];
+                {
+                    const char* row = uniform_row(a.Hsrc, grows[le], sender_bytes);
 #pragma unroll
-                for (int q = 0; q < NLM; ++q) {
-                    H[q] = ldv<F, CPL>(Hp + q * K);
+                    for (int c = 0; c < CPL; ++c)
 #pragma unroll
-                    for (int c = 0; c < CPL; ++c) mg[q].v[c] = F(0);
+                        for (int q = 0; q < NLM; ++q) H[c][q] = load_at<F>(row + q * (K * sizeof(F)), k[c] * sizeof(F));
                 }
-                if (!AHEAD) load_cf(le);
-                F Rv[P][CPL], Rdv[P][CPL];
+                const char* next = uniform_row(a.tabK, rows[le + 1], row_bytes);
+                const F* Bp = vals + (size_t)(le - sb) * BL::NV + (lane & (BL::LANES - 1));
+                F B[BL::REGS];
 #pragma unroll
-                for (int q = 0; q < P; ++q)
+                for (int j = 0; j < BL::REGS; ++j) B[j] = Bp[j * BL::LANES];
+                F V[CPL][NLM][4];     // message, R u.t1, R u.t2, R' u
+                if constexpr (!MX) {
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                        for (int q = 0; q < NLM; ++q) { V[c][q][1] = F(0); V[c][q][2] = F(0); }
+                }
+                static_for<0, P>([&](auto pc) {
+                    constexpr int p = decltype(pc)::value, l = PT::l(p), l2 = PT::l2(p), n2 = 2 * l2 + 1;
+                    constexpr int lme0 = PT::lme(p, 0), es = PT::num_e(l);
+                    constexpr bool starts = p == PT::first_with_l2(l2);    // the first path of this l2 starts the sums
+                    F R[CPL], Rd[CPL];
 #pragma unroll
                     for (int c = 0; c < CPL; ++c) {
-                        const Vec<F, 4> k4 = cf[q][c];
-                        Rv[q][c] = k4.v[0] + x * (k4.v[1] + x * (k4.v[2] + x * k4.v[3]));
-                        Rdv[q][c] = k4.v[1] + x * (F(2) * k4.v[2] + F(3) * x * k4.v[3]);
+                        // value and derivative by Horner's rule
+                        const Vec<F, 4> k4 = cf[c][p % W];
+                        const F q1 = k4.v[2] + x * k4.v[3], d1 = q1 + x * k4.v[3], q2 = k4.v[1] + x * q1;
+                        R[c] = k4.v[0] + x * q2;
+                        Rd[c] = q2 + x * d1;
                     }
-                if constexpr (AHEAD && decltype(ahead)::value) load_cf(le + 1);
-                // The B block of the edge is walked in steps (a few rows m of one path each).  Per path, the rows
-                // are summed first, u[m2][comp] = sum_m d[m] * (B, dB.t1, dB.t2)[m][m2], then one product
-                // with the sender feature per m2.  The LDS reads of the next step are issued before the
-                // arithmetic of the current one (two register buffers); the fence after each step keeps
-                // reads further ahead from being issued (all at once would need several hundred registers).
-                using ST = BwdSteps<LMAXH, sizeof(F) == 8>;
-                constexpr bool LOOKAHEAD = true;
-                Vec<F, 4> buf[LOOKAHEAD ? 2 : 1][ST::MAXLEN];
-                F u[CPL][2 * LMAXH + 1][3];
-                auto load_step = [&](auto sc, Vec<F, 4>* dst) {
-                    // (every table lookup lands in a constexpr variable: left to the optimizer, the path tables of the
-                    // l = 2 instantiation stay behind as loops that run on the device)
-                    constexpr int s = decltype(sc)::value, p = ST::path(s), n2 = 2 * PT::l2(p) + 1, len = ST::len(s);
-                    constexpr int first = (PT::boff(p) + ST::m0(s) * n2) * 4;
-                    const F* B4 = Bs + boffs + first;
+                    if constexpr (p + W < P) request_spline(cur, p + W); else request_spline(next, p % W);
+                    if constexpr (MX) {
+                        constexpr int T = BL::tiles(p);
+                        f32x4 u[CPL][T];
+                        static_for<0, 2 * l + 1>([&](auto mc) {
+                            constexpr int m = decltype(mc)::value;
+                            static_for<0, T>([&](auto tc) {
+                                constexpr int t = decltype(tc)::value, g = BL::group(p, t, m);
 #pragma unroll
-                    for (int q = 0; q < len; ++q) dst[q] = ldv<F, 4>(B4 + 4 * q);
-                };
-                if constexpr (LOOKAHEAD) load_step(std::integral_constant<int, 0>{}, buf[0]);
-                static_for<0, ST::count()>([&](auto sc) {
-                    constexpr int s = decltype(sc)::value, p = ST::path(s), m0 = ST::m0(s), m1 = ST::m1(s);
-                    constexpr int l = PT::l(p), l2 = PT::l2(p);
-                    constexpr int lme0 = PT::lme(p, 0), es = PT::num_e(l), n2 = 2 * l2 + 1;
-                    Vec<F, 4>* b4 = buf[LOOKAHEAD ? (s & 1) : 0];
-                    if constexpr (!LOOKAHEAD) load_step(sc, b4);
-                    else if constexpr (s + 1 < ST::count()) load_step(std::integral_constant<int, s + 1>{}, buf[(s + 1) & 1]);
+                                for (int c = 0; c < CPL; ++c)
+                                    u[c][t] = __builtin_amdgcn_mfma_f32_4x4x1f32(B[g / 16], d[c][lme0 + m * es],
+                                                                                 m == 0 ? f32x4{0, 0, 0, 0} : u[c][t], 4, g % 16, 0);
+                            });
+                        });
 #pragma unroll
-                    for (int c = 0; c < CPL; ++c) {
-#pragma unroll
-                        for (int m = m0; m < m1; ++m) {
-                            const F dd = d[c][lme0 + m * es];
+                        for (int c = 0; c < CPL; ++c)
 #pragma unroll
                             for (int m2 = 0; m2 < n2; ++m2) {
-                                const Vec<F, 4>& bb = b4[(m - m0) * n2 + m2];
-                                // the unused fourth word counts as used where the others are: the read stays a 16-byte
-                                // one (a 12-byte LDS read is slower) and is not waited for any earlier
-                                asm volatile("" : : "v"(bb.v[3]));
+                                F* s = V[c][l2 * l2 + m2];
 #pragma unroll
-                                for (int t = 0; t < 3; ++t)   // the first row of a path starts the sums
-                                    u[c][m2][t] = m == 0 ? dd * bb.v[t] : u[c][m2][t] + dd * bb.v[t];
+                                for (int t = 0; t < 3; ++t) {
+                                    const F uv = u[c][(3 * m2 + t) / 4][(3 * m2 + t) % 4];
+                                    s[t] = starts ? R[c] * uv : s[t] + R[c] * uv;
+                                    if (t == 0) s[3] = starts ? Rd[c] * uv : s[3] + Rd[c] * uv;
+                                }
                             }
-                        }
+                    } else {
+                        F u0[CPL][n2];
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                            for (int m2 = 0; m2 < n2; ++m2) u0[c][m2] = F(0);
+                        // the tangential sums take R d: no sums per path for them
+                        static_for<0, 2 * l + 1>([&](auto mc) {
+                            constexpr int m = decltype(mc)::value;
+#pragma unroll
+                            for (int c = 0; c < CPL; ++c) {
+                                const F dm = d[c][lme0 + m * es], rd = R[c] * dm;
+                                static_for<0, n2>([&](auto m2c) {
+                                    constexpr int m2 = decltype(m2c)::value, v = 3 * (PT::boff(p) + m * n2 + m2);
+                                    fmac_lane<v % 16>(u0[c][m2], B[v / 16], dm);
+                                    fmac_lane<(v + 1) % 16>(V[c][l2 * l2 + m2][1], B[(v + 1) / 16], rd);
+                                    fmac_lane<(v + 2) % 16>(V[c][l2 * l2 + m2][2], B[(v + 2) / 16], rd);
+                                });
+                            }
+                        });
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                            for (int m2 = 0; m2 < n2; ++m2) {
+                                F* s = V[c][l2 * l2 + m2];
+                                s[0] = starts ? R[c] * u0[c][m2] : s[0] + R[c] * u0[c][m2];
+                                s[3] = starts ? Rd[c] * u0[c][m2] : s[3] + Rd[c] * u0[c][m2];
+                            }
                     }
+                    // path by path
 #pragma unroll
                     for (int c = 0; c < CPL; ++c)
 #pragma unroll
                         for (int m2 = 0; m2 < n2; ++m2)
 #pragma unroll
-                            for (int t = 0; t < 3; ++t) tie(u[c][m2][t], boffs);
-                    if constexpr (m1 == 2 * l + 1) {
-#pragma unroll
-                        for (int c = 0; c < CPL; ++c) {
-                            const F R = Rv[p][c], Rd = Rdv[p][c];
-                            F s0 = F(0), s1 = F(0), s2 = F(0);
-#pragma unroll
-                            for (int m2 = 0; m2 < n2; ++m2) {
-                                const F h = H[l2 * l2 + m2].v[c];
-                                s0 += u[c][m2][0] * h; s1 += u[c][m2][1] * h; s2 += u[c][m2][2] * h;
-                                mg[l2 * l2 + m2].v[c] += R * u[c][m2][0];
-                            }
-                            srad += Rd * s0;
-                            g1 += R * s1; g2 += R * s2;
-                        }
-                        order_after(g1, g2, srad, boffs);
-#pragma unroll
-                        for (int m2 = 0; m2 < n2; ++m2)
-#pragma unroll
-                            for (int c = 0; c < CPL; ++c) pin(mg[l2 * l2 + m2].v[c]);
+                            for (int t = 0; t < 4; ++t) pin(V[c][l2 * l2 + m2][t]);
+                    if constexpr (MX) {
+                        // the matrix instructions of a path together: every change between the pipes costs about four cycles
+                        __builtin_amdgcn_sched_group_barrier(0x008, BL::tiles(p) * (2 * l + 1) * CPL, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, 100, 0);
                     }
+                    __builtin_amdgcn_sched_barrier(0);
                 });
-                if (a.msg && active) {
-                    F* mrow = a.msg + (size_t)(eb + le - a.msg_edge_begin) * NLM * K + k0;
+                cur = next;
+                F srad = F(0), g1 = F(0), g2 = F(0);
 #pragma unroll
-                    for (int q = 0; q < NLM; ++q) *reinterpret_cast<Vec<F, CPL>*>(mrow + q * K) = mg[q];
+                for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                    for (int q = 0; q < NLM; ++q) {
+                        const F h = H[c][q];
+                        srad += V[c][q][3] * h; g1 += V[c][q][1] * h; g2 += V[c][q][2] * h;
+                    }
+                if (a.msg) {
+                    char* mrow = reinterpret_cast<char*>(a.msg) + (unsigned long long)(unsigned)(eb + le - (int)a.msg_edge_begin) * sender_bytes;
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c)
+                        if (active[c]) {
+#pragma unroll
+                            for (int q = 0; q < NLM; ++q) *reinterpret_cast<F*>(mrow + q * (K * sizeof(F)) + k[c] * sizeof(F)) = V[c][q][0];
+                        }
                 }
+                // sums over the channels of the wavefront, in the feature precision (a fixed tree)
+                const F s = wave_sum3(srad, g1, g2);
+                if ((lane & 15) == 0) sums[le * 4 + (lane >> 4)] = s;
             }
-            // Sums over the channels of the wavefront (a fixed tree: bit-reproducible): the radial sum and the two
-            // tangential ones, in the feature precision; the force is put together from them in double.
-            const double sr = (double)wave_sum(srad), G1 = (double)wave_sum(g1), G2 = (double)wave_sum(g2);
-            const double* uf = us + le * 12;
-            const double fx = -(uf[0] * sr + uf[4] * G1 + uf[7] * G2);
-            const double fy = -(uf[1] * sr + uf[5] * G1 + uf[8] * G2);
-            const double fz = -(uf[2] * sr + uf[6] * G1 + uf[9] * G2);
-            if (lane == 0) {
-                double* f = fout + 3 * (size_t)(eb + le);
-                if (add_forces) { f[0] += fx; f[1] += fy; f[2] += fz; }
-                else { f[0] = fx; f[1] = fy; f[2] = fz; }
-            }
-        };
-        if constexpr (AHEAD) {
-            for (int le = 0; le + 1 < nE; ++le) edge(le, std::true_type{});
-            if (nE > 0) edge(nE - 1, std::false_type{});
-        } else {
-            // one copy of the edge's code: the unrolled walk of the coupling block is tens of KB of instructions, and
-            // a chunk's whole code path has to stay inside the instruction cache
-            for (int le = 0; le < nE; ++le) edge(le, std::false_type{});
+        }
+        wave_lds_sync();
+        // the forces of the chunk, put together in double
+        if (lane < nE) {
+            const double* fr = us + lane * 10;
+            const double sr = (double)sums[lane * 4], G2 = (double)sums[lane * 4 + 1], G1 = (double)sums[lane * 4 + 2];
+            const double fx = -(fr[0] * sr + fr[3] * G1 + fr[6] * G2);
+            const double fy = -(fr[1] * sr + fr[4] * G1 + fr[7] * G2);
+            const double fz = -(fr[2] * sr + fr[5] * G1 + fr[8] * G2);
+            double* f = fout + 3 * (size_t)(eb + lane);
+            if (add_forces) { f[0] += fx; f[1] += fy; f[2] += fz; }
+            else { f[0] = fx; f[1] = fy; f[2] = fz; }
         }
     }
 }
 
-template <typename F, int LMAXH, int CPL, int EC, bool BWD>
+// How many wavefronts share a receiver.  A wavefront alone takes 0.5 to 2 us per edge; with fewer receivers than the chip
+// holds wavefronts (2 048 of these kernels) a receiver's edges are dealt to two or four of them.
+inline int agg_parts(long units) { return units <= 4096 ? 4 : (units <= 8192 ? 2 : 1); }
+
+template <typename F, int LMAXH, int CPL, bool BWD>
 hipError_t launch_agg_t(const AggParams<F>& p, hipStream_t s)
 {
-    using WL = WaveLds<F, LMAXH, BWD>;
+    using EL = EdgeLds<F, LMAXH, BWD>;
     const int groups = (p.K + 64 * CPL - 1) / (64 * CPL);
-    if (p.K % CPL != 0) return hipErrorInvalidValue;
     if (BWD && groups > 1 && !p.fpart) return hipErrorInvalidValue;
-    const size_t lds = WL::lists(p.num_terms) + 4 * WL::per_wave(EC) + 4 * WL::prefetch_per_wave();
     if (!BWD && (p.node_begin != 0 || p.msg_edge_begin != 0)) return hipErrorInvalidValue;
     if (p.node_begin < 0 || p.node_begin > p.num_nodes) return hipErrorInvalidValue;
-    const long blocks = (long)((p.num_nodes - p.node_begin + 3) / 4) * groups;
+    const long nodes = p.num_nodes - p.node_begin;
+    // the forward sums depend on the parts in their last bits: a call with ghost nodes is split as one without
+    const int parts = agg_parts((long)(BWD ? nodes : p.split_nodes) * groups);
+    const long blocks = (nodes * parts + 3) / 4 * groups;
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
     dim3 grid((unsigned)blocks);
     void (*kern)(const AggParams<F>, const int);
-    if constexpr (BWD) kern = k_agg_bwd<F, LMAXH, CPL, EC>;
-    else kern = k_agg_fwd<F, LMAXH, CPL, EC>;
+    size_t lds = EL::total;
+    if constexpr (BWD) kern = k_agg_bwd<F, LMAXH, CPL>;
+    else {
+        kern = k_agg_fwd<F, LMAXH, CPL>;
+        const size_t handed = parts > 1 ? (size_t)2 * Paths<LMAXH>::NE * CPL * 64 * sizeof(F) : 0;   // two givers per block
+        lds = lds > handed ? lds : handed;
+    }
     if (lds > 64 * 1024) {
         hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (err != hipSuccess) return err;
     }
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, p, p.num_terms);
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, p, parts);
     return hipGetLastError();
 }
 
-// Channels per lane.  Two give paired loads and fewer broadcast reads per channel; the l <= 1 path list holds
-// 40 accumulators per channel, which leaves room for two channels only in the single-precision forward kernel.
+// Channels per lane: two where the registers hold them and more than one half-empty wavefront would result otherwise.
 template <typename F, int LMAXH, bool BWD>
 int agg_cpl(int K)
 {
-    const bool wide = LMAXH == 0;
-    return (wide && K > 64 && K % 2 == 0) ? 2 : 1;
+    return (LMAXH == 0 || (LMAXH == 1 && sizeof(F) == 4 && BWD)) && K > 64 ? 2 : 1;
 }
 
 template <typename F, int LMAXH, bool BWD>
 hipError_t launch_agg_sel(const AggParams<F>& p, hipStream_t s)
 {
-    // edges per chunk; the double-precision forward kernel of the ten-path list takes eight so that two blocks with
-    // their coefficient buffers fit a CU
-    // (l = 2 hidden features: the coupling block has 243 entries per edge, four edges of the adjoint fill the LDS share of a wavefront)
-    constexpr int EC = LMAXH == 0 ? 16 : (BWD ? (sizeof(F) == 4 && LMAXH == 1 ? 8 : 4) : (sizeof(F) == 8 ? 8 : 16));
-    // two channels per lane exist for the four-path list only (the ten-path kernels have no registers for them)
-    if constexpr (LMAXH == 0) {
-        if (agg_cpl<F, LMAXH, BWD>(p.K) == 2) return launch_agg_t<F, LMAXH, 2, EC, BWD>(p, s);
+    if constexpr (LMAXH == 0 || (LMAXH == 1 && sizeof(F) == 4 && BWD)) {
+        if (agg_cpl<F, LMAXH, BWD>(p.K) == 2) return launch_agg_t<F, LMAXH, 2, BWD>(p, s);
     }
-    return launch_agg_t<F, LMAXH, 1, EC, BWD>(p, s);
+    return launch_agg_t<F, LMAXH, 1, BWD>(p, s);
 }
 
 }  // namespace
@@ -728,7 +835,7 @@ hipError_t launch_agg_bwd(int L_max_H, const AggParams<F>& p, hipStream_t s)
 template <typename F>
 int agg_bwd_groups(int L_max_H, int K)
 {
-    const int cpl = L_max_H == 0 ? agg_cpl<F, 0, true>(K) : 1;
+    const int cpl = L_max_H == 0 ? agg_cpl<F, 0, true>(K) : (L_max_H == 1 ? agg_cpl<F, 1, true>(K) : 1);
     return (K + 64 * cpl - 1) / (64 * cpl);
 }
 // This file is compiled four times (SMX_EDGE_PART = 0..3), one object per

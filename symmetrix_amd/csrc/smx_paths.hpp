@@ -50,6 +50,12 @@ struct Paths {
     static constexpr int l(int p) { return get(p, 0); }
     static constexpr int l1(int p) { return get(p, 1); }
     static constexpr int l2(int p) { return get(p, 2); }
+    // first path with sender order l2_
+    static constexpr int first_with_l2(int l2_)
+    {
+        for (int p = 0; p < P; ++p) if (l2(p) == l2_) return p;
+        return -1;
+    }
     static constexpr int num_e(int l_)
     {
         int n = 0;

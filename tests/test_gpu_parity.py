@@ -877,3 +877,40 @@ def test_senders_with_many_edges(gpu, tmp_models, L_max, K, edge):
     f, d = orc.node_forces.reshape(-1, 3), ea["xyz"].reshape(-1, 3)
     W = 0.5 * (d.T @ f + f.T @ d)
     assert np.abs(V - W[[0, 1, 2, 0, 0, 1], [0, 1, 2, 1, 2, 2]]).max() <= 1e-9 * max(1.0, np.abs(W).max())
+
+
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("K,L_max,receivers,max_degree,terms", [
+    # degrees on both sides of the chunks of 16 and 17 edges and of the two and four parts a receiver is split into
+    (70, 1, 40, 37, 1), (130, 1, 24, 35, 1), (33, 2, 24, 34, 1), (70, 0, 40, 50, 1),
+    # more than 4 096 and 8 192 receivers: two wavefronts per receiver, then one
+    (16, 1, 4099, 3, 1), (16, 1, 8195, 3, 1),
+    # coupling entries of three terms
+    (32, 1, 20, 20, 3), (32, 2, 20, 20, 3),
+])
+def test_general_edge_kernels_at_the_edges_of_their_split(gpu, tmp_models, K, L_max, receivers, max_degree, terms, dtype):
+    model = H.tiny_model(K=K, L_max=L_max, n_pts=24, seed=K + L_max, pair=True)
+    if terms > 1:   # every coefficient as a sum of three
+        for key in ("Phi1_lme", "Phi1_lelm1lm2"):
+            model[key] = [v for v in model[key] for _ in range(terms)]
+        model["Phi1_clebsch_gordan"] = [v * w for v in model["Phi1_clebsch_gordan"] for w in (0.5, 0.75, -0.25)]
+    rng = np.random.default_rng(receivers)
+    degree = np.array([n % (max_degree + 1) for n in range(receivers)])
+    E = int(degree.sum())
+    species = rng.integers(0, 3, size=receivers).astype(np.int32)
+    senders = rng.integers(0, receivers, size=E).astype(np.int32)
+    x = rng.normal(size=(E, 3))
+    x *= (rng.uniform(0.8, 3.9, size=E) / np.linalg.norm(x, axis=1))[:, None]
+    args = (receivers, species, degree.astype(np.int32), senders, species[senders], x.ravel(), np.linalg.norm(x, axis=1))
+    orc = _oracle()(model)
+    eng = gpu(H.write_model(model, tmp_models / f"split_{K}_{L_max}_{receivers}_{terms}.json"), dtype)
+    print(f"case K={K} L_max={L_max} receivers={receivers} edges={E} terms={terms} {dtype}", flush=True)
+    orc.compute_node_energies_forces(*args)
+    eng.compute_node_energies_forces(*args)
+    names = ["A0", "Phi1", "H1_adj", "A0_adj"]
+    for name in names:
+        a, b = np.asarray(getattr(orc, name)), np.asarray(getattr(eng, name))
+        assert np.abs(a - b).max(initial=0.0) <= TOL[dtype]["inter"] * 10 * max(1.0, np.abs(a).max()), name
+    scale = max(1.0, np.abs(orc.node_forces).max())
+    assert np.abs(orc.node_energies - eng.node_energies).max() <= TOL[dtype]["E"] * 10 * max(1.0, np.abs(orc.node_energies).max())
+    assert np.abs(orc.node_forces - eng.node_forces).max() <= TOL[dtype]["F"] * scale
