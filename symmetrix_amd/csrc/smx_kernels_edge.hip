@@ -762,9 +762,17 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
     }
 }
 
-// How many wavefronts share a receiver.  A wavefront alone takes 0.5 to 2 us per edge; with fewer receivers than the chip
-// holds wavefronts (2 048 of these kernels) a receiver's edges are dealt to two or four of them.
-inline int agg_parts(long units) { return units <= 4096 ? 4 : (units <= 8192 ? 2 : 1); }
+// How many wavefronts share a receiver, of `units` receivers times channel groups.  A wavefront takes 0.5 to 2 us per edge,
+// and about 2 048 of them are in flight: fewer units leave SIMDs idle, up to three rounds of them leave the last round
+// nearly empty.  The adjoint gains up to three rounds (K = 128, l <= 1, single precision, 1 500 receivers: 214, 194, 157 us
+// for one, two and four wavefronts); the forward kernel, which has to add the parts, only where the chip is not full
+// (500 receivers: 52, 38, 41 us; 3 000: 153, 160, 163).
+template <bool BWD>
+int agg_parts(long units)
+{
+    if (BWD) return units <= 2048 ? 4 : (units <= 6144 ? 2 : 1);
+    return units <= 512 ? 4 : (units <= 3072 ? 2 : 1);
+}
 
 template <typename F, int LMAXH, int CPL, bool BWD>
 hipError_t launch_agg_t(const AggParams<F>& p, hipStream_t s)
@@ -776,7 +784,7 @@ hipError_t launch_agg_t(const AggParams<F>& p, hipStream_t s)
     if (p.node_begin < 0 || p.node_begin > p.num_nodes) return hipErrorInvalidValue;
     const long nodes = p.num_nodes - p.node_begin;
     // the forward sums depend on the parts in their last bits: a call with ghost nodes is split as one without
-    const int parts = agg_parts((long)(BWD ? nodes : p.split_nodes) * groups);
+    const int parts = agg_parts<BWD>((long)(BWD ? nodes : p.split_nodes) * groups);
     const long blocks = (nodes * parts + 3) / 4 * groups;
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;

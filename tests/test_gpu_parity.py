@@ -883,8 +883,8 @@ def test_senders_with_many_edges(gpu, tmp_models, L_max, K, edge):
 @pytest.mark.parametrize("K,L_max,receivers,max_degree,terms", [
     # degrees on both sides of the chunks of 16 and 17 edges and of the two and four parts a receiver is split into
     (70, 1, 40, 37, 1), (130, 1, 24, 35, 1), (33, 2, 24, 34, 1), (70, 0, 40, 50, 1),
-    # more than 4 096 and 8 192 receivers: two wavefronts per receiver, then one
-    (16, 1, 4099, 3, 1), (16, 1, 8195, 3, 1),
+    # two wavefronts per receiver, then one, in either direction
+    (16, 1, 515, 9, 1), (16, 1, 2051, 5, 1), (16, 1, 3075, 3, 1), (16, 1, 6147, 3, 1),
     # coupling entries of three terms
     (32, 1, 20, 20, 3), (32, 2, 20, 20, 3),
 ])
