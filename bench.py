@@ -40,23 +40,16 @@ sys.path.insert(0, HERE)
 
 HBM_PEAK = 8.0e12  # bytes/s, MI355X HBM3E
 
-# kernel behind each edge stage: channel-slice kernels (scalar hidden features and one radial table for all
-# species pairs) / general kernels
-SLICE_KERNEL = {"agg0_fwd": "k_slice_fwd_halves", "agg1_fwd": "k_slice_fwd_halves", "agg1_bwd": "k_slice_bwd_edge",
-                "agg0_bwd": "k_slice_bwd_edge", "sender_reduce": "k_sender_reduce_linear"}
-GENERAL_KERNEL = {"agg0_fwd": "k_agg_fwd", "agg1_fwd": "k_agg_fwd", "agg1_bwd": "k_agg_bwd", "agg0_bwd": "k_agg_bwd",
-                  "sender_reduce": "k_sender_reduce"}
+# kernel behind each edge stage: kernels for scalar sender features / general kernels
+SCALAR_KERNEL = {"agg0_fwd": "k_agg0_fwd", "agg1_fwd": "k_agg0_fwd", "agg1_bwd": "k_agg0_bwd", "agg0_bwd": "k_agg0_bwd",
+                 "sender_reduce": "k_sender_reduce_linear"}
+GENERAL_KERNEL = {"agg1_fwd": "k_agg_fwd", "agg1_bwd": "k_agg_bwd", "sender_reduce": "k_sender_reduce"}
 EDGE_STAGES = ["agg0_fwd", "agg1_fwd", "agg1_bwd", "sender_reduce", "agg0_bwd"]
 
 
-def stage_kernel(stage, L_max, distinct_tables):
+def stage_kernel(stage, L_max):
     """Name of the kernel that runs an edge stage for this kind of model."""
-    sliced = distinct_tables == 1
-    if stage.startswith("agg0"):
-        return (SLICE_KERNEL if sliced else GENERAL_KERNEL)[stage]
-    if stage == "sender_reduce":
-        return SLICE_KERNEL[stage] if L_max == 0 else GENERAL_KERNEL[stage]
-    return (SLICE_KERNEL if (sliced and L_max == 0) else GENERAL_KERNEL)[stage]
+    return (SCALAR_KERNEL if stage.startswith("agg0") or L_max == 0 else GENERAL_KERNEL)[stage]
 
 
 def measured_traffic(workload, dtype, stage, kernel):
@@ -476,7 +469,7 @@ def main():
         dom_s = res["stages"][dom] * 1e-3
         achieved = dom_bytes / dom_s / 1e9 if dom_s > 0 else 0.0
         total_bytes = sum(stage_bytes(k) for k in EDGE_STAGES) + (32 * E + 24 * N)
-        kernel = stage_kernel(dom, L_max, res["tables"])
+        kernel = stage_kernel(dom, L_max)
         prof_name = workload + ("_pairs" if pair_tables else "")
         profiled = scale == 1.0 and not ghosts
         stages_rl = {}
@@ -485,7 +478,7 @@ def main():
             if ms_k <= 0.0:
                 continue
             b_k = stage_bytes(k)
-            kern_k = stage_kernel(k, L_max, res["tables"])
+            kern_k = stage_kernel(k, L_max)
             ach = b_k / (ms_k * 1e-3) / 1e9
             stages_rl[k] = {"kernel": kern_k, "algorithmic_bytes": b_k, "kernel_ms": ms_k, "achieved": ach,
                             "frac": ach / (HBM_PEAK / 1e9),
@@ -600,8 +593,7 @@ def main():
             "roofline_stages": m2["roofline_stages"], "mfma": m2["mfma"], "contraction": m2["contraction"],
             "stages_ms": m2["res"]["stages"], "energy": m2["res"]["energy"],
         }
-        # the headline workload with one radial table per species pair (ten tables for four species): more than four
-        # distinct tables take the general edge kernels instead of the channel-slice ones
+        # the headline workload with one radial table per species pair (ten tables for four species)
         m3 = measure("off_small", args.dtype, max(5, args.steps // 2), args.warmup, pair_tables=True, both=False, host_leg=False)
         line["pair_dependent_tables"] = {
             "workload": m3["workload"], "dtype": line["dtype"], "ms_per_step": m3["res"]["ms"], "value": m3["value"],

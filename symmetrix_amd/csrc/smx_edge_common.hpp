@@ -1,0 +1,156 @@
+// What the edge kernels share: loads of spline and feature rows, lane broadcasts, sums over lanes, edge geometry, and how many
+// wavefronts work on a receiver.
+#pragma once
+
+#include "smx_device.hpp"
+#include "smx_kernels.hpp"
+
+namespace smx {
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <typename F>
+constexpr bool kMatrix = sizeof(F) == 4;
+
+// Lane-broadcast multiply-add of the double-precision kernels: acc += (b of lane N of the lane's 16-lane row) * v.  The
+// instruction reads b through DPP: b must not come from the vector instruction right before (here it comes from LDS).
+template <int N>
+__device__ __forceinline__ void fmac_lane(double& acc, double b, double v)
+{
+    asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(b), "v"(v), "n"(N));
+}
+
+// Loads and stores of a wavefront's rows: an address that is the same for all lanes, held in scalar registers, plus a 32-bit
+// offset per lane.
+template <typename T>
+__device__ __forceinline__ T load_at(const char* row, unsigned lane_bytes)
+{
+    return *reinterpret_cast<const T*>(row + lane_bytes);
+}
+// The four coefficients of one spline: 16 bytes in single precision, two halves of 16 bytes in double (a table row is
+// [path][half][K][16 bytes], so that every load instruction of a wavefront covers 1 KB without gaps).
+template <typename F>
+__device__ __forceinline__ Vec<F, 4> load_spline(const char* row, int path, unsigned K, unsigned k)
+{
+    if constexpr (sizeof(F) == 4) return load_at<Vec<F, 4>>(row + path * (K * 16), k * 16);
+    else {
+        Vec<F, 4> c;
+        const Vec<F, 2> lo = load_at<Vec<F, 2>>(row + 2 * path * (K * 16), k * 16);
+        const Vec<F, 2> hi = load_at<Vec<F, 2>>(row + (2 * path + 1) * (K * 16), k * 16);
+        c.v[0] = lo.v[0]; c.v[1] = lo.v[1]; c.v[2] = hi.v[0]; c.v[3] = hi.v[1];
+        return c;
+    }
+}
+// The same for a row whose byte offset from the start of the array the lane holds (lanes of one wavefront on different rows).
+template <typename F>
+__device__ __forceinline__ Vec<F, 4> load_spline_off(const F* tab, int path, unsigned K, unsigned off)
+{
+    const char* t = reinterpret_cast<const char*>(tab);
+    if constexpr (sizeof(F) == 4) return load_at<Vec<F, 4>>(t + path * (K * 16), off);
+    else {
+        Vec<F, 4> c;
+        const Vec<F, 2> lo = load_at<Vec<F, 2>>(t + 2 * path * (K * 16), off), hi = load_at<Vec<F, 2>>(t + (2 * path + 1) * (K * 16), off);
+        c.v[0] = lo.v[0]; c.v[1] = lo.v[1]; c.v[2] = hi.v[0]; c.v[3] = hi.v[1];
+        return c;
+    }
+}
+// row n of an array of rows of that many bytes, n the same in all lanes
+__device__ __forceinline__ const char* uniform_row(const void* base, int n, unsigned row_bytes)
+{
+    return reinterpret_cast<const char*>(base) + (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(n) * row_bytes;
+}
+// The value is final here: keeps the compiler from collecting the arithmetic of several paths, whose operands would all stay
+// live (it moves plain arithmetic across scheduling fences).
+template <typename F>
+__device__ __forceinline__ void pin(F& v)
+{
+    asm volatile("" : "+v"(v));
+}
+
+// The upper 32 lanes of a trade places with the lower 32 of b (swap_rows: the odd 16-lane rows of a with the even rows of b).
+// Added up afterwards, that sums both values over the halves (rows), the first in the lower and the second in the upper lanes.
+template <typename F>
+__device__ __forceinline__ void swap_halves(F& a, F& b)
+{
+    if constexpr (sizeof(F) == 4) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+    } else {
+        const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+        const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+        a = __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]);
+        b = __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
+    }
+}
+template <typename F>
+__device__ __forceinline__ void swap_rows(F& a, F& b)
+{
+    if constexpr (sizeof(F) == 4) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+    } else {
+        const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+        const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+        a = __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]);
+        b = __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
+    }
+}
+// What the lanes need of an edge before its features: spline interval and argument, table row, sender row.
+template <typename F>
+__device__ __forceinline__ void edge_head(const AggParams<F>& a, int e, int ti, double& r, double& x, int& row, int& grow)
+{
+    r = a.r[e];
+    const int n = spline_interval(r, a.spl_inv_h, a.spl_nodes - 2);
+    x = r - a.spl_h * n;
+    row = a.pair_table[pair_index(a.T, ti, a.neigh_types[e])] * (a.spl_nodes - 1) + n;
+    grow = a.gather[e];
+}
+
+// Direction of an edge and a frame orthogonal to it.  The harmonics depend on the direction only, so their gradient is
+// tangential: the derivative along a tangent is that of the homogeneous form over the length.
+struct EdgeFrame {
+    double dx, dy, dz, inv;              // edge vector, 1 / length
+    double nx, ny, nz;                   // direction
+    double t1x, t1y, t1z, t2x, t2y, t2z; // tangents
+};
+__device__ __forceinline__ void edge_frame(const double* xyz, EdgeFrame& f)
+{
+    f.dx = xyz[0]; f.dy = xyz[1]; f.dz = xyz[2];
+    f.inv = rsqrt_pos(f.dx * f.dx + f.dy * f.dy + f.dz * f.dz);
+    f.nx = f.dx * f.inv; f.ny = f.dy * f.inv; f.nz = f.dz * f.inv;
+    // t1 = n x a / |n x a| with a the axis the direction n is least aligned with (|n x a|^2 >= 2/3), t2 = n x t1
+    const double ax = fabs(f.nx), ay = fabs(f.ny), az = fabs(f.nz);
+    if (ax <= ay && ax <= az) { f.t1x = 0.0; f.t1y = f.nz; f.t1z = -f.ny; }
+    else if (ay <= az) { f.t1x = -f.nz; f.t1y = 0.0; f.t1z = f.nx; }
+    else { f.t1x = f.ny; f.t1y = -f.nx; f.t1z = 0.0; }
+    const double tn = rsqrt_pos(f.t1x * f.t1x + f.t1y * f.t1y + f.t1z * f.t1z);
+    f.t1x *= tn; f.t1y *= tn; f.t1z *= tn;
+    f.t2x = f.ny * f.t1z - f.nz * f.t1y; f.t2y = f.nz * f.t1x - f.nx * f.t1z; f.t2z = f.nx * f.t1y - f.ny * f.t1x;
+}
+// harmonic LM and its derivatives along the two tangents (the harmonics' axes are the permuted ones: z, x, y)
+template <int LM>
+__device__ __forceinline__ void ylm_tangential(const EdgeFrame& f, double& Y, double& d1, double& d2)
+{
+    double g0, g1, g2;
+    ylm_g<LM>(f.nz, f.nx, f.ny, Y, g0, g1, g2);
+    d1 = (g0 * f.t1z + g1 * f.t1x + g2 * f.t1y) * f.inv;
+    d2 = (g0 * f.t2z + g1 * f.t2x + g2 * f.t2y) * f.inv;
+}
+
+// How many wavefronts share a receiver, of `units` receivers times channel groups.  A wavefront takes 0.5 to 2 us per edge,
+// and about 2 048 of them are in flight: fewer units leave SIMDs idle, up to three rounds of them leave the last round
+// nearly empty.  The adjoint gains up to three rounds (K = 128, l <= 1, single precision, 1 500 receivers: 214, 194, 157 us
+// for one, two and four wavefronts); the forward kernel, which has to add the parts, only where the chip is not full
+// (500 receivers: 52, 38, 41 us; 3 000: 153, 160, 163).
+template <bool BWD>
+int agg_parts(long units)
+{
+    if (BWD) return units <= 2048 ? 4 : (units <= 6144 ? 2 : 1);
+    return units <= 512 ? 4 : (units <= 3072 ? 2 : 1);
+}
+
+}  // namespace
+}  // namespace smx

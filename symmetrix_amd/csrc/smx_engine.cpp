@@ -235,16 +235,10 @@ struct Engine : EngineBase {
     DVec<int> B0_start, B0_lm1, B1_start, B1_lm1;
     DVec<double> B0_c, B1_c;
     std::vector<long> A1w_off;   // per l
-    // channel-slice tables (see smx_kernels_slice.hip); CH = 0 disables the path for that layer
-    DVec<F> tabS0, tabS1;
-    int slice_CH0 = 0, slice_CH1 = 0, slice_W = 0, num_cus = 0;
-    // the same slices with the row padding of the adjoint kernel that gives every edge a lane of its own
-    // (empty when the forward table already has that row length, or when the kernel does not apply)
-    DVec<F> tabE0, tabE1;
-    DVec<F> tabF0, tabF1;   // forward-kernel layout of the same slices (when a slice is 32 bytes of channels)
+    int num_cus = 0;
     int more_terms1 = 0;       // an entry of layer 1's coupling list has more than two terms
     int split_nodes = 0;       // receivers that are not ghosts, of the evaluation under way
-    bool edge_lanes = false;
+    bool diagonal1 = false;    // scalar hidden features, and output lm of layer 1 is fed by cdiag1[lm] Y_lm alone
     double cdiag1[16] = {};
     DVec<double> fpart;
     DVec<double> H2w_H1, H2w_M1, ro1, ro2_w1, ro2_w2, E0;
@@ -276,7 +270,7 @@ struct Engine : EngineBase {
     long E1 = 0;   // leading edges whose receivers take part in layer 1 (all of them unless ghost nodes follow)
     int N_geo = 0;
     long geo_edges = 0;   // edges of the N_geo receivers
-    DVec<int> first_neigh, recv_order, scan_tmp, s_count, s_start, s_list, t_count, t_start, t_cursor, t_perm, flags;
+    DVec<int> first_neigh, scan_tmp, s_count, s_start, s_list, t_count, t_start, t_cursor, t_perm, flags;
     int sender_rows = 0;
     // pair terms: ZBL constants per species pair, density-normalisation splines, divisors of the last forward pass
     DVec<double> zbl_a, zbl_rmax, zbl_zz, A0spl, A1spl, div0, div1;
@@ -336,10 +330,17 @@ struct Engine : EngineBase {
             for (auto& w : hm.A1_weights) { A1w_off.push_back((long)all.size()); all.insert(all.end(), w.begin(), w.end()); }
             upload_as(A1w, all, s);
         }
-        build_slices(s);
-        // the general edge kernels read the tables as [interval][path][channel][4 coefficients]: one load instruction
-        // of a wavefront (one path, consecutive channels) then covers contiguous memory; layers served by the slice
-        // kernels need no copy
+        // layer 1 with scalar hidden features: whether every output lm is fed by harmonic lm alone
+        diagonal1 = hm.L_max == 0 && hm.num_B == 16;
+        for (int b = 0; diagonal1 && b < 16; ++b) {
+            cdiag1[b] = 0.0;
+            for (int t = hm.B_start[b]; t < hm.B_start[b + 1]; ++t) {
+                if (hm.B_lm1[t] != b) diagonal1 = false;
+                else cdiag1[b] += hm.B_c[t];
+            }
+        }
+        // the edge kernels read the tables as [interval][path][channel][4 coefficients], in double in two halves of 16 bytes
+        // per channel: one load instruction of a wavefront (one path, consecutive channels) then covers contiguous memory
         auto regroup = [&](const std::vector<std::vector<double>>& tables, int nspl, DVec<F>& dst) {
             const int R = hm.spl_nodes - 1, Kc = hm.K, Pn = nspl / Kc;
             std::vector<double> out((size_t)tables.size() * R * nspl * 4);
@@ -353,8 +354,8 @@ struct Engine : EngineBase {
                                 for (int q = h; q < h + V; ++q) out[o++] = t[((size_t)n * 4 + q) * nspl + pth * Kc + k];
             upload_as(dst, out, s);
         };
-        if (!slice_CH0) regroup(hm.tables0, hm.nspl0, tabK0);
-        if (!slice_CH1) regroup(hm.tables1, hm.nspl1, tabK1);
+        regroup(hm.tables0, hm.nspl0, tabK0);
+        regroup(hm.tables1, hm.nspl1, tabK1);
         // layer 0 couples Y_lm straight into output slot lm
         {
             std::vector<int> st(17), lm(16);
@@ -485,116 +486,6 @@ struct Engine : EngineBase {
         throw Error(SMX_ERANGE, what + "an edge length lies outside (0, r_cut): the radial spline tables do not cover it" + then);
     }
 
-    // Regroup a radial table per channel slice, or return 0 when the slice path does not apply.
-    int build_slice_table(const std::vector<std::vector<double>>& tables, int nspl, DVec<F>& dst, DVec<F>& edst, DVec<F>& fdst,
-                          hipStream_t s)
-    {
-        // One radial table only (species-independent radial functions, as models without a distance transform
-        // have).  A slice kernel holds one table at a time: with several, every table is a pass over all edges of
-        // which only its share does work, and already at three tables (two species) the general kernels, which read
-        // whichever table an edge needs from L2, are faster (0.92 against 1.32 ms per step at 3 000 atoms).
-        const int R = hm.spl_nodes - 1, Kc = hm.K;
-        if (nspl != 4 * Kc || tables.size() != 1) return 0;
-        hipDeviceProp_t prop;
-        int dev = 0;
-        HIPCHK(hipGetDevice(&dev));
-        HIPCHK(hipGetDeviceProperties(&prop, dev));
-        num_cus = prop.multiProcessorCount;
-        // LDS a single workgroup may use (opt-in limit where the runtime reports one)
-        size_t lds_cap = prop.sharedMemPerBlock;
-        if ((size_t)prop.sharedMemPerBlockOptin > lds_cap) lds_cap = prop.sharedMemPerBlockOptin;
-        if (lds_cap > 160 * 1024) lds_cap = 160 * 1024;
-        for (int CH = sizeof(F) == 8 ? 4 : 8; CH >= 2; CH /= 2) {
-            // row = [4 coefficients][4 paths][CH channels], padded as the kernels of this precision want it
-            const int W = slice_row_elements<F>(CH);
-            if (W == 0) continue;
-            if ((size_t)R * W * sizeof(F) > lds_cap) continue;
-            const int S = (Kc + CH - 1) / CH;
-            std::vector<F> buf((size_t)S * R * W, F(0));
-            for (int sl = 0; sl < S; ++sl)
-                for (int n = 0; n < R; ++n)
-                    for (int q = 0; q < 4; ++q)
-                        for (int pth = 0; pth < 4; ++pth)
-                            for (int c = 0; c < CH; ++c) {
-                                const int k = sl * CH + c;
-                                if (k < Kc)
-                                    buf[((size_t)sl * R + n) * W + (q * 4 + pth) * CH + c] =
-                                        (F)tables[0][((size_t)n * 4 + q) * nspl + pth * Kc + k];
-                            }
-            dst.upload(buf.data(), buf.size(), s);
-            HIPCHK(hipStreamSynchronize(s));
-            slice_W = W;
-            // adjoint kernel with one lane per edge: CH channels are 32 bytes, table slice and the staged adjoint
-            // rows of twelve wavefronts fit the LDS
-            edge_lanes = CH * sizeof(F) == 32 && slice_edge_lds_bytes<F>(hm.spl_nodes) <= lds_cap;
-            if (edge_lanes) {
-                const int We = slice_edge_row_elements<F>();
-                std::vector<F> eb((size_t)S * R * We, F(0));
-                for (size_t rowi = 0; rowi < (size_t)S * R; ++rowi)
-                    std::copy(buf.begin() + rowi * W, buf.begin() + rowi * W + 16 * CH, eb.begin() + rowi * We);
-                edst.upload(eb.data(), eb.size(), s);
-                HIPCHK(hipStreamSynchronize(s));
-                // forward kernel of such slices: per row [4 paths][2 halves][4 lanes][channels of the lane][2], the pair
-                // being coefficients (2 half, 2 half + 1)
-                const int cpln = CH / 4, Wf = 512 / (int)sizeof(F);
-                std::vector<F> fb((size_t)S * R * Wf, F(0));
-                for (int sl = 0; sl < S; ++sl)
-                    for (int n = 0; n < R; ++n)
-                        for (int pth = 0; pth < 4; ++pth)
-                            for (int hf = 0; hf < 2; ++hf)
-                                for (int ln = 0; ln < 4; ++ln)
-                                    for (int c = 0; c < cpln; ++c)
-                                        for (int j = 0; j < 2; ++j) {
-                                            const int k = sl * CH + ln * cpln + c;
-                                            if (k < Kc)
-                                                fb[((size_t)sl * R + n) * Wf + ((((pth * 2 + hf) * 4 + ln) * cpln + c) * 2 + j)] =
-                                                    (F)tables[0][((size_t)n * 4 + 2 * hf + j) * nspl + pth * Kc + k];
-                                        }
-                fdst.upload(fb.data(), fb.size(), s);
-                HIPCHK(hipStreamSynchronize(s));
-            }
-            return CH;
-        }
-        return 0;
-    }
-    void build_slices(hipStream_t s)
-    {
-        slice_CH0 = build_slice_table(hm.tables0, hm.nspl0, tabS0, tabE0, tabF0, s);
-        if (hm.L_max == 0) {
-            // layer 1 qualifies when every output slot lm is fed by harmonic lm alone
-            bool diag = hm.num_B == 16;
-            for (int b = 0; diag && b < 16; ++b) {
-                cdiag1[b] = 0.0;
-                for (int t = hm.B_start[b]; t < hm.B_start[b + 1]; ++t) {
-                    if (hm.B_lm1[t] != b) diag = false;
-                    else cdiag1[b] += hm.B_c[t];
-                }
-            }
-            if (diag) {
-                slice_CH1 = build_slice_table(hm.tables1, hm.nspl1, tabS1, tabE1, tabF1, s);
-            }
-        }
-    }
-    SliceParams<F> slice_params(int layer, int N, bool adjoint = false)
-    {
-        SliceParams<F> p{};
-        p.a = agg_params(layer, N);
-        p.tabS = layer == 0 ? tabS0.p : tabS1.p;
-        p.W = slice_W;
-        if (!adjoint && edge_lanes) p.tabF = layer == 0 ? tabF0.p : tabF1.p;
-        if (adjoint && edge_lanes) {
-            p.edge_lanes = 1;
-            DVec<F>& te = layer == 0 ? tabE0 : tabE1;
-            if (te.p) { p.tabS = te.p; p.W = slice_edge_row_elements<F>(); }
-        }
-        p.CH = layer == 0 ? slice_CH0 : slice_CH1;
-        for (int q = 0; q < 16; ++q) p.cdiag[q] = layer == 0 ? 1.0 : cdiag1[q];
-        p.E = E;
-        p.num_cus = num_cus;
-        p.order = recv_order.p;
-        return p;
-    }
-
     // ------------------------------------------------------------------
     // geometry handling
     void set_geometry_ptrs(int N, const int* nt, const int* nn, const int* ni, const int* nty, const double* x,
@@ -650,8 +541,6 @@ struct Engine : EngineBase {
         first_neigh.size_to((size_t)N + 1, s);
         scan_tmp.size_to((size_t)N / 1024 + 2, s);
         HIPCHK(launch_scan_exclusive(num_neigh, first_neigh.p, N, scan_tmp.p, s));
-        recv_order.size_to((size_t)N, s);
-        HIPCHK(launch_degree_order(N, first_neigh.p, recv_order.p, s));
         N_geo = N;
     }
     void build_type_groups(int N)
@@ -719,6 +608,8 @@ struct Engine : EngineBase {
         p.first_neigh = first_neigh.p; p.node_types = node_types; p.neigh_types = neigh_types;
         p.xyz = xyz; p.r = r; p.T = hm.T; p.spl_nodes = hm.spl_nodes; p.spl_h = hm.spl_h; p.spl_inv_h = 1.0 / hm.spl_h;
         p.num_edges = E; p.split_nodes = split_nodes > 0 ? split_nodes : N;
+        p.table_bytes = (layer == 0 ? tabK0.n : tabK1.n) * sizeof(F);
+        for (int q = 0; q < 16; ++q) p.cdiag[q] = layer == 0 ? 1.0 : cdiag1[q];
         if (layer == 0) {
             p.gather = neigh_types; p.Hsrc = H0.p; p.tab = tab0.p; p.tabK = tabK0.p; p.pair_table = pair_table0.p;
             p.B_start = B0_start.p; p.B_lm1 = B0_lm1.p; p.B_c = B0_c.p;
@@ -733,20 +624,39 @@ struct Engine : EngineBase {
         if (!p) throw Error(SMX_EINVAL, std::string("stage called before its inputs exist: ") + what);
     }
 
+    // Whether a layer's aggregation and adjoint take the kernels for scalar sender features: a diagonal coupling, and byte
+    // offsets into the tables and the sender rows (`rows` of them) that fit 32 bits.
+    bool scalar_edges(int layer, size_t rows) const
+    {
+        if (layer == 1 && !diagonal1) return false;
+        const size_t tables = layer == 0 ? hm.tables0.size() : hm.tables1.size();
+        const size_t row = (size_t)hm.K * sizeof(F), limit = (size_t)1 << 32;
+        return tables * (hm.spl_nodes - 1) * 16 * row < limit && rows * row < limit;
+    }
+    hipError_t agg_fwd(int layer, int N, F* out)
+    {
+        auto p = agg_params(layer, N);
+        p.out = out;
+        if (scalar_edges(layer, layer == 0 ? hm.T : H1.n / hm.K)) return launch_agg0_fwd<F>(p, stream);
+        return launch_agg_fwd<F>(layer == 0 ? 0 : hm.L_max, p, stream);
+    }
+    int agg_bwd_groups(int layer) const
+    {
+        if (scalar_edges(layer, layer == 0 ? hm.T : H1.n / hm.K)) return agg0_bwd_groups<F>(hm.K);
+        return smx::agg_bwd_groups<F>(layer == 0 ? 0 : hm.L_max, hm.K);
+    }
+    hipError_t agg_bwd(int layer, const AggParams<F>& p)
+    {
+        if (scalar_edges(layer, layer == 0 ? hm.T : H1.n / hm.K)) return launch_agg0_bwd<F>(p, stream);
+        return launch_agg_bwd<F>(layer == 0 ? 0 : hm.L_max, p, stream);
+    }
+
     // ---- stages ------------------------------------------------------
     void st_agg0_fwd(int N)
     {
         need(xyz, "xyz (compute_Y)"); need(r, "r (compute_R0)"); need(first_neigh.p, "num_neigh");
         Phi0.size_to((size_t)N * 16 * K(), stream);
-        if (slice_CH0) {
-            auto sp = slice_params(0, N);
-            sp.a.out = Phi0.p;
-            HIPCHK(launch_slice_fwd<F>(sp, stream));
-            return;
-        }
-        auto p = agg_params(0, N);
-        p.out = Phi0.p;
-        HIPCHK(launch_agg_fwd<F>(0, p, stream));
+        HIPCHK(agg_fwd(0, N, Phi0.p));
     }
     template <typename TA, typename TC, typename CT>
     GemmParams<TA, TC, CT> gemm_base(int N, bool typed)
@@ -872,15 +782,7 @@ struct Engine : EngineBase {
     {
         need(xyz, "xyz (compute_Y)"); need(r, "r (compute_R1)"); need(neigh_indices, "neigh_indices");
         Phi1.size_to((size_t)N * NE() * K(), stream);
-        if (slice_CH1) {
-            auto sp = slice_params(1, N);
-            sp.a.out = Phi1.p;
-            HIPCHK(launch_slice_fwd<F>(sp, stream));
-            return;
-        }
-        auto p = agg_params(1, N);
-        p.out = Phi1.p;
-        HIPCHK(launch_agg_fwd<F>(hm.L_max, p, stream));
+        HIPCHK(agg_fwd(1, N, Phi1.p));
     }
     void st_A1(int N, bool reverse, bool from_M1 = false)
     {
@@ -948,7 +850,7 @@ struct Engine : EngineBase {
         p.H2 = H2.p; p.H2_adj = H2_adj.p; p.H1_adj = H1_adj.p; p.M1_adj = M1_adj.p;
         p.node_energies = node_energies.p; p.zero_energies = zero_energies ? 1 : 0; p.energies_copy = energies_copy;
         p.guard = guard_live(); p.guard_clear = guard_status;
-        p.guard_forces = guard_status ? node_forces.p : nullptr; p.guard_forces_n = guard_status ? (long)node_forces.n : 0;
+        p.guard_forces = guard_status ? node_forces.p : nullptr; p.guard_copy = guard_status ? forces_copy : nullptr; p.guard_forces_n = guard_status ? (long)node_forces.n : 0;
         HIPCHK(launch_tail_fused<F>(p, stream));
         if (guard_status && rows > 0) guard_clear_enqueued = true;
         energies_copy = nullptr;
@@ -964,7 +866,7 @@ struct Engine : EngineBase {
         HIPCHK(launch_readout_fused<F>(N, rows, k, nlm, node_types, E0.p, ro1.p, ro2_w1.p, ro2_w2.p, hm.readout_2_scale,
                                        H1.p, H2.p, H2_adj.p, H1_adj.p, node_energies.p, zero_energies ? 1 : 0,
                                        energies_copy, guard_live(), guard_status, guard_status ? node_forces.p : nullptr,
-                                       guard_status ? (long)node_forces.n : 0, stream));
+                                       guard_status ? forces_copy : nullptr, guard_status ? (long)node_forces.n : 0, stream));
         if (guard_status && rows > 0) guard_clear_enqueued = true;
         energies_copy = nullptr;
     }
@@ -1008,33 +910,14 @@ struct Engine : EngineBase {
         H1_adj.resize(H1.n, stream);
         const int rows = (int)(H1.n / ((size_t)nlm * k));
         const size_t row_bytes = (size_t)nlm * k * sizeof(F);
-        if (!slice_CH1 && (size_t)E1 * row_bytes > msg_limit_bytes) {
+        if ((size_t)E1 * row_bytes > msg_limit_bytes) {
             agg1_bwd_chunked(N, rows, zero_dxyz, zero_H1_adj);
             return;
         }
         msg.size_to((size_t)E1 * nlm * k, stream);
-        stage_begin(ST_AGG1B);
-        if (slice_CH1) {
-            auto sp = slice_params(1, N, true);
-            const int S = (k + sp.CH - 1) / sp.CH;
-            fpart.size_to((size_t)S * 3 * E, stream);
-            sp.a.d_out = dPhi1.p; sp.a.msg = msg.p; sp.fpart = fpart.p;
-            HIPCHK(launch_slice_bwd<F>(sp, stream));
-            stage_end(ST_AGG1B);
-            stage_begin(ST_FSUM1);
-            if (carry_forces && sp.edge_lanes && slice_CH0 == slice_CH1) {
-                // the layer-0 adjoint of the same call adds its share to these partial forces and sums once
-                carried_edges = E1;
-                carried_accumulate = zero_dxyz ? 0 : 1;
-            } else {
-                HIPCHK(launch_fpart_reduce(E1, E, S, fpart.p, node_forces.p, zero_dxyz ? 0 : 1, nullptr, stream, guard_live()));
-            }
-            stage_end(ST_FSUM1);
-        } else {
-            auto p = agg_params(1, N);
-            p.d_out = dPhi1.p; p.forces = node_forces.p; p.accumulate_forces = zero_dxyz ? 0 : 1; p.msg = msg.p;
-            agg_bwd_general(hm.L_max, p, E1, ST_AGG1B, ST_FSUM1);
-        }
+        auto p = agg_params(1, N);
+        p.d_out = dPhi1.p; p.forces = node_forces.p; p.accumulate_forces = zero_dxyz ? 0 : 1; p.msg = msg.p;
+        agg_bwd_stage(1, p, E1, ST_AGG1B, ST_FSUM1);
         stage_begin(ST_SRED);
         if (sender_rows != rows) build_sender_lists(rows);
         if (fuse_reverse_H1 && nlm == 1 && sender_reduce_linear_ok(k) && M0.n == (size_t)rows * k) {
@@ -1048,9 +931,6 @@ struct Engine : EngineBase {
         }
         stage_end(ST_SRED);
     }
-    bool carry_forces = false;      // compute() lets the layer-1 partial forces wait for the layer-0 adjoint
-    long carried_edges = 0;         // ... and the stage left them in fpart for edges [0, carried_edges)
-    int carried_accumulate = 1;
     bool fuse_reverse_H1 = false;   // compute() wants reverse_H1 folded into the sender-side sum
     bool reverse_H1_done = false;   // ... and the stage did it
     // The same stage for edge lists whose messages do not fit the staging buffer: receivers are taken in
@@ -1081,7 +961,7 @@ struct Engine : EngineBase {
             }
             nchunks = (int)std::min<long>(N, 2L * nchunks);
         }
-        const int groups = agg_bwd_groups<F>(hm.L_max, k);
+        const int groups = agg_bwd_groups(1);
         if (groups > 1) fpart.size_to((size_t)groups * 3 * E, stream);
         if (sender_rows != rows) build_sender_lists(rows);
         HIPCHK(launch_sort_buckets(s_start.p, rows, s_list.p, stream));   // the windows below need the order in memory
@@ -1091,7 +971,7 @@ struct Engine : EngineBase {
             p.node_begin = bnd[c]; p.msg_edge_begin = fe[c];
             p.d_out = dPhi1.p; p.forces = node_forces.p; p.accumulate_forces = zero_dxyz ? 0 : 1; p.msg = msg.p;
             p.fpart = groups > 1 ? fpart.p : nullptr;
-            HIPCHK(launch_agg_bwd<F>(hm.L_max, p, stream));
+            HIPCHK(agg_bwd(1, p));
             HIPCHK(launch_sender_reduce<F>(rows, nlm * k, s_start.p, s_list.p, msg.p, H1_adj.p,
                                            (c == 0 && zero_H1_adj) ? 1 : 0, true, fe[c], fe[c + 1], stream));
         }
@@ -1107,48 +987,32 @@ struct Engine : EngineBase {
     {
         need(xyz, "xyz"); need(r, "r");
         node_forces.resize((size_t)3 * E, stream);
-        if (slice_CH0) {
-            auto sp = slice_params(0, N, true);
-            const int S = (K() + sp.CH - 1) / sp.CH;
-            fpart.size_to((size_t)S * 3 * E, stream);
-            sp.a.d_out = Phi0.p; sp.a.msg = nullptr; sp.fpart = fpart.p;
-            int accumulate = 1;
-            if (carried_edges > 0) {
-                // With carried layer-1 partial forces, edges past them (ghost receivers) have only this stage's share:
-                // the sum below overwrites, so the forces must not hold anything else for them.
-                sp.fpart_carry = carried_edges;
-                accumulate = carried_accumulate;
-                carried_edges = 0;
-            }
-            stage_begin(ST_AGG0B);
-            HIPCHK(launch_slice_bwd<F>(sp, stream));
-            stage_end(ST_AGG0B);
-            stage_begin(ST_FSUM0);
-            HIPCHK(launch_fpart_reduce(E, E, S, fpart.p, node_forces.p, accumulate, forces_copy, stream, guard_live()));
-            forces_copy = nullptr;
-            stage_end(ST_FSUM0);
-            return;
-        }
         auto p = agg_params(0, N);
         p.d_out = Phi0.p; p.forces = node_forces.p; p.accumulate_forces = 1; p.msg = nullptr;
-        agg_bwd_general(0, p, E, ST_AGG0B, ST_FSUM0);
+        agg_bwd_stage(0, p, E, ST_AGG0B, ST_FSUM0);
     }
-    // general adjoint kernel; wide models are cut into channel groups whose partial forces are added in order
-    void agg_bwd_general(int L_max_H, AggParams<F>& p, long edges, int st_kernel, int st_sum)
+    // Adjoint of an aggregation; wide models are cut into channel groups whose partial forces are added in order.  The last
+    // one of an evaluation (layer 0) writes the caller's copy of the forces as well.
+    void agg_bwd_stage(int layer, AggParams<F>& p, long edges, int st_kernel, int st_sum)
     {
-        const int groups = agg_bwd_groups<F>(L_max_H, K());
+        const int groups = agg_bwd_groups(layer);
+        double* copy = layer == 0 ? forces_copy : nullptr;
         if (groups > 1) {
             fpart.size_to((size_t)groups * 3 * E, stream);
             p.fpart = fpart.p;
+        } else if (copy && scalar_edges(0, hm.T)) {
+            p.forces_copy = copy;
+            forces_copy = nullptr;
         }
         stage_begin(st_kernel);
-        HIPCHK(launch_agg_bwd<F>(L_max_H, p, stream));
+        HIPCHK(agg_bwd(layer, p));
         stage_end(st_kernel);
+        stage_begin(st_sum);
         if (groups > 1) {
-            stage_begin(st_sum);
-            HIPCHK(launch_fpart_reduce(edges, E, groups, fpart.p, node_forces.p, p.accumulate_forces, nullptr, stream, guard_live()));
-            stage_end(st_sum);
+            HIPCHK(launch_fpart_reduce(edges, E, groups, fpart.p, node_forces.p, p.accumulate_forces, copy, stream, guard_live()));
+            if (copy) forces_copy = nullptr;
         }
+        stage_end(st_sum);
     }
 
     // ------------------------------------------------------------------
@@ -1162,7 +1026,7 @@ struct Engine : EngineBase {
             // whatever was half built is not trusted by the next call
             senders_counted = false; counters_clean = 0; sender_rows = -1;
             energies_copy = nullptr; forces_copy = nullptr;
-            carried_edges = 0; carry_forces = false; fuse_reverse_H1 = false;
+            fuse_reverse_H1 = false;
             // checks of the failed call may have raised the word that only its readout launch would have cleared
             if (guard_status && !guard_clear_enqueued) (void)launch_fill<int>(guard_status, 1, 0, stream);
             (void)launch_fill<int>(flags.p + 4, 1, 0, stream);
@@ -1206,7 +1070,7 @@ struct Engine : EngineBase {
         if (N <= 65536) {
             // one launch for first_neigh, degree order, species groups, the sender histogram and the sender offsets
             hipStream_t s = stream;
-            first_neigh.size_to((size_t)N + 1, s); recv_order.size_to((size_t)N, s);
+            first_neigh.size_to((size_t)N + 1, s);
             t_start.size_to((size_t)hm.T + 1, s); t_perm.size_to((size_t)N, s);
             clean_counters(s_count, N, counters_clean);
             s_start.size_to((size_t)N + 1, s);
@@ -1214,7 +1078,7 @@ struct Engine : EngineBase {
             InputChecks chk;
             chk.status = guard_status; chk.neigh_types = neigh_types; chk.r = r; chk.r_cut = hm.r_cut; chk.num_edges = E;
             chk.num_local_nodes = N1;
-            HIPCHK(launch_node_lists_count(num_neigh, N, first_neigh.p, recv_order.p, node_types, hm.T, t_start.p, t_perm.p,
+            HIPCHK(launch_node_lists_count(num_neigh, N, first_neigh.p, node_types, hm.T, t_start.p, t_perm.p,
                                            neigh_indices, E1, N, s_count.p, s_rank.p, s_start.p, flags.p + 4, chk, s));
             N_geo = N;
             senders_counted = true;
@@ -1253,7 +1117,6 @@ struct Engine : EngineBase {
         // per-species node groups and the degree order of the receivers cover the nodes of the current stages
         auto node_lists_for = [&](int n) {
             build_type_groups(n);
-            HIPCHK(launch_degree_order(n, first_neigh.p, recv_order.p, stream));
         };
         if (N1 < N) node_lists_for(N1);
         stage_begin(ST_AGG1F); st_agg1_fwd(N1); stage_end(ST_AGG1F);
@@ -1279,10 +1142,8 @@ struct Engine : EngineBase {
         st_scale(1, N1, true);
         stage_begin(ST_REVA1); st_A1(N1, true, fuse1); stage_end(ST_REVA1);
         fuse_reverse_H1 = N1 == N; reverse_H1_done = false;
-        // (the density normalisation of layer 0 adds to the forces in between: then they must already hold the layer-1 sum)
-        carry_forces = early_forces || !hm.A0_scaled; carried_edges = 0;
         st_agg1_bwd(N1, !early_forces, false);
-        fuse_reverse_H1 = false; carry_forces = false;
+        fuse_reverse_H1 = false;
         if (N1 < N) node_lists_for(N);
         stage_begin(ST_REVH1); if (!reverse_H1_done) st_H1(N, true); stage_end(ST_REVH1);
         stage_begin(ST_REVM0); if (!fuse0) st_reverse_M0(N); stage_end(ST_REVM0);
@@ -1308,7 +1169,7 @@ struct Engine : EngineBase {
     {
         const std::string s(name);
         energies_copy = nullptr; forces_copy = nullptr;
-        carried_edges = 0; carry_forces = false; fuse_reverse_H1 = false; guard_status = nullptr; split_nodes = 0;
+        fuse_reverse_H1 = false; guard_status = nullptr; split_nodes = 0;
         materialise_adjoints(true);
         if (N < 0) throw Error(SMX_EINVAL, "negative num_nodes");
         // A stage may cover the leading nodes of a longer edge list (the pair style runs layer 1 on its local

@@ -31,6 +31,7 @@ struct AggParams {
     const F* Hsrc;            // [rows][NLM][K]
     const F* tab;             // [table][nodes-1][4][P*K]
     const F* tabK;            // the same numbers for the general edge kernels: [table][nodes-1][P][K][4], in double [table][nodes-1][P][2][K][2]
+    size_t table_bytes;       // of tabK, all tables
     const int* pair_table;    // [T(T+1)/2] -> table
     int T;
     int spl_nodes;
@@ -45,7 +46,9 @@ struct AggParams {
     int accumulate_forces;    // bwd: add to forces instead of overwriting
     F* msg;                   // bwd: [E][NLM][K] adjoint message to the sender row, or null
     double* fpart;            // bwd: [channel groups][E][3] partial forces, needed when agg_bwd_groups() > 1
+    double* forces_copy;      // bwd, scalar kernels, one channel group: receives the forces as well (or null)
     long num_edges;
+    double cdiag[16];         // scalar kernels: output lm is fed by cdiag[lm] Y_lm
     int more_terms;           // some entry of the coupling list has more than two terms
     int split_nodes;          // fwd, general kernel: receivers that decide how many wavefronts share one (the local nodes of a call with ghosts)
     // bwd, general kernel only: receivers [node_begin, num_nodes) are processed and the message of edge e goes to
@@ -60,38 +63,16 @@ template <typename F> hipError_t launch_agg_bwd(int L_max_H, const AggParams<F>&
 // fpart[group][E][3] and launch_fpart_reduce adds them up
 template <typename F> int agg_bwd_groups(int L_max_H, int K);
 
-// Channel-slice variant of the same two stages for scalar hidden features
-// (L_max = 0 path structure: output slot lm is fed by path l(lm) and harmonic lm
-// only, with a per-slot coupling constant cdiag[lm]).  tabS is the radial table
-// regrouped per slice: [slice][table][interval][W] with row content
-// [4 coefficients][4 paths][CH channels] padded to W elements.
-template <typename F>
-struct SliceParams {
-    AggParams<F> a;
-    const F* tabS;
-    const F* tabF;     // forward kernel of 32-byte slices: rows [4 paths][2 halves][4 lanes][16 bytes], or null
-    int W;             // padded row length in elements
-    int CH;            // channels per slice
-    double cdiag[16];
-    double* fpart;     // bwd: [slices][E][3] partial forces
-    long E;
-    int num_cus;
-    const int* order;     // [num_nodes] receivers by decreasing degree: entry 4t+q is row q of task t
-    int units_per_die, slot_lines, num_units, receiver_groups;   // set by the launchers: block -> (slice, receiver group)
-    long fpart_carry;     // bwd, one lane per edge: edges [0, fpart_carry) add what fpart already holds (an earlier stage's partial forces)
-    int edge_lanes;       // bwd: one lane per edge (tabS rows padded to slice_edge_row_elements, CH * sizeof(F) = 32)
-};
-// row length (elements) and LDS bytes of the adjoint kernel with one lane per edge
-template <typename F> int slice_edge_row_elements();
-template <typename F> size_t slice_edge_lds_bytes(int spl_nodes);
-// padded row length W (elements) of the per-slice table for CH channels, 0 if the kernels cannot take that CH
-template <typename F> int slice_row_elements(int CH);
-template <typename F> hipError_t launch_slice_fwd(const SliceParams<F>& p, hipStream_t s);
-template <typename F> hipError_t launch_slice_bwd(const SliceParams<F>& p, hipStream_t s);
-// forces (+)= sum over slices of fpart, slices added in ascending order
+// The same two stages for scalar sender features (path list of L_max = 0) whose coupling is diagonal (cdiag), with tables and
+// sender rows of less than 4 GiB.
+template <typename F> hipError_t launch_agg0_fwd(const AggParams<F>& p, hipStream_t s);
+template <typename F> hipError_t launch_agg0_bwd(const AggParams<F>& p, hipStream_t s);
+template <typename F> int agg0_bwd_groups(int K);
+
+// forces (+)= sum over channel groups of fpart, added in ascending order
 // (`copy`, if not null, receives the same sums: the caller's output array of the whole-pipeline call;
 // `guard`, if not null and raised, makes every force NaN instead: the evaluation was skipped)
-hipError_t launch_fpart_reduce(long edges, long E, int nslices, const double* fpart, double* forces, int accumulate,
+hipError_t launch_fpart_reduce(long edges, long E, int groups, const double* fpart, double* forces, int accumulate,
                                double* copy, hipStream_t s, const int* guard = nullptr);
 
 // H_adj[j] (+)= sum of msg[e - e_lo] over the edges e of sender j, in ascending edge order; window: over those with
@@ -171,8 +152,6 @@ hipError_t launch_scale_bwd(int N, const int* first_neigh, const int* node_types
 // ---------------------------------------------------------------------------
 // Integer list preparation
 hipError_t launch_scan_exclusive(const int* in, int* out, int n, int* block_sums, hipStream_t s);  // out[n] = total
-// order[N]: receivers by decreasing degree
-hipError_t launch_degree_order(int N, const int* first_neigh, int* order, hipStream_t s);
 // Guard of an evaluation, carried by the last launch of the sender-list build: when the checks of this evaluation
 // raised the status word, first_neigh[n_first], tstart[n_tstart] and the sender offsets are zeroed (no edges, no species
 // groups: the kernels that follow then touch no unchecked index) and the status is ORed into the sticky word the
@@ -207,10 +186,10 @@ hipError_t launch_sender_lists(const int* gather, long E, int rows, int* count, 
 hipError_t launch_sort_buckets(const int* start, int rows, int* list, hipStream_t s);
 hipError_t launch_check_counts(const int* num_neigh, int N, const int* first_neigh, int num_local_nodes, long num_edges,
                                long num_local_edges, int* status, hipStream_t s);
-// first_neigh, degree order, species groups, the sender histogram count[rows] of `key[n]` with rank[n] = the place each
+// first_neigh, species groups, the sender histogram count[rows] of `key[n]` with rank[n] = the place each
 // entry took in its bucket, and the sender offsets sstart[rows + 1], in one launch (N, rows <= 65536).  The counters and
 // *ticket must be zero on entry (every sender-list build leaves them so).
-hipError_t launch_node_lists_count(const int* num_neigh, int N, int* first_neigh, int* order, const int* node_types, int T,
+hipError_t launch_node_lists_count(const int* num_neigh, int N, int* first_neigh, const int* node_types, int T,
                                    int* tstart, int* perm, const int* key, long n, int rows, int* count, int* rank,
                                    int* sstart, int* ticket, const InputChecks& chk, hipStream_t s);
 hipError_t launch_type_groups(const int* node_types, int N, int T, int* tcount, int* tstart, int* cursor,
@@ -303,7 +282,7 @@ template <typename F>
 hipError_t launch_readout_fused(int N, int rows, int K, int num_LM, const int* node_types, const double* atomic_energies,
                                 const double* w1, const double* W1, const double* w2, double scale, const F* H1,
                                 const double* H2, double* H2_adj, F* H1_adj, double* node_energies, int zero_energies,
-                                double* energies_copy, const int* guard, int* guard_clear, double* guard_forces,
+                                double* energies_copy, const int* guard, int* guard_clear, double* guard_forces, double* guard_copy,
                                 long guard_forces_n, hipStream_t s);
 // H2 (mace.cpp:820-845), the readout tail and reverse_H2 (mace.cpp:847-874) in one launch; K a multiple of 16
 // up to 128 (tail_fused_ok).  Atoms grouped by species (perm, tstart); H1_adj [rows][num_LM][K] is written
@@ -321,6 +300,7 @@ struct TailParams {
     const int* guard;        // live status of a device-resident evaluation (or null): raised -> energies are NaN
     int* guard_clear;        // the word the input checks of the next evaluation raise (or null): cleared here
     double* guard_forces;    // raised guard: these guard_forces_n edge-force components become NaN as well (the
+    double* guard_copy;      // (and those of the caller's array, if not null)
     long guard_forces_n;     // adjoint kernels of a skipped evaluation see no edges and write none)
 };
 bool tail_fused_ok(int K);

@@ -28,8 +28,7 @@
 //   double precision  v_fmac_f64 with the row broadcast of its DPP operand (row_newbcast:n),
 //                     at the rate of the plain instruction; every 16-lane row holds the
 //                     block.
-#include "smx_device.hpp"
-#include "smx_kernels.hpp"
+#include "smx_edge_common.hpp"
 #include "smx_paths.hpp"
 
 namespace smx {
@@ -37,11 +36,6 @@ namespace smx {
 namespace {
 
 constexpr int kChunk = 16;   // edges whose geometry is formed together
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename F>
-constexpr bool kMatrix = sizeof(F) == 4;
 
 // Which entry of B[path][m][m2] (and of its two tangential derivatives) every lane and register holds.
 //   matrix form:  register g / 16, lanes 4 (g % 16) + i hold row 4 tile + i of group g; a group is one matrix
@@ -124,84 +118,8 @@ struct EdgeLds {
     static constexpr size_t total = lists + 4 * per_wave;
 };
 
-// Lane-broadcast multiply-add of the double-precision kernels: acc += (b of lane N of the lane's 16-lane row) * v.  The
-// instruction reads b through DPP: b must not come from the vector instruction right before (here it comes from LDS).
-template <int N>
-__device__ __forceinline__ void fmac_lane(double& acc, double b, double v)
-{
-    asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(b), "v"(v), "n"(N));
-}
-
-template <typename F, int CPL>
-__device__ __forceinline__ Vec<F, CPL> ldv(const F* p)
-{
-    return *reinterpret_cast<const Vec<F, CPL>*>(p);
-}
-
-// Loads and stores of a wavefront's rows: an address that is the same for all lanes, held in scalar registers, plus a 32-bit
-// offset per lane.
-template <typename T>
-__device__ __forceinline__ T load_at(const char* row, unsigned lane_bytes)
-{
-    return *reinterpret_cast<const T*>(row + lane_bytes);
-}
-// The four coefficients of one spline: 16 bytes in single precision, two halves of 16 bytes in double (a table row is
-// [path][half][K][16 bytes], so that every load instruction of a wavefront covers 1 KB without gaps).
-template <typename F>
-__device__ __forceinline__ Vec<F, 4> load_spline(const char* row, int path, unsigned K, unsigned k)
-{
-    if constexpr (sizeof(F) == 4) return load_at<Vec<F, 4>>(row + path * (K * 16), k * 16);
-    else {
-        Vec<F, 4> c;
-        const Vec<F, 2> lo = load_at<Vec<F, 2>>(row + 2 * path * (K * 16), k * 16);
-        const Vec<F, 2> hi = load_at<Vec<F, 2>>(row + (2 * path + 1) * (K * 16), k * 16);
-        c.v[0] = lo.v[0]; c.v[1] = lo.v[1]; c.v[2] = hi.v[0]; c.v[3] = hi.v[1];
-        return c;
-    }
-}
-// row n of an array of rows of that many bytes, n the same in all lanes
-__device__ __forceinline__ const char* uniform_row(const void* base, int n, unsigned row_bytes)
-{
-    return reinterpret_cast<const char*>(base) + (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(n) * row_bytes;
-}
-// The value is final here: keeps the compiler from collecting the arithmetic of several paths, whose operands would all stay
-// live (it moves plain arithmetic across scheduling fences).
-template <typename F>
-__device__ __forceinline__ void pin(F& v)
-{
-    asm volatile("" : "+v"(v));
-}
-
 // Three sums over the 64 lanes at once: on return the lanes of row 0 hold the first, of row 2 the second, of rows 1 and 3
 // the third (a fixed tree).  Two values swap halves of the wavefront and are added, which sums both over the halves.
-template <typename F>
-__device__ __forceinline__ void swap_halves(F& a, F& b)
-{
-    if constexpr (sizeof(F) == 4) {
-        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-        a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
-    } else {
-        const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
-        const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
-        const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
-        a = __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]);
-        b = __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
-    }
-}
-template <typename F>
-__device__ __forceinline__ void swap_rows(F& a, F& b)
-{
-    if constexpr (sizeof(F) == 4) {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-        a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
-    } else {
-        const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
-        const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
-        const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
-        a = __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]);
-        b = __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
-    }
-}
 template <typename F>
 __device__ __forceinline__ F wave_sum3(F s, F g1, F g2)
 {
@@ -212,17 +130,6 @@ __device__ __forceinline__ F wave_sum3(F s, F g1, F g2)
     F x = a, y = g2 + zero;          // every row: g2
     swap_rows(x, y);
     return row_sum_strided<1>(x + y);
-}
-
-// What the lanes need of an edge before its features: spline interval and argument, table row, sender row.
-template <typename F>
-__device__ __forceinline__ void edge_head(const AggParams<F>& a, int e, int ti, double& r, double& x, int& row, int& grow)
-{
-    r = a.r[e];
-    const int n = spline_interval(r, a.spl_inv_h, a.spl_nodes - 2);
-    x = r - a.spl_h * n;
-    row = a.pair_table[pair_index(a.T, ti, a.neigh_types[e])] * (a.spl_nodes - 1) + n;
-    grow = a.gather[e];
 }
 
 // The coefficients of the block entries: value v = c0 Y[o0] + c1 Y[o1] (an entry of a real coupling has at most two terms;
@@ -578,33 +485,17 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
             edge_head(a, e, ti, r, x, row, grow);
             xs[lane] = x; rows[lane] = row; grows[lane] = grow;
             if (lane < nE) {
-                const double dx = a.xyz[3 * (size_t)e], dy = a.xyz[3 * (size_t)e + 1], dz = a.xyz[3 * (size_t)e + 2];
-                const double inv = rsqrt_pos(dx * dx + dy * dy + dz * dz);
-                // radial direction as the reference forms it: xyz / r with the caller's r
+                EdgeFrame f;
+                edge_frame(a.xyz + 3 * (size_t)e, f);
                 const double ir = rcp_pos(r);
-                const double nx = dx * inv, ny = dy * inv, nz = dz * inv;
-                // t1 = n x a / |n x a| with a the axis the direction n is least aligned with (|n x a|^2 >= 2/3), t2 = n x t1
-                const double ax = fabs(nx), ay = fabs(ny), az = fabs(nz);
-                double t1x, t1y, t1z;
-                if (ax <= ay && ax <= az) { t1x = 0.0; t1y = nz; t1z = -ny; }
-                else if (ay <= az) { t1x = -nz; t1y = 0.0; t1z = nx; }
-                else { t1x = ny; t1y = -nx; t1z = 0.0; }
-                const double tn = rsqrt_pos(t1x * t1x + t1y * t1y + t1z * t1z);
-                t1x *= tn; t1y *= tn; t1z *= tn;
-                const double t2x = ny * t1z - nz * t1y, t2y = nz * t1x - nx * t1z, t2z = nx * t1y - ny * t1x;
+                // radial direction as the reference forms it: xyz / r with the caller's r
                 double* fr = us + lane * 10;
-                fr[0] = dx * ir; fr[1] = dy * ir; fr[2] = dz * ir;
-                fr[3] = t1x; fr[4] = t1y; fr[5] = t1z; fr[6] = t2x; fr[7] = t2y; fr[8] = t2z;
-                // The derivative of a harmonic of the direction along a tangent is that of its homogeneous form over the
-                // length.  The harmonics' axes are the permuted ones (z, x, y).
+                fr[0] = f.dx * ir; fr[1] = f.dy * ir; fr[2] = f.dz * ir;
+                fr[3] = f.t1x; fr[4] = f.t1y; fr[5] = f.t1z; fr[6] = f.t2x; fr[7] = f.t2y; fr[8] = f.t2z;
                 double* y = Yt + lane * 48;
                 static_for<0, 16>([&](auto lc) {
                     constexpr int lm = decltype(lc)::value;
-                    double Y, g0, g1, g2;
-                    ylm_g<lm>(nz, nx, ny, Y, g0, g1, g2);
-                    y[lm] = Y;
-                    y[16 + lm] = (g0 * t1z + g1 * t1x + g2 * t1y) * inv;
-                    y[32 + lm] = (g0 * t2z + g1 * t2x + g2 * t2y) * inv;
+                    ylm_tangential<lm>(f, y[lm], y[16 + lm], y[32 + lm]);
                     if constexpr (lm % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // short live ranges
                 });
             }
@@ -762,18 +653,6 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
     }
 }
 
-// How many wavefronts share a receiver, of `units` receivers times channel groups.  A wavefront takes 0.5 to 2 us per edge,
-// and about 2 048 of them are in flight: fewer units leave SIMDs idle, up to three rounds of them leave the last round
-// nearly empty.  The adjoint gains up to three rounds (K = 128, l <= 1, single precision, 1 500 receivers: 214, 194, 157 us
-// for one, two and four wavefronts); the forward kernel, which has to add the parts, only where the chip is not full
-// (500 receivers: 52, 38, 41 us; 3 000: 153, 160, 163).
-template <bool BWD>
-int agg_parts(long units)
-{
-    if (BWD) return units <= 2048 ? 4 : (units <= 6144 ? 2 : 1);
-    return units <= 512 ? 4 : (units <= 3072 ? 2 : 1);
-}
-
 template <typename F, int LMAXH, int CPL, bool BWD>
 hipError_t launch_agg_t(const AggParams<F>& p, hipStream_t s)
 {
@@ -867,6 +746,11 @@ template int agg_bwd_groups<float>(int, int);
 
 // ---------------------------------------------------------------------------
 namespace {
+template <typename F, int N>
+__device__ __forceinline__ Vec<F, N> ldv(const F* p)
+{
+    return *reinterpret_cast<const Vec<F, N>*>(p);
+}
 // V consecutive elements per thread (16-byte accesses when the row width allows); four messages are requested
 // before the first is added, the additions keep the ascending edge order
 // WINDOW: slist is in ascending order in memory and the messages of the edges [e_lo, e_hi) are taken; otherwise all
@@ -1051,6 +935,31 @@ template hipError_t launch_sender_reduce_linear<float>(int, int, const int*, int
 
 template hipError_t launch_sender_reduce<double>(int, int, const int*, int*, const double*, double*, int, bool, long, long, hipStream_t);
 template hipError_t launch_sender_reduce<float>(int, int, const int*, int*, const float*, float*, int, bool, long, long, hipStream_t);
+
+// ---------------------------------------------------------------------------
+namespace {
+__global__ void k_fpart_reduce(long n3, long stride3, int groups, const double* fpart, double* forces, int accumulate,
+                               double* copy, const int* guard)
+{
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n3) return;
+    double s = accumulate ? forces[t] : 0.0;
+    for (int q = 0; q < groups; ++q) s += fpart[(size_t)q * stride3 + t];
+    // a skipped evaluation (inputs failed their checks) left nothing in fpart: its forces say so
+    if (guard && *guard) s = __builtin_nan("");
+    forces[t] = s;
+    if (copy) copy[t] = s;
+}
+}  // namespace
+hipError_t launch_fpart_reduce(long edges, long E, int groups, const double* fpart, double* forces, int accumulate,
+                               double* copy, hipStream_t s, const int* guard)
+{
+    const long n3 = 3 * edges;
+    if (n3 <= 0 || edges > E) return n3 <= 0 ? hipSuccess : hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_fpart_reduce, dim3((unsigned)((n3 + 255) / 256)), dim3(256), 0, s, n3, 3 * E, groups, fpart,
+                       forces, accumulate, copy, guard);
+    return hipGetLastError();
+}
 
 // ---------------------------------------------------------------------------
 namespace {

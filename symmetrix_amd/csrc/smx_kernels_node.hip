@@ -163,47 +163,6 @@ __global__ __launch_bounds__(1024) void k_type_groups(const int* node_types, int
     extern __shared__ int sh[];
     type_groups_body(node_types, N, T, tstart, perm, sh);
 }
-// Receivers in order of decreasing degree (counting sort on min(degree, 1023), one block).  The edge
-// kernels hand consecutive entries to the rows of a wavefront, which then finish together; the order
-// inside a degree class is whatever the LDS atomics leave and has no influence on any result.
-// `v` holds the CSR offsets (counts == false) or the degrees themselves (counts == true).
-__device__ void degree_order_body(int N, const int* v, int* order, bool counts = false)
-{
-    __shared__ int start[1024];
-    __shared__ int cur[1024];
-    __shared__ int wsum[16];
-    const int tid = threadIdx.x;
-    start[tid] = 0; cur[tid] = 0;
-    __syncthreads();
-    for (int i = tid; i < N; i += 1024) {
-        const int d = min(max(counts ? v[i] : v[i + 1] - v[i], 0), 1023);   // a negative count must not index below the table
-        atomicAdd(&start[1023 - d], 1);
-    }
-    __syncthreads();
-    // exclusive scan of the 1024 counts: wavefront scans, then the 16 wavefront totals
-    const int c = start[tid];
-    int incl = c;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int o = __shfl_up(incl, off, 64);
-        if ((tid & 63) >= off) incl += o;
-    }
-    if ((tid & 63) == 63) wsum[tid >> 6] = incl;
-    __syncthreads();
-    int base = 0;
-    for (int w = 0; w < (tid >> 6); ++w) base += wsum[w];
-    __syncthreads();
-    start[tid] = base + incl - c;
-    __syncthreads();
-    for (int i = tid; i < N; i += 1024) {
-        const int b = 1023 - min(max(counts ? v[i] : v[i + 1] - v[i], 0), 1023);
-        order[start[b] + atomicAdd(&cur[b], 1)] = i;
-    }
-}
-__global__ __launch_bounds__(1024) void k_degree_order(int N, const int* first_neigh, int* order)
-{
-    degree_order_body(N, first_neigh, order);
-}
 __global__ void k_check_range(const int* v, long n, int limit, int* flags)
 {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -247,11 +206,11 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_single(const int* in, int* 
 {
     scan_single_body(in, out, n);
 }
-__device__ void node_lists_part(const int* num_neigh, int N, int* first_neigh, int* order, const int* node_types, int T,
+__device__ void node_lists_part(const int* num_neigh, int N, int* first_neigh, const int* node_types, int T,
                                 int* tstart, int* perm, const int* key, long n, int rows, int* count, int* rank,
                                 const InputChecks& chk, int* sh)
 {
-    // the three node lists are independent of each other: a block each
+    // the two node lists are independent of each other: a block each
     if (blockIdx.x == 0) {
         scan_single_body(num_neigh, first_neigh, N);
         __syncthreads();   // first_neigh, written by this block, is read back below
@@ -263,9 +222,8 @@ __device__ void node_lists_part(const int* num_neigh, int N, int* first_neigh, i
         }
         return;
     }
-    if (blockIdx.x == 1) { degree_order_body(N, num_neigh, order, true); return; }
-    if (blockIdx.x == 2) { type_groups_body(node_types, N, T, tstart, perm, sh); return; }
-    constexpr int LIST_BLOCKS = 3;
+    if (blockIdx.x == 1) { type_groups_body(node_types, N, T, tstart, perm, sh); return; }
+    constexpr int LIST_BLOCKS = 2;
     for (long i = (long)(blockIdx.x - LIST_BLOCKS) * SCAN_BLOCK + threadIdx.x; i < n; i += (long)(gridDim.x - LIST_BLOCKS) * SCAN_BLOCK) {
         const int j = key[i];
         if (j >= 0 && j < rows) rank[i] = atomicAdd(&count[j], 1);   // the entry's place inside its bucket
@@ -283,20 +241,20 @@ __device__ void node_lists_part(const int* num_neigh, int N, int* first_neigh, i
         if (bad) atomicOr(chk.status, bad);
     }
 }
-// The node-level lists of one evaluation and its sender histogram in one launch: blocks 0, 1, 2 form one node list each
-// (first_neigh = exclusive scan of num_neigh, receivers by decreasing degree, species groups), the other blocks count the
+// The node-level lists of one evaluation and its sender histogram in one launch: blocks 0 and 1 form one node list each
+// (first_neigh = exclusive scan of num_neigh, species groups), the other blocks count the
 // senders (counters at zero on entry), which does not depend on the node lists.  With a ticket, the block that finishes last
 // turns the histogram into the sender offsets: a launch of its own costs 6 to 8 us of a small evaluation, but the fences of
 // the ticket cost more than that over many blocks (80 us over 2 048), so the launcher hands out tickets to small grids only.
 // With `chk.status` set the launch also checks everything the later kernels use as an address or a table argument
 // (species, sender rows, edge lengths, counts that add up to the edge totals) and raises bits in the status word.
-__global__ __launch_bounds__(SCAN_BLOCK) void k_node_lists_count(const int* num_neigh, int N, int* first_neigh, int* order,
+__global__ __launch_bounds__(SCAN_BLOCK) void k_node_lists_count(const int* num_neigh, int N, int* first_neigh,
                                                                 const int* node_types, int T, int* tstart, int* perm,
                                                                 const int* key, long n, int rows, int* count, int* rank,
                                                                 int* sstart, int* ticket, InputChecks chk)
 {
     extern __shared__ int sh[];
-    node_lists_part(num_neigh, N, first_neigh, order, node_types, T, tstart, perm, key, n, rows, count, rank, chk, sh);
+    node_lists_part(num_neigh, N, first_neigh, node_types, T, tstart, perm, key, n, rows, count, rank, chk, sh);
     if (!ticket) return;
     // every block's counts are out before it takes its ticket
     __shared__ int last;
@@ -323,7 +281,7 @@ __global__ void k_check_counts(const int* num_neigh, int N, const int* first_nei
 }
 }  // namespace
 
-hipError_t launch_node_lists_count(const int* num_neigh, int N, int* first_neigh, int* order, const int* node_types, int T,
+hipError_t launch_node_lists_count(const int* num_neigh, int N, int* first_neigh, const int* node_types, int T,
                                    int* tstart, int* perm, const int* key, long n, int rows, int* count, int* rank,
                                    int* sstart, int* ticket, const InputChecks& chk, hipStream_t s)
 {
@@ -332,7 +290,7 @@ hipError_t launch_node_lists_count(const int* num_neigh, int N, int* first_neigh
     const unsigned nb = 3 + (unsigned)std::max<long>(1, std::min<long>((work + SCAN_BLOCK - 1) / SCAN_BLOCK, 2048));
     const bool with_scan = nb <= 160;
     hipLaunchKernelGGL(k_node_lists_count, dim3(nb), dim3(SCAN_BLOCK), 2 * T * sizeof(int), s, num_neigh, N, first_neigh,
-                       order, node_types, T, tstart, perm, key, n, rows, count, rank, sstart, with_scan ? ticket : nullptr, chk);
+                       node_types, T, tstart, perm, key, n, rows, count, rank, sstart, with_scan ? ticket : nullptr, chk);
     if (!with_scan) hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(SCAN_BLOCK), 0, s, count, sstart, rows);
     return hipGetLastError();
 }
@@ -386,12 +344,6 @@ hipError_t launch_type_groups(const int* node_types, int N, int T, int* tcount, 
     // order inside a species group is left as placed: every output row of the products
     // that use this grouping is computed independently of its tile mates
     hipLaunchKernelGGL(k_type_groups, dim3(1), dim3(1024), 2 * T * sizeof(int), s, node_types, N, T, tstart, perm);
-    return hipGetLastError();
-}
-
-hipError_t launch_degree_order(int N, const int* first_neigh, int* order, hipStream_t s)
-{
-    if (N > 0) hipLaunchKernelGGL(k_degree_order, dim3(1), dim3(1024), 0, s, N, first_neigh, order);
     return hipGetLastError();
 }
 
@@ -699,7 +651,7 @@ __global__ __launch_bounds__(256) void k_readout_fused(int N, int rows, int K, i
                                                        const double* w2, double scale, const F* H1, const double* H2,
                                                        double* H2_adj, F* H1_adj, double* node_energies,
                                                        int zero_energies, double* energies_copy, const int* guard,
-                                                       int* guard_clear, double* guard_forces, long guard_forces_n)
+                                                       int* guard_clear, double* guard_forces, double* guard_copy, long guard_forces_n)
 {
     extern __shared__ double rsm[];
     // every reader of the check word has run (the sender lists come before the readout): clean for the next evaluation
@@ -712,8 +664,10 @@ __global__ __launch_bounds__(256) void k_readout_fused(int N, int rows, int K, i
             node_energies[i] = __builtin_nan("");
             if (energies_copy) energies_copy[i] = __builtin_nan("");
         }
-        for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < guard_forces_n; t += (long)gridDim.x * 256)
+        for (long t = (long)blockIdx.x * 256 + threadIdx.x; t < guard_forces_n; t += (long)gridDim.x * 256) {
             guard_forces[t] = __builtin_nan("");
+            if (guard_copy) guard_copy[t] = __builtin_nan("");
+        }
         return;
     }
     const int ldw = K + 1;                 // rows of W1 start two banks apart
@@ -805,8 +759,10 @@ __global__ __launch_bounds__(TAIL_BLOCK) void k_tail_fused(const TailParams<F> p
             if (p.energies_copy) p.energies_copy[i] = __builtin_nan("");
         }
         // ... and so do the edge forces, which the adjoint kernels will not touch (they see no edges)
-        for (long t = (long)blockIdx.x * TAIL_BLOCK + tid; t < p.guard_forces_n; t += (long)gridDim.x * TAIL_BLOCK)
+        for (long t = (long)blockIdx.x * TAIL_BLOCK + tid; t < p.guard_forces_n; t += (long)gridDim.x * TAIL_BLOCK) {
             p.guard_forces[t] = __builtin_nan("");
+            if (p.guard_copy) p.guard_copy[t] = __builtin_nan("");
+        }
         return;
     }
     // rows beyond the atoms (ghost rows of H1_adj) are cleared by all blocks together
@@ -975,7 +931,7 @@ hipError_t launch_readout_fused(int N, int rows, int K, int num_LM, const int* n
                                 const double* w1, const double* W1, const double* w2, double scale, const F* H1,
                                 const double* H2, double* H2_adj, F* H1_adj, double* node_energies, int zero_energies,
                                 double* energies_copy, const int* guard, int* guard_clear, double* guard_forces,
-                                long guard_forces_n, hipStream_t s)
+                                double* guard_copy, long guard_forces_n, hipStream_t s)
 {
     if (rows < N) return hipErrorInvalidValue;
     if (rows <= 0) return hipSuccess;
@@ -988,11 +944,11 @@ hipError_t launch_readout_fused(int N, int rows, int K, int num_LM, const int* n
     }
     hipLaunchKernelGGL(k_readout_fused<F>, dim3((rows + 15) / 16), dim3(256), lds, s, N, rows, K, num_LM, node_types,
                        atomic_energies, w1, W1, w2, scale, H1, H2, H2_adj, H1_adj, node_energies, zero_energies,
-                       energies_copy, guard, guard_clear, guard_forces, guard_forces_n);
+                       energies_copy, guard, guard_clear, guard_forces, guard_copy, guard_forces_n);
     return hipGetLastError();
 }
-template hipError_t launch_readout_fused<double>(int, int, int, int, const int*, const double*, const double*, const double*, const double*, double, const double*, const double*, double*, double*, double*, int, double*, const int*, int*, double*, long, hipStream_t);
-template hipError_t launch_readout_fused<float>(int, int, int, int, const int*, const double*, const double*, const double*, const double*, double, const float*, const double*, double*, float*, double*, int, double*, const int*, int*, double*, long, hipStream_t);
+template hipError_t launch_readout_fused<double>(int, int, int, int, const int*, const double*, const double*, const double*, const double*, double, const double*, const double*, double*, double*, double*, int, double*, const int*, int*, double*, double*, long, hipStream_t);
+template hipError_t launch_readout_fused<float>(int, int, int, int, const int*, const double*, const double*, const double*, const double*, double, const float*, const double*, double*, float*, double*, int, double*, const int*, int*, double*, double*, long, hipStream_t);
 
 
 // ===========================================================================

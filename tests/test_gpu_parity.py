@@ -885,17 +885,20 @@ def test_senders_with_many_edges(gpu, tmp_models, L_max, K, edge):
     (70, 1, 40, 37, 1), (130, 1, 24, 35, 1), (33, 2, 24, 34, 1), (70, 0, 40, 50, 1),
     # two wavefronts per receiver, then one, in either direction
     (16, 1, 515, 9, 1), (16, 1, 2051, 5, 1), (16, 1, 3075, 3, 1), (16, 1, 6147, 3, 1),
+    # scalar sender features: two edges at a time in chunks of 44 and 62, one to four channels per lane and an edge alone,
+    # channel groups that do not fill their lanes; at 48 channels tables beyond an L2 (four groups)
+    (20, 0, 40, 67, 1), (33, 0, 40, 60, 1), (65, 0, 12, 270, 1), (97, 0, 12, 270, 1), (130, 0, 24, 90, 1), (48, 0, 24, 40, 1),
     # coupling entries of three terms
     (32, 1, 20, 20, 3), (32, 2, 20, 20, 3),
 ])
 def test_general_edge_kernels_at_the_edges_of_their_split(gpu, tmp_models, K, L_max, receivers, max_degree, terms, dtype):
-    model = H.tiny_model(K=K, L_max=L_max, n_pts=24, seed=K + L_max, pair=True)
+    model = H.tiny_model(K=K, L_max=L_max, n_pts=180 if K == 48 else 24, seed=K + L_max, pair=True)
     if terms > 1:   # every coefficient as a sum of three
         for key in ("Phi1_lme", "Phi1_lelm1lm2"):
             model[key] = [v for v in model[key] for _ in range(terms)]
         model["Phi1_clebsch_gordan"] = [v * w for v in model["Phi1_clebsch_gordan"] for w in (0.5, 0.75, -0.25)]
     rng = np.random.default_rng(receivers)
-    degree = np.array([n % (max_degree + 1) for n in range(receivers)])
+    degree = np.linspace(0, max_degree, receivers).astype(int) if max_degree > receivers else np.arange(receivers) % (max_degree + 1)
     E = int(degree.sum())
     species = rng.integers(0, 3, size=receivers).astype(np.int32)
     senders = rng.integers(0, receivers, size=E).astype(np.int32)
