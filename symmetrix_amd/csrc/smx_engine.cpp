@@ -231,6 +231,8 @@ template <typename F>
 struct Engine : EngineBase {
     // ---- model on device
     DVec<F> tab0, tab1, tabK0, tabK1, H0, A0w, H1w, A1w;
+    DVec<F> linA0, linA0T, linA1, linA1T;    // the same weights in operand order (operand_weights)
+    DVec<F> M0_coef16, M1_coef16;            // contraction coefficients by column tile
     DVec<int> pair_table0, pair_table1;
     DVec<int> B0_start, B0_lm1, B1_start, B1_lm1;
     DVec<double> B0_c, B1_c;
@@ -300,6 +302,7 @@ struct Engine : EngineBase {
     long rf_clean = 0;              // the same for rf_count
 
     // ---- state (mace.hpp members)
+    DVec<F> dPhi0;     // adjoint of Phi0 where Phi0 stays (separate_dPhi0), else it takes Phi0's place
     DVec<F> Phi0, A0, A0_adj, M0, M0_grad, M0_adj, H1, H1_adj, Phi1, dPhi1, A1, A1_adj, M1, M1_grad, M1_adj, msg;
     DVec<double> H2, H2_adj, node_energies, node_forces, scratch_d;
 
@@ -420,8 +423,9 @@ struct Engine : EngineBase {
         M0_tables = M0_tables && poly_spec_shape((int)sizeof(F), hm.K, hm.num_LM).CB > 0;
         M1_tables = M1_tables && poly_spec_shape((int)sizeof(F), hm.K, 1).CB > 0;
         // slabs of the straight-line kernel: [species][channel block][monomial / V][CB][V]
-        auto slabs = [&](DVec<F>& dst, const PolySpec* polys, int NP) {
-            const PolySpecShape sh = poly_spec_shape((int)sizeof(F), hm.K, NP);
+        auto slabs = [&](DVec<F>& dst, const PolySpec* polys, int NP, bool by_column_tile) {
+            PolySpecShape sh = poly_spec_shape((int)sizeof(F), hm.K, NP);
+            if (by_column_tile) { sh.CB = 16; sh.kblocks = hm.K / 16; sh.slab_bytes = (unsigned)(poly_spec_offset(NP) * 16 * sizeof(F)); }
             constexpr int V = 16 / (int)sizeof(F);
             const size_t slab = sh.slab_bytes / sizeof(F);
             std::vector<F> h((size_t)hm.T * sh.kblocks * slab, F(0));
@@ -443,12 +447,53 @@ struct Engine : EngineBase {
             HIPCHK(hipGetDeviceProperties(&prop, device));
             num_cus = prop.multiProcessorCount;
         }
-        if (M0_tables) slabs(M0_slabs, hm.P0.data(), hm.num_LM);
-        if (M1_tables) slabs(M1_slabs, &hm.P1, 1);
+        if (M0_tables) slabs(M0_slabs, hm.P0.data(), hm.num_LM, false);
+        if (M1_tables) slabs(M1_slabs, &hm.P1, 1, false);
+        if (linear_ok(hm.K)) {
+            if (M0_tables) slabs(M0_coef16, hm.P0.data(), hm.num_LM, true);
+            if (M1_tables) slabs(M1_coef16, &hm.P1, 1, true);
+            operand_weights(s);
+        }
         poly_tables = (M0_tables ? 1 : 0) | (M1_tables ? 2 : 0);
         flags.resize(8, s);
         sticky.room(2); sticky.p[0] = sticky.p[1] = 0;
         HIPCHK(hipStreamSynchronize(s));
+    }
+
+    // Weights of the A-basis linears in the operand order of k_linear, [l][type][output block][column tile][step][64][V]:
+    // forward, and transposed for the adjoints.
+    void operand_weights(hipStream_t s)
+    {
+        const int K = hm.K;
+        constexpr int V = 16 / (int)sizeof(F);
+        std::vector<double> out;
+        // B(k, n) of a block of K columns
+        auto block = [&](int inner, auto&& B) {
+            for (int ct = 0; ct < K / 16; ++ct)
+                for (int st = 0; st < inner / (4 * V); ++st)
+                    for (int lane = 0; lane < 64; ++lane)
+                        for (int v = 0; v < V; ++v) out.push_back(B(4 * V * st + lane / 16 * V + v, ct * 16 + lane % 16));
+        };
+        auto done = [&](DVec<F>& dst) { upload_as(dst, out, s); out.clear(); };
+        for (int pass = 0; pass < 2; ++pass) {
+            for (int l = 0; l < 4; ++l)
+                for (int t = 0; t < hm.T; ++t) {
+                    const double* w = hm.A0_weights.data() + ((size_t)t * 4 + l) * K * K;
+                    block(K, [&](int k, int n) { return pass ? w[(size_t)n * K + k] : w[(size_t)k * K + n]; });
+                }
+            done(pass ? linA0T : linA0);
+        }
+        for (int l = 0; l < 4; ++l) {
+            const double* w = hm.A1_weights[l].data();
+            block(hm.num_e[l] * K, [&](int k, int n) { return w[(size_t)k * K + n]; });
+        }
+        done(linA1);
+        for (int l = 0; l < 4; ++l)
+            for (int eb = 0; eb < hm.num_e[l]; ++eb) {
+                const double* w = hm.A1_weights[l].data();
+                block(K, [&](int k, int n) { return w[((size_t)eb * K + n) * K + k]; });
+            }
+        done(linA1T);
     }
 
     // ---- input checks of an evaluation.  flags[0]: stage-level calls (read back at once); flags[2]: the word the checks
@@ -679,6 +724,81 @@ struct Engine : EngineBase {
         q.Kd = Kd; q.Nn = Nn; q.sub = sub;
         return q;
     }
+    LinearParams<F> linear_A0(int N, bool reverse)
+    {
+        const int k = K();
+        LinearParams<F> q{};
+        need(t_perm.p, "species groups");
+        q.num_nodes = N; q.K = k; q.T = hm.T; q.perm = t_perm.p; q.tstart = t_start.p;
+        q.W = reverse ? linA0T.p : linA0.p;
+        q.a_node_stride = q.out_node_stride = 16L * k; q.num_e_max = 1;
+        for (int lm = 0; lm < 16; ++lm) q.row_off[lm] = q.out_off[lm] = lm * k;
+        for (int l = 0; l < 4; ++l) {
+            q.inner[l] = k; q.num_e[l] = 1;
+            q.w_off[l] = (size_t)l * hm.T * k * k; q.w_type_stride[l] = (size_t)k * k;
+        }
+        return q;
+    }
+    // (`groups`: the contraction behind it depends on the species)
+    LinearParams<F> linear_A1(int N, bool reverse, bool groups)
+    {
+        const int k = K(), ne = NE();
+        LinearParams<F> q{};
+        q.num_nodes = N; q.K = k; q.T = hm.T;
+        if (groups) { need(t_perm.p, "species groups"); q.perm = t_perm.p; q.tstart = t_start.p; }
+        q.W = reverse ? linA1T.p : linA1.p;
+        (reverse ? q.out_node_stride : q.a_node_stride) = (long)ne * k;
+        (reverse ? q.a_node_stride : q.out_node_stride) = 16L * k;
+        size_t off = 0;
+        int lme = 0;
+        q.num_e_max = 1;
+        for (int l = 0; l < 4; ++l) {
+            const int nel = hm.num_e[l];
+            q.inner[l] = reverse ? k : nel * k; q.num_e[l] = reverse ? nel : 1;
+            q.num_e_max = std::max(q.num_e_max, q.num_e[l]);
+            q.w_off[l] = off;
+            off += (size_t)nel * k * k;
+            for (int m = 0; m < 2 * l + 1; ++m) {
+                const int lm = l * l + m;
+                (reverse ? q.out_off : q.row_off)[lm] = (lme + m * nel) * k;
+                (reverse ? q.row_off : q.out_off)[lm] = lm * k;
+            }
+            lme += (2 * l + 1) * nel;
+        }
+        return q;
+    }
+    // Whether the A-basis linears of N nodes take k_linear: it streams its operands through blocks of 16 atoms, and with few
+    // atoms the latency of that stream is longer than the row-streaming kernel and a contraction launch take (107 atoms of the
+    // l <= 1 model in double precision: 61 + 64 us against 28 + 69; 501 of the scalar one in single: 21 against 22; 1 000 in double 38
+    // against 48).  The local nodes decide, so that a call with ghost nodes gives the bits of one without.
+    bool use_linear(int N) const { return linear_ok(K()) && (split_nodes > 0 ? split_nodes : N) >= 512; }
+    // The layer-0 adjoint linear writes over Phi0, unless the evaluation keeps Phi0 to form A0 from it on request: with one
+    // polynomial per channel and no density normalisation A0 only ever exists in the registers of the contraction.
+    bool fused_contraction(int layer, int N) const
+    {
+        return use_linear(N) && !(layer == 0 ? hm.A0_scaled : hm.A1_scaled) && (layer == 0 ? M0_tables : M1_tables);
+    }
+    bool separate_dPhi0(int N) const { return fused_contraction(0, N) && NLM() == 1; }
+    // A0 (or A1) and its contraction in one launch
+    void st_linear_contraction(int layer, int N)
+    {
+        const size_t k = K();
+        if (layer == 0) {
+            A0.size_to((size_t)N * 16 * k, stream); M0.size_to((size_t)N * NLM() * k, stream);
+            auto q = linear_A0(N, false);
+            q.A = Phi0.p; q.M = M0.p; q.coef = M0_coef16.p;
+            const bool one = NLM() == 1;
+            if (one) { M0_grad.size_to((size_t)N * 16 * k, stream); q.M_grad = M0_grad.p; pending_A0 = N; }
+            else q.out = A0.p;
+            HIPCHK(launch_linear<F>(q, one ? 0 : 1, NLM(), stream));
+        } else {
+            A1.size_to((size_t)N * 16 * k, stream); M1.size_to((size_t)N * k, stream); M1_grad.size_to((size_t)N * 16 * k, stream);
+            auto q = linear_A1(N, false, true);
+            q.A = Phi1.p; q.M = M1.p; q.M_grad = M1_grad.p; q.coef = M1_coef16.p;
+            pending_A1 = N;
+            HIPCHK(launch_linear<F>(q, 0, 1, stream));
+        }
+    }
     // A0[i, l-block] = Phi0[i, l-block] . A0_weights[type_i][l]  (reverse: transposed weights)
     // `from_M0`: the adjoint product takes M0_grad . M0_adj (one polynomial per channel) as its operand
     // instead of a stored A0_adj
@@ -686,8 +806,15 @@ struct Engine : EngineBase {
     {
         const int k = K();
         const F* src = reverse ? (from_M0 ? M0_grad.p : A0_adj.p) : Phi0.p;
-        if (reverse) Phi0.size_to((size_t)N * 16 * k, stream); else A0.size_to((size_t)N * 16 * k, stream);
-        F* dst = reverse ? Phi0.p : A0.p;
+        DVec<F>& to = reverse ? (separate_dPhi0(N) ? dPhi0 : Phi0) : A0;
+        to.size_to((size_t)N * 16 * k, stream);
+        F* dst = to.p;
+        if (use_linear(N)) {
+            auto q = linear_A0(N, reverse);
+            q.A = src; q.out = dst; q.scale = from_M0 ? M0_adj.p : nullptr;
+            HIPCHK(launch_linear<F>(q, 2, 1, stream));
+            return;
+        }
         auto g = gemm_base<F, F, F>(N, true);
         g.nprob = 4;
         for (int l = 0; l < 4; ++l) {
@@ -788,6 +915,13 @@ struct Engine : EngineBase {
     {
         const int k = K(), ne = NE();
         if (reverse) dPhi1.size_to(Phi1.n, stream); else A1.size_to((size_t)N * 16 * k, stream);
+        if (use_linear(N)) {
+            auto q = linear_A1(N, reverse, false);
+            q.A = reverse ? (from_M1 ? M1_grad.p : A1_adj.p) : Phi1.p; q.out = reverse ? dPhi1.p : A1.p;
+            q.scale = from_M1 ? M1_adj.p : nullptr;
+            HIPCHK(launch_linear<F>(q, 2, 1, stream));
+            return;
+        }
         long lme_off = 0;
         auto g = gemm_base<F, F, F>(N, false);
         g.nprob = 4;
@@ -872,9 +1006,16 @@ struct Engine : EngineBase {
     }
     // node counts for which compute() left A1_adj / A0_adj unwritten (-1: they are current)
     int pending_A1_adj = -1, pending_A0_adj = -1;
+    int pending_A1 = -1, pending_A0 = -1;       // the same for A1 and A0 (st_linear_contraction)
     int pending_M0_grad = -1;   // compute() kept no layer-0 gradients for this many nodes: formed when somebody asks
+    void materialise_A()
+    {
+        if (pending_A0 >= 0) { const int n = pending_A0; pending_A0 = -1; if (n > 0) st_A0_lin(n, false); }
+        if (pending_A1 >= 0) { const int n = pending_A1; pending_A1 = -1; if (n > 0) st_A1(n, false); }
+    }
     void materialise_adjoints(bool gradients)
     {
+        if (gradients) materialise_A();
         if (pending_A1_adj >= 0) { st_reverse_M1(pending_A1_adj); pending_A1_adj = -1; }
         if (pending_A0_adj >= 0) { st_reverse_M0(pending_A0_adj); pending_A0_adj = -1; }
         if (gradients && pending_M0_grad >= 0) {
@@ -988,7 +1129,7 @@ struct Engine : EngineBase {
         need(xyz, "xyz"); need(r, "r");
         node_forces.resize((size_t)3 * E, stream);
         auto p = agg_params(0, N);
-        p.d_out = Phi0.p; p.forces = node_forces.p; p.accumulate_forces = 1; p.msg = nullptr;
+        p.d_out = separate_dPhi0(N) ? dPhi0.p : Phi0.p; p.forces = node_forces.p; p.accumulate_forces = 1; p.msg = nullptr;
         agg_bwd_stage(0, p, E, ST_AGG0B, ST_FSUM0);
     }
     // Adjoint of an aggregation; wide models are cut into channel groups whose partial forces are added in order.  The last
@@ -1109,10 +1250,16 @@ struct Engine : EngineBase {
             st_zbl(N1);
         }
         stage_begin(ST_AGG0F); st_agg0_fwd(N); stage_end(ST_AGG0F);
-        stage_begin(ST_A0LIN); st_A0_lin(N, false); stage_end(ST_A0LIN);
-        st_scale(0, N, false);
+        pending_A0 = pending_A1 = -1;
         pending_M0_grad = recompute_M0_grad() ? N : -1;
-        stage_begin(ST_M0); st_poly(N, false, pending_M0_grad >= 0 ? 1 : 0); stage_end(ST_M0);
+        if (fused_contraction(0, N)) {
+            stage_begin(ST_A0LIN); st_linear_contraction(0, N); stage_end(ST_A0LIN);
+            stage_begin(ST_M0); stage_end(ST_M0);
+        } else {
+            stage_begin(ST_A0LIN); st_A0_lin(N, false); stage_end(ST_A0LIN);
+            st_scale(0, N, false);
+            stage_begin(ST_M0); st_poly(N, false, pending_M0_grad >= 0 ? 1 : 0); stage_end(ST_M0);
+        }
         stage_begin(ST_H1); st_H1(N, false); stage_end(ST_H1);
         // per-species node groups and the degree order of the receivers cover the nodes of the current stages
         auto node_lists_for = [&](int n) {
@@ -1120,9 +1267,14 @@ struct Engine : EngineBase {
         };
         if (N1 < N) node_lists_for(N1);
         stage_begin(ST_AGG1F); st_agg1_fwd(N1); stage_end(ST_AGG1F);
-        stage_begin(ST_A1); st_A1(N1, false); stage_end(ST_A1);
-        st_scale(1, N1, false);
-        stage_begin(ST_M1); st_poly(N1, true); stage_end(ST_M1);
+        if (fused_contraction(1, N1)) {
+            stage_begin(ST_A1); st_linear_contraction(1, N1); stage_end(ST_A1);
+            stage_begin(ST_M1); stage_end(ST_M1);
+        } else {
+            stage_begin(ST_A1); st_A1(N1, false); stage_end(ST_A1);
+            st_scale(1, N1, false);
+            stage_begin(ST_M1); st_poly(N1, true); stage_end(ST_M1);
+        }
         if (tail_fused_ok(K())) {
             stage_begin(ST_H2); st_tail(N1, !hm.has_zbl); stage_end(ST_H2);
             stage_begin(ST_READOUT); stage_end(ST_READOUT);
@@ -1135,8 +1287,8 @@ struct Engine : EngineBase {
         // Without density normalisation nothing between reverse_M and the adjoint linear reads A_adj: the
         // linear then forms M_grad . M_adj itself while loading its rows (one polynomial per channel) and
         // A_adj is only written if somebody asks for it (get_array).
-        const bool fuse1 = !hm.A1_scaled && gemm_scaled_operand_ok(K(), K(), sizeof(F));
-        const bool fuse0 = !hm.A0_scaled && NLM() == 1 && gemm_scaled_operand_ok(K(), K(), sizeof(F));
+        const bool scaled_operand = use_linear(N) || gemm_scaled_operand_ok(K(), K(), sizeof(F));
+        const bool fuse1 = !hm.A1_scaled && scaled_operand, fuse0 = !hm.A0_scaled && NLM() == 1 && scaled_operand;
         stage_begin(ST_REVM1); if (!fuse1) st_reverse_M1(N1); stage_end(ST_REVM1);
         pending_A1_adj = fuse1 ? N1 : -1;
         st_scale(1, N1, true);
@@ -1280,6 +1432,7 @@ struct Engine : EngineBase {
         if (!out) return;
         // (arrays the evaluation left unwritten are formed when they are asked for; the others do not wait for that)
         if (s == "A1_adj" || s == "A0_adj" || s == "M0_grad") materialise_adjoints(s == "M0_grad");
+        if (s == "A0" || s == "A1") materialise_A();
         const double* src = nullptr;
         if (s == "Y" || s == "Y_grad") {
             scratch_d.size_to((size_t)E * 64, st);

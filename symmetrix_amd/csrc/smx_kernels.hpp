@@ -274,6 +274,28 @@ hipError_t launch_gemm(const GemmParams<TA, TC, CT>& p, hipStream_t s);
 bool gemm_scaled_operand_ok(int Kd, int Nn, size_t elem);
 
 // ---------------------------------------------------------------------------
+// Channel-mixing linears of the 16 (l, m) rows of an atom, with the contraction behind them (smx_kernels_linear.hip):
+//     out[node][lm (, e)][K] = sum over inner[l] of A[node][lm][.] W_l(, e)[.][K]   (times scale[node][.] on the operand)
+// Weights in operand order, [type][e][column tile of 16][inner / (4 V)][64 lanes][V], V = 16 bytes: lane 16 q + c holds
+// k = 4 V step + q V + (0 .. V - 1) of column c.  Contraction coefficients [type][column tile][monomials / V][16][V] of all NP
+// polynomials, lists padded as in smx_poly_shape.hpp.
+template <typename F>
+struct LinearParams {
+    int num_nodes, K, T;
+    const int* perm; const int* tstart;      // species groups, or null when nothing depends on the species
+    const F* A; long a_node_stride;
+    const F* scale;                          // [num_nodes][K] factor of the operand rows, or null
+    int inner[4], num_e[4], num_e_max;       // inner size and output blocks per l
+    int row_off[16];                         // of (l, m) in an operand row, elements
+    const F* W; size_t w_off[4], w_type_stride[4];
+    F* out; long out_node_stride; int out_off[16];
+    const F* coef; F* M; F* M_grad;
+};
+inline bool linear_ok(int K) { return K % 32 == 0; }     // whole pieces of a row, and column tiles in pairs
+// kind 0: M and M_grad of one polynomial, the linear's result is not stored; 1: out and M of NP polynomials; 2: out
+template <typename F> hipError_t launch_linear(const LinearParams<F>& p, int kind, int NP, hipStream_t s);
+
+// ---------------------------------------------------------------------------
 // Readout tail (MACE::compute_readouts, mace.cpp:876-903) in one launch: node_energies[i] (+)= E0[type] +
 // w1 . H1[i, l=0] + MLP_{K->16->1}(H2[i]) with W1[16][K], H2_adj = gradient of the network, H1_adj[rows][num_LM][K]
 // seeded with w1 in the scalar block of the first N rows and zero elsewhere.  guard / guard_clear / guard_forces: as

@@ -608,6 +608,10 @@ hipError_t launch_gemm(const GemmParams<TA, TC, CT>& p_in, hipStream_t s)
             if (best < 0 || padded < best) { best = padded; nt = c; }
         }
     }
+    // few rows: narrower tiles on more CUs (107 atoms, inner size 384, 128 columns, fp64: 29 blocks of the widest took 57 us)
+    long row_blocks = 0;
+    for (int z = 0; z < p.nprob; ++z) row_blocks += ((long)p.num_nodes * p.prob[z].sub + GM - 1) / GM;
+    while (nt > 1 && row_blocks * ((max_n + 16 * nt - 1) / (16 * nt)) < 192) nt = nt == 6 ? 2 : nt / 2;
     switch (nt) {
     case 1: return launch_gemm_t<TA, TC, CT, 1>(p, max_sub, max_n, s);
     case 2: return launch_gemm_t<TA, TC, CT, 2>(p, max_sub, max_n, s);
