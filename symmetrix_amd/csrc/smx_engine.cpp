@@ -450,7 +450,7 @@ struct Engine : EngineBase {
         if (M0_tables) slabs(M0_slabs, hm.P0.data(), hm.num_LM, false);
         if (M1_tables) slabs(M1_slabs, &hm.P1, 1, false);
         if (linear_ok(hm.K)) {
-            if (M0_tables) slabs(M0_coef16, hm.P0.data(), hm.num_LM, true);
+            if (M0_tables && hm.num_LM == 1) slabs(M0_coef16, hm.P0.data(), 1, true);
             if (M1_tables) slabs(M1_coef16, &hm.P1, 1, true);
             operand_weights(s);
         }
@@ -767,37 +767,34 @@ struct Engine : EngineBase {
         }
         return q;
     }
-    // Whether the A-basis linears of N nodes take k_linear: it streams its operands through blocks of 16 atoms, and with few
-    // atoms the latency of that stream is longer than the row-streaming kernel and a contraction launch take (107 atoms of the
-    // l <= 1 model in double precision: 61 + 64 us against 28 + 69; 501 of the scalar one in single: 21 against 22; 1 000 in double 38
-    // against 48).  The local nodes decide, so that a call with ghost nodes gives the bits of one without.
-    bool use_linear(int N) const { return linear_ok(K()) && (split_nodes > 0 ? split_nodes : N) >= 512; }
-    // The layer-0 adjoint linear writes over Phi0, unless the evaluation keeps Phi0 to form A0 from it on request: with one
-    // polynomial per channel and no density normalisation A0 only ever exists in the registers of the contraction.
+    // Whether the A-basis linears of N nodes take k_linear, and with the contraction behind them: it streams its operands
+    // through blocks of 16 atoms, and with few atoms the latency of that stream is longer than the row-streaming kernel (and a
+    // contraction launch) take.  Measured, us: linear and contraction 501 atoms 96 channels fp32 21 against 22, 1 000 fp64 32
+    // against 30, 2 000 34 against 40, 500 and 1 000 of the l <= 1 model fp64 65, 68 against 57, 88; adjoint linears alone 500
+    // fp32 17 against 16, fp64 24 against 33, l <= 1 24 and 31 against 32 and 57.  The local nodes decide, so that a call with ghost
+    // nodes gives the bits of one without.
+    int deciding_nodes(int N) const { return split_nodes > 0 ? split_nodes : N; }
+    bool use_linear(int N) const { return linear_ok(K()) && deciding_nodes(N) >= 512; }
     bool fused_contraction(int layer, int N) const
     {
-        return use_linear(N) && !(layer == 0 ? hm.A0_scaled : hm.A1_scaled) && (layer == 0 ? M0_tables : M1_tables);
+        return linear_ok(K()) && deciding_nodes(N) >= 1024 &&
+               (layer == 0 ? M0_tables && NLM() == 1 && !hm.A0_scaled : M1_tables && !hm.A1_scaled);
     }
-    bool separate_dPhi0(int N) const { return fused_contraction(0, N) && NLM() == 1; }
+    // The layer-0 adjoint linear writes over Phi0, unless the evaluation keeps Phi0 to form A0 from it on request.
+    bool separate_dPhi0(int N) const { return fused_contraction(0, N); }
     // A0 (or A1) and its contraction in one launch
     void st_linear_contraction(int layer, int N)
     {
         const size_t k = K();
-        if (layer == 0) {
-            A0.size_to((size_t)N * 16 * k, stream); M0.size_to((size_t)N * NLM() * k, stream);
-            auto q = linear_A0(N, false);
-            q.A = Phi0.p; q.M = M0.p; q.coef = M0_coef16.p;
-            const bool one = NLM() == 1;
-            if (one) { M0_grad.size_to((size_t)N * 16 * k, stream); q.M_grad = M0_grad.p; pending_A0 = N; }
-            else q.out = A0.p;
-            HIPCHK(launch_linear<F>(q, one ? 0 : 1, NLM(), stream));
-        } else {
-            A1.size_to((size_t)N * 16 * k, stream); M1.size_to((size_t)N * k, stream); M1_grad.size_to((size_t)N * 16 * k, stream);
-            auto q = linear_A1(N, false, true);
-            q.A = Phi1.p; q.M = M1.p; q.M_grad = M1_grad.p; q.coef = M1_coef16.p;
-            pending_A1 = N;
-            HIPCHK(launch_linear<F>(q, 0, 1, stream));
-        }
+        DVec<F>& M = layer == 0 ? M0 : M1;
+        DVec<F>& M_grad = layer == 0 ? M0_grad : M1_grad;
+        (layer == 0 ? A0 : A1).size_to((size_t)N * 16 * k, stream);
+        M.size_to((size_t)N * k, stream); M_grad.size_to((size_t)N * 16 * k, stream);
+        auto q = layer == 0 ? linear_A0(N, false) : linear_A1(N, false, true);
+        q.A = layer == 0 ? Phi0.p : Phi1.p; q.coef = layer == 0 ? M0_coef16.p : M1_coef16.p;
+        q.M = M.p; q.M_grad = M_grad.p;
+        HIPCHK(launch_linear<F>(q, stream));
+        (layer == 0 ? pending_A0 : pending_A1) = N;
     }
     // A0[i, l-block] = Phi0[i, l-block] . A0_weights[type_i][l]  (reverse: transposed weights)
     // `from_M0`: the adjoint product takes M0_grad . M0_adj (one polynomial per channel) as its operand
@@ -812,7 +809,7 @@ struct Engine : EngineBase {
         if (use_linear(N)) {
             auto q = linear_A0(N, reverse);
             q.A = src; q.out = dst; q.scale = from_M0 ? M0_adj.p : nullptr;
-            HIPCHK(launch_linear<F>(q, 2, 1, stream));
+            HIPCHK(launch_linear<F>(q, stream));
             return;
         }
         auto g = gemm_base<F, F, F>(N, true);
@@ -919,7 +916,7 @@ struct Engine : EngineBase {
             auto q = linear_A1(N, reverse, false);
             q.A = reverse ? (from_M1 ? M1_grad.p : A1_adj.p) : Phi1.p; q.out = reverse ? dPhi1.p : A1.p;
             q.scale = from_M1 ? M1_adj.p : nullptr;
-            HIPCHK(launch_linear<F>(q, 2, 1, stream));
+            HIPCHK(launch_linear<F>(q, stream));
             return;
         }
         long lme_off = 0;

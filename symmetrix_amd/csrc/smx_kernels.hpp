@@ -277,8 +277,8 @@ bool gemm_scaled_operand_ok(int Kd, int Nn, size_t elem);
 // Channel-mixing linears of the 16 (l, m) rows of an atom, with the contraction behind them (smx_kernels_linear.hip):
 //     out[node][lm (, e)][K] = sum over inner[l] of A[node][lm][.] W_l(, e)[.][K]   (times scale[node][.] on the operand)
 // Weights in operand order, [type][e][column tile of 16][inner / (4 V)][64 lanes][V], V = 16 bytes: lane 16 q + c holds
-// k = 4 V step + q V + (0 .. V - 1) of column c.  Contraction coefficients [type][column tile][monomials / V][16][V] of all NP
-// polynomials, lists padded as in smx_poly_shape.hpp.
+// k = 4 V step + q V + (0 .. V - 1) of column c.  With `coef` the polynomial of output slot 0 (one per channel) follows, and M and
+// M_grad are written instead of out: coefficients [type][column tile][monomials / V][16][V], padded as in smx_poly_shape.hpp.
 template <typename F>
 struct LinearParams {
     int num_nodes, K, T;
@@ -292,8 +292,7 @@ struct LinearParams {
     const F* coef; F* M; F* M_grad;
 };
 inline bool linear_ok(int K) { return K % 32 == 0; }     // whole pieces of a row, and column tiles in pairs
-// kind 0: M and M_grad of one polynomial, the linear's result is not stored; 1: out and M of NP polynomials; 2: out
-template <typename F> hipError_t launch_linear(const LinearParams<F>& p, int kind, int NP, hipStream_t s);
+template <typename F> hipError_t launch_linear(const LinearParams<F>& p, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Readout tail (MACE::compute_readouts, mace.cpp:876-903) in one launch: node_energies[i] (+)= E0[type] +

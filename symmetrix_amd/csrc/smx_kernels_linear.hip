@@ -47,9 +47,10 @@ __device__ __forceinline__ void load_into_lds(const void* from, unsigned to)
 template <int N>
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
-// KIND 0: linear and contraction with gradients (one polynomial); 1: linear, stored, and the values of NP polynomials;
-// 2: linear alone
-template <typename F, int WPB, int KIND, int NP, bool SCALED>
+// POLY: linear and contraction (one polynomial per channel, with gradients); else the linear alone.  (With several polynomials
+// per channel, values only, a launch of their own came out ahead: the 4 to 9 polynomials of the four atoms of a lane in turn are a
+// long chain for the few wavefronts here.)
+template <typename F, int WPB, bool POLY, bool SCALED>
 __global__ __launch_bounds__(64 * WPB, 2) void k_linear(const LinearParams<F> p)
 {
     using Op = MatOp<F>;
@@ -167,7 +168,7 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_linear(const LinearParams<F> p)
         node[r] = node_of(atom);
         live[r] = tile * 16 + atom < seg_n;
     }
-    if constexpr (KIND != 0) {
+    if constexpr (!POLY) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
             if (live[r]) {
@@ -178,59 +179,46 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_linear(const LinearParams<F> p)
                 });
             }
     }
-    if constexpr (KIND != 2) {
-        // coefficients of this block's channels: [column tile][16-byte group of monomials][16 channels], one polynomial at a time
-        static_for<0, NP>([&](auto pc) {
-            constexpr int P = decltype(pc)::value;
-            constexpr int G16 = poly_spec_padded(PolyTable<P>::N) / V, ALL16 = poly_spec_offset(NP) / V, FIRST16 = poly_spec_offset(P) / V;
-            __syncthreads();
-            {
-                const uint4* src = reinterpret_cast<const uint4*>(p.coef) + ((size_t)type * (p.K / 16) + ct) * ALL16 * 16 + FIRST16 * 16;
-                uint4* dst = reinterpret_cast<uint4*>(lin_lds) + (size_t)wave * G16 * 16;
-                for (int t = lane; t < G16 * 16; t += 64) dst[t] = src[t];
-            }
-            wave_lds_sync();      // a wavefront reads its own column tile only
-            const unsigned char* slab = lin_lds + (size_t)wave * G16 * 256 + r16 * 16;
-            for (int r = 0; r < 4; ++r) {
-                F x[16], gr[16], f = F(0);
+    if constexpr (POLY) {
+        // coefficients of this block's channels: [column tile][16-byte group of monomials][16 channels]
+        constexpr int G16 = poly_spec_padded(PolyTable<0>::N) / V;
+        __syncthreads();
+        {
+            const uint4* src = reinterpret_cast<const uint4*>(p.coef) + ((size_t)type * (p.K / 16) + ct) * G16 * 16;
+            uint4* dst = reinterpret_cast<uint4*>(lin_lds) + (size_t)wave * G16 * 16;
+            for (int t = lane; t < G16 * 16; t += 64) dst[t] = src[t];
+        }
+        wave_lds_sync();      // a wavefront reads its own column tile only
+        const unsigned char* slab = lin_lds + (size_t)wave * G16 * 256 + r16 * 16;
+        for (int r = 0; r < 4; ++r) {
+            F x[16], gr[16], f = F(0);
 #pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    x[q] = r == 0 ? acc[q][0] : (r == 1 ? acc[q][1] : (r == 2 ? acc[q][2] : acc[q][3]));
-                    gr[q] = F(0);
-                }
-                const int nd = r == 0 ? node[0] : (r == 1 ? node[1] : (r == 2 ? node[2] : node[3]));
-                const bool lv = r == 0 ? live[0] : (r == 1 ? live[1] : (r == 2 ? live[2] : live[3]));
-                poly_spec_body<F, P, KIND>(slab - (size_t)FIRST16 * 256, 256, x, gr, f, F(1));
-                if (lv) {
-                    p.M[((size_t)nd * NP + P) * p.K + col] = f;
-                    if constexpr (KIND == 0) {
-#pragma unroll
-                        for (int q = 0; q < 16; ++q) p.M_grad[((size_t)nd * 16 + q) * p.K + col] = gr[q];
-                    }
-                }
+            for (int q = 0; q < 16; ++q) {
+                x[q] = r == 0 ? acc[q][0] : (r == 1 ? acc[q][1] : (r == 2 ? acc[q][2] : acc[q][3]));
+                gr[q] = F(0);
             }
-        });
+            const int nd = r == 0 ? node[0] : (r == 1 ? node[1] : (r == 2 ? node[2] : node[3]));
+            const bool lv = r == 0 ? live[0] : (r == 1 ? live[1] : (r == 2 ? live[2] : live[3]));
+            poly_spec_body<F, 0, 0>(slab, 256, x, gr, f, F(1));
+            if (lv) {
+                p.M[(size_t)nd * p.K + col] = f;
+#pragma unroll
+                for (int q = 0; q < 16; ++q) p.M_grad[((size_t)nd * 16 + q) * p.K + col] = gr[q];
+            }
+        }
     }
 }
 
-template <typename F, int WPB, int KIND, int NP, bool SCALED>
+template <typename F, int WPB, bool POLY, bool SCALED>
 hipError_t launch_linear_t(const LinearParams<F>& p, hipStream_t s)
 {
     size_t lds = 3 * (size_t)256 * 64;
-    if constexpr (KIND != 2) {
-        int longest = 0;
-        for (int q = 0; q < NP; ++q) longest = std::max(longest, poly_spec_padded(kPolyTableLen[q]));
-        lds = std::max(lds, (size_t)WPB * longest * 16 * sizeof(F));
-    }
+    if (POLY) lds = std::max(lds, (size_t)WPB * poly_spec_padded(kPolyTableLen[0]) * 16 * sizeof(F));
     const long tiles = ((long)p.num_nodes + 15) / 16 + (p.perm ? p.T : 0);
     const long blocks = (tiles + 7) / 8 * 8 * (p.K / (16 * WPB)) * p.num_e_max;
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-    if (lds > 64 * 1024) {
-        hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(k_linear<F, WPB, KIND, NP, SCALED>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (err != hipSuccess) return err;
-    }
-    hipLaunchKernelGGL((k_linear<F, WPB, KIND, NP, SCALED>), dim3((unsigned)blocks), dim3(64 * WPB), lds, s, p);
+    if (lds > 64 * 1024) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_linear<F, WPB, POLY, SCALED>), dim3((unsigned)blocks), dim3(64 * WPB), lds, s, p);
     return hipGetLastError();
 }
 
@@ -238,35 +226,27 @@ hipError_t launch_linear_t(const LinearParams<F>& p, hipStream_t s)
 
 // Column tiles of a block: all that divide evenly, up to four (48 KB of LDS a block: three blocks on a CU).
 template <typename F>
-hipError_t launch_linear(const LinearParams<F>& p, int kind, int NP, hipStream_t s)
+hipError_t launch_linear(const LinearParams<F>& p, hipStream_t s)
 {
     if (p.num_nodes <= 0) return hipSuccess;
-    if (!linear_ok(p.K) || p.T <= 0) return hipErrorInvalidValue;
-    auto go = [&](auto kc, auto nc, auto sc) -> hipError_t {
-        constexpr int KIND = decltype(kc)::value, N = decltype(nc)::value;
-        constexpr bool S = decltype(sc)::value;
-        if (p.K % 64 == 0) return launch_linear_t<F, 4, KIND, N, S>(p, s);
-        if (p.K % 96 == 0) return launch_linear_t<F, 3, KIND, N, S>(p, s);
-        return launch_linear_t<F, 2, KIND, N, S>(p, s);
+    if (!linear_ok(p.K) || p.T <= 0 || (p.coef && (p.scale || p.num_e_max != 1))) return hipErrorInvalidValue;
+    auto go = [&](auto pc, auto sc) -> hipError_t {
+        constexpr bool POLY = decltype(pc)::value, SCALED = decltype(sc)::value;
+        if (p.K % 64 == 0) return launch_linear_t<F, 4, POLY, SCALED>(p, s);
+        if (p.K % 96 == 0) return launch_linear_t<F, 3, POLY, SCALED>(p, s);
+        return launch_linear_t<F, 2, POLY, SCALED>(p, s);
     };
-    constexpr std::integral_constant<int, 0> k0{};
-    constexpr std::integral_constant<int, 1> k1{};
-    constexpr std::integral_constant<int, 2> k2{};
-    if (kind == 2) return p.scale ? go(k2, k1, std::true_type{}) : go(k2, k1, std::false_type{});
-    if (p.scale) return hipErrorInvalidValue;
-    if (kind == 0 && NP == 1) return go(k0, k1, std::false_type{});
-    if (kind == 1 && NP == 4) return go(k1, std::integral_constant<int, 4>{}, std::false_type{});
-    if (kind == 1 && NP == 9) return go(k1, std::integral_constant<int, 9>{}, std::false_type{});
-    return hipErrorInvalidValue;
+    if (p.coef) return go(std::true_type{}, std::false_type{});
+    return p.scale ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
 }
 
 #ifndef SMX_LINEAR_PART
 #error "define SMX_LINEAR_PART (0: double, 1: float)"
 #endif
 #if SMX_LINEAR_PART == 0
-template hipError_t launch_linear<double>(const LinearParams<double>&, int, int, hipStream_t);
+template hipError_t launch_linear<double>(const LinearParams<double>&, hipStream_t);
 #else
-template hipError_t launch_linear<float>(const LinearParams<float>&, int, int, hipStream_t);
+template hipError_t launch_linear<float>(const LinearParams<float>&, hipStream_t);
 #endif
 
 }  // namespace smx
