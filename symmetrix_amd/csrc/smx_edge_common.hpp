@@ -140,6 +140,14 @@ __device__ __forceinline__ void ylm_tangential(const EdgeFrame& f, double& Y, do
     d2 = (g0 * f.t2z + g1 * f.t2x + g2 * f.t2y) * f.inv;
 }
 
+// Messages to the senders: 0.1 to 5 GB written once, and read once by the next launch.  As ordinary stores they drove the
+// spline tables and feature rows out of the L2s.
+template <typename T>
+__device__ __forceinline__ void store_stream(T* to, T v)
+{
+    __builtin_nontemporal_store(v, to);
+}
+
 // How many wavefronts share a receiver, of `units` receivers times channel groups.  A wavefront takes 0.5 to 2 us per edge,
 // and about 2 048 of them are in flight: fewer units leave SIMDs idle, up to three rounds of them leave the last round
 // nearly empty.  The adjoint gains up to three rounds (K = 128, l <= 1, single precision, 1 500 receivers: 214, 194, 157 us

@@ -630,7 +630,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                     for (int c = 0; c < CPL; ++c)
                         if (active[c]) {
 #pragma unroll
-                            for (int q = 0; q < NLM; ++q) *reinterpret_cast<F*>(mrow + q * (K * sizeof(F)) + k[c] * sizeof(F)) = V[c][q][0];
+                            for (int q = 0; q < NLM; ++q) store_stream(reinterpret_cast<F*>(mrow + q * (K * sizeof(F)) + k[c] * sizeof(F)), V[c][q][0]);
                         }
                 }
                 // sums over the channels of the wavefront, in the feature precision (a fixed tree)
@@ -751,6 +751,17 @@ __device__ __forceinline__ Vec<F, N> ldv(const F* p)
 {
     return *reinterpret_cast<const Vec<F, N>*>(p);
 }
+// of an array that is read once
+template <typename F, int N>
+__device__ __forceinline__ Vec<F, N> ldv_stream(const F* p)
+{
+    typedef F VV __attribute__((ext_vector_type(N)));
+    const VV t = __builtin_nontemporal_load(reinterpret_cast<const VV*>(p));
+    Vec<F, N> v;
+#pragma unroll
+    for (int c = 0; c < N; ++c) v.v[c] = t[c];
+    return v;
+}
 // V consecutive elements per thread (16-byte accesses when the row width allows); four messages are requested
 // before the first is added, the additions keep the ascending edge order
 // WINDOW: slist is in ascending order in memory and the messages of the edges [e_lo, e_hi) are taken; otherwise all
@@ -797,14 +808,14 @@ __global__ void k_sender_reduce(int rows, int width, const int* sstart, int* sli
         for (; t + 4 <= s1; t += 4) {
             Vec<F, V> m[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) m[i] = ldv<F, V>(msg + (size_t)(slist[t + i] - e_lo) * width + q);
+            for (int i = 0; i < 4; ++i) m[i] = ldv_stream<F, V>(msg + (size_t)(slist[t + i] - e_lo) * width + q);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int c = 0; c < V; ++c) acc.v[c] += m[i].v[c];
         }
         for (; t < s1; ++t) {
-            const Vec<F, V> m = ldv<F, V>(msg + (size_t)(slist[t] - e_lo) * width + q);
+            const Vec<F, V> m = ldv_stream<F, V>(msg + (size_t)(slist[t] - e_lo) * width + q);
 #pragma unroll
             for (int c = 0; c < V; ++c) acc.v[c] += m.v[c];
         }
@@ -878,14 +889,14 @@ __global__ __launch_bounds__(1024) void k_sender_reduce_linear(int rows, const i
                 for (; t + 4 <= s1; t += 4) {
                     Vec<F, V> m[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) m[i] = ldv<F, V>(msg + (size_t)slist[t + i] * K + q);
+                    for (int i = 0; i < 4; ++i) m[i] = ldv_stream<F, V>(msg + (size_t)slist[t + i] * K + q);
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
 #pragma unroll
                         for (int c = 0; c < V; ++c) acc.v[c] += m[i].v[c];
                 }
                 for (; t < s1; ++t) {
-                    const Vec<F, V> m = ldv<F, V>(msg + (size_t)slist[t] * K + q);
+                    const Vec<F, V> m = ldv_stream<F, V>(msg + (size_t)slist[t] * K + q);
 #pragma unroll
                     for (int c = 0; c < V; ++c) acc.v[c] += m.v[c];
                 }

@@ -436,7 +436,7 @@ __global__ __launch_bounds__(256, 2) void k_agg0_bwd(const AggParams<F> a, const
                     const unsigned off = (unsigned)le * sender_bytes;
 #pragma unroll
                     for (int c = 0; c < CPL; ++c)
-                        if (active[c]) *reinterpret_cast<F*>(mchunk + (off + k[c] * (unsigned)sizeof(F))) = V[c][0];
+                        if (active[c]) store_stream(reinterpret_cast<F*>(mchunk + (off + k[c] * (unsigned)sizeof(F))), V[c][0]);
                 }
             }
             const F s = edge_sum3<EW>(srad, g1, g2, lane);
