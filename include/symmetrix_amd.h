@@ -267,6 +267,10 @@ int smx_nlist_build_host(smx_nlist* nl, int num_atoms, const double* positions, 
  * (offsets[num_atoms][3], positions = folded + offsets * cell; *folded tells whether one of them is not zero). */
 int smx_nlist_build_box(smx_nlist* nl, int num_atoms, const double* positions, const int* types, const double* cell,
                         const int* pbc, double r_list, double r_cut, long long* offsets, int* folded, long* num_edges);
+/* wait = 0: builds from host positions may return as soon as the number of edges is known, with the arrays complete in the
+ * order of the null stream, which is where smx_evaluate_list takes them up (a caller that does nothing else with the list
+ * saves the time between the end of the search and the first launch after it). */
+int smx_nlist_set_wait(smx_nlist* nl, int wait);
 int smx_nlist_update_host(smx_nlist* nl, const double* positions, double r_cut, long* num_edges);
 int smx_nlist_inputs(smx_nlist* nl, const double** d_positions, const int** d_types);
 int smx_nlist_arrays(smx_nlist* nl, const int** num_neigh, const int** first_neigh, const int** neigh_indices,

@@ -52,6 +52,8 @@ class SymmetrixCalculator:
         self._species = np.full(max(self.evaluator.atomic_numbers) + 1, -1, dtype=np.int32)
         self._species[self.evaluator.atomic_numbers] = np.arange(len(self.evaluator.atomic_numbers))
         self._nlist = neighbors.DeviceNeighborList() if neighbor_list == "device" else None
+        if self._nlist is not None:
+            self._nlist.set_wait(False)     # the evaluation follows on the same stream
 
     def compute(self, positions, cell, atomic_numbers, pbc=(True, True, True)):
         Z = np.asarray(atomic_numbers).astype(np.int64).reshape(-1)

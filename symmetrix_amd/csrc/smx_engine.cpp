@@ -274,6 +274,8 @@ struct Engine : EngineBase {
     long geo_edges = 0;   // edges of the N_geo receivers
     DVec<int> first_neigh, scan_tmp, s_count, s_start, s_list, t_count, t_start, t_cursor, t_perm, flags;
     int sender_rows = 0;
+    long sender_edges = -1;        // edges that s_start / s_list cover
+    bool senders_differ = false;   // a caller's sender atoms were not the senders of the evaluation before
     // pair terms: ZBL constants per species pair, density-normalisation splines, divisors of the last forward pass
     DVec<double> zbl_a, zbl_rmax, zbl_zz, A0spl, A1spl, div0, div1;
     ZblParams zbl_params() const
@@ -614,7 +616,7 @@ struct Engine : EngineBase {
         HIPCHK(launch_sender_lists(neigh_indices, E1, rows, s_count.p, s_rank.p, s_start.p, s_list.p, scan_tmp.p,
                                    senders_counted, nullptr, s, input_guard(N_geo)));
         senders_counted = false;
-        sender_rows = rows;
+        sender_rows = rows; sender_edges = E1;
     }
     // stage-level calls: check whichever integer arrays this call brought
     void validate_stage_inputs(int N, bool have_nt, bool have_ni, bool have_nty, bool have_r)
@@ -1514,12 +1516,12 @@ struct Engine : EngineBase {
     // ------------------------------------------------------------------
     DVec<int> rf_send, rf_nodes, rf_count, rf_rank, rf_sstart, rf_slist;
     HostBuf<int> rf_nodes_host;
-    DVec<double> rf_out, rf_part;   // rf_out: [RF_HEAD: range flag, -, virial[6]][num_atoms][3]
+    DVec<double> rf_out, rf_part;   // rf_out: see fetch_reduction
     static constexpr size_t RF_HEAD = 8;
-    double* reduction_room(int num_atoms)
+    double* reduction_room(size_t values)
     {
         const double* before = rf_out.p;
-        rf_out.size_to(RF_HEAD + (size_t)3 * num_atoms, stream);
+        rf_out.size_to(RF_HEAD + values, stream);
         if (rf_out.p != before) HIPCHK(launch_fill<double>(rf_out.p, RF_HEAD, 0.0, stream));
         return rf_out.p;
     }
@@ -1560,16 +1562,30 @@ struct Engine : EngineBase {
         } else if (receiver_atom && geo_edges != E) {
             throw Error(SMX_EINVAL, "num_neigh of the last call does not cover every edge");
         }
-        double* out = reduction_room(atom_forces ? num_atoms : 0);
+        double* out = reduction_room(atom_forces ? (size_t)3 * num_atoms : 0);
+        // The senders of the evaluation's own lists, as a rule: those lists are used then, and compared with the caller's
+        // array on the way.  (Lists made anew from it: three launches, 30 us of a 230 us step at 501 atoms.)
+        const bool same_senders = atom_forces && !receiver_atom && !senders_differ && num_atoms == N_geo && sender_rows == num_atoms &&
+                                  sender_edges == E && geo_edges == E && E > 0;
+        auto device_senders = [&] {
+            if (sender_on_device) return sender_atom;
+            rf_send.size_to((size_t)E, s);
+            uploader.put(reinterpret_cast<char*>(rf_send.p), sender_atom, (size_t)E * sizeof(int), s);
+            uploader.next(s);
+            return (const int*)rf_send.p;
+        };
+        if (same_senders) {
+            g.senders = device_senders(); g.differ = reinterpret_cast<int*>(out + 1);
+            g.send_start = s_start.p; g.send_list = s_list.p;
+            g.atom_forces = out + RF_HEAD;
+            gather_forces(g, atoms, virial ? out + 2 : nullptr);
+            if (fetch_reduction(num_atoms, atom_forces, virial, nullptr)) return;
+            senders_differ = true;
+            g.senders = nullptr; g.differ = nullptr;
+        }
         int* flag = reinterpret_cast<int*>(out);
         if (atom_forces) {
-            const int* send = sender_atom;
-            if (!sender_on_device) {
-                rf_send.size_to((size_t)E, s);
-                uploader.put(reinterpret_cast<char*>(rf_send.p), sender_atom, (size_t)E * sizeof(int), s);
-                uploader.next(s);
-                send = rf_send.p;
-            }
+            const int* send = device_senders();
             clean_counters(rf_count, num_atoms, rf_clean);
             rf_rank.size_to((size_t)E, s);
             rf_sstart.size_to((size_t)num_atoms + 1, s); rf_slist.size_to((size_t)E, s);
@@ -1580,7 +1596,7 @@ struct Engine : EngineBase {
             g.atom_forces = out + RF_HEAD;
         }
         gather_forces(g, atoms, virial ? out + 2 : nullptr);
-        fetch_reduction(atom_forces, virial, num_atoms, 0, nullptr);
+        fetch_reduction(num_atoms, atom_forces, virial, nullptr);
     }
     void gather_forces(ForceGather& g, int atoms, double* d_virial)
     {
@@ -1592,40 +1608,35 @@ struct Engine : EngineBase {
         }
         HIPCHK(launch_force_gather(g, d_virial, stream));
     }
-    // the sums in one copy, and whatever `more` doubles follow them
-    void fetch_reduction(double* atom_forces, double* virial, int num_atoms, size_t more, double* more_out)
+    // The sums, [RF_HEAD: range flag, differ, virial[6]][num_atoms][3][energies], in one copy; false: the senders differed.
+    bool fetch_reduction(int num_atoms, double* atom_forces, double* virial, double* energies)
     {
-        const size_t nf = atom_forces ? (size_t)3 * num_atoms : 0, total = RF_HEAD + nf + more;
+        const size_t nf = atom_forces ? (size_t)3 * num_atoms : 0, total = RF_HEAD + nf + (energies ? num_atoms : 0);
         double* h = reinterpret_cast<double*>(host_out.room(total * sizeof(double)));
         HIPCHK(hipMemcpyAsync(h, rf_out.p, total * sizeof(double), hipMemcpyDeviceToHost, stream));
         HIPCHK(hipStreamSynchronize(stream));
-        if (*reinterpret_cast<const int*>(h)) {
-            HIPCHK(launch_fill<double>(rf_out.p, 1, 0.0, stream));
-            throw Error(SMX_EINVAL, "sender_atom out of range");
-        }
+        const bool differ = *reinterpret_cast<const int*>(h + 1) != 0, range = *reinterpret_cast<const int*>(h) != 0;
+        if (differ || range) HIPCHK(launch_fill<double>(rf_out.p, 2, 0.0, stream));
+        if (differ) return false;
+        if (range) throw Error(SMX_EINVAL, "sender_atom out of range");
         if (atom_forces) std::memcpy(atom_forces, h + RF_HEAD, nf * sizeof(double));
         if (virial) std::memcpy(virial, h + 2, 6 * sizeof(double));
-        if (more) std::memcpy(more_out, h + RF_HEAD + nf, more * sizeof(double));
+        if (energies) std::memcpy(energies, h + RF_HEAD + nf, (size_t)num_atoms * sizeof(double));
+        return true;
     }
     // Evaluation and reduction of one list on the device (receiver i and sender index are atoms) with the results in the
-    // caller's memory: the sender lists of the evaluation serve the reduction too, and everything comes back in one copy.
+    // caller's memory: the sender lists of the evaluation serve the reduction too, and everything comes back together.
     void evaluate_list(int N, const int* nt, const int* nn, const int* ni, const int* nty, const double* x, const double* rr,
                        long E_, double* energies, double* forces, double* virial) override
     {
-        double* out = nullptr;
-        {
-            const double* before = rf_out.p;
-            rf_out.size_to(RF_HEAD + (size_t)4 * N, stream);
-            out = rf_out.p;
-            if (out != before) HIPCHK(launch_fill<double>(out, RF_HEAD, 0.0, stream));
-        }
+        double* out = reduction_room((size_t)4 * N);
         compute(N, nt, nn, ni, nty, x, rr, E_, true, out + RF_HEAD + (size_t)3 * N, nullptr, -1, -1);
         ForceGather g{};
         g.num_nodes = N; g.first_neigh = first_neigh.p; g.forces = node_forces.p; g.xyz = xyz;
         g.send_start = s_start.p; g.send_list = s_list.p;
         g.atom_forces = out + RF_HEAD;
         gather_forces(g, N, out + 2);
-        fetch_reduction(forces, virial, N, (size_t)N, energies);
+        fetch_reduction(N, forces, virial, energies);
     }
 };
 
@@ -1708,6 +1719,10 @@ struct NeighborList {
     DVec<long long> keys, sorted;
     HostBuf<char> in_host;    // the same on its way there; every call waits for the stream before it returns
     HostBuf<int> totals;
+    DVec<unsigned long long> chain_sums;
+    HostBuf<unsigned long long> chain_total;
+    unsigned launches = 0;    // tag of the last chained launch
+    bool wait = true;         // false: a build from host positions returns when the number of edges is known (smx_nlist_set_wait)
     const double* shift_vec = nullptr;
     const int* shift_int = nullptr;
     double* pos_dev = nullptr;     // copies of host inputs (smx_nlist_build_host / smx_nlist_update_host)
@@ -1716,6 +1731,8 @@ struct NeighborList {
     int N = 0, num_shifts = 0;
     long E = 0, num_candidates = 0;
     double r_list = 0.0;
+
+    static constexpr size_t BRING_BYTES = (size_t)64 << 10;    // inputs brought by a kernel
 
     // Lists of up to this many atoms try every atom as a sender: the three launches that bin the atoms take longer.
     static constexpr int ALL_ATOMS = 512;
@@ -1750,7 +1767,8 @@ struct NeighborList {
             std::memcpy(h + bv + bi, h_pos, (size_t)24 * N);
             std::memcpy(h + bv + bi + bp, h_types, (size_t)4 * N);
         }
-        HIPCHK(hipMemcpyAsync(in_dev.p, h, total, hipMemcpyHostToDevice, s));
+        if (total <= BRING_BYTES) HIPCHK(launch_bring(in_dev.p, h, total, s));
+        else HIPCHK(hipMemcpyAsync(in_dev.p, h, total, hipMemcpyHostToDevice, s));
         shift_vec = reinterpret_cast<const double*>(in_dev.p);
         shift_int = reinterpret_cast<const int*>(in_dev.p + bv);
         pos_dev = h_pos ? reinterpret_cast<double*>(in_dev.p + bv + bi) : nullptr;
@@ -1780,6 +1798,40 @@ struct NeighborList {
         }
         for (int k = 0; k < 3; ++k)
             if (!(lo[k] <= hi[k]) || !(hi[k] - lo[k] < 1e300)) throw Error(SMX_EINVAL, "neighbour list: positions are not finite");
+    }
+
+    NlChain next_chain(hipStream_t s)
+    {
+        if (chain_sums.cap == 0) {
+            chain_sums.size_to((size_t)nl_blocks(NL_CHAIN_ATOMS), s);
+            HIPCHK(hipMemsetAsync(chain_sums.p, 0, chain_sums.n * sizeof(unsigned long long), s));
+        }
+        unsigned long long* total = chain_total.room(1);
+        if (++launches == 0) {      // (the tags begin again)
+            HIPCHK(hipMemsetAsync(chain_sums.p, 0, chain_sums.n * sizeof(unsigned long long), s));
+            launches = 1;
+        }
+        NlChain c;
+        c.sums = chain_sums.p; c.tag = (unsigned long long)launches << 32; c.host_total = total;
+        *total = 0;
+        return c;
+    }
+    // The total of a chained launch: after the stream has finished, or (early) as soon as the launch has written it, which is
+    // before its entries are complete.
+    long chained_total(const NlChain& c, bool early, hipStream_t s)
+    {
+        const volatile unsigned long long* word = c.host_total;
+        if (!early) HIPCHK(hipStreamSynchronize(s));
+        for (unsigned n = 1; *word >> 32 != c.tag >> 32; ++n) {
+            if (n % 4096) { __builtin_ia32_pause(); continue; }
+            const hipError_t state = hipStreamQuery(s);
+            if (state == hipErrorNotReady) continue;
+            HIPCHK(state);
+            if (*word >> 32 != c.tag >> 32) throw Error(SMX_EHIP, "neighbour list: the launch left no total");
+        }
+        const unsigned long long total = *word & 0xffffffffull;
+        if (total > 0x7fffffffull) throw Error(SMX_EINVAL, "neighbour list: more than 2^31 candidate pairs");
+        return (long)total;
     }
 
     // Candidates: every (receiver, sender, image) closer than r_list, ordered per receiver.  Edges: those closer than r_cut.
@@ -1827,48 +1879,69 @@ struct NeighborList {
         }
         const int* bs = all ? nullptr : bin_start.p;
         const int* ba = all ? nullptr : bin_atoms.p;
-        count.size_to((size_t)N, s);
-        HIPCHK(launch_nl_search(false, d_pos, N, g, bs, ba, num_shifts, shift_vec, zero_shift, r_list, count.p, nullptr, 0,
-                                nullptr, nullptr, nullptr, s));
-        HIPCHK(launch_scan_exclusive(count.p, cfirst.p, N, scan_tmp.p, s));
         const bool direct = r_list == r_cut;   // no skin: the candidates are the edges
+        const bool chained = N <= NL_CHAIN_ATOMS;
         if (sorted.cap == 0) { keys.size_to((size_t)64 * N, s); sorted.size_to((size_t)64 * N, s); }
         if (edge_capacity() == 0) edge_room((size_t)64 * N, s);
+        if (!chained) {
+            count.size_to((size_t)N, s);
+            HIPCHK(launch_nl_search(false, d_pos, N, g, bs, ba, num_shifts, shift_vec, zero_shift, r_list, count.p, nullptr, 0,
+                                    nullptr, nullptr, nullptr, nullptr, s));
+            HIPCHK(launch_scan_exclusive(count.p, cfirst.p, N, scan_tmp.p, s));
+        }
         for (;;) {
             const long room = (long)std::min(keys.cap, sorted.cap);
             const NlEdgeArrays edges = edge_arrays(d_types);
+            NlChain chain{};
+            if (chained) chain = next_chain(s);
             HIPCHK(launch_nl_search(true, d_pos, N, g, bs, ba, num_shifts, shift_vec, zero_shift, r_list, nullptr, cfirst.p,
-                                    direct ? std::min(room, edge_capacity()) : room, keys.p, sorted.p, direct ? &edges : nullptr, s));
-            HIPCHK(hipMemcpyAsync(totals.p, cfirst.p + N, sizeof(int), hipMemcpyDeviceToHost, s));
-            if (!direct) E = filter(d_pos, d_types, r_cut, room, s);   // waits for the stream
-            else HIPCHK(hipStreamSynchronize(s));
-            const long total = totals.p[0];
-            if (total < 0) throw Error(SMX_EINVAL, "neighbour list: more than 2^31 candidate pairs");
+                                    direct ? std::min(room, edge_capacity()) : room, keys.p, sorted.p, direct ? &edges : nullptr,
+                                    chained ? &chain : nullptr, s));
+            long total;
+            if (chained) {
+                total = chained_total(chain, !direct || (h_pos && !wait), s);
+            } else {
+                HIPCHK(hipMemcpyAsync(totals.p, cfirst.p + N, sizeof(int), hipMemcpyDeviceToHost, s));
+                HIPCHK(hipStreamSynchronize(s));
+                total = totals.p[0];
+                if (total < 0) throw Error(SMX_EINVAL, "neighbour list: more than 2^31 candidate pairs");
+            }
             num_candidates = total;
-            if (direct) E = total;
             if (total <= room && (!direct || total <= edge_capacity())) break;
             keys.size_to((size_t)total, s); sorted.size_to((size_t)total, s);
             if (direct) edge_room((size_t)total, s);
         }
+        E = direct ? num_candidates : filter(d_pos, d_types, r_cut, num_candidates, s);
         edge_room((size_t)E, s);
         return E;
     }
 
-    // edges: the candidates closer than r_cut at the given positions, in candidate order (`room`: what the candidate arrays
-    // hold; a list that does not fit has not been written and is not read)
+    // edges: the candidates closer than r_cut at the given positions, in candidate order (`room`: what the candidate arrays hold)
     long filter(const double* d_pos, const int* d_types, double r_cut, long room, hipStream_t s)
     {
-        totals.room(2);
         if (edge_capacity() == 0) edge_room((size_t)64 * N, s);
-        HIPCHK(launch_nl_filter(false, d_pos, N, cfirst.p, sorted.p, room, num_shifts, shift_vec, r_cut, num_neigh.p, nullptr, 0, nullptr, s));
-        HIPCHK(launch_scan_exclusive(num_neigh.p, first.p, N, scan_tmp.p, s));
+        const bool chained = N <= NL_CHAIN_ATOMS;
+        if (!chained) {
+            totals.room(2);
+            HIPCHK(launch_nl_filter(false, d_pos, N, cfirst.p, sorted.p, room, num_shifts, shift_vec, r_cut, num_neigh.p, nullptr, 0,
+                                    nullptr, nullptr, s));
+            HIPCHK(launch_scan_exclusive(num_neigh.p, first.p, N, scan_tmp.p, s));
+        }
         for (;;) {
             const long cap = edge_capacity();
             const NlEdgeArrays edges = edge_arrays(d_types);
-            HIPCHK(launch_nl_filter(true, d_pos, N, cfirst.p, sorted.p, room, num_shifts, shift_vec, r_cut, nullptr, first.p, cap, &edges, s));
-            HIPCHK(hipMemcpyAsync(totals.p + 1, first.p + N, sizeof(int), hipMemcpyDeviceToHost, s));
-            HIPCHK(hipStreamSynchronize(s));
-            const long total = totals.p[1];
+            NlChain chain{};
+            if (chained) chain = next_chain(s);
+            HIPCHK(launch_nl_filter(true, d_pos, N, cfirst.p, sorted.p, room, num_shifts, shift_vec, r_cut, num_neigh.p, first.p, cap,
+                                    &edges, chained ? &chain : nullptr, s));
+            long total;
+            if (chained) {
+                total = chained_total(chain, false, s);
+            } else {
+                HIPCHK(hipMemcpyAsync(totals.p + 1, first.p + N, sizeof(int), hipMemcpyDeviceToHost, s));
+                HIPCHK(hipStreamSynchronize(s));
+                total = totals.p[1];
+            }
             if (total <= cap) return total;
             edge_room((size_t)total, s);
         }
@@ -2280,6 +2353,13 @@ smx_nlist* smx_nlist_create(void)
     smx_nlist* out = nullptr;
     guarded([&] { out = reinterpret_cast<smx_nlist*>(new smx::NeighborList()); });
     return out;
+}
+int smx_nlist_set_wait(smx_nlist* nl, int wait)
+{
+    return guarded([&] {
+        if (!nl) throw smx::Error(SMX_EINVAL, "null argument");
+        reinterpret_cast<smx::NeighborList*>(nl)->wait = wait != 0;
+    });
 }
 void smx_nlist_free(smx_nlist* nl) { delete reinterpret_cast<smx::NeighborList*>(nl); }
 int smx_nlist_build(smx_nlist* nl, int num_atoms, const double* d_positions, const int* d_types, int num_shifts,

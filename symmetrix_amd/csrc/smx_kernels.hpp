@@ -94,6 +94,9 @@ struct NlGrid {
     double inv_bs[3];        // 1 / bin size
     int nb[3];               // bins per axis
 };
+// n bytes (a multiple of 16) of pinned host memory into device memory by a kernel: a few KB before a launch that needs them
+// arrive sooner than by a copy command, whose completion the launch waits for (24 atoms: 14 us).
+hipError_t launch_bring(void* to, const void* from_host, size_t n, hipStream_t s);
 hipError_t launch_nl_bbox(const double* pos, int N, double* part, int nblocks, hipStream_t s);
 hipError_t launch_nl_bins(const double* pos, int N, const NlGrid& g, int* atom_bin, int* bin_count, hipStream_t s);
 hipError_t launch_nl_bin_fill(int N, const int* atom_bin, const int* bin_start, int* bin_cursor, int* bin_atoms,
@@ -110,16 +113,28 @@ struct NlEdgeArrays {
     double* xyz;
     double* r;
 };
-// bin_start == nullptr: every atom is tried, no bins.  fill: the ordered keys go to `sorted` (keys: scratch of the same
-// size), and with `edges` every candidate is written as an edge.  Nothing is written where first[N] > capacity.
+// Offsets found inside the launch that uses them (chained_offset): one slot per block, a tag in the upper 32 bits that no
+// earlier launch on these slots had, and a word in host memory for tag | total (0xffffffff: too many).
+struct NlChain {
+    unsigned long long* sums;
+    unsigned long long tag;
+    unsigned long long* host_total;
+};
+// Up to this many atoms: a block reads the slots of all blocks before it (2 048 at most).  Beyond, launches for counting and
+// for the prefix sum are a small part of the whole.
+constexpr int NL_CHAIN_ATOMS = 8192;
+inline int nl_blocks(int N) { return (N + 3) / 4; }
+// bin_start == nullptr: every atom is tried, no bins (with a chain only).  fill: the ordered keys go to `sorted` (keys: scratch
+// of the same size), and with `edges` every candidate is written as an edge; offsets are read from `first`, or with a chain
+// found and written there.  Nothing is written past `capacity`.
 hipError_t launch_nl_search(bool fill, const double* pos, int N, const NlGrid& g, const int* bin_start,
                             const int* bin_atoms, int num_shifts, const double* shift_vec, int zero_shift,
-                            double r_cut, int* count, const int* first, long capacity, long long* keys, long long* sorted,
-                            const NlEdgeArrays* edges, hipStream_t s);
-// `room`: keys that `sorted` holds; with more candidates than that there are none in it, and no edges
-hipError_t launch_nl_filter(bool emit, const double* pos, int N, const int* cfirst, const long long* sorted, long room, int num_shifts,
-                            const double* shift_vec, double r_cut, int* count, const int* first, long capacity,
-                            const NlEdgeArrays* edges, hipStream_t s);
+                            double r_cut, int* count, int* first, long capacity, long long* keys, long long* sorted,
+                            const NlEdgeArrays* edges, const NlChain* chain, hipStream_t s);
+// `room`: keys that `sorted` holds; with more candidates than that there are no edges.  fill with a chain counts as well.
+hipError_t launch_nl_filter(bool fill, const double* pos, int N, const int* cfirst, const long long* sorted, long room, int num_shifts,
+                            const double* shift_vec, double r_cut, int* count, int* first, long capacity,
+                            const NlEdgeArrays* edges, const NlChain* chain, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Pair terms of the edge length alone (smx_kernels_pair.hip)
@@ -348,6 +363,8 @@ struct ForceGather {
     double* atom_forces;                             // [num_atoms][3] or null
     double* partial;                                 // [force_gather_blocks][6], needed for the virial, else null
     const int* flag;                                 // raised: the outputs are NaN (or null)
+    const int* senders;                              // sender atom of every edge, where send_list is another array's: compared,
+    int* differ;                                     // ... and set to 1 where they are not the same (null: not compared)
 };
 int force_gather_blocks(int num_atoms);
 hipError_t launch_force_gather(const ForceGather& g, double* virial, hipStream_t s);

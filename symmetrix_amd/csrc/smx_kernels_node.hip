@@ -972,7 +972,9 @@ __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
             const int s0 = a.send_start[at], n = a.send_start[at + 1] - s0;
             const int* sorted = wave_sorted_bucket<GATHER_CAP>(a.send_list, s0, n, bucket[wave], lane);
             for (int t = lane; t < n; t += 64) {
-                const double* f = a.forces + 3 * (size_t)sorted[t];
+                const int e = sorted[t];
+                if (a.senders && a.senders[e] != at) *a.differ = 1;
+                const double* f = a.forces + 3 * (size_t)e;
                 fx += f[0]; fy += f[1]; fz += f[2];
             }
         }

@@ -294,7 +294,7 @@ class DeviceNeighborList:
             raise RuntimeError("smx_nlist_create failed: " + self._L.smx_last_error().decode())
         self.num_atoms = 0
         self.num_edges = 0
-        self.ptr = {}
+        self._ptr = {}
         self._wrap = None      # lattice offsets taken off the positions of the last build_host
         self._cell = None
 
@@ -313,12 +313,23 @@ class DeviceNeighborList:
     _names = ("num_neigh", "first_neigh", "neigh_indices", "neigh_types", "neigh_shift", "xyz", "r", "positions", "node_types")
 
     def _refresh(self, E):
-        h, refs = self._C.c_void_p(self._h), self._out_refs
         self.num_edges = int(E)
-        self._lib.check(self._L.smx_nlist_arrays(h, *refs[:7]))
-        self._lib.check(self._L.smx_nlist_inputs(h, *refs[7:]))
-        self.ptr = {n: (p or 0) for n, p in zip(self._names, self._out)}
+        self._ptr = None
         return self.num_edges
+
+    @property
+    def ptr(self):
+        """Addresses of the edge arrays (and of the device copies of host inputs), by name."""
+        if self._ptr is None:
+            h, refs = self._C.c_void_p(self._h), self._out_refs
+            self._lib.check(self._L.smx_nlist_arrays(h, *refs[:7]))
+            self._lib.check(self._L.smx_nlist_inputs(h, *refs[7:]))
+            self._ptr = {n: (p or 0) for n, p in zip(self._names, self._out)}
+        return self._ptr
+
+    def set_wait(self, wait):
+        """False: build_host may return before the arrays are complete; work on the null stream finds them complete."""
+        self._lib.check(self._L.smx_nlist_set_wait(self._C.c_void_p(self._h), int(bool(wait))))
 
     def build(self, num_atoms, positions_ptr, types_ptr, cell, r_cut, pbc=(True, True, True), skin=0.0, stream=0):
         """New search: pairs within r_cut + skin are remembered, edges are the pairs within r_cut.

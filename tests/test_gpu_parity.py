@@ -498,6 +498,37 @@ def test_device_neighbor_list_update_equals_fresh_build():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("atoms,volume", [(1, 1.0), (3, 10.0), (4, 10.0), (5, 10.0), (40, 10.0), (512, 12.0), (513, 12.0),
+                                          (4097, 12.0), (8192, 14.0), (8193, 14.0)])
+def test_list_sizes_at_which_the_search_changes(atoms, volume):
+    """Bins or all atoms, offsets found inside the launch or by a prefix sum, more edges than there is room for at first and
+    more keys per receiver than fit the LDS (40 atoms in a wide cutoff): host builder's list, with and without a skin."""
+    from symmetrix_amd import neighbors
+    rng = np.random.default_rng(atoms)
+    cell = np.full(3, (atoms * volume) ** (1.0 / 3.0))
+    pos = rng.uniform(0, 1, size=(atoms, 3)) * cell
+    types = rng.integers(0, 3, size=atoms).astype(np.int32)
+    rc = 9.9 if atoms == 40 else 3.3
+    nl = neighbors.DeviceNeighborList()
+    for wait, skin in ((True, 0.0), (True, 0.7), (False, 0.0), (False, 0.7)):
+        nl.set_wait(wait)
+        print(f"atoms {atoms} wait {wait} skin {skin}", flush=True)
+        E = nl.build_host(pos, types, cell, rc, skin=skin)
+        ref = neighbors.neighbor_list(pos, cell, rc)
+        got = nl.to_host()
+        assert E == len(ref["r"])
+        for k in ("i", "j", "S", "xyz", "r", "first_neigh"):
+            assert np.array_equal(got[k], ref[k].reshape(got[k].shape)), k
+        if skin:
+            moved = pos + rng.uniform(-0.15, 0.15, size=pos.shape)
+            E = nl.update_host(moved, rc)
+            got, ref = nl.to_host(), neighbors.neighbor_list(moved, cell, rc, offsets=np.zeros((atoms, 3), dtype=int))
+            assert E == len(ref["r"])
+            for k in ("i", "j", "S", "xyz", "r", "first_neigh"):
+                assert np.array_equal(got[k], ref[k].reshape(got[k].shape)), k
+
+
+@pytest.mark.gpu
 def test_device_resident_loop_positions_to_forces(gpu, tmp_models):
     """positions on the device -> device neighbour list -> compute_device -> per-atom forces, against the host path."""
     import torch
