@@ -29,6 +29,7 @@ from __future__ import annotations
 import argparse
 import json
 import os
+import re
 import sys
 import tempfile
 import time
@@ -73,10 +74,10 @@ def measured_traffic(workload, dtype, stage, kernel):
 
 MFMA_PEAK = {"float64": 78.6e12, "float32": 157.3e12}   # dense matrix-core peaks of MI355X, flop/s
 # kernel behind each dense stage (as the kernel trace names it) when it runs in feature precision F
-DENSE_KERNEL = {"A0_lin": "k_gemm_rows<{F}, {F}, {F}, 3, false", "A1": "k_gemm_rows<{F}, {F}, {F}, 3, false",
-                "H1": "k_gemm_rows<{F}, {F}, {F}, 1, false", "H2": "k_tail_fused<{F}",
-                "rev_A1": "k_gemm_rows<{F}, {F}, {F}, 3, true", "rev_A0_lin": "k_gemm_rows<{F}, {F}, {F}, 3, true",
-                "rev_H1": "k_gemm_rows<{F}, {F}, {F}, 1, false"}
+DENSE_KERNEL = {"A0_lin": r"k_linear<{F}, \d, {one}, false>", "A1": r"k_linear<{F}, \d, true, false>",
+                "H1": r"k_gemm_rows<{F}, {F}, {F}, \d, false", "H2": r"k_tail_fused<{F}",
+                "rev_A1": r"k_linear<{F}, \d, false, true>", "rev_A0_lin": r"k_linear<{F}, \d, false, {one}>",
+                "rev_H1": r"k_gemm_rows<{F}, {F}, {F}, \d, false"}   # {one}: one polynomial per channel in layer 0
 
 
 def dense_flops(stage, N, K, n_LM, n_e):
@@ -129,15 +130,15 @@ def edge_valu_flops(stage, E, K, L_max):
     return per_edge.get(stage, 0) * E
 
 
-def measured_mfma_busy(workload, dtype, stage):
+def measured_mfma_busy(workload, dtype, stage, L_max):
     """Matrix-pipe busy share of the kernel behind a dense stage (SQ_VALU_MFMA_BUSY_CYCLES over SIMD cycles), from
     the rocprofv3 counter summary kept under profiles/; None when the file has no line for that kernel."""
     path = os.path.join(HERE, "profiles", f"bench_{workload}_shader_counters.txt")
     if not os.path.exists(path) or stage not in DENSE_KERNEL:
         return None
-    name = DENSE_KERNEL[stage].format(F="double" if dtype == "float64" else "float")
+    name = re.compile(DENSE_KERNEL[stage].format(F="double" if dtype == "float64" else "float", one="true" if L_max == 0 else "false"))
     for line in open(path):
-        if line.startswith(name) and line.rstrip().endswith("%"):
+        if name.match(line) and line.rstrip().endswith("%"):
             try:
                 return float(line.split()[-1].rstrip("%")) / 100.0
             except ValueError:
@@ -501,7 +502,7 @@ def main():
                 continue
             mfma[k] = {"flops": fl, "kernel_ms": ms_k, "achieved_tflops": fl / (ms_k * 1e-3) / 1e12, "peak_tflops": peak / 1e12,
                        "frac": fl / (ms_k * 1e-3) / peak,
-                       "mfma_busy_profiled": measured_mfma_busy(workload, dtype, k) if profiled and not pair_tables else None}
+                       "mfma_busy_profiled": measured_mfma_busy(workload, dtype, k, L_max) if profiled and not pair_tables else None}
         # the symmetric contractions: vector arithmetic against the vector peak, and their HBM side
         contraction = {}
         # (layer 0 with several polynomials per channel and the standard basis keeps no gradients: values in M0,
@@ -513,6 +514,9 @@ def main():
             if ms_k <= 0.0 or (k == "rev_M0" and not split0):
                 continue
             fl, by = contraction_work(n_k, K, L_max, layer, s_bytes, mode)
+            if ms_k < 0.006:
+                contraction[k] = {"flops": fl, "note": "evaluated in the launch of the layer's A-basis linear"}
+                continue
             vpeak = VALU_PEAK
             contraction[k] = {"kernel": "k_poly_spec" if res["contraction_tables"] & (1 << layer) else "k_poly", "mode": mode,
                               "flops": fl, "kernel_ms": ms_k, "achieved_tflops": fl / (ms_k * 1e-3) / 1e12,
