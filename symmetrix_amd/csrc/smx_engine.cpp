@@ -1532,8 +1532,9 @@ struct Engine : EngineBase {
         need(node_forces.p, "node_forces");
         if (node_forces.n != (size_t)3 * E) throw Error(SMX_EINVAL, "node_forces does not match the current edge list");
         if (!atom_forces && !virial) return;
+        if (virial && E > 0) need(xyz, "xyz");
         ForceGather g{};
-        g.num_nodes = N_geo; g.first_neigh = first_neigh.p; g.forces = node_forces.p; g.xyz = xyz;
+        g.num_nodes = N_geo; g.first_neigh = first_neigh.p; g.num_edges = E; g.forces = node_forces.p; g.xyz = xyz;
         int atoms = N_geo;
         if (atom_forces) {
             atoms = num_atoms;
@@ -1602,9 +1603,8 @@ struct Engine : EngineBase {
     {
         g.num_atoms = atoms;
         if (d_virial) {
-            rf_part.size_to((size_t)6 * std::max(1, force_gather_blocks(atoms)), stream);
+            rf_part.size_to((size_t)6 * force_gather_blocks(atoms), stream);
             g.partial = rf_part.p;
-            if (atoms == 0) HIPCHK(launch_fill<double>(d_virial, 6, 0.0, stream));
         }
         HIPCHK(launch_force_gather(g, d_virial, stream));
     }
@@ -1632,7 +1632,7 @@ struct Engine : EngineBase {
         double* out = reduction_room((size_t)4 * N);
         compute(N, nt, nn, ni, nty, x, rr, E_, true, out + RF_HEAD + (size_t)3 * N, nullptr, -1, -1);
         ForceGather g{};
-        g.num_nodes = N; g.first_neigh = first_neigh.p; g.forces = node_forces.p; g.xyz = xyz;
+        g.num_nodes = N; g.first_neigh = first_neigh.p; g.num_edges = E; g.forces = node_forces.p; g.xyz = xyz;
         g.send_start = s_start.p; g.send_list = s_list.p;
         g.atom_forces = out + RF_HEAD;
         gather_forces(g, N, out + 2);

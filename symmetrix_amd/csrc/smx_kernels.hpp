@@ -358,15 +358,16 @@ struct ForceGather {
     const int* send_start; int* send_list;           // edges by sender atom (null: no sender side)
     const int* node_start; const int* node_list;     // nodes whose edges count as received by the atom; null: node i is atom i
     int num_nodes;
-    const int* first_neigh;                          // [num_nodes + 1]
-    const double* forces; const double* xyz;         // [E][3]
+    const int* first_neigh;                          // [num_nodes + 1], or null without nodes
+    long num_edges;                                  // those beyond the nodes' have no receiver here: sender side and virial only
+    const double* forces; const double* xyz;         // [E][3] (xyz for the virial only)
     double* atom_forces;                             // [num_atoms][3] or null
     double* partial;                                 // [force_gather_blocks][6], needed for the virial, else null
     const int* flag;                                 // raised: the outputs are NaN (or null)
     const int* senders;                              // sender atom of every edge, where send_list is another array's: compared,
     int* differ;                                     // ... and set to 1 where they are not the same (null: not compared)
 };
-int force_gather_blocks(int num_atoms);
+int force_gather_blocks(int num_atoms);             // at least one: edges may be there without an atom
 hipError_t launch_force_gather(const ForceGather& g, double* virial, hipStream_t s);
 
 }  // namespace smx

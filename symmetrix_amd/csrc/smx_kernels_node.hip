@@ -960,6 +960,12 @@ template hipError_t launch_readout_fused<float>(int, int, int, int, const int*, 
 // gather of 24-byte forces at large ones.
 namespace {
 constexpr int GATHER_CAP = 512;
+__device__ __forceinline__ void add_virial(double (&v)[6], const double* d, const double* f)
+{
+    const double x = d[0], y = d[1], z = d[2];
+    v[0] += x * f[0]; v[1] += y * f[1]; v[2] += z * f[2];
+    v[3] += 0.5 * (x * f[1] + y * f[0]); v[4] += 0.5 * (x * f[2] + z * f[0]); v[5] += 0.5 * (y * f[2] + z * f[1]);
+}
 __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
 {
     __shared__ __align__(16) int bucket[4][GATHER_CAP];
@@ -985,11 +991,8 @@ __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
             const int node = a.node_list ? a.node_list[q] : q;
             for (int e = a.first_neigh[node] + lane; e < a.first_neigh[node + 1]; e += 64) {
                 const double* f = a.forces + 3 * (size_t)e;
-                const double* d = a.xyz + 3 * (size_t)e;
-                const double x = d[0], y = d[1], z = d[2];
                 fx -= f[0]; fy -= f[1]; fz -= f[2];
-                v[0] += x * f[0]; v[1] += y * f[1]; v[2] += z * f[2];
-                v[3] += 0.5 * (x * f[1] + y * f[0]); v[4] += 0.5 * (x * f[2] + z * f[0]); v[5] += 0.5 * (y * f[2] + z * f[1]);
+                if (a.partial) add_virial(v, a.xyz + 3 * (size_t)e, f);
             }
         }
         if (a.atom_forces) {
@@ -1000,6 +1003,11 @@ __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
         wave_lds_sync();   // the next atom's bucket overwrites this one's
     }
     if (!a.partial) return;
+    // Edges behind those of the nodes (the last counts covered the leading nodes of a longer edge list): every edge is in the
+    // virial.  After an evaluation that its input checks skipped these are all edges, and their forces are NaN.
+    for (long e = (a.first_neigh ? a.first_neigh[a.num_nodes] : 0) + (long)blockIdx.x * 256 + threadIdx.x; e < a.num_edges;
+         e += (long)gridDim.x * 256)
+        add_virial(v, a.xyz + 3 * (size_t)e, a.forces + 3 * (size_t)e);
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
         const double t = wave_sum(v[q]);
@@ -1021,11 +1029,10 @@ __global__ __launch_bounds__(384) void k_virial_finish(const double* partial, in
 }
 }  // namespace
 
-int force_gather_blocks(int num_atoms) { return std::min((num_atoms + 3) / 4, 2048); }
+int force_gather_blocks(int num_atoms) { return std::min(std::max((num_atoms + 3) / 4, 1), 2048); }
 hipError_t launch_force_gather(const ForceGather& g, double* virial, hipStream_t s)
 {
     const int nb = force_gather_blocks(g.num_atoms);
-    if (nb <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_force_gather, dim3(nb), dim3(256), 0, s, g);
     if (virial) hipLaunchKernelGGL(k_virial_finish, dim3(1), dim3(384), 0, s, g.partial, nb, g.flag, virial);
     return hipGetLastError();

@@ -84,6 +84,10 @@ extern "C" int smx_reduce_forces_device_noalloc(smx_model* m, int num_atoms, con
         smx::set_last_error("node_forces does not match the current edge list");
         return SMX_EINVAL;
     }
+    if (d_virial && v.num_edges > 0 && !v.xyz) {
+        smx::set_last_error("the virial needs the edge vectors (compute_Y)");
+        return SMX_EINVAL;
+    }
     rc = smx::noalloc_setup_current_device(&err);
     if (rc != SMX_OK) { smx::set_last_error(err); return rc; }
     int dev = 0;
@@ -107,7 +111,7 @@ extern "C" int smx_reduce_forces_device_noalloc(smx_model* m, int num_atoms, con
     // are NaN instead
     hipError_t e = smx::launch_fill<int>(flag, 1, 0, s);
     smx::ForceGather g{};
-    g.num_atoms = num_atoms; g.num_nodes = v.num_receivers; g.first_neigh = v.first_neigh;
+    g.num_atoms = num_atoms; g.num_nodes = v.num_receivers; g.first_neigh = v.first_neigh; g.num_edges = E;
     g.forces = v.node_forces; g.xyz = v.xyz; g.atom_forces = d_atom_forces; g.flag = flag;
     if (d_virial) g.partial = partial;
     if (d_atom_forces) {
