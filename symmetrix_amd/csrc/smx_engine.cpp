@@ -207,6 +207,7 @@ struct EngineBase {
     virtual void fill_array(const char* name, long n, double value) = 0;
     virtual void forces_view(ForcesView* v) = 0;
     virtual void check_device_status(bool on_device) = 0;   // the stream has been waited for
+    virtual void finish_host_call() = 0;                    // waits; an evaluation of host arrays that was refused raises
     virtual void evaluate_list(int N, const int* node_types, const int* num_neigh, const int* neigh_indices,
                                const int* neigh_types, const double* xyz, const double* r, long E, double* energies,
                                double* forces, double* virial) = 0;
@@ -275,6 +276,9 @@ struct Engine : EngineBase {
     DVec<int> first_neigh, scan_tmp, s_count, s_start, s_list, t_count, t_start, t_cursor, t_perm, flags;
     int sender_rows = 0;
     long sender_edges = -1;        // edges that s_start / s_list cover
+    bool guarded = false;          // offsets and lists are those of a whole-pipeline call, emptied if its checks failed (flags[3])
+    bool evaluating = false;       // a whole-pipeline call has begun to replace what the one before left
+    bool refused = false;          // the last one failed: there are no forces until something else makes some
     bool senders_differ = false;   // a caller's sender atoms were not the senders of the evaluation before
     // pair terms: ZBL constants per species pair, density-normalisation splines, divisors of the last forward pass
     DVec<double> zbl_a, zbl_rmax, zbl_zz, A0spl, A1spl, div0, div1;
@@ -535,6 +539,32 @@ struct Engine : EngineBase {
 
     // ------------------------------------------------------------------
     // geometry handling
+
+    // What a failed evaluation leaves is not used again: unchecked indices on the device, emptied lists, forces that were never
+    // computed.  Stage calls then need their inputs anew, and there is nothing to reduce.
+    void forget_evaluation()
+    {
+        node_types = num_neigh = neigh_indices = neigh_types = nullptr;
+        xyz = r = nullptr;
+        E = E1 = geo_edges = 0; N_geo = 0;
+        sender_rows = -1; sender_edges = -1; guarded = false;
+        node_forces.n = node_energies.n = 0;
+        pending_A1_adj = pending_A0_adj = pending_A1 = pending_A0 = pending_M0_grad = -1;
+        refused = true;
+    }
+    bool has_forces() const { return !refused || node_forces.n > 0; }
+    // word that tells whether the evaluation whose lists are in place was skipped
+    const int* skipped_word() const { return guarded ? flags.p + 3 : nullptr; }
+    void finish_host_call() override
+    {
+        HIPCHK(hipStreamSynchronize(stream));
+        try {
+            check_device_status(false);
+        } catch (...) {
+            forget_evaluation();
+            throw;
+        }
+    }
     void set_geometry_ptrs(int N, const int* nt, const int* nn, const int* ni, const int* nty, const double* x,
                            const double* rr, long E_, bool on_device)
     {
@@ -594,6 +624,7 @@ struct Engine : EngineBase {
     {
         hipStream_t s = stream;
         const int T = hm.T;
+        if (N > 0) need(node_types, "node_types");
         t_count.size_to(T, s); t_start.size_to((size_t)T + 1, s); t_cursor.size_to(T, s); t_perm.size_to(N, s);
         scan_tmp.size_to((size_t)std::max(N, T) / 1024 + 2, s);
         HIPCHK(launch_type_groups(node_types, N, T, t_count.p, t_start.p, t_cursor.p, t_perm.p, scan_tmp.p, s));
@@ -670,6 +701,14 @@ struct Engine : EngineBase {
     {
         if (!p) throw Error(SMX_EINVAL, std::string("stage called before its inputs exist: ") + what);
     }
+    // offsets and species of the edges of N receivers
+    void need_edges(int N)
+    {
+        need(first_neigh.p, "num_neigh");
+        if (N > N_geo) throw Error(SMX_EINVAL, "stage called for more nodes than the last num_neigh");
+        if (N > 0) need(node_types, "node_types");
+        if (E > 0) need(neigh_types, "neigh_types");
+    }
 
     // Whether a layer's aggregation and adjoint take the kernels for scalar sender features: a diagonal coupling, and byte
     // offsets into the tables and the sender rows (`rows` of them) that fit 32 bits.
@@ -701,7 +740,7 @@ struct Engine : EngineBase {
     // ---- stages ------------------------------------------------------
     void st_agg0_fwd(int N)
     {
-        need(xyz, "xyz (compute_Y)"); need(r, "r (compute_R0)"); need(first_neigh.p, "num_neigh");
+        need(xyz, "xyz (compute_Y)"); need(r, "r (compute_R0)"); need_edges(N);
         Phi0.size_to((size_t)N * 16 * K(), stream);
         HIPCHK(agg_fwd(0, N, Phi0.p));
     }
@@ -827,7 +866,7 @@ struct Engine : EngineBase {
     void st_scale(int layer, int N, bool reverse)
     {
         if (!(layer == 0 ? hm.A0_scaled : hm.A1_scaled)) return;
-        need(r, "r"); need(first_neigh.p, "num_neigh"); need(node_types, "node_types"); need(neigh_types, "neigh_types");
+        need(r, "r"); need_edges(N);
         DVec<double>& dv = layer == 0 ? div0 : div1;
         DVec<F>& A = layer == 0 ? A0 : A1;
         DVec<F>& Aa = layer == 0 ? A0_adj : A1_adj;
@@ -906,7 +945,7 @@ struct Engine : EngineBase {
     }
     void st_agg1_fwd(int N)
     {
-        need(xyz, "xyz (compute_Y)"); need(r, "r (compute_R1)"); need(neigh_indices, "neigh_indices");
+        need(xyz, "xyz (compute_Y)"); need(r, "r (compute_R1)"); need(neigh_indices, "neigh_indices"); need_edges(N);
         Phi1.size_to((size_t)N * NE() * K(), stream);
         HIPCHK(agg_fwd(1, N, Phi1.p));
     }
@@ -1044,7 +1083,7 @@ struct Engine : EngineBase {
     }
     void st_agg1_bwd(int N, bool zero_dxyz, bool zero_H1_adj)
     {
-        need(xyz, "xyz"); need(r, "r"); need(neigh_indices, "neigh_indices");
+        need(xyz, "xyz"); need(r, "r"); need(neigh_indices, "neigh_indices"); need_edges(N);
         const int k = K(), nlm = NLM();
         node_forces.resize((size_t)3 * E, stream);
         H1_adj.resize(H1.n, stream);
@@ -1125,7 +1164,7 @@ struct Engine : EngineBase {
     }
     void st_agg0_bwd(int N)
     {
-        need(xyz, "xyz"); need(r, "r");
+        need(xyz, "xyz"); need(r, "r"); need_edges(N);
         node_forces.resize((size_t)3 * E, stream);
         auto p = agg_params(0, N);
         p.d_out = separate_dPhi0(N) ? dPhi0.p : Phi0.p; p.forces = node_forces.p; p.accumulate_forces = 1; p.msg = nullptr;
@@ -1171,9 +1210,12 @@ struct Engine : EngineBase {
             if (guard_status && !guard_clear_enqueued) (void)launch_fill<int>(guard_status, 1, 0, stream);
             (void)launch_fill<int>(flags.p + 4, 1, 0, stream);
             guard_status = nullptr;
+            if (evaluating) forget_evaluation();
+            evaluating = false;
             throw;
         }
         guard_status = nullptr;
+        evaluating = refused = false;
     }
     void compute_impl(int N, const int* nt, const int* nn, const int* ni, const int* nty, const double* x,
                       const double* rr, long E_, bool on_device, double* d_energies, double* d_forces, int N_local,
@@ -1193,15 +1235,16 @@ struct Engine : EngineBase {
         if (!on_device) edges_from_counts_check(N, nn, E_);
         if (N == 0) {
             if (E_ != 0) throw Error(SMX_EINVAL, "edges without nodes");
-            E = 0; N_geo = 0;
+            E = 0; N_geo = 0; geo_edges = 0; sender_rows = -1; guarded = false;
             node_energies.size_to(0, stream); node_forces.size_to(0, stream);
             return;
         }
+        evaluating = true;
         stage_begin(ST_PREP);
         if (on_device) set_geometry_ptrs(N, nt, nn, ni, nty, x, rr, E_, true);
         else upload_inputs(N, nt, nn, ni, nty, x, rr, E_);
         if (N1 < N) E1 = E_local;
-        geo_edges = E_; split_nodes = N1;
+        geo_edges = E_; split_nodes = N1; guarded = true;
         // Range checks come before any kernel that uses these integers as indices: inside the list preparation, whose last
         // launch empties the lists when a check failed (input_guard).  Host arrays are checked the same way and the result
         // is looked at when the call waits for the stream anyway.
@@ -1336,8 +1379,18 @@ struct Engine : EngineBase {
             const long have = E_ >= 0 ? E_ : E;
             if (own_edges > have) throw Error(SMX_EINVAL, "sum(num_neigh) exceeds the number of edges");
         }
+        if (guarded) {
+            // (a device-resident evaluation before this call: were its arrays fit for use?)
+            int skipped = 0;
+            HIPCHK(hipMemcpyAsync(&skipped, flags.p + 3, sizeof(int), hipMemcpyDeviceToHost, stream));
+            HIPCHK(hipStreamSynchronize(stream));
+            if (skipped) forget_evaluation();
+        }
         set_geometry_ptrs(N, nt, nn, ni, nty, x, rr, E_, false);
-        if (nn) { build_first_neigh(N); E1 = own_edges; geo_edges = own_edges; }
+        if (nn) {
+            build_first_neigh(N); E1 = own_edges; geo_edges = own_edges;
+            if (guarded) { sender_edges = -1; guarded = false; }
+        }
         validate_stage_inputs(N, nt != nullptr, ni != nullptr, nty != nullptr, rr != nullptr);
         if (s == "Y" || s == "R0" || s == "R1") return;  // geometry remembered; evaluated inside the fused kernels
         if (s == "A0") { build_type_groups(N); st_agg0_fwd(N); st_A0_lin(N, false); }
@@ -1370,8 +1423,7 @@ struct Engine : EngineBase {
             // zbl.cpp:96-125 adds to the caller's node_energies / node_forces: here to the engine's arrays, which
             // grow like std::vector::resize (new entries zero) when the edge list changed
             if (hm.has_zbl) {
-                need(xyz, "xyz"); need(r, "r"); need(first_neigh.p, "num_neigh"); need(node_types, "node_types");
-                need(neigh_types, "neigh_types");
+                need(xyz, "xyz"); need(r, "r"); need_edges(N);
                 node_energies.resize((size_t)N, stream);
                 node_forces.resize((size_t)3 * E, stream);
                 st_zbl(N);
@@ -1427,7 +1479,7 @@ struct Engine : EngineBase {
         const size_t len = array_length(s);
         if (n) *n = (long)len;
         if (s == "Y" || s == "Y_grad") need(xyz, "xyz (compute_Y)");
-        if (s == "R0" || s == "R1") { need(r, "r (compute_R0/R1)"); need(first_neigh.p, "num_neigh"); need(node_types, "node_types"); }
+        if (s == "R0" || s == "R1") { need(r, "r (compute_R0/R1)"); need_edges(N_geo); }
         if (!out) return;
         // (arrays the evaluation left unwritten are formed when they are asked for; the others do not wait for that)
         if (s == "A1_adj" || s == "A0_adj" || s == "M0_grad") materialise_adjoints(s == "M0_grad");
@@ -1497,7 +1549,8 @@ struct Engine : EngineBase {
 
     void forces_view(ForcesView* v) override
     {
-        v->node_forces = node_forces.p; v->forces_len = (long)node_forces.n; v->xyz = xyz; v->first_neigh = first_neigh.p;
+        v->node_forces = has_forces() ? node_forces.p : nullptr; v->forces_len = (long)node_forces.n; v->xyz = xyz;
+        v->first_neigh = first_neigh.p; v->skipped = skipped_word();
         v->num_edges = E; v->num_receivers = N_geo; v->device = device;
     }
     // size a named array to n entries, all equal to `value`, without a host copy
@@ -1530,11 +1583,13 @@ struct Engine : EngineBase {
     {
         hipStream_t s = stream;
         need(node_forces.p, "node_forces");
+        if (!has_forces()) throw Error(SMX_EINVAL, "the last evaluation was refused: there are no forces to reduce");
         if (node_forces.n != (size_t)3 * E) throw Error(SMX_EINVAL, "node_forces does not match the current edge list");
         if (!atom_forces && !virial) return;
         if (virial && E > 0) need(xyz, "xyz");
         ForceGather g{};
         g.num_nodes = N_geo; g.first_neigh = first_neigh.p; g.num_edges = E; g.forces = node_forces.p; g.xyz = xyz;
+        g.skipped = skipped_word();
         int atoms = N_geo;
         if (atom_forces) {
             atoms = num_atoms;
@@ -1633,6 +1688,7 @@ struct Engine : EngineBase {
         compute(N, nt, nn, ni, nty, x, rr, E_, true, out + RF_HEAD + (size_t)3 * N, nullptr, -1, -1);
         ForceGather g{};
         g.num_nodes = N; g.first_neigh = first_neigh.p; g.num_edges = E; g.forces = node_forces.p; g.xyz = xyz;
+        g.skipped = skipped_word();
         g.send_start = s_start.p; g.send_list = s_list.p;
         g.atom_forces = out + RF_HEAD;
         gather_forces(g, N, out + 2);
@@ -2086,8 +2142,7 @@ int smx_compute_node_energies_forces(smx_model* m, int num_nodes, const int* nod
         if (num_edges > 0 && (!neigh_indices || !neigh_types || !xyz || !r)) throw smx::Error(SMX_EINVAL, "null edge array");
         e.stream = nullptr;
         e.compute(num_nodes, node_types, num_neigh, neigh_indices, neigh_types, xyz, r, num_edges, false, nullptr, nullptr, -1, -1);
-        HIPCHK(hipStreamSynchronize(e.stream));
-        e.check_device_status(false);
+        e.finish_host_call();
     });
 }
 
@@ -2118,8 +2173,7 @@ int smx_compute_ghosted(smx_model* m, int num_local_nodes, int num_ghost_nodes, 
         e.stream = nullptr;
         e.compute(n, node_types, num_neigh, neigh_indices, neigh_types, xyz, r, num_edges, false, nullptr, nullptr,
                   num_local_nodes, -1);
-        HIPCHK(hipStreamSynchronize(e.stream));
-        e.check_device_status(false);
+        e.finish_host_call();
     });
 }
 

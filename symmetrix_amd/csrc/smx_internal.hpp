@@ -12,6 +12,7 @@ struct ForcesView {
     const double* node_forces;   // [num_edges][3]
     const double* xyz;           // [num_edges][3]
     const int* first_neigh;      // [num_receivers + 1]
+    const int* skipped;          // not zero: the evaluation was skipped and these arrays say nothing (null: no such word)
     long num_edges, forces_len;
     int num_receivers;
     int device;                  // ordinal of the GPU that holds the model and these arrays

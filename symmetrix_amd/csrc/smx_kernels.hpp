@@ -363,7 +363,8 @@ struct ForceGather {
     const double* forces; const double* xyz;         // [E][3] (xyz for the virial only)
     double* atom_forces;                             // [num_atoms][3] or null
     double* partial;                                 // [force_gather_blocks][6], needed for the virial, else null
-    const int* flag;                                 // raised: the outputs are NaN (or null)
+    const int* flag;                                 // raised, or ...
+    const int* skipped;                              // ... this one: the outputs are NaN (each may be null)
     const int* senders;                              // sender atom of every edge, where send_list is another array's: compared,
     int* differ;                                     // ... and set to 1 where they are not the same (null: not compared)
 };

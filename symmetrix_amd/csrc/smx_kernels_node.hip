@@ -960,6 +960,7 @@ template hipError_t launch_readout_fused<float>(int, int, int, int, const int*, 
 // gather of 24-byte forces at large ones.
 namespace {
 constexpr int GATHER_CAP = 512;
+__device__ __forceinline__ bool no_result(const int* flag, const int* skipped) { return (flag && *flag) || (skipped && *skipped); }
 __device__ __forceinline__ void add_virial(double (&v)[6], const double* d, const double* f)
 {
     const double x = d[0], y = d[1], z = d[2];
@@ -997,14 +998,14 @@ __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
         }
         if (a.atom_forces) {
             fx = wave_sum(fx); fy = wave_sum(fy); fz = wave_sum(fz);
-            if (a.flag && *a.flag) fx = fy = fz = __builtin_nan("");
+            if (no_result(a.flag, a.skipped)) fx = fy = fz = __builtin_nan("");
             if (lane < 3) a.atom_forces[3 * (size_t)at + lane] = lane == 0 ? fx : (lane == 1 ? fy : fz);
         }
         wave_lds_sync();   // the next atom's bucket overwrites this one's
     }
     if (!a.partial) return;
     // Edges behind those of the nodes (the last counts covered the leading nodes of a longer edge list): every edge is in the
-    // virial.  After an evaluation that its input checks skipped these are all edges, and their forces are NaN.
+    // virial.
     for (long e = (a.first_neigh ? a.first_neigh[a.num_nodes] : 0) + (long)blockIdx.x * 256 + threadIdx.x; e < a.num_edges;
          e += (long)gridDim.x * 256)
         add_virial(v, a.xyz + 3 * (size_t)e, a.forces + 3 * (size_t)e);
@@ -1019,13 +1020,14 @@ __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
             (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 // the blocks' partial sums in a fixed order
-__global__ __launch_bounds__(384) void k_virial_finish(const double* partial, int nblocks, const int* flag, double* virial)
+__global__ __launch_bounds__(384) void k_virial_finish(const double* partial, int nblocks, const int* flag, const int* skipped,
+                                                      double* virial)
 {
     const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
     double v = 0.0;
     for (int b = lane; b < nblocks; b += 64) v += partial[(size_t)b * 6 + q];
     v = wave_sum(v);
-    if (lane == 0) virial[q] = flag && *flag ? __builtin_nan("") : v;
+    if (lane == 0) virial[q] = no_result(flag, skipped) ? __builtin_nan("") : v;
 }
 }  // namespace
 
@@ -1034,7 +1036,7 @@ hipError_t launch_force_gather(const ForceGather& g, double* virial, hipStream_t
 {
     const int nb = force_gather_blocks(g.num_atoms);
     hipLaunchKernelGGL(k_force_gather, dim3(nb), dim3(256), 0, s, g);
-    if (virial) hipLaunchKernelGGL(k_virial_finish, dim3(1), dim3(384), 0, s, g.partial, nb, g.flag, virial);
+    if (virial) hipLaunchKernelGGL(k_virial_finish, dim3(1), dim3(384), 0, s, g.partial, nb, g.flag, g.skipped, virial);
     return hipGetLastError();
 }
 

@@ -112,7 +112,7 @@ extern "C" int smx_reduce_forces_device_noalloc(smx_model* m, int num_atoms, con
     hipError_t e = smx::launch_fill<int>(flag, 1, 0, s);
     smx::ForceGather g{};
     g.num_atoms = num_atoms; g.num_nodes = v.num_receivers; g.first_neigh = v.first_neigh; g.num_edges = E;
-    g.forces = v.node_forces; g.xyz = v.xyz; g.atom_forces = d_atom_forces; g.flag = flag;
+    g.forces = v.node_forces; g.xyz = v.xyz; g.atom_forces = d_atom_forces; g.flag = flag; g.skipped = v.skipped;
     if (d_virial) g.partial = partial;
     if (d_atom_forces) {
         if (e == hipSuccess) e = smx::launch_fill<int>(count, num_atoms, 0, s);

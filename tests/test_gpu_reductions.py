@@ -67,9 +67,53 @@ def test_no_alloc_virial_of_a_skipped_evaluation_is_nan(tmp_models):
     eng.compute_device(len(sp), *[x.data_ptr() for x in d], len(ea["r"]))
     dF = torch.zeros((len(sp), 3), dtype=torch.float64, device="cuda:0"); dV = torch.zeros(6, dtype=torch.float64, device="cuda:0")
     _no_alloc(eng, len(sp), senders, dF, dV)
-    assert torch.isnan(dV).all() and torch.isnan(dF).any()
+    assert torch.isnan(dV).all() and torch.isnan(dF).all()
     dV.zero_()
     _no_alloc(eng, len(sp), senders, None, dV)
     assert torch.isnan(dV).all()
     with pytest.raises(ValueError):
         eng.synchronize()
+    # the reason is reported once; the sums stay NaN, whichever sender lists they are formed from
+    owners = np.arange(len(sp), dtype=np.int32)
+    for kw in (dict(), dict(receiver_atom=owners)):
+        F, V = eng.reduce_forces(len(sp), ea["neigh_indices"], virial=True, **kw)
+        assert np.isnan(F).all() and np.isnan(V).all()
+    # stage calls do not take up the unchecked arrays
+    with pytest.raises(ValueError, match="before its inputs exist"):
+        eng.compute_Phi1(len(sp), ea["num_neigh"], ea["neigh_indices"])
+
+
+def test_nothing_is_reduced_after_a_refused_evaluation(tmp_models):
+    """Host arrays that fail their checks: the call raises, and so does every use of what it would have computed, until an
+    evaluation or a sequence of stage calls has made new forces."""
+    from symmetrix_amd.mace import MACE
+    model = H.tiny_model(K=16, L_max=0, n_pts=48, seed=23, zbl=True)
+    eng = MACE(H.write_model(model, tmp_models / "refused.json"))
+    pos, cell, sp = H.small_system(30, seed=5)
+    nl, ea = H.edges_of(pos, cell, sp, model["r_cut"])
+    N, nt, nn, ni, nty, xyz, r = H.call_args(ea)
+    owners = np.arange(N, dtype=np.int32)
+    good = (N, nt, nn, ni, nty, xyz, r)
+    eng.compute_node_energies_forces(*good)
+    f_ref, (F_ref, V_ref) = eng.node_forces, eng.reduce_forces(N, ni, virial=True)
+    assert np.abs(F_ref).max() > 0.0
+    for key, at, value in (("species of an edge", 4, 3), ("species of a node", 1, -1), ("sender", 3, N), ("length", 6, 2.0 * model["r_cut"])):
+        bad = list(good)
+        bad[at] = good[at].copy(); bad[at][7] = value
+        print(key, flush=True)
+        with pytest.raises(ValueError):
+            eng.compute_node_energies_forces(*bad)
+        for kw in (dict(), dict(virial=True), dict(receiver_atom=owners)):
+            with pytest.raises(ValueError, match="refused"):
+                eng.reduce_forces(N, ni, **kw)
+        with pytest.raises(ValueError, match="before its inputs exist"):
+            eng.reverse_Phi1(N, nn, ni, xyz, r)      # (species are those of the refused call)
+        # forces made by stage calls alone
+        eng.compute_ZBL(N, nt, nn, nty, r, xyz)
+        f = eng.node_forces
+        assert np.isfinite(f).all() and np.abs(f).max() > 0.0
+        assert np.allclose(eng.reduce_forces(N, ni), H.atom_forces(nl, f, N), rtol=0, atol=1e-12 * max(1.0, np.abs(f).max()))
+        eng.compute_node_energies_forces(*good)
+        assert np.array_equal(eng.node_forces, f_ref)
+        F, V = eng.reduce_forces(N, ni, virial=True)
+        assert np.array_equal(F, F_ref) and np.array_equal(V, V_ref)
