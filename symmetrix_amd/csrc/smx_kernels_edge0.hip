@@ -33,7 +33,8 @@ struct Lds0 {
     static constexpr int NY = BWD ? 48 : 16;          // [lm][3]: harmonic, its two tangential derivatives; or harmonics
     static constexpr size_t val_bytes = ((size_t)CH * NY + 16) * sizeof(F);
     static constexpr size_t head_bytes = (size_t)(CH + 2) * (sizeof(F) + 2 * sizeof(unsigned));
-    static constexpr size_t sum_bytes = BWD ? (size_t)(CH + 2) * 4 * sizeof(F) : 0;
+    static constexpr size_t sum_bytes = BWD ? (size_t)(CH + 2) * 4 * sizeof(double) : 0;
+    static_assert(val_bytes % 16 == 0, "the sums begin on a 16-byte boundary");
     static constexpr size_t per_wave = (val_bytes + head_bytes + sum_bytes + 15) / 16 * 16;
 };
 
@@ -237,11 +238,13 @@ __global__ __launch_bounds__(256, 2) void k_agg0_fwd(const AggParams<F> a, const
 }
 
 // Three sums over the lanes of each half-wavefront (EW = 2) or over all lanes (EW = 1).  On return lane 0 of the half
-// holds s, lane 16 g1, lane 8 g2.
+// holds s, lane 16 g1, lane 8 g2.  In single precision two lanes (up to eight channels) are added as they are, everything beyond
+// in double: the forces come from sums over all channels, which cancel.
 template <int EW, typename F>
-__device__ __forceinline__ F edge_sum3(F s, F g1, F g2, int lane)
+__device__ __forceinline__ double edge_sum3(F s, F g1, F g2, int lane)
 {
     if constexpr (EW == 1) {
+        static_assert(sizeof(F) == 8, "half-wavefronts in single precision");
         F t = g2;
         swap_halves(s, t);
         F a = s + t;                     // lower half s, upper half g2
@@ -257,8 +260,8 @@ __device__ __forceinline__ F edge_sum3(F s, F g1, F g2, int lane)
         swap_rows(s, g1);
         swap_rows(g2, t);
         F x = s + g1, y = g2 + t;        // rows 0, 2: s; rows 1, 3: g1; y: g2 in every row
-        x += row_rotate<8>(x); y += row_rotate<8>(y);
-        F z = (lane & 8) ? y : x;
+        const F mine = (lane & 8) ? y : x, other = (lane & 8) ? x : y;      // the lane eight further on wants the other one
+        double z = (double)mine + (double)row_rotate<8>(other);
         z += half_mirror(z); z += lane_xor1(z); z += lane_xor2(z);
         return z;
     }
@@ -277,8 +280,8 @@ __global__ __launch_bounds__(256, 2) void k_agg0_bwd(const AggParams<F> a, const
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = lane / LPE, sl = lane % LPE;
     unsigned char* base = smem + (size_t)wave * L::per_wave;
     F* vals = reinterpret_cast<F*>(base);                       // [CH][16][3]
-    F* sums = reinterpret_cast<F*>(base + L::val_bytes);        // [CH + 2][4]
-    F* xs = sums + (CH + 2) * 4;                                // [CH + 2]
+    double* sums = reinterpret_cast<double*>(base + L::val_bytes);    // [CH + 2][4]
+    F* xs = reinterpret_cast<F*>(sums + (CH + 2) * 4);          // [CH + 2]
     unsigned* toff = reinterpret_cast<unsigned*>(xs + CH + 2);
     unsigned* goff = toff + CH + 2;
 
@@ -439,7 +442,7 @@ __global__ __launch_bounds__(256, 2) void k_agg0_bwd(const AggParams<F> a, const
                         if (active[c]) store_stream(reinterpret_cast<F*>(mchunk + (off + k[c] * (unsigned)sizeof(F))), V[c][0]);
                 }
             }
-            const F s = edge_sum3<EW>(srad, g1, g2, lane);
+            const double s = edge_sum3<EW>(srad, g1, g2, lane);
             if (writes) sums[le * 4 + out_slot] = s;
         }
         wave_lds_sync();
@@ -449,7 +452,7 @@ __global__ __launch_bounds__(256, 2) void k_agg0_bwd(const AggParams<F> a, const
             EdgeFrame f;
             edge_frame(a.xyz + 3 * e, f);
             const double ir = rcp_pos(a.r[e]);
-            const double sr = (double)sums[lane * 4] * ir, G1 = (double)sums[lane * 4 + 1], G2 = (double)sums[lane * 4 + 2];
+            const double sr = sums[lane * 4] * ir, G1 = sums[lane * 4 + 1], G2 = sums[lane * 4 + 2];
             double fx = -(f.dx * sr + f.t1x * G1 + f.t2x * G2);
             double fy = -(f.dy * sr + f.t1y * G1 + f.t2y * G2);
             double fz = -(f.dz * sr + f.t1z * G1 + f.t2z * G2);
