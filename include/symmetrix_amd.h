@@ -271,6 +271,9 @@ int smx_nlist_build_box(smx_nlist* nl, int num_atoms, const double* positions, c
  * order of the null stream, which is where smx_evaluate_list takes them up (a caller that does nothing else with the list
  * saves the time between the end of the search and the first launch after it). */
 int smx_nlist_set_wait(smx_nlist* nl, int wait);
+/* How often a thread block of a list kernel looks for the counts of the blocks before it until it counts their entries
+ * itself (default: 4096).  The list does not depend on it; 0, where no block looks, is for tests of that way. */
+int smx_nlist_set_chain_rounds(smx_nlist* nl, int rounds);
 int smx_nlist_update_host(smx_nlist* nl, const double* positions, double r_cut, long* num_edges);
 int smx_nlist_inputs(smx_nlist* nl, const double** d_positions, const int** d_types);
 int smx_nlist_arrays(smx_nlist* nl, const int** num_neigh, const int** first_neigh, const int** neigh_indices,

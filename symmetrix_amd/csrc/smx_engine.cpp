@@ -1778,6 +1778,7 @@ struct NeighborList {
     DVec<unsigned long long> chain_sums;
     HostBuf<unsigned long long> chain_total;
     unsigned launches = 0;    // tag of the last chained launch
+    int chain_rounds = NL_CHAIN_ROUNDS;
     bool wait = true;         // false: a build from host positions returns when the number of edges is known (smx_nlist_set_wait)
     const double* shift_vec = nullptr;
     const int* shift_int = nullptr;
@@ -1868,12 +1869,13 @@ struct NeighborList {
             launches = 1;
         }
         NlChain c;
-        c.sums = chain_sums.p; c.tag = (unsigned long long)launches << 32; c.host_total = total;
+        c.sums = chain_sums.p; c.tag = (unsigned long long)launches << 32; c.host_total = total; c.rounds = chain_rounds;
         *total = 0;
         return c;
     }
     // The total of a chained launch: after the stream has finished, or (early) as soon as the launch has written it, which is
-    // before its entries are complete.
+    // before its entries are complete.  The wait ends with the launch, whose blocks do not wait without a bound: the stream is
+    // asked now and then whether it has failed, or finished without a total.
     long chained_total(const NlChain& c, bool early, hipStream_t s)
     {
         const volatile unsigned long long* word = c.host_total;
@@ -2413,6 +2415,13 @@ int smx_nlist_set_wait(smx_nlist* nl, int wait)
     return guarded([&] {
         if (!nl) throw smx::Error(SMX_EINVAL, "null argument");
         reinterpret_cast<smx::NeighborList*>(nl)->wait = wait != 0;
+    });
+}
+int smx_nlist_set_chain_rounds(smx_nlist* nl, int rounds)
+{
+    return guarded([&] {
+        if (!nl || rounds < 0) throw smx::Error(SMX_EINVAL, "null list or negative number of rounds");
+        reinterpret_cast<smx::NeighborList*>(nl)->chain_rounds = rounds;
     });
 }
 void smx_nlist_free(smx_nlist* nl) { delete reinterpret_cast<smx::NeighborList*>(nl); }

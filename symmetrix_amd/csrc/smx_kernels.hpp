@@ -114,12 +114,15 @@ struct NlEdgeArrays {
     double* r;
 };
 // Offsets found inside the launch that uses them (chained_offset): one slot per block, a tag in the upper 32 bits that no
-// earlier launch on these slots had, and a word in host memory for tag | total (0xffffffff: too many).
+// earlier launch on these slots had, a word in host memory for tag | total (0xffffffff: too many), and how many times a block
+// looks at the slots before it counts for itself what it misses (0: it does not look).
 struct NlChain {
     unsigned long long* sums;
     unsigned long long tag;
     unsigned long long* host_total;
+    int rounds;
 };
+constexpr int NL_CHAIN_ROUNDS = 4096;     // several milliseconds, where a launch on an idle chip waits for microseconds
 // Up to this many atoms: a block reads the slots of all blocks before it (2 048 at most).  Beyond, launches for counting and
 // for the prefix sum are a small part of the whole.
 constexpr int NL_CHAIN_ATOMS = 8192;

@@ -76,12 +76,14 @@ __global__ void k_nl_bin_fill(int N, const int* atom_bin, const int* bin_start, 
 }
 
 // Where a receiver's entries begin, without launches for counting and for the prefix sum: every block publishes the number
-// of its entries, before it waits for anything, and adds up those of the blocks before it.  The waits end: blocks start in
-// order and publish first, and up to NL_CHAIN_ATOMS all of them (8 KB of LDS, under 64 registers, eight to a CU) are on the
-// chip together.  A published number carries the tag of the launch, so nothing is cleared between launches.  The last block hands the total to the host while the entries
-// are still being written.  (Counting, prefix sum and writing were three launches and the total a copy: 28 us of a 24-atom
-// list, 15 us of an update at 501 atoms.)
-__device__ __forceinline__ long chained_offset(const NlChain& ch, int c, int wave, int lane)
+// of its entries, before it waits for anything, and adds up those of the blocks before it.  No block depends on another one
+// running: after a bounded number of looks (blocks before it that have not started, whatever else is on the chip) a block
+// counts the entries of all receivers before its own itself, `count_of` by the wavefront that calls.  A published number
+// carries the tag of the launch, so nothing is cleared between launches.  The last block hands the total to the host while the
+// entries are still being written.  (Counting, prefix sum and writing were three launches and the total a copy: 28 us of a
+// 24-atom list, 15 us of an update at 501 atoms.)
+template <typename CountOf>
+__device__ __forceinline__ long chained_offset(const NlChain& ch, int c, int wave, int lane, CountOf&& count_of)
 {
     __shared__ int counts[4];
     __shared__ long long parts[4];
@@ -91,10 +93,11 @@ __device__ __forceinline__ long chained_offset(const NlChain& ch, int c, int wav
     if (threadIdx.x == 0)
         __hip_atomic_store(&ch.sums[blockIdx.x], ch.tag | sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     long long before = 0;
-    for (unsigned b0 = 0; b0 < blockIdx.x; b0 += 4 * 256) {
+    bool all = true;
+    for (unsigned b0 = 0; all && b0 < blockIdx.x; b0 += 4 * 256) {
         unsigned long long v[4];
-        bool all;
-        do {
+        all = false;
+        for (int look = 0; !all && look < ch.rounds; ++look) {
             all = true;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -102,14 +105,24 @@ __device__ __forceinline__ long chained_offset(const NlChain& ch, int c, int wav
                 v[q] = b < blockIdx.x ? __hip_atomic_load(&ch.sums[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : ch.tag;
                 all = all && (v[q] >> 32) == (ch.tag >> 32);
             }
-        } while (!all);
+        }
+        if (all) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) before += (long long)(v[q] & 0xffffffffull);
+            for (int q = 0; q < 4; ++q) before += (long long)(v[q] & 0xffffffffull);
+        }
     }
+    all = !__any(!all);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) before += __shfl_xor(before, off);
-    if (lane == 0) parts[wave] = before;
+    if (lane == 0) parts[wave] = all ? before : -1;
     __syncthreads();
+    if (parts[0] < 0 || parts[1] < 0 || parts[2] < 0 || parts[3] < 0) {
+        before = 0;
+        for (int k = wave; k < 4 * (int)blockIdx.x; k += 4) before += count_of(k);
+        __syncthreads();      // everybody has seen who gave up
+        if (lane == 0) parts[wave] = before;
+        __syncthreads();
+    }
     before = parts[0] + parts[1] + parts[2] + parts[3];
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
         const unsigned long long total = (unsigned long long)before + sum;
@@ -155,8 +168,8 @@ __global__ __launch_bounds__(256) void k_nl_search(const double* pos, int N, NlG
     const bool real = i < N;
     if (MODE != CHAIN && !real) return;
     const double reach = r_cut * (1.0 + 1e-9) + 1e-12;
-    // the receiver's keys in the order of the walk, to where HOW says; how many there are
-    auto search = [&](auto how, long e0) {
+    // the keys of receiver i in the order of the walk, to where HOW says; how many there are
+    auto search = [&](auto how, int i, long e0) {
         constexpr int HOW = decltype(how)::value;
         const double xi[3] = {pos[3 * (size_t)i], pos[3 * (size_t)i + 1], pos[3 * (size_t)i + 2]};
         int c = 0;
@@ -214,14 +227,14 @@ __global__ __launch_bounds__(256) void k_nl_search(const double* pos, int N, NlG
     constexpr std::integral_constant<int, KEYS_LDS> to_lds{};
     constexpr std::integral_constant<int, KEYS_GLOBAL> to_memory{};
     if constexpr (MODE == COUNT) {
-        const int c = search(none, 0);
+        const int c = search(none, i, 0);
         if (lane == 0) count[i] = c;
     } else {
         long e0;
         int n;
         if constexpr (MODE == CHAIN) {
-            n = real ? search(to_lds, 0) : 0;
-            e0 = chained_offset(chain, n, wave, lane);
+            n = real ? search(to_lds, i, 0) : 0;
+            e0 = chained_offset(chain, n, wave, lane, [&](int k) { return search(none, k, 0); });
             if (!real) return;
             if (lane == 0) {
                 first[i] = (int)e0;
@@ -238,8 +251,8 @@ __global__ __launch_bounds__(256) void k_nl_search(const double* pos, int N, NlG
         // at the total and takes more room)
         if (e0 + n > capacity) return;
         const bool in_lds = n <= SORT_KEYS;
-        if (!in_lds) search(to_memory, e0);
-        else if (MODE == FILL) search(to_lds, e0);
+        if (!in_lds) search(to_memory, i, e0);
+        else if (MODE == FILL) search(to_lds, i, e0);
         // rank of every key among the receiver's keys (they are distinct)
         if (in_lds) wave_lds_sync();
         else __threadfence();
@@ -275,8 +288,9 @@ __global__ __launch_bounds__(256) void k_nl_filter(const double* pos, int N, con
     if (MODE != CHAIN && !real) return;
     // candidates that did not fit were not written to `sorted`
     const bool there = cfirst[N] <= room;
-    const int c0 = real ? cfirst[i] : 0, n = real && there ? cfirst[i + 1] - c0 : 0;
-    auto walk = [&](auto emit, size_t e0) {
+    // kept candidates of receiver i
+    auto walk = [&](auto emit, int i, size_t e0) {
+        const int c0 = cfirst[i], n = there ? cfirst[i + 1] - c0 : 0;
         int kept = 0;
         for (int a0 = 0; a0 < n; a0 += 64) {
             const int a = a0 + lane;
@@ -297,18 +311,18 @@ __global__ __launch_bounds__(256) void k_nl_filter(const double* pos, int N, con
     };
     if constexpr (MODE == FILL) {
         if (!there || first[N] > capacity) return;
-        walk(std::true_type{}, (size_t)first[i]);
+        walk(std::true_type{}, i, (size_t)first[i]);
     } else {
-        const int kept = walk(std::false_type{}, 0);
+        const int kept = real ? walk(std::false_type{}, i, 0) : 0;
         if (real && lane == 0) count[i] = kept;
         if constexpr (MODE == CHAIN) {
-            const long e0 = chained_offset(chain, kept, wave, lane);
+            const long e0 = chained_offset(chain, kept, wave, lane, [&](int k) { return walk(std::false_type{}, k, 0); });
             if (!real) return;
             if (lane == 0) {
                 first[i] = (int)e0;
                 if (i == N - 1) first[N] = (int)(e0 + kept);
             }
-            if (e0 + kept <= capacity) walk(std::true_type{}, (size_t)e0);
+            if (e0 + kept <= capacity) walk(std::true_type{}, i, (size_t)e0);
         }
     }
 }

@@ -866,6 +866,39 @@ def test_layer0_gradients_on_request_follow_the_calls(gpu, tmp_models, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("atoms", [1, 4, 5, 107, 513, 1100])
+def test_list_blocks_that_stop_waiting_count_for_themselves(atoms):
+    """A block of a list kernel looks for the counts of the blocks before it a bounded number of times, then counts their
+    entries itself.  With no look at all every block goes that way: the same list, with and without bins, with and without a
+    skin, in an update, and where the first room is outgrown (513 atoms)."""
+    import torch
+    from symmetrix_amd import _lib, neighbors
+    assert torch.cuda.is_available()
+    rng = np.random.default_rng(atoms)
+    rc = 5.5 if atoms == 513 else 3.3
+    cell = np.full(3, (atoms * 8.0) ** (1.0 / 3.0))
+    pos = rng.uniform(0, 1, size=(atoms, 3)) * cell
+    types = rng.integers(0, 3, size=atoms).astype(np.int32)
+    nl = neighbors.DeviceNeighborList()
+    for rounds, wait, skin in ((0, True, 0.0), (0, True, 0.4), (0, False, 0.0), (1, True, 0.4), (4096, True, 0.4)):
+        _lib.check(_lib.lib().smx_nlist_set_chain_rounds(nl._C.c_void_p(nl._h), rounds))
+        nl.set_wait(wait)
+        print(f"{atoms} atoms, {rounds} rounds, wait {wait}, skin {skin}", flush=True)
+        E = nl.build_host(pos, types, cell, rc, skin=skin)
+        got, ref = nl.to_host(), neighbors.neighbor_list(pos, cell, rc)
+        assert E == len(ref["r"])
+        for k in ("i", "j", "S", "xyz", "r", "first_neigh"):
+            assert np.array_equal(got[k], ref[k].reshape(got[k].shape)), k
+        if skin:
+            moved = pos + rng.uniform(-0.1, 0.1, size=pos.shape)
+            E = nl.update_host(moved, rc)
+            got, ref = nl.to_host(), neighbors.neighbor_list(moved, cell, rc, offsets=np.zeros((atoms, 3), dtype=int))
+            assert E == len(ref["r"])
+            for k in ("i", "j", "S", "xyz", "r", "first_neigh"):
+                assert np.array_equal(got[k], ref[k].reshape(got[k].shape)), k
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("natoms,density,rc,skin", [(1, 0.2, 6.0, 0.0), (512, 0.1, 4.5, 0.0), (513, 0.1, 4.5, 0.0), (700, 0.9, 4.5, 0.0),
                                                     (200, 0.9, 4.5, 0.3), (600, 0.1, 3.0, 1.5)])
 def test_list_search_at_the_edges_of_its_ways(natoms, density, rc, skin):
