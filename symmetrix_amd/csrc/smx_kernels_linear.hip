@@ -39,10 +39,13 @@ template <> struct MatOp<float> {
 __device__ __forceinline__ int part_of(int slot, int atom) { return slot ^ ((atom >> 2) & 3); }
 // 1 KB of a wavefront from global memory (16 bytes per lane) into LDS at `to` + 16 lane.  In assembly: next to the compiler's
 // own form of this load it lets every read of the LDS, and every use of another load, wait for all loads in flight; here the
-// loop below waits by count.
+// loop below waits by count.  The LDS address goes through m0, which the load may read one wait state after the write (s_nop)
+// and has read when it is issued; m0 belongs to the compiler and is given back as it was.
 __device__ __forceinline__ void load_into_lds(const void* from, unsigned to)
 {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(to) : "memory", "m0");
+    unsigned m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(m0) : "v"(from), "s"(to) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
