@@ -47,8 +47,9 @@ __device__ __forceinline__ void load_into_lds(const void* from, unsigned to)
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
                  : "=&s"(m0) : "v"(from), "s"(to) : "memory");
 }
+// all but the N youngest loads have arrived, and every read of the LDS has
 template <int N>
-__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
 
 // POLY: linear and contraction (one polynomial per channel, with gradients); else the linear alone.  (With several polynomials
 // per channel, values only, a launch of their own came out ahead: the 4 to 9 polynomials of the four atoms of a lane in turn are a
@@ -131,8 +132,8 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_linear(const LinearParams<F> p)
     });
     auto step = [&](int c, auto slot_c) {
         constexpr int slot = decltype(slot_c)::value, ahead = (slot + AHEAD) % BUFS;
-        // the piece requested AHEAD steps ago is in LDS for everybody after this (no __syncthreads: its fence would wait for
-        // the younger pieces too)
+        // the piece requested AHEAD steps ago is in LDS for everybody after this, and everybody has read the piece of the step
+        // before, whose slot the next request overwrites (no __syncthreads: its fence would wait for the younger pieces too)
         wait_loads<(AHEAD - 1) * LOADS>();
 #pragma unroll
         for (int l = 0; l < 4; ++l) asm volatile("" : "+v"(b[slot][l]));      // (here, not after the requests below)
