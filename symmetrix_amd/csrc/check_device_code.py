@@ -6,6 +6,9 @@ instruction of a kind below is followed backwards, over all branches into it, th
 before it:
 
   m0      a load from memory into LDS needs one wait state after a write of m0, which holds its LDS address
+  dpp     an instruction that takes its first source from other lanes (DPP) needs two wait states after the vector
+          instruction that wrote that source, and five after one that wrote the execution mask; where it is the
+          double-precision multiply-add, one after a reciprocal, root or the like wrote any of its sources
 
 Usage: check_device_code.py libsymmetrix_amd.so [llvm-objdump].  The build runs it and fails on a violation.
 """
@@ -108,6 +111,30 @@ def writes_m0(mnemonic, operands):
     return operands.split(",")[0].strip() == "m0" and mnemonic.startswith("s_") and not mnemonic.startswith("s_cmp")
 
 
+REGISTERS = re.compile(r"v\[(\d+):(\d+)\]|v(\d+)")
+
+
+def vector_registers(operand):
+    m = REGISTERS.match(operand.strip())
+    if not m:
+        return set()
+    return {int(m.group(3))} if m.group(3) else set(range(int(m.group(1)), int(m.group(2)) + 1))
+
+
+def written_by_vector(mnemonic, operands):
+    """Vector registers that a vector arithmetic instruction writes."""
+    if not mnemonic.startswith("v_") or mnemonic.startswith(("v_cmp", "v_readlane", "v_readfirstlane")):
+        return set()
+    parts = operands.split(",")
+    out = vector_registers(parts[0])
+    if "swap" in mnemonic and len(parts) > 1:      # (both operands change)
+        out |= vector_registers(parts[1])
+    return out
+
+
+TRANSCENDENTAL = ("v_rcp", "v_rsq", "v_sqrt", "v_exp", "v_log", "v_sin", "v_cos")
+
+
 def violations(kernel):
     """Texts, and how many instructions of the kinds above there are."""
     bad, looked_at = [], 0
@@ -116,6 +143,18 @@ def violations(kernel):
             looked_at += 1
             for j in reached_within(kernel, i, 1, writes_m0):
                 bad.append(f"{kernel.name}: {mnemonic} at {kernel.address[i]:x} right after m0 was written at {kernel.address[j]:x}")
+        if "_dpp" in mnemonic:
+            looked_at += 1
+            parts = operands.split(",")
+            source = vector_registers(parts[1])
+            rules = [(2, lambda m, o: written_by_vector(m, o) & source, "its first source was written"),
+                     (5, lambda m, o: m.startswith("v_cmpx"), "the execution mask was written")]
+            if mnemonic.startswith("v_fmac_f64"):
+                sources = set().union(*(vector_registers(p) for p in parts[:3]))
+                rules.append((1, lambda m, o: m.startswith(TRANSCENDENTAL) and written_by_vector(m, o) & sources, "a source was written"))
+            for states, hit, what in rules:
+                for j in reached_within(kernel, i, states, hit):
+                    bad.append(f"{kernel.name}: {mnemonic} at {kernel.address[i]:x} too soon after {what} at {kernel.address[j]:x}")
     return bad, looked_at
 
 

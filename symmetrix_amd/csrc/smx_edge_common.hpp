@@ -14,7 +14,10 @@ template <typename F>
 constexpr bool kMatrix = sizeof(F) == 4;
 
 // Lane-broadcast multiply-add of the double-precision kernels: acc += (b of lane N of the lane's 16-lane row) * v.  The
-// instruction reads b through DPP: b must not come from the vector instruction right before (here it comes from LDS).
+// instruction reads b through DPP, which needs two wait states after a vector instruction that wrote b.  Here b comes from LDS;
+// that the compiler puts no move, spill or accumulator read of b in front of it is checked in the built code
+// (check_device_code.py: the build fails otherwise).  Its own form of the move from another lane is an instruction by itself,
+// not joined with the multiply-add: twice the instructions of these kernels' inner loops.
 template <int N>
 __device__ __forceinline__ void fmac_lane(double& acc, double b, double v)
 {
