@@ -303,7 +303,7 @@ struct Engine : EngineBase {
     double* energies_copy = nullptr;
     double* forces_copy = nullptr;
     bool senders_counted = false;   // the sender histogram (and s_rank) was formed by the fused node-list launch
-    DVec<int> s_rank;               // place of every edge inside its sender's bucket
+    DVec<int> s_rank;               // place of every edge inside its sender's bucket, until the buckets are filled; then scratch
     long counters_clean = 0;        // leading entries of s_count known to be zero (every sender-list build leaves them so)
     long rf_clean = 0;              // the same for rf_count
 
@@ -1102,11 +1102,12 @@ struct Engine : EngineBase {
         if (fuse_reverse_H1 && nlm == 1 && sender_reduce_linear_ok(k) && M0.n == (size_t)rows * k) {
             // scalar hidden features: reverse_H1 of the summed rows in the same launch
             M0_adj.size_to(M0.n, stream);
-            HIPCHK(launch_sender_reduce_linear<F>(rows, k, s_start.p, s_list.p, msg.p, H1_adj.p, zero_H1_adj ? 1 : 0, H1w.p,
+            HIPCHK(launch_sender_reduce_linear<F>(rows, k, s_start.p, s_list.p, s_rank.p, msg.p, H1_adj.p, zero_H1_adj ? 1 : 0, H1w.p,
                                                   M0_adj.p, stream));
             reverse_H1_done = true;
         } else {
-            HIPCHK(launch_sender_reduce<F>(rows, nlm * k, s_start.p, s_list.p, msg.p, H1_adj.p, zero_H1_adj ? 1 : 0, false, 0, E1, stream));
+            HIPCHK(launch_sender_reduce<F>(rows, nlm * k, s_start.p, s_list.p, s_rank.p, msg.p, H1_adj.p, zero_H1_adj ? 1 : 0,
+                                           false, 0, E1, stream));
         }
         stage_end(ST_SRED);
     }
@@ -1143,7 +1144,7 @@ struct Engine : EngineBase {
         const int groups = agg_bwd_groups(1);
         if (groups > 1) fpart.size_to((size_t)groups * 3 * E, stream);
         if (sender_rows != rows) build_sender_lists(rows);
-        HIPCHK(launch_sort_buckets(s_start.p, rows, s_list.p, stream));   // the windows below need the order in memory
+        HIPCHK(launch_sort_buckets(s_start.p, rows, s_list.p, s_rank.p, stream));   // the windows below need the order in memory
         stage_begin(ST_AGG1B);
         for (int c = 0; c < nchunks; ++c) {
             auto p = agg_params(1, bnd[c + 1]);
@@ -1151,7 +1152,7 @@ struct Engine : EngineBase {
             p.d_out = dPhi1.p; p.forces = node_forces.p; p.accumulate_forces = zero_dxyz ? 0 : 1; p.msg = msg.p;
             p.fpart = groups > 1 ? fpart.p : nullptr;
             HIPCHK(agg_bwd(1, p));
-            HIPCHK(launch_sender_reduce<F>(rows, nlm * k, s_start.p, s_list.p, msg.p, H1_adj.p,
+            HIPCHK(launch_sender_reduce<F>(rows, nlm * k, s_start.p, s_list.p, s_rank.p, msg.p, H1_adj.p,
                                            (c == 0 && zero_H1_adj) ? 1 : 0, true, fe[c], fe[c + 1], stream));
         }
         stage_end(ST_AGG1B);
@@ -1632,7 +1633,7 @@ struct Engine : EngineBase {
         };
         if (same_senders) {
             g.senders = device_senders(); g.differ = reinterpret_cast<int*>(out + 1);
-            g.send_start = s_start.p; g.send_list = s_list.p;
+            g.send_start = s_start.p; g.send_list = s_list.p; g.send_spare = s_rank.p;
             g.atom_forces = out + RF_HEAD;
             gather_forces(g, atoms, virial ? out + 2 : nullptr);
             if (fetch_reduction(num_atoms, atom_forces, virial, nullptr)) return;
@@ -1648,7 +1649,7 @@ struct Engine : EngineBase {
             scan_tmp.size_to((size_t)num_atoms / 1024 + 2, s);
             HIPCHK(launch_sender_lists(send, E, num_atoms, rf_count.p, rf_rank.p, rf_sstart.p, rf_slist.p, scan_tmp.p, false,
                                        flag, s));
-            g.send_start = rf_sstart.p; g.send_list = rf_slist.p;
+            g.send_start = rf_sstart.p; g.send_list = rf_slist.p; g.send_spare = rf_rank.p;
             g.atom_forces = out + RF_HEAD;
         }
         gather_forces(g, atoms, virial ? out + 2 : nullptr);
@@ -1689,7 +1690,7 @@ struct Engine : EngineBase {
         ForceGather g{};
         g.num_nodes = N; g.first_neigh = first_neigh.p; g.num_edges = E; g.forces = node_forces.p; g.xyz = xyz;
         g.skipped = skipped_word();
-        g.send_start = s_start.p; g.send_list = s_list.p;
+        g.send_start = s_start.p; g.send_list = s_list.p; g.send_spare = s_rank.p;
         g.atom_forces = out + RF_HEAD;
         gather_forces(g, N, out + 2);
         fetch_reduction(N, forces, virial, energies);

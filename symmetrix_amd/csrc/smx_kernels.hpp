@@ -76,15 +76,16 @@ hipError_t launch_fpart_reduce(long edges, long E, int groups, const double* fpa
                                double* copy, hipStream_t s, const int* guard = nullptr);
 
 // H_adj[j] (+)= sum of msg[e - e_lo] over the edges e of sender j, in ascending edge order; window: over those with
-// e_lo <= e < e_hi, and slist is in ascending order already (launch_sort_buckets)
+// e_lo <= e < e_hi, and slist is in ascending order already (launch_sort_buckets).  spare, here and below: scratch as long as
+// slist (the ranks of the list build have served), for rows whose edges do not fit the LDS
 template <typename F>
-hipError_t launch_sender_reduce(int rows, int width, const int* sstart, int* slist, const F* msg, F* H_adj,
+hipError_t launch_sender_reduce(int rows, int width, const int* sstart, int* slist, int* spare, const F* msg, F* H_adj,
                                 int zero_first, bool window, long e_lo, long e_hi, hipStream_t s);
 // The same sum for rows of K scalar features, followed by M_adj[rows][K] = H_adj . W^T (W [K][K], row n holding
 // the weights of input channel n: reverse_H1 of an L_max = 0 model) in the same launch; K as sender_reduce_linear_ok
 bool sender_reduce_linear_ok(int K);
 template <typename F>
-hipError_t launch_sender_reduce_linear(int rows, int K, const int* sstart, int* slist, const F* msg, F* H_adj,
+hipError_t launch_sender_reduce_linear(int rows, int K, const int* sstart, int* slist, int* spare, const F* msg, F* H_adj,
                                        int zero_first, const F* W, F* M_adj, hipStream_t s);
 
 // ---------------------------------------------------------------------------
@@ -201,7 +202,7 @@ struct InputChecks {
 hipError_t launch_sender_lists(const int* gather, long E, int rows, int* count, int* rank, int* sstart, int* slist,
                                int* block_sums, bool counted, int* range_flag, hipStream_t s,
                                const InputGuard& guard = InputGuard());
-hipError_t launch_sort_buckets(const int* start, int rows, int* list, hipStream_t s);
+hipError_t launch_sort_buckets(const int* start, int rows, int* list, int* spare, hipStream_t s);
 hipError_t launch_check_counts(const int* num_neigh, int N, const int* first_neigh, int num_local_nodes, long num_edges,
                                long num_local_edges, int* status, hipStream_t s);
 // first_neigh, species groups, the sender histogram count[rows] of `key[n]` with rank[n] = the place each
@@ -359,6 +360,7 @@ hipError_t launch_radial(int N, const int* first_neigh, const int* node_types, c
 struct ForceGather {
     int num_atoms;
     const int* send_start; int* send_list;           // edges by sender atom (null: no sender side)
+    int* send_spare;                                 // as long as send_list, for buckets that do not fit the LDS
     const int* node_start; const int* node_list;     // nodes whose edges count as received by the atom; null: node i is atom i
     int num_nodes;
     const int* first_neigh;                          // [num_nodes + 1], or null without nodes

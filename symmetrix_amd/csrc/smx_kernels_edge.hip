@@ -768,7 +768,7 @@ __device__ __forceinline__ Vec<F, N> ldv_stream(const F* p)
 // messages of the row are, and the block orders the row's edges in LDS first.
 constexpr int SENDER_CAP = 1024;
 template <typename F, int V, bool WINDOW>
-__global__ void k_sender_reduce(int rows, int width, const int* sstart, int* slist_, const F* msg,
+__global__ void k_sender_reduce(int rows, int width, const int* sstart, int* slist_, int* spare, const F* msg,
                                 F* H_adj, int zero_first, long e_lo, long e_hi)
 {
     __shared__ __align__(16) int bucket[WINDOW ? 1 : 2 * SENDER_CAP];
@@ -791,8 +791,7 @@ __global__ void k_sender_reduce(int rows, int width, const int* sstart, int* sli
         slist = bucket + SENDER_CAP;
         s0 = 0; s1 = n;
     } else {
-        if (threadIdx.x == 0) insertion_sort(slist_ + s0, s1 - s0);
-        __threadfence();
+        if (threadIdx.x < 64) wave_sorted_bucket<SENDER_CAP>(slist_, s0, s1 - s0, bucket, threadIdx.x, spare);
         __syncthreads();
     }
     if (s0 == s1 && !zero_first) return;
@@ -825,13 +824,13 @@ __global__ void k_sender_reduce(int rows, int width, const int* sstart, int* sli
 }  // namespace
 
 template <typename F>
-hipError_t launch_sender_reduce(int rows, int width, const int* sstart, int* slist, const F* msg,
+hipError_t launch_sender_reduce(int rows, int width, const int* sstart, int* slist, int* spare, const F* msg,
                                 F* H_adj, int zero_first, bool window, long e_lo, long e_hi, hipStream_t s)
 {
     if (rows <= 0) return hipSuccess;
     constexpr int V = 16 / (int)sizeof(F);
     auto go = [&](auto kern, int bs) {
-        hipLaunchKernelGGL(kern, dim3(rows), dim3(bs), 0, s, rows, width, sstart, slist, msg, H_adj, zero_first, e_lo, e_hi);
+        hipLaunchKernelGGL(kern, dim3(rows), dim3(bs), 0, s, rows, width, sstart, slist, spare, msg, H_adj, zero_first, e_lo, e_hi);
     };
     if (width % V == 0) {
         const int lanes = width / V;
@@ -853,8 +852,8 @@ hipError_t launch_sender_reduce(int rows, int width, const int* sstart, int* sli
 namespace {
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 template <typename F, int KT>
-__global__ __launch_bounds__(1024) void k_sender_reduce_linear(int rows, const int* sstart, int* slist_, const F* msg,
-                                                              F* H_adj, int zero_first, const F* W, F* M_adj)
+__global__ __launch_bounds__(1024) void k_sender_reduce_linear(int rows, const int* sstart, int* slist_, int* spare,
+                                                              const F* msg, F* H_adj, int zero_first, const F* W, F* M_adj)
 {
     constexpr int K = 16 * KT, ld = K + 1, V = 16 / (int)sizeof(F);
     constexpr int ROW_CAP = 256;
@@ -877,7 +876,7 @@ __global__ __launch_bounds__(1024) void k_sender_reduce_linear(int rows, const i
         const int rr = wave, j = row0 + rr;
         const int q = lane * V;
         const int first = j < rows ? sstart[j] : 0, n = j < rows ? sstart[j + 1] - first : 0;
-        const int* slist = wave_sorted_bucket<ROW_CAP>(slist_, first, n, bucket[wave], lane);
+        const int* slist = wave_sorted_bucket<ROW_CAP>(slist_, first, n, bucket[wave], lane, spare);
         if (q < K) {
             Vec<F, V> acc;
 #pragma unroll
@@ -926,26 +925,26 @@ __global__ __launch_bounds__(1024) void k_sender_reduce_linear(int rows, const i
 bool sender_reduce_linear_ok(int K) { return K == 32 || K == 48 || K == 64 || K == 96 || K == 128; }
 
 template <typename F>
-hipError_t launch_sender_reduce_linear(int rows, int K, const int* sstart, int* slist, const F* msg, F* H_adj,
+hipError_t launch_sender_reduce_linear(int rows, int K, const int* sstart, int* slist, int* spare, const F* msg, F* H_adj,
                                        int zero_first, const F* W, F* M_adj, hipStream_t s)
 {
     if (!sender_reduce_linear_ok(K)) return hipErrorInvalidValue;
     if (rows <= 0) return hipSuccess;
     const dim3 grid((unsigned)((rows + 15) / 16)), block(1024);
     switch (K / 16) {
-    case 2: hipLaunchKernelGGL((k_sender_reduce_linear<F, 2>), grid, block, 0, s, rows, sstart, slist, msg, H_adj, zero_first, W, M_adj); break;
-    case 3: hipLaunchKernelGGL((k_sender_reduce_linear<F, 3>), grid, block, 0, s, rows, sstart, slist, msg, H_adj, zero_first, W, M_adj); break;
-    case 4: hipLaunchKernelGGL((k_sender_reduce_linear<F, 4>), grid, block, 0, s, rows, sstart, slist, msg, H_adj, zero_first, W, M_adj); break;
-    case 6: hipLaunchKernelGGL((k_sender_reduce_linear<F, 6>), grid, block, 0, s, rows, sstart, slist, msg, H_adj, zero_first, W, M_adj); break;
-    default: hipLaunchKernelGGL((k_sender_reduce_linear<F, 8>), grid, block, 0, s, rows, sstart, slist, msg, H_adj, zero_first, W, M_adj); break;
+    case 2: hipLaunchKernelGGL((k_sender_reduce_linear<F, 2>), grid, block, 0, s, rows, sstart, slist, spare, msg, H_adj, zero_first, W, M_adj); break;
+    case 3: hipLaunchKernelGGL((k_sender_reduce_linear<F, 3>), grid, block, 0, s, rows, sstart, slist, spare, msg, H_adj, zero_first, W, M_adj); break;
+    case 4: hipLaunchKernelGGL((k_sender_reduce_linear<F, 4>), grid, block, 0, s, rows, sstart, slist, spare, msg, H_adj, zero_first, W, M_adj); break;
+    case 6: hipLaunchKernelGGL((k_sender_reduce_linear<F, 6>), grid, block, 0, s, rows, sstart, slist, spare, msg, H_adj, zero_first, W, M_adj); break;
+    default: hipLaunchKernelGGL((k_sender_reduce_linear<F, 8>), grid, block, 0, s, rows, sstart, slist, spare, msg, H_adj, zero_first, W, M_adj); break;
     }
     return hipGetLastError();
 }
-template hipError_t launch_sender_reduce_linear<double>(int, int, const int*, int*, const double*, double*, int, const double*, double*, hipStream_t);
-template hipError_t launch_sender_reduce_linear<float>(int, int, const int*, int*, const float*, float*, int, const float*, float*, hipStream_t);
+template hipError_t launch_sender_reduce_linear<double>(int, int, const int*, int*, int*, const double*, double*, int, const double*, double*, hipStream_t);
+template hipError_t launch_sender_reduce_linear<float>(int, int, const int*, int*, int*, const float*, float*, int, const float*, float*, hipStream_t);
 
-template hipError_t launch_sender_reduce<double>(int, int, const int*, int*, const double*, double*, int, bool, long, long, hipStream_t);
-template hipError_t launch_sender_reduce<float>(int, int, const int*, int*, const float*, float*, int, bool, long, long, hipStream_t);
+template hipError_t launch_sender_reduce<double>(int, int, const int*, int*, int*, const double*, double*, int, bool, long, long, hipStream_t);
+template hipError_t launch_sender_reduce<float>(int, int, const int*, int*, int*, const float*, float*, int, bool, long, long, hipStream_t);
 
 // ---------------------------------------------------------------------------
 namespace {

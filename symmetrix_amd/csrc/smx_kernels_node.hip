@@ -115,24 +115,15 @@ __global__ void k_place_ranked(const int* key, const int* rank, long n, int rows
 // Ascending order inside every bucket, in memory: for readers that take a window of the edges (the others order a bucket in
 // LDS as they read it).  One wavefront per bucket.
 constexpr int SORT_LDS = 1024;
-__global__ __launch_bounds__(64) void k_sort_buckets(const int* start, int rows, int* list)
+__global__ __launch_bounds__(64) void k_sort_buckets(const int* start, int rows, int* list, int* spare)
 {
-    __shared__ int buf[SORT_LDS];
+    __shared__ __align__(16) int buf[SORT_LDS];
     const int j = blockIdx.x;
     const int s0 = start[j], n = start[j + 1] - s0;
     if (n <= 1) return;
-    if (n <= SORT_LDS) {
-        for (int t = threadIdx.x; t < n; t += 64) buf[t] = list[s0 + t];
-        __syncthreads();
-        for (int t = threadIdx.x; t < n; t += 64) {
-            const int v = buf[t];
-            int rank = 0;
-            for (int q = 0; q < n; ++q) rank += buf[q] < v;
-            list[s0 + rank] = v;
-        }
-    } else if (threadIdx.x == 0) {
-        insertion_sort(list + s0, n);
-    }
+    const int* sorted = wave_sorted_bucket<SORT_LDS>(list, s0, n, buf, threadIdx.x, spare);
+    if (sorted == buf)
+        for (int t = threadIdx.x; t < n; t += 64) list[s0 + t] = sorted[t];
 }
 // species groups in one block: LDS histogram, scan over the (few) species, placement
 __device__ void type_groups_body(const int* node_types, int N, int T, int* tstart, int* perm, int* sh)
@@ -330,9 +321,9 @@ hipError_t launch_sender_lists(const int* gather, long E, int rows, int* count, 
     hipLaunchKernelGGL(k_place_ranked, dim3(nblk(threads, 256)), dim3(256), 0, s, gather, rank, E, rows, sstart, slist, count, guard);
     return hipGetLastError();
 }
-hipError_t launch_sort_buckets(const int* start, int rows, int* list, hipStream_t s)
+hipError_t launch_sort_buckets(const int* start, int rows, int* list, int* spare, hipStream_t s)
 {
-    if (rows > 0) hipLaunchKernelGGL(k_sort_buckets, dim3(rows), dim3(64), 0, s, start, rows, list);
+    if (rows > 0) hipLaunchKernelGGL(k_sort_buckets, dim3(rows), dim3(64), 0, s, start, rows, list, spare);
     return hipGetLastError();
 }
 
@@ -977,7 +968,7 @@ __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
         double fx = 0, fy = 0, fz = 0;
         if (a.send_start) {
             const int s0 = a.send_start[at], n = a.send_start[at + 1] - s0;
-            const int* sorted = wave_sorted_bucket<GATHER_CAP>(a.send_list, s0, n, bucket[wave], lane);
+            const int* sorted = wave_sorted_bucket<GATHER_CAP>(a.send_list, s0, n, bucket[wave], lane, a.send_spare);
             for (int t = lane; t < n; t += 64) {
                 const int e = sorted[t];
                 if (a.senders && a.senders[e] != at) *a.differ = 1;

@@ -118,7 +118,7 @@ extern "C" int smx_reduce_forces_device_noalloc(smx_model* m, int num_atoms, con
         if (e == hipSuccess) e = smx::launch_fill<int>(count, num_atoms, 0, s);
         if (e == hipSuccess)
             e = smx::launch_sender_lists(d_sender_atom, E, num_atoms, count, rank, send_start, send_list, block_sums, false, flag, s);
-        g.send_start = send_start; g.send_list = send_list;
+        g.send_start = send_start; g.send_list = send_list; g.send_spare = rank;
     } else if (e == hipSuccess) {
         e = smx::launch_check_range(d_sender_atom, E, num_atoms, flag, s);
     }

@@ -943,6 +943,48 @@ def test_senders_with_many_edges(gpu, tmp_models, L_max, K, edge):
     assert np.abs(V - W[[0, 1, 2, 0, 0, 1], [0, 1, 2, 1, 2, 2]]).max() <= 1e-9 * max(1.0, np.abs(W).max())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("L_max,K", [(0, 32), (1, 8)])
+@pytest.mark.parametrize("n", [255, 256, 257, 512, 513, 1024, 1025, 2100])
+def test_buckets_on_both_sides_of_the_lds(gpu, tmp_models, n, L_max, K):
+    """One sender of n edges among others of a few: buckets are ordered in the LDS of a wavefront (256 or 512 edges), of a
+    block (1 024), or through it into memory.  Sums against the oracle, and the same bits twice and where the adjoint takes
+    the receivers in chunks (which orders the buckets in memory first)."""
+    model = H.tiny_model(K=K, L_max=L_max, n_pts=32, seed=51, pair=False)
+    rng = np.random.default_rng(n)
+    N, extra = 7, 60
+    senders = rng.permutation(np.concatenate([np.full(n, 3), rng.choice([0, 1, 2, 4, 5], size=extra)])).astype(np.int32)
+    E = len(senders)
+    degree = np.bincount(rng.integers(0, N, size=E), minlength=N).astype(np.int32)
+    species = rng.integers(0, 3, size=N).astype(np.int32)
+    x = rng.normal(size=(E, 3))
+    x *= (rng.uniform(1.0, 3.9, size=E) / np.linalg.norm(x, axis=1))[:, None]
+    args = (N, species, degree, senders, species[senders], x.ravel(), np.linalg.norm(x, axis=1))
+    orc = _oracle()(model)
+    orc.compute_node_energies_forces(*args)
+    eng = gpu(H.write_model(model, tmp_models / f"buckets_{K}.json"), "float64")
+    print(f"{n} of {E} edges from one sender, K={K} L_max={L_max}", flush=True)
+    eng.compute_node_energies_forces(*args)
+    h, f = eng.H1_adj, eng.node_forces
+    assert np.abs(h - orc.H1_adj).max() <= 1e-10 * np.abs(orc.H1_adj).max()
+    assert np.abs(f - orc.node_forces).max() <= 1e-10 * np.abs(orc.node_forces).max()
+    receivers = np.repeat(np.arange(N), degree)
+    want = np.zeros((N, 3))
+    np.add.at(want, senders, f.reshape(-1, 3)); np.add.at(want, receivers, -f.reshape(-1, 3))
+    bound = 1e-13 * np.abs(f).max() * n
+    F = eng.reduce_forces(N, senders)
+    assert np.abs(F - want).max() <= bound
+    shifted = np.where(senders == 3, 6, senders)       # senders that are not the evaluation's: lists of their own
+    want = np.zeros((N, 3))
+    np.add.at(want, shifted, f.reshape(-1, 3)); np.add.at(want, receivers, -f.reshape(-1, 3))
+    assert np.abs(eng.reduce_forces(N, shifted) - want).max() <= bound
+    eng.compute_node_energies_forces(*args)
+    assert np.array_equal(eng.H1_adj, h) and np.array_equal(eng.node_forces, f) and np.array_equal(eng.reduce_forces(N, senders), F)
+    eng.set_staging_limit(int(degree.max()) * K * (1 if L_max == 0 else 4) * 8)
+    eng.compute_node_energies_forces(*args)
+    assert np.array_equal(eng.H1_adj, h) and np.array_equal(eng.node_forces, f)
+
+
 @pytest.mark.parametrize("dtype", ["float64", "float32"])
 @pytest.mark.parametrize("K,L_max,receivers,max_degree,terms", [
     # degrees on both sides of the chunks of 16 and 17 edges and of the two and four parts a receiver is split into
