@@ -1789,6 +1789,7 @@ struct NeighborList {
     int N = 0, num_shifts = 0;
     long E = 0, num_candidates = 0;
     double r_list = 0.0;
+    double density = 0.0;          // atoms and images considered by the last build, per volume
 
     static constexpr size_t BRING_BYTES = (size_t)64 << 10;    // inputs brought by a kernel
 
@@ -1856,6 +1857,25 @@ struct NeighborList {
         }
         for (int k = 0; k < 3; ++k)
             if (!(lo[k] <= hi[k]) || !(hi[k] - lo[k] < 1e300)) throw Error(SMX_EINVAL, "neighbour list: positions are not finite");
+    }
+
+    double image_density(const NlGrid& g, const double* h_shift_vec) const
+    {
+        double volume = 1.0;
+        for (int k = 0; k < 3; ++k) {
+            double lo = 0.0, hi = 0.0;
+            for (int q = 0; q < num_shifts; ++q) { lo = std::min(lo, h_shift_vec[3 * q + k]); hi = std::max(hi, h_shift_vec[3 * q + k]); }
+            volume *= g.hi[k] - g.lo[k] + hi - lo;
+        }
+        return volume > 0.0 ? (double)N * num_shifts / volume : 0.0;
+    }
+    // Pairs to make room for when an object has none: as many as a homogeneous system of this density has within r, between 64
+    // and 256 per atom (an eighth is added where the memory is taken).  Too little costs a second search: 64 for all, as this
+    // was, were too few for an fcc alloy at 6 A (78) and for water at 5 A with a skin of 0.6 A (73).
+    size_t first_room(double r) const
+    {
+        const double pairs = 4.0 / 3.0 * 3.14159265358979 * r * r * r * density;
+        return (size_t)N * (size_t)std::min(std::max(pairs, 64.0), 256.0);
     }
 
     NlChain next_chain(hipStream_t s)
@@ -1940,8 +1960,9 @@ struct NeighborList {
         const int* ba = all ? nullptr : bin_atoms.p;
         const bool direct = r_list == r_cut;   // no skin: the candidates are the edges
         const bool chained = N <= NL_CHAIN_ATOMS;
-        if (sorted.cap == 0) { keys.size_to((size_t)64 * N, s); sorted.size_to((size_t)64 * N, s); }
-        if (edge_capacity() == 0) edge_room((size_t)64 * N, s);
+        density = image_density(g, h_shift_vec);
+        if (sorted.cap == 0) { keys.size_to(first_room(r_list), s); sorted.size_to(first_room(r_list), s); }
+        if (edge_capacity() == 0) edge_room(first_room(r_cut), s);
         if (!chained) {
             count.size_to((size_t)N, s);
             HIPCHK(launch_nl_search(false, d_pos, N, g, bs, ba, num_shifts, shift_vec, zero_shift, r_list, count.p, nullptr, 0,
@@ -1978,7 +1999,7 @@ struct NeighborList {
     // edges: the candidates closer than r_cut at the given positions, in candidate order (`room`: what the candidate arrays hold)
     long filter(const double* d_pos, const int* d_types, double r_cut, long room, hipStream_t s)
     {
-        if (edge_capacity() == 0) edge_room((size_t)64 * N, s);
+        if (edge_capacity() == 0) edge_room(first_room(r_cut), s);
         const bool chained = N <= NL_CHAIN_ATOMS;
         if (!chained) {
             totals.room(2);

@@ -878,6 +878,8 @@ def test_list_blocks_that_stop_waiting_count_for_themselves(atoms):
     rc = 5.5 if atoms == 513 else 3.3
     cell = np.full(3, (atoms * 8.0) ** (1.0 / 3.0))
     pos = rng.uniform(0, 1, size=(atoms, 3)) * cell
+    if atoms == 513:
+        pos[:300] *= 0.5        # more pairs than a homogeneous system has
     types = rng.integers(0, 3, size=atoms).astype(np.int32)
     nl = neighbors.DeviceNeighborList()
     for rounds, wait, skin in ((0, True, 0.0), (0, True, 0.4), (0, False, 0.0), (1, True, 0.4), (4096, True, 0.4)):
