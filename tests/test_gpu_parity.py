@@ -946,6 +946,92 @@ def test_senders_with_many_edges(gpu, tmp_models, L_max, K, edge):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("K,receivers,max_degree", [(20, 40, 50), (64, 12, 40), (65, 24, 35), (130, 24, 35), (16, 515, 9), (16, 3100, 4)])
+def test_scalar_features_with_a_coupling_that_mixes_harmonics(gpu, tmp_models, K, receivers, max_degree, dtype):
+    """Scalar hidden features whose layer-1 coupling is not diagonal (an output lm is fed by a second harmonic of its l): the
+    general edge kernels for scalar features, with one and two channels per lane and several channel groups, one, two and four
+    wavefronts per receiver.  The same messages where the adjoint takes the receivers in chunks."""
+    model = H.tiny_model(K=K, L_max=0, n_pts=24, seed=K, pair=K != 64)
+    q = dict(zip(model["Phi1_lme"], model["Phi1_lelm1lm2"]))
+    assert len(q) == len(model["Phi1_lme"]) == 16            # diagonal so far
+    for lm, other, c in ((1, 3, 0.4), (4, 8, -0.7), (8, 5, 0.2), (9, 15, 0.9), (12, 11, -0.3)):
+        model["Phi1_lme"].append(lm); model["Phi1_lelm1lm2"].append(q[other]); model["Phi1_clebsch_gordan"].append(c)
+    rng = np.random.default_rng(receivers)
+    degree = np.linspace(0, max_degree, receivers).astype(int) if max_degree > receivers else np.arange(receivers) % (max_degree + 1)
+    E = int(degree.sum())
+    species = rng.integers(0, 3, size=receivers).astype(np.int32)
+    senders = rng.integers(0, receivers, size=E).astype(np.int32)
+    x = rng.normal(size=(E, 3))
+    x *= (rng.uniform(0.8, 3.9, size=E) / np.linalg.norm(x, axis=1))[:, None]
+    args = (receivers, species, degree.astype(np.int32), senders, species[senders], x.ravel(), np.linalg.norm(x, axis=1))
+    orc = _oracle()(model)
+    eng = gpu(H.write_model(model, tmp_models / f"mixed_{K}.json"), dtype)
+    print(f"case K={K} receivers={receivers} edges={E} {dtype}", flush=True)
+    orc.compute_node_energies_forces(*args)
+    eng.compute_node_energies_forces(*args)
+    for name in ("Phi1", "A1", "M1", "H2", "Phi1_adj", "H1_adj", "A0_adj"):
+        a, b = np.asarray(getattr(orc, name)), np.asarray(getattr(eng, name))
+        assert np.abs(a - b).max(initial=0.0) <= TOL[dtype]["inter"] * 10 * max(1.0, np.abs(a).max()), name
+    scale = max(1.0, np.abs(orc.node_forces).max())
+    assert np.abs(orc.node_energies - eng.node_energies).max() <= TOL[dtype]["E"] * 10 * max(1.0, np.abs(orc.node_energies).max())
+    assert np.abs(orc.node_forces - eng.node_forces).max() <= TOL[dtype]["F"] * scale
+    # in chunks: the same sums of messages bit for bit.  (The forces go on from the linear behind them, which is a launch of its
+    # own then; for some channel counts the other one forms it in double, in one launch with the sums: the oracle's tolerance.)
+    h = eng.H1_adj
+    eng.set_staging_limit(max(int(degree.max()), E // 3) * K * (8 if dtype == "float64" else 4))
+    eng.compute_node_energies_forces(*args)
+    assert np.array_equal(eng.H1_adj, h)
+    assert np.abs(orc.node_forces - eng.node_forces).max() <= TOL[dtype]["F"] * scale
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("L_max,zbl,density", [(0, False, False), (1, False, False), (0, True, True)])
+def test_arrays_that_an_evaluation_does_not_form(gpu, tmp_models, L_max, zbl, density, dtype):
+    """From 1 024 atoms on the A-basis and its adjoint stay in registers (without density normalisation) and are formed when
+    somebody asks: alone, in either order, after a stage call, with ghost nodes, and after an evaluation of fewer atoms whose
+    arrays are all written (600: the linears of the other kernel, 100: none of them)."""
+    from symmetrix_amd import neighbors
+    model = H.tiny_model(K=32, L_max=L_max, n_pts=32, seed=60 + L_max, r_cut=3.0, pair=False, zbl=zbl, density=density)
+    path = H.write_model(model, tmp_models / f"asked_{L_max}{int(zbl)}.json")
+    runs = {}
+    for n in (1100, 600, 100):
+        pos, cell, sp = H.small_system(n, density=0.06, seed=n)
+        nl, ea = H.edges_of(pos, cell, sp, model["r_cut"])
+        orc = _oracle()(model)
+        orc.compute_node_energies_forces(*H.call_args(ea))
+        runs[n] = (nl, ea, sp, orc)
+    eng = gpu(path, dtype)
+
+    def same(names, orc, rows=None):
+        for name in names:
+            a, b = np.asarray(getattr(orc, name)), np.asarray(getattr(eng, name))
+            if rows is not None:
+                a, b = a.reshape(rows, -1), b.reshape(-1, a.size // rows)[:rows]
+            assert a.shape == b.shape, name
+            assert np.abs(a - b).max() <= TOL[dtype]["inter"] * 10 * max(1.0, np.abs(a).max()), name
+
+    for n, names in ((1100, ("A0", "A1", "A0_adj", "A1_adj")), (1100, ("A1_adj", "A0_adj", "A1", "A0", "M0_grad", "M1_grad")),
+                     (600, ("A0_adj", "A0", "A1_adj", "A1")), (1100, ("A0_adj",)), (100, ("A1", "A0")), (1100, ("A1",))):
+        print(f"{n} atoms, L_max {L_max}, {dtype}: {' '.join(names)}", flush=True)
+        nl, ea, sp, orc = runs[n]
+        eng.compute_node_energies_forces(*H.call_args(ea))
+        same(names, orc)
+    # a stage call forms what is left before it does anything else
+    nl, ea, sp, orc = runs[1100]
+    eng.compute_node_energies_forces(*H.call_args(ea))
+    eng.reverse_M1(ea["num_nodes"], ea["node_types"])
+    same(("A1", "A0"), orc)
+    # ghost nodes: layer 0 covers them, layer 1 does not
+    ga = neighbors.ghost_edge_arrays(nl, sp)
+    eng.compute_ghosted(ga["num_local_nodes"], ga["num_ghost_nodes"], ga["node_types"], ga["num_neigh"], ga["neigh_indices"],
+                        ga["neigh_types"], ga["xyz"], ga["r"])
+    same(("A1", "A1_adj"), orc)
+    same(("A0",), orc, rows=len(sp))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("L_max,K", [(0, 32), (1, 8)])
 @pytest.mark.parametrize("n", [255, 256, 257, 512, 513, 1024, 1025, 2100])
 def test_buckets_on_both_sides_of_the_lds(gpu, tmp_models, n, L_max, K):
