@@ -187,7 +187,8 @@ int smx_set_staging_limit(smx_model* m, long bytes);
 
 /* Per-stage timing with HIP events on the stream the kernels run on.  When
  * enabled, every stage of the next compute is bracketed by events;
- * smx_get_stage_times synchronises and returns elapsed milliseconds per stage.
+ * smx_get_stage_times synchronises and returns elapsed milliseconds per stage, zero for a stage that had no launch
+ * of its own (another stage's launch did its work).
  * Stage names come back as a ';'-separated list from smx_stage_names. */
 int smx_set_profiling(smx_model* m, int enabled);
 const char* smx_stage_names(void);

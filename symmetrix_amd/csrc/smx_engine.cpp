@@ -226,6 +226,8 @@ struct EngineBase {
         HIPCHK(hipEventRecord(ev1[st], stream));
         ev_used[st] = true;
     }
+    // a stage without a launch of its own: another one's does its work, or there is none
+    void stage_absent(int st) { ev_used[st] = false; }
 };
 
 template <typename F>
@@ -1156,12 +1158,11 @@ struct Engine : EngineBase {
                                            (c == 0 && zero_H1_adj) ? 1 : 0, true, fe[c], fe[c + 1], stream));
         }
         stage_end(ST_AGG1B);
+        stage_absent(ST_SRED);
+        if (groups == 1) { stage_absent(ST_FSUM1); return; }
         stage_begin(ST_FSUM1);
-        if (groups > 1)
-            HIPCHK(launch_fpart_reduce(E1, E, groups, fpart.p, node_forces.p, zero_dxyz ? 0 : 1, nullptr, stream, guard_live()));
+        HIPCHK(launch_fpart_reduce(E1, E, groups, fpart.p, node_forces.p, zero_dxyz ? 0 : 1, nullptr, stream, guard_live()));
         stage_end(ST_FSUM1);
-        stage_begin(ST_SRED);
-        stage_end(ST_SRED);
     }
     void st_agg0_bwd(int N)
     {
@@ -1187,11 +1188,10 @@ struct Engine : EngineBase {
         stage_begin(st_kernel);
         HIPCHK(agg_bwd(layer, p));
         stage_end(st_kernel);
+        if (groups == 1) { stage_absent(st_sum); return; }
         stage_begin(st_sum);
-        if (groups > 1) {
-            HIPCHK(launch_fpart_reduce(edges, E, groups, fpart.p, node_forces.p, p.accumulate_forces, copy, stream, guard_live()));
-            if (copy) forces_copy = nullptr;
-        }
+        HIPCHK(launch_fpart_reduce(edges, E, groups, fpart.p, node_forces.p, p.accumulate_forces, copy, stream, guard_live()));
+        if (copy) forces_copy = nullptr;
         stage_end(st_sum);
     }
 
@@ -1297,7 +1297,7 @@ struct Engine : EngineBase {
         pending_M0_grad = recompute_M0_grad() ? N : -1;
         if (fused_contraction(0, N)) {
             stage_begin(ST_A0LIN); st_linear_contraction(0, N); stage_end(ST_A0LIN);
-            stage_begin(ST_M0); stage_end(ST_M0);
+            stage_absent(ST_M0);
         } else {
             stage_begin(ST_A0LIN); st_A0_lin(N, false); stage_end(ST_A0LIN);
             st_scale(0, N, false);
@@ -1312,7 +1312,7 @@ struct Engine : EngineBase {
         stage_begin(ST_AGG1F); st_agg1_fwd(N1); stage_end(ST_AGG1F);
         if (fused_contraction(1, N1)) {
             stage_begin(ST_A1); st_linear_contraction(1, N1); stage_end(ST_A1);
-            stage_begin(ST_M1); stage_end(ST_M1);
+            stage_absent(ST_M1);
         } else {
             stage_begin(ST_A1); st_A1(N1, false); stage_end(ST_A1);
             st_scale(1, N1, false);
@@ -1320,8 +1320,7 @@ struct Engine : EngineBase {
         }
         if (tail_fused_ok(K())) {
             stage_begin(ST_H2); st_tail(N1, !hm.has_zbl); stage_end(ST_H2);
-            stage_begin(ST_READOUT); stage_end(ST_READOUT);
-            stage_begin(ST_REVH2); stage_end(ST_REVH2);
+            stage_absent(ST_READOUT); stage_absent(ST_REVH2);
         } else {
             stage_begin(ST_H2); st_H2(N1); stage_end(ST_H2);
             stage_begin(ST_READOUT); st_readouts(N1, !hm.has_zbl); stage_end(ST_READOUT);
@@ -1332,7 +1331,8 @@ struct Engine : EngineBase {
         // A_adj is only written if somebody asks for it (get_array).
         const bool scaled_operand = use_linear(N) || gemm_scaled_operand_ok(K(), K(), sizeof(F));
         const bool fuse1 = !hm.A1_scaled && scaled_operand, fuse0 = !hm.A0_scaled && NLM() == 1 && scaled_operand;
-        stage_begin(ST_REVM1); if (!fuse1) st_reverse_M1(N1); stage_end(ST_REVM1);
+        if (fuse1) stage_absent(ST_REVM1);
+        else { stage_begin(ST_REVM1); st_reverse_M1(N1); stage_end(ST_REVM1); }
         pending_A1_adj = fuse1 ? N1 : -1;
         st_scale(1, N1, true);
         stage_begin(ST_REVA1); st_A1(N1, true, fuse1); stage_end(ST_REVA1);
@@ -1340,8 +1340,10 @@ struct Engine : EngineBase {
         st_agg1_bwd(N1, !early_forces, false);
         fuse_reverse_H1 = false;
         if (N1 < N) node_lists_for(N);
-        stage_begin(ST_REVH1); if (!reverse_H1_done) st_H1(N, true); stage_end(ST_REVH1);
-        stage_begin(ST_REVM0); if (!fuse0) st_reverse_M0(N); stage_end(ST_REVM0);
+        if (reverse_H1_done) stage_absent(ST_REVH1);
+        else { stage_begin(ST_REVH1); st_H1(N, true); stage_end(ST_REVH1); }
+        if (fuse0) stage_absent(ST_REVM0);
+        else { stage_begin(ST_REVM0); st_reverse_M0(N); stage_end(ST_REVM0); }
         pending_A0_adj = fuse0 ? N : -1;
         st_scale(0, N, true);
         stage_begin(ST_REVA0LIN); st_A0_lin(N, true, fuse0); stage_end(ST_REVA0LIN);

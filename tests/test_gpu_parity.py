@@ -1032,6 +1032,26 @@ def test_arrays_that_an_evaluation_does_not_form(gpu, tmp_models, L_max, zbl, de
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("L_max", [0, 1])
+def test_stages_without_a_launch_of_their_own_have_no_time(gpu, tmp_models, L_max):
+    """Whether a contraction ran inside its linear is told by the engine, not by how short its stage was."""
+    model = H.tiny_model(K=32, L_max=L_max, n_pts=32, seed=60 + L_max, r_cut=3.0, pair=False)
+    eng = gpu(H.write_model(model, tmp_models / f"stages_{L_max}.json"))
+    eng.set_profiling(True)
+    for n in (1100, 24, 1100):
+        pos, cell, sp = H.small_system(n, density=0.06, seed=n)
+        nl, ea = H.edges_of(pos, cell, sp, model["r_cut"])
+        eng.compute_node_energies_forces(*H.call_args(ea))
+        t = eng.stage_times()
+        print(f"{n} atoms: {t}", flush=True)
+        absent = {"readout", "rev_H2", "rev_M1", "force_sum0", "force_sum1"}
+        absent |= {"M1"} if n >= 1024 else set()
+        absent |= {"rev_H1", "rev_M0"} | ({"M0"} if n >= 1024 else set()) if L_max == 0 else set()
+        assert {k for k, v in t.items() if v == 0.0} == absent
+        assert all(v >= 0.0 for v in t.values())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("L_max,K", [(0, 32), (1, 8)])
 @pytest.mark.parametrize("n", [255, 256, 257, 512, 513, 1024, 1025, 2100])
 def test_buckets_on_both_sides_of_the_lds(gpu, tmp_models, n, L_max, K):
