@@ -216,65 +216,61 @@ __device__ __forceinline__ int count_below(const int* buf, int n, int v)
     }
     return rank;
 }
-// how many of the CAP ascending entries of `run` are below v
-template <int CAP>
-__device__ __forceinline__ int count_below_sorted(const int* run, int v)
+// The n distinct entries list[s0 ..] in ascending order in place, by the wavefront that calls: runs of RUN entries first, each
+// ordered in `buf` (LDS, RUN entries of this wavefront, 16-byte aligned) and left in spare[s0 ..], which nobody else uses; then
+// every entry is looked up in all other runs.  (RUN and not what the LDS holds: four entries per lane in registers.)
+constexpr int SORT_RUN = 256;
+__device__ __forceinline__ void wave_sort_in_memory(int* list, int s0, int n, int* buf, int lane, int* spare)
 {
-    int at = 0;
+    constexpr int RUN = SORT_RUN, PER = RUN / 64, none = 0x7fffffff;
+    auto to_lds = [&](const int* from, int c0) {
+        wave_lds_sync();
 #pragma unroll
-    for (int half = CAP / 2; half >= 1; half /= 2) at += run[at + half - 1] < v ? half : 0;
-    return at + (run[at] < v);
+        for (int q = 0; q < PER; ++q) buf[64 * q + lane] = c0 + 64 * q + lane < n ? from[s0 + c0 + 64 * q + lane] : none;
+        wave_lds_sync();
+    };
+    for (int c0 = 0; c0 < n; c0 += RUN) {
+        to_lds(list, c0);
+        for (int t = lane; t < min(RUN, n - c0); t += 64) {
+            const int v = buf[t];
+            spare[s0 + c0 + count_below(buf, min(RUN, n - c0), v)] = v;
+        }
+    }
+    __threadfence();
+    for (int v0 = 0; v0 < n; v0 += RUN) {
+        int v[PER], rank[PER];
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            v[q] = v0 + 64 * q + lane < n ? spare[s0 + v0 + 64 * q + lane] : none;
+            rank[q] = 64 * q + lane;
+        }
+        for (int c0 = 0; c0 < n; c0 += RUN) {
+            if (c0 == v0) continue;
+            to_lds(spare, c0);
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                int at = 0;
+                for (int half = RUN / 2; half >= 1; half /= 2) at += buf[at + half - 1] < v[q] ? half : 0;
+                rank[q] += at + (buf[at] < v[q]);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            if (v0 + 64 * q + lane < n) list[s0 + rank[q]] = v[q];
+    }
+    __threadfence();
 }
 // The n distinct entries list[s0 ..] in ascending order, for the wavefront that calls: in `buf` (LDS, CAP entries of this
-// wavefront, 16-byte aligned; the rank of an entry is the number of smaller ones).  A longer bucket is put in order in memory:
-// runs of CAP entries first, to spare[s0 ..] (which nobody else uses), then every entry is looked up in all runs.  Sums of the
-// messages of 400 senders with 260, 476 and 786 edges each (32 channels): 121, 200 and 317 us, by a lane that sorts in place
-// 3.5, 11 and 21 ms.  A launch that puts all buckets in order beforehand, a wavefront each: 84, 143 and 226 us, but 30, 75 and
-// 195 us itself.
+// wavefront, 16-byte aligned; the rank of an entry is the number of smaller ones), or, for a longer bucket, in memory.
+// Sums of the messages of 400 senders with 260, 476 and 786 edges each (32 channels): 119, 195 and 325 us, by a lane that
+// sorts in place 3.3, 11 and 21 ms.  (A launch that puts all buckets in order beforehand, a wavefront each: 84, 143 and 226 us,
+// but 30, 75 and 195 us itself.)
 template <int CAP>
 __device__ __forceinline__ const int* wave_sorted_bucket(int* list, int s0, int n, int* buf, int lane, int* spare)
 {
-    static_assert(CAP % 64 == 0 && (CAP & (CAP - 1)) == 0, "whole rounds of a wavefront, and halves");
+    static_assert(CAP % 64 == 0 && CAP >= SORT_RUN, "whole rounds of a wavefront, and room for a run");
     if (n > CAP) {
-        constexpr int none = 0x7fffffff;
-        auto to_lds = [&](const int* from, int c0, int (&v)[CAP / 64]) {
-            wave_lds_sync();
-#pragma unroll
-            for (int q = 0; q < CAP / 64; ++q) {
-                const int t = c0 + 64 * q + lane;
-                v[q] = t < n ? from[s0 + t] : none;
-                buf[64 * q + lane] = v[q];
-            }
-            wave_lds_sync();
-        };
-        int v[CAP / 64], other[CAP / 64];
-        for (int c0 = 0; c0 < n; c0 += CAP) {
-            to_lds(list, c0, v);
-#pragma unroll
-            for (int q = 0; q < CAP / 64; ++q) {
-                const int rank = count_below(buf, min(CAP, n - c0), v[q]);
-                if (c0 + 64 * q + lane < n) spare[s0 + c0 + rank] = v[q];
-            }
-        }
-        __threadfence();
-        for (int v0 = 0; v0 < n; v0 += CAP) {
-            int rank[CAP / 64];
-#pragma unroll
-            for (int q = 0; q < CAP / 64; ++q) {
-                v[q] = v0 + 64 * q + lane < n ? spare[s0 + v0 + 64 * q + lane] : none;
-                rank[q] = 64 * q + lane;
-            }
-            for (int c0 = 0; c0 < n; c0 += CAP) {
-                if (c0 == v0) continue;
-                to_lds(spare, c0, other);
-#pragma unroll
-                for (int q = 0; q < CAP / 64; ++q) rank[q] += count_below_sorted<CAP>(buf, v[q]);
-            }
-#pragma unroll
-            for (int q = 0; q < CAP / 64; ++q)
-                if (v0 + 64 * q + lane < n) list[s0 + rank[q]] = v[q];
-        }
-        __threadfence();
+        wave_sort_in_memory(list, s0, n, buf, lane, spare);
         return list + s0;
     }
     int v[CAP / 64];

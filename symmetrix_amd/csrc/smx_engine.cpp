@@ -1554,7 +1554,7 @@ struct Engine : EngineBase {
     {
         v->node_forces = has_forces() ? node_forces.p : nullptr; v->forces_len = (long)node_forces.n; v->xyz = xyz;
         v->first_neigh = first_neigh.p; v->skipped = skipped_word();
-        v->num_edges = E; v->num_receivers = N_geo; v->device = device;
+        v->num_edges = E; v->receiver_edges = geo_edges; v->num_receivers = N_geo; v->device = device;
     }
     // size a named array to n entries, all equal to `value`, without a host copy
     void fill_array(const char* name, long n, double value) override
@@ -1590,8 +1590,9 @@ struct Engine : EngineBase {
         if (node_forces.n != (size_t)3 * E) throw Error(SMX_EINVAL, "node_forces does not match the current edge list");
         if (!atom_forces && !virial) return;
         if (virial && E > 0) need(xyz, "xyz");
+        if (geo_edges > E) throw Error(SMX_EINVAL, "num_neigh of the last call covers more edges than there are");
         ForceGather g{};
-        g.num_nodes = N_geo; g.first_neigh = first_neigh.p; g.num_edges = E; g.forces = node_forces.p; g.xyz = xyz;
+        g.num_nodes = N_geo; g.first_neigh = first_neigh.p; g.node_edges = geo_edges; g.num_edges = E; g.forces = node_forces.p; g.xyz = xyz;
         g.skipped = skipped_word();
         int atoms = N_geo;
         if (atom_forces) {
@@ -1690,7 +1691,7 @@ struct Engine : EngineBase {
         double* out = reduction_room((size_t)4 * N);
         compute(N, nt, nn, ni, nty, x, rr, E_, true, out + RF_HEAD + (size_t)3 * N, nullptr, -1, -1);
         ForceGather g{};
-        g.num_nodes = N; g.first_neigh = first_neigh.p; g.num_edges = E; g.forces = node_forces.p; g.xyz = xyz;
+        g.num_nodes = N; g.first_neigh = first_neigh.p; g.node_edges = geo_edges; g.num_edges = E; g.forces = node_forces.p; g.xyz = xyz;
         g.skipped = skipped_word();
         g.send_start = s_start.p; g.send_list = s_list.p; g.send_spare = s_rank.p;
         g.atom_forces = out + RF_HEAD;

@@ -14,6 +14,7 @@ struct ForcesView {
     const int* first_neigh;      // [num_receivers + 1]
     const int* skipped;          // not zero: the evaluation was skipped and these arrays say nothing (null: no such word)
     long num_edges, forces_len;
+    long receiver_edges;         // of the receivers: the leading ones
     int num_receivers;
     int device;                  // ordinal of the GPU that holds the model and these arrays
 };

@@ -364,7 +364,8 @@ struct ForceGather {
     const int* node_start; const int* node_list;     // nodes whose edges count as received by the atom; null: node i is atom i
     int num_nodes;
     const int* first_neigh;                          // [num_nodes + 1], or null without nodes
-    long num_edges;                                  // those beyond the nodes' have no receiver here: sender side and virial only
+    long node_edges, num_edges;                      // edges of the nodes, all: those behind have no receiver here, but send and
+                                                     // are part of the virial
     const double* forces; const double* xyz;         // [E][3] (xyz for the virial only)
     double* atom_forces;                             // [num_atoms][3] or null
     double* partial;                                 // [force_gather_blocks][6], needed for the virial, else null

@@ -791,7 +791,7 @@ __global__ void k_sender_reduce(int rows, int width, const int* sstart, int* sli
         slist = bucket + SENDER_CAP;
         s0 = 0; s1 = n;
     } else {
-        if (threadIdx.x < 64) wave_sorted_bucket<SENDER_CAP>(slist_, s0, s1 - s0, bucket, threadIdx.x, spare);
+        if (threadIdx.x < 64) wave_sort_in_memory(slist_, s0, s1 - s0, bucket, threadIdx.x, spare);
         __syncthreads();
     }
     if (s0 == s1 && !zero_first) return;

@@ -958,12 +958,14 @@ __device__ __forceinline__ void add_virial(double (&v)[6], const double* d, cons
     v[0] += x * f[0]; v[1] += y * f[1]; v[2] += z * f[2];
     v[3] += 0.5 * (x * f[1] + y * f[0]); v[4] += 0.5 * (x * f[2] + z * f[0]); v[5] += 0.5 * (y * f[2] + z * f[1]);
 }
+template <bool BEHIND>
 __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
 {
     __shared__ __align__(16) int bucket[4][GATHER_CAP];
     __shared__ double red[4][6];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     double v[6] = {0, 0, 0, 0, 0, 0};
+    const bool nothing = no_result(a.flag, a.skipped);     // (asked for here, needed at the end)
     for (int at = blockIdx.x * 4 + wave; at < a.num_atoms; at += gridDim.x * 4) {
         double fx = 0, fy = 0, fz = 0;
         if (a.send_start) {
@@ -989,7 +991,7 @@ __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
         }
         if (a.atom_forces) {
             fx = wave_sum(fx); fy = wave_sum(fy); fz = wave_sum(fz);
-            if (no_result(a.flag, a.skipped)) fx = fy = fz = __builtin_nan("");
+            if (nothing) fx = fy = fz = __builtin_nan("");
             if (lane < 3) a.atom_forces[3 * (size_t)at + lane] = lane == 0 ? fx : (lane == 1 ? fy : fz);
         }
         wave_lds_sync();   // the next atom's bucket overwrites this one's
@@ -997,9 +999,9 @@ __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
     if (!a.partial) return;
     // Edges behind those of the nodes (the last counts covered the leading nodes of a longer edge list): every edge is in the
     // virial.
-    for (long e = (a.first_neigh ? a.first_neigh[a.num_nodes] : 0) + (long)blockIdx.x * 256 + threadIdx.x; e < a.num_edges;
-         e += (long)gridDim.x * 256)
-        add_virial(v, a.xyz + 3 * (size_t)e, a.forces + 3 * (size_t)e);
+    if constexpr (BEHIND)
+        for (long e = a.node_edges + (long)blockIdx.x * 256 + threadIdx.x; e < a.num_edges; e += (long)gridDim.x * 256)
+            add_virial(v, a.xyz + 3 * (size_t)e, a.forces + 3 * (size_t)e);
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
         const double t = wave_sum(v[q]);
@@ -1015,10 +1017,11 @@ __global__ __launch_bounds__(384) void k_virial_finish(const double* partial, in
                                                       double* virial)
 {
     const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const bool nothing = no_result(flag, skipped);
     double v = 0.0;
     for (int b = lane; b < nblocks; b += 64) v += partial[(size_t)b * 6 + q];
     v = wave_sum(v);
-    if (lane == 0) virial[q] = no_result(flag, skipped) ? __builtin_nan("") : v;
+    if (lane == 0) virial[q] = nothing ? __builtin_nan("") : v;
 }
 }  // namespace
 
@@ -1026,7 +1029,8 @@ int force_gather_blocks(int num_atoms) { return std::min(std::max((num_atoms + 3
 hipError_t launch_force_gather(const ForceGather& g, double* virial, hipStream_t s)
 {
     const int nb = force_gather_blocks(g.num_atoms);
-    hipLaunchKernelGGL(k_force_gather, dim3(nb), dim3(256), 0, s, g);
+    if (g.num_edges > g.node_edges) hipLaunchKernelGGL(k_force_gather<true>, dim3(nb), dim3(256), 0, s, g);
+    else hipLaunchKernelGGL(k_force_gather<false>, dim3(nb), dim3(256), 0, s, g);
     if (virial) hipLaunchKernelGGL(k_virial_finish, dim3(1), dim3(384), 0, s, g.partial, nb, g.flag, g.skipped, virial);
     return hipGetLastError();
 }

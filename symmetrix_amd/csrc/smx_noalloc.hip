@@ -80,7 +80,7 @@ extern "C" int smx_reduce_forces_device_noalloc(smx_model* m, int num_atoms, con
         smx::set_last_error("num_atoms is smaller than the number of receivers");
         return SMX_EINVAL;
     }
-    if (!v.node_forces || v.forces_len != 3 * v.num_edges) {
+    if (!v.node_forces || v.forces_len != 3 * v.num_edges || v.receiver_edges > v.num_edges) {
         smx::set_last_error("node_forces does not match the current edge list");
         return SMX_EINVAL;
     }
@@ -111,7 +111,7 @@ extern "C" int smx_reduce_forces_device_noalloc(smx_model* m, int num_atoms, con
     // are NaN instead
     hipError_t e = smx::launch_fill<int>(flag, 1, 0, s);
     smx::ForceGather g{};
-    g.num_atoms = num_atoms; g.num_nodes = v.num_receivers; g.first_neigh = v.first_neigh; g.num_edges = E;
+    g.num_atoms = num_atoms; g.num_nodes = v.num_receivers; g.first_neigh = v.first_neigh; g.node_edges = v.receiver_edges; g.num_edges = E;
     g.forces = v.node_forces; g.xyz = v.xyz; g.atom_forces = d_atom_forces; g.flag = flag; g.skipped = v.skipped;
     if (d_virial) g.partial = partial;
     if (d_atom_forces) {
