@@ -106,7 +106,7 @@ __device__ __forceinline__ void sph_l3_grad(double x, double y, double z, double
 
 // 1/sqrt(a) and 1/a for positive normal a: hardware estimate (about 23 bits) and two Newton steps, good to
 // the last bit or two.  The library forms (sqrt then divide, IEEE divide) cost four to five times as many
-// instructions, and the edge kernels evaluate them per (edge, channel slice).
+// instructions, and the edge kernels evaluate them for every edge.
 __device__ __forceinline__ double rsqrt_pos(double a)
 {
     double y = __builtin_amdgcn_rsq(a);

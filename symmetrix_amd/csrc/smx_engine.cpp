@@ -1252,7 +1252,7 @@ struct Engine : EngineBase {
         guard_status = flags.p + 2; guard_clear_enqueued = false; guard_on_device = on_device;
         if (!on_device && (hm.A0_scaled || hm.A1_scaled)) HIPCHK(launch_fill<int>(flags.p, 1, 0, stream));
         if (N <= 65536) {
-            // one launch for first_neigh, degree order, species groups, the sender histogram and the sender offsets
+            // one launch for first_neigh, species groups, the sender histogram and the sender offsets
             hipStream_t s = stream;
             first_neigh.size_to((size_t)N + 1, s);
             t_start.size_to((size_t)hm.T + 1, s); t_perm.size_to((size_t)N, s);
@@ -1304,11 +1304,8 @@ struct Engine : EngineBase {
             stage_begin(ST_M0); st_poly(N, false, pending_M0_grad >= 0 ? 1 : 0); stage_end(ST_M0);
         }
         stage_begin(ST_H1); st_H1(N, false); stage_end(ST_H1);
-        // per-species node groups and the degree order of the receivers cover the nodes of the current stages
-        auto node_lists_for = [&](int n) {
-            build_type_groups(n);
-        };
-        if (N1 < N) node_lists_for(N1);
+        // the species groups cover the nodes of the current stages
+        if (N1 < N) build_type_groups(N1);
         stage_begin(ST_AGG1F); st_agg1_fwd(N1); stage_end(ST_AGG1F);
         if (fused_contraction(1, N1)) {
             stage_begin(ST_A1); st_linear_contraction(1, N1); stage_end(ST_A1);
@@ -1339,7 +1336,7 @@ struct Engine : EngineBase {
         fuse_reverse_H1 = N1 == N; reverse_H1_done = false;
         st_agg1_bwd(N1, !early_forces, false);
         fuse_reverse_H1 = false;
-        if (N1 < N) node_lists_for(N);
+        if (N1 < N) build_type_groups(N);
         if (reverse_H1_done) stage_absent(ST_REVH1);
         else { stage_begin(ST_REVH1); st_H1(N, true); stage_end(ST_REVH1); }
         if (fuse0) stage_absent(ST_REVM0);

@@ -35,8 +35,7 @@ def _model_file(tmp_models, name, **override):
 @pytest.mark.parametrize("pair", [False, True], ids=["one_table", "pair_tables"])
 def test_tiny_configuration_at_full_size_against_the_oracle(gpu, tmp_models, pair, dtype):
     """192 atoms H/C/O at 0.10 atoms/A^3, K = 32, r_cut 5.0 A, 256 spline points: the configuration the reference
-    CPU path runs.  With one radial table (plain MACE) the channel-slice kernels serve both layers, with six pair
-    tables the general ones do."""
+    CPU path runs, with one radial table (plain MACE) and with six pair tables."""
     from oracle.oracle import OracleMACE
     from symmetrix_amd import neighbors, systems
     path, cfg = _model_file(tmp_models, "tiny", pair_dependent_radial=pair)

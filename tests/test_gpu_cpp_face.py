@@ -35,8 +35,7 @@ def _case(f, mode, Nl, Ng, rows, nt, nn, node_i, ni, nty, nj, halo_ghost, halo_o
                                                             (1, "float32", False, True), (0, "float64", True, False),
                                                             (0, "float32", True, True)])
 def test_cpp_caller_runs_the_three_pair_style_modes(tmp_path, L_max, dtype, one_table, density):
-    """`one_table`: one radial table for all species pairs, so that the channel-slice kernels run (the layer-1
-    partial forces wait for the layer-0 adjoint there, beside the ZBL and density-normalisation forces)."""
+    """`one_table`: one radial table for all species pairs."""
     if not os.path.exists(DRIVER):
         pytest.fail("tests/cpp/pair_modes_driver is not built: python -c 'import __graft_entry__ as g; g.build()'")
     model = H.tiny_model(K=16, L_max=L_max, n_pts=48, seed=12, pair=not one_table, zbl=True, density=density)

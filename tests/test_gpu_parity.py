@@ -54,7 +54,7 @@ CASES = [
     # K, L_max, atoms, pair-dependent radial
     (32, 0, 40, True), (32, 1, 40, True), (96, 0, 48, False), (128, 1, 36, True), (48, 1, 24, True),
     (20, 0, 17, True), (64, 1, 30, False), (128, 0, 30, True),
-    # wider than one block of channels: several channel groups, column tiles and slices
+    # wider than one block of channels: several channel groups and column tiles
     (256, 0, 20, False), (192, 1, 16, False),
     # hidden features up to l = 2 (128x0e+128x1o+128x2e and the like): 17 paths, 9 polynomials
     (16, 2, 30, True), (128, 2, 20, False), (40, 2, 26, True),
@@ -111,8 +111,7 @@ def test_monomials_outside_the_standard_basis_take_the_general_kernel(gpu, tmp_m
 @pytest.mark.parametrize("dtype", ["float64", "float32"])
 @pytest.mark.parametrize("K,natoms", [(20, 70), (96, 200), (33, 9)])
 def test_two_species_three_radial_tables(gpu, tmp_models, K, natoms, dtype):
-    """Scalar hidden features with a few distinct pair tables: the general edge kernels
-    (the channel-slice kernels hold one table)."""
+    """Scalar hidden features with a few distinct pair tables: the scalar edge kernels choose the table per edge."""
     model = H.tiny_model(K=K, L_max=0, T=(1, 8), n_pts=50, seed=K, pair=True)
     path = H.write_model(model, tmp_models / f"two_{K}.json")
     orc = _oracle()(model)
@@ -127,9 +126,8 @@ def test_two_species_three_radial_tables(gpu, tmp_models, K, natoms, dtype):
 
 @pytest.mark.parametrize("dtype", ["float64", "float32"])
 @pytest.mark.parametrize("K,natoms", [(24, 60), (7, 33)])
-def test_long_spline_tables_take_the_narrow_slice_kernels(gpu, tmp_models, K, natoms, dtype):
-    """One radial table with 400 nodes: a slice of 32 bytes of channels no longer fits the LDS, so the slices
-    are half as wide and the four-lanes-per-edge kernels of both directions run instead of the 32-byte ones."""
+def test_long_spline_tables(gpu, tmp_models, K, natoms, dtype):
+    """One radial table with 400 nodes (the other cases have 24 to 256)."""
     model = H.tiny_model(K=K, L_max=0, n_pts=400, seed=K, pair=False)
     path = H.write_model(model, tmp_models / f"long_{K}.json")
     orc = _oracle()(model)
@@ -147,18 +145,16 @@ def test_long_spline_tables_take_the_narrow_slice_kernels(gpu, tmp_models, K, na
 
 @pytest.mark.parametrize("dtype", ["float64", "float32"])
 @pytest.mark.parametrize("K,natoms", [(6, 41), (7, 33), (20, 52)])
-def test_channel_counts_that_leave_the_last_slice_incomplete(gpu, tmp_models, K, natoms, dtype):
-    """One radial table that fits the LDS in 32-byte slices (4 doubles or 8 floats of channels), scalar hidden
-    features, and a channel count that is no multiple of the slice: the last slice of the 32-byte kernels of both
-    directions has channels missing (K = 20 only in single precision), which they handle by element-wise loads and
-    stores compiled apart from the whole-slice code."""
+def test_channel_counts_that_leave_lanes_idle(gpu, tmp_models, K, natoms, dtype):
+    """Scalar hidden features and a channel count below the 32 lanes that an edge has: lanes beyond the last channel work
+    on another one with a zero adjoint, add nothing to the sums and store nothing."""
     model = H.tiny_model(K=K, L_max=0, n_pts=64, seed=100 + K, pair=False)
     path = H.write_model(model, tmp_models / f"partial_{K}.json")
     orc = _oracle()(model)
     eng = gpu(path, dtype)
     pos, cell, sp = H.small_system(natoms, seed=natoms)
     nl, ea = H.edges_of(pos, cell, sp, model["r_cut"])
-    print(f"case K={K} atoms={natoms} edges={len(ea['r'])} {dtype} incomplete last slice", flush=True)
+    print(f"case K={K} atoms={natoms} edges={len(ea['r'])} {dtype} idle lanes", flush=True)
     orc.compute_node_energies_forces(*H.call_args(ea))
     eng.compute_node_energies_forces(*H.call_args(ea))
     _compare(orc, eng, dtype)
@@ -576,10 +572,8 @@ def test_receiver_chunks_of_the_layer1_adjoint_change_nothing(gpu, tmp_models, d
         eng.compute_node_energies_forces(*H.call_args(ea))
 
 
-# (L_max, dtype, one radial table for all pairs, ZBL, density normalisation).  One table and scalar hidden features
-# take the channel-slice kernels, whose layer-1 partial forces wait in the staging array for the layer-0 adjoint
-# (K = 16 is a whole number of 32-byte slices in both precisions): with ghost nodes, ZBL or the density
-# normalisation the force array has other contributions before, between and beside those two.
+# (L_max, dtype, one radial table for all pairs, ZBL, density normalisation).  With ghost nodes, ZBL or the density
+# normalisation the force array has other contributions before, between and beside those of the two adjoints.
 MODE_CASES = [(0, "float64", False, False, False), (1, "float64", False, True, True), (0, "float32", False, True, False),
               (1, "float32", False, True, True), (2, "float64", False, True, True)]
 MODE_CASES += [(0, dt, True, zbl, dens) for dt in ("float64", "float32")
@@ -743,8 +737,8 @@ def test_device_resident_call_checks_its_inputs_on_the_device(gpu, tmp_models, L
     evaluation runs on emptied lists (no unchecked integer is used as an address), node energies and edge forces come
     back as NaN and the next synchronising call (synchronize, get_array, reduce_forces) raises.  Every kernel exits
     normally; the call after is unaffected, also when both are replays of one captured graph.
-    `big`: more than 65 536 atoms, where the preparation is made of separate launches; `one_table`: the
-    channel-slice kernels, whose forces come out of the sum over slices."""
+    `big`: more than 65 536 atoms, where the preparation is made of separate launches; `one_table`: one radial table for
+    all species pairs."""
     import torch
     from symmetrix_amd import neighbors, systems
     model = H.tiny_model(K=16 if big else 32, L_max=L_max, n_pts=48, seed=40 + L_max, r_cut=3.0 if big else 4.0,
