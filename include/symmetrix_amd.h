@@ -203,7 +203,10 @@ int smx_synchronize(smx_model* m);
  * receiver i; virial[6] = sum xyz (x) f_ij in LAMMPS order xx,yy,zz,xy,xz,yz.
  * receiver_atom/sender_atom map edge ends to atom rows; NULL receiver_atom
  * means the receiver of edge block i is atom i.  Uses the forces of the last
- * compute.  Outputs are host arrays. */
+ * compute.  Outputs are host arrays.  Every edge is part of the virial, also
+ * where the last num_neigh covered the leading nodes of a longer edge list.
+ * After an evaluation of host arrays that was refused there is nothing to
+ * reduce (SMX_EINVAL); after a skipped device-resident one the sums are NaN. */
 int smx_reduce_forces(smx_model* m, int num_atoms, const int* sender_atom, const int* receiver_atom,
                       double* atom_forces, double* virial);
 /* The same with sender_atom a device array (e.g. neigh_indices of smx_nlist_arrays) and receiver i = atom i. */
