@@ -1032,6 +1032,7 @@ struct Engine : EngineBase {
     void st_readouts(int N, bool zero_energies)
     {
         const int k = K(), nlm = NLM();
+        if (N > 0) need(node_types, "node_types");
         node_energies.resize((size_t)N, stream);
         H1_adj.size_to(H1.n, stream);
         H2_adj.size_to(H2.n, stream);
@@ -1391,7 +1392,16 @@ struct Engine : EngineBase {
             build_first_neigh(N); E1 = own_edges; geo_edges = own_edges;
             if (guarded) { sender_edges = -1; guarded = false; }
         }
-        validate_stage_inputs(N, nt != nullptr, ni != nullptr, nty != nullptr, rr != nullptr);
+        try {
+            validate_stage_inputs(N, nt != nullptr, ni != nullptr, nty != nullptr, rr != nullptr);
+        } catch (...) {
+            // arrays that failed their checks are not there for the next call
+            if (nt) node_types = nullptr;
+            if (ni) neigh_indices = nullptr;
+            if (nty) neigh_types = nullptr;
+            if (rr) r = nullptr;
+            throw;
+        }
         if (s == "Y" || s == "R0" || s == "R1") return;  // geometry remembered; evaluated inside the fused kernels
         if (s == "A0") { build_type_groups(N); st_agg0_fwd(N); st_A0_lin(N, false); }
         else if (s == "reverse_A0") { build_type_groups(N); st_A0_lin(N, true); st_agg0_bwd(N); }

@@ -117,3 +117,34 @@ def test_nothing_is_reduced_after_a_refused_evaluation(tmp_models):
         assert np.array_equal(eng.node_forces, f_ref)
         F, V = eng.reduce_forces(N, ni, virial=True)
         assert np.array_equal(F, F_ref) and np.array_equal(V, V_ref)
+
+
+def test_stage_inputs_that_were_refused_are_not_used_later(tmp_models):
+    """A stage call that refuses its arrays leaves none of them behind: later stages ask for them, and go on once they have
+    been given."""
+    from symmetrix_amd.mace import MACE
+    model = H.tiny_model(K=16, L_max=1, n_pts=48, seed=23)
+    eng = MACE(H.write_model(model, tmp_models / "stage_refused.json"))
+    pos, cell, sp = H.small_system(30, seed=5)
+    nl, ea = H.edges_of(pos, cell, sp, model["r_cut"])
+    N, nt, nn, ni, nty, xyz, r = H.call_args(ea)
+
+    def through_phi1():
+        eng.compute_Y(xyz); eng.compute_R0(N, nt, nn, nty, r); eng.compute_A0(N, nt, nn, nty)
+        eng.compute_M0(N, nt); eng.compute_H1(N); eng.compute_R1(N, nt, nn, nty, r); eng.compute_Phi1(N, nn, ni)
+        return eng.Phi1
+
+    ref = through_phi1()
+    for what, bad in (("species of the nodes", (nt + 3, nn, nty, r)), ("species of the edges", (nt, nn, nty - 1, r)),
+                      ("lengths", (nt, nn, nty, r + model["r_cut"]))):
+        print(what, flush=True)
+        with pytest.raises(ValueError):
+            eng.compute_R1(N, *bad)
+        with pytest.raises(ValueError, match="before its inputs exist"):
+            eng.compute_Phi1(N, nn, ni)
+        eng.compute_R1(N, nt, nn, nty, r)
+        eng.compute_Phi1(N, nn, ni)
+        assert np.array_equal(eng.Phi1, ref)
+    with pytest.raises(ValueError):
+        eng.compute_Phi1(N, nn, ni + N)
+    assert np.array_equal(through_phi1(), ref)
