@@ -236,6 +236,8 @@ struct Engine : EngineBase {
     DVec<F> tab0, tab1, tabK0, tabK1, H0, A0w, H1w, A1w;
     DVec<F> linA0, linA0T, linA1, linA1T;    // the same weights in operand order (operand_weights)
     DVec<F> M0_coef16, M1_coef16;            // contraction coefficients by column tile
+    DVec<F> H1wT;                            // transposes, for the kernels that take a chain of stages
+    DVec<double> H2w_H1T, H2w_M1T;
     DVec<int> pair_table0, pair_table1;
     DVec<int> B0_start, B0_lm1, B1_start, B1_lm1;
     DVec<double> B0_c, B1_c;
@@ -458,9 +460,23 @@ struct Engine : EngineBase {
         if (M0_tables) slabs(M0_slabs, hm.P0.data(), hm.num_LM, false);
         if (M1_tables) slabs(M1_slabs, &hm.P1, 1, false);
         if (linear_ok(hm.K)) {
-            if (M0_tables && hm.num_LM == 1) slabs(M0_coef16, hm.P0.data(), 1, true);
+            const bool chain = chain_ok(hm.K) && M0_tables && M1_tables;
+            if (M0_tables && (hm.num_LM == 1 || chain)) slabs(M0_coef16, hm.P0.data(), hm.num_LM, true);
             if (M1_tables) slabs(M1_coef16, &hm.P1, 1, true);
             operand_weights(s);
+            if (chain) {
+                auto transposed = [&](const std::vector<double>& w, auto& dst) {
+                    const size_t Kc = hm.K, n = w.size() / (Kc * Kc);
+                    std::vector<double> out(w.size());
+                    for (size_t b = 0; b < n; ++b)
+                        for (size_t i = 0; i < Kc; ++i)
+                            for (size_t j = 0; j < Kc; ++j) out[(b * Kc + j) * Kc + i] = w[(b * Kc + i) * Kc + j];
+                    upload_as(dst, out, s);
+                };
+                transposed(hm.H1_weights, H1wT);
+                transposed(hm.H2_weights_for_H1, H2w_H1T);
+                transposed(hm.H2_weights_for_M1, H2w_M1T);
+            }
         }
         poly_tables = (M0_tables ? 1 : 0) | (M1_tables ? 2 : 0);
         flags.resize(8, s);
@@ -823,8 +839,72 @@ struct Engine : EngineBase {
         return linear_ok(K()) && deciding_nodes(N) >= 1024 &&
                (layer == 0 ? M0_tables && NLM() == 1 && !hm.A0_scaled : M1_tables && !hm.A1_scaled);
     }
+    // Whether the node-local stages of an evaluation of N nodes run as chains (smx_kernels_chain.hip).  A chain reads all weights
+    // once per atom, the row tiles once per 16 atoms, and both gain from wider rows, so the line is one of atoms times channels.
+    // Whole evaluations, us, launches per stage against chains: one l, double, 96 channels 1 024 atoms 285 / 260, 1 536 atoms 339 /
+    // 366, 128 channels 768 atoms 322 / 279, 1 024 atoms 342 / 338, single, 96 channels 1 536 atoms 240 / 233; l <= 1, 128 channels
+    // double 512 atoms 514 / 444, single 768 atoms 410 / 399, 96 channels 348 / 325, 64 channels double 1 024 atoms 457 / 396;
+    // l <= 2, 128 channels double 400 atoms 759 / 686, 64 channels single 768 atoms 386 / 337.  Times of the stages are those of
+    // launches of their own, so an evaluation that takes them has these.
+    bool use_chains(int N) const
+    {
+        static const long most[3] = {98304, 65536, 49152};
+        return !profiling && split_nodes > 0 && chain_ok(K()) && M0_tables && M1_tables && !hm.A0_scaled && !hm.A1_scaled &&
+               (long)deciding_nodes(N) * K() <= most[hm.L_max];
+    }
     // The layer-0 adjoint linear writes over Phi0, unless the evaluation keeps Phi0 to form A0 from it on request.
-    bool separate_dPhi0(int N) const { return fused_contraction(0, N); }
+    bool separate_dPhi0(int N) const { return fused_contraction(0, N) || (use_chains(N) && NLM() == 1); }
+    ChainParams<F> chain_params(int N)
+    {
+        ChainParams<F> p{};
+        need(t_perm.p, "species groups");
+        p.N = N; p.K = K(); p.T = hm.T; p.perm = t_perm.p; p.tstart = t_start.p;
+        return p;
+    }
+    // A0, M0 and H1
+    void st_chain0(int N)
+    {
+        const size_t k = K(), nlm = NLM();
+        A0.size_to((size_t)N * 16 * k, stream);
+        M0.size_to((size_t)N * nlm * k, stream);
+        if (nlm == 1) M0_grad.size_to((size_t)N * 16 * k, stream);
+        if (H1.n != M0.n) H1.resize(M0.n, stream);   // mace.cpp:400
+        auto p = chain_params(N);
+        p.Phi = Phi0.p; p.W = linA0.p; p.WH1 = H1w.p; p.coef = M0_coef16.p;
+        p.A = A0.p; p.M = M0.p; p.M_grad = M0_grad.p; p.H1 = H1.p;
+        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain0<F, decltype(kc)::value>(p, hm.L_max, stream); }));
+        if (nlm == 1) pending_A0 = N;
+    }
+    // A1, M1, the tail and the adjoints back to dPhi1
+    void st_chain1(int N, bool zero_energies)
+    {
+        const size_t k = K();
+        A1.size_to((size_t)N * 16 * k, stream);
+        M1.size_to((size_t)N * k, stream); M1_grad.size_to((size_t)N * 16 * k, stream);
+        dPhi1.size_to(Phi1.n, stream);
+        auto p = chain_params(N);
+        p.Phi = Phi1.p; p.W = linA1.p; p.Wt = linA1T.p; p.WHt = H2w_H1T.p; p.WMt = H2w_M1T.p; p.coef = M1_coef16.p;
+        p.M = M1.p; p.M_grad = M1_grad.p; p.out = dPhi1.p;
+        const auto q = tail_params(N, zero_energies);
+        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain1<F, decltype(kc)::value>(p, q, hm.L_max, stream); }));
+        if (guard_status && q.rows > 0) guard_clear_enqueued = true;
+        energies_copy = nullptr;
+        pending_A1 = N; pending_A1_adj = N;
+    }
+    // the messages (`add_messages`: those of the last layer-1 adjoint are not in H1_adj yet), M0_adj, A0_adj and dPhi0
+    void st_chain2(int N, bool add_messages)
+    {
+        const size_t k = K();
+        M0_adj.size_to(M0.n, stream);
+        DVec<F>& to = separate_dPhi0(N) ? dPhi0 : Phi0;
+        to.size_to((size_t)N * 16 * k, stream);
+        if (add_messages && sender_rows != N) build_sender_lists(N);
+        auto p = chain_params(N);
+        p.Wt = linA0T.p; p.WH1 = H1wT.p; p.coef = M0_coef16.p; p.A = A0.p; p.M = M0_adj.p; p.M_grad = M0_grad.p; p.out = to.p;
+        p.msg = add_messages ? msg.p : nullptr; p.H1_adj = H1_adj.p; p.sstart = s_start.p; p.slist = s_list.p; p.spare = s_rank.p;
+        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain2<F, decltype(kc)::value>(p, hm.L_max, stream); }));
+        pending_A0_adj = N;
+    }
     // A0 (or A1) and its contraction in one launch
     void st_linear_contraction(int layer, int N)
     {
@@ -1007,7 +1087,7 @@ struct Engine : EngineBase {
         HIPCHK((launch_gemm<double, F, double>(g, stream)));
     }
     // H2, readouts and reverse_H2 of the full pipeline in one launch (they touch one atom's rows only)
-    void st_tail(int N, bool zero_energies)
+    TailParams<F> tail_params(int N, bool zero_energies)
     {
         const int k = K(), nlm = NLM();
         need(t_perm.p, "species groups");
@@ -1025,8 +1105,13 @@ struct Engine : EngineBase {
         p.node_energies = node_energies.p; p.zero_energies = zero_energies ? 1 : 0; p.energies_copy = energies_copy;
         p.guard = guard_live(); p.guard_clear = guard_status;
         p.guard_forces = guard_status ? node_forces.p : nullptr; p.guard_copy = guard_status ? forces_copy : nullptr; p.guard_forces_n = guard_status ? (long)node_forces.n : 0;
+        return p;
+    }
+    void st_tail(int N, bool zero_energies)
+    {
+        const auto p = tail_params(N, zero_energies);
         HIPCHK(launch_tail_fused<F>(p, stream));
-        if (guard_status && rows > 0) guard_clear_enqueued = true;
+        if (guard_status && p.rows > 0) guard_clear_enqueued = true;
         energies_copy = nullptr;
     }
     void st_readouts(int N, bool zero_energies)
@@ -1100,6 +1185,7 @@ struct Engine : EngineBase {
         auto p = agg_params(1, N);
         p.d_out = dPhi1.p; p.forces = node_forces.p; p.accumulate_forces = zero_dxyz ? 0 : 1; p.msg = msg.p;
         agg_bwd_stage(1, p, E1, ST_AGG1B, ST_FSUM1);
+        if (chain_messages) { messages_left = true; stage_absent(ST_SRED); return; }
         stage_begin(ST_SRED);
         if (sender_rows != rows) build_sender_lists(rows);
         if (fuse_reverse_H1 && nlm == 1 && sender_reduce_linear_ok(k) && M0.n == (size_t)rows * k) {
@@ -1114,6 +1200,8 @@ struct Engine : EngineBase {
         }
         stage_end(ST_SRED);
     }
+    bool chain_messages = false;    // compute() leaves the sender-side sum to the chain behind the layer-1 adjoint
+    bool messages_left = false;     // ... and the stage did so
     bool fuse_reverse_H1 = false;   // compute() wants reverse_H1 folded into the sender-side sum
     bool reverse_H1_done = false;   // ... and the stage did it
     // The same stage for edge lists whose messages do not fit the staging buffer: receivers are taken in
@@ -1207,7 +1295,7 @@ struct Engine : EngineBase {
             // whatever was half built is not trusted by the next call
             senders_counted = false; counters_clean = 0; sender_rows = -1;
             energies_copy = nullptr; forces_copy = nullptr;
-            fuse_reverse_H1 = false;
+            fuse_reverse_H1 = chain_messages = false;
             // checks of the failed call may have raised the word that only its readout launch would have cleared
             if (guard_status && !guard_clear_enqueued) (void)launch_fill<int>(guard_status, 1, 0, stream);
             (void)launch_fill<int>(flags.p + 4, 1, 0, stream);
@@ -1296,7 +1384,11 @@ struct Engine : EngineBase {
         stage_begin(ST_AGG0F); st_agg0_fwd(N); stage_end(ST_AGG0F);
         pending_A0 = pending_A1 = -1;
         pending_M0_grad = recompute_M0_grad() ? N : -1;
-        if (fused_contraction(0, N)) {
+        const bool chain = use_chains(N);
+        if (chain) {
+            stage_begin(ST_A0LIN); st_chain0(N); stage_end(ST_A0LIN);
+            stage_absent(ST_M0); stage_absent(ST_H1);
+        } else if (fused_contraction(0, N)) {
             stage_begin(ST_A0LIN); st_linear_contraction(0, N); stage_end(ST_A0LIN);
             stage_absent(ST_M0);
         } else {
@@ -1304,10 +1396,22 @@ struct Engine : EngineBase {
             st_scale(0, N, false);
             stage_begin(ST_M0); st_poly(N, false, pending_M0_grad >= 0 ? 1 : 0); stage_end(ST_M0);
         }
-        stage_begin(ST_H1); st_H1(N, false); stage_end(ST_H1);
+        if (!chain) { stage_begin(ST_H1); st_H1(N, false); stage_end(ST_H1); }
         // the species groups cover the nodes of the current stages
         if (N1 < N) build_type_groups(N1);
         stage_begin(ST_AGG1F); st_agg1_fwd(N1); stage_end(ST_AGG1F);
+        if (chain) {
+            stage_begin(ST_A1); st_chain1(N1, !hm.has_zbl); stage_end(ST_A1);
+            for (int st : {ST_M1, ST_H2, ST_READOUT, ST_REVH2, ST_REVM1, ST_REVA1}) stage_absent(st);
+            chain_messages = true; messages_left = false;
+            st_agg1_bwd(N1, !early_forces, false);
+            chain_messages = false;
+            if (N1 < N) build_type_groups(N);
+            stage_begin(ST_REVA0LIN); st_chain2(N, messages_left); stage_end(ST_REVA0LIN);
+            stage_absent(ST_REVH1); stage_absent(ST_REVM0);
+            finish_evaluation(N, N1, on_device);
+            return;
+        }
         if (fused_contraction(1, N1)) {
             stage_begin(ST_A1); st_linear_contraction(1, N1); stage_end(ST_A1);
             stage_absent(ST_M1);
@@ -1345,6 +1449,11 @@ struct Engine : EngineBase {
         pending_A0_adj = fuse0 ? N : -1;
         st_scale(0, N, true);
         stage_begin(ST_REVA0LIN); st_A0_lin(N, true, fuse0); stage_end(ST_REVA0LIN);
+        finish_evaluation(N, N1, on_device);
+    }
+    // the layer-0 adjoint, and what the caller's arrays still lack
+    void finish_evaluation(int N, int N1, bool on_device)
+    {
         st_agg0_bwd(N);
         // (a skipped evaluation: the readout launch has filled the forces with NaN, and every sum of partial forces
         // after it looks at the guard itself)

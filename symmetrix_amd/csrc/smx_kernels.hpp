@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "smx_poly_shape.hpp"
 
 namespace smx {
@@ -345,6 +347,43 @@ struct TailParams {
 };
 bool tail_fused_ok(int K);
 template <typename F> hipError_t launch_tail_fused(const TailParams<F>& p, hipStream_t s);
+
+// ---------------------------------------------------------------------------
+// The node-local stages between two aggregations in one launch each (smx_kernels_chain.hip), a block per atom: A0, M0, H1; A1,
+// M1, the readout tail and their adjoints (with the arrays of the tail in q); messages, M0_adj, A0_adj, dPhi0.  Standard product
+// basis in both layers, no density normalisation, with_channels(K).
+template <typename F>
+struct ChainParams {
+    int N, K, T;
+    const int* perm; const int* tstart;
+    const F* Phi;            // rows of the aggregation (0, 1)
+    const F* W; const F* Wt; // A-basis weights in operand order (0, 1), transposed ones (1, 2)
+    const F* WH1;            // [L_max + 1][K][K] of H1 (0), its transposes (2)
+    const double* WHt; const double* WMt;    // transposes of the tail's W_H1, W_M1 (1)
+    const F* coef;           // contraction coefficients by column tile: [species][column tile][monomials / V][16][V]
+    F* A;                    // A-basis: written (0) or read (2) where layer 0 has several polynomials per channel
+    F* M; F* M_grad;         // polynomials and gradients: written (0, 1); M0_adj is written, M0_grad read (2)
+    F* H1;                   // (0)
+    F* out;                  // dPhi1 (1), dPhi0 (2)
+    const F* msg; F* H1_adj; const int* sstart; int* slist; int* spare;     // (2)
+    unsigned lds_front, lds_part;    // set by the launchers
+};
+inline bool chain_ok(int K) { return K == 32 || K == 64 || K == 96 || K == 128; }
+template <typename F, int K> hipError_t launch_chain0(ChainParams<F> p, int L_max, hipStream_t s);
+template <typename F, int K> hipError_t launch_chain1(ChainParams<F> p, const TailParams<F>& q, int L_max, hipStream_t s);
+template <typename F, int K> hipError_t launch_chain2(ChainParams<F> p, int L_max, hipStream_t s);
+// f(K as a constant) for the numbers of channels above
+template <typename Fn>
+hipError_t with_channels(int K, Fn&& f)
+{
+    switch (K) {
+    case 32: return f(std::integral_constant<int, 32>{});
+    case 64: return f(std::integral_constant<int, 64>{});
+    case 96: return f(std::integral_constant<int, 96>{});
+    case 128: return f(std::integral_constant<int, 128>{});
+    default: return hipErrorInvalidValue;
+    }
+}
 template <typename T> hipError_t launch_fill(T* p, long n, T v, hipStream_t s);
 template <typename TS, typename TD> hipError_t launch_convert(const TS* src, TD* dst, long n, hipStream_t s);
 
