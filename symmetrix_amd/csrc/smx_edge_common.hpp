@@ -34,13 +34,13 @@ __device__ __forceinline__ T load_at(const char* row, unsigned lane_bytes)
 // The four coefficients of one spline: 16 bytes in single precision, two halves of 16 bytes in double (a table row is
 // [path][half][K][16 bytes], so that every load instruction of a wavefront covers 1 KB without gaps).
 template <typename F>
-__device__ __forceinline__ Vec<F, 4> load_spline(const char* row, int path, unsigned K, unsigned k)
+__device__ __forceinline__ Vec<F, 4> load_spline(const char* row, int path, unsigned K, unsigned k16)
 {
-    if constexpr (sizeof(F) == 4) return load_at<Vec<F, 4>>(row + path * (K * 16), k * 16);
+    if constexpr (sizeof(F) == 4) return load_at<Vec<F, 4>>(row + path * (K * 16), k16);
     else {
         Vec<F, 4> c;
-        const Vec<F, 2> lo = load_at<Vec<F, 2>>(row + 2 * path * (K * 16), k * 16);
-        const Vec<F, 2> hi = load_at<Vec<F, 2>>(row + (2 * path + 1) * (K * 16), k * 16);
+        const Vec<F, 2> lo = load_at<Vec<F, 2>>(row + 2 * path * (K * 16), k16);
+        const Vec<F, 2> hi = load_at<Vec<F, 2>>(row + (2 * path + 1) * (K * 16), k16);
         c.v[0] = lo.v[0]; c.v[1] = lo.v[1]; c.v[2] = hi.v[0]; c.v[3] = hi.v[1];
         return c;
     }
@@ -62,6 +62,22 @@ __device__ __forceinline__ Vec<F, 4> load_spline_off(const F* tab, int path, uns
 __device__ __forceinline__ const char* uniform_row(const void* base, int n, unsigned row_bytes)
 {
     return reinterpret_cast<const char*>(base) + (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(n) * row_bytes;
+}
+// The byte offset of a lane, formed anew: the address of a load is then scalar registers plus 32 bits per lane.  An offset that
+// stays the same is widened to 64 bits outside the loop otherwise, and every load pays for a 64-bit addition per lane (26 to 32
+// of 590 instructions per edge in the general adjoint; without them 50 000 atoms, l <= 1, single precision 17.6 -> 17.2 ms).
+__device__ __forceinline__ unsigned lane_offset(unsigned bytes)
+{
+    asm volatile("" : "+v"(bytes));
+    return bytes;
+}
+// Where row n (the same in all lanes) of an array begins, in bytes, plus `part`: an offset that stays in scalar registers (or the
+// compiler adds the part to every lane's address).
+__device__ __forceinline__ unsigned long long uniform_offset(int n, unsigned row_bytes, unsigned part)
+{
+    unsigned long long at = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(n) * row_bytes + part;
+    asm volatile("" : "+s"(at));
+    return at;
 }
 // The value is final here: keeps the compiler from collecting the arithmetic of several paths, whose operands would all stay
 // live (it moves plain arithmetic across scheduling fences).

@@ -258,17 +258,25 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
 
     Vec<F, 4> cf[CPL][W];
     F H[CPL][NLM], Hn[CPL][NLM];
+    unsigned k16[CPL], ks[CPL];      // byte offsets of this lane's channels in a table row and in a feature row
+    auto offsets = [&]() {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) { k16[c] = lane_offset(k[c] * 16); ks[c] = lane_offset(k[c] * (unsigned)sizeof(F)); }
+    };
+    offsets();
     const unsigned row_bytes = P * K * 4 * sizeof(F), sender_bytes = NLM * K * sizeof(F);
     auto request_spline = [&](const char* row, int path) {
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) cf[c][path % W] = load_spline<F>(row, path, K, k[c]);
+        for (int c = 0; c < CPL; ++c) cf[c][path % W] = load_spline<F>(row, path, K, k16[c]);
     };
     auto request_sender = [&](int le) {
-        const char* row = uniform_row(a.Hsrc, grows[le], sender_bytes);
+        const int grow = grows[le];
 #pragma unroll
-        for (int c = 0; c < CPL; ++c)
+        for (int q = 0; q < NLM; ++q) {
+            const char* part = reinterpret_cast<const char*>(a.Hsrc) + uniform_offset(grow, sender_bytes, q * (K * (unsigned)sizeof(F)));
 #pragma unroll
-            for (int q = 0; q < NLM; ++q) Hn[c][q] = load_at<F>(row + q * (K * sizeof(F)), k[c] * sizeof(F));
+            for (int c = 0; c < CPL; ++c) Hn[c][q] = load_at<F>(part, ks[c]);
+        }
     };
     const char* cur = nullptr;      // table row of the edge under way
     for (int eb = e0; eb < e1; eb += kChunk) {
@@ -303,6 +311,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
             block_values<LMAXH, false, MX, F, 16, SUB>(a, coef, offs, Yt + sb * 16, ns, vals, lane);
             wave_lds_sync();
             for (int le = sb; le < sb + ns; ++le) {
+                offsets();
                 const F x = (F)xs[le];
                 F B[BL::REGS];
 #pragma unroll
@@ -467,10 +476,16 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
         }
 
     Vec<F, 4> cf[CPL][W];
+    unsigned k16[CPL], ks[CPL];      // byte offsets of this lane's channels in a table row and in a feature row
+    auto offsets = [&]() {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) { k16[c] = lane_offset(k[c] * 16); ks[c] = lane_offset(k[c] * (unsigned)sizeof(F)); }
+    };
+    offsets();
     const unsigned row_bytes = P * K * 4 * sizeof(F), sender_bytes = NLM * K * sizeof(F);
     auto request_spline = [&](const char* row, int path) {
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) cf[c][path % W] = load_spline<F>(row, path, K, k[c]);
+        for (int c = 0; c < CPL; ++c) cf[c][path % W] = load_spline<F>(row, path, K, k16[c]);
     };
     const char* cur = nullptr;      // table row of the edge under way
     for (int eb = e0; eb < e1; eb += kChunk) {
@@ -511,15 +526,18 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
             block_values<LMAXH, true, MX, F, 48, SUB>(a, coef, offs, Yt + sb * 48, ns, vals, lane);
             wave_lds_sync();
             for (int le = sb; le < sb + ns; ++le) {
+                offsets();
                 const F x = (F)xs[le];
                 // the sender row is met at the end of the edge only: requested here, it has the whole edge to arrive
                 F H[CPL][NLM];
                 {
-                    const char* row = uniform_row(a.Hsrc, grows[le], sender_bytes);
+                    const int grow = grows[le];
 #pragma unroll
-                    for (int c = 0; c < CPL; ++c)
+                    for (int q = 0; q < NLM; ++q) {
+                        const char* part = reinterpret_cast<const char*>(a.Hsrc) + uniform_offset(grow, sender_bytes, q * (K * (unsigned)sizeof(F)));
 #pragma unroll
-                        for (int q = 0; q < NLM; ++q) H[c][q] = load_at<F>(row + q * (K * sizeof(F)), k[c] * sizeof(F));
+                        for (int c = 0; c < CPL; ++c) H[c][q] = load_at<F>(part, ks[c]);
+                    }
                 }
                 const char* next = uniform_row(a.tabK, rows[le + 1], row_bytes);
                 const F* Bp = vals + (size_t)(le - sb) * BL::NV + (lane & (BL::LANES - 1));
@@ -625,12 +643,15 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                         srad += V[c][q][3] * h; g1 += V[c][q][1] * h; g2 += V[c][q][2] * h;
                     }
                 if (a.msg) {
-                    char* mrow = reinterpret_cast<char*>(a.msg) + (unsigned long long)(unsigned)(eb + le - (int)a.msg_edge_begin) * sender_bytes;
+                    char* part[NLM];
+#pragma unroll
+                    for (int q = 0; q < NLM; ++q)
+                        part[q] = reinterpret_cast<char*>(a.msg) + uniform_offset(eb + le - (int)a.msg_edge_begin, sender_bytes, q * (K * (unsigned)sizeof(F)));
 #pragma unroll
                     for (int c = 0; c < CPL; ++c)
                         if (active[c]) {
 #pragma unroll
-                            for (int q = 0; q < NLM; ++q) store_stream(reinterpret_cast<F*>(mrow + q * (K * sizeof(F)) + k[c] * sizeof(F)), V[c][q][0]);
+                            for (int q = 0; q < NLM; ++q) store_stream(reinterpret_cast<F*>(part[q] + lane_offset(ks[c])), V[c][q][0]);
                         }
                 }
                 // sums over the channels of the wavefront, in the feature precision (a fixed tree)
