@@ -40,15 +40,26 @@ constexpr int kChunk = 16;   // edges whose geometry is formed together
 // Which entry of B[path][m][m2] (and of its two tangential derivatives) every lane and register holds.
 //   matrix form:  register g / 16, lanes 4 (g % 16) + i hold row 4 tile + i of group g; a group is one matrix
 //                 instruction: (path, row tile, inner index).  Forward: rows m, inner m2; adjoint: rows 3 m2 + t, inner m.
-//   DPP form:     register v / 16, lane v % 16 of every row: v = 3 (boff + m n2 + m2) + t, forward v = boff + m n2 + m2
-template <int LMAXH, bool BWD, bool MATRIX>
+//   DPP form:     register v / 16, lane v % 16 of every row: v = 3 (entry_off + m n2 + m2) + t, forward entry_off + m n2 + m2
+// CP: a path of the constant harmonic (l1 = 0, so l = l2) has none where it couples like with like only, as an equivariant model
+// does: u[m2] = c d[m2] needs no product with a block and has no tangential part.  10 of the 88 rows and columns for l <= 1, 35 of
+// 243 for l <= 2; the constants go into the adjoint rows as they are loaded, or into the sums as they are stored.  Evaluations of
+// 50 000 atoms, l <= 1, single: 17.2 -> 16.9 ms; 24 999 atoms, double: 12.5 -> 12.1 ms; 3 000 atoms, l <= 2: 1 720 -> 1 658 us.
+template <int LMAXH, bool BWD, bool MATRIX, bool CP>
 struct BlockLayout {
     using PT = Paths<LMAXH>;
+    static constexpr bool in(int p) { return !(CP && PT::l1(p) == 0); }     // whether the path has entries in the block
     static constexpr int n2(int p) { return 2 * PT::l2(p) + 1; }
     static constexpr int nm(int p) { return 2 * PT::l(p) + 1; }
     static constexpr int rows(int p) { return BWD ? 3 * n2(p) : nm(p); }
     static constexpr int inner(int p) { return BWD ? nm(p) : n2(p); }
-    static constexpr int tiles(int p) { return (rows(p) + 3) / 4; }
+    static constexpr int tiles(int p) { return in(p) ? (rows(p) + 3) / 4 : 0; }
+    static constexpr int entry_off(int p)
+    {
+        int n = 0;
+        for (int q = 0; q < p; ++q) n += in(q) ? nm(q) * n2(q) : 0;
+        return n;
+    }
     static constexpr int tile_off(int p)
     {
         int n = 0;
@@ -63,7 +74,7 @@ struct BlockLayout {
     }
     static constexpr int group(int p, int tile, int in) { return group_off(p) + tile * inner(p) + in; }
     static constexpr int TILES = tile_off(PT::P);
-    static constexpr int REGS = MATRIX ? (group_off(PT::P) + 15) / 16 : (PT::NB * (BWD ? 3 : 1) + 15) / 16;
+    static constexpr int REGS = MATRIX ? (group_off(PT::P) + 15) / 16 : (entry_off(PT::P) * (BWD ? 3 : 1) + 15) / 16;
     static constexpr int LANES = MATRIX ? 64 : 16;      // lanes that hold different entries
     static constexpr int NV = REGS * LANES;
     struct Table {
@@ -75,7 +86,8 @@ struct BlockLayout {
         Table t{};
         for (int v = 0; v < NV; ++v) { t.entry[v] = -1; t.comp[v] = 0; }
         for (int p = 0; p < PT::P; ++p) {
-            const int N2 = n2(p), NM = nm(p), bo = PT::boff(p), go = group_off(p), R = rows(p), IN = inner(p);
+            if (!in(p)) continue;
+            const int N2 = n2(p), NM = nm(p), bo = PT::boff(p), eo = entry_off(p), go = group_off(p), R = rows(p), IN = inner(p);
             if (MATRIX) {
                 for (int tl = 0; tl < tiles(p); ++tl)
                     for (int in = 0; in < IN; ++in)
@@ -89,7 +101,7 @@ struct BlockLayout {
             } else {
                 for (int b = 0; b < NM * N2; ++b)
                     for (int c = 0; c < (BWD ? 3 : 1); ++c) {
-                        const int v = BWD ? 3 * (bo + b) + c : bo + b;
+                        const int v = BWD ? 3 * (eo + b) + c : eo + b;
                         t.entry[v] = (short)(bo + b);
                         t.comp[v] = (unsigned char)c;
                     }
@@ -98,13 +110,13 @@ struct BlockLayout {
         return t;
     }
 };
-template <int LMAXH, bool BWD, bool MATRIX>
-__device__ const typename BlockLayout<LMAXH, BWD, MATRIX>::Table block_table = BlockLayout<LMAXH, BWD, MATRIX>::make();
+template <int LMAXH, bool BWD, bool MATRIX, bool CP>
+__device__ const typename BlockLayout<LMAXH, BWD, MATRIX, CP>::Table block_table = BlockLayout<LMAXH, BWD, MATRIX, CP>::make();
 
 // LDS of a block: the coefficients of the block entries, then a part for each of its four wavefronts
-template <typename F, int LMAXH, bool BWD>
+template <typename F, int LMAXH, bool BWD, bool CP>
 struct EdgeLds {
-    using BL = BlockLayout<LMAXH, BWD, kMatrix<F>>;
+    using BL = BlockLayout<LMAXH, BWD, kMatrix<F>, CP>;
     static constexpr int NY = BWD ? 48 : 16;     // harmonics (and their two tangential derivatives) of an edge
     // edges whose blocks are in LDS at a time: as many as leave room for two thread blocks on a CU
     static constexpr int SUB = BL::NV * (int)sizeof(F) > 3000 ? 2 : (BL::NV * (int)sizeof(F) > 1000 ? 4 : 8);
@@ -134,12 +146,12 @@ __device__ __forceinline__ F wave_sum3(F s, F g1, F g2)
 
 // The coefficients of the block entries: value v = c0 Y[o0] + c1 Y[o1] (an entry of a real coupling has at most two terms;
 // a file with longer ones sets more_terms and pays for a loop), copied to LDS once per thread block.
-template <int LMAXH, bool BWD, bool MATRIX, typename F>
+template <int LMAXH, bool BWD, bool MATRIX, bool CP, typename F>
 __device__ __forceinline__ void block_lists(const AggParams<F>& a, double* coef, int* offs)
 {
-    using BL = BlockLayout<LMAXH, BWD, MATRIX>;
+    using BL = BlockLayout<LMAXH, BWD, MATRIX, CP>;
     for (int v = threadIdx.x; v < BL::NV; v += 256) {
-        const int b = block_table<LMAXH, BWD, MATRIX>.entry[v], comp = block_table<LMAXH, BWD, MATRIX>.comp[v];
+        const int b = block_table<LMAXH, BWD, MATRIX, CP>.entry[v], comp = block_table<LMAXH, BWD, MATRIX, CP>.comp[v];
         double c0 = 0.0, c1 = 0.0;
         int o0 = 0, o1 = 0;
         if (b >= 0) {
@@ -151,11 +163,11 @@ __device__ __forceinline__ void block_lists(const AggParams<F>& a, double* coef,
         offs[v] = (comp * 16 + o0) | ((comp * 16 + o1) << 16);
     }
 }
-template <int LMAXH, bool BWD, bool MATRIX, typename F, int NY, int SUB>
+template <int LMAXH, bool BWD, bool MATRIX, bool CP, typename F, int NY, int SUB>
 __device__ __forceinline__ void block_values(const AggParams<F>& a, const double* coef, const int* offs, const double* Yt, int ns,
                                              F* vals, int lane)
 {
-    using BL = BlockLayout<LMAXH, BWD, MATRIX>;
+    using BL = BlockLayout<LMAXH, BWD, MATRIX, CP>;
 #pragma unroll
     for (int j = 0; j < (BL::NV + 63) / 64; ++j) {
         const int v = lane + 64 * j;
@@ -169,7 +181,7 @@ __device__ __forceinline__ void block_values(const AggParams<F>& a, const double
     }
     if (a.more_terms) {
         for (int v = lane; v < BL::NV; v += 64) {
-            const int b = block_table<LMAXH, BWD, MATRIX>.entry[v];
+            const int b = block_table<LMAXH, BWD, MATRIX, CP>.entry[v];
             if (b < 0) continue;
             for (int le = 0; le < ns; ++le) {
                 const double* y = Yt + le * NY + (offs[v] & 0xfff0);
@@ -195,13 +207,13 @@ constexpr int agg_blocks()
 // Forward: out[i, lme, k] = sum over the edges of R_path(r)[k] sum_m2 B[lme, m2] H[sender, m2, k].
 // Bound by the coefficient rows: P splines of 16 (32) bytes per channel and edge, 10 KB (20 KB) per edge and wavefront at
 // l <= 1, of the 64 bytes per cycle that a CU's vector cache hands out.
-template <typename F, int LMAXH, int CPL>
+template <typename F, int LMAXH, int CPL, bool CP>
 __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_agg_fwd(const AggParams<F> a, const int parts)
 {
     constexpr bool MX = kMatrix<F>;
     using PT = Paths<LMAXH>;
-    using BL = BlockLayout<LMAXH, false, MX>;
-    using EL = EdgeLds<F, LMAXH, false>;
+    using BL = BlockLayout<LMAXH, false, MX, CP>;
+    using EL = EdgeLds<F, LMAXH, false, CP>;
     constexpr int NE = PT::NE, P = PT::P, NLM = PT::NLM, SUB = EL::SUB;
     constexpr int W = P <= 5 ? P : 5;     // splines of the ring: requested W paths ahead
     extern __shared__ __align__(16) unsigned char smem[];
@@ -215,7 +227,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
     int* rows = reinterpret_cast<int*>(xs + kChunk + 1);                          // [kChunk + 1]
     int* grows = rows + kChunk + 1;                                               // [kChunk + 1]
 
-    block_lists<LMAXH, false, MX>(a, coef, offs);
+    block_lists<LMAXH, false, MX, CP>(a, coef, offs);
     __syncthreads();
 
     const unsigned K = (unsigned)a.K;
@@ -245,9 +257,12 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
 
     f32x4 tile[MX ? CPL : 1][MX ? BL::TILES : 1];
     F acc[MX ? 1 : CPL][MX ? 1 : NE];
+    F same[CPL][NLM];               // CP in matrix form: the sums of the paths of the constant harmonic
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
         if constexpr (MX) {
+#pragma unroll
+            for (int q = 0; q < NLM; ++q) same[c][q] = F(0);
 #pragma unroll
             for (int q = 0; q < BL::TILES; ++q) tile[c][q] = f32x4{0, 0, 0, 0};
         } else {
@@ -308,7 +323,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
         for (int sb = 0; sb < nE; sb += SUB) {
             const int ns = min(SUB, nE - sb);
             if (sb) wave_lds_sync();
-            block_values<LMAXH, false, MX, F, 16, SUB>(a, coef, offs, Yt + sb * 16, ns, vals, lane);
+            block_values<LMAXH, false, MX, CP, F, 16, SUB>(a, coef, offs, Yt + sb * 16, ns, vals, lane);
             wave_lds_sync();
             for (int le = sb; le < sb + ns; ++le) {
                 offsets();
@@ -333,7 +348,15 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
                         for (int m2 = 0; m2 < n2; ++m2) w[c][m2] = R * H[c][l2 * l2 + m2];
                     }
                     if constexpr (p + W < P) request_spline(cur, p + W); else request_spline(next, p % W);
-                    if constexpr (MX) {
+                    if constexpr (!BL::in(p)) {
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                            for (int m = 0; m < n2; ++m) {
+                                F& s = MX ? same[c][l2 * l2 + m] : acc[MX ? 0 : c][MX ? 0 : PT::lme(p, 0) + m * PT::num_e(l)];
+                                s += w[c][m];
+                            }
+                    } else if constexpr (MX) {
                         static_for<0, n2>([&](auto mc) {
                             static_for<0, BL::tiles(p)>([&](auto tc) {
                                 constexpr int g = BL::group(p, decltype(tc)::value, decltype(mc)::value), t = BL::tile_off(p) + decltype(tc)::value;
@@ -343,7 +366,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
                             });
                         });
                     } else {
-                        constexpr int bo = PT::boff(p), lme0 = PT::lme(p, 0), es = PT::num_e(l);
+                        constexpr int bo = BL::entry_off(p), lme0 = PT::lme(p, 0), es = PT::num_e(l);
                         static_for<0, n2>([&](auto mc) {
                             static_for<0, 2 * l + 1>([&](auto rc) {
                                 constexpr int v = bo + decltype(rc)::value * n2 + decltype(mc)::value;
@@ -354,7 +377,12 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
                         });
                     }
                     // path by path
-                    if constexpr (MX) {
+                    if constexpr (MX && !BL::in(p)) {
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                            for (int m = 0; m < n2; ++m) pin(same[c][l2 * l2 + m]);
+                    } else if constexpr (MX) {
 #pragma unroll
                         for (int c = 0; c < CPL; ++c)
 #pragma unroll
@@ -376,7 +404,8 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
     // sum lme of channel c of this lane
     auto value = [&](auto pc, auto mc, int c) -> F& {
         constexpr int p = decltype(pc)::value, m = decltype(mc)::value;
-        if constexpr (MX) return reinterpret_cast<F*>(&tile[c][BL::tile_off(p) + m / 4])[m % 4];
+        if constexpr (MX && !BL::in(p)) return same[c][PT::l2(p) * PT::l2(p) + m];
+        else if constexpr (MX) return reinterpret_cast<F*>(&tile[c][BL::tile_off(p) + m / 4])[m % 4];
         else return acc[c][PT::lme(p, 0) + m * PT::num_e(PT::l(p))];
     };
     auto every = [&](auto&& f) {      // f(lme, channel slot, sum)
@@ -400,6 +429,15 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
         if (part < h) every([&](int q, int c, F& v) { v += at[(size_t)(q * CPL + c) * 64]; });
     }
     if (!real || part != 0) return;
+    if constexpr (CP)
+        static_for<0, P>([&](auto pc) {
+            constexpr int p = decltype(pc)::value;
+            if constexpr (!BL::in(p))
+                static_for<0, 2 * PT::l(p) + 1>([&](auto mc) {
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c) value(pc, mc, c) *= (F)a.c_same[PT::l(p) * PT::l(p) + decltype(mc)::value];
+                });
+        });
     every([&](int q, int c, F& v) {
         if (active[c]) a.out[((size_t)i * NE + q) * K + k[c]] = v;
     });
@@ -417,15 +455,20 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
 // u[m2][t] = sum_m d[m] (B, dB.t1, dB.t2)[m][m2]; with R and R' of the path they add to four sums per m2,
 //   message R u[.][0],  R u[.][1],  R u[.][2],  R' u[.][0],
 // and only at the end of the edge these meet the sender feature (radial and two tangential forces).
-template <typename F, int LMAXH, int CPL>
+template <typename F, int LMAXH, int CPL, bool CP>
 __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_agg_bwd(const AggParams<F> a, const int parts)
 {
     constexpr bool MX = kMatrix<F>;
     using PT = Paths<LMAXH>;
-    using BL = BlockLayout<LMAXH, true, MX>;
-    using EL = EdgeLds<F, LMAXH, true>;
+    using BL = BlockLayout<LMAXH, true, MX, CP>;
+    using EL = EdgeLds<F, LMAXH, true, CP>;
     constexpr int NE = PT::NE, P = PT::P, NLM = PT::NLM, SUB = EL::SUB;
     constexpr int W = P <= 5 ? P : 5;     // splines of the ring: requested W paths ahead
+    constexpr auto first_tangential = [](int l2) {
+        for (int p = 0; p < P; ++p)
+            if (PT::l2(p) == l2 && BL::in(p)) return p;
+        return -1;
+    };
     extern __shared__ __align__(16) unsigned char smem[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     double* coef = reinterpret_cast<double*>(smem);
@@ -439,7 +482,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
     int* rows = reinterpret_cast<int*>(xs + kChunk + 1);
     int* grows = rows + kChunk + 1;
 
-    block_lists<LMAXH, true, MX>(a, coef, offs);
+    block_lists<LMAXH, true, MX, CP>(a, coef, offs);
     __syncthreads();
 
     const unsigned K = (unsigned)a.K;
@@ -474,6 +517,16 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
             const F v = a.d_out[((size_t)i * NE + q) * K + k[c]];
             d[c][q] = active[c] ? v : F(0);
         }
+    if constexpr (CP)
+        static_for<0, P>([&](auto pc) {
+            constexpr int p = decltype(pc)::value, l = PT::l(p);
+            if constexpr (!BL::in(p))
+                static_for<0, 2 * l + 1>([&](auto mc) {
+                    constexpr int m = decltype(mc)::value;
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c) d[c][PT::lme(p, 0) + m * PT::num_e(l)] *= (F)a.c_same[l * l + m];
+                });
+        });
 
     Vec<F, 4> cf[CPL][W];
     unsigned k16[CPL], ks[CPL];      // byte offsets of this lane's channels in a table row and in a feature row
@@ -523,7 +576,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
         for (int sb = 0; sb < nE; sb += SUB) {
             const int ns = min(SUB, nE - sb);
             if (sb) wave_lds_sync();
-            block_values<LMAXH, true, MX, F, 48, SUB>(a, coef, offs, Yt + sb * 48, ns, vals, lane);
+            block_values<LMAXH, true, MX, CP, F, 48, SUB>(a, coef, offs, Yt + sb * 48, ns, vals, lane);
             wave_lds_sync();
             for (int le = sb; le < sb + ns; ++le) {
                 offsets();
@@ -555,6 +608,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                     constexpr int p = decltype(pc)::value, l = PT::l(p), l2 = PT::l2(p), n2 = 2 * l2 + 1;
                     constexpr int lme0 = PT::lme(p, 0), es = PT::num_e(l);
                     constexpr bool starts = p == PT::first_with_l2(l2);    // the first path of this l2 starts the sums
+                    constexpr bool starts_t = p == first_tangential(l2);   // ... of the tangential parts
                     F R[CPL], Rd[CPL];
 #pragma unroll
                     for (int c = 0; c < CPL; ++c) {
@@ -565,7 +619,17 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                         Rd[c] = q2 + x * d1;
                     }
                     if constexpr (p + W < P) request_spline(cur, p + W); else request_spline(next, p % W);
-                    if constexpr (MX) {
+                    if constexpr (!BL::in(p)) {
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                            for (int m2 = 0; m2 < n2; ++m2) {
+                                const F dm = d[c][lme0 + m2 * es];
+                                F* s = V[c][l2 * l2 + m2];
+                                s[0] = starts ? R[c] * dm : s[0] + R[c] * dm;
+                                s[3] = starts ? Rd[c] * dm : s[3] + Rd[c] * dm;
+                            }
+                    } else if constexpr (MX) {
                         constexpr int T = BL::tiles(p);
                         f32x4 u[CPL][T];
                         static_for<0, 2 * l + 1>([&](auto mc) {
@@ -586,7 +650,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
 #pragma unroll
                                 for (int t = 0; t < 3; ++t) {
                                     const F uv = u[c][(3 * m2 + t) / 4][(3 * m2 + t) % 4];
-                                    s[t] = starts ? R[c] * uv : s[t] + R[c] * uv;
+                                    s[t] = (t == 0 ? starts : starts_t) ? R[c] * uv : s[t] + R[c] * uv;
                                     if (t == 0) s[3] = starts ? Rd[c] * uv : s[3] + Rd[c] * uv;
                                 }
                             }
@@ -603,7 +667,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                             for (int c = 0; c < CPL; ++c) {
                                 const F dm = d[c][lme0 + m * es], rd = R[c] * dm;
                                 static_for<0, n2>([&](auto m2c) {
-                                    constexpr int m2 = decltype(m2c)::value, v = 3 * (PT::boff(p) + m * n2 + m2);
+                                    constexpr int m2 = decltype(m2c)::value, v = 3 * (BL::entry_off(p) + m * n2 + m2);
                                     fmac_lane<v % 16>(u0[c][m2], B[v / 16], dm);
                                     fmac_lane<(v + 1) % 16>(V[c][l2 * l2 + m2][1], B[(v + 1) / 16], rd);
                                     fmac_lane<(v + 2) % 16>(V[c][l2 * l2 + m2][2], B[(v + 2) / 16], rd);
@@ -625,8 +689,9 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
 #pragma unroll
                         for (int m2 = 0; m2 < n2; ++m2)
 #pragma unroll
-                            for (int t = 0; t < 4; ++t) pin(V[c][l2 * l2 + m2][t]);
-                    if constexpr (MX) {
+                            for (int t = 0; t < 4; ++t)
+                                if (BL::in(p) || t == 0 || t == 3) pin(V[c][l2 * l2 + m2][t]);
+                    if constexpr (MX && BL::in(p)) {
                         // the matrix instructions of a path together: every change between the pipes costs about four cycles
                         __builtin_amdgcn_sched_group_barrier(0x008, BL::tiles(p) * (2 * l + 1) * CPL, 0);
                         __builtin_amdgcn_sched_group_barrier(0x002, 100, 0);
@@ -674,10 +739,10 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
     }
 }
 
-template <typename F, int LMAXH, int CPL, bool BWD>
+template <typename F, int LMAXH, int CPL, bool BWD, bool CP>
 hipError_t launch_agg_t(const AggParams<F>& p, hipStream_t s)
 {
-    using EL = EdgeLds<F, LMAXH, BWD>;
+    using EL = EdgeLds<F, LMAXH, BWD, CP>;
     const int groups = (p.K + 64 * CPL - 1) / (64 * CPL);
     if (BWD && groups > 1 && !p.fpart) return hipErrorInvalidValue;
     if (!BWD && (p.node_begin != 0 || p.msg_edge_begin != 0)) return hipErrorInvalidValue;
@@ -691,9 +756,9 @@ hipError_t launch_agg_t(const AggParams<F>& p, hipStream_t s)
     dim3 grid((unsigned)blocks);
     void (*kern)(const AggParams<F>, const int);
     size_t lds = EL::total;
-    if constexpr (BWD) kern = k_agg_bwd<F, LMAXH, CPL>;
+    if constexpr (BWD) kern = k_agg_bwd<F, LMAXH, CPL, CP>;
     else {
-        kern = k_agg_fwd<F, LMAXH, CPL>;
+        kern = k_agg_fwd<F, LMAXH, CPL, CP>;
         const size_t handed = parts > 1 ? (size_t)2 * Paths<LMAXH>::NE * CPL * 64 * sizeof(F) : 0;   // two givers per block
         lds = lds > handed ? lds : handed;
     }
@@ -713,13 +778,22 @@ int agg_cpl(int K)
     return (LMAXH == 0 || (LMAXH == 1 && sizeof(F) == 4 && BWD)) && K > 64 ? 2 : 1;
 }
 
+template <typename F, int LMAXH, int CPL, bool BWD>
+hipError_t launch_agg_cp(const AggParams<F>& p, hipStream_t s)
+{
+    // (scalar features come here with couplings that the scalar kernels do not take)
+    if constexpr (LMAXH > 0) {
+        if (p.constant_same) return launch_agg_t<F, LMAXH, CPL, BWD, true>(p, s);
+    }
+    return launch_agg_t<F, LMAXH, CPL, BWD, false>(p, s);
+}
 template <typename F, int LMAXH, bool BWD>
 hipError_t launch_agg_sel(const AggParams<F>& p, hipStream_t s)
 {
     if constexpr (LMAXH == 0 || (LMAXH == 1 && sizeof(F) == 4 && BWD)) {
-        if (agg_cpl<F, LMAXH, BWD>(p.K) == 2) return launch_agg_t<F, LMAXH, 2, BWD>(p, s);
+        if (agg_cpl<F, LMAXH, BWD>(p.K) == 2) return launch_agg_cp<F, LMAXH, 2, BWD>(p, s);
     }
-    return launch_agg_t<F, LMAXH, 1, BWD>(p, s);
+    return launch_agg_cp<F, LMAXH, 1, BWD>(p, s);
 }
 
 }  // namespace

@@ -13,6 +13,8 @@ ARRAYS = ["A0", "M0", "H1", "Phi1", "A1", "M1", "H2", "H2_adj", "M1_adj", "A1_ad
 
 def _both(tmp_models, K, L_max, n, dtype, density=0.1):
     """Whatever an evaluation leaves, by either way."""
+    import torch
+    assert torch.cuda.is_available()
     from symmetrix_amd.mace import MACE
     model = H.tiny_model(K=K, L_max=L_max, n_pts=48, seed=3 * K + L_max, r_cut=3.5, pair=False)
     eng = MACE(H.write_model(model, tmp_models / f"chains_{K}_{L_max}.json"), dtype)
