@@ -36,6 +36,9 @@ namespace smx {
 namespace {
 
 constexpr int kChunk = 16;   // edges whose geometry is formed together
+// Harmonics lie in LDS by entry, a chunk's edges side by side: a lane of block_values reads two edges at once.  Entries are 144
+// bytes apart, so that lanes at different entries meet different banks.
+constexpr int kEdgeStride = kChunk + 2;
 
 // Which entry of B[path][m][m2] (and of its two tangential derivatives) every lane and register holds.
 //   matrix form:  register g / 16, lanes 4 (g % 16) + i hold row 4 tile + i of group g; a group is one matrix
@@ -121,7 +124,7 @@ struct EdgeLds {
     // edges whose blocks are in LDS at a time: as many as leave room for two thread blocks on a CU
     static constexpr int SUB = BL::NV * (int)sizeof(F) > 3000 ? 2 : (BL::NV * (int)sizeof(F) > 1000 ? 4 : 8);
     static constexpr size_t lists = ((size_t)BL::NV * (2 * sizeof(double) + sizeof(int)) + 15) / 16 * 16;
-    static constexpr size_t y_bytes = (size_t)kChunk * NY * sizeof(double);
+    static constexpr size_t y_bytes = (size_t)NY * kEdgeStride * sizeof(double);
     static constexpr size_t frame_bytes = BWD ? (size_t)kChunk * 10 * sizeof(double) : 0;    // direction over r, tangents
     static constexpr size_t head_bytes = (size_t)(kChunk + 1) * (sizeof(double) + 2 * sizeof(int)) + 8;  // x, table row, sender row
     static constexpr size_t sum_bytes = BWD ? (size_t)kChunk * 4 * sizeof(F) : 0;
@@ -160,10 +163,10 @@ __device__ __forceinline__ void block_lists(const AggParams<F>& a, double* coef,
             if (s1 > s0 + 1) { c1 = a.B_c[s0 + 1]; o1 = a.B_lm1[s0 + 1]; }
         }
         coef[2 * v] = c0; coef[2 * v + 1] = c1;
-        offs[v] = (comp * 16 + o0) | ((comp * 16 + o1) << 16);
+        offs[v] = (comp * 16 + o0) * kEdgeStride | ((comp * 16 + o1) * kEdgeStride) << 16;
     }
 }
-template <int LMAXH, bool BWD, bool MATRIX, bool CP, typename F, int NY, int SUB>
+template <int LMAXH, bool BWD, bool MATRIX, bool CP, typename F, int SUB>
 __device__ __forceinline__ void block_values(const AggParams<F>& a, const double* coef, const int* offs, const double* Yt, int ns,
                                              F* vals, int lane)
 {
@@ -172,11 +175,15 @@ __device__ __forceinline__ void block_values(const AggParams<F>& a, const double
     for (int j = 0; j < (BL::NV + 63) / 64; ++j) {
         const int v = lane + 64 * j;
         if (BL::NV % 64 == 0 || v < BL::NV) {
-            const double c0 = coef[2 * v], c1 = coef[2 * v + 1];
+            const double2 c = *reinterpret_cast<const double2*>(coef + 2 * v);
             const int o = offs[v], o0 = o & 0xffff, o1 = o >> 16;
+            static_assert(SUB % 2 == 0, "pairs of edges");
 #pragma unroll
-            for (int le = 0; le < SUB; ++le)      // (past the chunk's last edge: numbers nobody reads)
-                vals[le * BL::NV + v] = (F)(c0 * Yt[le * NY + o0] + c1 * Yt[le * NY + o1]);
+            for (int le = 0; le < SUB; le += 2) {      // (past the chunk's last edge: numbers nobody reads)
+                const double2 y0 = *reinterpret_cast<const double2*>(Yt + o0 + le), y1 = *reinterpret_cast<const double2*>(Yt + o1 + le);
+                vals[le * BL::NV + v] = (F)(c.x * y0.x + c.y * y1.x);
+                vals[(le + 1) * BL::NV + v] = (F)(c.x * y0.y + c.y * y1.y);
+            }
         }
     }
     if (a.more_terms) {
@@ -184,9 +191,9 @@ __device__ __forceinline__ void block_values(const AggParams<F>& a, const double
             const int b = block_table<LMAXH, BWD, MATRIX, CP>.entry[v];
             if (b < 0) continue;
             for (int le = 0; le < ns; ++le) {
-                const double* y = Yt + le * NY + (offs[v] & 0xfff0);
+                const double* y = Yt + block_table<LMAXH, BWD, MATRIX, CP>.comp[v] * 16 * kEdgeStride + le;
                 double s = 0.0;
-                for (int t = a.B_start[b]; t < a.B_start[b + 1]; ++t) s += a.B_c[t] * y[a.B_lm1[t]];
+                for (int t = a.B_start[b]; t < a.B_start[b + 1]; ++t) s += a.B_c[t] * y[a.B_lm1[t] * kEdgeStride];
                 vals[le * BL::NV + v] = (F)s;
             }
         }
@@ -221,7 +228,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
     double* coef = reinterpret_cast<double*>(smem);
     int* offs = reinterpret_cast<int*>(coef + 2 * BL::NV);
     unsigned char* base = smem + EL::lists + (size_t)wave * EL::per_wave;
-    double* Yt = reinterpret_cast<double*>(base);                                 // [kChunk][16]
+    double* Yt = reinterpret_cast<double*>(base);                                 // [16][kEdgeStride]
     F* vals = reinterpret_cast<F*>(base + EL::y_bytes);                           // [SUB][NV]
     double* xs = reinterpret_cast<double*>(base + EL::y_bytes + EL::block_bytes); // [kChunk + 1]
     int* rows = reinterpret_cast<int*>(xs + kChunk + 1);                          // [kChunk + 1]
@@ -311,7 +318,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
                 double Y[16];
                 sph_l3(dz * inv, dx * inv, dy * inv, Y);
 #pragma unroll
-                for (int q = 0; q < 16; ++q) Yt[lane * 16 + q] = Y[q];
+                for (int q = 0; q < 16; ++q) Yt[q * kEdgeStride + lane] = Y[q];
             }
         }
         wave_lds_sync();
@@ -323,7 +330,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
         for (int sb = 0; sb < nE; sb += SUB) {
             const int ns = min(SUB, nE - sb);
             if (sb) wave_lds_sync();
-            block_values<LMAXH, false, MX, CP, F, 16, SUB>(a, coef, offs, Yt + sb * 16, ns, vals, lane);
+            block_values<LMAXH, false, MX, CP, F, SUB>(a, coef, offs, Yt + sb, ns, vals, lane);
             wave_lds_sync();
             for (int le = sb; le < sb + ns; ++le) {
                 offsets();
@@ -474,7 +481,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
     double* coef = reinterpret_cast<double*>(smem);
     int* offs = reinterpret_cast<int*>(coef + 2 * BL::NV);
     unsigned char* base = smem + EL::lists + (size_t)wave * EL::per_wave;
-    double* Yt = reinterpret_cast<double*>(base);                                 // [kChunk][3][16]: Y, dY.t1, dY.t2
+    double* Yt = reinterpret_cast<double*>(base);                                 // [3][16][kEdgeStride]: Y, dY.t1, dY.t2
     double* us = reinterpret_cast<double*>(base + EL::y_bytes);                   // [kChunk][10]: xyz / r, t1, t2, -
     F* vals = reinterpret_cast<F*>(base + EL::y_bytes + EL::frame_bytes);         // [SUB][NV]
     F* sums = vals + (size_t)SUB * BL::NV;                                        // [kChunk][4]: radial, t2, t1, (t2)
@@ -560,10 +567,10 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                 double* fr = us + lane * 10;
                 fr[0] = f.dx * ir; fr[1] = f.dy * ir; fr[2] = f.dz * ir;
                 fr[3] = f.t1x; fr[4] = f.t1y; fr[5] = f.t1z; fr[6] = f.t2x; fr[7] = f.t2y; fr[8] = f.t2z;
-                double* y = Yt + lane * 48;
+                double* y = Yt + lane;
                 static_for<0, 16>([&](auto lc) {
                     constexpr int lm = decltype(lc)::value;
-                    ylm_tangential<lm>(f, y[lm], y[16 + lm], y[32 + lm]);
+                    ylm_tangential<lm>(f, y[lm * kEdgeStride], y[(16 + lm) * kEdgeStride], y[(32 + lm) * kEdgeStride]);
                     if constexpr (lm % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // short live ranges
                 });
             }
@@ -576,7 +583,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
         for (int sb = 0; sb < nE; sb += SUB) {
             const int ns = min(SUB, nE - sb);
             if (sb) wave_lds_sync();
-            block_values<LMAXH, true, MX, CP, F, 48, SUB>(a, coef, offs, Yt + sb * 48, ns, vals, lane);
+            block_values<LMAXH, true, MX, CP, F, SUB>(a, coef, offs, Yt + sb, ns, vals, lane);
             wave_lds_sync();
             for (int le = sb; le < sb + ns; ++le) {
                 offsets();
