@@ -20,15 +20,34 @@ namespace smx {
 
 namespace {
 
+// a b + c into a register of its own.  Left alone, the compiler copies c first and accumulates in the copy where the registers of c
+// belong to the next load: 24 copies among the 218 instructions of the single-precision adjoint for 96 channels.
+__device__ __forceinline__ float fma_apart(float a, float b, float c)
+{
+    float r;
+    asm("v_fma_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ double fma_apart(double a, double b, double c) { return fma(a, b, c); }
+
 constexpr int lm_of_tile(int t) { return t == 0 ? 0 : (t == 1 ? 1 : (t == 2 ? 4 : (t == 3 ? 8 : (t == 4 ? 9 : 13)))); }
 
-// edges per chunk: one lane each (two are left for a look at the next chunk), as many as leave room for two thread blocks on a CU
-template <typename F, bool BWD>
-constexpr int chunk0() { return BWD && sizeof(F) == 8 ? 44 : 62; }
+// Wavefronts per SIMD (thread blocks per CU) of the adjoint: what the registers of its channels allow.  20 011 atoms, 96 channels,
+// single: adjoints of 275 and 264 us with two, 253 and 237 with three; 24 999 atoms, 128 channels, double 1.03 and 1.02 ms.
+template <typename F, int CPL>
+constexpr int bwd0_blocks() { return CPL <= (sizeof(F) == 8 ? 2 : 3) ? 3 : 2; }
+// edges per chunk: one lane each (two are left for a look at the next chunk), as many as leave room for the thread blocks of a CU
+template <typename F, bool BWD, int CPL>
+constexpr int chunk0()
+{
+    if (!BWD) return 62;
+    if (bwd0_blocks<F, CPL>() == 3) return sizeof(F) == 8 ? 30 : 54;
+    return sizeof(F) == 8 ? 44 : 62;
+}
 
-template <typename F, bool BWD>
+template <typename F, bool BWD, int CPL>
 struct Lds0 {
-    static constexpr int CH = chunk0<F, BWD>();
+    static constexpr int CH = chunk0<F, BWD, CPL>();
     static_assert(CH % 2 == 0 && CH + 2 <= 64, "whole iterations, and a lane for every entry");
     static constexpr int NY = BWD ? 48 : 16;          // [lm][3]: harmonic, its two tangential derivatives; or harmonics
     static constexpr size_t val_bytes = ((size_t)CH * NY + 16) * sizeof(F);
@@ -36,6 +55,7 @@ struct Lds0 {
     static constexpr size_t sum_bytes = BWD ? (size_t)(CH + 2) * 4 * sizeof(double) : 0;
     static_assert(val_bytes % 16 == 0, "the sums begin on a 16-byte boundary");
     static constexpr size_t per_wave = (val_bytes + head_bytes + sum_bytes + 15) / 16 * 16;
+    static_assert(!BWD || 4 * per_wave * bwd0_blocks<F, CPL>() <= 160 * 1024, "the thread blocks of a CU");
 };
 
 // interval, argument and rows of an edge; offsets of its table and sender rows in bytes (32 bits: launch_agg0_ok)
@@ -54,7 +74,7 @@ template <typename F, int CPL, int EW>
 __global__ __launch_bounds__(256, 2) void k_agg0_fwd(const AggParams<F> a, const int parts, const int group_channels)
 {
     constexpr bool MX = kMatrix<F>;
-    using L = Lds0<F, false>;
+    using L = Lds0<F, false, CPL>;
     constexpr int LPE = 64 / EW, CH = L::CH, CBSZ = EW == 2 ? 3 : 4;
     constexpr int W = MX || CPL <= 2 ? 4 : 2;          // splines requested ahead
     extern __shared__ __align__(16) unsigned char smem[];
@@ -269,10 +289,10 @@ __device__ __forceinline__ double edge_sum3(F s, F g1, F g2, int lane)
 
 // ---------------------------------------------------------------------------
 template <typename F, int CPL, int EW, bool MSG>
-__global__ __launch_bounds__(256, 2) void k_agg0_bwd(const AggParams<F> a, const int parts)
+__global__ __launch_bounds__(256, (bwd0_blocks<F, CPL>())) void k_agg0_bwd(const AggParams<F> a, const int parts)
 {
     constexpr bool MX = kMatrix<F>;
-    using L = Lds0<F, true>;
+    using L = Lds0<F, true, CPL>;
     constexpr int LPE = 64 / EW, CH = L::CH, CBSZ = EW == 2 ? 3 : 4, GPR = LPE / 4;   // groups of four rows per register
     constexpr int NB = MX ? 16 / GPR : 3;              // registers that hold an edge's harmonics
     constexpr int W = MX || CPL == 1 ? 4 : 2;          // splines requested ahead
@@ -312,6 +332,7 @@ __global__ __launch_bounds__(256, 2) void k_agg0_bwd(const AggParams<F> a, const
             const F v = a.d_out[((size_t)i * 16 + q) * K + k[c]];
             d[c][q] = active[c] ? v : F(0);
         }
+        d[c][0] *= (F)a.cdiag[0];
     }
     // the entries of an edge's harmonics this lane holds, one per register
     int pick[NB];
@@ -372,12 +393,16 @@ __global__ __launch_bounds__(256, 2) void k_agg0_bwd(const AggParams<F> a, const
 #pragma unroll
                 for (int c = 0; c < CPL; ++c) {
                     const Vec<F, 4> k4 = cf[c][l % W];
-                    const F q1 = k4.v[2] + x * k4.v[3], d1 = q1 + x * k4.v[3], q2 = k4.v[1] + x * q1;
-                    R[c] = k4.v[0] + x * q2;
+                    const F q1 = k4.v[2] + x * k4.v[3], d1 = q1 + x * k4.v[3], q2 = fma_apart(x, q1, k4.v[1]);
+                    R[c] = fma_apart(x, q2, k4.v[0]);
                     Rd[c] = q2 + x * d1;
                 }
                 if constexpr (l + W < 4) request_spline(cur, l + W); else request_spline(next, l % W);
-                if constexpr (MX) {
+                if constexpr (l == 0) {
+                    // the constant harmonic: its factor is in the adjoint row, and there is no tangential part
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c) { V[c][0] = R[c] * d[c][0]; V[c][3] = Rd[c] * d[c][0]; }
+                } else if constexpr (MX) {
                     f32x4 u[CPL];
                     static_for<l * l, (l + 1) * (l + 1)>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
@@ -387,44 +412,36 @@ __global__ __launch_bounds__(256, 2) void k_agg0_bwd(const AggParams<F> a, const
                     });
 #pragma unroll
                     for (int c = 0; c < CPL; ++c) {
-                        if constexpr (l == 0) {      // a constant harmonic: no tangential part
-                            V[c][0] = R[c] * u[c][0]; V[c][3] = Rd[c] * u[c][0]; V[c][1] = F(0); V[c][2] = F(0);
-                        } else {
-                            V[c][0] += R[c] * u[c][0]; V[c][3] += Rd[c] * u[c][0];
-                            V[c][1] += R[c] * u[c][1]; V[c][2] += R[c] * u[c][2];
-                        }
+                        V[c][0] += R[c] * u[c][0]; V[c][3] += Rd[c] * u[c][0];
+                        V[c][1] = l == 1 ? R[c] * u[c][1] : V[c][1] + R[c] * u[c][1];
+                        V[c][2] = l == 1 ? R[c] * u[c][2] : V[c][2] + R[c] * u[c][2];
                     }
                 } else {
-                    if constexpr (l == 0) {
-#pragma unroll
-                        for (int c = 0; c < CPL; ++c) { V[c][1] = F(0); V[c][2] = F(0); }
-                    }
                     F u0[CPL];
 #pragma unroll
-                    for (int c = 0; c < CPL; ++c) u0[c] = F(0);
+                    for (int c = 0; c < CPL; ++c) {
+                        u0[c] = F(0);
+                        if constexpr (l == 1) { V[c][1] = F(0); V[c][2] = F(0); }
+                    }
                     static_for<l * l, (l + 1) * (l + 1)>([&](auto qc) {
                         constexpr int q = decltype(qc)::value, v = 3 * q;
 #pragma unroll
                         for (int c = 0; c < CPL; ++c) {
                             fmac_lane<v % 16>(u0[c], B[v / 16], d[c][q]);
-                            if constexpr (l > 0) {
-                                const F rd = R[c] * d[c][q];
-                                fmac_lane<(v + 1) % 16>(V[c][1], B[(v + 1) / 16], rd);
-                                fmac_lane<(v + 2) % 16>(V[c][2], B[(v + 2) / 16], rd);
-                            }
+                            const F rd = R[c] * d[c][q];
+                            fmac_lane<(v + 1) % 16>(V[c][1], B[(v + 1) / 16], rd);
+                            fmac_lane<(v + 2) % 16>(V[c][2], B[(v + 2) / 16], rd);
                         }
                     });
 #pragma unroll
-                    for (int c = 0; c < CPL; ++c) {
-                        V[c][0] = l == 0 ? R[c] * u0[c] : V[c][0] + R[c] * u0[c];
-                        V[c][3] = l == 0 ? Rd[c] * u0[c] : V[c][3] + Rd[c] * u0[c];
-                    }
+                    for (int c = 0; c < CPL; ++c) { V[c][0] += R[c] * u0[c]; V[c][3] += Rd[c] * u0[c]; }
                 }
 #pragma unroll
                 for (int c = 0; c < CPL; ++c)
 #pragma unroll
-                    for (int t = MSG ? 0 : 1; t < 4; ++t) pin(V[c][t]);
-                if constexpr (MX) {
+                    for (int t = MSG ? 0 : 1; t < 4; ++t)
+                        if (l > 0 || t == 0 || t == 3) pin(V[c][t]);
+                if constexpr (MX && l > 0) {
                     __builtin_amdgcn_sched_group_barrier(0x008, (2 * l + 1) * CPL, 0);
                     __builtin_amdgcn_sched_group_barrier(0x002, 100, 0);
                 }
@@ -503,7 +520,7 @@ hipError_t launch0(const AggParams<F>& p, int group, hipStream_t s)
     const long blocks = (nodes * parts + 3) / 4 * groups;
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-    size_t lds = 4 * Lds0<F, BWD>::per_wave;
+    size_t lds = 4 * Lds0<F, BWD, CPL>::per_wave;
     const void* kern;
     if constexpr (BWD) kern = reinterpret_cast<const void*>(p.msg ? k_agg0_bwd<F, CPL, EW, true> : k_agg0_bwd<F, CPL, EW, false>);
     else {
