@@ -237,7 +237,6 @@ struct Engine : EngineBase {
     DVec<F> linA0, linA0T, linA1, linA1T;    // the same weights in operand order (operand_weights)
     DVec<F> M0_coef16, M1_coef16;            // contraction coefficients by column tile
     DVec<F> H1wT;                            // transposes, for the kernels that take a chain of stages
-    DVec<double> H2w_H1T, H2w_M1T;
     DVec<int> pair_table0, pair_table1;
     DVec<int> B0_start, B0_lm1, B1_start, B1_lm1;
     DVec<double> B0_c, B1_c;
@@ -250,7 +249,7 @@ struct Engine : EngineBase {
     bool constant_same1 = false;       // layer 1's paths of the constant harmonic couple like with like only, with these factors
     double c_same1[9] = {};
     DVec<double> fpart;
-    DVec<double> H2w_H1, H2w_M1, ro1, ro2_w1, ro2_w2, E0;
+    DVec<double> H2w_H1, H2w_M1, H2v_H1, H2v_M1, ro1, ro2_w1, ro2_w2, E0;
     struct DevPoly {
         DVec<int> packed, chunks;
         DVec<F> coef;
@@ -401,6 +400,22 @@ struct Engine : EngineBase {
         for (int b = 0; b < hm.num_B; ++b) more_terms1 |= hm.B_start[b + 1] - hm.B_start[b] > 2;
         upload_as(H2w_H1, hm.H2_weights_for_H1, s);
         upload_as(H2w_M1, hm.H2_weights_for_M1, s);
+        {
+            // first layer of the readout network times the transposed weights of H2: the gradient of H2 has rank 16
+            auto through_readout = [&](const std::vector<double>& w, auto& dst) {
+                const size_t Kc = hm.K, n = w.size() / (Kc * Kc);
+                std::vector<double> out(n * 16 * Kc);
+                for (size_t b = 0; b < n; ++b)
+                    for (size_t h = 0; h < 16; ++h)
+                        for (size_t i = 0; i < Kc; ++i) {
+                            double sum = 0.0;
+                            for (size_t j = 0; j < Kc; ++j) sum += hm.readout_2_w1[h * Kc + j] * w[(b * Kc + i) * Kc + j];
+                            out[(b * 16 + h) * Kc + i] = sum;
+                        }
+                upload_as(dst, out, s);
+            };
+            if (tail_fused_ok(hm.K)) { through_readout(hm.H2_weights_for_H1, H2v_H1); through_readout(hm.H2_weights_for_M1, H2v_M1); }
+        }
         upload_as(ro1, hm.readout_1_weights, s);
         upload_as(ro2_w1, hm.readout_2_w1, s);
         upload_as(ro2_w2, hm.readout_2_w2, s);
@@ -492,8 +507,6 @@ struct Engine : EngineBase {
                     upload_as(dst, out, s);
                 };
                 transposed(hm.H1_weights, H1wT);
-                transposed(hm.H2_weights_for_H1, H2w_H1T);
-                transposed(hm.H2_weights_for_M1, H2w_M1T);
             }
         }
         poly_tables = (M0_tables ? 1 : 0) | (M1_tables ? 2 : 0);
@@ -903,7 +916,7 @@ struct Engine : EngineBase {
         M1.size_to((size_t)N * k, stream); M1_grad.size_to((size_t)N * 16 * k, stream);
         dPhi1.size_to(Phi1.n, stream);
         auto p = chain_params(N);
-        p.Phi = Phi1.p; p.W = linA1.p; p.Wt = linA1T.p; p.WHt = H2w_H1T.p; p.WMt = H2w_M1T.p; p.coef = M1_coef16.p;
+        p.Phi = Phi1.p; p.W = linA1.p; p.Wt = linA1T.p; p.coef = M1_coef16.p;
         p.M = M1.p; p.M_grad = M1_grad.p; p.out = dPhi1.p;
         const auto q = tail_params(N, zero_energies);
         HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain1<F, decltype(kc)::value>(p, q, hm.L_max, stream); }));
@@ -1120,7 +1133,7 @@ struct Engine : EngineBase {
         p.N = N; p.rows = rows; p.K = k; p.num_LM = nlm; p.T = hm.T;
         p.perm = t_perm.p; p.tstart = t_start.p;
         p.E0 = E0.p; p.w1 = ro1.p; p.W1 = ro2_w1.p; p.w2 = ro2_w2.p; p.scale = hm.readout_2_scale;
-        p.H1 = H1.p; p.M1 = M1.p; p.W_H1 = H2w_H1.p; p.W_M1 = H2w_M1.p;
+        p.H1 = H1.p; p.M1 = M1.p; p.W_H1 = H2w_H1.p; p.W_M1 = H2w_M1.p; p.V_H1 = H2v_H1.p; p.V_M1 = H2v_M1.p;
         p.H2 = H2.p; p.H2_adj = H2_adj.p; p.H1_adj = H1_adj.p; p.M1_adj = M1_adj.p;
         p.node_energies = node_energies.p; p.zero_energies = zero_energies ? 1 : 0; p.energies_copy = energies_copy;
         p.guard = guard_live(); p.guard_clear = guard_status;

@@ -340,6 +340,8 @@ struct TailParams {
     const F* H1; const F* M1;
     const double* W_H1;      // [T][K][K]
     const double* W_M1;      // [K][K]
+    const double* V_H1;      // [T][16][K]: W1 . W_H1^T
+    const double* V_M1;      // [16][K]: W1 . W_M1^T
     double* H2; double* H2_adj; F* H1_adj; F* M1_adj;
     double* node_energies; int zero_energies; double* energies_copy;
     const int* guard;        // live status of a device-resident evaluation (or null): raised -> energies are NaN
@@ -362,7 +364,6 @@ struct ChainParams {
     const F* Phi;            // rows of the aggregation (0, 1)
     const F* W; const F* Wt; // A-basis weights in operand order (0, 1), transposed ones (1, 2)
     const F* WH1;            // [L_max + 1][K][K] of H1 (0), its transposes (2)
-    const double* WHt; const double* WMt;    // transposes of the tail's W_H1, W_M1 (1)
     const F* coef;           // contraction coefficients by column tile: [species][column tile][monomials / V][16][V]
     F* A;                    // A-basis: written (0) or read (2) where layer 0 has several polynomials per channel
     F* M; F* M_grad;         // polynomials and gradients: written (0, 1); M0_adj is written, M0_grad read (2)

@@ -328,8 +328,7 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
     // adjoint rows; H1[l = 0] and M1 behind them
     double* red = reinterpret_cast<double*>(smem);                // [S][K]
     double* h2 = red + S * K;                                     // [K]
-    double* xa = h2 + K;                                          // [K]: H2_adj
-    double* dots = xa + K;                                        // [17]
+    double* dots = h2 + K;                                        // [17]
     double* hg = dots + 17;                                       // [16]
     double* xh = reinterpret_cast<double*>(smem + p.lds_front);   // [2][K]: H1[l = 0] and M1
     const int ct = wave >> 1, set = wave & 1, column = ct * 16 + r16;
@@ -383,17 +382,24 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
     using TM = Mix<double, 1, 1, count, K>;
     const int sl = tid / (K / 2), pair = (tid - sl * (K / 2)) * 2, from = (sl % (S / 2)) * count;
     const size_t typed = (size_t)b.type * K * K;
-    auto tail_product = [&](const double* W_H1, const double* W_M1, const double* x_H1, const double* x_M1) {
-        TM mix(sl < S / 2 ? W_H1 : W_M1, 0, pair, from);
+    // H2 = H1[l = 0] . W_H1[type] + M1 . W_M1
+    {
+        TM mix(sl < S / 2 ? q.W_H1 + typed : q.W_M1, 0, pair, from);
         mix.begin();
         __syncthreads();
         typename TM::VV acc[1];
-        mix.run((sl < S / 2 ? x_H1 : x_M1) + from, acc, [](auto) { return 0; });
+        mix.run((sl < S / 2 ? xh : xh + K) + from, acc, [](auto) { return 0; });
         *reinterpret_cast<typename TM::VV*>(red + sl * K + pair) = acc[0];
         __syncthreads();
-    };
-    // H2 = H1[l = 0] . W_H1[type] + M1 . W_M1
-    tail_product(q.W_H1 + typed, q.W_M1, xh, xh + K);
+    }
+    // what the gradient of the hidden units is multiplied with below: a channel of H2_adj, H1_adj[l = 0] or M1_adj
+    const int back = tid / K, kb = tid - back * K;
+    double v[16];
+    if (back < 3) {
+        const double* from_hg = back == 0 ? q.W1 : (back == 1 ? q.V_H1 + (size_t)b.type * 16 * K : q.V_M1);
+#pragma unroll
+        for (int h = 0; h < 16; ++h) v[h] = from_hg[h * K + kb];
+    }
     if (own) {
         const double s = mixed<double, 1, K>(red, k);
         h2[k] = s;
@@ -427,15 +433,6 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
         }
     }
     __syncthreads();
-    if (own) {
-        double s = 0.0;
-#pragma unroll
-        for (int h = 0; h < 16; ++h) s += hg[h] * q.W1[h * K + k];
-        xa[k] = s;
-        q.H2_adj[node * K + k] = s;
-    }
-    // H1_adj[l = 0] = w1 + H2_adj . W_H1^T, M1_adj = H2_adj . W_M1^T
-    tail_product(p.WHt + typed, p.WMt, xa, xa);
     // the weights of the adjoint product, for what follows the next two barriers
     auto aim_back = [&](int e) {
 #pragma unroll
@@ -447,19 +444,22 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
         prod.begin();
     };
     aim_back(0);
-    F m1_adj = F(0);
-    if (own) {
-        double h = (double)(F)q.w1[k], m = 0.0;
+    // H2_adj = hg . W1, H1_adj[l = 0] = w1 + H2_adj . W_H1^T, M1_adj = H2_adj . W_M1^T
+    if (back < 3) {
+        double s = back == 1 ? (double)(F)q.w1[kb] : 0.0;
 #pragma unroll
-        for (int j = 0; j < S / 2; ++j) { h += red[j * K + k]; m += red[(S / 2 + j) * K + k]; }
-        m1_adj = (F)m;
-        q.H1_adj[node * width + k] = (F)h;
-#pragma unroll
-        for (int LM = 1; LM < NLM; ++LM) q.H1_adj[node * width + LM * K + k] = F(0);
-        q.M1_adj[node * K + k] = m1_adj;
+        for (int h = 0; h < 16; ++h) s += hg[h] * v[h];
+        if (back == 0) q.H2_adj[node * K + kb] = s;
+        else if (back == 1) q.H1_adj[node * width + kb] = (F)s;
+        else {
+            q.M1_adj[node * K + kb] = (F)s;
+            xh[K + kb] = s;
+        }
     }
+    for (int t = K + tid; t < width; t += T) q.H1_adj[node * width + t] = F(0);
     __syncthreads();
     if (own) {
+        const F m1_adj = (F)xh[K + k];
 #pragma unroll
         for (int i = 0; i < 16; ++i) *reinterpret_cast<F*>(smem + i * RS + k * sizeof(F)) = gr[i] * m1_adj;
     }
@@ -684,7 +684,7 @@ hipError_t launch_chain1(ChainParams<F> p, const TailParams<F>& q, int L_max, hi
     return with_degree(L_max, [&](auto lc) {
         constexpr int LH = decltype(lc)::value;
         constexpr size_t in = Paths<LH>::NE * K * sizeof(F) + 16 * kPad, rows = (size_t)16 * (K * sizeof(F) + kPad);
-        constexpr size_t tail = ((size_t)(mix_slices<1>() + 2) * K + 33) * sizeof(double);
+        constexpr size_t tail = ((size_t)(mix_slices<1>() + 1) * K + 33) * sizeof(double);
         p.lds_front = (unsigned)round16(std::max({in, rows, tail}));
         return launch_chain_t(k_chain1<F, LH, K>, (unsigned)p.N, chain_threads(K), p.lds_front + (size_t)2 * K * sizeof(double), s, p, q);
     });

@@ -74,13 +74,9 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_linear(const LinearParams<F> p)
     const int cb = rem / 8 % cols, e = rem / 8 / cols;
     int type = 0, tile = tile_index, seg0 = 0, seg_n = p.num_nodes;
     if (p.perm) {
-        type = -1;
-        for (int t = 0; t < p.T; ++t) {
-            const int n_t = p.tstart[t + 1] - p.tstart[t], tiles = (n_t + 15) / 16;
-            if (tile < tiles) { type = t; seg0 = p.tstart[t]; seg_n = n_t; break; }
-            tile -= tiles;
-        }
-        if (type < 0) return;
+        const RowTile at = row_tile(p.tstart, p.T, tile_index, lane);
+        if (at.type < 0) return;
+        type = at.type; tile = at.tile; seg0 = at.seg0; seg_n = at.seg_n;
     } else if (tile * 16 >= seg_n) {
         return;
     }
