@@ -125,34 +125,49 @@ __global__ __launch_bounds__(64) void k_sort_buckets(const int* start, int rows,
     if (sorted == buf)
         for (int t = threadIdx.x; t < n; t += 64) list[s0 + t] = sorted[t];
 }
-// species groups in one block: LDS histogram, scan over the (few) species, placement
-__device__ void type_groups_body(const int* node_types, int N, int T, int* tstart, int* perm, int* sh)
+// One block scans an array, or picks a species out of it, 16 consecutive elements per thread at a time: bound by the latency of a
+// load and of the block's scan per round, so that a round takes as many as there are registers for.
+constexpr int SCAN_ITEMS = 16, SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
+__device__ __forceinline__ void load_items(const int* in, int n, int i0, int beyond, int (&v)[SCAN_ITEMS])
 {
-    // sh: [T] counts, [T] cursors
-    int* cnt = sh;
-    int* cur = sh + T;
-    for (int t = threadIdx.x; t < T; t += blockDim.x) { cnt[t] = 0; cur[t] = 0; }
-    __syncthreads();
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-        const int t = node_types[i];
-        if (t >= 0 && t < T) atomicAdd(&cnt[t], 1);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int acc = 0;
-        for (int t = 0; t < T; ++t) { const int c = cnt[t]; cnt[t] = acc; tstart[t] = acc; acc += c; }
-        tstart[T] = acc;
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-        const int t = node_types[i];
-        if (t >= 0 && t < T) perm[cnt[t] + atomicAdd(&cur[t], 1)] = i;
+    if (i0 + SCAN_ITEMS <= n) {
+#pragma unroll
+        for (int q = 0; q < SCAN_ITEMS; ++q) v[q] = in[i0 + q];
+    } else {
+#pragma unroll
+        for (int q = 0; q < SCAN_ITEMS; ++q) v[q] = i0 + q < n ? in[i0 + q] : beyond;
     }
 }
-__global__ __launch_bounds__(1024) void k_type_groups(const int* node_types, int N, int T, int* tstart, int* perm)
+// species group t of a block of its own: where it begins (the number of atoms of smaller species), and its atoms in ascending
+// order.  (One block with counters in the LDS for all species took a serial chain of same-address atomics, two per atom.)
+__device__ void type_group_body(const int* node_types, int N, int T, int t, int* tstart, int* perm)
 {
-    extern __shared__ int sh[];
-    type_groups_body(node_types, N, T, tstart, perm, sh);
+    int before = 0, v[SCAN_ITEMS];
+    for (int b0 = 0; b0 < N; b0 += SCAN_TILE) {
+        load_items(node_types, N, b0 + (int)threadIdx.x * SCAN_ITEMS, -1, v);
+#pragma unroll
+        for (int q = 0; q < SCAN_ITEMS; ++q) before += v[q] >= 0 && v[q] < t;
+    }
+    int place;
+    block_scan_exclusive(before, &place);
+    if (threadIdx.x == 0) tstart[t] = place;
+    for (int b0 = 0; b0 < N; b0 += SCAN_TILE) {
+        const int i0 = b0 + (int)threadIdx.x * SCAN_ITEMS;
+        if (N > SCAN_TILE) load_items(node_types, N, i0, -1, v);
+        int mine = 0, total;
+#pragma unroll
+        for (int q = 0; q < SCAN_ITEMS; ++q) mine += v[q] == t;
+        int to = place + block_scan_exclusive(mine, &total);
+#pragma unroll
+        for (int q = 0; q < SCAN_ITEMS; ++q)
+            if (v[q] == t) perm[to++] = i0 + q;
+        place += total;
+    }
+    if (t == T - 1 && threadIdx.x == 0) tstart[T] = place;
+}
+__global__ __launch_bounds__(SCAN_BLOCK) void k_type_groups(const int* node_types, int N, int T, int* tstart, int* perm)
+{
+    type_group_body(node_types, N, T, blockIdx.x, tstart, perm);
 }
 __global__ void k_check_range(const int* v, long n, int limit, int* flags)
 {
@@ -182,13 +197,22 @@ inline unsigned nblk(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 // instead of three while the array is short
 __device__ void scan_single_body(const int* in, int* out, int n)
 {
-    int carry = 0;
-    for (int b0 = 0; b0 < n; b0 += SCAN_BLOCK) {
-        const int i = b0 + threadIdx.x;
-        const int v = i < n ? in[i] : 0;
-        int total;
-        const int ex = block_scan_exclusive(v, &total);
-        if (i < n) out[i] = carry + ex;
+    int carry = 0, v[SCAN_ITEMS];
+    for (int b0 = 0; b0 < n; b0 += SCAN_TILE) {
+        const int i0 = b0 + (int)threadIdx.x * SCAN_ITEMS;
+        load_items(in, n, i0, 0, v);
+        int sum = 0, total;
+#pragma unroll
+        for (int q = 0; q < SCAN_ITEMS; ++q) { const int x = v[q]; v[q] = sum; sum += x; }
+        const int ex = carry + block_scan_exclusive(sum, &total);
+        if (i0 + SCAN_ITEMS <= n) {
+#pragma unroll
+            for (int q = 0; q < SCAN_ITEMS; ++q) out[i0 + q] = ex + v[q];
+        } else {
+#pragma unroll
+            for (int q = 0; q < SCAN_ITEMS; ++q)
+                if (i0 + q < n) out[i0 + q] = ex + v[q];
+        }
         carry += total;
     }
     if (threadIdx.x == 0) out[n] = carry;
@@ -199,31 +223,28 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_single(const int* in, int* 
 }
 __device__ void node_lists_part(const int* num_neigh, int N, int* first_neigh, const int* node_types, int T,
                                 int* tstart, int* perm, const int* key, long n, int rows, int* count, int* rank,
-                                const InputChecks& chk, int* sh)
+                                const InputChecks& chk)
 {
-    // the two node lists are independent of each other: a block each
+    // the node lists do not depend on each other: a block for the scan, and one for every species
     if (blockIdx.x == 0) {
         scan_single_body(num_neigh, first_neigh, N);
         __syncthreads();   // first_neigh, written by this block, is read back below
-        if (chk.status) {
-            int bad = 0;
-            for (int i = threadIdx.x; i < N; i += SCAN_BLOCK) bad |= (num_neigh[i] < 0) | (node_types[i] < 0) | (node_types[i] >= T);
-            if (threadIdx.x == 0) bad |= (first_neigh[N] != (int)chk.num_edges) | (first_neigh[chk.num_local_nodes] != (int)n);
-            if (bad) atomicOr(chk.status, 1);
-        }
+        if (chk.status && threadIdx.x == 0 && ((first_neigh[N] != (int)chk.num_edges) | (first_neigh[chk.num_local_nodes] != (int)n)))
+            atomicOr(chk.status, 1);
         return;
     }
-    if (blockIdx.x == 1) { type_groups_body(node_types, N, T, tstart, perm, sh); return; }
-    constexpr int LIST_BLOCKS = 2;
-    for (long i = (long)(blockIdx.x - LIST_BLOCKS) * SCAN_BLOCK + threadIdx.x; i < n; i += (long)(gridDim.x - LIST_BLOCKS) * SCAN_BLOCK) {
+    if ((int)blockIdx.x <= T) { type_group_body(node_types, N, T, (int)blockIdx.x - 1, tstart, perm); return; }
+    const long first = (long)(blockIdx.x - 1 - T) * SCAN_BLOCK + threadIdx.x, step = (long)(gridDim.x - 1 - T) * SCAN_BLOCK;
+    for (long i = first; i < n; i += step) {
         const int j = key[i];
         if (j >= 0 && j < rows) rank[i] = atomicAdd(&count[j], 1);   // the entry's place inside its bucket
         else if (chk.status) atomicOr(chk.status, 1);
     }
     if (chk.status) {
-        // species and length of every edge (layer 0 covers the edges of ghost receivers as well)
         int bad = 0;
-        for (long i = (long)(blockIdx.x - LIST_BLOCKS) * SCAN_BLOCK + threadIdx.x; i < chk.num_edges; i += (long)(gridDim.x - LIST_BLOCKS) * SCAN_BLOCK) {
+        for (long i = first; i < N; i += step) bad |= (num_neigh[i] < 0) | (node_types[i] < 0) | (node_types[i] >= T);
+        // species and length of every edge (layer 0 covers the edges of ghost receivers as well)
+        for (long i = first; i < chk.num_edges; i += step) {
             const int t = chk.neigh_types[i];
             const double rr = chk.r[i];
             bad |= (t < 0 || t >= T) ? 1 : 0;
@@ -232,11 +253,14 @@ __device__ void node_lists_part(const int* num_neigh, int N, int* first_neigh, c
         if (bad) atomicOr(chk.status, bad);
     }
 }
-// The node-level lists of one evaluation and its sender histogram in one launch: blocks 0 and 1 form one node list each
-// (first_neigh = exclusive scan of num_neigh, species groups), the other blocks count the
+// The node-level lists of one evaluation and its sender histogram in one launch: blocks 0 to T form the node lists
+// (first_neigh = exclusive scan of num_neigh, the species groups), the other blocks count the
 // senders (counters at zero on entry), which does not depend on the node lists.  With a ticket, the block that finishes last
 // turns the histogram into the sender offsets: a launch of its own costs 6 to 8 us of a small evaluation, but the fences of
-// the ticket cost more than that over many blocks (80 us over 2 048), so the launcher hands out tickets to small grids only.
+// the ticket cost more than that over many blocks (83 blocks, 3 000 atoms: 21 us with the ticket, 19 without; 80 us over 2 048),
+// so the launcher hands out tickets to small grids only.  Larger ones are bound by the atomics (50 000 atoms, 1.4 million
+// edges: 92 us while one block each formed the node lists an element per thread at a time, now 60, the scan behind it 43 and
+// 14; 20 011 atoms 41 and 19, now 26 and 7).
 // With `chk.status` set the launch also checks everything the later kernels use as an address or a table argument
 // (species, sender rows, edge lengths, counts that add up to the edge totals) and raises bits in the status word.
 __global__ __launch_bounds__(SCAN_BLOCK) void k_node_lists_count(const int* num_neigh, int N, int* first_neigh,
@@ -244,8 +268,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_node_lists_count(const int* num_
                                                                 const int* key, long n, int rows, int* count, int* rank,
                                                                 int* sstart, int* ticket, InputChecks chk)
 {
-    extern __shared__ int sh[];
-    node_lists_part(num_neigh, N, first_neigh, node_types, T, tstart, perm, key, n, rows, count, rank, chk, sh);
+    node_lists_part(num_neigh, N, first_neigh, node_types, T, tstart, perm, key, n, rows, count, rank, chk);
     if (!ticket) return;
     // every block's counts are out before it takes its ticket
     __shared__ int last;
@@ -278,9 +301,9 @@ hipError_t launch_node_lists_count(const int* num_neigh, int N, int* first_neigh
 {
     if (N <= 0 || N > 64 * SCAN_BLOCK || T <= 0) return hipErrorInvalidValue;
     const long work = chk.status ? std::max(n, chk.num_edges) : n;
-    const unsigned nb = 3 + (unsigned)std::max<long>(1, std::min<long>((work + SCAN_BLOCK - 1) / SCAN_BLOCK, 2048));
-    const bool with_scan = nb <= 160;
-    hipLaunchKernelGGL(k_node_lists_count, dim3(nb), dim3(SCAN_BLOCK), 2 * T * sizeof(int), s, num_neigh, N, first_neigh,
+    const unsigned counting = (unsigned)std::max<long>(1, std::min<long>((work + SCAN_BLOCK - 1) / SCAN_BLOCK, 2048));
+    const bool with_scan = counting <= 48;
+    hipLaunchKernelGGL(k_node_lists_count, dim3(1 + T + counting), dim3(SCAN_BLOCK), 0, s, num_neigh, N, first_neigh,
                        node_types, T, tstart, perm, key, n, rows, count, rank, sstart, with_scan ? ticket : nullptr, chk);
     if (!with_scan) hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(SCAN_BLOCK), 0, s, count, sstart, rows);
     return hipGetLastError();
@@ -332,9 +355,7 @@ hipError_t launch_type_groups(const int* node_types, int N, int T, int* tcount, 
 {
     (void)tcount; (void)cursor; (void)block_sums;
     if (T <= 0) return hipSuccess;
-    // order inside a species group is left as placed: every output row of the products
-    // that use this grouping is computed independently of its tile mates
-    hipLaunchKernelGGL(k_type_groups, dim3(1), dim3(1024), 2 * T * sizeof(int), s, node_types, N, T, tstart, perm);
+    hipLaunchKernelGGL(k_type_groups, dim3(T), dim3(SCAN_BLOCK), 0, s, node_types, N, T, tstart, perm);
     return hipGetLastError();
 }
 

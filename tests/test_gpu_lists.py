@@ -1,0 +1,69 @@
+"""The list preparation of an evaluation: one block's scan and one block per species, at the edges of a thread's 16 elements, of
+a block's round, and of the number of blocks that count with a ticket."""
+import numpy as np
+import pytest
+
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 1025, 16383, 16385, 33000])
+def test_lists_of_any_length(tmp_models, n):
+    """Energies and forces of an atom depend on its own edges only: a system of n atoms in random order of species, with 0 to 3
+    edges each, against the same atoms a few at a time.  A row that the lists lose, repeat or give to another species differs in
+    the first digits; what is left is the order of sums (2^-53 of at most 640 terms, a dozen in a row)."""
+    import torch
+    assert torch.cuda.is_available()
+    from symmetrix_amd.mace import MACE
+    model = H.tiny_model(K=32, L_max=0, T=(1, 6, 7, 8), n_pts=16, seed=5, r_cut=3.0, pair=False)
+    eng = MACE(H.write_model(model, tmp_models / "lists.json"), "float64")
+    rng = np.random.default_rng(n)
+    species = rng.choice([0, 1, 3], n).astype(np.int32)       # the third species has no atom
+    num = rng.integers(0, 4, n).astype(np.int32)
+    if n > 1000:
+        num[:16 * 7] = 0
+        species[-200:] = 3
+    i = np.repeat(np.arange(n), num)
+    # neighbours inside groups of 8 consecutive atoms, which can be evaluated by themselves
+    j = np.minimum(i // 8 * 8 + rng.integers(0, 8, len(i)), n - 1).astype(np.int32)
+    r = rng.uniform(0.8, 2.9, len(i))
+    u = rng.normal(size=(len(i), 3))
+    xyz = u * (r / np.linalg.norm(u, axis=1))[:, None]
+    print(f"atoms={n} edges={len(i)}", flush=True)
+    eng.compute_node_energies_forces(n, species, num, j, species[j], xyz, r)
+    E, F = np.array(eng.node_energies), np.array(eng.node_forces).reshape(-1, 3)
+    assert np.isfinite(E).all() and np.isfinite(F).all()
+    first = np.concatenate([[0], np.cumsum(num)])
+    groups = np.unique(np.concatenate([[0, (n - 1) // 8], rng.integers(0, (n + 7) // 8, 12), np.arange(16384 // 8 - 1, 16384 // 8 + 1)]))
+    for g in groups[groups * 8 < n]:
+        a, b = g * 8, min(g * 8 + 8, n)
+        e = slice(first[a], first[b])
+        eng.compute_node_energies_forces(b - a, species[a:b], num[a:b], j[e] - a, species[j[e]], xyz[e], r[e])
+        assert np.abs(np.array(eng.node_energies) - E[a:b]).max() <= 1e-12 * np.abs(E).max()
+        f = np.array(eng.node_forces).reshape(-1, 3)
+        if len(f):
+            assert np.abs(f - F[e]).max() <= 1e-12 * max(np.abs(F).max(), 1.0)
+
+
+def test_lists_refuse_what_they_refused(tmp_models):
+    """A species or a sender out of range, a negative count: found by whichever block looks at it."""
+    import torch
+    assert torch.cuda.is_available()
+    from symmetrix_amd.mace import MACE
+    model = H.tiny_model(K=32, L_max=0, T=(1, 6, 8), n_pts=16, seed=5, r_cut=3.0, pair=False)
+    eng = MACE(H.write_model(model, tmp_models / "lists_bad.json"), "float64")
+    n = 20000
+    species, num = np.zeros(n, np.int32), np.ones(n, np.int32)
+    j = np.roll(np.arange(n), 1).astype(np.int32)
+    xyz, r = np.tile([0.0, 0.0, 1.0], (n, 1)), np.ones(n)
+    eng.compute_node_energies_forces(n, species, num, j, species, xyz, r)
+    good = np.array(eng.node_energies)
+    for at in (0, 17000, n - 1):
+        for which, value in ((0, 3), (0, -1), (2, n), (2, -1), (3, 3)):
+            args = [species.copy(), num, j.copy(), species.copy()]
+            args[which][at] = value
+            with pytest.raises(Exception):
+                eng.compute_node_energies_forces(n, *args, xyz, r)
+    eng.compute_node_energies_forces(n, species, num, j, species, xyz, r)
+    assert np.array_equal(np.array(eng.node_energies), good)
