@@ -2,8 +2,8 @@
 // cores (MACE::compute_A0 / compute_A1, the linears of reverse_A0 / reverse_A1, compute_M0 / compute_M1).
 //
 // A row tile is 16 atoms with the same (l, m), so the 16 (l, m) of an atom are 16 tiles, and the accumulators of one
-// wavefront (16 columns, 16 tiles) hold all 16 variables of an (atom, channel) in the registers of one lane: the polynomial of
-// the contraction is evaluated where the product left its variables.  A separate contraction launch read and wrote them once
+// wavefront (16 columns, 16 or 8 of the tiles) hold the variables of an (atom, channel) in the registers of one lane: the polynomial
+// of the contraction is evaluated where the product left its variables.  A separate contraction launch read and wrote them once
 // more and was itself bound by that traffic and its ramp (3 000 atoms, 96 channels, fp64: 34 + 21 us for the two launches).
 //
 // A thread block takes 16 atoms (of one species where weights or polynomials depend on it) and WPB column tiles, one per
@@ -53,25 +53,136 @@ __device__ __forceinline__ void load_into_lds(const void* from, unsigned to)
 template <int N>
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory"); }
 
+// The (l, m) that a wavefront takes: l = 0 and 3 (set 0) or l = 1 and 2 (set 1), eight each, or all 16 (set 2).
+constexpr int slots_of(int set) { return set == 2 ? 16 : 8; }
+constexpr int num_l(int set) { return set == 2 ? 4 : 2; }
+constexpr int l_of(int set, int j) { return set == 2 ? j : (set == 0 ? 3 * j : 1 + j); }
+constexpr int lm_of(int set, int slot) { return set == 2 ? slot : (set == 0 ? (slot == 0 ? 0 : 8 + slot) : 1 + slot); }
+
+// The product of a wavefront: 16 atoms, 16 columns, a set of (l, m).
+//   STAGED  (l, m) whose rows the block brings to LDS: those of the set, or all 16
+template <typename F, int WPB, int SET, int STAGED, bool SCALED>
+struct SetProduct {
+    using Op = MatOp<F>;
+    static constexpr int V = 16 / (int)sizeof(F), KC = 4 * V;      // elements per 16 bytes, per piece
+    static constexpr int PIECE = STAGED * 1024, AHEAD = 2, BUFS = AHEAD + 1, ROUNDS = (STAGED + WPB - 1) / WPB;
+    static constexpr int NL = num_l(SET), NS = slots_of(SET);
+    static constexpr int LOADS = ROUNDS + NL + (SCALED ? 1 : 0);     // of a wavefront per piece
+    typedef F VV __attribute__((ext_vector_type(V)));
+
+    template <typename NodeOf>
+    __device__ static __forceinline__ void run(const LinearParams<F>& p, unsigned char* lds, int wave, int lane, int ct, int e, int type,
+                                               NodeOf node_of, typename Op::acc_t (&acc)[NS])
+    {
+        const int r16 = lane & 15, g = lane >> 4;
+        int steps[4];                             // pieces per l
+#pragma unroll
+        for (int l = 0; l < 4; ++l) steps[l] = e < p.num_e[l] ? p.inner[l] / KC : 0;
+        const int nsteps = STAGED == 16 ? max(max(steps[0], steps[1]), max(steps[2], steps[3])) : max(steps[l_of(SET, 0)], steps[l_of(SET, 1)]);
+
+        // rows into LDS: a load instruction brings 1 KB, the pieces of 16 atoms for one (l, m)
+        const F* const from = p.A + (size_t)node_of(lane / 4) * p.a_node_stride + part_of(lane % 4, lane / 4) * V;
+        const unsigned lds0 = (unsigned)(unsigned long long)(__attribute__((address_space(3))) unsigned char*)lds;
+        int row_at[ROUNDS], row_off[ROUNDS], row_last[ROUNDS];      // (places left over repeat the last (l, m))
+#pragma unroll
+        for (int u = 0; u < ROUNDS; ++u) {
+            const int at = min(u * WPB + wave, STAGED - 1);
+            const int lm = STAGED == 16 ? at : lm_of(SET, at);
+            row_at[u] = at; row_off[u] = p.row_off[lm];
+            row_last[u] = max((lm < 1 ? steps[0] : (lm < 4 ? steps[1] : (lm < 9 ? steps[2] : steps[3]))) - 1, 0);
+        }
+        auto stage = [&](int c, int slot) {
+#pragma unroll
+            for (int u = 0; u < ROUNDS; ++u)
+                load_into_lds(from + row_off[u] + min(c, row_last[u]) * KC, lds0 + slot * PIECE + row_at[u] * 1024);
+        };
+        VV b[BUFS][NL], sc[BUFS];      // weights (and factors) of this piece and the AHEAD next ones
+        const F* w_lane[NL];
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            const int l = l_of(SET, j);
+            w_lane[j] = p.W + p.w_off[l] + (size_t)type * p.w_type_stride[l] +
+                        ((size_t)(min(e, p.num_e[l] - 1) * (p.K / 16) + ct) * (p.inner[l] / KC) * 64 + lane) * V;
+        }
+        const F* s_lane = SCALED ? p.scale + (size_t)node_of(r16) * p.K + g * V : nullptr;
+        auto request = [&](int c, VV (&w)[NL], VV& f) {
+#pragma unroll
+            for (int j = 0; j < NL; ++j)
+                w[j] = *reinterpret_cast<const VV*>(w_lane[j] + (size_t)max(min(c, steps[l_of(SET, j)] - 1), 0) * 64 * V);
+            if constexpr (SCALED) f = *reinterpret_cast<const VV*>(s_lane + c * KC);
+        };
+#pragma unroll
+        for (int q = 0; q < NS; ++q) acc[q] = {0, 0, 0, 0};
+        static_for<0, AHEAD>([&](auto cc) {
+            constexpr int c = decltype(cc)::value;
+            request(min(c, nsteps - 1), b[c], sc[c]);
+            stage(min(c, nsteps - 1), c);
+        });
+        auto step = [&](int c, auto slot_c) {
+            constexpr int slot = decltype(slot_c)::value, ahead = (slot + AHEAD) % BUFS;
+            // the piece requested AHEAD steps ago is in LDS for everybody after this, and everybody has read the piece of the step
+            // before, whose slot the next request overwrites (no __syncthreads: its fence would wait for the younger pieces too)
+            wait_loads<(AHEAD - 1) * LOADS>();
+#pragma unroll
+            for (int j = 0; j < NL; ++j) asm volatile("" : "+v"(b[slot][j]));      // (here, not after the requests below)
+            if constexpr (SCALED) asm volatile("" : "+v"(sc[slot]));
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            request(min(c + AHEAD, nsteps - 1), b[ahead], sc[ahead]);
+            stage(min(c + AHEAD, nsteps - 1), ahead);
+            const unsigned char* buf = lds + slot * PIECE + r16 * 64 + part_of(g, r16) * 16;
+            static_for<0, NL>([&](auto jc) {
+                constexpr int j = decltype(jc)::value, l = l_of(SET, j);
+                if (c < steps[l]) {
+                    static_for<0, NS>([&](auto qc) {
+                        constexpr int q = decltype(qc)::value, lm = lm_of(SET, q);
+                        if constexpr (lm_l(lm) == l) {
+                            VV a = *reinterpret_cast<const VV*>(buf + (STAGED == 16 ? lm : q) * 1024);
+                            if constexpr (SCALED) a *= sc[slot];
+#pragma unroll
+                            for (int t = 0; t < V; ++t) acc[q] = Op::run(a[t], b[slot][j][t], acc[q]);
+                        }
+                    });
+                }
+            });
+            asm volatile("" ::: "memory");
+        };
+        // BUFS steps a round, so that the registers of a piece are the same ones from its request to its use (steps past the last
+        // one multiply nothing), and one way out of the loop, so that the waits need not allow for others
+        for (int c = 0; c < nsteps; c += BUFS)
+            static_for<0, BUFS>([&](auto sl) { step(c + decltype(sl)::value, sl); });
+        wait_loads<0>();      // the pieces requested past the end land before the LDS changes hands
+    }
+};
+
 // POLY: linear and contraction (one polynomial per channel, with gradients); else the linear alone.  (With several polynomials
 // per channel, values only, a launch of their own came out ahead: the 4 to 9 polynomials of the four atoms of a lane in turn are a
 // long chain for the few wavefronts here.)
-template <typename F, int WPB, bool POLY, bool SCALED>
+//
+// A wavefront takes half of the (l, m), eight tiles: with all 16, a few thousand atoms give the SIMDs one or two wavefronts each,
+// and 3 000 atoms with 96 channels (1 128 wavefronts, 1 024 SIMDs) twice the time of an even share.  Half the registers also
+// leaves room for more blocks, whose stores and first loads then go on under the products of others (those were 20 to 25 % of the
+// time each).  All 16, and now, us: 3 000 atoms, 96 channels, double, with a contraction 51 / 42, without 42 / 32; 20 011 atoms,
+// single 133 / 111 and 108 / 96; 24 999 atoms, 128 channels, double, without 302 / 268; 50 000 atoms, single, the same 320 / 329.
+// Without the contraction the
+// halves are blocks of their own, which stage the rows of their half only.  With it both are in one block, and trade variables
+// through LDS.  Many atoms whose channels are multiples of 64 keep all 16 (l, m) with a contraction behind them (SPLIT false,
+// launch_linear): such a block stages rows for twice the columns.
+template <typename F, int WPB, bool POLY, bool SCALED, bool SPLIT>
 __global__ __launch_bounds__(64 * WPB, 2) void k_linear(const LinearParams<F> p)
 {
+    static_assert(SPLIT || POLY, "halves without a contraction");
     using Op = MatOp<F>;
-    constexpr int V = 16 / (int)sizeof(F), KC = 4 * V;      // elements per 16 bytes, per piece
-    constexpr int PIECE = 256 * 64, AHEAD = 2, BUFS = AHEAD + 1;
-    constexpr int LOADS = (16 + WPB - 1) / WPB + 4 + (SCALED ? 1 : 0);     // of a wavefront per piece
-    typedef F VV __attribute__((ext_vector_type(V)));
-    extern __shared__ __align__(16) unsigned char lin_lds[];      // [BUFS][16 (l, m)][16 atoms][64]; later the coefficients
+    constexpr int V = 16 / (int)sizeof(F), CT = POLY && SPLIT ? WPB / 2 : WPB, SETS = POLY ? 1 : 2;      // column tiles, blocks for the sets
+    extern __shared__ __align__(16) unsigned char lin_lds[];      // [BUFS][8 or 16 (l, m)][16 atoms][64]; later the coefficients
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
 
-    // Block -> (row tile, column block, output block e): the blocks that share rows are eight apart, on one die.
-    const int cols = p.K / (16 * WPB), per = cols * p.num_e_max;
+    // Block -> (row tile, column block, output block e, set): the blocks that share rows are eight apart, on one die.
+    const int cols = p.K / (16 * CT), per = cols * p.num_e_max * SETS;
     const int rem = blockIdx.x % (8 * per), tile_index = blockIdx.x / (8 * per) * 8 + rem % 8;
-    const int cb = rem / 8 % cols, e = rem / 8 / cols;
+    const int cb = rem / 8 % cols, e = rem / 8 / cols % p.num_e_max;
+    const int set = !SPLIT ? 2 : (POLY ? wave & 1 : rem / 8 / cols / p.num_e_max);
     int type = 0, tile = tile_index, seg0 = 0, seg_n = p.num_nodes;
     if (p.perm) {
         const RowTile at = row_tile(p.tstart, p.T, tile_index, lane);
@@ -80,88 +191,18 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_linear(const LinearParams<F> p)
     } else if (tile * 16 >= seg_n) {
         return;
     }
+    if (!POLY && (set == 0 ? e >= p.num_e[0] && e >= p.num_e[3] : e >= p.num_e[1] && e >= p.num_e[2])) return;
     // atom a of the tile; beyond the segment the last atom again, whose results are not stored
     auto node_of = [&](int a) {
         const int j = min(tile * 16 + a, seg_n - 1);
         return p.perm ? p.perm[seg0 + j] : j;
     };
-    const int ct = cb * WPB + wave;           // column tile of this wavefront
-    int steps[4];                             // pieces per l
-#pragma unroll
-    for (int l = 0; l < 4; ++l) steps[l] = e < p.num_e[l] ? p.inner[l] / KC : 0;
-    const int nsteps = max(max(steps[0], steps[1]), max(steps[2], steps[3]));
+    const int tile_in_block = POLY && SPLIT ? wave >> 1 : wave, ct = cb * CT + tile_in_block, col = ct * 16 + r16;      // column tile, column
+    typename Op::acc_t acc[SPLIT ? 8 : 16];
+    if constexpr (!SPLIT) SetProduct<F, WPB, 2, 16, SCALED>::run(p, lin_lds, wave, lane, ct, e, type, node_of, acc);
+    else if (set == 0) SetProduct<F, WPB, 0, POLY ? 16 : 8, SCALED>::run(p, lin_lds, wave, lane, ct, e, type, node_of, acc);
+    else SetProduct<F, WPB, 1, POLY ? 16 : 8, SCALED>::run(p, lin_lds, wave, lane, ct, e, type, node_of, acc);
 
-    // rows into LDS: a load instruction brings 1 KB, the pieces of 16 atoms for one (l, m)
-    const F* const from = p.A + (size_t)node_of(lane / 4) * p.a_node_stride + part_of(lane % 4, lane / 4) * V;
-    const unsigned lds0 = (unsigned)(unsigned long long)(__attribute__((address_space(3))) unsigned char*)lin_lds;
-    constexpr int ROUNDS = (16 + WPB - 1) / WPB;
-    int row_lm[ROUNDS], row_off[ROUNDS], row_last[ROUNDS];      // (places left over repeat the last (l, m))
-#pragma unroll
-    for (int u = 0; u < ROUNDS; ++u) {
-        const int lm = min(u * WPB + wave, 15);
-        row_lm[u] = lm; row_off[u] = p.row_off[lm];
-        row_last[u] = max((lm < 1 ? steps[0] : (lm < 4 ? steps[1] : (lm < 9 ? steps[2] : steps[3]))) - 1, 0);
-    }
-    auto stage = [&](int c, int slot) {
-#pragma unroll
-        for (int u = 0; u < ROUNDS; ++u)
-            load_into_lds(from + row_off[u] + min(c, row_last[u]) * KC, lds0 + slot * PIECE + row_lm[u] * 1024);
-    };
-    VV b[BUFS][4], sc[BUFS];      // weights (and factors) of this piece and the AHEAD next ones
-    const F* w_lane[4];
-#pragma unroll
-    for (int l = 0; l < 4; ++l)
-        w_lane[l] = p.W + p.w_off[l] + (size_t)type * p.w_type_stride[l] +
-                    ((size_t)(min(e, p.num_e[l] - 1) * (p.K / 16) + ct) * (p.inner[l] / KC) * 64 + lane) * V;
-    const F* s_lane = SCALED ? p.scale + (size_t)node_of(r16) * p.K + g * V : nullptr;
-    auto request = [&](int c, VV (&w)[4], VV& f) {
-#pragma unroll
-        for (int l = 0; l < 4; ++l) w[l] = *reinterpret_cast<const VV*>(w_lane[l] + (size_t)max(min(c, steps[l] - 1), 0) * 64 * V);
-        if constexpr (SCALED) f = *reinterpret_cast<const VV*>(s_lane + c * KC);
-    };
-
-    typename Op::acc_t acc[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = {0, 0, 0, 0};
-    static_for<0, AHEAD>([&](auto cc) {
-        constexpr int c = decltype(cc)::value;
-        request(min(c, nsteps - 1), b[c], sc[c]);
-        stage(min(c, nsteps - 1), c);
-    });
-    auto step = [&](int c, auto slot_c) {
-        constexpr int slot = decltype(slot_c)::value, ahead = (slot + AHEAD) % BUFS;
-        // the piece requested AHEAD steps ago is in LDS for everybody after this, and everybody has read the piece of the step
-        // before, whose slot the next request overwrites (no __syncthreads: its fence would wait for the younger pieces too)
-        wait_loads<(AHEAD - 1) * LOADS>();
-#pragma unroll
-        for (int l = 0; l < 4; ++l) asm volatile("" : "+v"(b[slot][l]));      // (here, not after the requests below)
-        if constexpr (SCALED) asm volatile("" : "+v"(sc[slot]));
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        request(min(c + AHEAD, nsteps - 1), b[ahead], sc[ahead]);
-        stage(min(c + AHEAD, nsteps - 1), ahead);
-        const unsigned char* buf = lin_lds + slot * PIECE + r16 * 64 + part_of(g, r16) * 16;
-        static_for<0, 4>([&](auto lc) {
-            constexpr int l = decltype(lc)::value;
-            if (c < steps[l]) {
-                static_for<l * l, (l + 1) * (l + 1)>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value;
-                    VV a = *reinterpret_cast<const VV*>(buf + q * 1024);
-                    if constexpr (SCALED) a *= sc[slot];
-#pragma unroll
-                    for (int t = 0; t < V; ++t) acc[q] = Op::run(a[t], b[slot][l][t], acc[q]);
-                });
-            }
-        });
-        asm volatile("" ::: "memory");
-    };
-    // BUFS steps a round, so that the registers of a piece are the same ones from its request to its use (steps past the last
-    // one multiply nothing), and one way out of the loop, so that the waits need not allow for others
-    for (int c = 0; c < nsteps; c += BUFS)
-        static_for<0, BUFS>([&](auto sl) { step(c + decltype(sl)::value, sl); });
-    wait_loads<0>();      // the pieces requested past the end land before the LDS changes hands
-
-    const int col = ct * 16 + r16;
     int node[4];
     bool live[4];
 #pragma unroll
@@ -171,37 +212,72 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_linear(const LinearParams<F> p)
         live[r] = tile * 16 + atom < seg_n;
     }
     if constexpr (!POLY) {
+        auto store = [&](auto set_c) {
+            constexpr int SET = decltype(set_c)::value;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (live[r]) {
-                F* o = p.out + (size_t)node[r] * p.out_node_stride + (size_t)e * p.K + col;
-                static_for<0, 16>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value, l = lm_l(q);
-                    if (e < p.num_e[l]) o[p.out_off[q]] = acc[q][r];
-                });
-            }
+            for (int r = 0; r < 4; ++r)
+                if (live[r]) {
+                    F* o = p.out + (size_t)node[r] * p.out_node_stride + (size_t)e * p.K + col;
+                    static_for<0, 8>([&](auto qc) {
+                        constexpr int q = decltype(qc)::value, lm = lm_of(SET, q), l = lm_l(lm);
+                        if (e < p.num_e[l]) o[p.out_off[lm]] = acc[q][r];
+                    });
+                }
+        };
+        if (set == 0) store(std::integral_constant<int, 0>{}); else store(std::integral_constant<int, 1>{});
     }
     if constexpr (POLY) {
+        // With halves, the two wavefronts of a column tile trade variables: the one ends with all 16 of a lane's atoms 0 and 1, the
+        // other with those of atoms 2 and 3.
+        constexpr int ATOMS = SPLIT ? 2 : 4;
+        F x[ATOMS][16];
+        if constexpr (SPLIT) {
+            F* const mine = reinterpret_cast<F*>(lin_lds) + (size_t)wave * 16 * 64 + lane;
+            const F* const other = reinterpret_cast<const F*>(lin_lds) + (size_t)(wave ^ 1) * 16 * 64 + lane;
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                mine[(2 * q) * 64] = set == 0 ? acc[q][2] : acc[q][0];
+                mine[(2 * q + 1) * 64] = set == 0 ? acc[q][3] : acc[q][1];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const F here = set == 0 ? acc[q][t] : acc[q][2 + t], there = other[(2 * q + t) * 64];
+                    x[t][lm_of(0, q)] = set == 0 ? here : there;
+                    x[t][lm_of(1, q)] = set == 0 ? there : here;
+                }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 16; ++q)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) x[t][q] = acc[q][t];
+        }
         // coefficients of this block's channels: [column tile][16-byte group of monomials][16 channels]
         constexpr int G16 = poly_spec_padded(PolyTable<0>::N) / V;
         __syncthreads();
         {
-            const uint4* src = reinterpret_cast<const uint4*>(p.coef) + ((size_t)type * (p.K / 16) + ct) * G16 * 16;
-            uint4* dst = reinterpret_cast<uint4*>(lin_lds) + (size_t)wave * G16 * 16;
-            for (int t = lane; t < G16 * 16; t += 64) dst[t] = src[t];
+            const uint4* src = reinterpret_cast<const uint4*>(p.coef) + ((size_t)type * (p.K / 16) + cb * CT) * G16 * 16;
+            uint4* dst = reinterpret_cast<uint4*>(lin_lds);
+            for (int t = tid; t < CT * G16 * 16; t += 64 * WPB) dst[t] = src[t];
         }
-        wave_lds_sync();      // a wavefront reads its own column tile only
-        const unsigned char* slab = lin_lds + (size_t)wave * G16 * 256 + r16 * 16;
-        for (int r = 0; r < 4; ++r) {
-            F x[16], gr[16], f = F(0);
+        __syncthreads();
+        const unsigned char* slab = lin_lds + (size_t)tile_in_block * G16 * 256 + r16 * 16;
+        const int first = SPLIT && set == 1 ? 2 : 0;
+#pragma unroll 1
+        for (int t = 0; t < ATOMS; ++t) {
+            F v[16], gr[16], f = F(0);
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
-                x[q] = r == 0 ? acc[q][0] : (r == 1 ? acc[q][1] : (r == 2 ? acc[q][2] : acc[q][3]));
+                v[q] = t == 0 ? x[0][q] : (t == 1 ? x[1][q] : (t == 2 ? x[ATOMS - 2][q] : x[ATOMS - 1][q]));
                 gr[q] = F(0);
             }
+            const int r = first + t;
             const int nd = r == 0 ? node[0] : (r == 1 ? node[1] : (r == 2 ? node[2] : node[3]));
             const bool lv = r == 0 ? live[0] : (r == 1 ? live[1] : (r == 2 ? live[2] : live[3]));
-            poly_spec_body<F, 0, 0>(slab, 256, x, gr, f, F(1));
+            poly_spec_body<F, 0, 0>(slab, 256, v, gr, f, F(1));
             if (lv) {
                 p.M[(size_t)nd * p.K + col] = f;
 #pragma unroll
@@ -211,35 +287,44 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_linear(const LinearParams<F> p)
     }
 }
 
-template <typename F, int WPB, bool POLY, bool SCALED>
+template <typename F, int WPB, bool POLY, bool SCALED, bool SPLIT = true>
 hipError_t launch_linear_t(const LinearParams<F>& p, hipStream_t s)
 {
-    size_t lds = 3 * (size_t)256 * 64;
-    if (POLY) lds = std::max(lds, (size_t)WPB * poly_spec_padded(kPolyTableLen[0]) * 16 * sizeof(F));
+    constexpr int CT = POLY && SPLIT ? WPB / 2 : WPB;
+    size_t lds = 3 * (size_t)(POLY ? 16 : 8) * 1024;
+    if (POLY) lds = std::max({lds, (size_t)CT * poly_spec_padded(kPolyTableLen[0]) * 16 * sizeof(F), (size_t)WPB * 16 * 64 * sizeof(F)});
     const long tiles = ((long)p.num_nodes + 15) / 16 + (p.perm ? p.T : 0);
-    const long blocks = (tiles + 7) / 8 * 8 * (p.K / (16 * WPB)) * p.num_e_max;
+    const long blocks = (tiles + 7) / 8 * 8 * (p.K / (16 * CT)) * p.num_e_max * (POLY ? 1 : 2);
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
     if (lds > 64 * 1024) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_linear<F, WPB, POLY, SCALED>), dim3((unsigned)blocks), dim3(64 * WPB), lds, s, p);
+    hipLaunchKernelGGL((k_linear<F, WPB, POLY, SCALED, SPLIT>), dim3((unsigned)blocks), dim3(64 * WPB), lds, s, p);
     return hipGetLastError();
 }
 
 }  // namespace
 
-// Column tiles of a block: all that divide evenly, up to four (48 KB of LDS a block: three blocks on a CU).
+// Column tiles of a block: all that divide evenly, up to four (24 KB of LDS a block); with a contraction two, each with both halves
+// of the (l, m), or four without halves.
 template <typename F>
 hipError_t launch_linear(const LinearParams<F>& p, hipStream_t s)
 {
     if (p.num_nodes <= 0) return hipSuccess;
     if (!linear_ok(p.K) || p.T <= 0 || (p.coef && (p.scale || p.num_e_max != 1))) return hipErrorInvalidValue;
-    auto go = [&](auto pc, auto sc) -> hipError_t {
-        constexpr bool POLY = decltype(pc)::value, SCALED = decltype(sc)::value;
-        if (p.K % 64 == 0) return launch_linear_t<F, 4, POLY, SCALED>(p, s);
-        if (p.K % 96 == 0) return launch_linear_t<F, 3, POLY, SCALED>(p, s);
-        return launch_linear_t<F, 2, POLY, SCALED>(p, s);
+    if (p.coef) {
+        // Blocks with all (l, m) once there are enough to even out over 256 CUs, which hold two (double) or three at a time: A1 of
+        // layers l <= 1 at 128 channels, halves / all: double 3 000 atoms 107 / 119 us, 9 000 276 / 305, 12 000 373 / 329,
+        // 24 999 770 / 710; single 3 000 62 / 68, 4 500 95 / 100, 6 000 118 / 106, 50 000 830 / 735.
+        const long whole = ((long)p.num_nodes + 15) / 16 * (p.K / 64);
+        if (p.K % 64 == 0 && whole > (sizeof(F) == 8 ? 1152 : 640)) return launch_linear_t<F, 4, true, false, false>(p, s);
+        return launch_linear_t<F, 4, true, false>(p, s);
+    }
+    auto go = [&](auto sc) -> hipError_t {
+        constexpr bool SCALED = decltype(sc)::value;
+        if (p.K % 64 == 0) return launch_linear_t<F, 4, false, SCALED>(p, s);
+        if (p.K % 96 == 0) return launch_linear_t<F, 3, false, SCALED>(p, s);
+        return launch_linear_t<F, 2, false, SCALED>(p, s);
     };
-    if (p.coef) return go(std::true_type{}, std::false_type{});
-    return p.scale ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+    return p.scale ? go(std::true_type{}) : go(std::false_type{});
 }
 
 #ifndef SMX_LINEAR_PART
