@@ -235,7 +235,6 @@ struct Engine : EngineBase {
     // ---- model on device
     DVec<F> tab0, tab1, tabK0, tabK1, H0, A0w, H1w, A1w;
     DVec<F> linA0, linA0T, linA1, linA1T;    // the same weights in operand order (operand_weights)
-    DVec<F> M0_coef16, M1_coef16;            // contraction coefficients by column tile
     DVec<F> H1wT;                            // transposes, for the kernels that take a chain of stages
     DVec<int> pair_table0, pair_table1;
     DVec<int> B0_start, B0_lm1, B1_start, B1_lm1;
@@ -261,7 +260,7 @@ struct Engine : EngineBase {
     DVec<const int4*> pp_packed;
     DVec<const int*> pp_chunks;
     DVec<const F*> pp_coef;
-    DVec<F> M0_slabs, M1_slabs;   // coefficients of the straight-line contraction kernel (poly_spec_shape layout)
+    DVec<F> M0_slabs, M1_slabs;   // contraction coefficients by column tile (smx_poly_shape.hpp)
     DVec<int> pp_nent;
     bool M0_tables = false, M1_tables = false;   // every polynomial of the layer maps onto its compile-time table
 
@@ -465,20 +464,18 @@ struct Engine : EngineBase {
         M1_tables = hm.P1.table == 0;
         M0_tables = M0_tables && poly_spec_shape((int)sizeof(F), hm.K, hm.num_LM).CB > 0;
         M1_tables = M1_tables && poly_spec_shape((int)sizeof(F), hm.K, 1).CB > 0;
-        // slabs of the straight-line kernel: [species][channel block][monomial / V][CB][V]
-        auto slabs = [&](DVec<F>& dst, const PolySpec* polys, int NP, bool by_column_tile) {
-            PolySpecShape sh = poly_spec_shape((int)sizeof(F), hm.K, NP);
-            if (by_column_tile) { sh.CB = 16; sh.kblocks = hm.K / 16; sh.slab_bytes = (unsigned)(poly_spec_offset(NP) * 16 * sizeof(F)); }
+        // slabs of the straight-line polynomials: [species][column tile][monomial / V][16][V]
+        auto slabs = [&](DVec<F>& dst, const PolySpec* polys, int NP) {
             constexpr int V = 16 / (int)sizeof(F);
-            const size_t slab = sh.slab_bytes / sizeof(F);
-            std::vector<F> h((size_t)hm.T * sh.kblocks * slab, F(0));
+            const size_t tiles = (size_t)(hm.K + 15) / 16, slab = (size_t)poly_spec_offset(NP) * 16;
+            std::vector<F> h((size_t)hm.T * tiles * slab, F(0));
             for (int P = 0; P < NP; ++P) {
                 const int tn = kPolyTableLen[polys[P].table], m0 = poly_spec_offset(P);
                 for (int t = 0; t < hm.T; ++t)
                     for (int i = 0; i < tn; ++i)
                         for (int k = 0; k < hm.K; ++k) {
-                            const int m = m0 + i, kb = k / sh.CB, kloc = k % sh.CB;
-                            h[((size_t)t * sh.kblocks + kb) * slab + ((size_t)(m / V) * sh.CB + kloc) * V + m % V] =
+                            const int m = m0 + i;
+                            h[((size_t)t * tiles + k / 16) * slab + ((size_t)(m / V) * 16 + k % 16) * V + m % V] =
                                 (F)polys[P].table_coef[((size_t)t * tn + i) * hm.K + k];
                         }
             }
@@ -490,12 +487,10 @@ struct Engine : EngineBase {
             HIPCHK(hipGetDeviceProperties(&prop, device));
             num_cus = prop.multiProcessorCount;
         }
-        if (M0_tables) slabs(M0_slabs, hm.P0.data(), hm.num_LM, false);
-        if (M1_tables) slabs(M1_slabs, &hm.P1, 1, false);
+        if (M0_tables) slabs(M0_slabs, hm.P0.data(), hm.num_LM);
+        if (M1_tables) slabs(M1_slabs, &hm.P1, 1);
         if (linear_ok(hm.K)) {
             const bool chain = chain_ok(hm.K) && M0_tables && M1_tables;
-            if (M0_tables && (hm.num_LM == 1 || chain)) slabs(M0_coef16, hm.P0.data(), hm.num_LM, true);
-            if (M1_tables) slabs(M1_coef16, &hm.P1, 1, true);
             operand_weights(s);
             if (chain) {
                 auto transposed = [&](const std::vector<double>& w, auto& dst) {
@@ -903,7 +898,7 @@ struct Engine : EngineBase {
         if (nlm == 1) M0_grad.size_to((size_t)N * 16 * k, stream);
         if (H1.n != M0.n) H1.resize(M0.n, stream);   // mace.cpp:400
         auto p = chain_params(N);
-        p.Phi = Phi0.p; p.W = linA0.p; p.WH1 = H1w.p; p.coef = M0_coef16.p;
+        p.Phi = Phi0.p; p.W = linA0.p; p.WH1 = H1w.p; p.coef = M0_slabs.p;
         p.A = A0.p; p.M = M0.p; p.M_grad = M0_grad.p; p.H1 = H1.p;
         HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain0<F, decltype(kc)::value>(p, hm.L_max, stream); }));
         if (nlm == 1) pending_A0 = N;
@@ -916,7 +911,7 @@ struct Engine : EngineBase {
         M1.size_to((size_t)N * k, stream); M1_grad.size_to((size_t)N * 16 * k, stream);
         dPhi1.size_to(Phi1.n, stream);
         auto p = chain_params(N);
-        p.Phi = Phi1.p; p.W = linA1.p; p.Wt = linA1T.p; p.coef = M1_coef16.p;
+        p.Phi = Phi1.p; p.W = linA1.p; p.Wt = linA1T.p; p.coef = M1_slabs.p;
         p.M = M1.p; p.M_grad = M1_grad.p; p.out = dPhi1.p;
         const auto q = tail_params(N, zero_energies);
         HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain1<F, decltype(kc)::value>(p, q, hm.L_max, stream); }));
@@ -933,7 +928,7 @@ struct Engine : EngineBase {
         to.size_to((size_t)N * 16 * k, stream);
         if (add_messages && sender_rows != N) build_sender_lists(N);
         auto p = chain_params(N);
-        p.Wt = linA0T.p; p.WH1 = H1wT.p; p.coef = M0_coef16.p; p.A = A0.p; p.M = M0_adj.p; p.M_grad = M0_grad.p; p.out = to.p;
+        p.Wt = linA0T.p; p.WH1 = H1wT.p; p.coef = M0_slabs.p; p.A = A0.p; p.M = M0_adj.p; p.M_grad = M0_grad.p; p.out = to.p;
         p.msg = add_messages ? msg.p : nullptr; p.H1_adj = H1_adj.p; p.sstart = s_start.p; p.slist = s_list.p; p.spare = s_rank.p;
         HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain2<F, decltype(kc)::value>(p, hm.L_max, stream); }));
         pending_A0_adj = N;
@@ -947,7 +942,7 @@ struct Engine : EngineBase {
         (layer == 0 ? A0 : A1).size_to((size_t)N * 16 * k, stream);
         M.size_to((size_t)N * k, stream); M_grad.size_to((size_t)N * 16 * k, stream);
         auto q = layer == 0 ? linear_A0(N, false) : linear_A1(N, false, true);
-        q.A = layer == 0 ? Phi0.p : Phi1.p; q.coef = layer == 0 ? M0_coef16.p : M1_coef16.p;
+        q.A = layer == 0 ? Phi0.p : Phi1.p; q.coef = layer == 0 ? M0_slabs.p : M1_slabs.p;
         q.M = M.p; q.M_grad = M_grad.p;
         HIPCHK(launch_linear<F>(q, stream));
         (layer == 0 ? pending_A0 : pending_A1) = N;

@@ -183,7 +183,12 @@ PolySpec build_poly(int num_lm, int T, int K, const std::vector<std::vector<int>
     const unsigned char (*tab)[3] = poly_table(canon_table, &tn);
     if (tab) {
         std::map<std::tuple<int, int, int>, int> where;
-        for (int i = 0; i < tn; ++i) where[std::make_tuple((int)tab[i][0], (int)tab[i][1], (int)tab[i][2])] = i;
+        for (int i = 0; i < tn; ++i) {
+            // a file's monomials have the constant (16) in front, then their variables in ascending order
+            int key[3] = {tab[i][0], tab[i][1], tab[i][2]};
+            std::sort(key, key + 3, [](int a, int b) { return (a + 1) % 17 < (b + 1) % 17; });
+            where[std::make_tuple(key[0], key[1], key[2])] = i;
+        }
         std::vector<int> slot(ents.size(), -1);
         bool inside = true;
         for (size_t i = 0; i < ents.size() && inside; ++i) {

@@ -275,11 +275,11 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain0(
         F x[16], gr[16], f = F(0);
 #pragma unroll
         for (int q = 0; q < 16; ++q) { x[q] = *reinterpret_cast<const F*>(smem + q * RS + k * sizeof(F)); gr[q] = F(0); }
-        if constexpr (lm == 0) poly_spec_run<F, 0, LH == 0 ? 0 : 1>(first, x, gr, f, F(1));
+        if constexpr (lm == 0) poly_spec_run<F, 0, LH == 0 ? 0 : 1, false>(first, x, gr, f, F(1));
         else {
             Coef<F, lm> next(coef, 256);
             next.begin();
-            poly_spec_run<F, lm, 1>(next, x, gr, f, F(1));
+            poly_spec_run<F, lm, 1, false>(next, x, gr, f, F(1));
         }
         if (!own) return;
         xm[k * NP + lm] = f;
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
         F x[16], f = F(0);
 #pragma unroll
         for (int i = 0; i < 16; ++i) { x[i] = *reinterpret_cast<const F*>(smem + i * RS + k * sizeof(F)); gr[i] = F(0); }
-        poly_spec_run<F, 0, 0>(coef, x, gr, f, F(1));
+        poly_spec_run<F, 0, 0, false>(coef, x, gr, f, F(1));
         xh[K + k] = (double)f;
         p.M[node * K + k] = f;
 #pragma unroll
@@ -603,7 +603,7 @@ __global__ __launch_bounds__(chain_threads(K), LH == 0 ? chain_waves<F>(K) : 4) 
                 asm volatile("" ::: "memory");      // (the coefficients of the other polynomials stay where they are)
                 Coef<F, lm, 2> coef(coefficients<F, K>(p.coef, poly_spec_offset(NP) / V, b.type, k), 256);
                 coef.begin();
-                poly_spec_run<F, lm, 2>(coef, x, gr, f, ym[k * NP + lm]);
+                poly_spec_run<F, lm, 2, false>(coef, x, gr, f, ym[k * NP + lm]);
             });
 #pragma unroll
             for (int i = 0; i < 16; ++i) part[(slot * 16 + i) * K + k] = gr[i];

@@ -14,12 +14,17 @@ namespace {
 // For harmonics up to l = 3 and correlation order 3 the monomials of output slot LM are a compile-time table
 // (smx_poly_tables.inc), so the walk is straight-line code and the 16 variables of an atom stay in registers -- no
 // index loads, no variables in LDS.  The LDS holds the coefficients instead: a block owns one species and one block
-// of CB channels, copies that slab ([monomials of all polynomials][CB], laid out by the loader as 16-byte groups per
-// channel, see poly_spec_shape) once and then takes a run of `chunk` atoms of the species, AG atoms at a time, one
-// thread per (atom, channel).  Per monomial x_a x_b x_c the thread forms w x_a and x_b x_c once; three multiply-adds
-// give the gradient terms (the product rule holds as written for repeated indices) and one more the value: six
-// instructions.  Used when every polynomial of the launch maps onto its table (the loader checks); other files take
-// the list-walking kernel of smx_kernels_node.hip.
+// of CB channels, copies that slab (whole column tiles of 16 channels, [monomials of all polynomials][16] each, see
+// smx_poly_shape.hpp) once and then takes a run of `chunk` atoms of the species, AG atoms at a time, one thread per (atom, channel).
+// Used when every polynomial of the launch maps onto its table (the loader checks); other files take the list-walking kernel of
+// smx_kernels_node.hip.
+//
+// Bound by the LDS (8 cycles per 16-byte read of a wavefront), the multiply-adds and the traffic of the variables about equally.
+// Nested polynomials (smx_poly_body.hpp) and slabs with offsets known to the compiler (which kept 30 address registers before, and
+// spilled), values / adjoints before and now, us: four polynomials, 128 channels, 50 000 atoms single 210 / 375 to 146 / 258,
+// 24 999 atoms double 207 / 384 to 134 / 235, 3 000 atoms double 58 / 99 to 40 / 66; nine polynomials, 3 000 atoms single 51 / 82
+// to 33 / 52.  Two atoms per thread, which share the coefficients they read: 131 / 240, 150 / 240 (double, the adjoints at half the
+// wavefronts), 38 / 66 and 32 / 51.
 constexpr int SPEC_BT = 256;     // threads per block
 
 template <typename F, int COUNT, int MODE>
@@ -38,7 +43,7 @@ __global__ __launch_bounds__(SPEC_BT, sizeof(F) == 8 ? 4 : 5) void k_poly_spec(c
     if (type < 0) return;
     {   // the slab of (species, channel block): contiguous, a multiple of 16 bytes
         const uint4* src = reinterpret_cast<const uint4*>(reinterpret_cast<const unsigned char*>(a.table_slabs) +
-                                                          ((size_t)type * sh.kblocks + kb) * sh.slab_bytes);
+                                                          ((size_t)type * sh.kblocks + kb) * sh.slab_bytes);      // (whole column tiles)
         uint4* dst = reinterpret_cast<uint4*>(spec_lds);
         const int n16 = (int)(sh.slab_bytes / 16);
         for (int i = tid; i < n16; i += SPEC_BT) dst[i] = src[i];
@@ -48,8 +53,7 @@ __global__ __launch_bounds__(SPEC_BT, sizeof(F) == 8 ? 4 : 5) void k_poly_spec(c
     const int k = kb * sh.CB + kloc;
     const bool klive = ag < sh.AG && k < a.K;
     const unsigned kk = k < a.K ? k : a.K - 1;
-    const unsigned char* slab_k = spec_lds + (size_t)kloc * 16;
-    const int row_stride = sh.CB * 16;
+    const unsigned char* slab_k = spec_lds + (kloc / 16) * (poly_spec_offset(COUNT) * 16 * (int)sizeof(F)) + kloc % 16 * 16;
     const int j0 = u * chunk, j1 = j0 + chunk < seg_n ? j0 + chunk : seg_n;
     for (int jb = j0; jb < j1; jb += sh.AG) {
         const int j = jb + ag;
@@ -72,7 +76,7 @@ __global__ __launch_bounds__(SPEC_BT, sizeof(F) == 8 ? 4 : 5) void k_poly_spec(c
 #pragma unroll
                 for (int q = 0; q < 16; ++q) g[q] = F(0);
             }
-            poly_spec_body<F, P, MODE>(slab_k, row_stride, x, g, f, madj);
+            poly_spec_body<F, P, MODE>(slab_k, 256, x, g, f, madj);
             madj = madj_next;
             if (live) {
                 if constexpr (MODE == 0) {

@@ -7,9 +7,10 @@
 namespace smx {
 
 // Coefficient slabs of the straight-line contraction kernel.  The monomials of polynomials 0..NP-1 follow one another,
-// each list padded with zero coefficients to a multiple of four; a slab holds them for one species and CB channels
-// as [monomial / V][CB][V], V = 16 / sizeof(F): a thread reads V coefficients of its channel with one 16-byte LDS
-// read, the lanes of a wavefront side by side.  The loader lays the coefficients out with the same function.
+// each list padded with zero coefficients to a multiple of four; a slab holds them for one species and the column tiles (16
+// channels) of a block as [column tile][monomial / V][16][V], V = 16 / sizeof(F): a thread reads V coefficients of its channel
+// with one 16-byte LDS read, 16 lanes side by side, at an offset that the compiler knows.  The loader lays the coefficients out with
+// the same function.
 constexpr int poly_spec_padded(int n) { return (n + 3) / 4 * 4; }
 constexpr int poly_spec_offset(int lm)   // padded monomials in front of polynomial lm (lm = NP: all of them)
 {
