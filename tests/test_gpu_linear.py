@@ -10,12 +10,12 @@ pytestmark = pytest.mark.gpu
 ARRAYS = ["M1", "M1_grad", "M1_adj", "A1_adj", "A0_adj", "H1", "H1_adj", "node_energies"]
 
 
-def _engine(tmp_models, K, L_max, dtype, T=(1, 6, 8)):
+def _engine(tmp_models, K, L_max, dtype, density=False):
     import torch
     assert torch.cuda.is_available()
     from symmetrix_amd.mace import MACE
-    model = H.tiny_model(K=K, L_max=L_max, T=T, n_pts=16, seed=K + L_max, r_cut=3.0, pair=False)
-    eng = MACE(H.write_model(model, tmp_models / f"linear_{K}_{L_max}.json"), dtype)
+    model = H.tiny_model(K=K, L_max=L_max, T=(1, 6, 8), n_pts=16 if not density else 48, seed=K + L_max, r_cut=3.0, pair=False, density=density)
+    eng = MACE(H.write_model(model, tmp_models / f"linear_{K}_{L_max}_{int(density)}.json"), dtype)
     eng.set_profiling(True)      # small systems would take chains of stages otherwise
     return model, eng
 
@@ -56,12 +56,13 @@ def test_both_kinds_of_wavefront(tmp_models, K, L_max, dtype, n):
 
 
 @pytest.mark.parametrize("dtype", ["float64", "float32"])
-@pytest.mark.parametrize("K,n", [(160, 17), (96, 33), (32, 16)])
-def test_against_the_oracle(tmp_models, K, n, dtype):
-    """Five pairs of column tiles (in pairs only), three tiles, one pair; rows of a tile left over and none."""
+@pytest.mark.parametrize("K,n,density", [(160, 17, False), (96, 33, False), (32, 16, False), (160, 9, True), (128, 20, True), (20, 7, True)])
+def test_against_the_oracle(tmp_models, K, n, density, dtype):
+    """Five pairs of column tiles (in pairs only), three tiles, one pair; rows of a tile left over and none.  With density
+    normalisation: rows of more, of exactly and of less than the 2 048 elements that a block takes at a time."""
     from oracle.oracle import OracleMACE
     from tests.test_gpu_parity import _compare
-    model, eng = _engine(tmp_models, K, 1, dtype)
+    model, eng = _engine(tmp_models, K, 1, dtype, density=density)
     pos, cell, sp = H.small_system(n, seed=n)
     nl, ea = H.edges_of(pos, cell, sp, model["r_cut"])
     orc = OracleMACE(model)
