@@ -74,9 +74,9 @@ def measured_traffic(workload, dtype, stage, kernel):
 
 MFMA_PEAK = {"float64": 78.6e12, "float32": 157.3e12}   # dense matrix-core peaks of MI355X, flop/s
 # kernel behind each dense stage (as the kernel trace names it) when it runs in feature precision F
-DENSE_KERNEL = {"A0_lin": r"k_linear<{F}, \d, {one}, false>", "A1": r"k_linear<{F}, \d, true, false>",
+DENSE_KERNEL = {"A0_lin": r"k_linear<{F}, \d, {one}, false, (true|false)>", "A1": r"k_linear<{F}, \d, true, false, (true|false)>",
                 "H1": r"k_gemm_rows<{F}, {F}, {F}, \d, false", "H2": r"k_tail_fused<{F}",
-                "rev_A1": r"k_linear<{F}, \d, false, true>", "rev_A0_lin": r"k_linear<{F}, \d, false, {one}>",
+                "rev_A1": r"k_linear<{F}, \d, false, true, true>", "rev_A0_lin": r"k_linear<{F}, \d, false, {one}, true>",
                 "rev_H1": r"k_gemm_rows<{F}, {F}, {F}, \d, false"}   # {one}: one polynomial per channel in layer 0
 
 
@@ -103,7 +103,7 @@ def contraction_work(n_atoms, K, L_max, layer, s_bytes, mode="both"):
     value only ("value") two products and one multiply-add (4; 3; 2); the adjoint that forms the gradient again
     ("adjoint") three products and three multiply-adds (9; 5; 2).  Bytes: the 16 variables in; out, per polynomial,
     the value ("both", "value") and its 16 gradient components ("both"); the adjoint reads the polynomials' adjoints
-    and writes 16 sums."""
+    and writes 16 sums.  (The kernel of several polynomials nests these sums and executes about 0.6 of the operations.)"""
     from symmetrix_amd import cg
     per_degree = {"both": {1: 3, 2: 7, 3: 10}, "value": {1: 2, 2: 3, 3: 4}, "adjoint": {1: 2, 2: 5, 3: 9}}[mode]
     flops_per = 0

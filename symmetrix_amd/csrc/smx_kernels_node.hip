@@ -258,7 +258,7 @@ __device__ void node_lists_part(const int* num_neigh, int N, int* first_neigh, c
 // senders (counters at zero on entry), which does not depend on the node lists.  With a ticket, the block that finishes last
 // turns the histogram into the sender offsets: a launch of its own costs 6 to 8 us of a small evaluation, but the fences of
 // the ticket cost more than that over many blocks (83 blocks, 3 000 atoms: 21 us with the ticket, 19 without; 80 us over 2 048),
-// so the launcher hands out tickets to small grids only.  Larger ones are bound by the atomics (50 000 atoms, 1.4 million
+// so the launcher hands out tickets to small grids only.  Larger ones are bound by the atomics (50 000 atoms, 3.9 million
 // edges: 92 us while one block each formed the node lists an element per thread at a time, now 60, the scan behind it 43 and
 // 14; 20 011 atoms 41 and 19, now 26 and 7).
 // With `chk.status` set the launch also checks everything the later kernels use as an address or a table argument
