@@ -8,7 +8,7 @@
 // All of them touch the rows of one atom only, so a thread block takes one atom through all of its stages, with everything
 // between them in LDS.  As launches of their own the stages of a small system were a row of dependent launches of 6 to 20 us,
 // each of which waited for its first loads and filled a few CUs: 24 atoms, 96 channels, double precision 96 us in eight launches,
-// now 9 + 18 + 11 (an evaluation 142, now 86); 107 atoms, 128 channels, l <= 1: 170 us in ten, now 17 + 42 + 34.
+// now 10 + 18 + 11; 107 atoms, 128 channels, l <= 1: 170 us in ten, now 17 + 43 + 33.
 // Bound by the weights, which every block reads once: 295 KB (96 channels, double, one A-basis product) at 64 bytes per cycle
 // and CU; between the products by the latency of dependent loads.
 //
