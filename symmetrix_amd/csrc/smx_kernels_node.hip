@@ -145,6 +145,7 @@ __device__ __forceinline__ void load_items(const int* in, int n, int i0, int bey
 }
 // species group t of a block of its own: where it begins (the number of atoms of smaller species), and its atoms in ascending
 // order.  (One block with counters in the LDS for all species took a serial chain of same-address atomics, two per atom.)
+// N > 0: without an element there is no round that fills v.
 template <int ITEMS>
 __device__ void type_group_items(const int* node_types, int N, int T, int t, int* tstart, int* perm)
 {
@@ -388,6 +389,7 @@ hipError_t launch_type_groups(const int* node_types, int N, int T, int* tcount, 
 {
     (void)tcount; (void)cursor; (void)block_sums;
     if (T <= 0) return hipSuccess;
+    if (N <= 0) return launch_fill<int>(tstart, (long)T + 1, 0, s);   // empty groups: the kernel needs an element to load
     hipLaunchKernelGGL(k_type_groups, dim3(T), dim3(SCAN_BLOCK), 0, s, node_types, N, T, tstart, perm);
     return hipGetLastError();
 }
