@@ -117,7 +117,8 @@ int smx_set_num_H1_rows(smx_model* m, int rows);
 /* Stage-level entry points, one per public method of class MACE
  * (mace.hpp:29-164).  Edge geometry is remembered from the last
  * smx_compute_Y (xyz) and smx_compute_R0/R1 (r, types), as the reference
- * remembers Y, R0 and R1. */
+ * remembers Y, R0 and R1.  An array of no elements (no nodes, no edges) may be
+ * NULL. */
 int smx_compute_Y(smx_model* m, const double* xyz, long n3);                             /* mace.cpp:118-148 */
 int smx_compute_R0(smx_model* m, int num_nodes, const int* node_types, const int* num_neigh,
                    const int* neigh_types, const double* r, long num_edges);            /* mace.cpp:66-90 */

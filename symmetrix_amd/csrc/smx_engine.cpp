@@ -1742,7 +1742,7 @@ struct Engine : EngineBase {
         if (atom_forces) {
             atoms = num_atoms;
             if (num_atoms <= 0) throw Error(SMX_EINVAL, "num_atoms must be positive");
-            if (!sender_atom) throw Error(SMX_EINVAL, "sender_atom is required");
+            if (!sender_atom && E > 0) throw Error(SMX_EINVAL, "sender_atom is required");
             if (receiver_atom) {
                 // receiver_atom[i] = atom row of receiver block i: the blocks of every atom, in ascending order
                 if (geo_edges != E) throw Error(SMX_EINVAL, "num_neigh of the last call does not cover every edge");
@@ -1903,6 +1903,16 @@ void require_device()
         throw smx::Error(SMX_ENODEVICE, std::string("kernels are built for gfx950 only; found ") + prop.gcnArchName);
     checked = dev;
 }
+
+// A stage call leaves the arrays it does not take (nullptr here) as they were.  An array without an element may come as a null
+// pointer (an empty vector's): it is there, and empty.
+template <typename T>
+const T* given(const T* p, long n)
+{
+    static const T none{};
+    return p || n != 0 ? p : &none;
+}
+std::nullptr_t given(std::nullptr_t, long) { return nullptr; }
 
 smx::EngineBase& E(smx_model* m)
 {
@@ -2371,7 +2381,8 @@ int smx_set_num_H1_rows(smx_model* m, int rows)
 }
 
 #define SMX_STAGE(fn, name, NT, NN, NI, NTY, XYZ, R, EE, FA, FB) \
-    return guarded([&] { auto& e = E(m); e.stream = nullptr; e.stage(name, num_nodes, NT, NN, NI, NTY, XYZ, R, EE, FA, FB); HIPCHK(hipStreamSynchronize(e.stream)); })
+    return guarded([&] { auto& e = E(m); e.stream = nullptr; e.stage(name, num_nodes, given(NT, num_nodes), given(NN, num_nodes), given(NI, EE), \
+        given(NTY, EE), given(XYZ, EE), given(R, EE), EE, FA, FB); HIPCHK(hipStreamSynchronize(e.stream)); })
 
 int smx_compute_Y(smx_model* m, const double* xyz, long n3)
 {

@@ -95,3 +95,49 @@ def test_cpp_caller_runs_the_three_pair_style_modes(tmp_path, L_max, dtype, one_
         assert np.abs(F - f_ref).max() <= ftol, name
         # a ghost node's edges are copies of its owner's edge vectors, so the sum over all copies is the same virial
         assert np.abs(vir - v_ref).max() <= vtol * vscale, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L_max,dtype,terms", [(0, "float64", True), (1, "float32", False)])
+def test_cpp_caller_on_a_rank_without_atoms(tmp_path, L_max, dtype, terms):
+    """What a rank of a decomposed run calls while no atom is on it, from its first step on: all modes with vectors that never
+    held anything (null pointers), ghost rows of H1 among them; then atoms without an edge, and a rank with both."""
+    if not os.path.exists(DRIVER):
+        pytest.fail("tests/cpp/pair_modes_driver is not built: python -c 'import __graft_entry__ as g; g.build()'")
+    model = H.tiny_model(K=16, L_max=L_max, n_pts=48, seed=13, zbl=terms, density=terms)
+    path = H.write_model(model, tmp_path / "m.json")
+    pos, cell, sp = H.small_system(20, seed=22)
+    nl, ea = H.edges_of(pos, cell, sp, model["r_cut"])
+    N, rows = len(sp), 4
+    i0, d0, three = np.zeros(0, np.int32), np.zeros(0), np.zeros(3, np.int32)
+    types = np.array([2, 0, 1], np.int32)
+    empty = (2, 4, 3, 1)
+    case, out = tmp_path / "case.bin", tmp_path / "out.bin"
+    with open(case, "wb") as f:
+        np.array([len(empty) + 3], dtype=np.int64).tofile(f)
+        for mode in empty:
+            _case(f, mode, 0, 0, rows, i0, i0, i0, i0, i0, i0, i0, i0, d0, d0)
+        for mode in (2, 4):
+            _case(f, mode, 3, 0, 3, types, three, np.arange(3), i0, i0, i0, i0, i0, d0, d0)
+        _case(f, 2, N, 0, N, ea["node_types"], ea["num_neigh"], np.arange(N), ea["neigh_indices"], ea["neigh_types"],
+              ea["neigh_indices"], i0, i0, ea["xyz"], ea["r"])
+    res = subprocess.run([DRIVER, path, "0" if dtype == "float64" else "1", str(case), str(out)], capture_output=True,
+                         text=True, timeout=100)
+    print(res.stdout, res.stderr, flush=True)
+    assert res.returncode == 0, res.stderr
+    raw, o = np.fromfile(out, dtype=np.float64), 0
+    for _ in empty:
+        assert not raw[o:o + 1 + 3 * rows + 6].any()
+        o += 1 + 3 * rows + 6
+    etol, ftol = (1e-10, 1e-8) if dtype == "float64" else (1e-5, 1e-4)      # the bar of the parity tests
+    alone = OracleMACE(model)
+    alone.compute_node_energies_forces(3, types, three, i0, i0, d0, d0)
+    for _ in range(2):
+        assert np.abs(raw[o + 1:o + 4] - alone.node_energies).max() <= etol * np.abs(alone.node_energies).max()
+        assert not raw[o + 4:o + 4 + 9 + 6].any()
+        o += 1 + 3 + 9 + 6
+    orc = OracleMACE(model)
+    orc.compute_node_energies_forces(*H.call_args(ea))
+    assert np.abs(raw[o + 1:o + 1 + N] - orc.node_energies).max() <= etol * np.abs(orc.node_energies).max()
+    assert np.abs(raw[o + 1 + N:o + 1 + 4 * N].reshape(N, 3) - H.atom_forces(nl, orc.node_forces, N)).max() <= ftol
+    assert o + 1 + 4 * N + 6 == len(raw)
