@@ -981,16 +981,22 @@ def test_scalar_features_with_a_coupling_that_mixes_harmonics(gpu, tmp_models, K
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["float64", "float32"])
-@pytest.mark.parametrize("L_max,zbl,density", [(0, False, False), (1, False, False), (0, True, True)])
-def test_arrays_that_an_evaluation_does_not_form(gpu, tmp_models, L_max, zbl, density, dtype):
-    """From 1 024 atoms on the A-basis and its adjoint stay in registers (without density normalisation) and are formed when
-    somebody asks: alone, in either order, after a stage call, with ghost nodes, and after an evaluation of fewer atoms whose
-    arrays are all written (600: the linears of the other kernel, 100: none of them)."""
+@pytest.mark.parametrize("L_max,K,most,terms", [
+    # 160 channels have no chains: from 1 024 atoms linears with the contraction in them, 600 the linears alone, 100 neither
+    (0, 160, 1100, False), (1, 160, 1100, False),
+    # 32 channels: chains up to 3 072 (l = 0) and 2 048 atoms (l <= 1), linears with the contraction above
+    (0, 32, 3100, False), (1, 32, 2100, False),
+    # pair repulsion and density normalisation: the linears alone
+    (0, 32, 1100, True)])
+def test_arrays_that_an_evaluation_does_not_form(gpu, tmp_models, L_max, K, most, terms, dtype):
+    """The A-basis and its adjoint stay in registers where the contraction is evaluated behind the linear (in its launch, or in
+    a chain) and are formed when somebody asks: alone, in either order, after a stage call, with ghost nodes, and after an
+    evaluation of fewer atoms that takes other kernels."""
     from symmetrix_amd import neighbors
-    model = H.tiny_model(K=32, L_max=L_max, n_pts=32, seed=60 + L_max, r_cut=3.0, pair=False, zbl=zbl, density=density)
-    path = H.write_model(model, tmp_models / f"asked_{L_max}{int(zbl)}.json")
+    model = H.tiny_model(K=K, L_max=L_max, n_pts=32, seed=60 + L_max, r_cut=3.0, pair=False, zbl=terms, density=terms)
+    path = H.write_model(model, tmp_models / f"asked_{L_max}{K}{int(terms)}.json")
     runs = {}
-    for n in (1100, 600, 100):
+    for n in (most, 600, 100):
         pos, cell, sp = H.small_system(n, density=0.06, seed=n)
         nl, ea = H.edges_of(pos, cell, sp, model["r_cut"])
         orc = _oracle()(model)
@@ -1006,14 +1012,22 @@ def test_arrays_that_an_evaluation_does_not_form(gpu, tmp_models, L_max, zbl, de
             assert a.shape == b.shape, name
             assert np.abs(a - b).max() <= TOL[dtype]["inter"] * 10 * max(1.0, np.abs(a).max()), name
 
-    for n, names in ((1100, ("A0", "A1", "A0_adj", "A1_adj")), (1100, ("A1_adj", "A0_adj", "A1", "A0", "M0_grad", "M1_grad")),
-                     (600, ("A0_adj", "A0", "A1_adj", "A1")), (1100, ("A0_adj",)), (100, ("A1", "A0")), (1100, ("A1",))):
-        print(f"{n} atoms, L_max {L_max}, {dtype}: {' '.join(names)}", flush=True)
+    for n, names in ((most, ("A0", "A1", "A0_adj", "A1_adj")), (most, ("A1_adj", "A0_adj", "A1", "A0", "M0_grad", "M1_grad")),
+                     (600, ("A0_adj", "A0", "A1_adj", "A1")), (most, ("A0_adj",)), (100, ("A1", "A0")), (most, ("A1",))):
+        print(f"{n} atoms, K {K}, L_max {L_max}, {dtype}: {' '.join(names)}", flush=True)
         nl, ea, sp, orc = runs[n]
         eng.compute_node_energies_forces(*H.call_args(ea))
         same(names, orc)
+    # the largest size takes launches per stage (chains differ in the last bits)
+    nl, ea, sp, orc = runs[most]
+    eng.set_profiling(True)
+    eng.compute_node_energies_forces(*H.call_args(ea))
+    per_stage = np.array(eng.node_energies)
+    assert (eng.stage_times()["M1"] == 0.0) == (not terms)      # (the contraction in the launch of its linear)
+    eng.set_profiling(False)
+    eng.compute_node_energies_forces(*H.call_args(ea))
+    assert np.array_equal(per_stage, eng.node_energies)
     # a stage call forms what is left before it does anything else
-    nl, ea, sp, orc = runs[1100]
     eng.compute_node_energies_forces(*H.call_args(ea))
     eng.reverse_M1(ea["num_nodes"], ea["node_types"])
     same(("A1", "A0"), orc)
