@@ -874,11 +874,17 @@ struct Engine : EngineBase {
     // double 512 atoms 514 / 444, single 768 atoms 410 / 399, 96 channels 348 / 325, 64 channels double 1 024 atoms 457 / 396;
     // l <= 2, 128 channels double 400 atoms 759 / 686, 64 channels single 768 atoms 386 / 337.  Times of the stages are those of
     // launches of their own, so an evaluation that takes them has these.
+    // Ghost nodes take a block each in the chains of layer 0 and none in that of layer 1, so that all nodes have a line of their
+    // own: local / all nodes, us as above: one l, double, 96 channels 400 / 1 117 263 / 231, 600 / 1 547 285 / 301; single, 128
+    // channels 400 / 1 100 225 / 204, 600 / 1 547 243 / 270, 96 channels 600 / 1 547 195 / 189, 768 / 1 866 212 / 211; l <= 1, 128
+    // channels double 400 / 1 100 508 / 496, single 341 / 321, 600 / 1 474 366 / 416, 64 channels double 768 / 1 776 382 / 376,
+    // 1 000 / 2 181 430 / 439, 96 channels single 400 / 1 634 354 / 343, 600 / 2 182 416 / 452; l <= 2, 64 channels double 768 /
+    // 1 776 636 / 632.
     bool use_chains(int N) const
     {
-        static const long most[3] = {98304, 65536, 49152};
+        static const long most[3] = {98304, 65536, 49152}, most_nodes = sizeof(F) == 8 ? 139264 : 163840;
         return !profiling && split_nodes > 0 && chain_ok(K()) && M0_tables && M1_tables && !hm.A0_scaled && !hm.A1_scaled &&
-               (long)deciding_nodes(N) * K() <= most[hm.L_max];
+               (long)split_nodes * K() <= most[hm.L_max] && (long)N * K() <= most_nodes;
     }
     // The layer-0 adjoint linear writes over Phi0, unless the evaluation keeps Phi0 to form A0 from it on request.
     bool separate_dPhi0(int N) const { return fused_contraction(0, N) || (use_chains(N) && NLM() == 1); }
