@@ -163,18 +163,18 @@ struct SetProduct {
 // and 3 000 atoms with 96 channels (1 128 wavefronts, 1 024 SIMDs) twice the time of an even share.  Half the registers also
 // leaves room for more blocks, whose stores and first loads then go on under the products of others (those were 20 to 25 % of the
 // time each).  All 16, and now, us: 3 000 atoms, 96 channels, double, with a contraction 51 / 42, without 42 / 32; 20 011 atoms,
-// single 133 / 111 and 108 / 96; 24 999 atoms, 128 channels, double, without 302 / 268; 50 000 atoms, single, the same 320 / 329.
-// Without the contraction the
-// halves are blocks of their own, which stage the rows of their half only.  With it both are in one block, and trade variables
-// through LDS.  Many atoms whose channels are multiples of 64 keep all 16 (l, m) with a contraction behind them (SPLIT false,
-// launch_linear): such a block stages rows for twice the columns.  Three wavefronts per SIMD with halves and a contraction: at 172
-// registers instead of 168 there were two, and an evaluation of 3 000 atoms, 96 channels, double took 462 us instead of 449.
+// single 133 / 111 and 108 / 96; 24 999 atoms, 128 channels, double, without 302 / 268.  Without the contraction the halves are
+// blocks of their own, which stage the rows of their half only.  With it both are in one block, and trade variables through LDS.
+// Many atoms whose channels are multiples of 64 keep all 16 (l, m) (SPLIT false) with a contraction behind them, where a block of
+// halves stages rows for half the columns, and in single precision without one and without factors: rules in launch_linear.
+// Three wavefronts per SIMD with halves and a contraction: at 172 registers instead of 168 there were two, and an evaluation of
+// 3 000 atoms, 96 channels, double took 462 us instead of 449.
 template <typename F, int WPB, bool POLY, bool SCALED, bool SPLIT>
 __global__ __launch_bounds__(64 * WPB, POLY && SPLIT ? 3 : 2) void k_linear(const LinearParams<F> p)
 {
-    static_assert(SPLIT || POLY, "halves without a contraction");
     using Op = MatOp<F>;
-    constexpr int V = 16 / (int)sizeof(F), CT = POLY && SPLIT ? WPB / 2 : WPB, SETS = POLY ? 1 : 2;      // column tiles, blocks for the sets
+    constexpr int V = 16 / (int)sizeof(F);
+    constexpr int CT = POLY && SPLIT ? WPB / 2 : WPB, SETS = POLY || !SPLIT ? 1 : 2;      // column tiles, blocks for the sets
     extern __shared__ __align__(16) unsigned char lin_lds[];      // [BUFS][8 or 16 (l, m)][16 atoms][64]; later the coefficients
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(64 * WPB, POLY && SPLIT ? 3 : 2) void k_linear(cons
     } else if (tile * 16 >= seg_n) {
         return;
     }
-    if (!POLY && (set == 0 ? e >= p.num_e[0] && e >= p.num_e[3] : e >= p.num_e[1] && e >= p.num_e[2])) return;
+    if (!POLY && SPLIT && (set == 0 ? e >= p.num_e[0] && e >= p.num_e[3] : e >= p.num_e[1] && e >= p.num_e[2])) return;
     // atom a of the tile; beyond the segment the last atom again, whose results are not stored
     auto node_of = [&](int a) {
         const int j = min(tile * 16 + a, seg_n - 1);
@@ -219,13 +219,15 @@ __global__ __launch_bounds__(64 * WPB, POLY && SPLIT ? 3 : 2) void k_linear(cons
             for (int r = 0; r < 4; ++r)
                 if (live[r]) {
                     F* o = p.out + (size_t)node[r] * p.out_node_stride + (size_t)e * p.K + col;
-                    static_for<0, 8>([&](auto qc) {
+                    static_for<0, slots_of(SET)>([&](auto qc) {
                         constexpr int q = decltype(qc)::value, lm = lm_of(SET, q), l = lm_l(lm);
                         if (e < p.num_e[l]) o[p.out_off[lm]] = acc[q][r];
                     });
                 }
         };
-        if (set == 0) store(std::integral_constant<int, 0>{}); else store(std::integral_constant<int, 1>{});
+        if constexpr (!SPLIT) store(std::integral_constant<int, 2>{});
+        else if (set == 0) store(std::integral_constant<int, 0>{});
+        else store(std::integral_constant<int, 1>{});
     }
     if constexpr (POLY) {
         // With halves, the two wavefronts of a column tile trade variables: the one ends with all 16 of a lane's atoms 0 and 1, the
@@ -292,10 +294,10 @@ template <typename F, int WPB, bool POLY, bool SCALED, bool SPLIT = true>
 hipError_t launch_linear_t(const LinearParams<F>& p, hipStream_t s)
 {
     constexpr int CT = POLY && SPLIT ? WPB / 2 : WPB;
-    size_t lds = 3 * (size_t)(POLY ? 16 : 8) * 1024;
+    size_t lds = 3 * (size_t)(POLY || !SPLIT ? 16 : 8) * 1024;
     if (POLY) lds = std::max({lds, (size_t)CT * poly_spec_padded(kPolyTableLen[0]) * 16 * sizeof(F), (size_t)WPB * 16 * 64 * sizeof(F)});
     const long tiles = ((long)p.num_nodes + 15) / 16 + (p.perm ? p.T : 0);
-    const long blocks = (tiles + 7) / 8 * 8 * (p.K / (16 * CT)) * p.num_e_max * (POLY ? 1 : 2);
+    const long blocks = (tiles + 7) / 8 * 8 * (p.K / (16 * CT)) * p.num_e_max * (POLY || !SPLIT ? 1 : 2);
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
     if (lds > 64 * 1024) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_linear<F, WPB, POLY, SCALED, SPLIT>), dim3((unsigned)blocks), dim3(64 * WPB), lds, s, p);
@@ -304,23 +306,34 @@ hipError_t launch_linear_t(const LinearParams<F>& p, hipStream_t s)
 
 }  // namespace
 
-// Column tiles of a block: all that divide evenly, up to four (24 KB of LDS a block); with a contraction two, each with both halves
-// of the (l, m), or four without halves.
+// Column tiles of a block: all that divide evenly, up to four (24 KB of LDS a block, 48 KB with all (l, m)); with a contraction
+// two, each with both halves of the (l, m), or four without halves.
 template <typename F>
 hipError_t launch_linear(const LinearParams<F>& p, hipStream_t s)
 {
     if (p.num_nodes <= 0) return hipSuccess;
     if (!linear_ok(p.K) || p.T <= 0 || (p.coef && (p.scale || p.num_e_max != 1))) return hipErrorInvalidValue;
+    const long whole = ((long)p.num_nodes + 15) / 16 * (p.K / 64);      // blocks of four column tiles, all (l, m)
     if (p.coef) {
         // Blocks with all (l, m) once there are enough to even out over 256 CUs, which hold two (double) or three at a time: A1 of
         // layers l <= 1 at 128 channels, halves / all: double 3 000 atoms 107 / 119 us, 9 000 276 / 305, 12 000 373 / 329,
         // 24 999 770 / 710; single 3 000 62 / 68, 4 500 95 / 100, 6 000 118 / 106, 50 000 830 / 735.
-        const long whole = ((long)p.num_nodes + 15) / 16 * (p.K / 64);
         if (p.K % 64 == 0 && whole > (sizeof(F) == 8 ? 1152 : 640)) return launch_linear_t<F, 4, true, false, false>(p, s);
         return launch_linear_t<F, 4, true, false>(p, s);
     }
     auto go = [&](auto sc) -> hipError_t {
         constexpr bool SCALED = decltype(sc)::value;
+        if constexpr (sizeof(F) == 4 && !SCALED) {
+            // Single precision without factors keeps all (l, m) over many atoms: the weights are read half as often.  Halves / all,
+            // us: adjoint of A1 (output blocks), l <= 1, 128 channels 1 000 atoms 23 / 28, 2 000 42 / 38, 6 000 114 / 104, 50 000
+            // 894 / 775, 64 channels 6 000 40 / 40, 8 000 51 / 48; A1 (longer sums) 128 channels 4 500 82 / 87, 6 000 98 / 91,
+            // 50 000 779 / 705, 64 channels 8 000 40 / 40, 12 000 58 / 56; A0 and its adjoint 128 channels 8 000 57 / 68, 15 000
+            // 103 / 101, 50 000 340 / 331, 64 channels 25 000 54 / 60, 35 000 80 / 81, 50 000 121 / 115.  With factors halves win
+            // at every size (50 000 atoms 295 / 303), and in double (50 000 atoms, 96 channels 384 / 435; A0 24 999 atoms, 128
+            // channels 277 / 317), and in columns of 96 (50 000 atoms 222 / 236).
+            const int inner = std::max({p.inner[0], p.inner[1], p.inner[2], p.inner[3]});
+            if (p.K % 64 == 0 && whole > (p.num_e_max > 1 ? 384 : (inner > p.K ? 640 : 2048))) return launch_linear_t<F, 4, false, false, false>(p, s);
+        }
         if (p.K % 64 == 0) return launch_linear_t<F, 4, false, SCALED>(p, s);
         if (p.K % 96 == 0) return launch_linear_t<F, 3, false, SCALED>(p, s);
         return launch_linear_t<F, 2, false, SCALED>(p, s);

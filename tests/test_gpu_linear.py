@@ -55,6 +55,36 @@ def test_both_kinds_of_wavefront(tmp_models, K, L_max, dtype, n):
         assert np.abs(got - forces[s]).max() <= (1e-5 if dtype == "float32" else 1e-12) * max(np.abs(got).max(), 1e-3)
 
 
+# density normalisation: no factors and no contraction in the linears.  The first size is past the lines of all of them (single
+# precision), the second past that of the adjoint of A1 only, the third is double and has halves throughout.
+@pytest.mark.parametrize("K,L_max,dtype,n", [(128, 1, "float32", 16385), (64, 2, "float32", 6145), (64, 1, "float64", 18433)])
+def test_both_kinds_without_a_contraction(tmp_models, K, L_max, dtype, n):
+    """As above, bit for bit, against the first 600 and the last 601 atoms (wavefronts with halves)."""
+    _, eng = _engine(tmp_models, K, L_max, dtype, density=True)
+    rng = np.random.default_rng(n)
+    species = rng.integers(0, 3, n).astype(np.int32)
+    i, cut = np.arange(n), n - 601
+    start = np.where(i < cut, i // 10 * 10, cut + (i - cut) // 10 * 10)
+    size = np.minimum(np.where(i < cut, np.minimum(start + 10, cut), n) - start, 10)
+    j = (start + (i - start + 1 + rng.integers(0, 2, n)) % size).astype(np.int32)
+    r = rng.uniform(0.8, 2.9, n)
+    u = rng.normal(size=(n, 3))
+    xyz = u * (r / np.linalg.norm(u, axis=1))[:, None]
+    one = np.ones(n, np.int32)
+    names = ["A0", "A1", "A1_adj", "A0_adj", "Phi1_adj", "node_energies"]
+    print(f"K={K} L_max={L_max} atoms={n} {dtype}", flush=True)
+    eng.compute_node_energies_forces(n, species, one, j, species[j], xyz, r)
+    whole = {name: np.array(getattr(eng, name)).reshape(n, -1) for name in names}
+    forces = np.array(eng.node_forces).reshape(n, 3)
+    assert np.isfinite(forces).all()
+    for a, b in ((0, 600), (cut, n)):
+        s = slice(a, b)
+        eng.compute_node_energies_forces(b - a, species[s], one[s], j[s] - a, species[j[s]], xyz[s], r[s])
+        for name in names:
+            assert np.array_equal(np.array(getattr(eng, name)).reshape(b - a, -1), whole[name][s]), name
+        assert np.array_equal(np.array(eng.node_forces).reshape(-1, 3), forces[s])
+
+
 @pytest.mark.parametrize("dtype", ["float64", "float32"])
 @pytest.mark.parametrize("K,n,density", [(160, 17, False), (96, 33, False), (32, 16, False), (160, 9, True), (128, 20, True), (20, 7, True)])
 def test_against_the_oracle(tmp_models, K, n, density, dtype):
