@@ -16,6 +16,8 @@
 // copied 130 KB per block first.
 #include "smx_edge_common.hpp"
 
+#include <algorithm>
+
 namespace smx {
 
 namespace {
@@ -33,21 +35,23 @@ __device__ __forceinline__ double fma_apart(double a, double b, double c) { retu
 constexpr int lm_of_tile(int t) { return t == 0 ? 0 : (t == 1 ? 1 : (t == 2 ? 4 : (t == 3 ? 8 : (t == 4 ? 9 : 13)))); }
 
 // Wavefronts per SIMD (thread blocks per CU) of the adjoint: what the registers of its channels allow.  20 011 atoms, 96 channels,
-// single: adjoints of 275 and 264 us with two, 253 and 237 with three; 24 999 atoms, 128 channels, double 1.03 and 1.02 ms.
+// single: adjoints of 275 and 264 us with two, 253 and 237 with three; double, two channels per lane, layer 0: 600 atoms, 64 and 128
+// channels 24 / 21 and 33 / 30, 10 000 atoms 243 / 231 and 455 / 441, 24 999 atoms 1 033 / 1 008 (l <= 1), 50 000 atoms 2 828 /
+// 2 858 (78 edges an atom).  Where messages are stored as well, double and two channels per lane: see launch0.
 template <typename F, int CPL>
 constexpr int bwd0_blocks() { return CPL <= (sizeof(F) == 8 ? 2 : 3) ? 3 : 2; }
 // edges per chunk: one lane each (two are left for a look at the next chunk), as many as leave room for the thread blocks of a CU
-template <typename F, bool BWD, int CPL>
+template <typename F, bool BWD, int BPC>
 constexpr int chunk0()
 {
     if (!BWD) return 62;
-    if (bwd0_blocks<F, CPL>() == 3) return sizeof(F) == 8 ? 30 : 54;
+    if (BPC == 3) return sizeof(F) == 8 ? 30 : 54;
     return sizeof(F) == 8 ? 44 : 62;
 }
 
-template <typename F, bool BWD, int CPL>
+template <typename F, bool BWD, int BPC>
 struct Lds0 {
-    static constexpr int CH = chunk0<F, BWD, CPL>();
+    static constexpr int CH = chunk0<F, BWD, BPC>();
     static_assert(CH % 2 == 0 && CH + 2 <= 64, "whole iterations, and a lane for every entry");
     static constexpr int NY = BWD ? 48 : 16;          // [lm][3]: harmonic, its two tangential derivatives; or harmonics
     static constexpr size_t val_bytes = ((size_t)CH * NY + 16) * sizeof(F);
@@ -55,7 +59,7 @@ struct Lds0 {
     static constexpr size_t sum_bytes = BWD ? (size_t)(CH + 2) * 4 * sizeof(double) : 0;
     static_assert(val_bytes % 16 == 0, "the sums begin on a 16-byte boundary");
     static constexpr size_t per_wave = (val_bytes + head_bytes + sum_bytes + 15) / 16 * 16;
-    static_assert(!BWD || 4 * per_wave * bwd0_blocks<F, CPL>() <= 160 * 1024, "the thread blocks of a CU");
+    static_assert(!BWD || 4 * per_wave * BPC <= 160 * 1024, "the thread blocks of a CU");
 };
 
 // interval, argument and rows of an edge; offsets of its table and sender rows in bytes (32 bits: launch_agg0_ok)
@@ -74,7 +78,7 @@ template <typename F, int CPL, int EW>
 __global__ __launch_bounds__(256, 2) void k_agg0_fwd(const AggParams<F> a, const int parts, const int group_channels)
 {
     constexpr bool MX = kMatrix<F>;
-    using L = Lds0<F, false, CPL>;
+    using L = Lds0<F, false, 2>;
     constexpr int LPE = 64 / EW, CH = L::CH, CBSZ = EW == 2 ? 3 : 4;
     constexpr int W = MX || CPL <= 2 ? 4 : 2;          // splines requested ahead
     extern __shared__ __align__(16) unsigned char smem[];
@@ -288,11 +292,11 @@ __device__ __forceinline__ double edge_sum3(F s, F g1, F g2, int lane)
 }
 
 // ---------------------------------------------------------------------------
-template <typename F, int CPL, int EW, bool MSG>
-__global__ __launch_bounds__(256, (bwd0_blocks<F, CPL>())) void k_agg0_bwd(const AggParams<F> a, const int parts)
+template <typename F, int CPL, int EW, bool MSG, int BPC>
+__global__ __launch_bounds__(256, BPC) void k_agg0_bwd(const AggParams<F> a, const int parts)
 {
     constexpr bool MX = kMatrix<F>;
-    using L = Lds0<F, true, CPL>;
+    using L = Lds0<F, true, BPC>;
     constexpr int LPE = 64 / EW, CH = L::CH, CBSZ = EW == 2 ? 3 : 4, GPR = LPE / 4;   // groups of four rows per register
     constexpr int NB = MX ? 16 / GPR : 3;              // registers that hold an edge's harmonics
     constexpr int W = MX || CPL == 1 ? 4 : 2;          // splines requested ahead
@@ -520,26 +524,30 @@ hipError_t launch0(const AggParams<F>& p, int group, hipStream_t s)
     const long blocks = (nodes * parts + 3) / 4 * groups;
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-    size_t lds = 4 * Lds0<F, BWD, CPL>::per_wave;
-    const void* kern;
-    if constexpr (BWD) kern = reinterpret_cast<const void*>(p.msg ? k_agg0_bwd<F, CPL, EW, true> : k_agg0_bwd<F, CPL, EW, false>);
-    else {
-        kern = reinterpret_cast<const void*>(k_agg0_fwd<F, CPL, EW>);
-        const size_t handed = parts > 1 ? (size_t)2 * (16 / EW) * CPL * 64 * sizeof(F) : 0;   // two givers per block
-        lds = lds > handed ? lds : handed;
-    }
-    if (lds > 64 * 1024) {
-        hipError_t err = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (err != hipSuccess) return err;
-    }
-    const dim3 grid((unsigned)blocks), block(256);
+    auto go = [&](auto kern, size_t lds, auto... args) {
+        if (lds > 64 * 1024) {
+            hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (err != hipSuccess) return err;
+        }
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), lds, s, p, args...);
+        return hipGetLastError();
+    };
     if constexpr (BWD) {
-        if (p.msg) hipLaunchKernelGGL((k_agg0_bwd<F, CPL, EW, true>), grid, block, lds, s, p, parts);
-        else hipLaunchKernelGGL((k_agg0_bwd<F, CPL, EW, false>), grid, block, lds, s, p, parts);
+        constexpr int BPC = bwd0_blocks<F, CPL>();
+        constexpr size_t lds = 4 * Lds0<F, true, BPC>::per_wave;
+        if (!p.msg) return go(k_agg0_bwd<F, CPL, EW, false, BPC>, lds, parts);
+        // With messages, double and two channels per lane, the third wavefront costs from where a receiver has one to itself: us, three
+        // / two: 64 channels 600 atoms 22 / 24, 3 000 60 / 63, 6 500 118 / 112, 20 000 357 / 337, 50 000 901 / 844, 128 channels 600
+        // 32 / 35, 3 000 102 / 104, 6 500 208 / 207, 20 000 658 / 620, 50 000 1 604 / 1 529.  (One channel per lane: 50 000 atoms
+        // 514 / 550.  Three wavefronts and two edges at a time spill five registers: few receivers gain all the same.)
+        if constexpr (BPC == 3 && sizeof(F) == 8 && CPL == 2) {
+            if (parts == 1) return go(k_agg0_bwd<F, CPL, EW, true, 2>, 4 * Lds0<F, true, 2>::per_wave, parts);
+        }
+        return go(k_agg0_bwd<F, CPL, EW, true, BPC>, lds, parts);
     } else {
-        hipLaunchKernelGGL((k_agg0_fwd<F, CPL, EW>), grid, block, lds, s, p, parts, group);
+        const size_t handed = parts > 1 ? (size_t)2 * (16 / EW) * CPL * 64 * sizeof(F) : 0;   // two givers per block
+        return go(k_agg0_fwd<F, CPL, EW>, std::max(4 * Lds0<F, false, 2>::per_wave, handed), parts, group);
     }
-    return hipGetLastError();
 }
 template <typename F, bool BWD>
 hipError_t launch0_sel(const AggParams<F>& p, hipStream_t s)

@@ -1110,6 +1110,8 @@ def test_buckets_on_both_sides_of_the_lds(gpu, tmp_models, n, L_max, K):
     # scalar sender features: two edges at a time in chunks of 44 and 62, one to four channels per lane and an edge alone,
     # channel groups that do not fill their lanes; at 48 channels tables beyond an L2 (four groups)
     (20, 0, 40, 67, 1), (33, 0, 40, 60, 1), (65, 0, 12, 270, 1), (97, 0, 12, 270, 1), (130, 0, 24, 90, 1), (48, 0, 24, 40, 1),
+    # a wavefront per receiver, two channels per lane: two wavefronts per SIMD in double, chunks of 44 edges, two at a time and one
+    (64, 0, 6145, 47, 1), (128, 0, 6145, 47, 1),
     # coupling entries of three terms
     (32, 1, 20, 20, 3), (32, 2, 20, 20, 3),
 ])
