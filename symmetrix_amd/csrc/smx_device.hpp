@@ -197,8 +197,6 @@ __device__ __forceinline__ double wave_sum(double v)
     return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
 }
 
-// Orders the LDS traffic of one wavefront: what its lanes wrote before is
-// visible to all its lanes after.  No other wavefront is involved.
 // Row tiles of 16 atoms of one species, numbered so that those of species t begin at tstart[t] / 16 + t: enough for each, and the
 // tile of a number is found with one load per lane instead of a walk over the species that waits for each in turn (0.3 to 0.5 us
 // a species, at the start of every block).  tstart[T] / 16 + T numbers, some of them without a tile (type -1).
@@ -220,6 +218,8 @@ __device__ __forceinline__ RowTile row_tile(const int* tstart, int T, int index,
     return r;
 }
 
+// Orders the LDS traffic of one wavefront: what its lanes wrote before is
+// visible to all its lanes after.  No other wavefront is involved.
 __device__ __forceinline__ void wave_lds_sync()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
