@@ -1131,7 +1131,7 @@ struct Engine : EngineBase {
         const int rows = (int)(H1.n / ((size_t)nlm * k));
         if (rows < N || M1.n < (size_t)N * k) throw Error(SMX_EINVAL, "readouts called before H1 and M1 exist for these nodes");
         TailParams<F> p{};
-        p.N = N; p.rows = rows; p.K = k; p.num_LM = nlm; p.T = hm.T;
+        p.N = N; p.rows = rows; p.K = k; p.num_LM = nlm; p.T = hm.T; p.num_cus = num_cus;
         p.perm = t_perm.p; p.tstart = t_start.p;
         p.E0 = E0.p; p.w1 = ro1.p; p.W1 = ro2_w1.p; p.w2 = ro2_w2.p; p.scale = hm.readout_2_scale;
         p.H1 = H1.p; p.M1 = M1.p; p.W_H1 = H2w_H1.p; p.W_M1 = H2w_M1.p; p.V_H1 = H2v_H1.p; p.V_M1 = H2v_M1.p;

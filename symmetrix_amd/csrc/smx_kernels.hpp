@@ -349,6 +349,7 @@ struct TailParams {
     double* guard_forces;    // raised guard: these guard_forces_n edge-force components become NaN as well (the
     double* guard_copy;      // (and those of the caller's array, if not null)
     long guard_forces_n;     // adjoint kernels of a skipped evaluation see no edges and write none)
+    int num_cus;             // of the device: how many blocks run at once
 };
 bool tail_fused_ok(int K);
 template <typename F> hipError_t launch_tail_fused(const TailParams<F>& p, hipStream_t s);

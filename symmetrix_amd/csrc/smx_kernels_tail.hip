@@ -18,6 +18,8 @@
 #include "smx_device.hpp"
 #include "smx_kernels.hpp"
 
+#include <algorithm>
+
 namespace smx {
 
 namespace {
@@ -238,7 +240,7 @@ static hipError_t launch_tail_fused_t(const TailParams<F>& p, hipStream_t s)
         if (err != hipSuccess) return err;
     }
     // a block per tile while the chip holds them all at once, then as many tiles to each of the blocks that it holds
-    const int tiles = (p.N + 15) / 16 + p.T, at_once = 256 * tail_blocks_per_cu(KT), per = (tiles + at_once - 1) / at_once;
+    const int tiles = (p.N + 15) / 16 + p.T, at_once = std::max(p.num_cus, 1) * tail_blocks_per_cu(KT), per = (tiles + at_once - 1) / at_once;
     hipLaunchKernelGGL((k_tail_fused<F, KT>), dim3((unsigned)((tiles + per - 1) / per)), dim3(64 * KT), lds, s, p, per);
     return hipGetLastError();
 }
