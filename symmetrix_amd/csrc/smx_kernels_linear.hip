@@ -168,7 +168,7 @@ struct SetProduct {
 // Many atoms whose channels are multiples of 64 keep all 16 (l, m) (SPLIT false) with a contraction behind them, where a block of
 // halves stages rows for half the columns, and in single precision without one and without factors: rules in launch_linear.
 // Three wavefronts per SIMD with halves and a contraction: at 172 registers instead of 168 there were two, and an evaluation of
-// 3 000 atoms, 96 channels, double took 462 us instead of 449.
+// 3 000 atoms, 96 channels, double took 462 us instead of 449 (four column tiles in double spill two registers for it).
 template <typename F, int WPB, bool POLY, bool SCALED, bool SPLIT>
 __global__ __launch_bounds__(64 * WPB, POLY && SPLIT ? 3 : 2) void k_linear(const LinearParams<F> p)
 {

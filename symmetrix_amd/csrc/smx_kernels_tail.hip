@@ -14,7 +14,7 @@
 // 24 999 atoms 198 -> 78 us, 20 011 atoms, 96 channels 98 -> 53 us, 3 000 atoms 23.4 -> 18.3 us.
 //
 // Compiled without the hoisting of machine instructions out of loops: it kept the constants of exp in 22 registers over the
-// tiles, and spilled as many weights (K = 96).
+// tiles, and spilled as many weights (K = 96).  At three wavefronts per SIMD 96 channels still spill 12 registers (single 2).
 #include "smx_device.hpp"
 #include "smx_kernels.hpp"
 
