@@ -12,7 +12,7 @@ Prints ONE JSON line.  Besides the driver's fields it carries
   roofline_stages   the same figures for every edge stage (aggregations, their adjoints, the sender-side sum)
   mfma          the dense channel-mixing stages against the matrix-core peak (algorithmic flops / stage time), with the
                 matrix-pipe busy share rocprofv3 counted for the stage's kernel (profiles/)
-  contraction   the two symmetric contractions against the vector-arithmetic peak (flops of the monomial walk / stage
+  contraction   the two symmetric contractions against the vector-arithmetic peak (flops of the nested polynomials / stage
                 time) and their HBM side (variables in, values and gradients out)
   cpu_baseline  the CPU oracle (serial fp64 restatement of the reference path)
                 timed on this host on the same workload
@@ -76,46 +76,54 @@ MFMA_PEAK = {"float64": 78.6e12, "float32": 157.3e12}   # dense matrix-core peak
 # kernel behind each dense stage (as the kernel trace names it) when it runs in feature precision F
 DENSE_KERNEL = {"A0_lin": r"k_linear<{F}, \d, {one}, false, (true|false)>", "A1": r"k_linear<{F}, \d, true, false, (true|false)>",
                 "H1": r"k_gemm_rows<{F}, {F}, {F}, \d, false", "H2": r"k_tail_fused<{F}",
-                "rev_A1": r"k_linear<{F}, \d, false, true, true>", "rev_A0_lin": r"k_linear<{F}, \d, false, {one}, true>",
+                "rev_A1": r"k_linear<{F}, \d, false, true, true>", "rev_A0_lin": r"k_linear<{F}, \d, false, {one}, (true|false)>",
                 "rev_H1": r"k_gemm_rows<{F}, {F}, {F}, \d, false"}   # {one}: one polynomial per channel in layer 0
 
 
 def dense_flops(stage, N, K, n_LM, n_e):
-    """Algorithmic flops per evaluation of a dense stage: 2 x rows x K x K multiply-adds per atom for the products
-    (A0 linear: 16 rows; H1: n_LM; A1: n_e rows of K into 16 / n_e, i.e. 2 n_e K^2; H2: two K x K products), the
-    readout network 2 x 16 K each way, and as much again for each adjoint."""
+    """Flops per evaluation of a dense stage: 2 x rows x K x K multiply-adds per atom for the products (A0 linear: 16 rows;
+    H1: n_LM; A1: n_e rows of K into 16 / n_e, i.e. 2 n_e K^2), as much again for each adjoint; H2 and the tail behind it
+    two K x K products, and four with the 16 hidden units (the units, and the three adjoints of rank 16)."""
     per_atom = {
         "A0_lin": 32 * K * K, "rev_A0_lin": 32 * K * K,
         "H1": 2 * n_LM * K * K, "rev_H1": 2 * n_LM * K * K,
         "A1": 2 * n_e * K * K, "rev_A1": 2 * n_e * K * K,
-        "H2": 8 * K * K + 128 * K,      # H2, readout network with its gradient, reverse_H2: one launch
+        "H2": 4 * K * K + 128 * K,      # H2, readout network with its gradient, reverse_H2: one launch
     }
     return per_atom[stage] * N
 
 
-VALU_PEAK = 78.6e12   # vector multiply-add peak of MI355X, flop/s, double or (unpacked) single precision
+# vector multiply-add peaks of MI355X, flop/s (32-bit multiply-adds issue in half the cycles of 64-bit ones)
+VALU_PEAK = {"float64": 78.6e12, "float32": 157.3e12}
+
+
+def nested_tables():
+    """The monomials of the polynomials of the standard product basis in the nested order of the contraction kernels."""
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("gen_poly_tables", os.path.join(HERE, "symmetrix_amd", "csrc", "gen_poly_tables.py"))
+    gen = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(gen)
+    return [gen.nested(t) for t in gen.tables()]
 
 
 def contraction_work(n_atoms, K, L_max, layer, s_bytes, mode="both"):
-    """Arithmetic and HBM bytes of one symmetric-contraction launch by the algorithm, with the monomial lists of the
-    standard product basis (harmonics up to l = 3, correlation 3).  Per atom, channel and monomial x_a x_b x_c:
-    value and gradient ("both") two products and four multiply-adds (10 flops; 7 and 3 for degrees two and one);
-    value only ("value") two products and one multiply-add (4; 3; 2); the adjoint that forms the gradient again
-    ("adjoint") three products and three multiply-adds (9; 5; 2).  Bytes: the 16 variables in; out, per polynomial,
-    the value ("both", "value") and its 16 gradient components ("both"); the adjoint reads the polynomials' adjoints
-    and writes 16 sums.  (The kernel of several polynomials nests these sums and executes about 0.6 of the operations.)"""
-    from symmetrix_amd import cg
-    per_degree = {"both": {1: 3, 2: 7, 3: 10}, "value": {1: 2, 2: 3, 3: 4}, "adjoint": {1: 2, 2: 5, 3: 9}}[mode]
+    """Arithmetic and HBM bytes of one symmetric-contraction launch, with the monomial lists of the standard product basis
+    (harmonics up to l = 3, correlation 3) in the nested form sum_p x_p sum_q x_q (w_pq + sum_c w_pqc x_c) that the kernels
+    evaluate.  Flops per atom and channel: a monomial of degree three a multiply-add for the value of its pair and one for
+    the gradient, of degree two an addition, of degree one a multiply-add for the value and one operation for the gradient; a
+    pair (p, q) a product and two multiply-adds, a p a multiply-add for the value and one operation for the gradient ("both";
+    "value" leaves the gradients away, and "adjoint", which forms them again times the polynomial's adjoint, the values).  Bytes:
+    the 16 variables in; out, per polynomial, the value ("both", "value") and its 16 gradient components ("both"); the adjoint
+    reads the polynomials' adjoints and writes 16 sums."""
+    gradient, value = mode != "value", mode != "adjoint"
+    polys = (L_max + 1) ** 2 if layer == 0 else 1
     flops_per = 0
-    polys = 0
-    for L in range((L_max if layer == 0 else 0) + 1):
-        terms = cg.symmetric_contraction_terms(L, 3, 3)
-        for M in range(2 * L + 1):
-            keys = set()
-            for t in terms:
-                keys |= set(t[M].keys())
-            flops_per += sum(per_degree[len(k)] for k in keys)
-            polys += 1
+    for table in nested_tables()[:polys]:
+        one = 16      # the constant
+        flops_per += sum((2 if c != one else 1) + (2 if gradient and c != one else 0) for p, q, c in table if p != one)
+        flops_per += sum((2 if value else 0) + ((1 if value else 2) if gradient else 0) for p, q, c in table if p == one)
+        flops_per += (2 + (3 if gradient else 0)) * len({(p, q) for p, q, c in table if p != one})
+        flops_per += ((2 if value else 0) + ((1 if value else 3) if gradient else 0)) * len({p for p, q, c in table if p != one})
     words = {"both": 16 + 17 * polys, "value": 16 + polys, "adjoint": 32 + polys}[mode]
     return flops_per * n_atoms * K, words * K * s_bytes * n_atoms
 
@@ -489,7 +497,7 @@ def main():
                 # the same stage against the vector arithmetic it cannot do without (the bound that bites: about
                 # 20 bytes of HBM data per edge and channel against one to several hundred multiply-adds)
                 stages_rl[k]["valu"] = {"flops": fl, "achieved_tflops": fl / (ms_k * 1e-3) / 1e12,
-                                        "peak_tflops": VALU_PEAK / 1e12, "frac": fl / (ms_k * 1e-3) / VALU_PEAK}
+                                        "peak_tflops": VALU_PEAK[dtype] / 1e12, "frac": fl / (ms_k * 1e-3) / VALU_PEAK[dtype]}
         mfma = {}
         for k in ("A0_lin", "H1", "A1", "H2", "rev_A1", "rev_H1", "rev_A0_lin"):
             ms_k = res["stages"].get(k, 0.0)
@@ -517,7 +525,7 @@ def main():
             if ms_k == 0.0:
                 contraction[k] = {"flops": fl, "note": "evaluated in the launch of the layer's A-basis linear"}
                 continue
-            vpeak = VALU_PEAK
+            vpeak = VALU_PEAK[dtype]
             contraction[k] = {"kernel": "k_poly_spec" if res["contraction_tables"] & (1 << layer) else "k_poly", "mode": mode,
                               "flops": fl, "kernel_ms": ms_k, "achieved_tflops": fl / (ms_k * 1e-3) / 1e12,
                               "peak_tflops": vpeak / 1e12, "valu_frac": fl / (ms_k * 1e-3) / vpeak,
