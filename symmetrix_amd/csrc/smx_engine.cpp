@@ -170,6 +170,21 @@ static void upload_as(DVec<T>& d, const std::vector<S>& h, hipStream_t s)
     HIPCHK(hipStreamSynchronize(s));  // tmp goes out of scope
 }
 
+// the bf16 number nearest to x, as its bits, and back
+static unsigned short bf16_of(float x)
+{
+    unsigned u;
+    std::memcpy(&u, &x, 4);
+    return (unsigned short)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+}
+static float float_of_bf16(unsigned short h)
+{
+    const unsigned u = (unsigned)h << 16;
+    float x;
+    std::memcpy(&x, &u, 4);
+    return x;
+}
+
 static const char* kStageNames =
     "prep;agg0_fwd;A0_lin;M0;H1;agg1_fwd;A1;M1;H2;readout;rev_H2;rev_M1;rev_A1;agg1_bwd;sender_reduce;"
     "rev_H1;rev_M0;rev_A0_lin;agg0_bwd;force_sum1;force_sum0";
@@ -235,6 +250,7 @@ struct Engine : EngineBase {
     // ---- model on device
     DVec<F> tab0, tab1, tabK0, tabK1, H0, A0w, H1w, A1w;
     DVec<F> linA0, linA0T, linA1, linA1T;    // the same weights in operand order (operand_weights)
+    DVec<unsigned short> splitA0, splitA0T, splitA1, splitA1T;    // ... and in single precision in three bf16 parts (split_weights)
     DVec<F> H1wT;                            // transposes, for the kernels that take a chain of stages
     DVec<int> pair_table0, pair_table1;
     DVec<int> B0_start, B0_lm1, B1_start, B1_lm1;
@@ -492,6 +508,7 @@ struct Engine : EngineBase {
         if (linear_ok(hm.K)) {
             const bool chain = chain_ok(hm.K) && M0_tables && M1_tables;
             operand_weights(s);
+            if (sizeof(F) == 4 && (hm.K % 128 == 0 || hm.K % 96 == 0)) split_weights(s);
             if (chain) {
                 auto transposed = [&](const std::vector<double>& w, auto& dst) {
                     const size_t Kc = hm.K, n = w.size() / (Kc * Kc);
@@ -510,40 +527,72 @@ struct Engine : EngineBase {
         HIPCHK(hipStreamSynchronize(s));
     }
 
-    // Weights of the A-basis linears in the operand order of k_linear, [l][type][output block][column tile][step][64][V]:
-    // forward, and transposed for the adjoints.
-    void operand_weights(hipStream_t s)
+    // Every matrix of the A-basis linears and of their adjoints, in the order [l][type][output block]: f(inner size, B(k, n)); done(i)
+    // after the last one of an array: 0 A0, 1 its transpose, 2 A1, 3 its transpose.
+    template <typename Block, typename Done>
+    void linear_weights(Block&& block, Done&& done)
     {
         const int K = hm.K;
-        constexpr int V = 16 / (int)sizeof(F);
-        std::vector<double> out;
-        // B(k, n) of a block of K columns
-        auto block = [&](int inner, auto&& B) {
-            for (int ct = 0; ct < K / 16; ++ct)
-                for (int st = 0; st < inner / (4 * V); ++st)
-                    for (int lane = 0; lane < 64; ++lane)
-                        for (int v = 0; v < V; ++v) out.push_back(B(4 * V * st + lane / 16 * V + v, ct * 16 + lane % 16));
-        };
-        auto done = [&](DVec<F>& dst) { upload_as(dst, out, s); out.clear(); };
         for (int pass = 0; pass < 2; ++pass) {
             for (int l = 0; l < 4; ++l)
                 for (int t = 0; t < hm.T; ++t) {
                     const double* w = hm.A0_weights.data() + ((size_t)t * 4 + l) * K * K;
                     block(K, [&](int k, int n) { return pass ? w[(size_t)n * K + k] : w[(size_t)k * K + n]; });
                 }
-            done(pass ? linA0T : linA0);
+            done(pass);
         }
         for (int l = 0; l < 4; ++l) {
             const double* w = hm.A1_weights[l].data();
             block(hm.num_e[l] * K, [&](int k, int n) { return w[(size_t)k * K + n]; });
         }
-        done(linA1);
+        done(2);
         for (int l = 0; l < 4; ++l)
             for (int eb = 0; eb < hm.num_e[l]; ++eb) {
                 const double* w = hm.A1_weights[l].data();
                 block(K, [&](int k, int n) { return w[((size_t)eb * K + n) * K + k]; });
             }
-        done(linA1T);
+        done(3);
+    }
+    // ... in the operand order of k_linear and of the chains, [column tile][step][64][V]
+    void operand_weights(hipStream_t s)
+    {
+        constexpr int V = 16 / (int)sizeof(F);
+        std::vector<double> out;
+        linear_weights([&](int inner, auto&& B) {
+            for (int ct = 0; ct < hm.K / 16; ++ct)
+                for (int st = 0; st < inner / (4 * V); ++st)
+                    for (int lane = 0; lane < 64; ++lane)
+                        for (int v = 0; v < V; ++v) out.push_back(B(4 * V * st + lane / 16 * V + v, ct * 16 + lane % 16));
+        }, [&](int i) {
+            DVec<F>* const to[4] = {&linA0, &linA0T, &linA1, &linA1T};
+            upload_as(*to[i], out, s);
+            out.clear();
+        });
+    }
+    // ... of k_linear32: [column tile][piece of 32 terms][part][64][8], w = part 0 + part 1 + part 2 in bf16, rounded to nearest
+    void split_weights(hipStream_t s)
+    {
+        std::vector<unsigned short> out;
+        linear_weights([&](int inner, auto&& B) {
+            for (int ct = 0; ct < hm.K / 16; ++ct)
+                for (int st = 0; st < inner / 32; ++st) {
+                    const size_t at = out.size();
+                    out.resize(at + 3 * 512);
+                    for (int i = 0; i < 512; ++i) {
+                        float rest = (float)B(32 * st + i / 128 * 8 + i % 8, ct * 16 + i / 8 % 16);
+                        for (int part = 0; part < 3; ++part) {
+                            const unsigned short h = bf16_of(rest);
+                            out[at + part * 512 + i] = h;
+                            rest -= float_of_bf16(h);
+                        }
+                    }
+                }
+        }, [&](int i) {
+            DVec<unsigned short>* const to[4] = {&splitA0, &splitA0T, &splitA1, &splitA1T};
+            to[i]->upload(out.data(), out.size(), s);
+            HIPCHK(hipStreamSynchronize(s));   // out changes
+            out.clear();
+        });
     }
 
     // ---- input checks of an evaluation.  flags[0]: stage-level calls (read back at once); flags[2]: the word the checks
@@ -817,7 +866,8 @@ struct Engine : EngineBase {
         LinearParams<F> q{};
         need(t_perm.p, "species groups");
         q.num_nodes = N; q.K = k; q.T = hm.T; q.perm = t_perm.p; q.tstart = t_start.p;
-        q.W = reverse ? linA0T.p : linA0.p;
+        q.W = reverse ? linA0T.p : linA0.p; q.W_split = reverse ? splitA0T.p : splitA0.p;
+        q.split_nodes = deciding_nodes(N);
         q.a_node_stride = q.out_node_stride = 16L * k; q.num_e_max = 1;
         for (int lm = 0; lm < 16; ++lm) q.row_off[lm] = q.out_off[lm] = lm * k;
         for (int l = 0; l < 4; ++l) {
@@ -833,7 +883,8 @@ struct Engine : EngineBase {
         LinearParams<F> q{};
         q.num_nodes = N; q.K = k; q.T = hm.T;
         if (groups) { need(t_perm.p, "species groups"); q.perm = t_perm.p; q.tstart = t_start.p; }
-        q.W = reverse ? linA1T.p : linA1.p;
+        q.W = reverse ? linA1T.p : linA1.p; q.W_split = reverse ? splitA1T.p : splitA1.p;
+        q.split_nodes = deciding_nodes(N);
         (reverse ? q.out_node_stride : q.a_node_stride) = (long)ne * k;
         (reverse ? q.a_node_stride : q.out_node_stride) = 16L * k;
         size_t off = 0;

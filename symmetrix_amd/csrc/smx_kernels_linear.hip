@@ -313,6 +313,9 @@ hipError_t launch_linear(const LinearParams<F>& p, hipStream_t s)
 {
     if (p.num_nodes <= 0) return hipSuccess;
     if (!linear_ok(p.K) || p.T <= 0 || (p.coef && (p.scale || p.num_e_max != 1))) return hipErrorInvalidValue;
+    if constexpr (sizeof(F) == 4) {
+        if (linear32_ok(p)) return launch_linear32(p, s);
+    }
     const long whole = ((long)p.num_nodes + 15) / 16 * (p.K / 64);      // blocks of four column tiles, all (l, m)
     if (p.coef) {
         // Blocks with all (l, m) once there are enough to even out over 256 CUs, which hold two (double) or three at a time: A1 of
