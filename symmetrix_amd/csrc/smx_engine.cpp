@@ -946,10 +946,15 @@ struct Engine : EngineBase {
         p.N = N; p.K = K(); p.T = hm.T; p.perm = t_perm.p; p.tstart = t_start.p;
         return p;
     }
-    // A0, M0 and H1
+    // A0, M0 and H1, with chain_edges(0) the layer-0 aggregation before them
     void st_chain0(int N)
     {
         const size_t k = K(), nlm = NLM();
+        const bool edges = chain_edges(0);
+        if (edges) {
+            need(xyz, "xyz"); need(r, "r"); need_edges(N);
+            Phi0.size_to((size_t)N * 16 * k, stream);
+        }
         A0.size_to((size_t)N * 16 * k, stream);
         M0.size_to((size_t)N * nlm * k, stream);
         if (nlm == 1) M0_grad.size_to((size_t)N * 16 * k, stream);
@@ -957,13 +962,36 @@ struct Engine : EngineBase {
         auto p = chain_params(N);
         p.Phi = Phi0.p; p.W = linA0.p; p.WH1 = H1w.p; p.coef = M0_slabs.p;
         p.A = A0.p; p.M = M0.p; p.M_grad = M0_grad.p; p.H1 = H1.p;
-        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain0<F, decltype(kc)::value>(p, hm.L_max, stream); }));
+        auto agg = agg_params(0, N);
+        agg.out = Phi0.p;
+        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain0<F, decltype(kc)::value>(p, edges ? &agg : nullptr, hm.L_max, stream); }));
         if (nlm == 1) pending_A0 = N;
     }
-    // A1, M1, the tail and the adjoints back to dPhi1
-    void st_chain1(int N, bool zero_energies)
+    // Whether the chains of a layer take its aggregation and the adjoint of it along (scalar features): not where a CU holds one
+    // block and there are more blocks than CUs, whose aggregations as launches of their own spread better.  Whole evaluations, us,
+    // separate / along: one l, double, 96 channels 24 atoms 87 / 78, 256 102 / 86, 300 135 / 142, 1 000 246 / 267, 128 channels 256
+    // 118 / 105, 300 167 / 182, 64 channels 200 76 / 61, 1 500 213 / 203, 32 channels 1 000 99 / 88, 2 000 158 / 143, 3 000 194 / 197;
+    // single, 96 channels 24 71 / 60, 501 96 / 87, 1 000 165 / 152, 128 channels 256 88 / 77, 400 125 / 129, 64 channels 1 500 156 / 144,
+    // 32 channels 3 000 149 / 141; l <= 1 (layer 0 only), 128 channels double 107 201 / 198, 256 250 / 242, 500 442 / 443, single 200
+    // 150 / 142, 96 channels 600 303 / 309, 64 channels 1 000 258 / 253; l <= 2, 64 channels double 700 507 / 503.
+    bool chain_edges(int layer) const
+    {
+        if (!scalar_edges(layer, layer == 0 ? hm.T : H1.n / hm.K) || (layer == 1 && NLM() > 1)) return false;
+        if (split_nodes <= num_cus) return true;
+        if (sizeof(F) == 8) return hm.K <= 64 && split_nodes <= 2048;
+        return hm.K <= 64 || (hm.K == 96 && NLM() == 1);
+    }
+    bool chain1_messages() const { return chain_edges(1) && (size_t)E1 * hm.K * sizeof(F) <= msg_limit_bytes; }
+    // A1, M1, the tail and the adjoints back to dPhi1, the aggregation before and its adjoint behind them where that is so
+    void st_chain1(int N, bool zero_energies, bool zero_forces)
     {
         const size_t k = K();
+        if (chain_edges(1)) {
+            need(xyz, "xyz"); need(r, "r"); need(neigh_indices, "neigh_indices"); need_edges(N);
+            Phi1.size_to((size_t)N * NE() * k, stream);
+        }
+        messages_left = chain1_messages();
+        if (messages_left) msg.size_to((size_t)E1 * k, stream);
         A1.size_to((size_t)N * 16 * k, stream);
         M1.size_to((size_t)N * k, stream); M1_grad.size_to((size_t)N * 16 * k, stream);
         dPhi1.size_to(Phi1.n, stream);
@@ -971,12 +999,15 @@ struct Engine : EngineBase {
         p.Phi = Phi1.p; p.W = linA1.p; p.Wt = linA1T.p; p.coef = M1_slabs.p;
         p.M = M1.p; p.M_grad = M1_grad.p; p.out = dPhi1.p;
         const auto q = tail_params(N, zero_energies);
-        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain1<F, decltype(kc)::value>(p, q, hm.L_max, stream); }));
+        auto agg = agg_params(1, N);
+        agg.out = Phi1.p; agg.msg = messages_left ? msg.p : nullptr; agg.forces = node_forces.p; agg.accumulate_forces = zero_forces ? 0 : 1;
+        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain1<F, decltype(kc)::value>(p, q, chain_edges(1) ? &agg : nullptr, hm.L_max, stream); }));
         if (guard_status && q.rows > 0) guard_clear_enqueued = true;
         energies_copy = nullptr;
         pending_A1 = N; pending_A1_adj = N;
     }
-    // the messages (`add_messages`: those of the last layer-1 adjoint are not in H1_adj yet), M0_adj, A0_adj and dPhi0
+    // the messages (`add_messages`: those of the last layer-1 adjoint are not in H1_adj yet), M0_adj, A0_adj, dPhi0, and with chain_edges(0)
+    // the adjoint of the layer-0 aggregation, which writes the caller's copy of the forces as well
     void st_chain2(int N, bool add_messages)
     {
         const size_t k = K();
@@ -987,7 +1018,11 @@ struct Engine : EngineBase {
         auto p = chain_params(N);
         p.Wt = linA0T.p; p.WH1 = H1wT.p; p.coef = M0_slabs.p; p.A = A0.p; p.M = M0_adj.p; p.M_grad = M0_grad.p; p.out = to.p;
         p.msg = add_messages ? msg.p : nullptr; p.H1_adj = H1_adj.p; p.sstart = s_start.p; p.slist = s_list.p; p.spare = s_rank.p;
-        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain2<F, decltype(kc)::value>(p, hm.L_max, stream); }));
+        auto agg = agg_params(0, N);
+        agg.forces = node_forces.p; agg.accumulate_forces = 1; agg.forces_copy = forces_copy;
+        const bool edges = chain_edges(0);
+        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain2<F, decltype(kc)::value>(p, edges ? &agg : nullptr, hm.L_max, stream); }));
+        if (edges) forces_copy = nullptr;
         pending_A0_adj = N;
     }
     // A0 (or A1) and its contraction in one launch
@@ -1466,10 +1501,11 @@ struct Engine : EngineBase {
             HIPCHK(launch_fill<double>(node_energies.p, (long)N1, 0.0, stream));
             st_zbl(N1);
         }
-        stage_begin(ST_AGG0F); st_agg0_fwd(N); stage_end(ST_AGG0F);
+        const bool chain = use_chains(N);
+        if (chain && chain_edges(0)) stage_absent(ST_AGG0F);
+        else { stage_begin(ST_AGG0F); st_agg0_fwd(N); stage_end(ST_AGG0F); }
         pending_A0 = pending_A1 = -1;
         pending_M0_grad = recompute_M0_grad() ? N : -1;
-        const bool chain = use_chains(N);
         if (chain) {
             stage_begin(ST_A0LIN); st_chain0(N); stage_end(ST_A0LIN);
             stage_absent(ST_M0); stage_absent(ST_H1);
@@ -1484,19 +1520,27 @@ struct Engine : EngineBase {
         if (!chain) { stage_begin(ST_H1); st_H1(N, false); stage_end(ST_H1); }
         // the species groups cover the nodes of the current stages
         if (N1 < N) build_type_groups(N1);
-        stage_begin(ST_AGG1F); st_agg1_fwd(N1); stage_end(ST_AGG1F);
         if (chain) {
-            stage_begin(ST_A1); st_chain1(N1, !hm.has_zbl); stage_end(ST_A1);
+            if (chain_edges(1)) stage_absent(ST_AGG1F);
+            else { stage_begin(ST_AGG1F); st_agg1_fwd(N1); stage_end(ST_AGG1F); }
+            stage_begin(ST_A1); st_chain1(N1, !hm.has_zbl, !early_forces); stage_end(ST_A1);
             for (int st : {ST_M1, ST_H2, ST_READOUT, ST_REVH2, ST_REVM1, ST_REVA1}) stage_absent(st);
-            chain_messages = true; messages_left = false;
-            st_agg1_bwd(N1, !early_forces, false);
-            chain_messages = false;
+            if (messages_left) {
+                for (int st : {ST_AGG1B, ST_FSUM1, ST_SRED}) stage_absent(st);
+            } else {
+                chain_messages = true;
+                st_agg1_bwd(N1, !early_forces, false);
+                chain_messages = false;
+            }
             if (N1 < N) build_type_groups(N);
             stage_begin(ST_REVA0LIN); st_chain2(N, messages_left); stage_end(ST_REVA0LIN);
-            stage_absent(ST_REVH1); stage_absent(ST_REVM0);
-            finish_evaluation(N, N1, on_device);
+            for (int st : {ST_REVH1, ST_REVM0}) stage_absent(st);
+            if (!chain_edges(0)) st_agg0_bwd(N);
+            else for (int st : {ST_AGG0B, ST_FSUM0}) stage_absent(st);
+            finish_evaluation(N1, on_device);
             return;
         }
+        stage_begin(ST_AGG1F); st_agg1_fwd(N1); stage_end(ST_AGG1F);
         if (fused_contraction(1, N1)) {
             stage_begin(ST_A1); st_linear_contraction(1, N1); stage_end(ST_A1);
             stage_absent(ST_M1);
@@ -1534,12 +1578,12 @@ struct Engine : EngineBase {
         pending_A0_adj = fuse0 ? N : -1;
         st_scale(0, N, true);
         stage_begin(ST_REVA0LIN); st_A0_lin(N, true, fuse0); stage_end(ST_REVA0LIN);
-        finish_evaluation(N, N1, on_device);
+        st_agg0_bwd(N);
+        finish_evaluation(N1, on_device);
     }
     // the layer-0 adjoint, and what the caller's arrays still lack
-    void finish_evaluation(int N, int N1, bool on_device)
+    void finish_evaluation(int N1, bool on_device)
     {
-        st_agg0_bwd(N);
         // (a skipped evaluation: the readout launch has filled the forces with NaN, and every sum of partial forces
         // after it looks at the guard itself)
         if (guard_status && !guard_clear_enqueued) HIPCHK(launch_fill<int>(guard_status, 1, 0, stream));

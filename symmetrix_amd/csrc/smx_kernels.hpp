@@ -368,7 +368,7 @@ template <typename F>
 struct ChainParams {
     int N, K, T;
     const int* perm; const int* tstart;
-    const F* Phi;            // rows of the aggregation (0, 1)
+    const F* Phi;            // rows of the aggregation (0, 1), where it is not in the same launch
     const F* W; const F* Wt; // A-basis weights in operand order (0, 1), transposed ones (1, 2)
     const F* WH1;            // [L_max + 1][K][K] of H1 (0), its transposes (2)
     const F* coef;           // contraction coefficients by column tile: [species][column tile][monomials / V][16][V]
@@ -377,12 +377,12 @@ struct ChainParams {
     F* H1;                   // (0)
     F* out;                  // dPhi1 (1), dPhi0 (2)
     const F* msg; F* H1_adj; const int* sstart; int* slist; int* spare;     // (2)
-    unsigned lds_front, lds_part;    // set by the launchers
+    unsigned lds_front, lds_part, lds_edges;    // set by the launchers
 };
 inline bool chain_ok(int K) { return K == 32 || K == 64 || K == 96 || K == 128; }
-template <typename F, int K> hipError_t launch_chain0(ChainParams<F> p, int L_max, hipStream_t s);
-template <typename F, int K> hipError_t launch_chain1(ChainParams<F> p, const TailParams<F>& q, int L_max, hipStream_t s);
-template <typename F, int K> hipError_t launch_chain2(ChainParams<F> p, int L_max, hipStream_t s);
+template <typename F, int K> hipError_t launch_chain0(ChainParams<F> p, const AggParams<F>* agg, int L_max, hipStream_t s);
+template <typename F, int K> hipError_t launch_chain1(ChainParams<F> p, const TailParams<F>& q, const AggParams<F>* agg, int L_max, hipStream_t s);
+template <typename F, int K> hipError_t launch_chain2(ChainParams<F> p, const AggParams<F>* agg, int L_max, hipStream_t s);
 // f(K as a constant) for the numbers of channels above
 template <typename Fn>
 hipError_t with_channels(int K, Fn&& f)

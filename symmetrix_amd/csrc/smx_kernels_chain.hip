@@ -8,9 +8,13 @@
 // All of them touch the rows of one atom only, so a thread block takes one atom through all of its stages, with everything
 // between them in LDS.  As launches of their own the stages of a small system were a row of dependent launches of 6 to 20 us,
 // each of which waited for its first loads and filled a few CUs: 24 atoms, 96 channels, double precision 96 us in eight launches,
-// now 10 + 18 + 11; 107 atoms, 128 channels, l <= 1: 170 us in ten, now 17 + 43 + 33.
-// Bound by the weights, which every block reads once: 295 KB (96 channels, double, one A-basis product) at 64 bytes per cycle
-// and CU; between the products by the latency of dependent loads.
+// in chains 10 + 18 + 11; 107 atoms, 128 channels, l <= 1: 170 us in ten, in chains 17 + 43 + 33.
+// The aggregation before a chain and its adjoint behind it touch the rows of one receiver and its edges, and go into the same launch
+// for scalar features where that pays (smx_chain_edges.hpp; the rule is the caller's): 24 atoms 8 + 10, 7 + 18 + 13 and 11 + 12 us in
+// seven launches, now 17 + 33 + 19 in three, and a device-resident evaluation 87 -> 78; 256 atoms 102 -> 86, single precision 501
+// atoms 97 -> 87.
+// Bound by what one CU reads, at 64 bytes per cycle: 295 KB of weights (96 channels, double, one A-basis product), 470 KB of spline
+// coefficients (38 edges); between them by the latency of dependent loads.
 //
 // Products.  A wavefront owns 16 columns and 8 of the 16 (l, m): either l = 0 and 3 or l = 1 and 2, which is the same work.  Its
 // four 16-lane rows share the inner index (every row a quarter of each piece of 64 bytes) and are added up at the end.  Weights
@@ -19,7 +23,7 @@
 // further than a multiple of 128 apart in LDS: four rows and the four quarters of a piece meet all banks.
 // (Four atoms per block, which share every weight, came out behind the row tiles of k_linear where those fill the chip: 3 000
 // atoms, 96 channels, double: 53 + 106 + 84 us against 60 + 112 + 61.)
-#include "smx_edge_common.hpp"
+#include "smx_chain_edges.hpp"
 #include "smx_paths.hpp"
 #include "smx_poly_body.hpp"
 
@@ -119,7 +123,7 @@ struct Product {
     }
 };
 
-// Block -> atom, in the order of the species groups.
+// Block -> atom, in the order of the species groups: blocks that run together read the same weights.
 struct BlockAtom {
     int type, node;       // species (-1: nothing to do)
 };
@@ -217,6 +221,54 @@ __device__ __forceinline__ const unsigned char* coefficients(const F* coef, int 
 template <typename F> constexpr int kCoefAhead = sizeof(F) == 8 ? 3 : 4;
 template <typename F, int LM, int AHEAD = kCoefAhead<F>> using Coef = PolyCoef<F, LM, AHEAD>;
 
+// The polynomial of output slot 0 of all channels, value and gradient, in kSlices parts by groups of wavefronts:
+// part[slice][17][K] gets the sums over the slice, gradient before value; polynomial_value() adds them up.  Evaluations with one, two and
+// four slices, us: 96 channels, double 24 atoms 78.8 / 77.6 / 80.2, 107 81.8 / 80.7 / 83.6, 600 215 / 213 / 223; 64 channels 200 62.7 /
+// 61.1 / 63.5; single, 96 channels 501 89.6 / 88.6 / 89.5.
+constexpr int kSlices = 2;
+template <typename F, int K> constexpr size_t slice_bytes() { return (size_t)kSlices * 17 * K * sizeof(F); }
+template <typename F, int K, unsigned RS>
+struct SlicedPolynomial {
+    static constexpr int per = (K + 63) / 64 * 64;
+    static_assert(chain_threads(K) / per >= kSlices, "a group of wavefronts for every slice");
+    Coef<F, 0> coef;
+    int slot, k;
+    bool own;
+    __device__ __forceinline__ SlicedPolynomial(const F* from, int groups16, int type, int tid)
+        : coef(coefficients<F, K>(from, groups16, type, min(tid % per, K - 1)), 256), slot(__builtin_amdgcn_readfirstlane(tid / per)),
+          k(tid % per), own(tid % per < K) {}
+    __device__ __forceinline__ void begin()
+    {
+        static_for<0, kSlices>([&](auto sc) {
+            if (slot == decltype(sc)::value) coef.template begin<poly_slice<F, 0>(decltype(sc)::value, kSlices)>();
+        });
+    }
+    // rows: the variables, rows RS bytes apart
+    __device__ __forceinline__ void run(const unsigned char* rows, F* part)
+    {
+        if (slot >= kSlices) return;
+        F x[16], g[16], f = F(0);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) { x[q] = *reinterpret_cast<const F*>(rows + q * RS + min(k, K - 1) * sizeof(F)); g[q] = F(0); }
+        static_for<0, kSlices>([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            if (slot == s) poly_spec_run<F, 0, 0, false, kCoefAhead<F>, poly_slice<F, 0>(s, kSlices), poly_slice<F, 0>(s + 1, kSlices)>(coef, x, g, f, F(1));
+        });
+        if (!own) return;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) part[(slot * 17 + q) * K + k] = g[q];
+        part[(slot * 17 + 16) * K + k] = f;
+    }
+};
+template <typename F, int K>
+__device__ __forceinline__ F polynomial_value(const F* part, int t)      // entry t of [17][K]
+{
+    F s = part[t];
+#pragma unroll
+    for (int j = 1; j < kSlices; ++j) s += part[j * 17 * K + t];
+    return s;
+}
+
 // An atom's operand rows into LDS, 16 bytes at a time, all of a thread's words requested before the first is stored;
 // row_of(lme): the LDS row of a memory row
 template <typename F, int ROWS, int K, typename RowOf>
@@ -234,8 +286,9 @@ __device__ __forceinline__ void stage_rows(const F* from, unsigned char* dst, Ro
 }
 
 // ---------------------------------------------------------------------------
-template <typename F, int LH, int K>
-__global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain0(const ChainParams<F> p)
+// EDGES (here and below): the aggregation before the node-local stages, or its adjoint behind them, in the same launch.
+template <typename F, int LH, int K, bool EDGES>
+__global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain0(const ChainParams<F> p, const AggParams<F> agg)
 {
     constexpr int NP = (LH + 1) * (LH + 1), V = 16 / (int)sizeof(F), KC = 4 * V, T = chain_threads(K);
     constexpr unsigned RS = K * sizeof(F) + kPad;
@@ -243,64 +296,96 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain0(
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
     const BlockAtom b = block_atom(p.perm, p.tstart, p.T, lane);
     if (b.type < 0) return;
+    const size_t node = b.node;
+    const int type = b.type;
     F* xm = reinterpret_cast<F*>(smem + p.lds_front);       // [K][NP]: M0
     const int ct = wave >> 1, set = wave & 1, column = ct * 16 + r16;
+    if constexpr (EDGES) {
+        F sum[2];
+        ChainEdges<F, K>(wave, lane).forward(agg, (int)node, type, smem + p.lds_part, tid, lane, sum);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int t = tid + j * T, row = t / K;
+            *reinterpret_cast<F*>(smem + row * RS + (t - row * K) * sizeof(F)) = sum[j];
+            if constexpr (LH == 0) agg.out[node * 16 * K + t] = sum[j];     // (A0 may be asked for, and is formed from them)
+        }
+    }
     Product<F, true> prod;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int l = set == 0 ? 3 * j : 1 + j;
-        prod.wp[j] = p.W + ((size_t)l * p.T + b.type) * K * K + ((size_t)ct * (K / KC) * 64 + lane) * V;
+        prod.wp[j] = p.W + ((size_t)l * p.T + type) * K * K + ((size_t)ct * (K / KC) * 64 + lane) * V;
         prod.steps[j] = K / KC;
     }
     prod.begin();
-    stage_rows<F, 16, K>(p.Phi + (size_t)b.node * 16 * K, smem, [](unsigned row) { return row; });
+    if constexpr (!EDGES) stage_rows<F, 16, K>(p.Phi + node * 16 * K, smem, [](unsigned row) { return row; });
     __syncthreads();
     F out[2];
     prod.run(set, smem + lm_of_slot(set, r16 & 7) * RS + g * 16, out);
-    // polynomials: K threads each, in whole wavefronts
-    constexpr int per = (K + 63) / 64 * 64, slots = T / per;
-    const int slot = __builtin_amdgcn_readfirstlane(tid / per), k = min(tid - slot * per, K - 1);
-    const bool own = tid - slot * per < K;
-    const unsigned char* coef = coefficients<F, K>(p.coef, poly_spec_offset(NP) / V, b.type, k);
-    Coef<F, 0> first(coef, 256);
-    if (slot == 0) first.begin();
-    __syncthreads();
+    auto leave = [&]() {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int lm = lm_of_slot(set, slot_of_quad(j, g));
-        *reinterpret_cast<F*>(smem + lm * RS + column * sizeof(F)) = out[j];
-        if constexpr (LH > 0) p.A[((size_t)b.node * 16 + lm) * K + column] = out[j];
+        for (int j = 0; j < 2; ++j) {
+            const int lm = lm_of_slot(set, slot_of_quad(j, g));
+            *reinterpret_cast<F*>(smem + lm * RS + column * sizeof(F)) = out[j];
+            if constexpr (LH > 0) p.A[(node * 16 + lm) * K + column] = out[j];
+        }
+    };
+    if constexpr (LH == 0) {
+        SlicedPolynomial<F, K, RS> poly(p.coef, poly_spec_offset(NP) / V, type, tid);
+        poly.begin();
+        __syncthreads();
+        leave();
+        __syncthreads();
+        F* part = reinterpret_cast<F*>(smem + p.lds_part);
+        poly.run(smem, part);
+        __syncthreads();
+        for (int t = tid; t < 17 * K; t += T) {
+            const F s = polynomial_value<F, K>(part, t);
+            if (t < 16 * K) p.M_grad[node * 16 * K + t] = s;
+            else {
+                xm[t - 16 * K] = s;
+                p.M[node * K + t - 16 * K] = s;
+            }
+        }
+    } else {
+        // polynomials: K threads each, in whole wavefronts
+        constexpr int per = (K + 63) / 64 * 64, slots = T / per;
+        const int slot = __builtin_amdgcn_readfirstlane(tid / per), k = min(tid - slot * per, K - 1);
+        const bool own = tid - slot * per < K;
+        const unsigned char* coef = coefficients<F, K>(p.coef, poly_spec_offset(NP) / V, type, k);
+        Coef<F, 0> first(coef, 256);
+        if (slot == 0) first.begin();
+        __syncthreads();
+        leave();
+        __syncthreads();
+        static_for<0, NP>([&](auto pc) {
+            constexpr int lm = decltype(pc)::value;
+            if (lm % slots != slot) return;
+            F x[16], gr[16], f = F(0);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) { x[q] = *reinterpret_cast<const F*>(smem + q * RS + k * sizeof(F)); gr[q] = F(0); }
+            if constexpr (lm == 0) poly_spec_run<F, 0, 1, false>(first, x, gr, f, F(1));
+            else {
+                Coef<F, lm> next(coef, 256);
+                next.begin();
+                poly_spec_run<F, lm, 1, false>(next, x, gr, f, F(1));
+            }
+            if (!own) return;
+            xm[k * NP + lm] = f;
+            p.M[(node * NP + lm) * K + k] = f;
+        });
     }
-    __syncthreads();
-    static_for<0, NP>([&](auto pc) {
-        constexpr int lm = decltype(pc)::value;
-        if (lm % slots != slot) return;
-        F x[16], gr[16], f = F(0);
-#pragma unroll
-        for (int q = 0; q < 16; ++q) { x[q] = *reinterpret_cast<const F*>(smem + q * RS + k * sizeof(F)); gr[q] = F(0); }
-        if constexpr (lm == 0) poly_spec_run<F, 0, LH == 0 ? 0 : 1, false>(first, x, gr, f, F(1));
-        else {
-            Coef<F, lm> next(coef, 256);
-            next.begin();
-            poly_spec_run<F, lm, 1, false>(next, x, gr, f, F(1));
-        }
-        if (!own) return;
-        xm[k * NP + lm] = f;
-        p.M[((size_t)b.node * NP + lm) * K + k] = f;
-        if constexpr (LH == 0) {
-#pragma unroll
-            for (int q = 0; q < 16; ++q) p.M_grad[((size_t)b.node * 16 + q) * K + k] = gr[q];
-        }
-    });
     F* red = reinterpret_cast<F*>(smem);
     mix_rows<F, NP, LH + 1, K>(xm, p.WH1, red, tid);
-    for (int t = tid; t < NP * K; t += T) p.H1[(size_t)b.node * NP * K + t] = mixed<F, NP, K>(red, t);
+    for (int t = tid; t < NP * K; t += T) p.H1[node * NP * K + t] = mixed<F, NP, K>(red, t);
 }
 
 // ---------------------------------------------------------------------------
-template <typename F, int LH, int K>
-__global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(const ChainParams<F> p, const TailParams<F> q)
+// (EDGES: scalar hidden features with a diagonal coupling)
+template <typename F, int LH, int K, bool EDGES>
+__global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(const ChainParams<F> p, const TailParams<F> q, const AggParams<F> agg)
 {
+    static_assert(!EDGES || LH == 0, "scalar hidden features");
     using PT = Paths<LH>;
     constexpr int NLM = (LH + 1) * (LH + 1), NE = PT::NE, V = 16 / (int)sizeof(F), KC = 4 * V, S = mix_slices<1>();
     constexpr int T = chain_threads(K), width = NLM * K;
@@ -327,6 +412,7 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
     const BlockAtom b = block_atom(p.perm, p.tstart, p.T, lane);
     if (b.type < 0) return;
     const size_t node = b.node;
+    const int type = b.type;
     // LDS: operand rows, then the 16 rows of the A-basis in their place, then what the tail needs (in double), then the
     // adjoint rows; H1[l = 0] and M1 behind them
     double* red = reinterpret_cast<double*>(smem);                // [S][K]
@@ -347,12 +433,24 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
         prod.steps[j] = nel_of(l) * (K / KC);
         prod.wp[j] = p.W + (size_t)blocks_before(l) * K * K + ((size_t)ct * prod.steps[j] * 64 + lane) * V;
     }
-    prod.begin();
-    stage_rows<F, NE, K>(p.Phi + node * NE * K, smem, [&](unsigned lme) {
-        const int l = lme < (unsigned)lme0[1] ? 0 : (lme < (unsigned)lme0[2] ? 1 : (lme < (unsigned)lme0[3] ? 2 : 3));
-        const unsigned in = lme - lme_of(l);
-        return (unsigned)(l * l) + (l == 0 ? 0u : (l == 1 ? in / nel[1] : (l == 2 ? in / nel[2] : in / nel[3])));
-    });
+    if constexpr (EDGES) {
+        F sum[2];
+        ChainEdges<F, K>(wave, lane).forward(agg, (int)node, type, smem + p.lds_part, tid, lane, sum);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int t = tid + j * T, row = t / K;
+            *reinterpret_cast<F*>(smem + row * RS + (t - row * K) * sizeof(F)) = sum[j];
+            agg.out[node * 16 * K + t] = sum[j];
+        }
+        prod.begin();
+    } else {
+        prod.begin();
+        stage_rows<F, NE, K>(p.Phi + node * NE * K, smem, [&](unsigned lme) {
+            const int l = lme < (unsigned)lme0[1] ? 0 : (lme < (unsigned)lme0[2] ? 1 : (lme < (unsigned)lme0[3] ? 2 : 3));
+            const unsigned in = lme - lme_of(l);
+            return (unsigned)(l * l) + (l == 0 ? 0u : (l == 1 ? in / nel[1] : (l == 2 ? in / nel[2] : in / nel[3])));
+        });
+    }
     const bool own = tid < K;                  // this thread's channel
     const int k = own ? tid : 0;
     if (own) xh[k] = (double)q.H1[node * width + k];
@@ -362,29 +460,34 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
         const int lm = lm_of_slot(set, r16 & 7), l = lm_l(lm);
         prod.run(set, smem + (unsigned)(lme_of(l) + (lm - l * l) * nel_of(l)) * (K * sizeof(F)) + lm * kPad + g * 16, out);
     }
-    Coef<F, 0> coef(coefficients<F, K>(p.coef, poly_spec_offset(1) / V, b.type, k), 256);
-    if (own) coef.begin();
+    SlicedPolynomial<F, K, RS> poly(p.coef, poly_spec_offset(1) / V, type, tid);
+    poly.begin();
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < 2; ++j) *reinterpret_cast<F*>(smem + lm_of_slot(set, slot_of_quad(j, g)) * RS + column * sizeof(F)) = out[j];
     __syncthreads();
-    // M1; its gradient stays with the thread of the channel
-    F gr[16];
-    if (own) {
-        F x[16], f = F(0);
+    // M1; its gradient stays with the threads that formed it
+    F gr[2];
+    {
+        F* part = reinterpret_cast<F*>(smem + p.lds_part);
+        poly.run(smem, part);
+        __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 16; ++i) { x[i] = *reinterpret_cast<const F*>(smem + i * RS + k * sizeof(F)); gr[i] = F(0); }
-        poly_spec_run<F, 0, 0, false>(coef, x, gr, f, F(1));
-        xh[K + k] = (double)f;
-        p.M[node * K + k] = f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) p.M_grad[(node * 16 + i) * K + k] = gr[i];
+        for (int j = 0; j < 2; ++j) {
+            gr[j] = polynomial_value<F, K>(part, tid + j * T);
+            p.M_grad[node * 16 * K + tid + j * T] = gr[j];
+        }
+        if (own) {
+            const F f = polynomial_value<F, K>(part, 16 * K + k);
+            xh[K + k] = (double)f;
+            p.M[node * K + k] = f;
+        }
     }
     // two products with K x K weights at once: the lower half of the slices takes the first matrix, the upper the second
     constexpr int count = 2 * K / S;
     using TM = Mix<double, 1, 1, count, K>;
     const int sl = tid / (K / 2), pair = (tid - sl * (K / 2)) * 2, from = (sl % (S / 2)) * count;
-    const size_t typed = (size_t)b.type * K * K;
+    const size_t typed = (size_t)type * K * K;
     // H2 = H1[l = 0] . W_H1[type] + M1 . W_M1
     {
         TM mix(sl < S / 2 ? q.W_H1 + typed : q.W_M1, 0, pair, from);
@@ -399,7 +502,7 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
     const int back = tid / K, kb = tid - back * K;
     double v[16];
     if (back < 3) {
-        const double* from_hg = back == 0 ? q.W1 : (back == 1 ? q.V_H1 + (size_t)b.type * 16 * K : q.V_M1);
+        const double* from_hg = back == 0 ? q.W1 : (back == 1 ? q.V_H1 + (size_t)type * 16 * K : q.V_M1);
 #pragma unroll
         for (int h = 0; h < 16; ++h) v[h] = from_hg[h * K + kb];
     }
@@ -430,7 +533,7 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
 #pragma unroll
         for (int off = 8; off >= 1; off >>= 1) e += __shfl_xor(e, off, 64);
         if (tid == 0) {
-            const double en = (q.zero_energies ? 0.0 : q.node_energies[node]) + q.E0[b.type] + (e + dots[16]);
+            const double en = (q.zero_energies ? 0.0 : q.node_energies[node]) + q.E0[type] + (e + dots[16]);
             q.node_energies[node] = en;
             if (q.energies_copy) q.energies_copy[node] = en;
         }
@@ -461,10 +564,10 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
     }
     for (int t = K + tid; t < width; t += T) q.H1_adj[node * width + t] = F(0);
     __syncthreads();
-    if (own) {
-        const F m1_adj = (F)xh[K + k];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) *reinterpret_cast<F*>(smem + i * RS + k * sizeof(F)) = gr[i] * m1_adj;
+    for (int j = 0; j < 2; ++j) {
+        const int t = tid + j * T, row = t / K, c = t - row * K;
+        *reinterpret_cast<F*>(smem + row * RS + c * sizeof(F)) = gr[j] * (F)xh[K + c];
     }
     __syncthreads();
     // dPhi1 = A1_adj . W^T, output block by output block
@@ -479,6 +582,14 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
             const int lm = lm_of_slot(set, slot_of_quad(j, g)), l = lm_l(lm), n = nel_of(l);
             if (e < n) p.out[(node * NE + lme_of(l) + (lm - l * l) * n + e) * K + column] = o[j];
         }
+        if constexpr (EDGES) {
+            if (!agg.msg) return;          // (the messages do not fit their array: launches of their own)
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 2; ++j) *reinterpret_cast<F*>(smem + lm_of_slot(set, slot_of_quad(j, g)) * RS + column * sizeof(F)) = o[j];
+            __syncthreads();
+            ChainEdges<F, K>(wave, lane).template adjoint<true>(agg, (int)node, type, smem, RS, smem + p.lds_part, tid, lane);
+        }
     }
 }
 
@@ -490,8 +601,8 @@ template <int NP> constexpr int kMsgWords = NP == 1 ? 4 : 8;     // 16-byte word
 // per CU (K / 32 wavefronts per SIMD) l <= 1 spills none up to 96 channels; evaluations, us, as it is / so: 32 channels 200 atoms
 // 120 / 118, 1 000 243 / 246; 64 channels 48 117.5 / 117.2, 200 140 / 138, 768 288 / 294 (no second block on a CU); 96 channels,
 // where there is one block either way, 107 153 / 151, 500 324 / 320.
-template <typename F, int LH, int K>
-__global__ __launch_bounds__(chain_threads(K), LH == 0 ? chain_waves<F>(K) : 4) void k_chain2(const ChainParams<F> p)
+template <typename F, int LH, int K, bool EDGES>
+__global__ __launch_bounds__(chain_threads(K), LH == 0 ? chain_waves<F>(K) : 4) void k_chain2(const ChainParams<F> p, const AggParams<F> agg)
 {
     constexpr int NP = (LH + 1) * (LH + 1), V = 16 / (int)sizeof(F), KC = 4 * V, T = chain_threads(K), width = NP * K;
     constexpr unsigned RS = K * sizeof(F) + kPad;
@@ -502,6 +613,7 @@ __global__ __launch_bounds__(chain_threads(K), LH == 0 ? chain_waves<F>(K) : 4) 
     const BlockAtom b = block_atom(p.perm, p.tstart, p.T, lane);
     if (b.type < 0) return;
     const size_t node = b.node;
+    const int type = b.type;
     F* xm = reinterpret_cast<F*>(smem + p.lds_front);       // [K][NP]: H1_adj
     F* ym = xm + width;                                     // [K][NP]: M0_adj
     F* red = reinterpret_cast<F*>(smem);                    // messages, then partial sums, before the operand rows
@@ -510,7 +622,7 @@ __global__ __launch_bounds__(chain_threads(K), LH == 0 ? chain_waves<F>(K) : 4) 
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int l = set == 0 ? 3 * j : 1 + j;
-        prod.wp[j] = p.Wt + ((size_t)l * p.T + b.type) * K * K + ((size_t)ct * (K / KC) * 64 + lane) * V;
+        prod.wp[j] = p.Wt + ((size_t)l * p.T + type) * K * K + ((size_t)ct * (K / KC) * 64 + lane) * V;
         prod.steps[j] = K / KC;
     }
     // The messages to this atom, added to what is there in ascending edge order (the order of a sum by launches of their own,
@@ -608,7 +720,7 @@ __global__ __launch_bounds__(chain_threads(K), LH == 0 ? chain_waves<F>(K) : 4) 
                 constexpr int lm = decltype(pc)::value;
                 if (lm % slots != slot) return;
                 asm volatile("" ::: "memory");      // (the coefficients of the other polynomials stay where they are)
-                Coef<F, lm, 2> coef(coefficients<F, K>(p.coef, poly_spec_offset(NP) / V, b.type, k), 256);
+                Coef<F, lm, 2> coef(coefficients<F, K>(p.coef, poly_spec_offset(NP) / V, type, k), 256);
                 coef.begin();
                 poly_spec_run<F, lm, 2, false>(coef, x, gr, f, ym[k * NP + lm]);
             });
@@ -631,6 +743,13 @@ __global__ __launch_bounds__(chain_threads(K), LH == 0 ? chain_waves<F>(K) : 4) 
     prod.run(set, smem + lm_of_slot(set, r16 & 7) * RS + g * 16, o);
 #pragma unroll
     for (int j = 0; j < 2; ++j) p.out[(node * 16 + lm_of_slot(set, slot_of_quad(j, g))) * K + column] = o[j];
+    if constexpr (EDGES) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; ++j) *reinterpret_cast<F*>(smem + lm_of_slot(set, slot_of_quad(j, g)) * RS + column * sizeof(F)) = o[j];
+        __syncthreads();
+        ChainEdges<F, K>(wave, lane).template adjoint<false>(agg, (int)node, type, smem, RS, smem + p.lds_edges, tid, lane);
+    }
 }
 
 template <typename Kernel, typename... Args>
@@ -670,7 +789,7 @@ constexpr int kK = 32 * (SMX_CHAIN_PART / 2 % 4 + 1);
 
 #if SMX_CHAIN_PART / 8 == 0
 template <typename F, int K>
-hipError_t launch_chain0(ChainParams<F> p, int L_max, hipStream_t s)
+hipError_t launch_chain0(ChainParams<F> p, const AggParams<F>* agg, int L_max, hipStream_t s)
 {
     if (p.N <= 0) return hipSuccess;
     if (p.T <= 0) return hipErrorInvalidValue;
@@ -678,13 +797,18 @@ hipError_t launch_chain0(ChainParams<F> p, int L_max, hipStream_t s)
         constexpr int LH = decltype(lc)::value, NP = (LH + 1) * (LH + 1);
         constexpr size_t rows = (size_t)16 * (K * sizeof(F) + kPad), sums = (size_t)mix_slices<NP>() * NP * K * sizeof(F);
         p.lds_front = (unsigned)round16(std::max(rows, sums));
-        return launch_chain_t(k_chain0<F, LH, K>, (unsigned)p.N, chain_threads(K), p.lds_front + (size_t)NP * K * sizeof(F), s, p);
+        size_t lds = p.lds_front + (size_t)NP * K * sizeof(F);
+        p.lds_part = (unsigned)round16(lds);
+        if (LH == 0) lds = p.lds_part + slice_bytes<F, K>();
+        if (!agg) return launch_chain_t(k_chain0<F, LH, K, false>, (unsigned)p.N, chain_threads(K), lds, s, p, AggParams<F>{});
+        lds = std::max(lds, p.lds_part + ChainEdges<F, K>::fwd_bytes);
+        return launch_chain_t(k_chain0<F, LH, K, true>, (unsigned)p.N, chain_threads(K), lds, s, p, *agg);
     });
 }
-template hipError_t launch_chain0<chain_t, kK>(ChainParams<chain_t>, int, hipStream_t);
+template hipError_t launch_chain0<chain_t, kK>(ChainParams<chain_t>, const AggParams<chain_t>*, int, hipStream_t);
 #elif SMX_CHAIN_PART / 8 == 1
 template <typename F, int K>
-hipError_t launch_chain1(ChainParams<F> p, const TailParams<F>& q, int L_max, hipStream_t s)
+hipError_t launch_chain1(ChainParams<F> p, const TailParams<F>& q, const AggParams<F>* agg, int L_max, hipStream_t s)
 {
     if (q.rows <= 0) return hipSuccess;
     if (p.N <= 0 || p.T <= 0 || q.rows < q.N || q.N != p.N) return hipErrorInvalidValue;
@@ -693,13 +817,22 @@ hipError_t launch_chain1(ChainParams<F> p, const TailParams<F>& q, int L_max, hi
         constexpr size_t in = Paths<LH>::NE * K * sizeof(F) + 16 * kPad, rows = (size_t)16 * (K * sizeof(F) + kPad);
         constexpr size_t tail = ((size_t)(mix_slices<1>() + 1) * K + 33) * sizeof(double);
         p.lds_front = (unsigned)round16(std::max({in, rows, tail}));
-        return launch_chain_t(k_chain1<F, LH, K>, (unsigned)p.N, chain_threads(K), p.lds_front + (size_t)2 * K * sizeof(double), s, p, q);
+        p.lds_part = (unsigned)round16(p.lds_front + (size_t)2 * K * sizeof(double));
+        size_t lds = p.lds_part + slice_bytes<F, K>();
+        if constexpr (LH == 0) {
+            if (agg) {
+                lds = std::max({lds, p.lds_part + ChainEdges<F, K>::fwd_bytes, p.lds_part + ChainEdges<F, K>::bwd_bytes});
+                return launch_chain_t(k_chain1<F, LH, K, true>, (unsigned)p.N, chain_threads(K), lds, s, p, q, *agg);
+            }
+        }
+        if (agg) return hipErrorInvalidValue;
+        return launch_chain_t(k_chain1<F, LH, K, false>, (unsigned)p.N, chain_threads(K), lds, s, p, q, AggParams<F>{});
     });
 }
-template hipError_t launch_chain1<chain_t, kK>(ChainParams<chain_t>, const TailParams<chain_t>&, int, hipStream_t);
+template hipError_t launch_chain1<chain_t, kK>(ChainParams<chain_t>, const TailParams<chain_t>&, const AggParams<chain_t>*, int, hipStream_t);
 #else
 template <typename F, int K>
-hipError_t launch_chain2(ChainParams<F> p, int L_max, hipStream_t s)
+hipError_t launch_chain2(ChainParams<F> p, const AggParams<F>* agg, int L_max, hipStream_t s)
 {
     if (p.N <= 0) return hipSuccess;
     if (p.T <= 0) return hipErrorInvalidValue;
@@ -710,11 +843,15 @@ hipError_t launch_chain2(ChainParams<F> p, int L_max, hipStream_t s)
         p.lds_front = (unsigned)round16(std::max(rows, sums));
         size_t lds = p.lds_front + (size_t)2 * NP * K * sizeof(F);
         p.lds_part = (unsigned)round16(lds);
+        p.lds_edges = (unsigned)round16(rows);
         if (LH > 0) lds = p.lds_part + (size_t)kPolySlots * 16 * K * sizeof(F);
-        return launch_chain_t(k_chain2<F, LH, K>, (unsigned)p.N, chain_threads(K), std::max(lds, stage), s, p);
+        lds = std::max(lds, stage);
+        if (!agg) return launch_chain_t(k_chain2<F, LH, K, false>, (unsigned)p.N, chain_threads(K), lds, s, p, AggParams<F>{});
+        lds = std::max(lds, p.lds_edges + ChainEdges<F, K>::bwd_bytes);
+        return launch_chain_t(k_chain2<F, LH, K, true>, (unsigned)p.N, chain_threads(K), lds, s, p, *agg);
     });
 }
-template hipError_t launch_chain2<chain_t, kK>(ChainParams<chain_t>, int, hipStream_t);
+template hipError_t launch_chain2<chain_t, kK>(ChainParams<chain_t>, const AggParams<chain_t>*, int, hipStream_t);
 #endif
 
 }  // namespace smx

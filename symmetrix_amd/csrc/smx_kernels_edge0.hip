@@ -22,18 +22,6 @@ namespace smx {
 
 namespace {
 
-// a b + c into a register of its own.  Left alone, the compiler copies c first and accumulates in the copy where the registers of c
-// belong to the next load: 24 copies among the 218 instructions of the single-precision adjoint for 96 channels.
-__device__ __forceinline__ float fma_apart(float a, float b, float c)
-{
-    float r;
-    asm("v_fma_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ double fma_apart(double a, double b, double c) { return fma(a, b, c); }
-
-constexpr int lm_of_tile(int t) { return t == 0 ? 0 : (t == 1 ? 1 : (t == 2 ? 4 : (t == 3 ? 8 : (t == 4 ? 9 : 13)))); }
-
 // Wavefronts per SIMD (thread blocks per CU) of the adjoint: what the registers of its channels allow.  20 011 atoms, 96 channels,
 // single: adjoints of 275 and 264 us with two, 253 and 237 with three; double, two channels per lane, layer 0: 600 atoms, 64 and 128
 // channels 24 / 21 and 33 / 30, 10 000 atoms 243 / 231 and 455 / 441, 24 999 atoms 1 033 / 1 008 (l <= 1), 50 000 atoms 2 828 /
@@ -61,17 +49,6 @@ struct Lds0 {
     static constexpr size_t per_wave = (val_bytes + head_bytes + sum_bytes + 15) / 16 * 16;
     static_assert(!BWD || 4 * per_wave * BPC <= 160 * 1024, "the thread blocks of a CU");
 };
-
-// interval, argument and rows of an edge; offsets of its table and sender rows in bytes (32 bits: launch_agg0_ok)
-template <typename F>
-__device__ __forceinline__ void edge_offsets(const AggParams<F>& a, int e, int ti, unsigned row_bytes, unsigned sender_bytes, F* xs,
-                                             unsigned* toff, unsigned* goff, int slot)
-{
-    double r, x;
-    int row, grow;
-    edge_head(a, e, ti, r, x, row, grow);
-    xs[slot] = (F)x; toff[slot] = (unsigned)row * row_bytes; goff[slot] = (unsigned)grow * sender_bytes;
-}
 
 // ---------------------------------------------------------------------------
 template <typename F, int CPL, int EW>
@@ -259,36 +236,6 @@ __global__ __launch_bounds__(256, 2) void k_agg0_fwd(const AggParams<F> a, const
 #pragma unroll
             for (int j = 0; j < NR; ++j) a.out[((size_t)i * 16 + EW * j + sub) * K + k[c]] = out[c][j];
         }
-}
-
-// Three sums over the lanes of each half-wavefront (EW = 2) or over all lanes (EW = 1).  On return lane 0 of the half
-// holds s, lane 16 g1, lane 8 g2.  In single precision two lanes (up to eight channels) are added as they are, everything beyond
-// in double: the forces come from sums over all channels, which cancel.
-template <int EW, typename F>
-__device__ __forceinline__ double edge_sum3(F s, F g1, F g2, int lane)
-{
-    if constexpr (EW == 1) {
-        static_assert(sizeof(F) == 8, "half-wavefronts in single precision");
-        F t = g2;
-        swap_halves(s, t);
-        F a = s + t;                     // lower half s, upper half g2
-        F u = g1;
-        swap_halves(g1, u);
-        F b = g1 + u;                    // g1 in both
-        swap_rows(a, b);                 // rows 0, 2: a, rows 1, 3: b
-        F x = a + b;
-        x = row_sum_strided<1>(x);       // row 0: s, row 1: g1, row 2: g2, row 3: g1
-        return x;
-    } else {
-        F t = g2;
-        swap_rows(s, g1);
-        swap_rows(g2, t);
-        F x = s + g1, y = g2 + t;        // rows 0, 2: s; rows 1, 3: g1; y: g2 in every row
-        const F mine = (lane & 8) ? y : x, other = (lane & 8) ? x : y;      // the lane eight further on wants the other one
-        double z = (double)mine + (double)row_rotate<8>(other);
-        z += half_mirror(z); z += lane_xor1(z); z += lane_xor2(z);
-        return z;
-    }
 }
 
 // ---------------------------------------------------------------------------

@@ -32,18 +32,22 @@ struct PolyCoef {
                     buf[GI % (AHEAD + 1)][j] = *reinterpret_cast<const V4*>(slab_k + (size_t)(ROW0 + r0 + j) * row_stride_bytes);
         }
     }
+    template <int FROM = 0>
     __device__ __forceinline__ void begin()
     {
-        static_for<0, AHEAD>([&](auto gc) { request<decltype(gc)::value>(); });
+        static_for<FROM, FROM + AHEAD>([&](auto gc) { request<decltype(gc)::value>(); });
     }
 };
+// Groups of coefficients from which slice `slice` of `slices` of a polynomial begins.
+template <typename F, int LM> constexpr int poly_slice(int slice, int slices) { return (PolyTable<LM>::N + spec_group<F>() - 1) / spec_group<F>() * slice / slices; }
 
 // MODE 0: values and gradients (M, M_grad); 1: values only; 2: adjoint, A_adj = sum over the polynomials of
 // M_adj[polynomial] * gradient, recomputed from the variables (the coefficient is scaled, the value dropped).
 //
 // NESTED: the sums in the form below; else monomial by monomial, nearly twice the instructions, which do not wait for each other:
 // for a polynomial per thread on an otherwise idle SIMD (24 to 501 atoms: evaluations 1 to 2 % shorter).
-template <typename F, int LM, int MODE, bool NESTED, int AHEAD>
+// FROM, TO: the groups of coefficients that are taken (monomial by monomial only: their sums do not need each other).
+template <typename F, int LM, int MODE, bool NESTED, int AHEAD, int FROM = 0, int TO = PolyCoef<F, LM, AHEAD>::NG>
 __device__ __forceinline__ void poly_spec_run(PolyCoef<F, LM, AHEAD>& w16, F (&x)[16], F (&g)[16], F& f, F madj)
 {
     using TB = PolyTable<LM>;
@@ -53,12 +57,13 @@ __device__ __forceinline__ void poly_spec_run(PolyCoef<F, LM, AHEAD>& w16, F (&x
     //     g_c += w_pqc x_p x_q,  g_q += x_p S_pq,  g_p += Q_p
     // (the product rule holds as written for repeated indices): two multiply-adds per monomial, three more per pair, two per p,
     // about 300 for the value and gradient of a polynomial of 90 to 112 monomials.  Monomial by monomial they were 530 to 640.
+    static_assert(!NESTED || (FROM == 0 && TO == NG), "nested sums are whole ones");
     F tp, pr, S, Q;      // x_p (times M_adj in mode 2), tp x_q
     // The next group is requested before the current one is used; compiler and scheduling barriers keep all groups from being
     // requested at once (the variables would spill).
-    static_for<0, NG>([&](auto gc) {
+    static_for<FROM, TO>([&](auto gc) {
         constexpr int gi = decltype(gc)::value;
-        w16.template request<gi + AHEAD>();
+        if constexpr (gi + AHEAD < TO) w16.template request<gi + AHEAD>();
         asm volatile("" ::: "memory");     // no read of a later group moves above this line
         __builtin_amdgcn_sched_barrier(0);
         constexpr int end = gi * G + G < TB::N ? gi * G + G : TB::N;
