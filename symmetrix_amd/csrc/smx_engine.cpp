@@ -597,7 +597,7 @@ struct Engine : EngineBase {
 
     // ---- input checks of an evaluation.  flags[0]: stage-level calls (read back at once); flags[2]: the word the checks
     // of the running evaluation raise; flags[3]: its copy for the kernels after the list preparation ("live": raised ->
-    // energies and forces are NaN); flags[4]: ticket of the list preparation.  The evaluation clears flags[2] again in its
+    // energies and forces are NaN); flags[4]: ticket of the list preparation, flags[5]: of the virial (both zero between launches).  The evaluation clears flags[2] again in its
     // readout launch, after the last reader, so every evaluation, eager or a replayed graph, starts from a clean word.
     // sticky: what failed and has not been reported, in host memory, written by the list preparation and read by the next
     // call that waits for the stream (a host-array call reports at its own end).
@@ -1418,7 +1418,7 @@ struct Engine : EngineBase {
             fuse_reverse_H1 = chain_messages = false;
             // checks of the failed call may have raised the word that only its readout launch would have cleared
             if (guard_status && !guard_clear_enqueued) (void)launch_fill<int>(guard_status, 1, 0, stream);
-            (void)launch_fill<int>(flags.p + 4, 1, 0, stream);
+            (void)launch_fill<int>(flags.p + 4, 2, 0, stream);
             guard_status = nullptr;
             if (evaluating) forget_evaluation();
             evaluating = false;
@@ -1909,6 +1909,7 @@ struct Engine : EngineBase {
         if (d_virial) {
             rf_part.size_to((size_t)6 * force_gather_blocks(atoms), stream);
             g.partial = rf_part.p;
+            g.ticket = flags.p + 5;
         }
         HIPCHK(launch_force_gather(g, d_virial, stream));
     }

@@ -419,6 +419,7 @@ struct ForceGather {
     const double* forces; const double* xyz;         // [E][3] (xyz for the virial only)
     double* atom_forces;                             // [num_atoms][3] or null
     double* partial;                                 // [force_gather_blocks][6], needed for the virial, else null
+    int* ticket;                                     // with partial: a word that is zero, and is zero again afterwards
     const int* flag;                                 // raised, or ...
     const int* skipped;                              // ... this one: the outputs are NaN (each may be null)
     const int* senders;                              // sender atom of every edge, where send_list is another array's: compared,

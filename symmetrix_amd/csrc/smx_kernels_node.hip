@@ -811,8 +811,11 @@ __device__ __forceinline__ void add_virial(double (&v)[6], const double* d, cons
     v[0] += x * f[0]; v[1] += y * f[1]; v[2] += z * f[2];
     v[3] += 0.5 * (x * f[1] + y * f[0]); v[4] += 0.5 * (x * f[2] + z * f[0]); v[5] += 0.5 * (y * f[2] + z * f[1]);
 }
+// The block that finishes last adds up the partial sums of the virial, in a fixed order.  (A launch of its own for that: 4 to 5 us of a
+// small evaluation.)  The sums and the count of finished blocks go past the L2 of a die, by themselves: a fence would write back and
+// drop everything in it.
 template <bool BEHIND>
-__global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
+__global__ __launch_bounds__(256) void k_force_gather(const ForceGather a, double* virial)
 {
     __shared__ __align__(16) int bucket[4][GATHER_CAP];
     __shared__ double red[4][6];
@@ -860,21 +863,33 @@ __global__ __launch_bounds__(256) void k_force_gather(const ForceGather a)
         const double t = wave_sum(v[q]);
         if (lane == 0) red[wave][q] = t;
     }
+    __shared__ int last;
     __syncthreads();
-    if (threadIdx.x < 6)
-        a.partial[(size_t)blockIdx.x * 6 + threadIdx.x] =
-            (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
-}
-// the blocks' partial sums in a fixed order
-__global__ __launch_bounds__(384) void k_virial_finish(const double* partial, int nblocks, const int* flag, const int* skipped,
-                                                      double* virial)
-{
-    const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const bool nothing = no_result(flag, skipped);
-    double v = 0.0;
-    for (int b = lane; b < nblocks; b += 64) v += partial[(size_t)b * 6 + q];
-    v = wave_sum(v);
-    if (lane == 0) virial[q] = nothing ? __builtin_nan("") : v;
+    if (wave == 0) {
+        if (lane < 6)
+            __hip_atomic_store(a.partial + (size_t)blockIdx.x * 6 + lane, (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // the sums have arrived before the block counts as finished
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (lane == 0) last = __hip_atomic_fetch_add(a.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    for (int q = wave; q < 6; q += 4) {
+        double t = 0.0;
+        const int n = (int)gridDim.x;
+        for (int b0 = lane; b0 < n; b0 += 8 * 64) {
+            double x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                x[j] = __hip_atomic_load(a.partial + (size_t)min(b0 + 64 * j, n - 1) * 6 + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) t += b0 + 64 * j < n ? x[j] : 0.0;
+        }
+        t = wave_sum(t);
+        if (lane == 0) virial[q] = nothing ? __builtin_nan("") : t;
+    }
+    if (threadIdx.x == 0) *a.ticket = 0;
 }
 }  // namespace
 
@@ -882,9 +897,9 @@ int force_gather_blocks(int num_atoms) { return std::min(std::max((num_atoms + 3
 hipError_t launch_force_gather(const ForceGather& g, double* virial, hipStream_t s)
 {
     const int nb = force_gather_blocks(g.num_atoms);
-    if (g.num_edges > g.node_edges) hipLaunchKernelGGL(k_force_gather<true>, dim3(nb), dim3(256), 0, s, g);
-    else hipLaunchKernelGGL(k_force_gather<false>, dim3(nb), dim3(256), 0, s, g);
-    if (virial) hipLaunchKernelGGL(k_virial_finish, dim3(1), dim3(384), 0, s, g.partial, nb, g.flag, g.skipped, virial);
+    if ((g.partial != nullptr) != (virial != nullptr) || (virial && !g.ticket)) return hipErrorInvalidValue;
+    if (g.num_edges > g.node_edges) hipLaunchKernelGGL(k_force_gather<true>, dim3(nb), dim3(256), 0, s, g, virial);
+    else hipLaunchKernelGGL(k_force_gather<false>, dim3(nb), dim3(256), 0, s, g, virial);
     return hipGetLastError();
 }
 

@@ -19,7 +19,7 @@ constexpr int kVirialBlocks = 2048;   // most that launch_force_gather leaves pa
 
 constexpr size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 // layout of the scratch array (byte offsets, every part 256-byte aligned)
-constexpr size_t kOffFlag = 0;                                                          // int[64]
+constexpr size_t kOffFlag = 0;                                                          // int[64]: range flag, ticket
 constexpr size_t kOffCount = kOffFlag + 256;                                            // int[atoms]: counters
 constexpr size_t kOffSendStart = kOffCount + align256((size_t)kMaxAtoms * sizeof(int));     // int[atoms + 1]
 constexpr size_t kOffBlockSums = kOffSendStart + align256(((size_t)kMaxAtoms + 1) * sizeof(int)); // int[atoms / 1024 + 2]
@@ -109,11 +109,11 @@ extern "C" int smx_reduce_forces_device_noalloc(smx_model* m, int num_atoms, con
     const long E = v.num_edges;
     // an out-of-range sender index cannot be reported through a return code without a host synchronisation: the outputs
     // are NaN instead
-    hipError_t e = smx::launch_fill<int>(flag, 1, 0, s);
+    hipError_t e = smx::launch_fill<int>(flag, 2, 0, s);
     smx::ForceGather g{};
     g.num_atoms = num_atoms; g.num_nodes = v.num_receivers; g.first_neigh = v.first_neigh; g.node_edges = v.receiver_edges; g.num_edges = E;
     g.forces = v.node_forces; g.xyz = v.xyz; g.atom_forces = d_atom_forces; g.flag = flag; g.skipped = v.skipped;
-    if (d_virial) g.partial = partial;
+    if (d_virial) { g.partial = partial; g.ticket = flag + 1; }
     if (d_atom_forces) {
         if (e == hipSuccess) e = smx::launch_fill<int>(count, num_atoms, 0, s);
         if (e == hipSuccess)
