@@ -23,6 +23,11 @@ __device__ __forceinline__ void fmac_lane(double& acc, double b, double v)
 {
     asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(b), "v"(v), "n"(N));
 }
+template <int N>
+__device__ __forceinline__ void fmac_lane(float& acc, float b, float v)
+{
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(b), "v"(v), "n"(N));
+}
 
 // Loads and stores of a wavefront's rows: an address that is the same for all lanes, held in scalar registers, plus a 32-bit
 // offset per lane.

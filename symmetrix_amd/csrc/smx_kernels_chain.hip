@@ -33,12 +33,6 @@ namespace smx {
 
 namespace {
 
-template <int N>
-__device__ __forceinline__ void fmac_lane(float& acc, float b, float v)
-{
-    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(b), "v"(v), "n"(N));
-}
-
 constexpr int kPad = 64;       // bytes behind a row in LDS
 __device__ __forceinline__ int lm_of_slot(int set, int slot) { return set == 0 ? (slot == 0 ? 0 : 8 + slot) : 1 + slot; }
 __device__ __forceinline__ int slot_of_quad(int quad, int g) { return 4 * quad + ((g & 1) << 1 | g >> 1); }

@@ -42,7 +42,8 @@ constexpr int kEdgeStride = kChunk + 2;
 
 // Which entry of B[path][m][m2] (and of its two tangential derivatives) every lane and register holds.
 //   matrix form:  register g / 16, lanes 4 (g % 16) + i hold row 4 tile + i of group g; a group is one matrix
-//                 instruction: (path, row tile, inner index).  Forward: rows m, inner m2; adjoint: rows 3 m2 + t, inner m.
+//                 instruction: (path, row tile, inner index).  Forward: rows m, inner m2; adjoint: rows 3 m2 + t, inner m;
+//                 odd rows behind them in DPP form, v = odd_off + m.
 //   DPP form:     register v / 16, lane v % 16 of every row: v = 3 (entry_off + m n2 + m2) + t, forward entry_off + m n2 + m2
 // CP: a path of the constant harmonic (l1 = 0, so l = l2) has none where it couples like with like only, as an equivariant model
 // does: u[m2] = c d[m2] needs no product with a block and has no tangential part.  10 of the 88 rows and columns for l <= 1, 35 of
@@ -56,7 +57,15 @@ struct BlockLayout {
     static constexpr int nm(int p) { return 2 * PT::l(p) + 1; }
     static constexpr int rows(int p) { return BWD ? 3 * n2(p) : nm(p); }
     static constexpr int inner(int p) { return BWD ? nm(p) : n2(p); }
-    static constexpr int tiles(int p) { return in(p) ? (rows(p) + 3) / 4 : 0; }
+    // The ninth of nine rows has no tile of its own: a multiply-add with a lane broadcast costs half of a matrix instruction.
+    static constexpr bool odd(int p) { return MATRIX && BWD && in(p) && rows(p) > 4 && rows(p) % 4 == 1; }
+    static constexpr int tiles(int p) { return in(p) ? (odd(p) ? rows(p) / 4 : (rows(p) + 3) / 4) : 0; }
+    static constexpr int odd_off(int p)
+    {
+        int n = 0;
+        for (int q = 0; q < p; ++q) n += odd(q) ? inner(q) : 0;
+        return n;
+    }
     static constexpr int entry_off(int p)
     {
         int n = 0;
@@ -79,7 +88,8 @@ struct BlockLayout {
     static constexpr int TILES = tile_off(PT::P);
     static constexpr int REGS = MATRIX ? (group_off(PT::P) + 15) / 16 : (entry_off(PT::P) * (BWD ? 3 : 1) + 15) / 16;
     static constexpr int LANES = MATRIX ? 64 : 16;      // lanes that hold different entries
-    static constexpr int NV = REGS * LANES;
+    static constexpr int ODD_REGS = (odd_off(PT::P) + 15) / 16;      // of the odd rows: every 16 lanes hold the same
+    static constexpr int NV = REGS * LANES + ODD_REGS * 16;
     struct Table {
         short entry[NV];           // index into B, or -1: zero
         unsigned char comp[NV];    // 0: B, 1, 2: derivative along the first, second tangent
@@ -92,6 +102,12 @@ struct BlockLayout {
             if (!in(p)) continue;
             const int N2 = n2(p), NM = nm(p), bo = PT::boff(p), eo = entry_off(p), go = group_off(p), R = rows(p), IN = inner(p);
             if (MATRIX) {
+                if (odd(p))
+                    for (int in = 0; in < IN; ++in) {
+                        const int v = REGS * LANES + odd_off(p) + in;
+                        t.entry[v] = (short)(bo + in * N2 + (R - 1) / 3);
+                        t.comp[v] = (unsigned char)((R - 1) % 3);
+                    }
                 for (int tl = 0; tl < tiles(p); ++tl)
                     for (int in = 0; in < IN; ++in)
                         for (int i = 0; i < 4; ++i) {
@@ -122,7 +138,7 @@ struct EdgeLds {
     using BL = BlockLayout<LMAXH, BWD, kMatrix<F>, CP>;
     static constexpr int NY = BWD ? 48 : 16;     // harmonics (and their two tangential derivatives) of an edge
     // edges whose blocks are in LDS at a time: as many as leave room for two thread blocks on a CU
-    static constexpr int SUB = BL::NV * (int)sizeof(F) > 3000 ? 2 : (BL::NV * (int)sizeof(F) > 1000 ? 4 : 8);
+    static constexpr int SUB = BL::NV * (int)sizeof(F) > 2600 ? 2 : (BL::NV * (int)sizeof(F) > 1000 ? 4 : 8);
     static constexpr size_t lists = ((size_t)BL::NV * (2 * sizeof(double) + sizeof(int)) + 15) / 16 * 16;
     static constexpr size_t y_bytes = (size_t)NY * kEdgeStride * sizeof(double);
     static constexpr size_t frame_bytes = BWD ? (size_t)kChunk * 10 * sizeof(double) : 0;    // direction over r, tangents
@@ -601,9 +617,11 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                 }
                 const char* next = uniform_row(a.tabK, rows[le + 1], row_bytes);
                 const F* Bp = vals + (size_t)(le - sb) * BL::NV + (lane & (BL::LANES - 1));
-                F B[BL::REGS];
+                F B[BL::REGS], Bodd[BL::ODD_REGS + 1];
 #pragma unroll
                 for (int j = 0; j < BL::REGS; ++j) B[j] = Bp[j * BL::LANES];
+#pragma unroll
+                for (int j = 0; j < BL::ODD_REGS; ++j) Bodd[j] = vals[(size_t)(le - sb) * BL::NV + BL::REGS * BL::LANES + j * 16 + (lane & 15)];
                 F V[CPL][NLM][4];     // message, R u.t1, R u.t2, R' u
                 if constexpr (!MX) {
 #pragma unroll
@@ -637,8 +655,9 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                                 s[3] = starts ? Rd[c] * dm : s[3] + Rd[c] * dm;
                             }
                     } else if constexpr (MX) {
-                        constexpr int T = BL::tiles(p);
+                        constexpr int T = BL::tiles(p), R3 = BL::rows(p);
                         f32x4 u[CPL][T];
+                        F uodd[CPL];
                         static_for<0, 2 * l + 1>([&](auto mc) {
                             constexpr int m = decltype(mc)::value;
                             static_for<0, T>([&](auto tc) {
@@ -649,6 +668,15 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                                                                                  m == 0 ? f32x4{0, 0, 0, 0} : u[c][t], 4, g % 16, 0);
                             });
                         });
+                        if constexpr (BL::odd(p)) {
+#pragma unroll
+                            for (int c = 0; c < CPL; ++c) uodd[c] = F(0);
+                            static_for<0, 2 * l + 1>([&](auto mc) {
+                                constexpr int m = decltype(mc)::value, v = BL::odd_off(p) + m;
+#pragma unroll
+                                for (int c = 0; c < CPL; ++c) fmac_lane<v % 16>(uodd[c], Bodd[v / 16], d[c][lme0 + m * es]);
+                            });
+                        }
 #pragma unroll
                         for (int c = 0; c < CPL; ++c)
 #pragma unroll
@@ -656,7 +684,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                                 F* s = V[c][l2 * l2 + m2];
 #pragma unroll
                                 for (int t = 0; t < 3; ++t) {
-                                    const F uv = u[c][(3 * m2 + t) / 4][(3 * m2 + t) % 4];
+                                    const F uv = BL::odd(p) && 3 * m2 + t == R3 - 1 ? uodd[c] : u[c][(3 * m2 + t) / 4 < T ? (3 * m2 + t) / 4 : 0][(3 * m2 + t) % 4];
                                     s[t] = (t == 0 ? starts : starts_t) ? R[c] * uv : s[t] + R[c] * uv;
                                     if (t == 0) s[3] = starts ? Rd[c] * uv : s[3] + Rd[c] * uv;
                                 }
