@@ -1,0 +1,45 @@
+"""Adjoints of the edge aggregations over the channels and receivers at which their sums are formed in other ways: four, two and one
+wavefront per receiver, one to three channels per lane, with messages and without, l <= 1 and 2 on rows of three that end in the
+ninth.  Copies of one small system that do not see each other: each must give what the oracle gives for one of them."""
+import numpy as np
+import pytest
+
+from tests import helpers as H
+from tests.test_gpu_parity import TOL
+
+pytestmark = pytest.mark.gpu
+
+ARRAYS = ["Phi1_adj", "H1_adj", "A0_adj"]
+
+
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("K,L_max", [(40, 0), (64, 0), (96, 0), (128, 0), (64, 1), (96, 1), (128, 1), (64, 2), (128, 2)])
+def test_copies_of_one_system(tmp_models, K, L_max, dtype):
+    import torch
+    assert torch.cuda.is_available()
+    from oracle.oracle import OracleMACE
+    from symmetrix_amd.mace import MACE
+    model = H.tiny_model(K=K, L_max=L_max, n_pts=32, seed=K + L_max, r_cut=3.5, pair=False)
+    rng = np.random.default_rng(K + L_max)
+    degree = np.array([0, 1, 5, 15, 31, 46, 63, 8], np.int32)
+    n, E = len(degree), int(degree.sum())
+    species = rng.integers(0, 3, n).astype(np.int32)
+    senders = rng.integers(0, n, E).astype(np.int32)
+    x = rng.normal(size=(E, 3))
+    x *= (rng.uniform(1.0, 3.4, E) / np.linalg.norm(x, axis=1))[:, None]
+    r = np.linalg.norm(x, axis=1)
+    orc = OracleMACE(model)
+    orc.compute_node_energies_forces(n, species, degree, senders, species[senders], x.ravel(), r)
+    eng = MACE(H.write_model(model, tmp_models / f"adjoints_{K}_{L_max}.json"), dtype)
+    for copies in (75, 325, 790):
+        print(f"K={K} L_max={L_max} receivers={n * copies} edges={E * copies} {dtype}", flush=True)
+        shifted = (senders[None, :] + n * np.arange(copies, dtype=np.int32)[:, None]).ravel().astype(np.int32)
+        eng.compute_node_energies_forces(n * copies, np.tile(species, copies), np.tile(degree, copies), shifted,
+                                         np.tile(species[senders], copies), np.tile(x.ravel(), copies), np.tile(r, copies))
+        for name in ARRAYS:
+            want = np.asarray(getattr(orc, name)).reshape(n, -1)
+            got = np.asarray(getattr(eng, name)).reshape(copies, n, -1)
+            assert np.abs(got - want).max() <= TOL[dtype]["inter"] * 10 * max(1.0, np.abs(want).max()), name
+        want = orc.node_forces.reshape(E, 3)
+        got = eng.node_forces.reshape(copies, E, 3)
+        assert np.abs(got - want).max() <= TOL[dtype]["F"] * max(1.0, np.abs(want).max())
