@@ -210,16 +210,17 @@ struct ChainEdges {
                         V[1] = l == 1 ? R * u[1] : V[1] + R * u[1];
                         V[2] = l == 1 ? R * u[2] : V[2] + R * u[2];
                     } else {
-                        F u0 = F(0);
-                        if constexpr (l == 1) { V[1] = F(0); V[2] = F(0); }
+                        // as k_agg0_bwd: the same bits with the edges in the chain and without
+                        F u[3] = {F(0), F(0), F(0)};
                         static_for<l * l, (l + 1) * (l + 1)>([&](auto qc) {
                             constexpr int q = decltype(qc)::value, v = 3 * q;
-                            fmac_lane<v % 16>(u0, B[v / 16], d[q]);
-                            const F rd = R * d[q];
-                            fmac_lane<(v + 1) % 16>(V[1], B[(v + 1) / 16], rd);
-                            fmac_lane<(v + 2) % 16>(V[2], B[(v + 2) / 16], rd);
+                            fmac_lane<v % 16>(u[0], B[v / 16], d[q]);
+                            fmac_lane<(v + 1) % 16>(u[1], B[(v + 1) / 16], d[q]);
+                            fmac_lane<(v + 2) % 16>(u[2], B[(v + 2) / 16], d[q]);
                         });
-                        V[0] += R * u0; V[3] += Rd * u0;
+                        V[0] += R * u[0]; V[3] += Rd * u[0];
+                        V[1] = l == 1 ? R * u[1] : V[1] + R * u[1];
+                        V[2] = l == 1 ? R * u[2] : V[2] + R * u[2];
                     }
 #pragma unroll
                     for (int t = MSG ? 0 : 1; t < 4; ++t)

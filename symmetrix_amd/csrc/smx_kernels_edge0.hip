@@ -371,32 +371,36 @@ __global__ __launch_bounds__(256, BPC) void k_agg0_bwd(const AggParams<F> a, con
                     // Sums per order, and the radial function once for each: 2 l - 1 multiplications fewer per channel.  With / without
                     // messages, us: 128 channels, 9 000 atoms 279 -> 274 / 249 -> 242, 9 999 atoms (l <= 1) 433 -> 420, 64 channels,
                     // 20 000 atoms 348 -> 343 / 308 -> 306.  Two channels per lane, three wavefronts and messages have no registers
-                    // for them (12 spilled; 64 channels, 6 000 atoms 115 -> 137): there the radial function goes into the products.
-                    constexpr bool INTO = MSG && CPL == 2 && BPC == 3;
-                    F u[CPL][3];
+                    // for three sums side by side (12 spilled, 64 channels, 6 000 atoms 115 -> 137; one by one 113); elsewhere one by
+                    // one is slower (249 and 438 us of the 242 and 420 above).
+                    constexpr bool ONE = MSG && CPL == 2 && BPC == 3;
+                    constexpr int T = ONE ? 1 : 3;
+                    static_for<0, 3 / T>([&](auto tc) {
+                        constexpr int t0 = decltype(tc)::value * T;
+                        F u[CPL][T];
 #pragma unroll
-                    for (int c = 0; c < CPL; ++c) {
+                        for (int c = 0; c < CPL; ++c)
 #pragma unroll
-                        for (int t = 0; t < 3; ++t) u[c][t] = F(0);
-                        if constexpr (INTO && l == 1) { V[c][1] = F(0); V[c][2] = F(0); }
-                    }
-                    static_for<l * l, (l + 1) * (l + 1)>([&](auto qc) {
-                        constexpr int q = decltype(qc)::value, v = 3 * q;
+                            for (int t = 0; t < T; ++t) u[c][t] = F(0);
+                        static_for<l * l, (l + 1) * (l + 1)>([&](auto qc) {
+                            constexpr int q = decltype(qc)::value;
 #pragma unroll
-                        for (int c = 0; c < CPL; ++c) {
-                            fmac_lane<v % 16>(u[c][0], B[v / 16], d[c][q]);
-                            const F rd = INTO ? R[c] * d[c][q] : d[c][q];
-                            fmac_lane<(v + 1) % 16>(INTO ? V[c][1] : u[c][1], B[(v + 1) / 16], rd);
-                            fmac_lane<(v + 2) % 16>(INTO ? V[c][2] : u[c][2], B[(v + 2) / 16], rd);
-                        }
+                            for (int c = 0; c < CPL; ++c)
+                                static_for<0, T>([&](auto uc) {
+                                    constexpr int t = decltype(uc)::value, v = 3 * q + t0 + t;
+                                    fmac_lane<v % 16>(u[c][t], B[v / 16], d[c][q]);
+                                });
+                        });
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                            for (int t = 0; t < T; ++t) {
+                                F& s = V[c][t0 + t];
+                                s = t0 + t > 0 && l == 1 ? R[c] * u[c][t] : s + R[c] * u[c][t];
+                                if (t0 + t == 0) V[c][3] += Rd[c] * u[c][t];
+                                if constexpr (ONE) pin(s);
+                            }
                     });
-#pragma unroll
-                    for (int c = 0; c < CPL; ++c) {
-                        V[c][0] += R[c] * u[c][0]; V[c][3] += Rd[c] * u[c][0];
-                        if constexpr (!INTO)
-#pragma unroll
-                            for (int t = 1; t < 3; ++t) V[c][t] = l == 1 ? R[c] * u[c][t] : V[c][t] + R[c] * u[c][t];
-                    }
                 }
 #pragma unroll
                 for (int c = 0; c < CPL; ++c)
@@ -495,9 +499,8 @@ hipError_t launch0(const AggParams<F>& p, int group, hipStream_t s)
         constexpr size_t lds = 4 * Lds0<F, true, BPC>::per_wave;
         if (!p.msg) return go(k_agg0_bwd<F, CPL, EW, false, BPC>, lds, parts);
         // With messages, double and two channels per lane, the third wavefront costs from where a receiver has one to itself: us, three
-        // / two: 64 channels 600 atoms 22 / 24, 3 000 60 / 63, 6 500 118 / 112, 20 000 357 / 337, 50 000 901 / 844, 128 channels 600
-        // 32 / 35, 3 000 102 / 104, 6 500 208 / 207, 20 000 658 / 620, 50 000 1 604 / 1 529.  (One channel per lane: 50 000 atoms
-        // 514 / 550.  Three wavefronts and two edges at a time spill five registers: few receivers gain all the same.)
+        // / two: 64 channels 600 atoms 22 / 24, 6 500 117 / 113, 20 000 352 / 346, 50 000 880 / 840, 128 channels 600 32 / 35,
+        // 6 500 215 / 210, 20 000 653 / 620.  (One channel per lane: 50 000 atoms 514 / 550.)
         if constexpr (BPC == 3 && sizeof(F) == 8 && CPL == 2) {
             if (parts == 1) return go(k_agg0_bwd<F, CPL, EW, true, 2>, 4 * Lds0<F, true, 2>::per_wave, parts);
         }
