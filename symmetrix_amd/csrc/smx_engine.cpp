@@ -261,7 +261,7 @@ struct Engine : EngineBase {
     int split_nodes = 0;       // receivers that are not ghosts, of the evaluation under way
     bool diagonal1 = false;    // scalar hidden features, and output lm of layer 1 is fed by cdiag1[lm] Y_lm alone
     double cdiag1[16] = {};
-    bool constant_same1 = false;       // layer 1's paths of the constant harmonic couple like with like only, with these factors
+    bool selected1 = false;            // layer 1 couples by the selection rules only; with the constant harmonic, by these factors
     double c_same1[9] = {};
     DVec<double> fpart;
     DVec<double> H2w_H1, H2w_M1, H2v_H1, H2v_M1, ro1, ro2_w1, ro2_w2, E0;
@@ -396,19 +396,18 @@ struct Engine : EngineBase {
         upload_as(B1_start, hm.B_start, s);
         upload_as(B1_lm1, hm.B_lm1, s);
         upload_as(B1_c, hm.B_c, s);
-        constant_same1 = true;
+        selected1 = true;
         for (int pth = 0, b0 = 0; pth < hm.num_paths; ++pth) {
-            const int l = hm.Phi1_l[pth], n = 2 * l + 1, n2 = 2 * hm.Phi1_l2[pth] + 1;
-            for (int m = 0; hm.Phi1_l1[pth] == 0 && m < n; ++m)
+            const int l = hm.Phi1_l[pth], l1 = hm.Phi1_l1[pth], l2 = hm.Phi1_l2[pth], n = 2 * l + 1, n2 = 2 * l2 + 1;
+            for (int m = 0; m < n; ++m)
                 for (int m2 = 0; m2 < n2; ++m2) {
                     const int b = b0 + m * n2 + m2;
                     double c = 0.0;
                     for (int t = hm.B_start[b]; t < hm.B_start[b + 1]; ++t) {
-                        constant_same1 = constant_same1 && hm.B_lm1[t] == 0;
+                        selected1 = selected1 && (l1 != 0 || hm.B_lm1[t] == 0) && (components_couple(l, m, l1, l2, m2) || hm.B_c[t] == 0.0);
                         c += hm.B_c[t];
                     }
-                    if (m == m2) c_same1[l * l + m] = c;
-                    else if (c != 0.0) constant_same1 = false;
+                    if (l1 == 0 && m == m2) c_same1[l * l + m] = c;
                 }
             b0 += n * n2;
         }
@@ -781,7 +780,7 @@ struct Engine : EngineBase {
         p.num_edges = E; p.split_nodes = split_nodes > 0 ? split_nodes : N;
         p.table_bytes = (layer == 0 ? tabK0.n : tabK1.n) * sizeof(F);
         for (int q = 0; q < 16; ++q) p.cdiag[q] = layer == 0 ? 1.0 : cdiag1[q];
-        p.constant_same = layer == 1 && constant_same1;
+        p.selected = layer == 1 && selected1;
         for (int q = 0; q < 9; ++q) p.c_same[q] = c_same1[q];
         if (layer == 0) {
             p.gather = neigh_types; p.Hsrc = H0.p; p.tab = tab0.p; p.tabK = tabK0.p; p.pair_table = pair_table0.p;

@@ -51,8 +51,9 @@ struct AggParams {
     double* forces_copy;      // bwd, scalar kernels, one channel group: receives the forces as well (or null)
     long num_edges;
     double cdiag[16];         // scalar kernels: output lm is fed by cdiag[lm] Y_lm
-    // the paths of the constant harmonic (l1 = 0) couple like with like only, component l^2 + m with this factor
-    int constant_same;
+    // components couple by the selection rules only (components_couple); like with like through the constant harmonic (l1 = 0),
+    // component l^2 + m with this factor
+    int selected;
     double c_same[9];
     int more_terms;           // some entry of the coupling list has more than two terms
     int split_nodes;          // fwd, general kernel: receivers that decide how many wavefronts share one (the local nodes of a call with ghosts)

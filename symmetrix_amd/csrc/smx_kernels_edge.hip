@@ -49,6 +49,9 @@ constexpr int kEdgeStride = kChunk + 2;
 // does: u[m2] = c d[m2] needs no product with a block and has no tangential part.  10 of the 88 rows and columns for l <= 1, 35 of
 // 243 for l <= 2; the constants go into the adjoint rows as they are loaded, or into the sums as they are stored.  Evaluations of
 // 50 000 atoms, l <= 1, single: 17.2 -> 16.9 ms; 24 999 atoms, double: 12.5 -> 12.1 ms; 3 000 atoms, l <= 2: 1 720 -> 1 658 us.
+// In DPP form the pairs that the selection rules exclude have none either (6 of the 78 others, 28 of 208): the adjoint is bound by
+// its instructions, us: 24 999 atoms, l <= 1 3 882 -> 3 843, 3 000 463 -> 454; l <= 2, 128 channels 3 000 1 369 -> 1 306, 64 channels
+// 5 000 1 184 -> 1 101.  (The matrix form multiplies four rows at a time, of which never all are excluded.)
 template <int LMAXH, bool BWD, bool MATRIX, bool CP>
 struct BlockLayout {
     using PT = Paths<LMAXH>;
@@ -69,9 +72,18 @@ struct BlockLayout {
     static constexpr int entry_off(int p)
     {
         int n = 0;
-        for (int q = 0; q < p; ++q) n += in(q) ? nm(q) * n2(q) : 0;
+        for (int q = 0; q < p; ++q) n += in(q) ? pairs(q, nm(q), 0) : 0;
         return n;
     }
+    static constexpr bool has(int p, int m, int m2) { return MATRIX || !CP || components_couple(PT::l(p), m, PT::l1(p), PT::l2(p), m2); }
+    // pairs of path p before (m, m2) that have an entry
+    static constexpr int pairs(int p, int m, int m2)
+    {
+        int n = 0;
+        for (int b = 0; b < m * n2(p) + m2; ++b) n += has(p, b / n2(p), b % n2(p));
+        return n;
+    }
+    static constexpr int entry(int p, int m, int m2) { return entry_off(p) + pairs(p, m, m2); }
     static constexpr int tile_off(int p)
     {
         int n = 0;
@@ -118,9 +130,10 @@ struct BlockLayout {
                             t.comp[v] = (unsigned char)(BWD ? row % 3 : 0);
                         }
             } else {
-                for (int b = 0; b < NM * N2; ++b)
-                    for (int c = 0; c < (BWD ? 3 : 1); ++c) {
-                        const int v = BWD ? 3 * (eo + b) + c : eo + b;
+                for (int b = 0, e = eo; b < NM * N2; ++b)
+                    for (int c = 0; has(p, b / N2, b % N2) && c < (BWD ? 3 : 1); ++c) {
+                        const int v = BWD ? 3 * e + c : e;
+                        if (c == (BWD ? 2 : 0)) ++e;
                         t.entry[v] = (short)(bo + b);
                         t.comp[v] = (unsigned char)c;
                     }
@@ -389,13 +402,15 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, false>())) void k_a
                             });
                         });
                     } else {
-                        constexpr int bo = BL::entry_off(p), lme0 = PT::lme(p, 0), es = PT::num_e(l);
+                        constexpr int lme0 = PT::lme(p, 0), es = PT::num_e(l);
                         static_for<0, n2>([&](auto mc) {
                             static_for<0, 2 * l + 1>([&](auto rc) {
-                                constexpr int v = bo + decltype(rc)::value * n2 + decltype(mc)::value;
+                                constexpr int v = BL::entry(p, decltype(rc)::value, decltype(mc)::value);
+                                if constexpr (BL::has(p, decltype(rc)::value, decltype(mc)::value)) {
 #pragma unroll
-                                for (int c = 0; c < CPL; ++c)
-                                    fmac_lane<v % 16>(acc[c][lme0 + decltype(rc)::value * es], B[v / 16], w[c][decltype(mc)::value]);
+                                    for (int c = 0; c < CPL; ++c)
+                                        fmac_lane<v % 16>(acc[c][lme0 + decltype(rc)::value * es], B[v / 16], w[c][decltype(mc)::value]);
+                                }
                             });
                         });
                     }
@@ -695,17 +710,26 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                         for (int c = 0; c < CPL; ++c)
 #pragma unroll
                             for (int m2 = 0; m2 < n2; ++m2) u0[c][m2] = F(0);
-                        // the tangential sums take R d: no sums per path for them
+                        // the tangential sums take R d: no sums per path for them, except where those are fewer than the components
+                        // (24 999 atoms 3 843 -> 3 761 us, 3 000 454 -> 450)
+                        constexpr bool PER_PATH = 2 * n2 < 2 * l;
+                        F ut[CPL][n2][2];
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c)
+#pragma unroll
+                            for (int m2 = 0; m2 < n2; ++m2) ut[c][m2][0] = ut[c][m2][1] = F(0);
                         static_for<0, 2 * l + 1>([&](auto mc) {
                             constexpr int m = decltype(mc)::value;
 #pragma unroll
                             for (int c = 0; c < CPL; ++c) {
-                                const F dm = d[c][lme0 + m * es], rd = R[c] * dm;
+                                const F dm = d[c][lme0 + m * es], rd = PER_PATH ? dm : R[c] * dm;
                                 static_for<0, n2>([&](auto m2c) {
-                                    constexpr int m2 = decltype(m2c)::value, v = 3 * (BL::entry_off(p) + m * n2 + m2);
-                                    fmac_lane<v % 16>(u0[c][m2], B[v / 16], dm);
-                                    fmac_lane<(v + 1) % 16>(V[c][l2 * l2 + m2][1], B[(v + 1) / 16], rd);
-                                    fmac_lane<(v + 2) % 16>(V[c][l2 * l2 + m2][2], B[(v + 2) / 16], rd);
+                                    constexpr int m2 = decltype(m2c)::value, v = 3 * BL::entry(p, m, m2);
+                                    if constexpr (BL::has(p, m, m2)) {
+                                        fmac_lane<v % 16>(u0[c][m2], B[v / 16], dm);
+                                        fmac_lane<(v + 1) % 16>(PER_PATH ? ut[c][m2][0] : V[c][l2 * l2 + m2][1], B[(v + 1) / 16], rd);
+                                        fmac_lane<(v + 2) % 16>(PER_PATH ? ut[c][m2][1] : V[c][l2 * l2 + m2][2], B[(v + 2) / 16], rd);
+                                    }
                                 });
                             }
                         });
@@ -716,6 +740,7 @@ __global__ __launch_bounds__(256, (agg_blocks<F, LMAXH, CPL, true>())) void k_ag
                                 F* s = V[c][l2 * l2 + m2];
                                 s[0] = starts ? R[c] * u0[c][m2] : s[0] + R[c] * u0[c][m2];
                                 s[3] = starts ? Rd[c] * u0[c][m2] : s[3] + Rd[c] * u0[c][m2];
+                                if constexpr (PER_PATH) { s[1] += R[c] * ut[c][m2][0]; s[2] += R[c] * ut[c][m2][1]; }
                             }
                     }
                     // path by path
@@ -818,7 +843,7 @@ hipError_t launch_agg_cp(const AggParams<F>& p, hipStream_t s)
 {
     // (scalar features come here with couplings that the scalar kernels do not take)
     if constexpr (LMAXH > 0) {
-        if (p.constant_same) return launch_agg_t<F, LMAXH, CPL, BWD, true>(p, s);
+        if (p.selected) return launch_agg_t<F, LMAXH, CPL, BWD, true>(p, s);
     }
     return launch_agg_t<F, LMAXH, CPL, BWD, false>(p, s);
 }

@@ -43,3 +43,33 @@ def test_copies_of_one_system(tmp_models, K, L_max, dtype):
         want = orc.node_forces.reshape(E, 3)
         got = eng.node_forces.reshape(copies, E, 3)
         assert np.abs(got - want).max() <= TOL[dtype]["F"] * max(1.0, np.abs(want).max())
+
+
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("K,L_max", [(32, 1), (72, 2)])
+def test_coupling_outside_the_selection_rules(tmp_models, K, L_max, dtype):
+    """A file that couples two components which no rotation-equivariant product couples: the way that leaves none out."""
+    import torch
+    assert torch.cuda.is_available()
+    from oracle.oracle import OracleMACE
+    from symmetrix_amd import cg
+    from symmetrix_amd.mace import MACE
+    model = H.tiny_model(K=K, L_max=L_max, n_pts=32, seed=K, r_cut=3.5, pair=False)
+    paths = cg.tensor_product_paths(3, L_max)
+    which = paths.index((2, 1, 1))
+    num_e = [sum(1 for p in paths if p[0] == l) for l in range(4)]
+    e = which - sum(1 for p in paths if p[0] < 2)
+    q = sum((2 * a + 1) * (2 * b + 1) for _, a, b in paths[:which])
+    model["Phi1_lme"].append(num_e[0] + 3 * num_e[1] + 0 * num_e[2] + e)     # m = 0: m = -2 of l = 2
+    model["Phi1_lelm1lm2"].append(q + 2 * 3 + 1)                             # m1 = 1 of l1 = 1, m2 = 0 of l2 = 1
+    model["Phi1_clebsch_gordan"].append(0.6)
+    pos, cell, sp = H.small_system(30, seed=K)
+    _, ea = H.edges_of(pos, cell, sp, model["r_cut"])
+    orc, eng = OracleMACE(model), MACE(H.write_model(model, tmp_models / f"rules_{K}_{L_max}.json"), dtype)
+    print(f"K={K} L_max={L_max} edges={len(ea['r'])} {dtype}", flush=True)
+    orc.compute_node_energies_forces(*H.call_args(ea))
+    eng.compute_node_energies_forces(*H.call_args(ea))
+    for name in ["Phi1"] + ARRAYS:
+        want, got = np.asarray(getattr(orc, name)), np.asarray(getattr(eng, name))
+        assert np.abs(got - want).max() <= TOL[dtype]["inter"] * 10 * max(1.0, np.abs(want).max()), name
+    assert np.abs(eng.node_forces - orc.node_forces).max() <= TOL[dtype]["F"] * max(1.0, np.abs(orc.node_forces).max())
