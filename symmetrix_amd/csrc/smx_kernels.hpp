@@ -47,7 +47,7 @@ struct AggParams {
     double* forces;           // bwd: [E][3]
     int accumulate_forces;    // bwd: add to forces instead of overwriting
     F* msg;                   // bwd: [E][NLM][K] adjoint message to the sender row, or null
-    double* fpart;            // bwd: [channel groups][E][3] partial forces, needed when agg_bwd_groups() > 1
+    double* fpart;            // bwd: [shares][E][3] partial forces, needed when agg_bwd_groups() > 1
     double* forces_copy;      // bwd, scalar kernels, one channel group: receives the forces as well (or null)
     long num_edges;
     double cdiag[16];         // scalar kernels: output lm is fed by cdiag[lm] Y_lm
@@ -65,8 +65,8 @@ struct AggParams {
 
 template <typename F> hipError_t launch_agg_fwd(int L_max_H, const AggParams<F>& p, hipStream_t s);
 template <typename F> hipError_t launch_agg_bwd(int L_max_H, const AggParams<F>& p, hipStream_t s);
-// number of channel groups launch_agg_bwd splits K into; with more than one, the forces come out as
-// fpart[group][E][3] and launch_fpart_reduce adds them up
+// shares of a force, one per channel group and set of paths that launch_agg_bwd splits the work into; with more than one, the
+// forces come out as fpart[share][E][3] and launch_fpart_reduce adds them up
 template <typename F> int agg_bwd_groups(int L_max_H, int K);
 
 // The same two stages for scalar sender features (path list of L_max = 0) whose coupling is diagonal (cdiag), with tables and
@@ -75,7 +75,7 @@ template <typename F> hipError_t launch_agg0_fwd(const AggParams<F>& p, hipStrea
 template <typename F> hipError_t launch_agg0_bwd(const AggParams<F>& p, hipStream_t s);
 template <typename F> int agg0_bwd_groups(int K);
 
-// forces (+)= sum over channel groups of fpart, added in ascending order
+// forces (+)= sum over the shares in fpart, added in ascending order
 // (`copy`, if not null, receives the same sums: the caller's output array of the whole-pipeline call;
 // `guard`, if not null and raised, makes every force NaN instead: the evaluation was skipped)
 hipError_t launch_fpart_reduce(long edges, long E, int groups, const double* fpart, double* forces, int accumulate,
