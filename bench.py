@@ -73,11 +73,14 @@ def measured_traffic(workload, dtype, stage, kernel):
 
 
 MFMA_PEAK = {"float64": 78.6e12, "float32": 157.3e12}   # dense matrix-core peaks of MI355X, flop/s
+# (of the precision's own products; k_linear32 forms a single-precision product from bfloat16 ones, so its bound is higher)
 # kernel behind each dense stage (as the kernel trace names it) when it runs in feature precision F
-DENSE_KERNEL = {"A0_lin": r"k_linear<{F}, \d, {one}, false, (true|false)>", "A1": r"k_linear<{F}, \d, true, false, (true|false)>",
+DENSE_KERNEL = {"A0_lin": r"{L}{one}, false(, (true|false))?>", "A1": r"{L}true, false(, (true|false))?>",
                 "H1": r"k_gemm_rows<{F}, {F}, {F}, \d, false", "H2": r"k_tail_fused<{F}",
-                "rev_A1": r"k_linear<{F}, \d, false, true, true>", "rev_A0_lin": r"k_linear<{F}, \d, false, {one}, (true|false)>",
+                "rev_A1": r"{L}false, true(, true)?>", "rev_A0_lin": r"{L}false, {one}(, (true|false))?>",
                 "rev_H1": r"k_gemm_rows<{F}, {F}, {F}, \d, false"}   # {one}: one polynomial per channel in layer 0
+# {L}: the linears' kernels up to their arguments (with a contraction, with factors)
+LINEARS = {"float64": r"k_linear<double, \d, ", "float32": r"(k_linear<float, \d, |k_linear32<\d, \d, )"}
 
 
 def dense_flops(stage, N, K, n_LM, n_e):
@@ -144,7 +147,8 @@ def measured_mfma_busy(workload, dtype, stage, L_max):
     path = os.path.join(HERE, "profiles", f"bench_{workload}_shader_counters.txt")
     if not os.path.exists(path) or stage not in DENSE_KERNEL:
         return None
-    name = re.compile(DENSE_KERNEL[stage].format(F="double" if dtype == "float64" else "float", one="true" if L_max == 0 else "false"))
+    name = re.compile(DENSE_KERNEL[stage].format(F="double" if dtype == "float64" else "float", L=LINEARS[dtype],
+                                                 one="true" if L_max == 0 else "false"))
     for line in open(path):
         if name.match(line) and line.rstrip().endswith("%"):
             try:
