@@ -65,7 +65,9 @@ void smx_model_free(smx_model* m);
  * "num_radial_tables_0/1" (radial tables per layer) and "contraction_tables"
  * (bit 0 / bit 1 set when the symmetric contraction of layer 0 / layer 1 has all
  * its monomials inside the standard product basis and runs the kernel compiled
- * for it; a file with other monomials takes the general kernel). */
+ * for it; a file with other monomials takes the general kernel); "edges_in_chains"
+ * (bit 0 / bit 1 set when the last evaluation was a small one whose chains of
+ * node-local stages took the sums over the edges of layer 0 / layer 1 along). */
 int smx_model_get_int(const smx_model* m, const char* key, int* out);
 int smx_model_get_double(const smx_model* m, const char* key, double* out);
 /* atomic_numbers[T], atomic_energies[T], mace.hpp:25-26.  *n receives the length. */

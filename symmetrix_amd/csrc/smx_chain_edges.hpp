@@ -131,7 +131,7 @@ struct ChainEdges {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const F* r = red + tid + j * T;
-            out[j] = (r[0] + r[16 * K]) + (r[2 * 16 * K] + r[3 * 16 * K]);
+            out[j] = (r[0] + r[2 * 16 * K]) + (r[16 * K] + r[3 * 16 * K]);      // (as k_agg0_fwd hands them down)
         }
     }
 

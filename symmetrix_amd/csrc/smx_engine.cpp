@@ -203,6 +203,7 @@ struct EngineBase {
     int precision = 0;
     int poly_tables = 0;            // bit 0 / bit 1: layer 0 / layer 1 contraction runs the table-specialised kernel
     int contraction_tables() const { return poly_tables; }
+    int edges_in_chains = 0;        // bit 0 / bit 1: the chains of the last evaluation took the aggregation of layer 0 / layer 1 along
     int device = 0;                 // ordinal of the GPU the model was loaded on
     hipStream_t stream = nullptr;   // stream of the current call
     bool profiling = false;
@@ -817,6 +818,7 @@ struct Engine : EngineBase {
     {
         auto p = agg_params(layer, N);
         p.out = out;
+        p.as_chains = layer == 0 && ghosts_apart(N);
         if (scalar_edges(layer, layer == 0 ? hm.T : H1.n / hm.K)) return launch_agg0_fwd<F>(p, stream);
         return launch_agg_fwd<F>(layer == 0 ? 0 : hm.L_max, p, stream);
     }
@@ -945,11 +947,11 @@ struct Engine : EngineBase {
         p.N = N; p.K = K(); p.T = hm.T; p.perm = t_perm.p; p.tstart = t_start.p;
         return p;
     }
-    // A0, M0 and H1, with chain_edges(0) the layer-0 aggregation before them
+    // A0, M0 and H1, with chain_edges the layer-0 aggregation before them
     void st_chain0(int N)
     {
         const size_t k = K(), nlm = NLM();
-        const bool edges = chain_edges(0);
+        const bool edges = chain_edges(0, N);
         if (edges) {
             need(xyz, "xyz"); need(r, "r"); need_edges(N);
             Phi0.size_to((size_t)N * 16 * k, stream);
@@ -966,30 +968,41 @@ struct Engine : EngineBase {
         HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain0<F, decltype(kc)::value>(p, edges ? &agg : nullptr, hm.L_max, stream); }));
         if (nlm == 1) pending_A0 = N;
     }
-    // Whether the chains of a layer take its aggregation and the adjoint of it along (scalar features): not where a CU holds one
-    // block and there are more blocks than CUs, whose aggregations as launches of their own spread better.  Whole evaluations, us,
-    // separate / along: one l, double, 96 channels 24 atoms 87 / 78, 256 102 / 86, 300 135 / 142, 1 000 246 / 267, 128 channels 256
-    // 118 / 105, 300 167 / 182, 64 channels 200 76 / 61, 1 500 213 / 203, 32 channels 1 000 99 / 88, 2 000 158 / 143, 3 000 194 / 197;
-    // single, 96 channels 24 71 / 60, 501 96 / 87, 1 000 165 / 152, 128 channels 256 88 / 77, 400 125 / 129, 64 channels 1 500 156 / 144,
-    // 32 channels 3 000 149 / 141; l <= 1 (layer 0 only), 128 channels double 107 201 / 198, 256 250 / 242, 500 442 / 443, single 200
-    // 150 / 142, 96 channels 600 303 / 309, 64 channels 1 000 258 / 253; l <= 2, 64 channels double 700 507 / 503.
-    bool chain_edges(int layer) const
+    // Whether the chains of a layer, of N nodes, take its aggregation and the adjoint of it along (scalar features): not where a CU
+    // holds one block and there are more blocks than CUs, whose aggregations as launches of their own spread better.  Whole
+    // evaluations, us, separate / along: one l, double, 96 channels 24 atoms 87 / 78, 256 102 / 86, 300 135 / 142, 1 000 246 / 267, 128
+    // channels 256 118 / 105, 300 167 / 182, 64 channels 200 76 / 61, 1 500 213 / 203, 32 channels 1 000 99 / 88, 2 000 158 / 143,
+    // 3 000 194 / 197; single, 96 channels 24 71 / 60, 501 96 / 87, 1 000 165 / 152, 128 channels 256 88 / 77, 400 125 / 129, 64
+    // channels 1 500 156 / 144, 32 channels 3 000 149 / 141; l <= 1 (layer 0 only), 128 channels double 107 201 / 198, 256 250 / 242,
+    // 500 442 / 443, single 200 150 / 142, 96 channels 600 303 / 309, 64 channels 1 000 258 / 253; l <= 2, 64 channels double 700
+    // 507 / 503.
+    // Ghost nodes have blocks in layer 0 only, so that all nodes have a line of their own there: local / all nodes, us as above
+    // (separate in the order of the chains): one l, double, 96 channels 230 / 748 190 / 183, 256 / 850 209 / 212, 128 channels
+    // 100 / 405 159 / 160, 150 / 591 203 / 213, 200 / 686 212 / 220, 250 / 842 256 / 271, 32 channels 1 850 / 3 721 211 / 211, 2 048 / 3 959
+    // 215 / 220; single, 128 channels 230 / 748 155 / 153, 256 / 850 171 / 179, 64 channels (l <= 1) 200 / 798 156 / 144; l <= 1, double, 96
+    // channels 170 / 659 314 / 312, 200 / 798 350 / 366, 128 channels 96 / 469 272 / 275, 120 / 561 322 / 335, 200 / 798 428 / 458, single, 128
+    // channels 170 / 659 228 / 226, 200 / 798 254 / 267, 96 channels 256 / 913 237 / 229; l <= 2, 128 channels double 120 / 561 430 / 445,
+    // single 170 / 659 328 / 321, 200 / 798 368 / 380, 96 channels double 200 / 798 501 / 502, single 256 / 913 340 / 331.
+    bool chain_edges(int layer, int N) const
     {
         if (!scalar_edges(layer, layer == 0 ? hm.T : H1.n / hm.K) || (layer == 1 && NLM() > 1)) return false;
-        if (split_nodes <= num_cus) return true;
-        if (sizeof(F) == 8) return hm.K <= 64 && split_nodes <= 2048;
-        return hm.K <= 64 || (hm.K == 96 && NLM() == 1);
+        if (sizeof(F) == 4 && (hm.K <= 64 || (hm.K == 96 && NLM() == 1))) return true;
+        if (sizeof(F) == 8 && hm.K <= 64) return split_nodes <= 2048 && N <= 3840;
+        return split_nodes <= num_cus && N <= (sizeof(F) == 8 ? (hm.K == 96 ? 3 : 2) : (hm.K == 96 ? 6 : 3)) * num_cus;
     }
-    bool chain1_messages() const { return chain_edges(1) && (size_t)E1 * hm.K * sizeof(F) <= msg_limit_bytes; }
+    // Chains whose layer-0 aggregation is a launch of its own for the ghost nodes' sake: the sums over the edges of a receiver run in
+    // the order of the chains, so that a call with ghost nodes gives the bits of one without.
+    bool ghosts_apart(int N) const { return use_chains(N) && !chain_edges(0, N) && chain_edges(0, split_nodes); }
+    bool chain1_messages(int N) const { return chain_edges(1, N) && (size_t)E1 * hm.K * sizeof(F) <= msg_limit_bytes; }
     // A1, M1, the tail and the adjoints back to dPhi1, the aggregation before and its adjoint behind them where that is so
     void st_chain1(int N, bool zero_energies, bool zero_forces)
     {
         const size_t k = K();
-        if (chain_edges(1)) {
+        if (chain_edges(1, N)) {
             need(xyz, "xyz"); need(r, "r"); need(neigh_indices, "neigh_indices"); need_edges(N);
             Phi1.size_to((size_t)N * NE() * k, stream);
         }
-        messages_left = chain1_messages();
+        messages_left = chain1_messages(N);
         if (messages_left) msg.size_to((size_t)E1 * k, stream);
         A1.size_to((size_t)N * 16 * k, stream);
         M1.size_to((size_t)N * k, stream); M1_grad.size_to((size_t)N * 16 * k, stream);
@@ -1000,12 +1013,12 @@ struct Engine : EngineBase {
         const auto q = tail_params(N, zero_energies);
         auto agg = agg_params(1, N);
         agg.out = Phi1.p; agg.msg = messages_left ? msg.p : nullptr; agg.forces = node_forces.p; agg.accumulate_forces = zero_forces ? 0 : 1;
-        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain1<F, decltype(kc)::value>(p, q, chain_edges(1) ? &agg : nullptr, hm.L_max, stream); }));
+        HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain1<F, decltype(kc)::value>(p, q, chain_edges(1, N) ? &agg : nullptr, hm.L_max, stream); }));
         if (guard_status && q.rows > 0) guard_clear_enqueued = true;
         energies_copy = nullptr;
         pending_A1 = N; pending_A1_adj = N;
     }
-    // the messages (`add_messages`: those of the last layer-1 adjoint are not in H1_adj yet), M0_adj, A0_adj, dPhi0, and with chain_edges(0)
+    // the messages (`add_messages`: those of the last layer-1 adjoint are not in H1_adj yet), M0_adj, A0_adj, dPhi0, and with chain_edges
     // the adjoint of the layer-0 aggregation, which writes the caller's copy of the forces as well
     void st_chain2(int N, bool add_messages)
     {
@@ -1019,7 +1032,7 @@ struct Engine : EngineBase {
         p.msg = add_messages ? msg.p : nullptr; p.H1_adj = H1_adj.p; p.sstart = s_start.p; p.slist = s_list.p; p.spare = s_rank.p;
         auto agg = agg_params(0, N);
         agg.forces = node_forces.p; agg.accumulate_forces = 1; agg.forces_copy = forces_copy;
-        const bool edges = chain_edges(0);
+        const bool edges = chain_edges(0, N);
         HIPCHK(with_channels(K(), [&](auto kc) { return launch_chain2<F, decltype(kc)::value>(p, edges ? &agg : nullptr, hm.L_max, stream); }));
         if (edges) forces_copy = nullptr;
         pending_A0_adj = N;
@@ -1501,7 +1514,9 @@ struct Engine : EngineBase {
             st_zbl(N1);
         }
         const bool chain = use_chains(N);
-        if (chain && chain_edges(0)) stage_absent(ST_AGG0F);
+        edges_in_chains = 0;
+        if (chain && chain_edges(0, N)) edges_in_chains = 1;
+        if (edges_in_chains) stage_absent(ST_AGG0F);
         else { stage_begin(ST_AGG0F); st_agg0_fwd(N); stage_end(ST_AGG0F); }
         pending_A0 = pending_A1 = -1;
         pending_M0_grad = recompute_M0_grad() ? N : -1;
@@ -1520,7 +1535,7 @@ struct Engine : EngineBase {
         // the species groups cover the nodes of the current stages
         if (N1 < N) build_type_groups(N1);
         if (chain) {
-            if (chain_edges(1)) stage_absent(ST_AGG1F);
+            if (chain_edges(1, N1)) { edges_in_chains |= 2; stage_absent(ST_AGG1F); }
             else { stage_begin(ST_AGG1F); st_agg1_fwd(N1); stage_end(ST_AGG1F); }
             stage_begin(ST_A1); st_chain1(N1, !hm.has_zbl, !early_forces); stage_end(ST_A1);
             for (int st : {ST_M1, ST_H2, ST_READOUT, ST_REVH2, ST_REVM1, ST_REVA1}) stage_absent(st);
@@ -1534,7 +1549,7 @@ struct Engine : EngineBase {
             if (N1 < N) build_type_groups(N);
             stage_begin(ST_REVA0LIN); st_chain2(N, messages_left); stage_end(ST_REVA0LIN);
             for (int st : {ST_REVH1, ST_REVM0}) stage_absent(st);
-            if (!chain_edges(0)) st_agg0_bwd(N);
+            if (!chain_edges(0, N)) st_agg0_bwd(N);
             else for (int st : {ST_AGG0B, ST_FSUM0}) stage_absent(st);
             finish_evaluation(N1, on_device);
             return;
@@ -2381,6 +2396,7 @@ int smx_model_get_int(const smx_model* m, const char* key, int* out)
         else if (k == "num_radial_tables_0") *out = (int)h.tables0.size();
         else if (k == "num_radial_tables_1") *out = (int)h.tables1.size();
         else if (k == "contraction_tables") *out = m->eng->contraction_tables();
+        else if (k == "edges_in_chains") *out = m->eng->edges_in_chains;
         else throw smx::Error(SMX_EINVAL, "unknown integer key '" + k + "'");
     });
 }

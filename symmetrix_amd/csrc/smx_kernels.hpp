@@ -57,6 +57,7 @@ struct AggParams {
     double c_same[9];
     int more_terms;           // some entry of the coupling list has more than two terms
     int split_nodes;          // fwd, general kernel: receivers that decide how many wavefronts share one (the local nodes of a call with ghosts)
+    int as_chains;            // fwd, scalar kernels: four wavefronts per receiver, sums in the order of the chains (smx_chain_edges.hpp)
     // bwd, general kernel only: receivers [node_begin, num_nodes) are processed and the message of edge e goes to
     // row e - msg_edge_begin of msg (edge lists too long for one staging buffer are taken in receiver chunks)
     int node_begin;

@@ -80,10 +80,13 @@ __global__ __launch_bounds__(256, 2) void k_agg0_fwd(const AggParams<F> a, const
         active[c] = ch < a.K && c * LPE + sl < group_channels;
         k[c] = active[c] ? (unsigned)ch : 0u;
     }
+    // Edges of this wavefront: the e1 - e0 from e0 on, or (as_chains: four parts, two edges at a time) two of every eight.
+    const bool dealt = a.as_chains;
     int e0 = 0, e1 = 0, ti = 0;
     if (real) {
         const int b = a.first_neigh[i], n = a.first_neigh[i + 1] - b;
-        e0 = b + (int)((long)n * part / parts); e1 = b + (int)((long)n * (part + 1) / parts);
+        e0 = b + (dealt ? EW * part : (int)((long)n * part / parts));
+        e1 = dealt ? e0 + n / (4 * EW) * EW + min(max(n % (4 * EW) - EW * part, 0), EW) : b + (int)((long)n * (part + 1) / parts);
         ti = a.node_types[i];
     }
     e0 = __builtin_amdgcn_readfirstlane(e0); e1 = __builtin_amdgcn_readfirstlane(e1);
@@ -120,7 +123,8 @@ __global__ __launch_bounds__(256, 2) void k_agg0_fwd(const AggParams<F> a, const
         wave_lds_sync();
         if (lane < slots + EW) {
             // the entries from nE on: the first edges of the next chunk (past the last edge of the part: the last one again)
-            const int e = min(eb + lane, e1 - 1);
+            int e = min(eb + lane, e1 - 1);
+            if (dealt) e += (e - e0) / EW * (3 * EW);
             edge_offsets(a, e, ti, row_bytes, sender_bytes, xs, toff, goff, lane);
             if (lane < nE) {
                 const double dx = a.xyz[3 * (size_t)e], dy = a.xyz[3 * (size_t)e + 1], dz = a.xyz[3 * (size_t)e + 2];
@@ -482,7 +486,8 @@ hipError_t launch0(const AggParams<F>& p, int group, hipStream_t s)
     if (!BWD && (p.node_begin != 0 || p.msg_edge_begin != 0)) return hipErrorInvalidValue;
     if (p.node_begin < 0 || p.node_begin > p.num_nodes) return hipErrorInvalidValue;
     const long nodes = p.num_nodes - p.node_begin;
-    const int parts = agg_parts<BWD>((long)(BWD ? nodes : p.split_nodes) * groups);
+    if (!BWD && p.as_chains && EW != 2) return hipErrorInvalidValue;
+    const int parts = !BWD && p.as_chains ? 4 : agg_parts<BWD>((long)(BWD ? nodes : p.split_nodes) * groups);
     const long blocks = (nodes * parts + 3) / 4 * groups;
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;

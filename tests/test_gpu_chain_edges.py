@@ -44,3 +44,52 @@ def test_sizes_at_the_rule(tmp_models, K, n, dtype):
     """With the edges and without, where a CU holds one block and there are as many atoms as CUs, or one more."""
     degree = np.random.default_rng(n).integers(0, 12, n)
     _compare(*_both(tmp_models, K, 0, dtype, degree, n), dtype)
+
+
+def _with_ghosts(tmp_models, K, L_max, n, dtype, all_nodes):
+    """n atoms by their owners, and with the neighbours across the box as ghost nodes; ghosts without an edge make up all_nodes."""
+    import torch
+    assert torch.cuda.is_available()
+    from symmetrix_amd import neighbors
+    from symmetrix_amd.mace import MACE
+    model = H.tiny_model(K=K, L_max=L_max, n_pts=48, seed=3 * K + L_max, r_cut=3.5, pair=False)
+    eng = MACE(H.write_model(model, tmp_models / f"chain_ghosts_{K}_{L_max}.json"), dtype)
+    pos, cell, sp = H.small_system(n, density=0.1, seed=n + K)
+    nl, ea = H.edges_of(pos, cell, sp, model["r_cut"])
+    g = neighbors.ghost_edge_arrays(nl, sp)
+    more = all_nodes - n - g["num_ghost_nodes"]
+    assert more >= 0 and g["num_ghost_nodes"] > 0
+    none = np.zeros(more, np.int32)
+    print(f"K={K} L_max={L_max} local={n} all={all_nodes} edges={len(g['r'])} {dtype}", flush=True)
+    eng.compute_node_energies_forces(*H.call_args(ea))
+    own = {name: np.array(getattr(eng, name)) for name in ("node_energies", "M0", "H1", "Phi1")}
+    own["forces"] = eng.reduce_forces(n, ea["neigh_indices"])
+    own["route"] = eng._int("edges_in_chains")
+    eng.compute_ghosted(n, all_nodes - n, np.concatenate([g["node_types"], none]), np.concatenate([g["num_neigh"], none]),
+                        g["neigh_indices"], g["neigh_types"], g["xyz"], g["r"])
+    got = {name: np.array(getattr(eng, name))[:len(own[name])] for name in ("node_energies", "M0", "H1", "Phi1")}
+    receivers = np.concatenate([g["receiver_atom"], np.zeros(more, np.int32)])
+    got["forces"] = eng.reduce_forces(n, g["sender_atom"], receivers)
+    got["route"] = eng._int("edges_in_chains")
+    return own, got
+
+
+# rounds: of blocks that the CUs hold one of each; nodes where they hold several.  (64 channels reach the line that the chains have for
+# all nodes before.)
+@pytest.mark.parametrize("K,L_max,dtype,n,rounds,nodes", [(96, 0, "float64", 100, 3, 0), (128, 0, "float64", 100, 2, 0), (128, 0, "float32", 100, 3, 0),
+                                                          (128, 1, "float64", 100, 2, 0), (96, 1, "float32", 100, 6, 0),
+                                                          (128, 2, "float32", 100, 3, 0), (32, 0, "float64", 1000, 0, 3840)])
+def test_ghost_nodes_decide_layer_0(tmp_models, K, L_max, dtype, n, rounds, nodes):
+    """Ghost nodes have blocks of their own in the chains of layer 0: beyond a number of them the edges of layer 0 are a launch of their
+    own, with the bits of the chains."""
+    import torch
+    line = nodes + rounds * torch.cuda.get_device_properties(0).multi_processor_count
+    for nodes in (line, line + 1):
+        own, got = _with_ghosts(tmp_models, K, L_max, n, dtype, nodes)
+        assert own["route"] == (3 if L_max == 0 else 1)
+        assert got["route"] == own["route"] - (nodes > line)
+        for name in ("node_energies", "M0", "H1", "Phi1"):
+            assert np.array_equal(got[name], own[name]), name
+        # (sums over the images of an atom in another order)
+        tol = 1e-12 if dtype == "float64" else 1e-4
+        assert np.abs(got["forces"] - own["forces"]).max() <= tol * np.abs(own["forces"]).max()
