@@ -175,6 +175,7 @@ static unsigned short bf16_of(float x)
 {
     unsigned u;
     std::memcpy(&u, &x, 4);
+    if (x != x) return 0x7fc0;
     return (unsigned short)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
 static float float_of_bf16(unsigned short h)
@@ -569,7 +570,7 @@ struct Engine : EngineBase {
             out.clear();
         });
     }
-    // ... of k_linear32: [column tile][piece of 32 terms][part][64][8], w = part 0 + part 1 + part 2 in bf16, rounded to nearest
+    // ... of k_linear32: [column tile][piece of 32 terms][part][64][8], w kSplitScale = part 0 + part 1 + part 2 in bf16, rounded to nearest
     void split_weights(hipStream_t s)
     {
         std::vector<unsigned short> out;
@@ -579,7 +580,7 @@ struct Engine : EngineBase {
                     const size_t at = out.size();
                     out.resize(at + 3 * 512);
                     for (int i = 0; i < 512; ++i) {
-                        float rest = (float)B(32 * st + i / 128 * 8 + i % 8, ct * 16 + i / 8 % 16);
+                        float rest = (float)B(32 * st + i / 128 * 8 + i % 8, ct * 16 + i / 8 % 16) * kSplitScale;
                         for (int part = 0; part < 3; ++part) {
                             const unsigned short h = bf16_of(rest);
                             out[at + part * 512 + i] = h;

@@ -314,8 +314,8 @@ struct LinearParams {
     int inner[4], num_e[4], num_e_max;       // inner size and output blocks per l
     int row_off[16];                         // of (l, m) in an operand row, elements
     const F* W; size_t w_off[4], w_type_stride[4];
-    const unsigned short* W_split;           // single precision: the weights as three bf16 parts, offsets and strides three times those of
-                                             // W, or null
+    const unsigned short* W_split;           // single precision: the weights times kSplitScale as three bf16 parts, offsets and strides
+                                             // three times those of W, or null
     int split_nodes;                         // nodes that decide which kernel it is (the local ones of a call with ghosts)
     F* out; long out_node_stride; int out_off[16];
     const F* coef; F* M; F* M_grad;
@@ -323,6 +323,7 @@ struct LinearParams {
 inline bool linear_ok(int K) { return K % 32 == 0; }     // whole pieces of a row, and column tiles in pairs
 template <typename F> hipError_t launch_linear(const LinearParams<F>& p, hipStream_t s);
 // the part of launch_linear that runs on bf16 parts of the numbers (smx_kernels_linear32.hip)
+constexpr float kSplitScale = 16777216.0f;
 bool linear32_ok(const LinearParams<float>& p);
 hipError_t launch_linear32(const LinearParams<float>& p, hipStream_t s);
 

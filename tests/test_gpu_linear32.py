@@ -68,3 +68,85 @@ def test_contraction(tmp_models, K, L_max, n):
     eng.compute_node_energies_forces(*H.call_args(ea))
     assert eng.stage_times()["M1"] == 0.0      # in the launch of the linear
     _compare(orc, eng, "float32")
+
+
+def _check_range(got, x, w, what):
+    """As in test_products where the parts form a sum; numbers above 2^103 and sums above 2^80 are sums in single precision, of a rounding
+    a term.  A rounding is half of the smallest number of single precision, 2^-149, at least: one of them at the end of a sum of parts, one a
+    term else."""
+    K = w.shape[0]
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref, size = x @ w, np.abs(x) @ np.abs(w)
+        plain = (np.abs(x) >= 2.0 ** 103).any(-1)[..., None] | (np.abs(w) >= 2.0 ** 103).any(0) | (size >= 2.0 ** 79)
+        assert np.array_equal(np.isnan(got), np.isnan(ref)), what
+        assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)]), what
+        ok = np.isfinite(ref) & (size <= 3.4e38)      # (single precision may not hold a larger sum on the way)
+        err = np.abs(got - ref) - np.where(plain, K, 6 * K / 32 + 2) * 2.0 ** -24 * size
+    assert (err <= np.where(plain, K, 1) * 2.0 ** -150)[ok].all(), what
+
+
+@pytest.mark.parametrize("weights", [False, True])
+@pytest.mark.parametrize("K", [96, 128])
+def test_range(tmp_models, K, weights):
+    """Rows of all sizes that single precision holds, infinities and NaN; columns of weights of all sizes."""
+    import torch
+    assert torch.cuda.is_available()
+    from symmetrix_amd.mace import MACE
+    n = 1030
+    model = H.tiny_model(K=K, L_max=0, T=(1, 6, 8), n_pts=16, seed=K, r_cut=3.0, pair=False, density=False)
+    W = [np.array(w).reshape(K, K) for w in model["A1_weights"]]
+    if weights:
+        for c, power in enumerate([-140, -122, -112, -100, 76, 100, 110, 120]):
+            for w in W:
+                w[:, c] *= 2.0 ** power
+        model["A1_weights"] = [w.ravel().tolist() for w in W]
+    W = [w.astype(np.float32).astype(np.float64) for w in W]
+    eng = MACE(H.write_model(model, tmp_models / f"linear32_range_{K}_{weights}.json"), "float32")
+    rng = np.random.default_rng(K)
+    x = rng.normal(size=(n, 16, K))
+    for i, power in ((0, -140), (1, -126), (17, -112), (18, -100), (33, 76), (34, 100), (50, 120)):
+        x[i] *= 2.0 ** power
+    x[51, :, :] = 0.0
+    x[66, :, 7] = np.inf
+    x[67, :, 8] = -np.inf
+    x[82, :, 9] = np.nan
+    x[98, :, 10] = np.finfo(np.float32).max
+    x[114, :, ::2] *= 2.0 ** 110
+    x[114, :, 1::2] *= 2.0 ** -130
+    x = x.astype(np.float32).astype(np.float64)
+    print(f"K={K} atoms={n} weights={weights}", flush=True)
+    eng.Phi1 = x.ravel()
+    eng.compute_A1(n)
+    A1 = np.array(eng.A1).reshape(n, 16, K)
+    eng.A1_adj = x.ravel()
+    eng.reverse_A1(n)
+    Phi1_adj = np.array(eng.Phi1_adj).reshape(n, 16, K)
+    for l in range(4):
+        m = slice(l * l, (l + 1) ** 2)
+        _check_range(A1[:, m], x[:, m], W[l], "A1")
+        _check_range(Phi1_adj[:, m], x[:, m], W[l].T, "Phi1_adj")
+
+
+def test_small_factors(tmp_models):
+    """Energies so small that the factors of the adjoint rows are next to the smallest numbers."""
+    import torch
+    assert torch.cuda.is_available()
+    from symmetrix_amd.mace import MACE
+    K, n = 128, 528
+    model = H.tiny_model(K=K, L_max=0, T=(1, 6, 8), n_pts=16, seed=7, r_cut=3.0, pair=False, density=False)
+    for name in ("readout_1_weights", "readout_2_weights_2"):
+        model[name] = (np.array(model[name]) * 2.0 ** -118).tolist()
+    eng = MACE(H.write_model(model, tmp_models / "linear32_small.json"), "float32")
+    eng.set_profiling(True)
+    ea, _ = _system(model, n)
+    eng.compute_node_energies_forces(*H.call_args(ea))
+    get = lambda name: np.array(getattr(eng, name)).reshape(n, -1, K)
+    A1_adj, Phi1_adj = get("A1_adj"), get("Phi1_adj")
+    print(f"largest factor {np.abs(A1_adj).max():.2e}, edges {len(ea['r'])}", flush=True)
+    assert 0.0 < np.abs(A1_adj).max() < 2.0 ** -100
+    for l in range(4):
+        w = np.array(model["A1_weights"][l], dtype=np.float32).astype(np.float64).reshape(K, K)
+        m = slice(l * l, (l + 1) ** 2)
+        # (A1_adj is rounded to the smallest number, and the operand is a product like it)
+        err = np.abs(Phi1_adj[:, m] - A1_adj[:, m] @ w.T) - (6 * K / 32 + 3) * 2.0 ** -24 * (np.abs(A1_adj[:, m]) @ np.abs(w.T))
+        assert (err <= 2.0 ** -149 * (2 + np.abs(w.T).sum(0))).all()
