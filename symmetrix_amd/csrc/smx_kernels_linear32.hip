@@ -4,7 +4,7 @@
 //
 // A number of 24 bits is the sum of three bf16 numbers of 8 bits each, rounded to nearest, exactly:  x = x0 + x1 + x2.  Of the nine
 // products of two such numbers the six with indices up to 2 in sum are formed, exactly, and added in single precision; what is left
-// out is below 2^-25 of the product.
+// out is x1 w2 + x2 w1 + x2 w2, with |x1| <= 2^-8 and |x2| <= 2^-17 of the leading bit of x: up to 1.002 2^-24 of the product.
 // Both operands are multiplied by 2^24 first, so that the parts of every number down to the smallest one are normal numbers, and the sums by
 // 2^-48.  Numbers above 2^103, infinities, NaN and sums above 2^80 end in an infinity or NaN for it: such sums are formed again, in
 // single precision as they are (plain_sums).  Evaluations without and with that, us: 96 channels 20 011 atoms 1 331 / 1 333, 128 channels,
