@@ -22,8 +22,8 @@ def _engine(tmp_models, K, L_max):
     return model, eng
 
 
-# 16 columns per wavefront (few atoms) and 32 at 128 channels, two blocks of columns at 256; 96 channels; remainders of a row tile
-@pytest.mark.parametrize("K,L_max,n", [(128, 0, 513), (128, 0, 2049), (128, 1, 527), (128, 1, 2065), (128, 2, 1025), (256, 0, 640), (96, 0, 1025), (96, 2, 1039)])
+# 16 columns per wavefront (few atoms) and 32 at 128 channels, two and three blocks of columns at 192 to 288; 96 channels; remainders of a row tile
+@pytest.mark.parametrize("K,L_max,n", [(128, 0, 513), (128, 0, 2049), (128, 1, 527), (128, 1, 2065), (128, 2, 1025), (256, 0, 640), (96, 0, 1025), (96, 2, 1039), (192, 0, 1025), (288, 1, 1030)])
 def test_products(tmp_models, K, L_max, n):
     """What is left out of a product is at most 1.002 2^-24 of it, its factors are exact, and a sum of `inner` terms is rounded 6 / 32
     times a term: (6 inner / 32 + 2) 2^-24 of the sum of magnitudes at most."""
@@ -56,7 +56,7 @@ def test_products(tmp_models, K, L_max, n):
             off += ne
 
 
-@pytest.mark.parametrize("K,L_max,n", [(128, 0, 2049), (128, 1, 1040), (128, 2, 1024)])
+@pytest.mark.parametrize("K,L_max,n", [(128, 0, 2049), (128, 1, 1040), (128, 2, 1024), (256, 0, 2049)])
 def test_contraction(tmp_models, K, L_max, n):
     from oracle.oracle import OracleMACE
     from tests.test_gpu_parity import _compare
