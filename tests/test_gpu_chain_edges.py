@@ -11,12 +11,13 @@ pytestmark = pytest.mark.gpu
 DEGREES = [0, 1, 7, 8, 9, 79, 80, 81, 119, 120, 121, 248]
 
 
-def _both(tmp_models, K, L_max, dtype, degree, seed):
+def _both(tmp_models, K, L_max, dtype, degree, seed, along, zbl=False):
+    """Whatever an evaluation leaves, with chains and by launches per stage; along: layers whose edges the chains took."""
     import torch
     assert torch.cuda.is_available()
     from symmetrix_amd.mace import MACE
-    model = H.tiny_model(K=K, L_max=L_max, n_pts=48, seed=5 * K + L_max, r_cut=3.5, pair=False)
-    eng = MACE(H.write_model(model, tmp_models / f"chain_edges_{K}_{L_max}.json"), dtype)
+    model = H.tiny_model(K=K, L_max=L_max, n_pts=48, seed=5 * K + L_max, r_cut=3.5, pair=False, zbl=zbl)
+    eng = MACE(H.write_model(model, tmp_models / f"chain_edges_{K}_{L_max}_{int(zbl)}.json"), dtype)
     rng = np.random.default_rng(seed)
     N, E = len(degree), int(np.sum(degree))
     species = rng.integers(0, 3, N).astype(np.int32)
@@ -28,6 +29,7 @@ def _both(tmp_models, K, L_max, dtype, degree, seed):
     for per_stage in (False, True):
         eng.set_profiling(per_stage)
         eng.compute_node_energies_forces(N, species, np.asarray(degree, np.int32), senders, species[senders], x.ravel(), np.linalg.norm(x, axis=1))
+        assert eng._int("edges_in_chains") == (0 if per_stage else along)
         out.append({name: np.array(getattr(eng, name)) for name in ARRAYS})
     return out
 
@@ -36,14 +38,26 @@ def _both(tmp_models, K, L_max, dtype, degree, seed):
 @pytest.mark.parametrize("L_max", [0, 1, 2])
 @pytest.mark.parametrize("K", [32, 64, 96, 128])
 def test_receivers_of_all_lengths(tmp_models, K, L_max, dtype):
-    _compare(*_both(tmp_models, K, L_max, dtype, np.random.default_rng(K).permutation(DEGREES), K + L_max), dtype)
+    along = 3 if L_max == 0 else 1
+    _compare(*_both(tmp_models, K, L_max, dtype, np.random.default_rng(K).permutation(DEGREES), K + L_max, along), dtype)
 
 
-@pytest.mark.parametrize("K,n,dtype", [(96, 256, "float64"), (96, 257, "float64"), (128, 257, "float32"), (96, 300, "float32"), (64, 300, "float64")])
-def test_sizes_at_the_rule(tmp_models, K, n, dtype):
-    """With the edges and without, where a CU holds one block and there are as many atoms as CUs, or one more."""
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("K,L_max", [(64, 0), (96, 0), (128, 1)])
+def test_forces_that_are_there_before(tmp_models, K, L_max, dtype):
+    """Pair repulsion: every adjoint adds to its forces."""
+    _compare(*_both(tmp_models, K, L_max, dtype, DEGREES, K, 3 if L_max == 0 else 1, zbl=True), dtype)
+
+
+# beyond: atoms more than CUs that hold a block each; n: atoms where they hold several
+@pytest.mark.parametrize("K,beyond,n,dtype,along", [(96, 0, 0, "float64", 3), (96, 1, 0, "float64", 0), (128, 0, 0, "float32", 3), (128, 1, 0, "float32", 0),
+                                                    (96, 44, 0, "float32", 3), (64, 44, 0, "float64", 3), (32, 0, 2048, "float64", 3), (32, 0, 2049, "float64", 0)])
+def test_sizes_at_the_rule(tmp_models, K, beyond, n, dtype, along):
+    """With the edges and without, where a CU holds one block and there are as many atoms as CUs, or one more, and elsewhere."""
+    import torch
+    n = n or torch.cuda.get_device_properties(0).multi_processor_count + beyond
     degree = np.random.default_rng(n).integers(0, 12, n)
-    _compare(*_both(tmp_models, K, 0, dtype, degree, n), dtype)
+    _compare(*_both(tmp_models, K, 0, dtype, degree, n, along), dtype)
 
 
 def _with_ghosts(tmp_models, K, L_max, n, dtype, all_nodes):
