@@ -73,7 +73,8 @@ def measured_traffic(workload, dtype, stage, kernel):
 
 
 MFMA_PEAK = {"float64": 78.6e12, "float32": 157.3e12}   # dense matrix-core peaks of MI355X, flop/s
-# (of the precision's own products; k_linear32 forms a single-precision product from bfloat16 ones, so its bound is higher)
+# k_linear32 forms a single-precision product from six bfloat16 ones (dense peak 2.5 Pflop/s)
+MFMA_PEAK_BF16_PARTS = 2.5e15 / 6
 # kernel behind each dense stage (as the kernel trace names it) when it runs in feature precision F
 DENSE_KERNEL = {"A0_lin": r"{L}{one}, false(, (true|false))?>", "A1": r"{L}true, false(, (true|false))?>",
                 "H1": r"k_gemm_rows<{F}, {F}, {F}, \d, false", "H2": r"k_tail_fused<{F}",
@@ -81,6 +82,19 @@ DENSE_KERNEL = {"A0_lin": r"{L}{one}, false(, (true|false))?>", "A1": r"{L}true,
                 "rev_H1": r"k_gemm_rows<{F}, {F}, {F}, \d, false"}   # {one}: one polynomial per channel in layer 0
 # {L}: the linears' kernels up to their arguments (with a contraction, with factors)
 LINEARS = {"float64": r"k_linear<double, \d, ", "float32": r"(k_linear<float, \d, |k_linear32<\d, \d, )"}
+
+
+def dense_peak(stage, dtype, N, K, L_max, contraction):
+    """Matrix-core peak behind a dense stage.  The linears of the A-basis take k_linear32 by its dispatch's rule (N: local nodes;
+    contraction: the symmetric contraction is in the same launch, behind sums of K terms in layer 0 and for scalar hidden features)."""
+    if stage == "H2":      # the tail works in double whatever the feature precision
+        return MFMA_PEAK["float64"]
+    if dtype == "float32" and stage in ("A0_lin", "A1", "rev_A1", "rev_A0_lin") and N >= 512:
+        if K % 128 == 0 and (not contraction or N >= 2048 or (stage == "A1" and L_max > 0)):
+            return MFMA_PEAK_BF16_PARTS
+        if K % 96 == 0 and not contraction and N >= 1024:
+            return MFMA_PEAK_BF16_PARTS
+    return MFMA_PEAK[dtype]
 
 
 def dense_flops(stage, N, K, n_LM, n_e):
@@ -507,8 +521,8 @@ def main():
             ms_k = res["stages"].get(k, 0.0)
             n_k = (N + N_ghost) if k in ("A0_lin", "H1", "rev_H1", "rev_A0_lin") else N
             fl = dense_flops(k, n_k, K, n_LM, n_e)
-            # the tail works in double whatever the feature precision; a stage folded into another launch has no time of its own
-            peak = MFMA_PEAK["float64"] if k == "H2" else MFMA_PEAK[dtype]
+            # (a stage folded into another launch has no time of its own)
+            peak = dense_peak(k, dtype, N, K, L_max, res["stages"].get({"A0_lin": "M0", "A1": "M1"}.get(k), 1.0) == 0.0)
             if ms_k == 0.0:
                 mfma[k] = {"flops": fl, "note": "folded into another launch (sender_reduce carries reverse_H1 for scalar hidden features)"}
                 continue
