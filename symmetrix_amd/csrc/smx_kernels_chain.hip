@@ -132,9 +132,11 @@ __device__ __forceinline__ BlockAtom block_atom(const int* perm, const int* tsta
 
 constexpr int chain_threads(int K) { return 8 * K; }      // two sets of (l, m) for every 16 columns
 // Wavefronts per SIMD the kernels are compiled for: one block of 128 channels on a CU, two of 64, four of 32, and two of 96 channels
-// in single precision.  There k_chain1 spills 9 to 15 registers for it, which pays where CUs have a second block: evaluations,
-// us, with six / with four and nothing spilled: l = 0, 24 atoms 67 / 67, 107 76 / 72, 300 92 / 96, 501 96 / 101, 1 000 165 / 173;
-// l <= 1, 107 145 / 141, 500 223 / 228.
+// in single precision.  There k_chain1 spills 12 registers with the edges (l = 0) and 2 without, k_chain0 of l <= 2 with the edges 7,
+// which pays where CUs have a second block: evaluations, us, with six / with four and nothing spilled: l = 0, 24 atoms 57 / 57, 107
+// 65 / 64, 256 76 / 74, 300 93 / 107, 501 98 / 114, 1 000 171 / 203; l <= 1, 107 120 / 118, 256 144 / 142, 500 216 / 225; l <= 2, 24
+// 156 / 151, 256 221 / 218, 400 337 / 351.  In double precision k_chain1 of l = 0 with the edges spills 2 registers from 64 channels on,
+// k_chain0 of l <= 2 with the edges 4 at 32 channels.
 template <typename F> constexpr int chain_waves(int K) { return sizeof(F) == 4 && K == 96 ? 6 : 4; }
 
 // The products of a few rows per atom (polynomials, scalar features) with K x K weights: a thread takes 16 bytes of columns and a
@@ -591,10 +593,11 @@ __global__ __launch_bounds__(chain_threads(K), chain_waves<F>(K)) void k_chain1(
 constexpr int kBucket = 256;       // edges of a sender that are put in order in LDS
 constexpr int kPolySlots = 4;      // groups of wavefronts that share the polynomials of layer 0
 template <int NP> constexpr int kMsgWords = NP == 1 ? 4 : 8;     // 16-byte words of messages that a thread brings at once
-// In double precision l <= 1 spills 38 to 42 registers of the polynomials' adjoints, l <= 2 up to 8.  With the registers of one block
-// per CU (K / 32 wavefronts per SIMD) l <= 1 spills none up to 96 channels; evaluations, us, as it is / so: 32 channels 200 atoms
-// 120 / 118, 1 000 243 / 246; 64 channels 48 117.5 / 117.2, 200 140 / 138, 768 288 / 294 (no second block on a CU); 96 channels,
-// where there is one block either way, 107 153 / 151, 500 324 / 320.
+// In double precision l <= 1 spills 38 to 48 registers of the polynomials' adjoints (44 at 128 channels with the edges, 38 without, where
+// the wavefronts of a block leave 128 registers each in any case), l <= 2 up to 8.  With the registers of one block per CU (K / 32
+// wavefronts per SIMD) l <= 1 spills none up to 96 channels; evaluations, us, as it is / so: 32 channels 200 atoms 109 / 109, 1 000
+// 246 / 245; 64 channels 48 121 / 120, 200 141 / 139, 768 390 / 404 (no second block on a CU); 96 channels, where there is one block
+// either way, 107 159 / 158, 250 233 / 231, 500 427 / 425.
 template <typename F, int LH, int K, bool EDGES>
 __global__ __launch_bounds__(chain_threads(K), LH == 0 ? chain_waves<F>(K) : 4) void k_chain2(const ChainParams<F> p, const AggParams<F> agg)
 {

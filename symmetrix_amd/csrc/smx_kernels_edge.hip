@@ -264,7 +264,8 @@ __device__ __forceinline__ void block_values(const AggParams<F>& a, const double
 template <typename F, int LMAXH, int CPL, bool BWD>
 constexpr int path_sets() { return LMAXH == 2 && (!BWD || sizeof(F) == 8 || CPL == 2) ? 2 : 1; }
 
-// Thread blocks per CU (wavefronts per SIMD) the kernels are compiled for: 168 or 256 registers a lane
+// Thread blocks per CU (wavefronts per SIMD) the kernels are compiled for: 168 or 256 registers a lane (none spilled, except 8 by the
+// adjoint of l <= 2 in double precision for files that couple outside the selection rules)
 template <typename F, int LMAXH, int CPL, bool BWD>
 constexpr int agg_blocks()
 {
@@ -1191,6 +1192,7 @@ hipError_t launch_fpart_reduce(long edges, long E, int groups, const double* fpa
 
 // ---------------------------------------------------------------------------
 namespace {
+// (for callers that ask for the harmonics; spills 6 registers)
 __global__ void k_sph_harm(const double* xyz, long E, double* Y, double* Yg)
 {
     const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;

@@ -25,7 +25,7 @@ namespace {
 // Wavefronts per SIMD (thread blocks per CU) of the adjoint: what the registers of its channels allow.  20 011 atoms, 96 channels,
 // single: adjoints of 275 and 264 us with two, 253 and 237 with three; double, two channels per lane, layer 0: 600 atoms, 64 and 128
 // channels 24 / 21 and 33 / 30, 10 000 atoms 243 / 231 and 455 / 441, 24 999 atoms 1 033 / 1 008 (l <= 1), 50 000 atoms 2 828 /
-// 2 858 (78 edges an atom).  Where messages are stored as well, double and two channels per lane: see launch0.
+// 2 858 (78 edges an atom; two edges at a time without messages spill one register).  Where messages are stored as well, double and two channels per lane: see launch0.
 template <typename F, int CPL>
 constexpr int bwd0_blocks() { return CPL <= (sizeof(F) == 8 ? 2 : 3) ? 3 : 2; }
 // edges per chunk: one lane each (two are left for a look at the next chunk), as many as leave room for the thread blocks of a CU
