@@ -210,7 +210,7 @@ struct ChainEdges {
                         V[1] = l == 1 ? R * u[1] : V[1] + R * u[1];
                         V[2] = l == 1 ? R * u[2] : V[2] + R * u[2];
                     } else {
-                        // as k_agg0_bwd: the same bits with the edges in the chain and without
+                        // as k_agg0_bwd: the sums of an order with the same bits (what follows adds channels in another order there)
                         F u[3] = {F(0), F(0), F(0)};
                         static_for<l * l, (l + 1) * (l + 1)>([&](auto qc) {
                             constexpr int q = decltype(qc)::value, v = 3 * q;

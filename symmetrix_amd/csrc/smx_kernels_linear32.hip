@@ -407,7 +407,8 @@ hipError_t launch_linear32_t(const LinearParams<float>& p, hipStream_t s)
 
 }  // namespace
 
-// 128 channels (and multiples): always, so that the sums of an atom do not depend on the size of the system.  96: from 1 024 atoms.
+// 128 channels (and multiples): linears without a contraction always, so that from 512 atoms on, where the launches of row tiles begin, the
+// sums of an atom do not depend on the size of the system.  A contraction behind sums of K terms from 2 048 atoms; 96 channels from 1 024.
 // k_linear / this, us, launches alone: 128 channels A0 600 atoms 9.9 / 10.7, 1 500 15.8 / 12.4, 10 000 66 / 44, 50 000 310 / 230; its
 // adjoint (factors) 600 12.5 / 12.1, 50 000 331 / 250; adjoint of A1, l <= 1, 600 17 / 13, 3 000 52 / 39, 50 000 702 / 532; A1 and its
 // contraction, l <= 1, 1 100 36.7 / 38.8, 3 000 54.8 / 41.1, 10 000 145 / 127, 30 000 406 / 357; l = 0 1 100 18.7 / 23.5, 3 000 27.5 /
