@@ -975,8 +975,9 @@ struct Engine : EngineBase {
     // channels 256 118 / 105, 300 167 / 182, 64 channels 200 76 / 61, 1 500 213 / 203, 32 channels 1 000 99 / 88, 2 000 158 / 143,
     // 3 000 194 / 197; single, 96 channels 24 71 / 60, 501 96 / 87, 1 000 165 / 152, 128 channels 256 88 / 77, 400 125 / 129, 64
     // channels 1 500 156 / 144, 32 channels 3 000 149 / 141; l <= 1 (layer 0 only), 128 channels double 107 201 / 198, 256 250 / 242,
-    // 500 442 / 443, single 200 150 / 142, 96 channels 600 303 / 309, 64 channels 1 000 258 / 253; l <= 2, 64 channels double 700
-    // 507 / 503.
+    // 500 442 / 443, single 200 150 / 142, 96 channels 600 303 / 309, 64 channels 1 000 258 / 253; l <= 2, 128 channels double 24 228 / 227,
+    // 128 292 / 288, 256 449 / 447, single 24 183 / 172, 256 268 / 255, 96 channels double 24 190 / 187, 256 382 / 377, single 250 222 / 208, 64
+    // channels double 24 161 / 154, 700 558 / 545, single 700 337 / 328.
     // Ghost nodes have blocks in layer 0 only, so that all nodes have a line of their own there: local / all nodes, us as above
     // (separate in the order of the chains): one l, double, 96 channels 230 / 748 190 / 183, 256 / 850 209 / 212, 128 channels
     // 100 / 405 159 / 160, 150 / 591 203 / 213, 200 / 686 212 / 220, 250 / 842 256 / 271, 32 channels 1 850 / 3 721 211 / 211, 2 048 / 3 959
