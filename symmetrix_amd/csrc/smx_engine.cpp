@@ -1445,6 +1445,7 @@ struct Engine : EngineBase {
                       const double* rr, long E_, bool on_device, double* d_energies, double* d_forces, int N_local,
                       long E_local)
     {
+        edges_in_chains = 0;
         if (N < 0 || E_ < 0) throw Error(SMX_EINVAL, "negative num_nodes or num_edges");
         if (E_ > 2147483647L) throw Error(SMX_EINVAL, "more than 2^31 - 1 edges: edge offsets are 32-bit");
         // ghost nodes (the last N - N1 nodes and their edges) go through layer 0 only: their H1 rows feed the
@@ -1516,7 +1517,6 @@ struct Engine : EngineBase {
             st_zbl(N1);
         }
         const bool chain = use_chains(N);
-        edges_in_chains = 0;
         if (chain && chain_edges(0, N)) edges_in_chains = 1;
         if (edges_in_chains) stage_absent(ST_AGG0F);
         else { stage_begin(ST_AGG0F); st_agg0_fwd(N); stage_end(ST_AGG0F); }
